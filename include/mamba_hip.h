@@ -437,18 +437,22 @@ int ssd_combined_bwd(const SsdParams *p, mamba_stream_t stream);
  * has another sequence id than l.  x, out, dout, dx are of `dtype` and addressed through
  * (batch, channel, position) element strides; either the position stride or the
  * channel stride of all of them must be 1 (the two layouts of the callers).  weight
- * (dim, width), bias (dim), dweight, dbias are fp32 contiguous; dweight and dbias MUST be
- * zero on entry (the kernels add into them).  width is 2, 3 or 4.
- * The backward pass re-computes the pre-activation from x.
+ * (dim, width) and bias (dim) are contiguous, of `weight_dtype`.  width is 2, 3 or 4.
+ * The backward pass re-computes the pre-activation from x.  With dw_part, a caller-owned fp32 workspace of
+ * causal_conv1d_bwd_nparts(p) x dim x 5 (contents ignored), the workgroups leave their sums of the filter and bias
+ * gradients there and the call adds them up in a fixed order into dweight (dim, width) and dbias (dim), written in
+ * `weight_dtype`: no atomics, the same bits every time.  Without dw_part dweight and dbias are fp32 and MUST be zero
+ * on entry: the kernels add into them.
  * ------------------------------------------------------------------------- */
 typedef struct CausalConvParams {
   int32_t batch, dim, seqlen, width;
   int32_t dtype; /* MAMBA_F32 / MAMBA_BF16 / MAMBA_F16 */
   int32_t silu;  /* 1: SiLU after the convolution */
-  int32_t reserved0, reserved1;
+  int32_t weight_dtype; /* dtype code of weight and bias (and, with dw_part, of dweight and dbias); MAMBA_F32 = 0 */
+  int32_t reserved1;
   const void *x;
-  const float *weight;
-  const float *bias;      /* nullable */
+  const void *weight;
+  const void *bias;       /* nullable */
   const int32_t *seq_idx; /* nullable, (batch, seqlen) contiguous */
   void *out;              /* forward only */
   int64_t x_bs, x_cs, x_ls; /* batch / channel / position stride */
@@ -456,12 +460,13 @@ typedef struct CausalConvParams {
   /* ---- backward only ---- */
   const void *dout;
   void *dx;
-  float *dweight;
-  float *dbias; /* nullable */
+  void *dweight;
+  void *dbias; /* nullable */
   int64_t dout_bs, dout_cs, dout_ls;
   int64_t dx_bs, dx_cs, dx_ls;
-  /* deterministic backward (all null: float atomics): fixed-point scale {s, 1 / s} on the device and int64 shadows
-   * of dweight (dim, width) and dbias (dim), zero on entry; the caller converts them with ssd_det_convert */
+  /* deterministic backward without dw_part (all null: float atomics): fixed-point scale {s, 1 / s} on the device and
+   * int64 shadows of dweight (dim, width) and dbias (dim), zero on entry; the caller converts them with
+   * ssd_det_convert */
   const float *det_scale;
   int64_t *det_dweight, *det_dbias;
 } CausalConvParams;
@@ -488,10 +493,14 @@ typedef struct CausalConvUpdateParams {
   int32_t state_rows; /* rows of conv_state; an index outside [0, state_rows) is a padding entry */
   int32_t weight_dtype; /* dtype code of weight and bias (MAMBA_F32 = 0 / MAMBA_BF16 / MAMBA_F16) */
   const void *x;
+  float *dw_part; /* nullable, see above */
   void *conv_state;
   const void *weight; /* (dim, width) of weight_dtype, contiguous */
   const void *bias;   /* nullable; (dim) of weight_dtype */
   void *out;
+/* Partial sums the backward call leaves in dw_part for these sizes, strides and pointers on the current device (> 0),
+ * or an error code. */
+int causal_conv1d_bwd_nparts(const CausalConvParams *p);
   const int32_t *conv_state_indices; /* nullable */
   int64_t x_bs, x_cs, x_ls;
   int64_t out_bs, out_cs, out_ls;

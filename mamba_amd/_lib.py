@@ -72,12 +72,12 @@ class SsdParams(ctypes.Structure):
 
 class CausalConvParams(ctypes.Structure):
     _fields_ = (
-        [(n, c_i32) for n in ("batch", "dim", "seqlen", "width", "dtype", "silu", "reserved0", "reserved1")]
+        [(n, c_i32) for n in ("batch", "dim", "seqlen", "width", "dtype", "silu", "weight_dtype", "reserved1")]
         + [(n, c_vp) for n in ("x", "weight", "bias", "seq_idx", "out")]
         + [(n, c_i64) for n in ("x_bs", "x_cs", "x_ls", "out_bs", "out_cs", "out_ls")]
         + [(n, c_vp) for n in ("dout", "dx", "dweight", "dbias")]
         + [(n, c_i64) for n in ("dout_bs", "dout_cs", "dout_ls", "dx_bs", "dx_cs", "dx_ls")]
-        + [(n, c_vp) for n in ("det_scale", "det_dweight", "det_dbias")]
+        + [(n, c_vp) for n in ("det_scale", "det_dweight", "det_dbias", "dw_part")]
     )
 
 

@@ -12,6 +12,8 @@
 // The backward pass re-computes the pre-activation from x instead of storing it.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int MAXW = 4;
@@ -22,54 +24,162 @@ DEVI float dsilu(float pre) {  // d/dpre silu(pre)
 }
 DEVI float silu_f(float v) { return v * sigmoid_f(v); }
 
-// Shared sums (dweight, dbias): float atomics, or -- deterministic mode, p.det_scale set -- 64-bit integer atomics
-// on terms scaled to a fixed point, whose result does not depend on the order of the adds (see SsdParams).
-DEVI void conv_acc_add(const CausalConvParams &p, float *dst, int64_t *shadow, int64_t idx, float v) {
-  if (p.det_scale) {
-    det_add(shadow, idx, v, p.det_scale[0]);
-  } else {
-    unsafeAtomicAdd(dst + idx, v);
+// A workgroup's sums for channel c: taps (right-aligned as in load_taps) and bias.  Its own row `part` of dw_part
+// where the caller gave that workspace; else float atomics into the shared sums, or -- p.det_scale set -- 64-bit
+// integer atomics on terms scaled to a fixed point, whose result does not depend on the order of the adds (see
+// SsdParams).
+constexpr int NSUM = MAXW + 1;
+DEVI void conv_sums_out(const CausalConvParams &p, int part, int c, const float (&dw)[MAXW], float db) {
+  if (p.dw_part) {
+    float *dst = p.dw_part + ((int64_t)part * p.dim + c) * NSUM;
+#pragma unroll
+    for (int k = 0; k < MAXW; ++k) dst[k] = dw[k];
+    dst[MAXW] = db;
+    return;
   }
-}
-
-// Taps right-aligned in 4 slots: slot 3 multiplies x[l], slot 0 multiplies x[l - 3].
-DEVI void load_taps(const CausalConvParams &p, int c, float (&w)[MAXW], float &bias) {
+  auto add = [&](void *sum, int64_t *shadow, int64_t idx, float v) {
+    if (v == 0.f) return;
+    if (p.det_scale) det_add(shadow, idx, v, p.det_scale[0]);
+    else unsafeAtomicAdd(static_cast<float *>(sum) + idx, v);
+  };
 #pragma unroll
   for (int k = 0; k < MAXW; ++k) {
     const int j = k - (MAXW - p.width);
-    w[k] = j >= 0 ? p.weight[(int64_t)c * p.width + j] : 0.f;
+    if (j >= 0) add(p.dweight, p.det_dweight, (int64_t)c * p.width + j, dw[k]);
   }
-  bias = p.bias ? p.bias[c] : 0.f;
+  if (p.dbias) add(p.dbias, p.det_dbias, c, db);
+}
+
+// dweight / dbias: the rows of dw_part added up in order, written in the parameters' dtype.  One thread per (channel,
+// tap or bias), eight rows in flight.
+__global__ __launch_bounds__(256) void conv_reduce_kernel(const CausalConvParams p, int nparts) {
+  const int i = blockIdx.x * 256 + threadIdx.x, row = p.dim * NSUM;
+  if (i >= row) return;
+  const int c = i / NSUM, k = i - c * NSUM;
+  if (k == MAXW ? !p.dbias : k < MAXW - p.width) return;
+  const float *src = p.dw_part + i;
+  float acc = 0.f;
+  int q = 0;
+  for (; q + 8 <= nparts; q += 8) {
+    float v[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] = src[(int64_t)(q + j) * row];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc += v[j];
+  }
+  for (; q < nparts; ++q) acc += src[(int64_t)q * row];
+  if (k == MAXW) st_param(p.dbias, p.weight_dtype, c, acc);
+  else st_param(p.dweight, p.weight_dtype, (int64_t)c * p.width + k - (MAXW - p.width), acc);
+}
+
+// Taps of n channels c0 .. (n <= NCH; the last one again beyond), right-aligned in 4 slots: slot 3 multiplies x[l], slot
+// 0 multiplies x[l - 3].  One switch over the dtype around all of the loads: a switch per value makes every load wait
+// for the one before it.
+template <int NCH> DEVI void load_taps(const CausalConvParams &p, int c0, int n, float (&w)[NCH][MAXW], float (&bias)[NCH]) {
+  auto run = [&](auto *wt, auto *bt) {
+    typedef std::remove_const_t<std::remove_pointer_t<decltype(wt)>> W;
+    W wr[NCH][MAXW], br[NCH];
+    const int lead = MAXW - p.width;
+#pragma unroll
+    for (int e = 0; e < NCH; ++e) {
+      const int64_t c = c0 + min(e, n - 1);
+#pragma unroll
+      for (int k = 0; k < MAXW; ++k) wr[e][k] = wt[c * p.width + max(k - lead, 0)];
+      br[e] = bt ? bt[c] : W{};
+    }
+#pragma unroll
+    for (int e = 0; e < NCH; ++e) {
+#pragma unroll
+      for (int k = 0; k < MAXW; ++k) w[e][k] = k >= lead ? ld1<W>(&wr[e][k]) : 0.f;
+      bias[e] = bt ? ld1<W>(&br[e]) : 0.f;
+    }
+  };
+  switch (p.weight_dtype) {
+    case MAMBA_BF16: run(static_cast<const bf16_t *>(p.weight), static_cast<const bf16_t *>(p.bias)); break;
+    case MAMBA_F16: run(static_cast<const f16_t *>(p.weight), static_cast<const f16_t *>(p.bias)); break;
+    default: run(static_cast<const float *>(p.weight), static_cast<const float *>(p.bias)); break;
+  }
 }
 
 // ------------------------------------------------------------------ position-contiguous rows
-// Element j of win[] is position l0 - 3 + j; positions outside [0, L) read as 0.
-template <typename T, bool VEC, int NWIN> DEVI void load_window(const T *row, int l0, int L, float (&win)[NWIN]) {
-  static_assert(NWIN == 11 || NWIN == 19, "3 halo positions, 8 own, optionally 8 following");
-  if constexpr (VEC) {  // l0 is a multiple of 8, L a multiple of 8, the row 16-byte aligned
-    Pack8<T> prev, cur, next;
-    prev.load(row + max(l0 - 8, 0));
-    cur.load(row + l0);
-    if (NWIN == 19) next.load(row + min(l0 + 8, L - 8));
-    float a[8], c[8];
-    prev.unpack(a);
-    cur.unpack(c);
+// A workgroup of 256 threads is `tx` threads along the positions (8 each) by 256 / tx channels; the host picks tx, a
+// power of two of 16 .. 256, so that short rows leave few threads without positions.
+struct RowPos {
+  int c, b, l0, tx, slot;
+  bool live;
+};
+// WAVE: a wave lies inside one channel (tx >= 64), whose taps are then scalar loads
+template <bool WAVE> DEVI RowPos row_position(const CausalConvParams &p, int txlog) {
+  RowPos q;
+  q.tx = 1 << txlog;
+  q.slot = threadIdx.x >> txlog;
+  if (WAVE) q.slot = __builtin_amdgcn_readfirstlane(q.slot);
+  q.c = blockIdx.y * (256 >> txlog) + q.slot;
+  q.b = blockIdx.z;
+  q.l0 = (blockIdx.x * q.tx + (threadIdx.x & (q.tx - 1))) * 8;
+  q.live = q.c < p.dim && q.l0 < p.seqlen;
+  return q;
+}
+
+// How the rows are reached: element by element (L < 8), in 16-byte pieces of aligned rows of whole pieces, or in 16-byte
+// pieces at any alignment with a ragged last piece.
+constexpr int SCALAR = 0, ALIGNED = 1, ANY = 2;
+
+// Positions l0 - 3 .. of a row, l0 a multiple of 8: the previous piece (for its last 3), this one and, NEXT, the
+// following one, from positions that keep inside the row.  load() only requests them, so that a kernel can request
+// every window it needs before it uses the first; window() puts them in place: element j is position l0 - 3 + j, 0
+// outside [0, L).
+template <typename T, int MODE, bool NEXT> struct RowWindow {
+  static constexpr int NWIN = NEXT ? 19 : 11;
+  Pack8<T> prev, cur, next;
+  float s[NWIN];
+  DEVI void load(const T *row, int l0, int L) {
+    if constexpr (MODE == ALIGNED) {
+      prev.load(row + max(l0 - 8, 0));
+      cur.load(row + l0);
+      if (NEXT) next.load(row + min(l0 + 8, L - 8));
+    } else if constexpr (MODE == ANY) {
+      prev.load_any(row + max(l0 - 8, 0));
+      cur.load_any(row + min(l0, L - 8));
+      if (NEXT) next.load_any(row + min(l0 + 8, L - 8));
+    } else {
 #pragma unroll
-    for (int j = 0; j < 3; ++j) win[j] = l0 >= 8 ? a[5 + j] : 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) win[3 + j] = c[j];
-    if constexpr (NWIN == 19) {
-      float n[8];
-      next.unpack(n);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) win[11 + j] = l0 + 8 < L ? n[j] : 0.f;
+      for (int j = 0; j < NWIN; ++j) {
+        const int l = l0 - 3 + j;
+        s[j] = (l >= 0 && l < L) ? ld1<T>(row + l) : 0.f;
+      }
     }
+  }
+  DEVI void window(int l0, int L, float (&win)[NWIN]) const {
+    if constexpr (MODE == SCALAR) {
+#pragma unroll
+      for (int j = 0; j < NWIN; ++j) win[j] = s[j];
+    } else {
+      float a[8], c[8], n[8];
+      prev.unpack(a);
+      cur.unpack(c);
+      if (MODE == ANY) row8_place(l0, L, c);
+#pragma unroll
+      for (int j = 0; j < 3; ++j) win[j] = l0 >= 8 ? a[5 + j] : 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) win[3 + j] = c[j];
+      if constexpr (NEXT) {
+        next.unpack(n);
+        if (MODE == ANY) row8_place(l0 + 8, L, n);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) win[11 + j] = l0 + 8 < L ? n[j] : 0.f;
+      }
+    }
+  }
+};
+// 8 results at l0: 16 bytes, or element by element in the last piece of a ragged row
+template <typename T, int MODE> DEVI void store_row8(T *row, int l0, int L, const float (&o)[8]) {
+  if constexpr (MODE == ALIGNED) {
+    st8<T>(row + l0, o);
+  } else if (MODE == ANY && l0 + 8 <= L) {
+    st8_any<T>(row + l0, o);
   } else {
-#pragma unroll
-    for (int j = 0; j < NWIN; ++j) {
-      const int l = l0 - 3 + j;
-      win[j] = (l >= 0 && l < L) ? ld1<T>(row + l) : 0.f;
-    }
+    st8_guard<T, false>(row + l0, min(8, L - l0), o);
   }
 }
 template <int NWIN> DEVI void load_ids(const int32_t *seq, int l0, int L, int (&ids)[NWIN]) {
@@ -80,14 +190,18 @@ template <int NWIN> DEVI void load_ids(const int32_t *seq, int l0, int L, int (&
   }
 }
 
-template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_rows_fwd_kernel(const CausalConvParams p) {
-  const int L = p.seqlen, c = blockIdx.y, b = blockIdx.z;
-  const int l0 = (blockIdx.x * 256 + threadIdx.x) * 8;
-  if (l0 >= L) return;
-  float w[MAXW], bias;
-  load_taps(p, c, w, bias);
+template <typename T, int MODE, bool WAVE> __global__ __launch_bounds__(256) void conv_rows_fwd_kernel(const CausalConvParams p, int txlog) {
+  const RowPos q = row_position<WAVE>(p, txlog);
+  if (!q.live) return;
+  const int L = p.seqlen, c = q.c, b = q.b, l0 = q.l0;
+  RowWindow<T, MODE, false> rx;
+  rx.load(static_cast<const T *>(p.x) + b * p.x_bs + c * p.x_cs, l0, L);
+  float wt[1][MAXW], bt[1];
+  load_taps<1>(p, c, 1, wt, bt);
+  const float(&w)[MAXW] = wt[0];
+  const float bias = bt[0];
   float win[11];
-  load_window<T, VEC, 11>(static_cast<const T *>(p.x) + b * p.x_bs + c * p.x_cs, l0, L, win);
+  rx.window(l0, L, win);
   int ids[11];
   if (p.seq_idx) load_ids<11>(p.seq_idx + (int64_t)b * L, l0, L, ids);
   float o[8];
@@ -102,19 +216,52 @@ template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_rows
     }
     o[i] = p.silu ? silu_f(v) : v;
   }
-  st8_guard<T, VEC>(static_cast<T *>(p.out) + b * p.out_bs + c * p.out_cs + l0, min(8, L - l0), o);
+  store_row8<T, MODE>(static_cast<T *>(p.out) + b * p.out_bs + c * p.out_cs, l0, L, o);
 }
 
-template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_rows_bwd_kernel(const CausalConvParams p) {
-  const int L = p.seqlen, c = blockIdx.y, b = blockIdx.z;
-  const int l0 = (blockIdx.x * 256 + threadIdx.x) * 8;
+// Sum over the tx threads of a channel: DPP adds inside rows of 16 lanes, then between the rows of a wave, then (tx >
+// 64) between waves through LDS.  The channel's last thread of its first wave holds the result: returns whether this
+// thread does.
+DEVI bool channel_sum(float (&v)[NSUM], int tx, float (*red)[NSUM]) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+#pragma unroll
+  for (int k = 0; k < NSUM; ++k) {
+    float x = row_sum_to_last(v[k]);
+    if (tx >= 32) x += dpp_f<DPP_ROW_BCAST15, 0xa>(0.f, x);
+    if (tx >= 64) x += dpp_f<DPP_ROW_BCAST31, 0xc>(0.f, x);
+    v[k] = x;
+  }
+  if (tx <= 64) return (threadIdx.x & (tx - 1)) == (unsigned)tx - 1;
+  if (lane == 63) {
+#pragma unroll
+    for (int k = 0; k < NSUM; ++k) red[wave][k] = v[k];
+  }
+  __syncthreads();
+  const int waves = tx >> 6;
+  if (lane != 63 || (wave & (waves - 1)) != 0) return false;
+  for (int w = 1; w < waves; ++w) {
+#pragma unroll
+    for (int k = 0; k < NSUM; ++k) v[k] += red[wave + w][k];
+  }
+  return true;
+}
+
+template <typename T, int MODE, bool WAVE> __global__ __launch_bounds__(256) void conv_rows_bwd_kernel(const CausalConvParams p, int txlog) {
+  __shared__ float red[4][NSUM];
+  const RowPos q = row_position<WAVE>(p, txlog);
+  const int L = p.seqlen, c = q.c, b = q.b, l0 = q.l0;
   float dw[MAXW] = {0.f, 0.f, 0.f, 0.f}, db = 0.f;
-  if (l0 < L) {
-    float w[MAXW], bias;
-    load_taps(p, c, w, bias);
+  if (q.live) {
+    RowWindow<T, MODE, true> rx, rg;
+    rx.load(static_cast<const T *>(p.x) + b * p.x_bs + c * p.x_cs, l0, L);
+    rg.load(static_cast<const T *>(p.dout) + b * p.dout_bs + c * p.dout_cs, l0, L);
+    float wt[1][MAXW], bt[1];
+    load_taps<1>(p, c, 1, wt, bt);
+    const float(&w)[MAXW] = wt[0];
+    const float bias = bt[0];
     float xw[19], gw[19];  // x and dout at positions l0 - 3 .. l0 + 15 (dout's halo is not used)
-    load_window<T, VEC, 19>(static_cast<const T *>(p.x) + b * p.x_bs + c * p.x_cs, l0, L, xw);
-    load_window<T, VEC, 19>(static_cast<const T *>(p.dout) + b * p.dout_bs + c * p.dout_cs, l0, L, gw);
+    rx.window(l0, L, xw);
+    rg.window(l0, L, gw);
     int ids[19];
     if (p.seq_idx) load_ids<19>(p.seq_idx + (int64_t)b * L, l0, L, ids);
     // gradient of the pre-activation at positions l0 .. l0 + 10 (own 8 and the 3 that still see them)
@@ -150,19 +297,12 @@ template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_rows
       }
       db += dpre[i];
     }
-    st8_guard<T, VEC>(static_cast<T *>(p.dx) + b * p.dx_bs + c * p.dx_cs + l0, min(8, L - l0), o);
+    store_row8<T, MODE>(static_cast<T *>(p.dx) + b * p.dx_bs + c * p.dx_cs, l0, L, o);
   }
-  // one atomic per wave and tap
-#pragma unroll
-  for (int k = 0; k < MAXW; ++k) dw[k] = wave_sum_to_last(dw[k]);
-  db = wave_sum_to_last(db);
-  if ((threadIdx.x & 63) == 63) {
-#pragma unroll
-    for (int k = 0; k < MAXW; ++k) {
-      const int j = k - (MAXW - p.width);
-      if (j >= 0 && dw[k] != 0.f) conv_acc_add(p, p.dweight, p.det_dweight, (int64_t)c * p.width + j, dw[k]);
-    }
-    if (p.dbias && db != 0.f) conv_acc_add(p, p.dbias, p.det_dbias, c, db);
+  float sums[NSUM] = {dw[0], dw[1], dw[2], dw[3], db};
+  if (channel_sum(sums, q.tx, red) && c < p.dim) {
+    const float taps[MAXW] = {sums[0], sums[1], sums[2], sums[3]};
+    conv_sums_out(p, b * gridDim.x + blockIdx.x, c, taps, sums[MAXW]);
   }
 }
 
@@ -184,8 +324,7 @@ template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_cl_f
   const int lbeg = (blockIdx.y * NRUN + run) * RUN, lend = min(lbeg + RUN, L);
   if (lbeg >= L) return;
   float w[8][MAXW], bias[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) load_taps(p, min(c0 + e, p.dim - 1), w[e], bias[e]);
+  load_taps<8>(p, c0, nch, w, bias);
   const T *xb = static_cast<const T *>(p.x) + b * p.x_bs + c0;
   T *ob = static_cast<T *>(p.out) + b * p.out_bs + c0;
   const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L : nullptr;
@@ -256,8 +395,7 @@ template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_cl_b
   }
   if (nch > 0 && lbeg < L) {
     float w[8][MAXW], bias[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) load_taps(p, min(c0 + e, p.dim - 1), w[e], bias[e]);
+    load_taps<8>(p, c0, nch, w, bias);
     const T *xb = static_cast<const T *>(p.x) + b * p.x_bs + c0;
     const T *gb = static_cast<const T *>(p.dout) + b * p.dout_bs + c0;
     T *dxb = static_cast<T *>(p.dx) + b * p.dx_bs + c0;
@@ -352,7 +490,7 @@ template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_cl_b
       }
     }
   }
-  // the four runs of a channel group are summed in LDS, then one atomic per channel and tap
+  // the four runs of a channel group are summed in LDS, then leave once per channel and tap
   if (run > 0) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -366,18 +504,16 @@ template <typename T, bool VEC> __global__ __launch_bounds__(256) void conv_cl_b
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       if (e >= nch) break;
+      float taps[MAXW], v = db[e];
 #pragma unroll
       for (int k = 0; k < MAXW; ++k) {
-        float v = dw[e][k];
+        taps[k] = dw[e][k];
 #pragma unroll
-        for (int r = 0; r < NRUN - 1; ++r) v += red[r][cg][e * (MAXW + 1) + k];
-        const int j = k - (MAXW - p.width);
-        if (j >= 0 && v != 0.f) conv_acc_add(p, p.dweight, p.det_dweight, (int64_t)(c0 + e) * p.width + j, v);
+        for (int r = 0; r < NRUN - 1; ++r) taps[k] += red[r][cg][e * (MAXW + 1) + k];
       }
-      float v = db[e];
 #pragma unroll
       for (int r = 0; r < NRUN - 1; ++r) v += red[r][cg][e * (MAXW + 1) + MAXW];
-      if (p.dbias && v != 0.f) conv_acc_add(p, p.dbias, p.det_dbias, c0 + e, v);
+      conv_sums_out(p, b * gridDim.y + blockIdx.y, c0 + e, taps, v);
     }
   }
 }
@@ -414,7 +550,8 @@ template <> DEVI u32x4 pack4<float>(const float (&v)[4]) {
 
 // The forward pass in the same form: 4 channels per thread, the next four positions requested before the current
 // four are worked on.
-template <typename T> __global__ __launch_bounds__(256) void conv_cl_fwd4_kernel(const CausalConvParams p) {
+// RUN: positions per thread, 32 where the grid fills the chip, 8 where it does not.
+template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_fwd4_kernel(const CausalConvParams p) {
   typedef typename Raw4<T>::type raw_t;
   constexpr int CPT = 4;
   const int L = p.seqlen, b = blockIdx.z;
@@ -424,8 +561,7 @@ template <typename T> __global__ __launch_bounds__(256) void conv_cl_fwd4_kernel
   const int lbeg = (blockIdx.y * NRUN + run) * RUN, lend = min(lbeg + RUN, L);
   if (lbeg >= L) return;
   float w[CPT][MAXW], bias[CPT];
-#pragma unroll
-  for (int e = 0; e < CPT; ++e) load_taps(p, c0 + e, w[e], bias[e]);
+  load_taps<CPT>(p, c0, CPT, w, bias);
   const T *xb = static_cast<const T *>(p.x) + b * p.x_bs + c0;
   T *ob = static_cast<T *>(p.out) + b * p.out_bs + c0;
   const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L : nullptr;
@@ -490,7 +626,8 @@ template <typename T> __global__ __launch_bounds__(256) void conv_cl_fwd4_kernel
 }
 
 // RUN: positions per thread.  A run costs a 6-position warm-up, the taps, and its share of the reduction of the
-// filter gradients: long runs (128) where the grid still fills the chip, the forward kernel's 32 otherwise.
+// filter gradients: long runs (128) where the grid still fills the chip, else 32, and 8 where even those leave compute
+// units without work (the walk down a run is a serial chain: with few workgroups its length is the kernel's time).
 template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bwd4_kernel(const CausalConvParams p) {
   typedef typename Raw4<T>::type raw_t;
   constexpr int CPT = 4;
@@ -509,8 +646,7 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bw
   }
   if (live && lbeg < L) {
     float w[CPT][MAXW], bias[CPT];
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) load_taps(p, c0 + e, w[e], bias[e]);
+    load_taps<CPT>(p, c0, CPT, w, bias);
     const T *xb = static_cast<const T *>(p.x) + b * p.x_bs + c0;
     const T *gb = static_cast<const T *>(p.dout) + b * p.dout_bs + c0;
     T *dxb = static_cast<T *>(p.dx) + b * p.dx_bs + c0;
@@ -615,7 +751,7 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bw
       }
     }
   }
-  // the four runs of a channel group are summed in LDS, then one atomic per channel and tap
+  // the four runs of a channel group are summed in LDS, then leave once per channel and tap
   if (run > 0) {
 #pragma unroll
     for (int e = 0; e < CPT; ++e) {
@@ -628,18 +764,16 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bw
   if (run == 0 && live) {
 #pragma unroll
     for (int e = 0; e < CPT; ++e) {
+      float taps[MAXW], v = db[e];
 #pragma unroll
       for (int k = 0; k < MAXW; ++k) {
-        float v = dw[e][k];
+        taps[k] = dw[e][k];
 #pragma unroll
-        for (int r = 0; r < NRUN - 1; ++r) v += red[r][cg][e * (MAXW + 1) + k];
-        const int j = k - (MAXW - p.width);
-        if (j >= 0 && v != 0.f) conv_acc_add(p, p.dweight, p.det_dweight, (int64_t)(c0 + e) * p.width + j, v);
+        for (int r = 0; r < NRUN - 1; ++r) taps[k] += red[r][cg][e * (MAXW + 1) + k];
       }
-      float v = db[e];
 #pragma unroll
       for (int r = 0; r < NRUN - 1; ++r) v += red[r][cg][e * (MAXW + 1) + MAXW];
-      if (p.dbias && v != 0.f) conv_acc_add(p, p.dbias, p.det_dbias, c0 + e, v);
+      conv_sums_out(p, b * gridDim.y + blockIdx.y, c0 + e, taps, v);
     }
   }
 }
@@ -650,15 +784,6 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bw
 // (what the reference spells, for one new position and state_len = W, as roll + insert + dot:
 // mamba_ssm/modules/mamba2.py:291-296).  The shift runs in place in ascending order, which is safe
 // because every entry is written from a higher index of the same thread's own row.
-// one filter tap or bias value of the dtype the caller's parameters have
-DEVI float ld_param(const void *base, int dtype, int64_t i) {
-  switch (dtype) {
-    case MAMBA_BF16: return ld1<bf16_t>(static_cast<const bf16_t *>(base) + i);
-    case MAMBA_F16: return ld1<f16_t>(static_cast<const f16_t *>(base) + i);
-    default: return static_cast<const float *>(base)[i];
-  }
-}
-
 template <typename T, typename S> __global__ __launch_bounds__(256) void conv_update_kernel(const CausalConvUpdateParams p) {
   const int c = blockIdx.x * 256 + threadIdx.x, b = blockIdx.y;
   if (c >= p.dim) return;
@@ -734,52 +859,93 @@ int check(const CausalConvParams *p, bool bwd) {
   if (p->batch > 65535) return MAMBA_E_UNSUPPORTED;
   if (!bwd && !p->out) return MAMBA_E_BADARG;
   if (bwd && (!p->dout || !p->dx || !p->dweight)) return MAMBA_E_BADARG;
-  if (bwd && p->det_scale && (!p->det_dweight || (p->dbias && !p->det_dbias))) return MAMBA_E_BADARG;
+  if (p->weight_dtype < MAMBA_F32 || p->weight_dtype > MAMBA_F16) return MAMBA_E_BADARG;
+  if (bwd && !p->dw_part && p->weight_dtype != MAMBA_F32) return MAMBA_E_BADARG;  // the atomic sums are fp32
+  if (bwd && !p->dw_part && p->det_scale && (!p->det_dweight || (p->dbias && !p->det_dbias))) return MAMBA_E_BADARG;
   if (p->x_ls != 1 && p->x_cs != 1) return MAMBA_E_UNSUPPORTED;
   return MAMBA_OK;
 }
 
 bool al16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 
-template <typename T> int launch_conv(const CausalConvParams &p, bool bwd, hipStream_t s) {
-  const int64_t m = 16 / sizeof(T);
-  const bool rows = p.x_ls == 1 && (bwd ? p.dout_ls == 1 && p.dx_ls == 1 : p.out_ls == 1);
-  auto ok = [&](const void *q, int64_t a, int64_t b2) { return al16(q) && a % m == 0 && b2 % m == 0; };
-  if (rows) {
-    if (p.dim > 65535) return MAMBA_E_UNSUPPORTED;
-    const bool vec = p.seqlen % 8 == 0 && ok(p.x, p.x_bs, p.x_cs) &&
-                     (bwd ? ok(p.dout, p.dout_bs, p.dout_cs) && ok(p.dx, p.dx_bs, p.dx_cs) : ok(p.out, p.out_bs, p.out_cs));
-    dim3 grid((p.seqlen + 2047) / 2048, p.dim, p.batch);
-    if (bwd) {
-      if (vec) hipLaunchKernelGGL((conv_rows_bwd_kernel<T, true>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((conv_rows_bwd_kernel<T, false>), grid, dim3(256), 0, s, p);
-    } else {
-      if (vec) hipLaunchKernelGGL((conv_rows_fwd_kernel<T, true>), grid, dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((conv_rows_fwd_kernel<T, false>), grid, dim3(256), 0, s, p);
+// Which kernel serves a problem, on which grid.
+struct Plan {
+  bool rows, vec;        // vec: the channel-last kernels of 16-byte pieces
+  int mode, txlog, run;  // rows: access and threads along the positions; channel-last: positions per thread
+  dim3 grid;
+  int nparts;      // rows of dw_part the backward kernel writes
+};
+
+int plan_conv(const CausalConvParams &p, bool bwd, Plan &q) {
+  const int64_t m = p.dtype == MAMBA_F32 ? 4 : 8;
+  q.rows = p.x_ls == 1 && (bwd ? p.dout_ls == 1 && p.dx_ls == 1 : p.out_ls == 1);
+  if (q.rows) {
+    auto al = [&](const void *ptr, int64_t a, int64_t b2) { return al16(ptr) && a % m == 0 && b2 % m == 0; };
+    q.mode = p.seqlen % 8 == 0 && al(p.x, p.x_bs, p.x_cs) &&
+                     (bwd ? al(p.dout, p.dout_bs, p.dout_cs) && al(p.dx, p.dx_bs, p.dx_cs) : al(p.out, p.out_bs, p.out_cs))
+                 ? ALIGNED
+                 : p.seqlen >= 8 ? ANY : SCALAR;
+    // the widest split of the positions among the ones that leave the fewest threads idle
+    const int units = (p.seqlen + 7) / 8;
+    int best = -1;
+    for (int t = 8; t >= 4; --t) {
+      const int covered = (units + (1 << t) - 1) >> t << t;
+      if (best < 0 || covered < best) best = covered, q.txlog = t;
     }
-  } else {
-    const bool cl = p.x_cs == 1 && (bwd ? p.dout_cs == 1 && p.dx_cs == 1 : p.out_cs == 1);
-    if (!cl) return MAMBA_E_UNSUPPORTED;
-    const bool vec = p.dim % 8 == 0 && ok(p.x, p.x_bs, p.x_ls) &&
-                     (bwd ? ok(p.dout, p.dout_bs, p.dout_ls) && ok(p.dx, p.dx_bs, p.dx_ls) : ok(p.out, p.out_bs, p.out_ls));
-    const int ygrid = (p.seqlen + RUN * NRUN - 1) / (RUN * NRUN);
-    if (ygrid > 65535) return MAMBA_E_UNSUPPORTED;
-    dim3 grid((p.dim + 511) / 512, ygrid, p.batch);
-    if (bwd) {
-      if (vec) {
-        constexpr int LONG = 128;
-        const int xg = (p.dim + 255) / 256, ylong = (p.seqlen + LONG * NRUN - 1) / (LONG * NRUN);
-        if ((int64_t)xg * ylong * p.batch >= 2 * (int64_t)cu_count())
-          hipLaunchKernelGGL((conv_cl_bwd4_kernel<T, LONG>), dim3(xg, ylong, p.batch), dim3(256), 0, s, p);
-        else
-          hipLaunchKernelGGL((conv_cl_bwd4_kernel<T, RUN>), dim3(xg, ygrid, p.batch), dim3(256), 0, s, p);
-      }
-      else hipLaunchKernelGGL((conv_cl_bwd_kernel<T, false>), grid, dim3(256), 0, s, p);
-    } else {
-      if (vec) hipLaunchKernelGGL((conv_cl_fwd4_kernel<T>), dim3((p.dim + 255) / 256, ygrid, p.batch), dim3(256), 0, s, p);
-      else hipLaunchKernelGGL((conv_cl_fwd_kernel<T, false>), grid, dim3(256), 0, s, p);
-    }
+    const int per = 256 >> q.txlog;
+    if ((p.dim + per - 1) / per > 65535) return MAMBA_E_UNSUPPORTED;
+    q.grid = dim3(best >> q.txlog, (p.dim + per - 1) / per, p.batch);
+    q.nparts = (int)q.grid.x * p.batch;
+    return MAMBA_OK;
   }
+  if (!(p.x_cs == 1 && (bwd ? p.dout_cs == 1 && p.dx_cs == 1 : p.out_cs == 1))) return MAMBA_E_UNSUPPORTED;
+  auto ok = [&](const void *ptr, int64_t a, int64_t b2) { return al16(ptr) && a % m == 0 && b2 % m == 0; };
+  q.vec = p.dim % 8 == 0 && ok(p.x, p.x_bs, p.x_ls) &&
+          (bwd ? ok(p.dout, p.dout_bs, p.dout_ls) && ok(p.dx, p.dx_bs, p.dx_ls) : ok(p.out, p.out_bs, p.out_ls));
+  const int xg = q.vec ? (p.dim + 255) / 256 : (p.dim + 511) / 512;
+  auto yg = [&](int run) { return (p.seqlen + run * NRUN - 1) / (run * NRUN); };
+  auto fills = [&](int run, int times) { return (int64_t)xg * yg(run) * p.batch >= times * (int64_t)cu_count(); };
+  q.run = RUN;
+  if (q.vec) {
+    if (bwd && fills(128, 2)) q.run = 128;
+    else if (!fills(RUN, bwd ? 1 : 2) && yg(8) <= 65535) q.run = 8;
+  }
+  if (yg(q.run) > 65535) return MAMBA_E_UNSUPPORTED;
+  q.grid = dim3(xg, yg(q.run), p.batch);
+  q.nparts = (int)q.grid.y * p.batch;
+  return MAMBA_OK;
+}
+
+template <typename T> int launch_conv(const CausalConvParams &p, bool bwd, hipStream_t s) {
+  Plan q{};
+  const int rc = plan_conv(p, bwd, q);
+  if (rc != MAMBA_OK) return rc;
+  const dim3 block(256);
+  if (q.rows) {
+#define CONV_ROWS(MODE)                                                                                                     \
+  if (q.txlog >= 6) {                                                                                                       \
+    if (bwd) hipLaunchKernelGGL((conv_rows_bwd_kernel<T, MODE, true>), q.grid, block, 0, s, p, q.txlog);                    \
+    else hipLaunchKernelGGL((conv_rows_fwd_kernel<T, MODE, true>), q.grid, block, 0, s, p, q.txlog);                        \
+  } else {                                                                                                                  \
+    if (bwd) hipLaunchKernelGGL((conv_rows_bwd_kernel<T, MODE, false>), q.grid, block, 0, s, p, q.txlog);                   \
+    else hipLaunchKernelGGL((conv_rows_fwd_kernel<T, MODE, false>), q.grid, block, 0, s, p, q.txlog);                       \
+  }
+    if (q.mode == ALIGNED) CONV_ROWS(ALIGNED)
+    else if (q.mode == ANY) CONV_ROWS(ANY)
+    else CONV_ROWS(SCALAR)
+#undef CONV_ROWS
+  } else if (bwd) {
+    if (!q.vec) hipLaunchKernelGGL((conv_cl_bwd_kernel<T, false>), q.grid, block, 0, s, p);
+    else if (q.run == 128) hipLaunchKernelGGL((conv_cl_bwd4_kernel<T, 128>), q.grid, block, 0, s, p);
+    else if (q.run == 8) hipLaunchKernelGGL((conv_cl_bwd4_kernel<T, 8>), q.grid, block, 0, s, p);
+    else hipLaunchKernelGGL((conv_cl_bwd4_kernel<T, RUN>), q.grid, block, 0, s, p);
+  } else {
+    if (!q.vec) hipLaunchKernelGGL((conv_cl_fwd_kernel<T, false>), q.grid, block, 0, s, p);
+    else if (q.run == 8) hipLaunchKernelGGL((conv_cl_fwd4_kernel<T, 8>), q.grid, block, 0, s, p);
+    else hipLaunchKernelGGL((conv_cl_fwd4_kernel<T, RUN>), q.grid, block, 0, s, p);
+  }
+  if (bwd && p.dw_part)
+    hipLaunchKernelGGL(conv_reduce_kernel, dim3((p.dim * NSUM + 255) / 256), block, 0, s, p, q.nparts);
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
 }
 
@@ -809,6 +975,13 @@ template <typename T> int launch_update(const CausalConvUpdateParams &p, hipStre
 
 extern "C" int causal_conv1d_fwd(const CausalConvParams *p, mamba_stream_t stream) { return dispatch(p, false, stream); }
 extern "C" int causal_conv1d_bwd(const CausalConvParams *p, mamba_stream_t stream) { return dispatch(p, true, stream); }
+
+extern "C" int causal_conv1d_bwd_nparts(const CausalConvParams *p) {
+  if (!p || p->batch <= 0 || p->dim <= 0 || p->seqlen <= 0 || p->batch > 65535) return MAMBA_E_BADARG;
+  Plan q{};
+  const int rc = plan_conv(*p, true, q);
+  return rc == MAMBA_OK ? q.nparts : rc;
+}
 
 extern "C" int causal_conv1d_update(const CausalConvUpdateParams *p, mamba_stream_t stream) {
   if (!p || !p->x || !p->conv_state || !p->weight || !p->out) return MAMBA_E_BADARG;

@@ -9,7 +9,6 @@ There is no CPU or PyTorch fallback: CPU tensors raise.
 import torch
 
 from mamba_amd import _lib
-from mamba_amd.utils.determinism import fixed_point_scale, use_deterministic_mode
 
 
 def _strides_bcl(t):
@@ -29,12 +28,20 @@ def _like_layout(x):
     return torch.empty(b, L, d, dtype=x.dtype, device=x.device).transpose(1, 2)
 
 
-def _fill(p, x, weight32, bias32, seq_idx, activation):
+def _params(weight, bias):
+    """The filter and bias as the kernels read them: contiguous, one dtype of fp32, bf16 and fp16."""
+    w, b = weight.detach(), bias.detach() if bias is not None else None
+    if w.dtype not in _lib.DTYPE_CODE or (b is not None and b.dtype != w.dtype):
+        w, b = w.float(), b.float() if b is not None else None
+    return w.contiguous(), b.contiguous() if b is not None else None
+
+
+def _fill(p, x, weight, bias, seq_idx, activation):
     batch, dim, seqlen = x.shape
-    p.batch, p.dim, p.seqlen, p.width = batch, dim, seqlen, weight32.shape[1]
-    p.dtype = _lib.DTYPE_CODE[x.dtype]
+    p.batch, p.dim, p.seqlen, p.width = batch, dim, seqlen, weight.shape[1]
+    p.dtype, p.weight_dtype = _lib.DTYPE_CODE[x.dtype], _lib.DTYPE_CODE[weight.dtype]
     p.silu = int(activation in ("silu", "swish"))
-    p.x, p.weight, p.bias, p.seq_idx = x.data_ptr(), weight32.data_ptr(), _lib.ptr(bias32), _lib.ptr(seq_idx)
+    p.x, p.weight, p.bias, p.seq_idx = x.data_ptr(), weight.data_ptr(), _lib.ptr(bias), _lib.ptr(seq_idx)
     p.x_bs, p.x_cs, p.x_ls = _strides_bcl(x)
 
 
@@ -60,14 +67,13 @@ def causal_conv1d_fwd(x, weight, bias=None, seq_idx=None, activation=None, out=N
     if not _usable(x):
         x = x.contiguous()
     seq_idx = seq_idx.contiguous() if seq_idx is not None else None
-    w32 = weight.detach().float().contiguous()
-    b32 = bias.detach().float().contiguous() if bias is not None else None
+    w, bv = _params(weight, bias)
     if out is None:
         out = _like_layout(x)
     elif out.shape != x.shape or out.dtype != x.dtype or out.stride(2 if x.stride(2) == 1 else 1) != 1:
         raise RuntimeError("causal_conv1d: out must match x in shape, dtype and layout")
     p = _lib.CausalConvParams()
-    _fill(p, x, w32, b32, seq_idx, activation)
+    _fill(p, x, w, bv, seq_idx, activation)
     p.out = out.data_ptr()
     p.out_bs, p.out_cs, p.out_ls = _strides_bcl(out)
     with torch.cuda.device(x.device):
@@ -94,31 +100,23 @@ def causal_conv1d_bwd(x, weight, bias, dout, seq_idx=None, activation=None, dx=N
     elif dx.shape != x.shape or dx.dtype != x.dtype or dx.stride(2 if rows else 1) != 1:
         raise RuntimeError("causal_conv1d: dx must match x in shape, dtype and layout")
     seq_idx = seq_idx.contiguous() if seq_idx is not None else None
-    w32 = weight.detach().float().contiguous()
-    b32 = bias.detach().float().contiguous() if bias is not None else None
-    dw32 = torch.zeros_like(w32)
-    db32 = torch.zeros_like(b32) if b32 is not None else None
+    w, bv = _params(weight, bias)
+    dw, db = torch.empty_like(w), torch.empty_like(bv) if bv is not None else None
     p = _lib.CausalConvParams()
-    _fill(p, x, w32, b32, seq_idx, activation)
-    p.dout, p.dx, p.dweight, p.dbias = dout.data_ptr(), dx.data_ptr(), dw32.data_ptr(), _lib.ptr(db32)
+    _fill(p, x, w, bv, seq_idx, activation)
+    p.dout, p.dx, p.dweight, p.dbias = dout.data_ptr(), dx.data_ptr(), dw.data_ptr(), _lib.ptr(db)
     p.dout_bs, p.dout_cs, p.dout_ls = _strides_bcl(dout)
     p.dx_bs, p.dx_cs, p.dx_ls = _strides_bcl(dx)
-    det = use_deterministic_mode()
-    if det:
-        # integer shadows of the two shared sums and the call's fixed-point scale (mamba_amd/utils/determinism.py)
-        sw = torch.zeros(w32.numel(), dtype=torch.int64, device=x.device)
-        sb = torch.zeros(b32.numel(), dtype=torch.int64, device=x.device) if b32 is not None else None
-        scale = fixed_point_scale(dout)
-        p.det_scale, p.det_dweight, p.det_dbias = scale.data_ptr(), sw.data_ptr(), _lib.ptr(sb)
     with torch.cuda.device(x.device):
-        lib, stream = _lib.load(), _lib.current_stream(x.device)
-        _lib.check(lib.causal_conv1d_bwd(p, stream), "causal_conv1d_bwd")
-        if det:
-            _lib.check(lib.ssd_det_convert(sw.data_ptr(), dw32.data_ptr(), sw.numel(), scale.data_ptr(), stream), "ssd_det_convert")
-            if sb is not None:
-                _lib.check(lib.ssd_det_convert(sb.data_ptr(), db32.data_ptr(), sb.numel(), scale.data_ptr(), stream),
-                           "ssd_det_convert")
-    return dx, dw32.to(weight.dtype), (db32.to(bias.dtype) if bias is not None else None)
+        lib = _lib.load()
+        nparts = lib.causal_conv1d_bwd_nparts(p)
+        if nparts <= 0:
+            _lib.check(nparts or -1, "causal_conv1d_bwd_nparts")
+        # one row of filter and bias sums per workgroup, added up in order by the call: the same bits every time
+        part = torch.empty(nparts, x.shape[1], 5, dtype=torch.float32, device=x.device)
+        p.dw_part = part.data_ptr()
+        _lib.check(lib.causal_conv1d_bwd(p, _lib.current_stream(x.device)), "causal_conv1d_bwd")
+    return dx, dw.to(weight.dtype), (db.to(bias.dtype) if bias is not None else None)
 
 
 class CausalConv1dFn(torch.autograd.Function):

@@ -310,8 +310,8 @@ typedef struct SsdParams {
   const void *dout;
   const float *dfinal_states;           /* nullable, (b, H, P, N) */
   void *dx, *dz;                        /* `dtype`, (b, L, H, P): dz contiguous, dx with the strides below */
-  void *ddt;                            /* `dt_dtype`, contiguous (b, L, H) */
-  void *dB, *dC;                        /* `dtype`, contiguous (b, L, G, N); nullable: when set, ssd_combined_bwd leaves the
+  void *ddt;                            /* `dt_dtype`, (b, L, H) with the strides at the end of the struct */
+  void *dB, *dC;                        /* `dtype`, (b, L, G, N) with the strides at the end of the struct; nullable: when set, ssd_combined_bwd leaves the
                                            finished sums of dB32 / dC32 here in the operands' dtype (its last stage writes
                                            them, so no conversion pass over the fp32 sums is needed) */
   float *dA, *ddt_bias;                 /* (H) fp32, zero on entry */
@@ -369,6 +369,11 @@ int ssd_chunk_scan_fwd_fused(const SsdParams *p, mamba_stream_t stream);
  * final_states, reads dt_out / dA_cumsum, initial_states, seq_idx; `states` is not touched.  Replaces the pair
  * _chunk_state_fwd + _state_passing_fwd of mamba_ssm/ops/triton/ssd_combined.py:375-382. */
 int ssd_chunk_state_passing_fwd(const SsdParams *p, mamba_stream_t stream);
+  /* element strides of ddt, dB and dC (slices of wider gradient buffers; dB / dC with unit dstate stride); a tensor
+   * whose three strides are all 0 is contiguous */
+  int64_t ddt_bs, ddt_ls, ddt_hs;
+  int64_t dB_bs, dB_ls, dB_gs;
+  int64_t dC_bs, dC_ls, dC_gs;
 /* cumsum; chunk_state + state_passing (in one launch, ssd_chunk_state_passing_fwd, where it applies and batch x heads
  * is at least three quarters of the compute units); then the fused scan when supported, else bmm + chunk_scan */
 int ssd_combined_fwd(const SsdParams *p, mamba_stream_t stream);

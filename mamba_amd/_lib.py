@@ -69,6 +69,7 @@ class SsdParams(ctypes.Structure):
                                "det_dA", "det_ddt_bias", "states_lp", "dstates_lp")]
     )
 
+        + [(n, c_i64) for n in ("ddt_bs", "ddt_ls", "ddt_hs", "dB_bs", "dB_ls", "dB_gs", "dC_bs", "dC_ls", "dC_gs")]
 
 class CausalConvParams(ctypes.Structure):
     _fields_ = (

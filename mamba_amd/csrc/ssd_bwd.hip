@@ -14,13 +14,25 @@
 // with g = dout * silu(z).
 #include "ssd_common.hpp"
 
+#include <algorithm>
+
 namespace {
 
 // The heads of a group are spread over this many workgroups (each sums ~8 heads in registers and
 // adds its partial result atomically).
 __host__ __device__ inline int head_splits(int heads_per_group) { return (heads_per_group + 7) / 8; }
-// The dCB kernel's lists are twice as long (~16 heads).
-__host__ __device__ inline int dcb_head_splits(int heads_per_group) { return (heads_per_group + 15) / 16; }
+// The dCB kernel's lists are twice as long (~16 heads), and shorter where the tiles alone leave compute units without
+// work (a workgroup's head takes ~2 us, one after the other: 24 heads on 2 x 4 chunks took 34 us in lists of 12, 10 in
+// lists of 2): as many lists as give every CU four workgroups, two heads at least, where there would be fewer than two.
+// A group that fits one list stays whole from one workgroup for 8 CUs on: its tiles are then stored, not added into
+// cleared memory.
+inline int dcb_head_splits(const SsdParams *p) {
+  const int hpg = p->nheads / p->ngroups, nt = (p->chunk_size + 63) / 64;
+  const int64_t tiles = (int64_t)nt * (nt + 1) / 2 * p->nchunks * p->batch * p->ngroups, want = 4 * (int64_t)cu_count();
+  const int lists = (hpg + 15) / 16;
+  if (tiles * lists >= (lists == 1 ? want / 32 : want / 2)) return lists;
+  return std::max<int>(lists, (int)std::min<int64_t>((hpg + 1) / 2, want / tiles));
+}
 
 __global__ __launch_bounds__(256) void det_convert_kernel(const int64_t *__restrict__ src, float *__restrict__ dst, int64_t n,
                                                           const float *__restrict__ scale) {
@@ -1047,7 +1059,7 @@ struct DcbShared {
 // lp: this workgroup owns its tile, and the next stage takes it as bf16 (what its MFMA operand would round the fp32
 // tile to anyway): the tile is stored as bf16, packed at the start of the dCB buffer.
 template <typename T, bool SPLIT, bool DET, bool FORM_CB, bool BELOW, int FASTP>
-DEVI void dcb_tile(const SsdParams &p, DcbShared &sh, const Block3 blk, const int lt, const int st, const bool lp) {
+DEVI void dcb_tile(const SsdParams &p, DcbShared &sh, const Block3 blk, const int lt, const int st, const bool lp, const int nsplit) {
   GemmLds &lds = sh.lds;
   auto &hA_l = sh.hA_l;
   auto &hA_s = sh.hA_s;
@@ -1058,7 +1070,7 @@ DEVI void dcb_tile(const SsdParams &p, DcbShared &sh, const Block3 blk, const in
   const int lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
   const int i = lane & 15, gq = lane >> 4;
   const int Q = p.chunk_size, L = p.seqlen, P = p.headdim, H = p.nheads, G = p.ngroups;
-  const int hpg = H / G, nsplit = dcb_head_splits(hpg);
+  const int hpg = H / G;
   const int c = blk.y, bg = blk.z / nsplit, hs = blk.z % nsplit, b = bg / G, g = bg % G;
   const int t0 = c * Q, qlim = min(Q, L - t0);
   const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L + t0 : nullptr;
@@ -1338,29 +1350,29 @@ DEVI void dcb_tile(const SsdParams &p, DcbShared &sh, const Block3 blk, const in
 }
 
 template <typename T, bool SPLIT, bool DET, bool FORM_CB = false>
-__global__ __launch_bounds__(256, 4) void bwd_dcb_kernel(const SsdParams p) {
+__global__ __launch_bounds__(256, 4) void bwd_dcb_kernel(const SsdParams p, const int nsplit) {
   __shared__ DcbShared sh;
   const Block3 blk = xcd_block();
   int lt = 0, rem = blk.x;
   while (rem > lt) { rem -= lt + 1; ++lt; }
   const int st = rem;
   if (lt != st)
-    dcb_tile<T, SPLIT, DET, FORM_CB, true, 0>(p, sh, blk, lt, st, false);
+    dcb_tile<T, SPLIT, DET, FORM_CB, true, 0>(p, sh, blk, lt, st, false, nsplit);
   else
-    dcb_tile<T, SPLIT, DET, FORM_CB, false, 0>(p, sh, blk, lt, st, false);
+    dcb_tile<T, SPLIT, DET, FORM_CB, false, 0>(p, sh, blk, lt, st, false, nsplit);
 }
 // bf16 operands on 16-byte aligned rows of FASTP = 32 or 64 values, no integer shadows
 template <bool FORM_CB, int FASTP>
-__global__ __launch_bounds__(256, 4) void bwd_dcb_rows_kernel(const SsdParams p, const int lp) {
+__global__ __launch_bounds__(256, 4) void bwd_dcb_rows_kernel(const SsdParams p, const int lp, const int nsplit) {
   __shared__ DcbShared sh;
   const Block3 blk = xcd_block();
   int lt = 0, rem = blk.x;
   while (rem > lt) { rem -= lt + 1; ++lt; }
   const int st = rem;
   if (lt != st)
-    dcb_tile<bf16_t, false, false, FORM_CB, true, FASTP>(p, sh, blk, lt, st, lp != 0);
+    dcb_tile<bf16_t, false, false, FORM_CB, true, FASTP>(p, sh, blk, lt, st, lp != 0, nsplit);
   else
-    dcb_tile<bf16_t, false, false, FORM_CB, false, FASTP>(p, sh, blk, lt, st, lp != 0);
+    dcb_tile<bf16_t, false, false, FORM_CB, false, FASTP>(p, sh, blk, lt, st, lp != 0, nsplit);
 }
 
 // ------------------------------------------------------------- bmm bwd
@@ -1437,7 +1449,7 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
   // dst[(row of the chunk) * G * N + column] += tile.  This stage is the last one to add into dB32 / dC32 and its
   // tiles cover every row once: with `fin` set the sum leaves here in the operands' dtype as well (dB / dC), and no
   // separate conversion pass over the fp32 sums is needed.
-  auto add_tile = [&](const GemmAccWide &acc, float *dst, void *fin) {
+  auto add_tile = [&](const GemmAccWide &acc, float *dst, void *fin, int64_t fin_bs, int64_t fin_ls, int64_t fin_gs) {
 #pragma unroll
     for (int tm = 0; tm < 2; ++tm)
 #pragma unroll
@@ -1445,11 +1457,12 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
         const int m = mt * GB + wm * 32 + tm * 16 + gq * 4 + r;
         if (m >= qlim) continue;
         const int64_t at = (((int64_t)b * L + t0 + m) * G + g) * N + nt * WB + wn * 64 + i;
+        const int64_t fat = b * fin_bs + (t0 + m) * fin_ls + g * fin_gs + nt * WB + wn * 64 + i;
         float *row = dst + at;
 #pragma unroll
         for (int tn = 0; tn < 4; ++tn) {
           const float v = row[tn * 16] + acc.v[tm][tn][r];
-          if (fin) st1<T>(static_cast<T *>(fin) + at + tn * 16, v);  // the finished sum: nobody reads the fp32 one
+          if (fin) st1<T>(static_cast<T *>(fin) + fat + tn * 16, v);  // the finished sum: nobody reads the fp32 one
           else row[tn * 16] = v;
         }
       }
@@ -1463,7 +1476,7 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
     const T *Ba = static_cast<const T *>(p.B) + b * p.B_bs + g * p.B_gs + (int64_t)t0 * p.B_ls + nt * WB;
     WideTrStager<SPLIT, T, WB> sb(lds.bh, lds.bl, Ba, p.B_ls, WB, nullptr, tid);
     block_gemm_wide<SPLIT>(acc, lds, kend, sa, sb, tid);
-    add_tile(acc, p.dC32, p.dC);
+    add_tile(acc, p.dC32, p.dC, p.dC_bs, p.dC_ls, p.dC_gs);
   }
   if (which == 0) lds_barrier();  // the first product's last operand reads end before the second one's first commit
   if (which != 1) {
@@ -1475,7 +1488,7 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
     const T *Ca = static_cast<const T *>(p.C) + b * p.C_bs + g * p.C_gs + (int64_t)(t0 + k0) * p.C_ls + nt * WB;
     WideTrStager<SPLIT, T, WB> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, nullptr, tid);
     block_gemm_wide<SPLIT>(acc, lds, qlim - k0, sa, sb, tid);
-    add_tile(acc, p.dB32, p.dB);
+    add_tile(acc, p.dB32, p.dB, p.dB_bs, p.dB_ls, p.dB_gs);
   }
 }
 
@@ -1541,7 +1554,7 @@ DEVI void chunk_cumsum_bwd_body(const SsdParams &p, int bx, int by, int bz) {
       const float v = p.dt_softplus ? softplus_f(x) : x;
       if (v < p.dt_min || v > p.dt_max) ddt = 0.f;
       if (p.dt_softplus && x <= 20.f) ddt *= sigmoid_f(x);
-      st_dyn(p.ddt, ((int64_t)b * L + t) * H + h, p.dt_dtype, ddt);
+      st_dyn(p.ddt, b * p.ddt_bs + t * p.ddt_ls + h * p.ddt_hs, p.dt_dtype, ddt);
     }
     dAterm = wave_sum_to_last(dAterm);
     ddt = wave_sum_to_last(ddt);
@@ -1764,7 +1777,7 @@ static bool bmm_bwd_wide_ok(const SsdParams *p);
 // tile and the bmm stage's operand is bf16 anyway (the stages on their own keep the fp32 tiles their interface names).
 static int64_t bmm_cumsum_workgroups(const SsdParams *p);
 static bool dcb_tiles_lp(const SsdParams *p) {
-  return dcb_rows_ok(p) && p->dCB && dcb_head_splits(p->nheads / p->ngroups) == 1 && bmm_bwd_wide_ok(p) &&
+  return dcb_rows_ok(p) && p->dCB && dcb_head_splits(p) == 1 && bmm_bwd_wide_ok(p) &&
          bmm_cumsum_workgroups(p) <= 0x7fffffff;  // (the one-launch form of the last two stages is the reader)
 }
 
@@ -1772,29 +1785,35 @@ static int ssd_bwd_dcb_one(const SsdParams *p, mamba_stream_t stream, bool lp) {
   int rc = check_bwd(p);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int nt = tiles(p->chunk_size);
-  dim3 grid(nt * (nt + 1) / 2, p->nchunks, p->batch * p->ngroups * dcb_head_splits(p->nheads / p->ngroups));
+  const int nt = tiles(p->chunk_size), nsplit = dcb_head_splits(p);
+  dim3 grid(nt * (nt + 1) / 2, p->nchunks, p->batch * p->ngroups * nsplit);
   if (dcb_rows_ok(p)) {
     const int lpi = lp ? 1 : 0;
     if (p->headdim == 64) {
-      if (p->CB) hipLaunchKernelGGL((bwd_dcb_rows_kernel<false, 64>), grid, dim3(256), 0, s, *p, lpi);
-      else hipLaunchKernelGGL((bwd_dcb_rows_kernel<true, 64>), grid, dim3(256), 0, s, *p, lpi);
+      if (p->CB) hipLaunchKernelGGL((bwd_dcb_rows_kernel<false, 64>), grid, dim3(256), 0, s, *p, lpi, nsplit);
+      else hipLaunchKernelGGL((bwd_dcb_rows_kernel<true, 64>), grid, dim3(256), 0, s, *p, lpi, nsplit);
     } else {
-      if (p->CB) hipLaunchKernelGGL((bwd_dcb_rows_kernel<false, 32>), grid, dim3(256), 0, s, *p, lpi);
-      else hipLaunchKernelGGL((bwd_dcb_rows_kernel<true, 32>), grid, dim3(256), 0, s, *p, lpi);
+      if (p->CB) hipLaunchKernelGGL((bwd_dcb_rows_kernel<false, 32>), grid, dim3(256), 0, s, *p, lpi, nsplit);
+      else hipLaunchKernelGGL((bwd_dcb_rows_kernel<true, 32>), grid, dim3(256), 0, s, *p, lpi, nsplit);
     }
     return launched();
   }
   if (!p->CB) {  // the workgroups form their tiles of C B^T themselves (default mode only: ssd_bwd_overwrites)
     if (p->det_scale) return MAMBA_E_BADARG;
     switch (p->dtype) {
-      case MAMBA_BF16: hipLaunchKernelGGL((bwd_dcb_kernel<bf16_t, false, false, true>), grid, dim3(256), 0, s, *p); break;
-      case MAMBA_F16: hipLaunchKernelGGL((bwd_dcb_kernel<f16_t, true, false, true>), grid, dim3(256), 0, s, *p); break;
-      default: hipLaunchKernelGGL((bwd_dcb_kernel<float, true, false, true>), grid, dim3(256), 0, s, *p); break;
+      case MAMBA_BF16: hipLaunchKernelGGL((bwd_dcb_kernel<bf16_t, false, false, true>), grid, dim3(256), 0, s, *p, nsplit); break;
+      case MAMBA_F16: hipLaunchKernelGGL((bwd_dcb_kernel<f16_t, true, false, true>), grid, dim3(256), 0, s, *p, nsplit); break;
+      default: hipLaunchKernelGGL((bwd_dcb_kernel<float, true, false, true>), grid, dim3(256), 0, s, *p, nsplit); break;
     }
     return launched();
   }
-  SSD_DISPATCH_DET(bwd_dcb_kernel, grid)
+#define SSD_LAUNCH_DCB(T, SPLIT)                                                                                      \
+  if (p->det_scale) hipLaunchKernelGGL((bwd_dcb_kernel<T, SPLIT, true>), grid, dim3(256), 0, s, *p, nsplit);          \
+  else hipLaunchKernelGGL((bwd_dcb_kernel<T, SPLIT, false>), grid, dim3(256), 0, s, *p, nsplit);
+  if (p->dtype == MAMBA_BF16) { SSD_LAUNCH_DCB(bf16_t, false) }
+  else if (p->dtype == MAMBA_F16) { SSD_LAUNCH_DCB(f16_t, true) }
+  else { SSD_LAUNCH_DCB(float, true) }
+#undef SSD_LAUNCH_DCB
   return launched();
 }
 
@@ -1820,12 +1839,13 @@ static int ssd_bmm_chunk_bwd_one(const SsdParams *p_in, mamba_stream_t stream) {
   return launched();
 }
 
+static SsdParams with_grad_strides(const SsdParams &p);
 static int ssd_chunk_cumsum_bwd_one(const SsdParams *p, mamba_stream_t stream) {
   int rc = check_bwd(p);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
   dim3 grid(p->nchunks, (p->nheads + CSB_HT - 1) / CSB_HT, p->batch);
-  hipLaunchKernelGGL(chunk_cumsum_bwd_kernel, grid, dim3(256), 0, s, *p);
+  hipLaunchKernelGGL(chunk_cumsum_bwd_kernel, grid, dim3(256), 0, s, with_grad_strides(*p));
   return launched();
 }
 
@@ -1843,27 +1863,38 @@ static bool bmm_bwd_wide_ok(const SsdParams *p) {
          reinterpret_cast<uintptr_t>(p->dCB) % 16 == 0;
 }
 
-// dst[i] = T(src[i]): the fp32 sums of dB / dC in the operands' dtype, for the paths whose last stage does not
-// write them itself
-template <typename T> __global__ __launch_bounds__(256) void cast_sum_kernel(const float *__restrict__ src, T *__restrict__ dst, int64_t n) {
+// The strides of ddt, dB and dC as the kernels take them: all 0 in the caller's struct means contiguous.
+static SsdParams with_grad_strides(const SsdParams &p) {
+  SsdParams q = p;
+  const int64_t L = p.seqlen, H = p.nheads, G = p.ngroups, N = p.dstate;
+  if (!(q.ddt_bs | q.ddt_ls | q.ddt_hs)) q.ddt_bs = L * H, q.ddt_ls = H, q.ddt_hs = 1;
+  if (!(q.dB_bs | q.dB_ls | q.dB_gs)) q.dB_bs = L * G * N, q.dB_ls = G * N, q.dB_gs = N;
+  if (!(q.dC_bs | q.dC_ls | q.dC_gs)) q.dC_bs = L * G * N, q.dC_ls = G * N, q.dC_gs = N;
+  return q;
+}
+
+// The fp32 sums of dB / dC in the operands' dtype, for the paths whose last stage does not write them itself: one
+// thread per element, blockIdx.y = 0 the dB sums, 1 the dC sums.
+template <typename T> __global__ __launch_bounds__(256) void cast_sums_kernel(const SsdParams p) {
+  const bool is_c = blockIdx.y != 0;
+  T *dst = static_cast<T *>(is_c ? p.dC : p.dB);
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (i < n) st1<T>(dst + i, src[i]);
+  if (!dst || i >= (int64_t)p.batch * p.seqlen * p.ngroups * p.dstate) return;
+  const int n = i % p.dstate, g = (i / p.dstate) % p.ngroups;
+  const int64_t row = i / ((int64_t)p.dstate * p.ngroups), b = row / p.seqlen, t = row - b * p.seqlen;
+  const int64_t at = is_c ? b * p.dC_bs + t * p.dC_ls + g * p.dC_gs : b * p.dB_bs + t * p.dB_ls + g * p.dB_gs;
+  st1<T>(dst + at + n, (is_c ? p.dC32 : p.dB32)[i]);
 }
 static int cast_sums(const SsdParams *p, mamba_stream_t stream) {
   const int64_t n = (int64_t)p->batch * p->seqlen * p->ngroups * p->dstate;
   if ((!p->dB && !p->dC) || n == 0) return MAMBA_OK;
   if ((n + 255) / 256 > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)((n + 255) / 256));
-  for (int k = 0; k < 2; ++k) {
-    void *dst = k ? p->dC : p->dB;
-    const float *src = k ? p->dC32 : p->dB32;
-    if (!dst) continue;
-    switch (p->dtype) {
-      case MAMBA_BF16: hipLaunchKernelGGL(cast_sum_kernel<bf16_t>, grid, dim3(256), 0, s, src, static_cast<bf16_t *>(dst), n); break;
-      case MAMBA_F16: hipLaunchKernelGGL(cast_sum_kernel<f16_t>, grid, dim3(256), 0, s, src, static_cast<f16_t *>(dst), n); break;
-      default: hipLaunchKernelGGL(cast_sum_kernel<float>, grid, dim3(256), 0, s, src, static_cast<float *>(dst), n); break;
-    }
+  const dim3 grid((unsigned)((n + 255) / 256), 2);
+  switch (p->dtype) {
+    case MAMBA_BF16: hipLaunchKernelGGL(cast_sums_kernel<bf16_t>, grid, dim3(256), 0, s, *p); break;
+    case MAMBA_F16: hipLaunchKernelGGL(cast_sums_kernel<f16_t>, grid, dim3(256), 0, s, *p); break;
+    default: hipLaunchKernelGGL(cast_sums_kernel<float>, grid, dim3(256), 0, s, *p); break;
   }
   return launched();
 }
@@ -1874,9 +1905,10 @@ static int64_t bmm_cumsum_workgroups(const SsdParams *p) {
   return (int64_t)tiles(p->chunk_size) * (p->dstate / WB) * p->nchunks * p->batch * p->ngroups +
          (int64_t)p->nchunks * ((p->nheads + CSB_HT - 1) / CSB_HT) * p->batch;
 }
-static int bmm_and_cumsum_bwd(const SsdParams *p, mamba_stream_t stream, bool lp = false) {
-  int rc = check_bwd(p);
+static int bmm_and_cumsum_bwd(const SsdParams *p_in, mamba_stream_t stream, bool lp = false) {
+  int rc = check_bwd(p_in);
   if (rc) return rc;
+  const SsdParams filled = with_grad_strides(*p_in), *p = &filled;
   const int64_t bmm_x = tiles(p->chunk_size) * (p->dstate / WB), bmm_y = p->nchunks, bmm_z = (int64_t)p->batch * p->ngroups;
   const int64_t cs_x = p->nchunks, cs_y = (p->nheads + CSB_HT - 1) / CSB_HT, cs_z = p->batch;
   // few tiles (fewer than four workgroups per CU): a workgroup per product instead of one per tile
@@ -1971,11 +2003,11 @@ static int ssd_combined_bwd_one(const SsdParams *p, mamba_stream_t stream) {
 extern "C" int ssd_bwd_overwrites(const SsdParams *p) {
   if (!p || check_bwd(p) != MAMBA_OK || p->det_scale || (int64_t)p->batch * p->nheads > SSD_MAX_GRID_ROWS) return 0;
   int flags = 0;
-  if (dcb_head_splits(p->nheads / p->ngroups) == 1) flags |= SSD_OVERWRITES_DCB;
+  if (dcb_head_splits(p) == 1) flags |= SSD_OVERWRITES_DCB;
   if (ssd_bwd_dbc_fused_owns(p)) flags |= SSD_OVERWRITES_DBC;
   // CB: only the dCB stage and the tiled dx kernel read it.  Where the fused dx kernel runs and a group is one head
   // list (so that each tile of C B^T would be formed once), the dCB stage can form its tiles itself.
-  if (dcb_head_splits(p->nheads / p->ngroups) == 1 && ssd_bwd_dx_fused_supported(p)) flags |= SSD_BWD_FORMS_CB;
+  if (dcb_head_splits(p) == 1 && ssd_bwd_dx_fused_supported(p)) flags |= SSD_BWD_FORMS_CB;
   return flags;
 }
 

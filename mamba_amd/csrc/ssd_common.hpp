@@ -833,7 +833,7 @@ inline SsdParams ssd_batch_slice(const SsdParams &p, int64_t b0, int nb) {
   adv(q.states, c * H * P * N, 4), adv(q.states_lp, c * H * P * N, 2), adv(q.final_states, H * P * N, 4);
   adv(q.CB, c * G * Q * Q, 4);
   adv(q.dout, p.dout_bs, es), adv(q.dfinal_states, H * P * N, 4), adv(q.dx, p.dx_bs, es), adv(q.dz, L * H * P, es);
-  adv(q.ddt, L * H, ds), adv(q.dB, L * G * N, es), adv(q.dC, L * G * N, es), adv(q.dinitial_states, H * P * N, 4);
+  adv(q.ddt, p.ddt_ls ? p.ddt_bs : L * H, ds), adv(q.dB, p.dB_ls ? p.dB_bs : L * G * N, es), adv(q.dC, p.dC_ls ? p.dC_bs : L * G * N, es), adv(q.dinitial_states, H * P * N, 4);
   adv(q.dstates, c * H * P * N, 4), adv(q.dstates_lp, c * H * P * N, 2);
   adv(q.ddA_cumsum, H * c * Q, 4), adv(q.ddt_out, H * c * Q, 4), adv(q.dCB, c * G * Q * Q, 4);
   adv(q.dB32, L * G * N, 4), adv(q.dC32, L * G * N, 4), adv(q.gbuf, L * H * P, es);

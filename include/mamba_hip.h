@@ -116,7 +116,7 @@ typedef struct MambaScanParams {
   int32_t delta_softplus;
   int32_t bc_const; /* bit 0: B is an input-independent (dim, dstate) fp32 matrix; bit 1: C likewise */
   int32_t a_complex; /* 1: complex A (see above) */
-  int32_t reserved0;
+  int32_t nseg;      /* segments of the sequence (see seg_ws); 0 or 1: the whole sequence in one go */
 
   const void *u, *delta, *A, *B, *C;
   const void *D, *z, *delta_bias; /* nullable */
@@ -140,15 +140,16 @@ typedef struct MambaScanParams {
    * which the call then adds up in a fixed order into dB / dC below (with a complex A: nparts = 1 and
    * a last axis of 2 * seqlen).  dA_part: (batch, dim, dstate), dD_part, ddelta_bias_part:
    * (batch, dim) -- written, the caller sums them over batch.  For an input-independent B (C),
-   * dB32 (dC32) is instead (batch, dim, dstate) partials, written like dA_part, and dB (dC) is unused. */
+   * dB32 (dC32) is instead (batch, dim, dstate) partials, written like dA_part, and dB (dC) is unused.  With nseg > 1
+   * the leading extent of dA_part, dD_part, ddelta_bias_part and of such dB32 / dC32 is batch * nseg. */
   float *dB32, *dC32, *dA_part, *dD_part, *ddelta_bias_part;
   int64_t dout_bs, dout_ds;
   int64_t du_bs, du_ds;
   int64_t ddelta_bs, ddelta_ds;
   int64_t dz_bs, dz_ds;
   int64_t outz_bs, outz_ds;
-  /* gradients of per-position B and C: (batch, ngroups, dstate, seqlen) of `dtype`, contiguous
-   * ((..., 2 * seqlen) with a complex A) */
+  /* gradients of per-position B and C: (batch, ngroups, dstate, seqlen) of `dtype` ((..., 2 * seqlen) with a complex
+   * A), strides at the end of the struct */
   void *dB, *dC;
   /* ---- deterministic backward with a complex A (all null: float atomics there; a real A needs none of this, its
    * backward pass has no atomics) ----
@@ -160,12 +161,30 @@ typedef struct MambaScanParams {
    * mamba_ssm/utils/determinism.py:21-27. */
   const float *det_scale;
   int64_t *det_dB, *det_dC;
+  /* ---- splitting the sequence (real A) ----
+   * A batch x channels too small to fill the GPU is served by cutting the sequence into nseg segments that run side by
+   * side: a first kernel forms what each segment adds to the state (forward) or to the adjoint (backward) that leaves
+   * it, and the scan kernels start every segment from the composition of the ones before (after) it.  seg_ws is a
+   * caller-owned fp32 workspace of batch * nseg * dim * (dstate + 2), contents ignored on entry, required when
+   * nseg > 1.  mamba1_scan_segments gives the nseg that suits a problem.  No counterpart in the reference. */
+  float *seg_ws;
+  /* ---- backward, optional ----
+   * element strides of dB / dC (batch, group, state; unit position stride), all 0: contiguous; and the finished sums
+   * of dA_part (dim, dstate), dD_part (dim), ddelta_bias_part (dim) over their leading extent, added up in a fixed
+   * order by the launch that adds up dB32 / dC32 (nullable: the caller sums the partials) */
+  int64_t dB_bs, dB_gs, dB_ns;
+  int64_t dC_bs, dC_gs, dC_ns;
+  float *dA, *dD, *ddelta_bias;
 } MambaScanParams;
+
+/* The number of segments (>= 1) that suits a problem on the current device: from batch, dim, seqlen, dstate, ngroups,
+ * dtype and a_complex; `backward` for mamba1_scan_bwd. */
+int mamba1_scan_segments(const MambaScanParams *p, int backward);
 
 int mamba1_scan_fwd(const MambaScanParams *p, mamba_stream_t stream);
 int mamba1_scan_bwd(const MambaScanParams *p, mamba_stream_t stream);
 /* Number of per-workgroup partials the backward call writes into dB32 / dC32 for these sizes on the
- * current device (> 0), or an error code.  Uses batch, dim, seqlen, dstate, ngroups, bc_const, a_complex. */
+ * current device (> 0), or an error code.  Uses batch, dim, seqlen, dstate, ngroups, bc_const, a_complex, nseg. */
 int mamba1_scan_bwd_nparts(const MambaScanParams *p);
 
 /* No counterpart in the reference.  For callers that cannot allocate device memory -- code under HIP
@@ -350,6 +369,11 @@ typedef struct SsdParams {
    * Required (non-NULL) for MAMBA_BF16, ignored for the other dtypes, which keep the fp32 `states` (in place) and
    * `dstates`. */
   void *states_lp, *dstates_lp;
+  /* element strides of ddt, dB and dC (slices of wider gradient buffers; dB / dC with unit dstate stride); a tensor
+   * whose three strides are all 0 is contiguous */
+  int64_t ddt_bs, ddt_ls, ddt_hs;
+  int64_t dB_bs, dB_ls, dB_gs;
+  int64_t dC_bs, dC_ls, dC_gs;
 } SsdParams;
 
 /* forward stages, in launch order */
@@ -369,11 +393,6 @@ int ssd_chunk_scan_fwd_fused(const SsdParams *p, mamba_stream_t stream);
  * final_states, reads dt_out / dA_cumsum, initial_states, seq_idx; `states` is not touched.  Replaces the pair
  * _chunk_state_fwd + _state_passing_fwd of mamba_ssm/ops/triton/ssd_combined.py:375-382. */
 int ssd_chunk_state_passing_fwd(const SsdParams *p, mamba_stream_t stream);
-  /* element strides of ddt, dB and dC (slices of wider gradient buffers; dB / dC with unit dstate stride); a tensor
-   * whose three strides are all 0 is contiguous */
-  int64_t ddt_bs, ddt_ls, ddt_hs;
-  int64_t dB_bs, dB_ls, dB_gs;
-  int64_t dC_bs, dC_ls, dC_gs;
 /* cumsum; chunk_state + state_passing (in one launch, ssd_chunk_state_passing_fwd, where it applies and batch x heads
  * is at least three quarters of the compute units); then the fused scan when supported, else bmm + chunk_scan */
 int ssd_combined_fwd(const SsdParams *p, mamba_stream_t stream);
@@ -474,10 +493,14 @@ typedef struct CausalConvParams {
    * ssd_det_convert */
   const float *det_scale;
   int64_t *det_dweight, *det_dbias;
+  float *dw_part; /* nullable, see above */
 } CausalConvParams;
 
 int causal_conv1d_fwd(const CausalConvParams *p, mamba_stream_t stream);
 int causal_conv1d_bwd(const CausalConvParams *p, mamba_stream_t stream);
+/* Partial sums the backward call leaves in dw_part for these sizes, strides and pointers on the current device (> 0),
+ * or an error code. */
+int causal_conv1d_bwd_nparts(const CausalConvParams *p);
 
 /* -------------------------------------------------------------------------
  * Causal conv1d, decode step: with xn = [conv_state, x] along the position axis,
@@ -498,14 +521,10 @@ typedef struct CausalConvUpdateParams {
   int32_t state_rows; /* rows of conv_state; an index outside [0, state_rows) is a padding entry */
   int32_t weight_dtype; /* dtype code of weight and bias (MAMBA_F32 = 0 / MAMBA_BF16 / MAMBA_F16) */
   const void *x;
-  float *dw_part; /* nullable, see above */
   void *conv_state;
   const void *weight; /* (dim, width) of weight_dtype, contiguous */
   const void *bias;   /* nullable; (dim) of weight_dtype */
   void *out;
-/* Partial sums the backward call leaves in dw_part for these sizes, strides and pointers on the current device (> 0),
- * or an error code. */
-int causal_conv1d_bwd_nparts(const CausalConvParams *p);
   const int32_t *conv_state_indices; /* nullable */
   int64_t x_bs, x_cs, x_ls;
   int64_t out_bs, out_cs, out_ls;
@@ -544,12 +563,11 @@ int causal_conv1d_varlen_states(const CausalConvVarlenParams *p, mamba_stream_t 
  *   x' = norm_before_gate ? x : x * silu(z);   y = (x' - mean) * rstd * weight + bias;
  *   out = norm_before_gate ? y * silu(z) : y;  statistics per (row, group), mean = 0 when is_rms.
  * x, z, out, dy, dx, dz are (rows, dim) with unit channel stride and the given row strides, all
- * of `dtype`; weight / bias are fp32 (dim); mean / rstd are fp32 (rows, dim / group_size), written
+ * of `dtype`; weight / bias are (dim) of `weight_dtype`; mean / rstd are fp32 (rows, dim / group_size), written
  * by the forward call and read by the backward call (mean may be null when is_rms).
  * Backward: dw_part / db_part are caller-provided fp32 (nparts, dim) workspaces (any nparts in
- * 1..65536; a team of 8 .. 1024 threads, the smallest power of two with 16 * threads >= group_size (128
- * skipped), works on each (group, part), and a few thousand teams fill the GPU); dweight / dbias are
- * overwritten with their sums.  group_size <= 32768.
+ * 1..65536; norm_gated_bwd_nparts gives the number that fills the GPU once); dweight / dbias are
+ * overwritten with their sums, in `weight_dtype`.  group_size <= 32768.
  * ------------------------------------------------------------------------- */
 typedef struct NormGatedParams {
   int32_t rows, dim, group_size;
@@ -560,8 +578,8 @@ typedef struct NormGatedParams {
   float eps;
   const void *x;
   const void *z; /* nullable: no gate */
-  const float *weight;
-  const float *bias; /* nullable */
+  const void *weight;
+  const void *bias;  /* nullable */
   void *out;         /* forward only */
   float *mean;       /* nullable when is_rms */
   float *rstd;
@@ -570,15 +588,19 @@ typedef struct NormGatedParams {
   const void *dy;
   void *dx;
   void *dz; /* null iff z is null */
-  float *dweight;
-  float *dbias; /* null iff bias is null */
+  void *dweight;
+  void *dbias; /* null iff bias is null */
   float *dw_part;
   float *db_part; /* null iff bias is null */
   int64_t dy_rs, dx_rs, dz_rs;
+  int32_t weight_dtype; /* dtype code of weight, bias, dweight and dbias (MAMBA_F32 = 0) */
+  int32_t reserved;
 } NormGatedParams;
 
 int norm_gated_fwd(const NormGatedParams *p, mamba_stream_t stream);
 int norm_gated_bwd(const NormGatedParams *p, mamba_stream_t stream);
+/* The number of partial rows (nparts) that suits these rows, dim, group_size and dtype on the current device. */
+int norm_gated_bwd_nparts(const NormGatedParams *p);
 
 /* -------------------------------------------------------------------------
  * LayerNorm / RMSNorm of (x + residual) with the sum handed on: the norm in front of every mixer
@@ -597,9 +619,10 @@ int norm_gated_bwd(const NormGatedParams *p, mamba_stream_t stream);
  * x, out, dy, dx are (rows, dim) of `dtype`; residual, residual_out, dresidual, dresidual_in of
  * `res_dtype` (equal to dtype, or fp32); unit channel stride, row strides given.  In the backward
  * call `x` is the summed input the forward call wrote (residual_out, or x itself when there was
- * neither a residual nor a residual_out), of res_dtype.  weight / bias fp32 (dim); mean / rstd fp32
+ * neither a residual nor a residual_out), of res_dtype.  weight / bias (dim) of weight_dtype; mean / rstd fp32
  * (rows), mean nullable when is_rms.  dw_part / db_part: fp32 (nparts, dim) workspaces, any nparts
- * in 1..65536; dweight / dbias are overwritten with the sums.  dim <= 32768.
+ * in 1..65536 (norm_residual_bwd_nparts gives the number that fills the GPU once); dweight / dbias are overwritten
+ * with the sums, in weight_dtype.  dim <= 32768.
  * ------------------------------------------------------------------------- */
 typedef struct NormResidualParams {
   int32_t rows, dim;
@@ -607,11 +630,11 @@ typedef struct NormResidualParams {
   int32_t is_rms;
   int32_t nparts; /* backward only */
   float eps;
-  int32_t reserved;
+  int32_t weight_dtype; /* dtype code of weight, bias, weight1, bias1 and their gradients (MAMBA_F32 = 0) */
   const void *x;
   const void *residual; /* forward, nullable */
-  const float *weight;
-  const float *bias;  /* nullable */
+  const void *weight;
+  const void *bias;   /* nullable */
   void *out;          /* forward only */
   void *residual_out; /* forward, nullable */
   float *mean;        /* nullable when is_rms */
@@ -622,8 +645,8 @@ typedef struct NormResidualParams {
   const void *dresidual; /* nullable */
   void *dx;
   void *dresidual_in; /* nullable */
-  float *dweight;
-  float *dbias; /* null iff bias is null */
+  void *dweight;
+  void *dbias; /* null iff bias is null */
   float *dw_part;
   float *db_part; /* null iff bias is null */
   int64_t dy_rs, dresidual_rs, dx_rs, dresidual_in_rs;
@@ -633,13 +656,13 @@ typedef struct NormResidualParams {
   const int64_t *seeds;  /* 2 device words, required when dropout_p > 0 */
   uint8_t *mask;         /* forward, nullable: (rows, dim) bytes, dense */
   uint8_t *mask1;        /* forward, nullable: the same for x1 */
-  const float *weight1;  /* (dim) */
-  const float *bias1;    /* (dim), nullable */
+  const void *weight1;   /* (dim) */
+  const void *bias1;     /* (dim), nullable */
   void *out1;            /* forward, required with weight1 */
   const void *dy1;       /* backward, required with weight1 */
   void *dx1;             /* backward, required with x1 */
-  float *dweight1;       /* backward, required with weight1, like dweight */
-  float *dbias1;         /* null iff bias1 is null */
+  void *dweight1;        /* backward, required with weight1, like dweight */
+  void *dbias1;          /* null iff bias1 is null */
   float *dw1_part;       /* (nparts, dim) workspaces like dw_part / db_part */
   float *db1_part;
   int64_t x1_rs, out1_rs, dy1_rs, dx1_rs;
@@ -649,6 +672,8 @@ typedef struct NormResidualParams {
 
 int norm_residual_fwd(const NormResidualParams *p, mamba_stream_t stream);
 int norm_residual_bwd(const NormResidualParams *p, mamba_stream_t stream);
+/* The number of partial rows (nparts) that suits these rows, dim and dtypes on the current device. */
+int norm_residual_bwd_nparts(const NormResidualParams *p);
 
 #ifdef __cplusplus
 }

@@ -20,7 +20,7 @@ c_i32, c_i64, c_vp, c_f32 = ctypes.c_int32, ctypes.c_int64, ctypes.c_void_p, cty
 
 class MambaScanParams(ctypes.Structure):
     _fields_ = (
-        [(n, c_i32) for n in ("batch", "dim", "seqlen", "dstate", "ngroups", "dtype", "delta_softplus", "bc_const", "a_complex", "reserved0")]
+        [(n, c_i32) for n in ("batch", "dim", "seqlen", "dstate", "ngroups", "dtype", "delta_softplus", "bc_const", "a_complex", "nseg")]
         + [(n, c_vp) for n in ("u", "delta", "A", "B", "C", "D", "z", "delta_bias", "out", "ckpt")]
         + [(n, c_i64) for n in ("u_bs", "u_ds", "delta_bs", "delta_ds", "z_bs", "z_ds", "out_bs", "out_ds",
                                 "B_bs", "B_gs", "B_ns", "C_bs", "C_gs", "C_ns")]
@@ -28,7 +28,9 @@ class MambaScanParams(ctypes.Structure):
                                "ddelta_bias_part")]
         + [(n, c_i64) for n in ("dout_bs", "dout_ds", "du_bs", "du_ds", "ddelta_bs", "ddelta_ds", "dz_bs", "dz_ds",
                                 "outz_bs", "outz_ds")]
-        + [("dB", c_vp), ("dC", c_vp), ("det_scale", c_vp), ("det_dB", c_vp), ("det_dC", c_vp)]
+        + [(n, c_vp) for n in ("dB", "dC", "det_scale", "det_dB", "det_dC", "seg_ws")]
+        + [(n, c_i64) for n in ("dB_bs", "dB_gs", "dB_ns", "dC_bs", "dC_gs", "dC_ns")]
+        + [(n, c_vp) for n in ("dA", "dD", "ddelta_bias")]
     )
 
 
@@ -67,9 +69,9 @@ class SsdParams(ctypes.Structure):
         + [(n, c_i64) for n in ("dout_bs", "dout_ls", "dout_hs", "dx_bs", "dx_ls", "dx_hs")]
         + [(n, c_vp) for n in ("det_scale", "det_dD", "det_ddA_cumsum", "det_ddt_out", "det_dCB", "det_dB", "det_dC",
                                "det_dA", "det_ddt_bias", "states_lp", "dstates_lp")]
+        + [(n, c_i64) for n in ("ddt_bs", "ddt_ls", "ddt_hs", "dB_bs", "dB_ls", "dB_gs", "dC_bs", "dC_ls", "dC_gs")]
     )
 
-        + [(n, c_i64) for n in ("ddt_bs", "ddt_ls", "ddt_hs", "dB_bs", "dB_ls", "dB_gs", "dC_bs", "dC_ls", "dC_gs")]
 
 class CausalConvParams(ctypes.Structure):
     _fields_ = (
@@ -108,13 +110,14 @@ class NormGatedParams(ctypes.Structure):
         + [(n, c_i64) for n in ("x_rs", "z_rs", "out_rs")]
         + [(n, c_vp) for n in ("dy", "dx", "dz", "dweight", "dbias", "dw_part", "db_part")]
         + [(n, c_i64) for n in ("dy_rs", "dx_rs", "dz_rs")]
+        + [(n, c_i32) for n in ("weight_dtype", "reserved")]
     )
 
 
 class NormResidualParams(ctypes.Structure):
     _fields_ = (
         [(n, c_i32) for n in ("rows", "dim", "dtype", "res_dtype", "is_rms", "nparts")]
-        + [("eps", ctypes.c_float), ("reserved", c_i32)]
+        + [("eps", ctypes.c_float), ("weight_dtype", c_i32)]
         + [(n, c_vp) for n in ("x", "residual", "weight", "bias", "out", "residual_out", "mean", "rstd")]
         + [(n, c_i64) for n in ("x_rs", "residual_rs", "out_rs", "residual_out_rs")]
         + [(n, c_vp) for n in ("dy", "dresidual", "dx", "dresidual_in", "dweight", "dbias", "dw_part", "db_part")]
@@ -154,6 +157,8 @@ def load():
         fn.restype = ctypes.c_int
     lib.mamba1_scan_bwd_nparts.argtypes = [ctypes.POINTER(MambaScanParams)]
     lib.mamba1_scan_bwd_nparts.restype = ctypes.c_int
+    lib.mamba1_scan_segments.argtypes = [ctypes.POINTER(MambaScanParams), ctypes.c_int]
+    lib.mamba1_scan_segments.restype = ctypes.c_int
     lib.mamba1_scan_fwd_noalloc.argtypes = [ctypes.POINTER(MambaScanParams), c_vp, c_vp]
     lib.mamba1_scan_fwd_noalloc.restype = ctypes.c_int
     lib.mamba_hip_init.argtypes = []
@@ -192,6 +197,11 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = [ctypes.POINTER(NormGatedParams), c_vp]
         fn.restype = ctypes.c_int
+    for name, params in (("norm_gated_bwd_nparts", NormGatedParams), ("norm_residual_bwd_nparts", NormResidualParams),
+                         ("causal_conv1d_bwd_nparts", CausalConvParams)):
+        fn = getattr(lib, name)
+        fn.argtypes = [ctypes.POINTER(params)]
+        fn.restype = ctypes.c_int
     lib.mamba_hip_mfma_probe.argtypes = [c_vp, ctypes.c_int, ctypes.c_int, c_vp]
     lib.mamba_hip_mfma_probe.restype = ctypes.c_int64
     lib.mamba_hip_valu_probe.argtypes = [c_vp, ctypes.c_int, ctypes.c_int, c_vp]
@@ -221,8 +231,8 @@ _torch_ext = False  # False: not tried yet; None: not built or switched off
 
 
 def torch_ext():
-    """The C++ host side of the decode-step operators (mamba_amd/_torch_ext.so, built by
-    `python -m mamba_amd.build` from csrc/torch_ext.cpp), or None when it has not been built or
+    """The C++ host side of the operators (mamba_amd/_torch_ext.so, built by
+    `python -m mamba_amd.build` from csrc/torch_*.cpp), or None when it has not been built or
     MAMBA_AMD_NO_TORCH_EXT=1 is set.  It only shortens the host time of a call: with or without it
     the same kernels of the same library run."""
     global _torch_ext
@@ -235,6 +245,8 @@ def torch_ext():
             try:
                 from mamba_amd import _torch_ext as ext
                 if ext.abi_version() == _lib.mamba_hip_query(0):
+                    from mamba_amd.utils import determinism
+                    determinism.tell(ext)
                     _torch_ext = ext
             except ImportError:
                 pass

@@ -98,6 +98,10 @@ template <typename T> struct Pack8 {
   u32x4 w;
   DEVI void load(const T *p) { w = *reinterpret_cast<const u32x4 *>(p); }  // 16-byte aligned
   DEVI void load_global(const T *p) { w = *(const GLOBAL_AS u32x4 *)p; }
+  DEVI void load_any(const T *p) {  // any element alignment
+    typedef u32x4 a2 __attribute__((aligned(2)));
+    w = *(const GLOBAL_AS a2 *)p;
+  }
   DEVI void store_global(T *p) const { *(GLOBAL_AS u32x4 *)p = w; }
   DEVI void zero() { w = u32x4{0, 0, 0, 0}; }
   DEVI void pack(const float (&v)[8]) {
@@ -126,6 +130,12 @@ template <> struct Pack8<float> {
   }
   DEVI void load_global(const float *p) {
     const f32x4 a = *(const GLOBAL_AS f32x4 *)p, b = *(const GLOBAL_AS f32x4 *)(p + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+    v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+  DEVI void load_any(const float *p) {
+    typedef f32x4 a4 __attribute__((aligned(4)));
+    const f32x4 a = *(const GLOBAL_AS a4 *)p, b = *(const GLOBAL_AS a4 *)(p + 4);
     v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
     v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
   }
@@ -194,20 +204,98 @@ template <typename T, bool VEC> DEVI void st8_guard_global(T *p, int nvalid, con
 // a destination that is not wanted) writes to `spare`, 32 bytes of its own that nobody reads.  A branch around a
 // store makes the compiler's count of the memory operations in flight inexact after it, and the next wait for an
 // older load then waits for the stores as well.
-template <typename T, bool VEC>
+// MODE (see Mamba-1's row modes): 0 = element by element, 1 = 16-byte pieces of aligned rows, 2 = 16-byte pieces at any
+// alignment (the caller stores what a ragged row's last piece holds by st8_tail).
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+template <typename T, int MODE>
 DEVI void st8_or_spare_global(T *p, int nvalid, bool wanted, T *spare, const float (&v)[8]) {
-  if constexpr (VEC) {
+  if constexpr (MODE != 0) {
     T *dst = (wanted && nvalid >= 8) ? p : spare;
     if constexpr (DT<T>::id == MAMBA_F32) {
-      *(GLOBAL_AS f32x4 *)dst = f32x4{v[0], v[1], v[2], v[3]};
-      *(GLOBAL_AS f32x4 *)(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
+      *(GLOBAL_AS f32x4_a4 *)dst = f32x4{v[0], v[1], v[2], v[3]};
+      *(GLOBAL_AS f32x4_a4 *)(dst + 4) = f32x4{v[4], v[5], v[6], v[7]};
     } else {
       Pack8<T> k;
       k.pack(v);
-      *(GLOBAL_AS u32x4 *)dst = k.w;
+      *(GLOBAL_AS u32x4_a2 *)dst = k.w;
     }
   } else {
     if (wanted) st8_guard<T, false>(p, nvalid, v);
+  }
+}
+
+// 8 consecutive elements at any element address: gfx950 serves 16-byte global accesses at element alignment, so rows
+// that start off a 16-byte boundary (odd sequence lengths, slices) need no element-wise path.
+template <typename T> DEVI void ld8_any(const T *p, float (&o)[8]) {
+  if constexpr (DT<T>::id == MAMBA_F32) {
+    const f32x4 a = *(const GLOBAL_AS f32x4_a4 *)p, b = *(const GLOBAL_AS f32x4_a4 *)(p + 4);
+    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w;
+    o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
+  } else {
+    Pack8<T> k;
+    k.w = *(const GLOBAL_AS u32x4_a2 *)p;
+    k.unpack(o);
+  }
+}
+
+template <typename T> DEVI void st8_any(T *p, const float (&v)[8]) {
+  if constexpr (DT<T>::id == MAMBA_F32) {
+    *(GLOBAL_AS f32x4_a4 *)p = f32x4{v[0], v[1], v[2], v[3]};
+    *(GLOBAL_AS f32x4_a4 *)(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
+  } else {
+    Pack8<T> k;
+    k.pack(v);
+    *(GLOBAL_AS u32x4_a2 *)p = k.w;
+  }
+}
+
+// Elements l .. l + 7 of a row of L >= 8 as floats, whatever the row's alignment and L: a 16-byte load from a position
+// that keeps inside the row (row8_raw), moved into place where it had to be shifted back (row8_place); positions
+// outside [0, L) read as 0.
+template <typename T> DEVI void row8_raw(const T *row, int l, int L, float (&o)[8]) {
+  ld8_any<T>(row + min(max(l, 0), L - 8), o);
+}
+DEVI void row8_place(int l, int L, float (&o)[8]) {
+  const int shift = l - min(max(l, 0), L - 8);  // 0 inside the row, 1 .. 7 in its last piece
+  if (shift != 0) {
+#pragma unroll
+    for (int bit = 4; bit >= 1; bit >>= 1) {
+      const bool on = shift & bit;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float up = i + bit < 8 ? o[i + bit] : 0.f;
+        o[i] = on ? up : o[i];
+      }
+    }
+    if (shift < 0 || shift >= 8) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = 0.f;
+    }
+  }
+}
+
+// Parameters (filters, norm weights) are read in the dtype the caller keeps them in; the switch is the same in
+// every lane and outside every loop.
+DEVI float ld_param(const void *base, int dtype, int64_t i) {
+  switch (dtype) {
+    case MAMBA_BF16: return ld1<bf16_t>(static_cast<const bf16_t *>(base) + i);
+    case MAMBA_F16: return ld1<f16_t>(static_cast<const f16_t *>(base) + i);
+    default: return static_cast<const float *>(base)[i];
+  }
+}
+DEVI void ld8_param(const void *base, int dtype, int64_t i, float (&o)[8]) {
+  switch (dtype) {
+    case MAMBA_BF16: ld8_any<bf16_t>(static_cast<const bf16_t *>(base) + i, o); break;
+    case MAMBA_F16: ld8_any<f16_t>(static_cast<const f16_t *>(base) + i, o); break;
+    default: ld8_any<float>(static_cast<const float *>(base) + i, o); break;
+  }
+}
+DEVI void st_param(void *base, int dtype, int64_t i, float v) {
+  switch (dtype) {
+    case MAMBA_BF16: st1<bf16_t>(static_cast<bf16_t *>(base) + i, v); break;
+    case MAMBA_F16: st1<f16_t>(static_cast<f16_t *>(base) + i, v); break;
+    default: static_cast<float *>(base)[i] = v; break;
   }
 }
 

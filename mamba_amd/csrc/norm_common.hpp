@@ -90,33 +90,106 @@ DEVI void store_row(T *row, int col, int gs, const float (&v)[K][8]) {
   }
 }
 
-// dweight[c] = sum over parts of dw_part[part][c] (and the same for dbias): 64 channels x 16 slices
-// of the parts per workgroup.
-__global__ __launch_bounds__(1024) void norm_reduce_kernel(const float *dw_part, const float *db_part, float *dw,
-                                                           float *db, int nparts, int dim) {
-  __shared__ float s[2][16][64];
-  const int cl = threadIdx.x & 63, sl = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + cl;
-  float a = 0.f, b = 0.f;
-  if (c < dim)
-    for (int q = sl; q < nparts; q += 16) {
-      a += dw_part[(int64_t)q * dim + c];
-      if (db_part) b += db_part[(int64_t)q * dim + c];
+// The norm's parameters of this thread's channels, zero past the end
+template <int K, int TEAM>
+DEVI void load_params(const void *base, int dtype, int64_t off, int col, int gs, float (&v)[K][8]) {
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int c = col + k * TEAM * 8;
+    if (c + 8 <= gs) {
+      ld8_param(base, dtype, off + c, v[k]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[k][e] = c + e < gs ? ld_param(base, dtype, off + c + e) : 0.f;
     }
-  s[0][sl][cl] = a;
-  s[1][sl][cl] = b;
-  __syncthreads();
-  if (sl == 0 && c < dim) {
+  }
+}
+
+// Sums over a workgroup of blockDim.x threads (whole waves), whatever their number: DPP adds inside a wave, the waves'
+// totals through LDS in alternating slots (one barrier per sum).
+struct WideSum {
+  float *red;  // LDS: 2 slots x 16 waves x 2 floats
+  int slot = 0, nw;
+  DEVI explicit WideSum(float *lds) : red(lds), nw(blockDim.x >> 6) {}
+  DEVI void sum2(float &a, float &b) {
+    a = wave_sum_to_last(a);
+    b = wave_sum_to_last(b);
+    if (nw == 1) {
+      a = readlane_f(a, 63);
+      b = readlane_f(b, 63);
+      return;
+    }
+    float *s = red + slot * 32;
+    if ((threadIdx.x & 63) == 63) *reinterpret_cast<f32x2 *>(s + (threadIdx.x >> 6) * 2) = f32x2{a, b};
+    lds_barrier();
     a = 0.f;
     b = 0.f;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      a += s[0][q][cl];
-      b += s[1][q][cl];
+    for (int w = 0; w < nw; ++w) {
+      const f32x2 v = *reinterpret_cast<const f32x2 *>(s + w * 2);
+      a += v.x;
+      b += v.y;
     }
-    dw[c] = a;
-    if (db) db[c] = b;
+    slot ^= 1;
   }
+};
+
+// threads of a workgroup that holds `channels` channels (a multiple of 8, at most 8192), 8 per thread
+inline int wide_threads(int channels) { return (channels / 8 + 63) / 64 * 64; }
+// workgroups of that many threads which a CU holds at once at `waves_per_simd` waves per SIMD
+inline int wide_resident(int threads, int waves_per_simd) { return max(1, waves_per_simd * 4 / (threads / 64)); }
+
+// Column sums of up to four (nparts, dim) workspaces, in the order of the parts, written in the parameters' dtype:
+// blockIdx.y is the workspace, a workgroup takes 16 channels (64 bytes of every row) on 128 slices of the parts, four
+// of a thread's rows in flight.  (64 channels x 16 slices of 1024 threads took 25 us for 1024 parts of 2560 channels:
+// 40 workgroups, one row at a time per thread.)
+struct ReduceJobs {
+  const float *part[4];
+  void *out[4];
+};
+template <bool VEC> __global__ __launch_bounds__(512) void norm_reduce_kernel(const ReduceJobs jobs, int dtype, int nparts, int dim) {
+  constexpr int SLICES = 128;
+  __shared__ f32x4 s[SLICES][4];
+  const float *src = jobs.part[blockIdx.y];
+  const int q = threadIdx.x & 3, sl = threadIdx.x >> 2;
+  const int c = blockIdx.x * 16 + q * 4;
+  auto row4 = [&](int part) -> f32x4 {
+    const float *r = src + (int64_t)part * dim + c;
+    if constexpr (VEC) {
+      return c < dim ? *(const GLOBAL_AS f32x4 *)r : f32x4{0.f, 0.f, 0.f, 0.f};
+    } else {
+      f32x4 v = {0.f, 0.f, 0.f, 0.f};
+      if (c < dim) v.x = r[0];
+      if (c + 1 < dim) v.y = r[1];
+      if (c + 2 < dim) v.z = r[2];
+      if (c + 3 < dim) v.w = r[3];
+      return v;
+    }
+  };
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  int part = sl;
+  for (; part + 3 * SLICES < nparts; part += 4 * SLICES) {
+    const f32x4 v0 = row4(part), v1 = row4(part + SLICES), v2 = row4(part + 2 * SLICES), v3 = row4(part + 3 * SLICES);
+    acc += (v0 + v1) + (v2 + v3);
+  }
+  for (; part < nparts; part += SLICES) acc += row4(part);
+  s[sl][q] = acc;
+  __syncthreads();
+#pragma unroll
+  for (int half = SLICES / 2; half >= 1; half >>= 1) {
+    if (sl < half) s[sl][q] += s[sl + half][q];
+    __syncthreads();
+  }
+  if (threadIdx.x < 16 && blockIdx.x * 16 + threadIdx.x < dim)
+    st_param(jobs.out[blockIdx.y], dtype, blockIdx.x * 16 + threadIdx.x, reinterpret_cast<const float *>(&s[0][0])[threadIdx.x]);
+}
+
+inline int launch_reduce(const ReduceJobs &jobs, int njobs, int dtype, int nparts, int dim, hipStream_t st) {
+  bool vec = dim % 4 == 0;
+  for (int i = 0; i < njobs; ++i) vec = vec && (reinterpret_cast<uintptr_t>(jobs.part[i]) & 15) == 0;
+  const dim3 grid((dim + 15) / 16, njobs), block(512);
+  if (vec) norm_reduce_kernel<true><<<grid, block, 0, st>>>(jobs, dtype, nparts, dim);
+  else norm_reduce_kernel<false><<<grid, block, 0, st>>>(jobs, dtype, nparts, dim);
+  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
 }
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }

@@ -46,8 +46,8 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_fwd_kernel(const
   const int gs = p.group_size, ngroups = p.dim / gs;
   const int64_t g0 = (int64_t)it.group * gs;
   float w[K][8], b[K][8];
-  load_row<float, VEC, K, TEAM>(p.weight + g0, it.col, gs, w);
-  if (p.bias) load_row<float, VEC, K, TEAM>(p.bias + g0, it.col, gs, b);
+  load_params<K, TEAM>(p.weight, p.weight_dtype, g0, it.col, gs, w);
+  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, g0, it.col, gs, b);
   const T *xp = static_cast<const T *>(p.x) + g0;
   const T *zp = p.z ? static_cast<const T *>(p.z) + g0 : nullptr;
   T *op = static_cast<T *>(p.out) + g0;
@@ -124,8 +124,8 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_bwd_kernel(const
   const int gs = p.group_size, ngroups = p.dim / gs;
   const int64_t g0 = (int64_t)it.group * gs;
   float w[K][8], b[K][8], dw[K][8], db[K][8];
-  load_row<float, VEC, K, TEAM>(p.weight + g0, it.col, gs, w);
-  if (p.bias) load_row<float, VEC, K, TEAM>(p.bias + g0, it.col, gs, b);
+  load_params<K, TEAM>(p.weight, p.weight_dtype, g0, it.col, gs, w);
+  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, g0, it.col, gs, b);
 #pragma unroll
   for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -220,29 +220,21 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_bwd_kernel(const
 
 // The forward pass in the same form as norm_bwd_wide_kernel (below): a part of the rows per workgroup, the next
 // row requested before the current one is used, no branch around a row's loads or stores.
-template <typename T, int TEAM, bool HAS_Z>
-__global__ __launch_bounds__(TEAM, 8) void norm_fwd_wide_kernel(const NormGatedParams p, int nparts) {
-  __shared__ float lds[2 * (TEAM / 64) * 2];
-  TeamSum<TEAM> ts(lds);
+template <typename T, bool HAS_Z>
+__global__ __launch_bounds__(1024, 8) void norm_fwd_wide_kernel(const NormGatedParams p, int nparts) {
+  __shared__ __align__(16) float lds[64];
+  WideSum ts(lds);
   const int gs = p.group_size, ngroups = p.dim / gs, rows = p.rows;
   const int group = blockIdx.x % ngroups, part = blockIdx.x / ngroups;
-  const int col = threadIdx.x * 8;
-  if (__builtin_amdgcn_readfirstlane(col) >= gs) {
-    for (int r = part; r < rows; r += nparts) {
-      float a = 0.f, b = 0.f;
-      if (!p.is_rms) ts.sum2(a, b);
-      a = b = 0.f;  // sum2 hands back the team's totals
-      ts.sum2(a, b);
-    }
-    return;
-  }
+  const bool real = (int)threadIdx.x * 8 < gs;
+  const int col = min((int)threadIdx.x * 8, gs - 8);
   if (part >= rows) return;
   const int64_t c0 = (int64_t)group * gs + col;
   float w[8], b[8];
-  ld8<float>(p.weight + c0, w);
+  ld8_param(p.weight, p.weight_dtype, c0, w);
 #pragma unroll
   for (int e = 0; e < 8; ++e) b[e] = 0.f;
-  if (p.bias) ld8<float>(p.bias + c0, b);
+  if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
   const T *xp = static_cast<const T *>(p.x) + c0;
   const T *zp = HAS_Z ? static_cast<const T *>(p.z) + c0 : xp;
   T *op = static_cast<T *>(p.out) + c0;
@@ -272,6 +264,7 @@ __global__ __launch_bounds__(TEAM, 8) void norm_fwd_wide_kernel(const NormGatedP
     if (!p.is_rms) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) mean += x[e];
+      mean = real ? mean : 0.f;
       ts.sum2(mean, dummy);
       mean *= inv_n;
     }
@@ -281,6 +274,7 @@ __global__ __launch_bounds__(TEAM, 8) void norm_fwd_wide_kernel(const NormGatedP
       x[e] -= mean;
       var = __builtin_fmaf(x[e], x[e], var);
     }
+    var = real ? var : 0.f;
     dummy = 0.f;
     ts.sum2(var, dummy);
     const float rstd = 1.f / sqrtf(var * inv_n + p.eps);
@@ -302,33 +296,27 @@ __global__ __launch_bounds__(TEAM, 8) void norm_fwd_wide_kernel(const NormGatedP
   }
 }
 
-// The backward pass for groups of 1024 < group_size <= 8192 channels in whole waves' worth (multiples of 512), rows
-// of 16-byte pieces: a workgroup of 256 / 512 / 1024 threads per (part, group), one piece per thread, so that a
-// wave holds either 512 channels or none (5120 channels on 1024 threads: 10 waves of 16 work, 6 only take part in the
-// team's sums, in a loop of their own).  No branch surrounds a load or a store of the loop over the rows: the row
-// after next's operands are requested (the last row again at the end) before the current row's are used, and the
-// waits the compiler places then name exactly the loads they need.  With the guarded accesses of norm_bwd_kernel
-// every wait was for everything in flight, the row just requested included, and a row cost its whole latency.
-template <typename T, int TEAM, bool HAS_Z>
-__global__ __launch_bounds__(TEAM) void norm_bwd_wide_kernel(const NormGatedParams p) {
-  __shared__ float lds[2 * (TEAM / 64) * 2];
-  TeamSum<TEAM> ts(lds);
+// The backward pass for groups of 1024 < group_size <= 8192 channels (a multiple of 8), rows of 16-byte pieces: a
+// workgroup of just as many waves as the group needs per (part, group), 8 channels per thread (threads past the end of
+// the group stand on its last 8 channels: they load, compute and store what that thread does and add nothing to the
+// sums).  No branch surrounds a load or a store of the loop over the rows: the next row's operands are requested (the
+// last row again at the end) before the current row's are used, and the waits the compiler places then name exactly the
+// loads they need.  With the guarded accesses of norm_bwd_kernel every wait was for everything in flight, the row just
+// requested included, and a row cost its whole latency.
+template <typename T, bool HAS_Z>
+__global__ __launch_bounds__(1024) void norm_bwd_wide_kernel(const NormGatedParams p) {
+  __shared__ __align__(16) float lds[64];
+  WideSum ts(lds);
   const int gs = p.group_size, ngroups = p.dim / gs, nparts = p.nparts, rows = p.rows;
   const int group = blockIdx.x % ngroups, part = blockIdx.x / ngroups;
-  const int col = threadIdx.x * 8;
-  if (__builtin_amdgcn_readfirstlane(col) >= gs) {
-    for (int r = part; r < rows; r += nparts) {
-      float a = 0.f, b = 0.f;
-      ts.sum2(a, b);
-    }
-    return;
-  }
+  const bool real = (int)threadIdx.x * 8 < gs;
+  const int col = min((int)threadIdx.x * 8, gs - 8);
   const int64_t c0 = (int64_t)group * gs + col;
   float w[8], b[8], dw[8], db[8];
-  ld8<float>(p.weight + c0, w);
+  ld8_param(p.weight, p.weight_dtype, c0, w);
 #pragma unroll
   for (int e = 0; e < 8; ++e) b[e] = dw[e] = db[e] = 0.f;
-  if (p.bias) ld8<float>(p.bias + c0, b);
+  if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
   const T *xp = static_cast<const T *>(p.x) + c0;
   const T *gp = static_cast<const T *>(p.dy) + c0;
   const T *zp = HAS_Z ? static_cast<const T *>(p.z) + c0 : xp;
@@ -381,6 +369,8 @@ __global__ __launch_bounds__(TEAM) void norm_bwd_wide_kernel(const NormGatedPara
         x[e] = xhat;
         g[e] = wdy;
       }
+      c1 = real ? c1 : 0.f;
+      c2 = real ? c2 : 0.f;
       ts.sum2(c1, c2);
       c1 *= inv_n;
       c2 = p.is_rms ? 0.f : c2 * inv_n;
@@ -423,8 +413,7 @@ __global__ __launch_bounds__(TEAM) void norm_bwd_wide_kernel(const NormGatedPara
 template <typename T> bool vec_ok(const NormGatedParams &p, bool bwd) {
   constexpr int per16 = 16 / (int)sizeof(T);  // elements per 16 bytes: loads of 8 need 8-element alignment of fp32 too
   (void)per16;
-  bool ok = p.group_size % 8 == 0 && p.x_rs % 8 == 0 && p.out_rs % 8 == 0 && aligned16(p.x) && aligned16(p.weight) &&
-            (!p.bias || aligned16(p.bias));
+  bool ok = p.group_size % 8 == 0 && p.x_rs % 8 == 0 && p.out_rs % 8 == 0 && aligned16(p.x);
   if (!bwd) ok = ok && aligned16(p.out);
   if (p.z) ok = ok && p.z_rs % 8 == 0 && aligned16(p.z);
   if (bwd) {
@@ -471,30 +460,28 @@ template <typename T, bool VEC> int pick_team(const NormGatedParams &p, bool bwd
   return pick_k<T, 1024, VEC>(p, bwd, st);
 }
 
-template <typename T, int TEAM> int launch_wide(const NormGatedParams &p, bool bwd, hipStream_t st) {
-  // forward: as many parts as workgroups the chip holds at once (2048 threads per CU), never more than rows
-  const int ngroups = p.dim / p.group_size;
-  const int nparts = bwd ? p.nparts : max(1, min(p.rows, cu_count() * (2048 / TEAM) / ngroups));
+bool wide_group(int gs) { return gs > 1024 && gs <= 8192 && gs % 8 == 0; }
+
+template <typename T> int launch_wide(const NormGatedParams &p, bool bwd, hipStream_t st) {
+  // forward: as many parts as workgroups the chip holds at once, never more than rows
+  const int ngroups = p.dim / p.group_size, threads = wide_threads(p.group_size);
+  const int nparts = bwd ? p.nparts : max(1, min(p.rows, cu_count() * wide_resident(threads, 8) / ngroups));
   const int64_t wgs = (int64_t)ngroups * nparts;
   if (wgs > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
-  const dim3 grid((unsigned)wgs), block(TEAM);
+  const dim3 grid((unsigned)wgs), block(threads);
   if (bwd) {
-    if (p.z) norm_bwd_wide_kernel<T, TEAM, true><<<grid, block, 0, st>>>(p);
-    else norm_bwd_wide_kernel<T, TEAM, false><<<grid, block, 0, st>>>(p);
+    if (p.z) norm_bwd_wide_kernel<T, true><<<grid, block, 0, st>>>(p);
+    else norm_bwd_wide_kernel<T, false><<<grid, block, 0, st>>>(p);
   } else {
-    if (p.z) norm_fwd_wide_kernel<T, TEAM, true><<<grid, block, 0, st>>>(p, nparts);
-    else norm_fwd_wide_kernel<T, TEAM, false><<<grid, block, 0, st>>>(p, nparts);
+    if (p.z) norm_fwd_wide_kernel<T, true><<<grid, block, 0, st>>>(p, nparts);
+    else norm_fwd_wide_kernel<T, false><<<grid, block, 0, st>>>(p, nparts);
   }
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
 }
 
 template <typename T> int run(const NormGatedParams &p, bool bwd, hipStream_t st) {
   const bool vec = vec_ok<T>(p, bwd);
-  if (vec && p.rows > 0 && p.group_size > 1024 && p.group_size <= 8192 && p.group_size % 512 == 0) {
-    if (p.group_size <= 2048) return launch_wide<T, 256>(p, bwd, st);
-    if (p.group_size <= 4096) return launch_wide<T, 512>(p, bwd, st);
-    return launch_wide<T, 1024>(p, bwd, st);
-  }
+  if (vec && p.rows > 0 && wide_group(p.group_size)) return launch_wide<T>(p, bwd, st);
   return vec ? pick_team<T, true>(p, bwd, st) : pick_team<T, false>(p, bwd, st);
 }
 
@@ -502,6 +489,7 @@ int check(const NormGatedParams *p, bool bwd) {
   if (!p) return MAMBA_E_BADARG;
   if (p->rows < 0 || p->dim <= 0 || p->group_size <= 0 || p->dim % p->group_size != 0) return MAMBA_E_BADARG;
   if (p->group_size > 32768) return MAMBA_E_UNSUPPORTED;
+  if (p->weight_dtype < MAMBA_F32 || p->weight_dtype > MAMBA_F16) return MAMBA_E_BADARG;
   if (!p->x || !p->weight || !p->rstd) return MAMBA_E_BADARG;
   if (!p->is_rms && !p->mean) return MAMBA_E_BADARG;
   if (!bwd && !p->out) return MAMBA_E_BADARG;
@@ -529,10 +517,10 @@ int dispatch(const NormGatedParams *p, bool bwd, hipStream_t st) {
     }
   }
   if (rc != MAMBA_OK || !bwd) return rc;
-  norm_reduce_kernel<<<dim3((p->dim + 63) / 64), dim3(1024), 0, st>>>(p->dw_part, p->bias ? p->db_part : nullptr,
-                                                                       p->dweight, p->bias ? p->dbias : nullptr,
-                                                                       p->nparts, p->dim);
-  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
+  ReduceJobs jobs{};
+  jobs.part[0] = p->dw_part, jobs.out[0] = p->dweight;
+  if (p->bias) jobs.part[1] = p->db_part, jobs.out[1] = p->dbias;
+  return launch_reduce(jobs, p->bias ? 2 : 1, p->weight_dtype, p->nparts, p->dim, st);
 }
 
 }  // namespace
@@ -542,4 +530,19 @@ extern "C" int norm_gated_fwd(const NormGatedParams *p, mamba_stream_t stream) {
 }
 extern "C" int norm_gated_bwd(const NormGatedParams *p, mamba_stream_t stream) {
   return dispatch(p, true, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int norm_gated_bwd_nparts(const NormGatedParams *p) {
+  if (!p || p->rows <= 0 || p->dim <= 0 || p->group_size <= 0 || p->dim % p->group_size != 0) return MAMBA_E_BADARG;
+  const int ngroups = p->dim / p->group_size, gs = p->group_size;
+  int parts;
+  if (wide_group(gs)) {
+    parts = cu_count() * wide_resident(wide_threads(gs), 4) / ngroups;
+  } else {
+    int team = 8;
+    while (team < 64 && gs > 16 * team) team *= 2;
+    if (gs > 1024) team = gs <= 4096 ? 256 : 1024;
+    parts = 2048 * 64 / team / ngroups;
+  }
+  return max(1, min(min(p->rows, parts), 65536));
 }

@@ -55,8 +55,8 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_fwd_kernel(c
   if (!my_part<TEAM>(nparts, part, col)) return;
   const int n = p.dim;
   float w[K][8], b[K][8];
-  load_row<float, VEC, K, TEAM>(p.weight, col, n, w);
-  if (p.bias) load_row<float, VEC, K, TEAM>(p.bias, col, n, b);
+  load_params<K, TEAM>(p.weight, p.weight_dtype, 0, col, n, w);
+  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, 0, col, n, b);
   const T *xp = static_cast<const T *>(p.x);
   const R *rp = static_cast<const R *>(p.residual);
   T *op = static_cast<T *>(p.out);
@@ -132,8 +132,8 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_fwd_kernel(c
     if constexpr (EXTRA) {
       if (p.weight1) {  // the second set of norm parameters on the same normalised row
         float w1[K][8], b1[K][8], y1[K][8];
-        load_row<float, VEC, K, TEAM>(p.weight1, col, n, w1);
-        if (p.bias1) load_row<float, VEC, K, TEAM>(p.bias1, col, n, b1);
+        load_params<K, TEAM>(p.weight1, p.weight_dtype, 0, col, n, w1);
+        if (p.bias1) load_params<K, TEAM>(p.bias1, p.weight_dtype, 0, col, n, b1);
 #pragma unroll
         for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_bwd_kernel(c
   if (!my_part<TEAM>(nparts, part, col)) return;
   const int n = p.dim;
   float w[K][8], dw[K][8], db[K][8];
-  load_row<float, VEC, K, TEAM>(p.weight, col, n, w);
+  load_params<K, TEAM>(p.weight, p.weight_dtype, 0, col, n, w);
 #pragma unroll
   for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_bwd_kernel(c
     for (int k = 0; k < K; ++k)
 #pragma unroll
       for (int e = 0; e < 8; ++e) w1[k][e] = dw1[k][e] = db1[k][e] = 0.f;
-    if (two) load_row<float, VEC, K, TEAM>(p.weight1, col, n, w1);
+    if (two) load_params<K, TEAM>(p.weight1, p.weight_dtype, 0, col, n, w1);
   }
   const bool drop = EXTRA && p.dropout_p > 0.f;
   const float keep_scale = drop ? 1.f / (1.f - p.dropout_p) : 1.f;
@@ -284,14 +284,16 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_bwd_kernel(c
   }
 }
 
+bool is_extra(const NormResidualParams &p) { return p.x1 || p.rowscale || p.weight1 || p.dropout_p > 0.f; }
+
 bool vec_ok(const NormResidualParams &p, bool bwd) {
   auto ok = [](const void *q, int64_t rs) { return !q || (aligned16(q) && rs % 8 == 0); };
-  bool v = p.dim % 8 == 0 && aligned16(p.weight) && aligned16(p.bias) && ok(p.x, p.x_rs);
+  bool v = p.dim % 8 == 0 && ok(p.x, p.x_rs);
   if (!bwd) v = v && ok(p.residual, p.residual_rs) && ok(p.out, p.out_rs) && ok(p.residual_out, p.residual_out_rs);
   else
     v = v && ok(p.dy, p.dy_rs) && ok(p.dresidual, p.dresidual_rs) && ok(p.dx, p.dx_rs) &&
         ok(p.dresidual_in, p.dresidual_in_rs) && aligned16(p.dw_part) && aligned16(p.db_part);
-  v = v && aligned16(p.weight1) && aligned16(p.bias1) && ok(p.x1, p.x1_rs) && ok(p.out1, p.out1_rs) &&
+  v = v && ok(p.x1, p.x1_rs) && ok(p.out1, p.out1_rs) &&
       ok(p.dy1, p.dy1_rs) && ok(p.dx1, p.dx1_rs) && aligned16(p.dw1_part) && aligned16(p.db1_part);
   return v;
 }
@@ -300,8 +302,7 @@ template <typename T, typename R, int TEAM, int K, bool VEC> int launch(const No
   constexpr int WGT = TEAM < 256 ? 256 : TEAM;
   const int nparts = bwd ? p.nparts : min(p.rows, 16384);
   const int wgs = (nparts + WGT / TEAM - 1) / (WGT / TEAM);
-  const bool extra = p.x1 || p.rowscale || p.weight1 || p.dropout_p > 0.f;
-  if (extra) {
+  if (is_extra(p)) {
     if (bwd) norm_res_bwd_kernel<T, R, TEAM, K, VEC, true><<<dim3(wgs), dim3(WGT), 0, st>>>(p);
     else norm_res_fwd_kernel<T, R, TEAM, K, VEC, true><<<dim3(wgs), dim3(WGT), 0, st>>>(p, nparts);
   } else {
@@ -340,6 +341,7 @@ int dispatch(const NormResidualParams *p, bool bwd, hipStream_t st) {
   if (!p || !p->x || !p->weight || !p->rstd) return MAMBA_E_BADARG;
   if (p->rows <= 0 || p->dim <= 0) return MAMBA_E_BADARG;
   if (p->dim > 32768) return MAMBA_E_UNSUPPORTED;
+  if (p->weight_dtype < MAMBA_F32 || p->weight_dtype > MAMBA_F16) return MAMBA_E_BADARG;
   if (!p->is_rms && !p->mean) return MAMBA_E_BADARG;
   if (!bwd && !p->out) return MAMBA_E_BADARG;
   if (bwd) {
@@ -366,14 +368,16 @@ int dispatch(const NormResidualParams *p, bool bwd, hipStream_t st) {
     default: return MAMBA_E_BADARG;
   }
   if (rc != MAMBA_OK || !bwd) return rc;
-  norm_reduce_kernel<<<dim3((p->dim + 63) / 64), dim3(1024), 0, st>>>(p->dw_part, p->bias ? p->db_part : nullptr,
-                                                                       p->dweight, p->bias ? p->dbias : nullptr,
-                                                                       p->nparts, p->dim);
-  if (p->weight1)
-    norm_reduce_kernel<<<dim3((p->dim + 63) / 64), dim3(1024), 0, st>>>(p->dw1_part, p->bias1 ? p->db1_part : nullptr,
-                                                                         p->dweight1, p->bias1 ? p->dbias1 : nullptr,
-                                                                         p->nparts, p->dim);
-  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
+  ReduceJobs jobs{};
+  int n = 0;
+  auto add = [&](const float *part, void *out) {
+    if (out) jobs.part[n] = part, jobs.out[n++] = out;
+  };
+  add(p->dw_part, p->dweight);
+  if (p->bias) add(p->db_part, p->dbias);
+  if (p->weight1) add(p->dw1_part, p->dweight1);
+  if (p->weight1 && p->bias1) add(p->db1_part, p->dbias1);
+  return launch_reduce(jobs, n, p->weight_dtype, p->nparts, p->dim, st);
 }
 
 }  // namespace
@@ -383,4 +387,12 @@ extern "C" int norm_residual_fwd(const NormResidualParams *p, mamba_stream_t str
 }
 extern "C" int norm_residual_bwd(const NormResidualParams *p, mamba_stream_t stream) {
   return dispatch(p, true, static_cast<hipStream_t>(stream));
+}
+
+// Rows are dealt to as many workgroups (teams) as the chip holds at once; every part is one row of the workspace that
+// the reduction reads again.
+extern "C" int norm_residual_bwd_nparts(const NormResidualParams *p) {
+  if (!p || p->rows <= 0 || p->dim <= 0) return MAMBA_E_BADARG;
+  const int team = p->dim <= 1024 ? 64 : p->dim <= 4096 ? 256 : p->dim <= 8192 ? 512 : 1024;
+  return max(1, min(p->rows, 4096 * 64 / team));
 }

@@ -78,6 +78,14 @@ def _rows(t, what):
     return t
 
 
+def _params(*tensors):
+    """The norm's parameters as the kernels read them: contiguous, all in one dtype of fp32, bf16 and fp16."""
+    kinds = {t.dtype for t in tensors if t is not None}
+    one = len(kinds) == 1 and next(iter(kinds)) in _lib.DTYPE_CODE
+    conv = lambda t: None if t is None else (t if one else t.float()).contiguous()
+    return [conv(t) for t in tensors]
+
+
 def _layer_norm_fwd(x, weight, bias, eps, residual=None, x1=None, weight1=None, bias1=None, dropout_p=0.0,
                     rowscale=None, residual_dtype=None, is_rms_norm=False, return_dropout_mask=False):
     """x, residual, x1: (rows, dim).  Returns (y, y1, mean, rstd, residual_out, seeds, dropout_mask, dropout_mask1)
@@ -125,9 +133,10 @@ def _layer_norm_fwd(x, weight, bias, eps, residual=None, x1=None, weight1=None, 
             dropout_mask = torch.empty(M, N, dtype=torch.bool, device=x.device)
             dropout_mask1 = torch.empty(M, N, dtype=torch.bool, device=x.device) if x1 is not None else None
     if M > 0:
-        f32 = lambda t: t.float().contiguous() if t is not None else None
-        w32, b32, w132, b132, rs32 = f32(weight), f32(bias), f32(weight1), f32(bias1), f32(rowscale)
+        w32, b32, w132, b132 = _params(weight, bias, weight1, bias1)
+        rs32 = rowscale.float().contiguous() if rowscale is not None else None
         p = _lib.NormResidualParams()
+        p.weight_dtype = _lib.DTYPE_CODE[w32.dtype]
         p.rows, p.dim, p.dtype, p.res_dtype = M, N, _lib.DTYPE_CODE[x.dtype], _lib.DTYPE_CODE[res_dtype]
         p.is_rms, p.eps = int(is_rms_norm), eps
         p.x, p.residual, p.weight, p.bias = x.data_ptr(), _lib.ptr(residual), w32.data_ptr(), _lib.ptr(b32)
@@ -174,28 +183,18 @@ def _layer_norm_bwd(dy, x, weight, bias, eps, mean, rstd, dresidual=None, dy1=No
         z = lambda t: torch.zeros_like(t) if t is not None else None
         return (dx, z(weight), z(bias), dresidual_in if dresidual_in is not None else (dx if has_residual else None),
                 dx1, z(weight1), z(bias1))
-    team = 64 if N <= 1024 else 256 if N <= 4096 else 512 if N <= 8192 else 1024
-    nparts = max(1, min(M, 4096 * 64 // team))
-    nb = (2 if bias is not None else 1) + (0 if weight1 is None else 2 if bias1 is not None else 1)
-    parts = torch.empty(nb, nparts, N, dtype=torch.float32, device=x.device)
-    sums = torch.empty(nb, N, dtype=torch.float32, device=x.device)
-    f32 = lambda t: t.float().contiguous() if t is not None else None
-    w32, b32, w132, b132, rs32 = f32(weight), f32(bias), f32(weight1), f32(bias1), f32(rowscale)
+    w32, b32, w132, b132 = _params(weight, bias, weight1, bias1)
+    rs32 = rowscale.float().contiguous() if rowscale is not None else None
     p = _lib.NormResidualParams()
+    p.weight_dtype = _lib.DTYPE_CODE[w32.dtype]
     p.rows, p.dim, p.dtype, p.res_dtype = M, N, _lib.DTYPE_CODE[x_dtype], _lib.DTYPE_CODE[x.dtype]
-    p.is_rms, p.eps, p.nparts = int(is_rms_norm), eps, nparts
+    p.is_rms, p.eps = int(is_rms_norm), eps
     p.x, p.weight, p.bias, p.mean, p.rstd = x.data_ptr(), w32.data_ptr(), _lib.ptr(b32), _lib.ptr(mean), rstd.data_ptr()
     p.x_rs = x.stride(0)
     p.dy, p.dy_rs, p.dx, p.dx_rs = dy.data_ptr(), dy.stride(0), dx.data_ptr(), dx.stride(0)
     p.dresidual, p.dresidual_rs = _lib.ptr(dresidual), dresidual.stride(0) if dresidual is not None else 0
     p.dresidual_in = _lib.ptr(dresidual_in)
     p.dresidual_in_rs = dresidual_in.stride(0) if dresidual_in is not None else 0
-    slot = 0
-    p.dweight, p.dw_part = sums[slot].data_ptr(), parts[slot].data_ptr()
-    slot += 1
-    if bias is not None:
-        p.dbias, p.db_part = sums[slot].data_ptr(), parts[slot].data_ptr()
-        ib, slot = slot, slot + 1
     p.rowscale, p.seeds, p.dropout_p = _lib.ptr(rs32), _lib.ptr(seeds), dropout_p
     if has_x1:
         p.x1, p.x1_rs = x.data_ptr(), x.stride(0)  # only says that there was a second input: it is not read
@@ -203,17 +202,20 @@ def _layer_norm_bwd(dy, x, weight, bias, eps, mean, rstd, dresidual=None, dy1=No
     if weight1 is not None:
         p.weight1, p.bias1 = w132.data_ptr(), _lib.ptr(b132)
         p.dy1, p.dy1_rs = dy1.data_ptr(), dy1.stride(0)
-        p.dweight1, p.dw1_part = sums[slot].data_ptr(), parts[slot].data_ptr()
-        iw1, slot = slot, slot + 1
-        if bias1 is not None:
-            p.dbias1, p.db1_part = sums[slot].data_ptr(), parts[slot].data_ptr()
-            ib1 = slot
     with torch.cuda.device(x.device):
-        _lib.check(_lib.load().norm_residual_bwd(p, _lib.current_stream(x.device)), "norm_residual_bwd")
-    dw = sums[0].to(weight.dtype)
-    db = sums[ib].to(bias.dtype) if bias is not None else None
-    dw1 = sums[iw1].to(weight1.dtype) if weight1 is not None else None
-    db1 = sums[ib1].to(bias1.dtype) if bias1 is not None else None
+        lib = _lib.load()
+        p.nparts = lib.norm_residual_bwd_nparts(p)
+        given = [(t, g, q) for t, g, q in ((weight, "dweight", "dw_part"), (bias, "dbias", "db_part"),
+                                           (weight1, "dweight1", "dw1_part"), (bias1, "dbias1", "db1_part")) if t is not None]
+        parts = torch.empty(len(given), p.nparts, N, dtype=torch.float32, device=x.device)
+        sums = torch.empty(len(given), N, dtype=w32.dtype, device=x.device)
+        grads = {}
+        for i, (t, g, q) in enumerate(given):
+            setattr(p, g, sums[i].data_ptr())
+            setattr(p, q, parts[i].data_ptr())
+            grads[g] = (sums[i], t.dtype)
+        _lib.check(lib.norm_residual_bwd(p, _lib.current_stream(x.device)), "norm_residual_bwd")
+    dw, db, dw1, db1 = (grads[g][0].to(grads[g][1]) if g in grads else None for g in ("dweight", "dbias", "dweight1", "dbias1"))
     if has_residual and dresidual_in is None:
         dresidual_in = dx
     return dx, dw, db, dresidual_in, dx1, dw1, db1
@@ -297,14 +299,21 @@ class LayerNormFn(torch.autograd.Function):
 
 def layer_norm_fn(x, weight, bias, residual=None, x1=None, weight1=None, bias1=None, eps=1e-6, dropout_p=0.0,
                   rowscale=None, prenorm=False, residual_in_fp32=False, is_rms_norm=False, return_dropout_mask=False):
+    if x1 is None and weight1 is None and bias1 is None and rowscale is None and dropout_p == 0.0 and not return_dropout_mask:
+        ext = _lib.torch_ext()
+        if ext is not None:
+            # the same node in C++ (csrc/torch_norm_conv.cpp); None = a case for the code below
+            r = ext.norm_residual(x, weight, bias, residual, eps, bool(prenorm), bool(residual_in_fp32), bool(is_rms_norm))
+            if r is not None:
+                return r
     return LayerNormFn.apply(x, weight, bias, residual, x1, weight1, bias1, eps, dropout_p, rowscale, prenorm,
                              residual_in_fp32, is_rms_norm, return_dropout_mask)
 
 
 def rms_norm_fn(x, weight, bias, residual=None, x1=None, weight1=None, bias1=None, eps=1e-6, dropout_p=0.0,
                 rowscale=None, prenorm=False, residual_in_fp32=False, return_dropout_mask=False):
-    return LayerNormFn.apply(x, weight, bias, residual, x1, weight1, bias1, eps, dropout_p, rowscale, prenorm,
-                             residual_in_fp32, True, return_dropout_mask)
+    return layer_norm_fn(x, weight, bias, residual, x1, weight1, bias1, eps, dropout_p, rowscale, prenorm, residual_in_fp32,
+                         True, return_dropout_mask)
 
 
 class RMSNorm(torch.nn.Module):

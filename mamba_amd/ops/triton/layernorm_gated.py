@@ -39,12 +39,19 @@ def _rows(t, what):
     return t
 
 
-def _common(p, x, weight32, bias32, z, eps, group_size, norm_before_gate, is_rms_norm):
+def _params(weight, bias):
+    """The norm's parameters as the kernels read them: contiguous, one dtype of fp32, bf16 and fp16."""
+    if weight.dtype not in _lib.DTYPE_CODE or (bias is not None and bias.dtype != weight.dtype):
+        weight, bias = weight.float(), bias.float() if bias is not None else None
+    return weight.contiguous(), bias.contiguous() if bias is not None else None
+
+
+def _common(p, x, weight, bias, z, eps, group_size, norm_before_gate, is_rms_norm):
     M, N = x.shape
     p.rows, p.dim, p.group_size = M, N, group_size
-    p.dtype = _lib.DTYPE_CODE[x.dtype]
+    p.dtype, p.weight_dtype = _lib.DTYPE_CODE[x.dtype], _lib.DTYPE_CODE[weight.dtype]
     p.is_rms, p.norm_before_gate, p.eps = int(is_rms_norm), int(norm_before_gate), eps
-    p.x, p.z, p.weight, p.bias = x.data_ptr(), _lib.ptr(z), weight32.data_ptr(), _lib.ptr(bias32)
+    p.x, p.z, p.weight, p.bias = x.data_ptr(), _lib.ptr(z), weight.data_ptr(), _lib.ptr(bias)
     p.x_rs = x.stride(0)
     p.z_rs = z.stride(0) if z is not None else 0
 
@@ -83,10 +90,9 @@ def _layer_norm_fwd(x, weight, bias, eps, z=None, out=None, group_size=None, nor
     rstd = torch.empty(M, ngroups, dtype=torch.float32, device=x.device)
     if M == 0:
         return out, mean, rstd
-    w32 = weight.float().contiguous()
-    b32 = bias.float().contiguous() if bias is not None else None
+    w, bv = _params(weight, bias)
     p = _lib.NormGatedParams()
-    _common(p, x, w32, b32, z, eps, group_size, norm_before_gate, is_rms_norm)
+    _common(p, x, w, bv, z, eps, group_size, norm_before_gate, is_rms_norm)
     p.out, p.out_rs, p.mean, p.rstd = out.data_ptr(), out.stride(0), _lib.ptr(mean), rstd.data_ptr()
     with torch.cuda.device(x.device):
         _lib.check(_lib.load().norm_gated_fwd(p, _lib.current_stream(x.device)), "norm_gated_fwd")
@@ -115,12 +121,11 @@ def _layer_norm_bwd(dy, x, weight, bias, eps, mean, rstd, z=None, group_size=Non
         dz = torch.empty(M, N, dtype=x.dtype, device=x.device)
     if M == 0:
         return dx, torch.zeros_like(weight), torch.zeros_like(bias) if bias is not None else None, dz
-    # enough teams of threads to fill the GPU several times over, never more parts than rows
-    # the threads per (row, group) norm_gated.hip picks
-    team = next((t for t in (8, 16, 32, 64, 256) if group_size <= 16 * t), 1024)
-    if group_size % 512 == 0 and 2048 < group_size <= 4096:
-        team = 512
-    nparts = max(1, min(M, (4096 * 64 // team) // ngroups, 65536))
+    w, bv = _params(weight, bias)
+    p = _lib.NormGatedParams()
+    _common(p, x, w, bv, z, eps, group_size, norm_before_gate, is_rms_norm)
+    with torch.cuda.device(x.device):
+        p.nparts = nparts = _lib.load().norm_gated_bwd_nparts(p)
     nb = 2 if bias is not None else 1
     parts = torch.empty(nb, nparts, N, dtype=torch.float32, device=x.device)
     sums = torch.empty(nb, N, dtype=torch.float32, device=x.device)

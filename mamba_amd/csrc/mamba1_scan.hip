@@ -34,13 +34,179 @@ int mamba1_bwd_k4_launch(const MambaScanParams &p, int pa, int pb, int nparts, h
 
 namespace {
 
+// ------------------------------------------------------------------ segments of the sequence
+// With few (batch, channel) rows the chip is filled by cutting the sequence into p.nseg segments (p.seg_ws).  A
+// segment's part of the recurrence is a (decay, value) pair per (channel, state), as a lane's and a tile's are: the
+// value is formed by scan_seg_fwd_kernel, the decay is exp(A * sum of the segment's steps), and the scan kernels compose
+// the pairs of the segments before theirs when they start.  The adjoint is handled the same way from the other end
+// (scan_seg_bwd_kernel).  seg_ws: values (batch, nseg, dim, N), then the sums of the steps (batch, nseg, dim), then the
+// first steps (batch, nseg, dim; backward only).
+DEVI int64_t seg_row(const MambaScanParams &p, int b, int seg, int d) { return ((int64_t)b * p.nseg + seg) * p.dim + d; }
+DEVI float *seg_sums(const MambaScanParams &p) { return p.seg_ws + (int64_t)p.batch * p.nseg * p.dim * p.dstate; }
+DEVI float *seg_firsts(const MambaScanParams &p) { return seg_sums(p) + (int64_t)p.batch * p.nseg * p.dim; }
+
+// State entering this workgroup's segment (A2 = A log2 e)
+DEVI float seg_state_in(const MambaScanParams &p, const Geo &q, int d, int n, float A2) {
+  float h = 0.f;
+  for (int s = 0; s < q.seg; ++s) {
+    const int64_t row = seg_row(p, q.b, s, d);
+    h = __builtin_fmaf(fast_exp2(A2 * seg_sums(p)[row]), h, p.seg_ws[row * p.dstate + n]);
+  }
+  return h;
+}
+// Adjoint at the first position of the segment after this workgroup's, and the decay of that position
+DEVI float seg_adjoint_in(const MambaScanParams &p, const Geo &q, int d, int n, float A2, float &decay) {
+  float g = 0.f;
+  decay = 0.f;
+  for (int s = q.nseg - 1; s > q.seg; --s) {
+    const int64_t row = seg_row(p, q.b, s, d);
+    const float first = seg_firsts(p)[row];
+    // from the first position of segment s + 1 back to that of segment s; `decay` is the former's
+    g = __builtin_fmaf(fast_exp2(A2 * (seg_sums(p)[row] - first)) * decay, g, p.seg_ws[row * p.dstate + n]);
+    decay = fast_exp2(A2 * first);
+  }
+  return g;
+}
+
+// What every segment adds.  Forward: the state after the segment from a zero state, sum over t of
+// exp(A (steps after t)) B_t step_t u_t.  Backward: the adjoint at the segment's first position from a zero adjoint
+// behind it, sum over t of exp(A (steps after the first position up to t)) C_t dy_t.  Either way a lane runs its 8
+// steps from zero and weights the result with one exponential of the steps between it and the segment's end (start):
+// no scan across lanes and no carry, only one sum over the 16 lanes of a row at the end.  Where it runs the chip is
+// short of waves and a segment short of tiles, so latency bounds it: no LDS and no barrier (a lane reads its 8 items of
+// the B or C rows itself, the same 256 bytes for the four rows of every wave, from the caches), a group of states'
+// items requested ahead, workgroups of four independent waves.
+constexpr int SEG_THREADS = 256, SEG_CH = SEG_THREADS / 64 * ROWS;
+template <typename T, int MODE, int BC, bool BWD>
+__global__ __launch_bounds__(SEG_THREADS, BWD || sizeof(T) == 4 ? 3 : 4) void scan_seg_kernel(const MambaScanParams p) {
+  constexpr bool CONST_BC = BWD ? (BC & 2) != 0 : (BC & 1) != 0;  // the operand is one value per channel and state
+  constexpr int NG = sizeof(T) == 4 ? 2 : 4;                      // states whose items are requested together
+  const int N = p.dstate, L = p.seqlen;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & (RL - 1);
+  const int Dg = p.dim / p.ngroups, cblocks = (Dg + SEG_CH - 1) / SEG_CH;
+  const int g = blockIdx.x / cblocks, b = blockIdx.y;
+  const int seg = blockIdx.z + (BWD ? 1 : 0);  // backward: segment 0 sends its adjoint nowhere
+  const int all = (L + TILE - 1) / TILE, per = tiles_per_segment(all, p.nseg);
+  const int tile0 = seg * per, tile1 = min(all, tile0 + per), ntiles = tile1 - tile0;
+  const int dend = (g + 1) * Dg, dw = g * Dg + (int)(blockIdx.x % cblocks) * SEG_CH + (tid >> 4);
+  const bool valid = dw < dend;
+  const int d = min(dw, dend - 1);
+  const T *urow = BWD ? (const T *)p.dout + b * p.dout_bs + d * p.dout_ds : (const T *)p.u + b * p.u_bs + d * p.u_ds;
+  const T *drow = (const T *)p.delta + b * p.delta_bs + d * p.delta_ds;
+  const bool gated = BWD && p.z;
+  const T *zrow = gated ? (const T *)p.z + b * p.z_bs + d * p.z_ds : drow;
+  const float bias = p.delta_bias ? ((const float *)p.delta_bias)[d] : 0.f;
+  const int64_t row = seg_row(p, b, seg, d);
+  const T *Sg = BWD ? (const T *)p.C + b * p.C_bs + g * p.C_gs : (const T *)p.B + b * p.B_bs + g * p.B_gs;
+  const int64_t S_ns = BWD ? p.C_ns : p.B_ns;
+  auto tile_of = [&](int k) { return BWD ? tile0 + k : tile1 - 1 - k; };
+  for (int n0 = 0; n0 < N; n0 += NB16) {
+    float acc[NB16], A2[NB16];
+#pragma unroll
+    for (int n = 0; n < NB16; ++n) {
+      acc[n] = 0.f;
+      A2[n] = n0 + n < N ? ((const float *)p.A)[(int64_t)d * N + n0 + n] * kLog2e : 0.f;
+    }
+    Pack8<T> ku, kd, kz, ks[2][NG];
+    auto fetch_rows = [&](int k) {
+      const int tl = tile_of(k) * TILE + c * KI;
+      load_items<T, MODE>(ku, urow, tl, L, KI);
+      load_items<T, MODE>(kd, drow, tl, L, KI);
+      if (BWD) load_items<T, MODE>(kz, zrow, tl, L, KI);
+    };
+    auto fetch_states = [&](Pack8<T>(&dst)[NG], int k, int n) {
+      if (CONST_BC) return;
+#pragma unroll
+      for (int s = 0; s < NG; ++s)
+        load_items<T, MODE>(dst[s], Sg + (int64_t)min(n0 + n + s, N - 1) * S_ns, tile_of(k) * TILE + c * KI, L, KI);
+    };
+    float run = 0.f, first = 0.f;  // steps of the tiles already taken; the segment's first step
+    fetch_rows(0);
+    fetch_states(ks[0], 0, 0);
+    for (int k = 0; k < ntiles; ++k) {
+      // A lane in a ragged row's last piece reads 8 items from L - 8 on like the other rows' lanes, and leaves out the
+      // ones before its own (nothing has to be moved into place: the order is what counts).
+      const int tl = tile_of(k) * TILE + c * KI, shift = tl - min(tl, L - KI);
+      float x[8], dl[8], z[8], dsum = 0.f;
+      ku.unpack(x);
+      kd.unpack(dl);
+      if (BWD) kz.unpack(z);
+      const int kn = min(k + 1, ntiles - 1);  // (the last tile again at the end)
+      fetch_rows(kn);
+      if (gated) {
+#pragma unroll
+        for (int i = 0; i < KI; ++i) x[i] *= z[i] * sigmoid_f(z[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < KI; ++i) {
+        float v = dl[i] + bias;
+        if (p.delta_softplus) v = softplus_f(v);
+        dl[i] = i >= shift ? v : 0.f;
+        x[i] = i >= shift ? x[i] : 0.f;
+        if (!BWD) x[i] *= dl[i];
+        dsum += dl[i];
+      }
+      float incl = dsum;  // steps of the row's lanes up to and with this one
+      incl += dpp_f<DPP_ROW_SHR + 1>(0.f, incl);
+      incl += dpp_f<DPP_ROW_SHR + 2>(0.f, incl);
+      incl += dpp_f<DPP_ROW_SHR + 4>(0.f, incl);
+      incl += dpp_f<DPP_ROW_SHR + 8>(0.f, incl);
+      const float total = __shfl(incl, lane | (RL - 1), 64);
+      if (BWD && k == 0) {
+        float own = dl[0];
+#pragma unroll
+        for (int i = 1; i < KI; ++i) own = i == shift ? dl[i] : own;
+        first = __shfl(own, lane & ~(RL - 1), 64);
+      }
+      const float away = BWD ? run + (incl - dsum) + dl[0] - first : run + (total - incl);
+      run += total;
+#pragma unroll
+      for (int n = 0; n < NB16; n += NG) {
+        const int cur = (n / NG) & 1;
+        if (n + NG < NB16) fetch_states(ks[cur ^ 1], k, n + NG);
+        else fetch_states(ks[cur ^ 1], kn, 0);
+#pragma unroll
+        for (int s = 0; s < NG; ++s) {
+          float v[8];
+          if constexpr (CONST_BC) {
+            load_bc<1>(v, nullptr, BWD ? p.C : p.B, d, N, n0 + n + s, n + s, c);
+          } else {
+            ks[cur][s].unpack(v);
+          }
+          // (x is zero past the end and A2 for padded states, whose sums are not stored)
+          float h;
+          if constexpr (BWD) {
+            h = x[KI - 1] * v[KI - 1];
+#pragma unroll
+            for (int i = KI - 2; i >= 0; --i) h = __builtin_fmaf(fast_exp2(dl[i + 1] * A2[n + s]), h, x[i] * v[i]);
+          } else {
+            h = x[0] * v[0];
+#pragma unroll
+            for (int i = 1; i < KI; ++i) h = __builtin_fmaf(fast_exp2(dl[i] * A2[n + s]), h, x[i] * v[i]);
+          }
+          acc[n + s] = __builtin_fmaf(fast_exp2(away * A2[n + s]), h, acc[n + s]);
+        }
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < NB16; ++n) {
+      const float v = row_sum_to_last(acc[n]);
+      if (c == RL - 1 && valid && n0 + n < N) p.seg_ws[row * N + n0 + n] = v;
+    }
+    if (c == RL - 1 && valid && n0 == 0) {
+      seg_sums(p)[row] = run;
+      if (BWD) seg_firsts(p)[row] = first;
+    }
+  }
+}
+
 // ------------------------------------------------------------------ forward
 // BC: bit 0 = B is an input-independent (dim, dstate) fp32 matrix, bit 1 = C likewise
 // (selective_scan_fwd_kernel.cuh:74 kIsVariableB / kIsVariableC false).
 // HALF: a checkpoint every 64 positions instead of every 128 (the state entering lane 8 of a row is the state after
 // the tile's first 64 positions): ckpt is then (batch, dim, ceil(L / 64), N).  For the backward kernel that walks
 // 64-position tiles (mamba1_scan_bwd_k4.hip).
-template <typename T, bool VEC, int BC, bool HALF>
+template <typename T, int MODE, int BC, bool HALF>
 __global__ __launch_bounds__(NTHREADS, 4) void scan_fwd_kernel(const MambaScanParams p, const int passes) {
   extern __shared__ __align__(16) float smem[];
   const int N = p.dstate, L = p.seqlen;
@@ -63,12 +229,13 @@ __global__ __launch_bounds__(NTHREADS, 4) void scan_fwd_kernel(const MambaScanPa
 
   for (int i = tid; i < passes * PASS_CH * NP; i += NTHREADS) {
     const int ch = i / NP, n = i % NP, d = d0 + ch;
-    A2s[i] = (d < q.dend && n < N) ? Ag[(int64_t)d * N + n] * kLog2e : 0.f;
-    hcar[i] = 0.f;
+    const float A2 = (d < q.dend && n < N) ? Ag[(int64_t)d * N + n] * kLog2e : 0.f;
+    A2s[i] = A2;
+    hcar[i] = (d < q.dend && n < N) ? seg_state_in(p, q, d, n, A2) : 0.f;
   }
   lds_barrier();
 
-  for (int tile = 0; tile < q.ntiles; ++tile) {
+  for (int tile = q.tile0; tile < q.tile1; ++tile) {
     const int t0 = tile * TILE, tl = t0 + c * KI;
     for (int r = 0; r < passes; ++r) {
       if (d0 + r * PASS_CH >= q.dend) break;  // the whole pass lies past the group (the same in every wave)
@@ -79,12 +246,14 @@ __global__ __launch_bounds__(NTHREADS, 4) void scan_fwd_kernel(const MambaScanPa
       float u[8], dl[8], du[8], y[8], dsum = 0.f;
       Pack8<T> ku, kd, kz;  // raw rows: every load is issued before the first conversion
       kz.zero();
-      load_items<T, VEC>(ku, (const T *)p.u + b * p.u_bs + d * p.u_ds, tl, L, nvalid);
-      load_items<T, VEC>(kd, (const T *)p.delta + b * p.delta_bs + d * p.delta_ds, tl, L, nvalid);
-      if (p.z) load_items<T, VEC>(kz, (const T *)p.z + b * p.z_bs + d * p.z_ds, tl, L, nvalid);
+      load_items<T, MODE>(ku, (const T *)p.u + b * p.u_bs + d * p.u_ds, tl, L, nvalid);
+      load_items<T, MODE>(kd, (const T *)p.delta + b * p.delta_bs + d * p.delta_ds, tl, L, nvalid);
+      if (p.z) load_items<T, MODE>(kz, (const T *)p.z + b * p.z_bs + d * p.z_ds, tl, L, nvalid);
       const float bias = p.delta_bias ? ((const float *)p.delta_bias)[d] : 0.f;
       ku.unpack(u);
       kd.unpack(dl);
+      place_items<MODE>(u, t0, tl, L);
+      place_items<MODE>(dl, t0, tl, L);
 #pragma unroll
       for (int i = 0; i < KI; ++i) {
         float x = dl[i] + bias;
@@ -99,7 +268,7 @@ __global__ __launch_bounds__(NTHREADS, 4) void scan_fwd_kernel(const MambaScanPa
       for (int nb = 0; nb < NBLK; ++nb) {
         if (BC != 3 && (NBLK > 1 || r == 0)) {
           lds_barrier();
-          stage_bc<T, VEC, BC>(Bs, Cs, Bg, p.B_ns, Cg, p.C_ns, nb * NB16, N, t0, L, tid);
+          stage_bc<T, MODE, BC>(Bs, Cs, Bg, p.B_ns, Cg, p.C_ns, nb * NB16, N, t0, L, tid);
           lds_barrier();
         }
         const float *A2row = A2s + chw * NP + nb * NB16;
@@ -157,10 +326,17 @@ __global__ __launch_bounds__(NTHREADS, 4) void scan_fwd_kernel(const MambaScanPa
       if (p.z) {
         float z[8];
         kz.unpack(z);
+        place_items<MODE>(z, t0, tl, L);
 #pragma unroll
         for (int i = 0; i < KI; ++i) y[i] *= z[i] * sigmoid_f(z[i]);
       }
-      st8_guard<T, VEC>((T *)p.out + b * p.out_bs + d * p.out_ds + tl, nvalid, y);
+      T *const orow = (T *)p.out + b * p.out_bs + d * p.out_ds + tl;
+      if constexpr (MODE == ROWS_ANY) {
+        if (nvalid >= KI) st8_any<T>(orow, y);
+        st8_tail<T, MODE>(orow, true, t0, L, nvalid, y);
+      } else {
+        st8_guard<T, MODE == ROWS_ALIGNED>(orow, nvalid, y);
+      }
       if (valid) {  // a row's own lanes wrote its slots of hcar: no other wave touches them
         const float *hfin = hcar + chw * NP;
         if constexpr (HALF) {
@@ -185,7 +361,7 @@ __global__ __launch_bounds__(NTHREADS, 4) void scan_fwd_kernel(const MambaScanPa
 // partial number (workgroup's place in its group), or after every pass and block when the states come
 // in blocks of 16 (the host side then asks for one pass).
 // CKH: the checkpoints come every 64 positions (see scan_fwd_kernel): the state entering tile t is slot 2 t - 1.
-template <typename T, bool VEC, int BC, bool CKH>
+template <typename T, int MODE, int BC, bool CKH>
 __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParams p, const int passes) {
   constexpr bool ck_half = CKH;
   extern __shared__ __align__(16) float smem[];
@@ -227,9 +403,11 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
 
   for (int i = tid; i < WCH * NP; i += NTHREADS) {
     const int ch = i / NP, n = i % NP, d = d0 + ch;
-    A1s[i] = (d < q.dend && n < N) ? Ag[(int64_t)d * N + n] : 0.f;
-    gcar[i] = 0.f;
-    anx[i] = 0.f;
+    const float A1 = (d < q.dend && n < N) ? Ag[(int64_t)d * N + n] : 0.f;
+    A1s[i] = A1;
+    float a_next = 0.f;
+    gcar[i] = (d < q.dend && n < N) ? seg_adjoint_in(p, q, d, n, A1 * kLog2e, a_next) : 0.f;
+    anx[i] = a_next;
     dAacc[i] = 0.f;
     if constexpr (BC != 0) {
       dBcacc[i] = 0.f;
@@ -272,17 +450,17 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
     // row where there is no z): with the same memory operations on every path through a step the compiler counts
     // those in flight exactly, and a wait for these rows leaves the younger stores of the step before draining.
     k.ck = *(const GLOBAL_AS float *)(w.ckpt + (int64_t)max(ck_half ? 2 * tile - 1 : tile - 1, 0) * N + min(c, N - 1));
-    load_items<T, VEC>(k.u, w.u, tl, L, nvalid);
-    load_items<T, VEC>(k.delta, w.delta, tl, L, nvalid);
-    load_items<T, VEC>(k.dout, w.dout, tl, L, nvalid);
-    load_items<T, VEC>(k.z, w.z, tl, L, nvalid);
+    load_items<T, MODE>(k.u, w.u, tl, L, nvalid);
+    load_items<T, MODE>(k.delta, w.delta, tl, L, nvalid);
+    load_items<T, MODE>(k.dout, w.dout, tl, L, nvalid);
+    load_items<T, MODE>(k.z, w.z, tl, L, nvalid);
   };
   int npass = 0;  // passes that hold at least one channel of the group (the same in every wave)
   while (npass < passes && d0 + npass * PASS_CH < q.dend) ++npass;
   Rows nxt;
-  fetch_rows(nxt, ntiles - 1, 0);
+  fetch_rows(nxt, q.tile1 - 1, 0);
 
-  for (int tile = ntiles - 1; tile >= 0; --tile) {
+  for (int tile = q.tile1 - 1; tile >= q.tile0; --tile) {
     const int t0 = tile * TILE, tl = t0 + c * KI;
     for (int r = 0; r < npass; ++r) {
       const int chw = r * PASS_CH + chl;
@@ -298,6 +476,9 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
         nxt.u.unpack(u);
         nxt.delta.unpack(dl);
         nxt.dout.unpack(dy);
+        place_items<MODE>(u, t0, tl, L);
+        place_items<MODE>(dl, t0, tl, L);
+        place_items<MODE>(dy, t0, tl, L);
 #pragma unroll
         for (int i = 0; i < KI; ++i) {  // lanes past the end read a clamped position: mask them
           u[i] = (i < nvalid) ? u[i] : 0.f;
@@ -306,6 +487,7 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
         if (has_z) {
           float z[8];
           nxt.z.unpack(z);
+          place_items<MODE>(z, t0, tl, L);
 #pragma unroll
           for (int i = 0; i < KI; ++i) dy[i] *= z[i] * sigmoid_f(z[i]);
         }
@@ -341,7 +523,7 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
       for (int nb = 0; nb < NBLK; ++nb) {
         if (BC != 3 && (NBLK > 1 || r == 0)) {
           lds_barrier();
-          stage_bc<T, VEC, BC>(Bs, Cs, Bg, p.B_ns, Cg, p.C_ns, nb * NB16, N, t0, L, tid);
+          stage_bc<T, MODE, BC>(Bs, Cs, Bg, p.B_ns, Cg, p.C_ns, nb * NB16, N, t0, L, tid);
           for (int i = tid * 4; i < 2 * ACC_FLOATS; i += NTHREADS * 4)  // dBs and dCs are adjacent
             *reinterpret_cast<f32x4 *>(dBs + i) = f32x4{0.f, 0.f, 0.f, 0.f};
           lds_barrier();
@@ -506,8 +688,8 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
             const int t = t0 + 4 * q4;
             if (n0 + n >= N || t >= L) continue;
             float *dst = (which ? p.dC32 : p.dB32) + (part * N + n0 + n) * L + t;
-            if (VEC) {
-              *reinterpret_cast<f32x4 *>(dst) = v;
+            if (MODE == ROWS_ALIGNED || (MODE == ROWS_ANY && t + 3 < L)) {
+              *(GLOBAL_AS f32x4_a4 *)dst = v;
             } else {
               dst[0] = v.x;
               if (t + 1 < L) dst[1] = v.y;
@@ -521,12 +703,13 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
         float o[8];
         const BwdRow<T> w = rows[chw];
         Pack8<T> z_k, dout_k;  // read again here rather than held through the state loop: they come from the caches
-        load_items<T, VEC>(z_k, w.z, tl, L, nvalid);
-        load_items<T, VEC>(dout_k, w.dout, tl, L, nvalid);
+        load_items<T, MODE>(z_k, w.z, tl, L, nvalid);
+        load_items<T, MODE>(dout_k, w.dout, tl, L, nvalid);
         float dbs = 0.f, dDs = 0.f;
 #pragma unroll
         for (int i = 0; i < KI; ++i) o[i] = __builtin_fmaf(dl[i], acc[i], Dd * dy[i]);
-        st8_or_spare_global<T, VEC>(w.du + tl, nvalid, true, spare, o);
+        st8_or_spare_global<T, MODE>(w.du + tl, nvalid, true, spare, o);
+        st8_tail<T, MODE>(w.du + tl, true, t0, L, nvalid, o);
 #pragma unroll
         for (int i = 0; i < KI; ++i) {
           float gd = __builtin_fmaf(u[i], acc[i], dd[i]);
@@ -536,12 +719,15 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
           dbs += gd;
           dDs = __builtin_fmaf(dy[i], u[i], dDs);
         }
-        st8_or_spare_global<T, VEC>(w.ddelta + tl, nvalid, true, spare, o);
+        st8_or_spare_global<T, MODE>(w.ddelta + tl, nvalid, true, spare, o);
+        st8_tail<T, MODE>(w.ddelta + tl, true, t0, L, nvalid, o);
         float oz[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         if (has_z) {
           float z[8], dout[8];
           z_k.unpack(z);
           dout_k.unpack(dout);
+          place_items<MODE>(z, t0, tl, L);
+          place_items<MODE>(dout, t0, tl, L);
 #pragma unroll
           for (int i = 0; i < KI; ++i) {
             const float yf = __builtin_fmaf(Dd, u[i], y[i]);
@@ -550,8 +736,10 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
             oz[i] = yf * z[i] * s;
           }
         }
-        st8_or_spare_global<T, VEC>(w.dz + tl, nvalid, has_z, spare, o);
-        st8_or_spare_global<T, VEC>(w.out_z + tl, nvalid, w.out_z != nullptr, spare, oz);
+        st8_or_spare_global<T, MODE>(w.dz + tl, nvalid, has_z, spare, o);
+        st8_or_spare_global<T, MODE>(w.out_z + tl, nvalid, w.out_z != nullptr, spare, oz);
+        st8_tail<T, MODE>(w.dz + tl, has_z, t0, L, nvalid, o);
+        st8_tail<T, MODE>(w.out_z + tl, w.out_z != nullptr, t0, L, nvalid, oz);
         dbs = row_sum_to_last(dbs);
         dDs = row_sum_to_last(dDs);
         if (c == RL - 1) {
@@ -562,50 +750,82 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
     }
   }
   lds_barrier();
-  // per-(batch, channel) partial sums; the caller reduces over batch
+  // per-(batch, segment, channel) partial sums, reduced over batch and segments afterwards
+  const int64_t bseg = (int64_t)b * q.nseg + q.seg;
   for (int i = tid; i < WCH * N; i += NTHREADS) {
     const int ch = i / N, n = i % N, d = d0 + ch;
     if (d >= q.dend) continue;
-    p.dA_part[((int64_t)b * p.dim + d) * N + n] = dAacc[ch * NP + n];
-    if constexpr (BC & 1) p.dB32[((int64_t)b * p.dim + d) * N + n] = dBcacc[ch * NP + n];
-    if constexpr (BC & 2) p.dC32[((int64_t)b * p.dim + d) * N + n] = dCcacc[ch * NP + n];
+    p.dA_part[(bseg * p.dim + d) * N + n] = dAacc[ch * NP + n];
+    if constexpr (BC & 1) p.dB32[(bseg * p.dim + d) * N + n] = dBcacc[ch * NP + n];
+    if constexpr (BC & 2) p.dC32[(bseg * p.dim + d) * N + n] = dCcacc[ch * NP + n];
   }
   for (int ch = tid; ch < WCH; ch += NTHREADS) {
     const int d = d0 + ch;
     if (d >= q.dend) continue;
-    p.dD_part[(int64_t)b * p.dim + d] = dDacc[ch];
-    p.ddelta_bias_part[(int64_t)b * p.dim + d] = dbacc[ch];
+    p.dD_part[bseg * p.dim + d] = dDacc[ch];
+    p.ddelta_bias_part[bseg * p.dim + d] = dbacc[ch];
   }
 }
 
-// out[row, e] = sum over parts of part[row, part, e], in the order of the parts, converted to T; one
-// thread per 4 consecutive elements e of the row's `row_len`.
-template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void reduce_parts_kernel(const float *__restrict__ parts, T *__restrict__ out,
-                                                           int64_t rows, int nparts, int64_t row_len) {
-  const int64_t quad = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t per_row = (row_len + 3) / 4;
-  if (quad >= rows * per_row) return;
-  const int64_t row = quad / per_row, e = (quad - row * per_row) * 4;
-  const float *src = parts + row * nparts * row_len + e;
-  T *dst = out + row * row_len + e;
-  if (VEC) {
-    f32x4 v = *reinterpret_cast<const f32x4 *>(src);
-    for (int k = 1; k < nparts; ++k) {
-      const f32x4 w = *reinterpret_cast<const f32x4 *>(src + (int64_t)k * row_len);
-      v.x += w.x; v.y += w.y; v.z += w.z; v.w += w.w;
-    }
-    if constexpr (DT<T>::id == MAMBA_F32) {
-      *reinterpret_cast<f32x4 *>(dst) = v;
-    } else if constexpr (DT<T>::id == MAMBA_BF16) {
-      *reinterpret_cast<u32x2 *>(dst) = u32x2{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+// The sums that leave the backward kernels as partials, in one launch, every sum in the order of its parts.  Workgroups
+// [0, nbc) form dB / dC (dB first): a thread takes 4 consecutive positions of one (batch, group, state) row, four parts
+// in flight.  The others form dA, dD and ddelta_bias: a thread per value, over batch x segments.
+struct ReduceGeo {
+  int nparts, nsum, nbc, per_row;  // partials of dB / dC; of the others; workgroups of dB / dC; quads of a row
+  int64_t rows, row_len;           // rows of one operand (batch x groups x states) and its positions
+};
+template <typename T>
+__global__ __launch_bounds__(256) void reduce_parts_kernel(const MambaScanParams p, const ReduceGeo r) {
+  if ((int)blockIdx.x >= r.nbc) {
+    const int64_t DN = (int64_t)p.dim * p.dstate * (p.a_complex ? 2 : 1), i = (int64_t)(blockIdx.x - r.nbc) * 256 + threadIdx.x;
+    const float *src;
+    float *dst;
+    int64_t at = i, stride = p.dim;
+    if (i < DN) {
+      src = p.dA_part, dst = p.dA, stride = DN;
+    } else if (i < DN + p.dim) {
+      src = p.dD_part, dst = p.dD, at = i - DN;
     } else {
-      *reinterpret_cast<u32x2 *>(dst) = u32x2{pack_f16(v.x, v.y), pack_f16(v.z, v.w)};
+      src = p.ddelta_bias_part, dst = p.ddelta_bias, at = i - DN - p.dim;
+      if (at >= p.dim) return;
     }
+    if (!dst) return;
+    float v = 0.f;
+    for (int k = 0; k < r.nsum; ++k) v += src[k * stride + at];
+    dst[at] = v;
+    return;
+  }
+  const bool first_c = (p.bc_const & 1) != 0;  // dB is no per-position gradient: the workgroups belong to dC
+  const int half = first_c || (p.bc_const & 2) ? r.nbc : r.nbc / 2;
+  const bool is_c = first_c || (int)blockIdx.x >= half;
+  const int64_t quad = (int64_t)(is_c && !first_c ? blockIdx.x - half : blockIdx.x) * 256 + threadIdx.x;
+  if (quad >= r.rows * r.per_row) return;
+  const int64_t row = quad / r.per_row;
+  const int e = (int)(quad - row * r.per_row) * 4, len = (int)r.row_len;
+  const int N = p.dstate, n = (int)(row % N);
+  const int64_t bg = row / N, b = bg / p.ngroups, g = bg - b * p.ngroups;
+  const float *src = (is_c ? p.dC32 : p.dB32) + (bg * r.nparts * N + n) * r.row_len + e;
+  T *dst = static_cast<T *>(is_c ? p.dC : p.dB) + (is_c ? b * p.dC_bs + g * p.dC_gs + n * p.dC_ns : b * p.dB_bs + g * p.dB_gs + n * p.dB_ns) + e;
+  const int64_t pitch = N * r.row_len;
+  if (e + 4 <= len) {
+    f32x4 v = *(const GLOBAL_AS f32x4_a4 *)src;
+    int k = 1;
+    for (; k + 4 <= r.nparts; k += 4) {
+      f32x4 w[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) w[j] = *(const GLOBAL_AS f32x4_a4 *)(src + (k + j) * pitch);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v += w[j];
+    }
+    for (; k < r.nparts; ++k) v += *(const GLOBAL_AS f32x4_a4 *)(src + k * pitch);
+    typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+    if constexpr (DT<T>::id == MAMBA_F32) *(GLOBAL_AS f32x4_a4 *)dst = v;
+    else if constexpr (DT<T>::id == MAMBA_BF16) *(GLOBAL_AS u32x2_a2 *)dst = u32x2{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+    else *(GLOBAL_AS u32x2_a2 *)dst = u32x2{pack_f16(v.x, v.y), pack_f16(v.z, v.w)};
   } else {
-    for (int i = 0; i < 4 && e + i < row_len; ++i) {
+    for (int i = 0; i < 4 && e + i < len; ++i) {
       float v = src[i];
-      for (int k = 1; k < nparts; ++k) v += src[(int64_t)k * row_len + i];
+      for (int k = 1; k < r.nparts; ++k) v += src[k * pitch + i];
       st1<T>(dst + i, v);
     }
   }
@@ -664,21 +884,66 @@ bool use_mx(const MambaScanParams &p) {
 // Passes of PASS_CH channels a backward workgroup takes per tile.  More passes mean fewer, larger
 // partials of dB / dC; the count is chosen so that the workgroups still fill whole rounds over the
 // compute units (one workgroup per unit): the smallest rounds * passes wins, ties go to more passes.
-int bwd_passes(const MambaScanParams &p) {
+int bwd_passes(const MambaScanParams &p, int64_t *cost_out = nullptr) {
   const int np = (p.dstate + NB16 - 1) / NB16 * NB16;
-  if (np > NB16) return 1;  // states in blocks: the sums leave after every block
   const int Dg = p.dim / p.ngroups, cus = compute_units();
+  const int64_t nseg = std::max(1, p.nseg);
   int best = 1;
   int64_t best_cost = -1;
   for (int r = 1; r <= MAX_PASSES; ++r) {
+    if (r > 1 && np > NB16) break;  // states in blocks: the sums leave after every block
     if ((use_mx(p) ? mamba1_bwd_mx_lds(r, np) : bwd_lds(r, np, p.bc_const & 3)) > LDS_LIMIT) break;
     if (r > 1 && (r - 1) * PASS_CH >= Dg) break;
-    const int64_t wgs = (int64_t)p.batch * p.ngroups * ((Dg + PASS_CH * r - 1) / (PASS_CH * r));
+    const int64_t wgs = (int64_t)p.batch * nseg * p.ngroups * ((Dg + PASS_CH * r - 1) / (PASS_CH * r));
     const int64_t cost = (wgs + cus - 1) / cus * r;
     if (best_cost < 0 || cost <= best_cost) {
       best_cost = cost;
       best = r;
     }
+  }
+  if (cost_out) *cost_out = std::max<int64_t>(1, best_cost);
+  return best;
+}
+
+// Segments of the sequence: the split with the least estimated time in us, for 16 states.  The terms were fitted to the
+// times of 1 .. 32 segments at 13 sizes (batch 1 - 8, 768 - 5120 channels, 256 - 8192 positions; within 10 % of almost
+// all).  A tile of a round of forward workgroups takes 6.4, half as much again where two share a CU; one of a round of
+// backward workgroups (one per CU) 13 per pass and a third of that for what the passes share; a round's start and end
+// 2 and 5.3.  The pass over the segments (all but one) takes 3.0 (forward) or 4.5 (backward) a tile, twice that from four
+// of its workgroups per CU on, and every segment 0.9 or 1.8 for its launch and for going through the segments before it.
+// A split has to promise 6 %.  Measured: 1536 channels x 777 positions of one sequence 50 -> 30 us forward, 133 -> 63
+// backward; from about 256 workgroups on one segment is left.
+constexpr int MAX_SEGMENTS = 32;
+int scan_segments(const MambaScanParams &p, bool bwd) {
+  const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
+  const int64_t rows = (int64_t)p.batch * p.ngroups;
+  const int64_t wgs = rows * ((Dg + PASS_CH - 1) / PASS_CH), seg_wgs = rows * ((Dg + SEG_CH - 1) / SEG_CH);
+  if (p.a_complex || p.batch > 65535 || k4_mode() || use_mx(p)) return 1;
+  const int blocks = (p.dstate + NB16 - 1) / NB16;
+  int best = 1;
+  double best_cost = -1.0;
+  for (int s = 1; s <= std::min(ntiles, MAX_SEGMENTS); ++s) {
+    const int per = (ntiles + s - 1) / s;
+    if (s > 1 && (s - 1) * per >= ntiles) continue;  // leaves the last segment empty
+    double tiles, rounds;
+    if (bwd) {
+      MambaScanParams q = p;
+      q.nseg = s;
+      int64_t rounds_passes = 1;
+      const int r = bwd_passes(q, &rounds_passes);
+      tiles = 13.0 * (double)rounds_passes * (1.0 + 0.33 / r);
+      rounds = 5.3 * (double)rounds_passes / r;
+    } else {
+      const int64_t n = (wgs * s + 2 * cus - 1) / (2 * cus);
+      tiles = 6.4 * (double)n * (wgs * s > cus ? 1.47 : 1.0);
+      rounds = 2.0 * (double)n;
+    }
+    double cost = tiles * blocks * per + rounds;
+    if (s > 1) {
+      const double share = std::max(1.0, 0.52 * (double)((seg_wgs * (s - 1) + cus - 1) / cus));
+      cost = 1.06 * (cost + (bwd ? 4.5 : 3.0) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
+    }
+    if (best_cost < 0 || cost < best_cost) best_cost = cost, best = s;
   }
   return best;
 }
@@ -744,8 +1009,17 @@ int launch(KernelT kernel, const MambaScanParams &p, int passes, size_t lds, hip
   const int cblocks = (Dg + PASS_CH * passes - 1) / (PASS_CH * passes);
   if (lds > LDS_LIMIT) return MAMBA_E_UNSUPPORTED;
   if (!mamba1_allow_lds(reinterpret_cast<const void *>(kernel), lds)) return MAMBA_E_LAUNCH;
-  dim3 grid(p.ngroups * cblocks, p.batch), block(NTHREADS);
+  dim3 grid(p.ngroups * cblocks, p.batch, std::max(1, p.nseg)), block(NTHREADS);
   hipLaunchKernelGGL(kernel, grid, block, lds, stream, p, passes);
+  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
+}
+
+template <typename T, int BC, bool BWD> int launch_segments(const MambaScanParams &p, int mode, hipStream_t stream) {
+  if (p.nseg <= 1) return MAMBA_OK;
+  const int Dg = p.dim / p.ngroups;
+  const dim3 grid(p.ngroups * ((Dg + SEG_CH - 1) / SEG_CH), p.batch, p.nseg - 1), block(SEG_THREADS);
+  if (mode == ROWS_ALIGNED) hipLaunchKernelGGL((scan_seg_kernel<T, ROWS_ALIGNED, BC, BWD>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((scan_seg_kernel<T, ROWS_ANY, BC, BWD>), grid, block, 0, stream, p);
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
 }
 
@@ -755,6 +1029,11 @@ int check_common(const MambaScanParams *p) {
   if (p->dim % p->ngroups != 0) return MAMBA_E_BADARG;
   if (p->dstate > MAX_DSTATE) return MAMBA_E_UNSUPPORTED;
   if (p->dtype != MAMBA_F32 && p->dtype != MAMBA_BF16 && p->dtype != MAMBA_F16) return MAMBA_E_BADARG;
+  if (p->nseg > 1) {  // every segment holds at least one tile
+    const int ntiles = (p->seqlen + TILE - 1) / TILE, per = (ntiles + p->nseg - 1) / p->nseg;
+    if (!p->seg_ws || p->nseg > MAX_SEGMENTS || (p->nseg - 1) * per >= ntiles) return MAMBA_E_BADARG;
+    if (p->a_complex || p->batch > 65535 || k4_mode() || use_mx(*p)) return MAMBA_E_UNSUPPORTED;
+  }
   return MAMBA_OK;
 }
 
@@ -773,35 +1052,43 @@ bool vec_ok(const MambaScanParams &p, bool bwd) {
   return v && ok(p.dout, p.dout_bs, p.dout_ds) && ok(p.du, p.du_bs, p.du_ds) &&
          ok(p.ddelta, p.ddelta_bs, p.ddelta_ds) && ok(p.dz, p.dz_bs, p.dz_ds) && ok(p.out_z, p.outz_bs, p.outz_ds);
 }
-
-template <typename T>
-int reduce_parts(const float *parts, void *out, int64_t rows, int nparts, int64_t row_len, hipStream_t stream) {
-  const int64_t quads = rows * ((row_len + 3) / 4);
-  if ((quads + 255) / 256 > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
-  const dim3 grid((unsigned)((quads + 255) / 256)), block(256);
-  T *o = static_cast<T *>(out);
-  if (row_len % 4 == 0 && aligned16(parts) && aligned16(out))
-    hipLaunchKernelGGL((reduce_parts_kernel<T, true>), grid, block, 0, stream, parts, o, rows, nparts, row_len);
-  else
-    hipLaunchKernelGGL((reduce_parts_kernel<T, false>), grid, block, 0, stream, parts, o, rows, nparts, row_len);
-  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
+int row_mode(const MambaScanParams &p, bool bwd) {
+  return vec_ok(p, bwd) ? ROWS_ALIGNED : p.seqlen >= KI ? ROWS_ANY : ROWS_SCALAR;
 }
 
-// dB / dC of per-position operands: the partials summed in a fixed order into the outputs
-template <typename T> int reduce_dBC(const MambaScanParams &p, int nparts, hipStream_t stream) {
-  const int64_t rows = (int64_t)p.batch * p.ngroups;
-  const int64_t row_len = (int64_t)p.dstate * p.seqlen * (p.a_complex ? 2 : 1);
-  int rc = MAMBA_OK;
-  if (!(p.bc_const & 1)) rc = reduce_parts<T>(p.dB32, p.dB, rows, nparts, row_len, stream);
-  if (rc == MAMBA_OK && !(p.bc_const & 2)) rc = reduce_parts<T>(p.dC32, p.dC, rows, nparts, row_len, stream);
-  return rc;
+// dB / dC of per-position operands and, where the caller wants the finished sums, dA, dD and ddelta_bias.  `which`: bit
+// 0 the former, bit 1 the latter (a problem served in slices of batch rows adds those up once, at the end).
+template <typename T> int reduce_sums(const MambaScanParams &p_in, int nparts, int which, hipStream_t stream) {
+  MambaScanParams p = p_in;
+  ReduceGeo r{};
+  const int64_t cx = p.a_complex ? 2 : 1, G = p.ngroups, N = p.dstate;
+  r.nparts = nparts, r.nsum = p.batch * std::max(1, p.nseg);
+  r.row_len = p.seqlen * cx;
+  r.rows = (int64_t)p.batch * G * N;
+  r.per_row = (int)((r.row_len + 3) / 4);
+  if (!(p.dB_bs | p.dB_gs | p.dB_ns)) p.dB_bs = G * N * r.row_len, p.dB_gs = N * r.row_len, p.dB_ns = r.row_len;
+  if (!(p.dC_bs | p.dC_gs | p.dC_ns)) p.dC_bs = G * N * r.row_len, p.dC_gs = N * r.row_len, p.dC_ns = r.row_len;
+  const int operands = (which & 1) ? ((p.bc_const & 1) ? 0 : 1) + ((p.bc_const & 2) ? 0 : 1) : 0;
+  const int64_t each = (r.rows * r.per_row + 255) / 256, nbc = operands * each;
+  int64_t sums = 0;
+  if ((which & 2) && (p.dA || p.dD || p.ddelta_bias)) sums = ((int64_t)p.dim * (N * cx + 2) + 255) / 256;
+  if (nbc + sums == 0) return MAMBA_OK;
+  if (nbc + sums > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
+  r.nbc = (int)nbc;
+  hipLaunchKernelGGL(reduce_parts_kernel<T>, dim3((unsigned)(nbc + sums)), dim3(256), 0, stream, p, r);
+  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
+}
+template <typename T> int reduce_dBC(const MambaScanParams &p, const MambaScanParams &plan, int nparts, hipStream_t stream) {
+  return reduce_sums<T>(p, nparts, p.batch == plan.batch ? 3 : 1, stream);
 }
 
 // `plan`: the whole problem, of which p may be a slice of batch rows; it decides the passes per workgroup and with
 // them the number of dB / dC partials, which must be the same for every slice.
 template <typename T, bool BWD, int BC> int dispatch_bc(const MambaScanParams &p, const MambaScanParams &plan, hipStream_t stream) {
   const int np = (p.dstate + NB16 - 1) / NB16 * NB16;
-  const bool vec = vec_ok(p, BWD);
+  const int mode = row_mode(p, BWD);
+  int rc = launch_segments<T, BC, BWD>(p, mode, stream);
+  if (rc != MAMBA_OK) return rc;
   if (!BWD) {
     // MAMBA_AMD_FWD_MIN_LDS (bytes): a measurement hook.  A workgroup that asks for more LDS shares its CU with fewer
     // others (160 KB per CU), which is how the kernel's speed against resident waves per SIMD is measured.
@@ -809,43 +1096,45 @@ template <typename T, bool BWD, int BC> int dispatch_bc(const MambaScanParams &p
     const bool half = k4_mode();
     const size_t lds = fwd_lds(1, np, half) > min_lds ? fwd_lds(1, np, half) : min_lds;
     if (half)
-      return vec ? launch(scan_fwd_kernel<T, true, BC, true>, p, 1, lds, stream)
-                 : launch(scan_fwd_kernel<T, false, BC, true>, p, 1, lds, stream);
-    return vec ? launch(scan_fwd_kernel<T, true, BC, false>, p, 1, lds, stream)
-               : launch(scan_fwd_kernel<T, false, BC, false>, p, 1, lds, stream);
+      return mode == ROWS_ALIGNED ? launch(scan_fwd_kernel<T, ROWS_ALIGNED, BC, true>, p, 1, lds, stream)
+                                  : launch(scan_fwd_kernel<T, ROWS_SCALAR, BC, true>, p, 1, lds, stream);
+    switch (mode) {
+      case ROWS_ALIGNED: return launch(scan_fwd_kernel<T, ROWS_ALIGNED, BC, false>, p, 1, lds, stream);
+      case ROWS_ANY: return launch(scan_fwd_kernel<T, ROWS_ANY, BC, false>, p, 1, lds, stream);
+      default: return launch(scan_fwd_kernel<T, ROWS_SCALAR, BC, false>, p, 1, lds, stream);
+    }
   }
   if (use_k4(plan)) {
     const K4Plan k = k4_plan(plan);
-    if (vec) {
+    if (mode == ROWS_ALIGNED) {
       if constexpr (std::is_same_v<T, bf16_t> && BC == 0) {
-        const int rc = mamba1_bwd_k4_launch(p, k.pa, k.pb, k.nparts, stream);
-        return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, k.nparts, stream);
+        rc = mamba1_bwd_k4_launch(p, k.pa, k.pb, k.nparts, stream);
+        return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, plan, k.nparts, stream);
       }
     }
     // rows the 4-item kernel does not take (unaligned views): the default kernel with as many passes as a long and a
     // short workgroup together, whose partials are fewer than the workspace was sized for: the others are cleared
     const int64_t bytes = (int64_t)p.batch * p.ngroups * k.nparts * p.dstate * p.seqlen * 4;
-    int rc = mamba_hip_zero(p.dB32, bytes, stream);
+    rc = mamba_hip_zero(p.dB32, bytes, stream);
     if (rc == MAMBA_OK) rc = mamba_hip_zero(p.dC32, bytes, stream);
     if (rc != MAMBA_OK) return rc;
     const int passes = k.pa == k.pb ? k.pa : k.pa + k.pb;
-    rc = launch(scan_bwd_kernel<T, false, BC, true>, p, passes, bwd_lds(passes, np, BC), stream);
-    return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, k.nparts, stream);
+    rc = launch(scan_bwd_kernel<T, ROWS_SCALAR, BC, true>, p, passes, bwd_lds(passes, np, BC), stream);
+    return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, plan, k.nparts, stream);
   }
   const int passes = bwd_passes(plan);
   if (use_mx(p)) {
-    const int rc = mamba1_bwd_mx_launch(p, passes, vec, stream);
-    return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, bwd_nparts(plan), stream);
+    rc = mamba1_bwd_mx_launch(p, passes, mode == ROWS_ALIGNED, stream);
+    return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, plan, bwd_nparts(plan), stream);
   }
   const size_t lds = bwd_lds(passes, np, BC);
-  int rc;
   if (k4_mode())
-    rc = vec ? launch(scan_bwd_kernel<T, true, BC, true>, p, passes, lds, stream)
-             : launch(scan_bwd_kernel<T, false, BC, true>, p, passes, lds, stream);
-  else
-    rc = vec ? launch(scan_bwd_kernel<T, true, BC, false>, p, passes, lds, stream)
-             : launch(scan_bwd_kernel<T, false, BC, false>, p, passes, lds, stream);
-  return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, bwd_nparts(plan), stream);
+    rc = mode == ROWS_ALIGNED ? launch(scan_bwd_kernel<T, ROWS_ALIGNED, BC, true>, p, passes, lds, stream)
+                              : launch(scan_bwd_kernel<T, ROWS_SCALAR, BC, true>, p, passes, lds, stream);
+  else if (mode == ROWS_ALIGNED) rc = launch(scan_bwd_kernel<T, ROWS_ALIGNED, BC, false>, p, passes, lds, stream);
+  else if (mode == ROWS_ANY) rc = launch(scan_bwd_kernel<T, ROWS_ANY, BC, false>, p, passes, lds, stream);
+  else rc = launch(scan_bwd_kernel<T, ROWS_SCALAR, BC, false>, p, passes, lds, stream);
+  return rc != MAMBA_OK ? rc : reduce_dBC<T>(p, plan, bwd_nparts(plan), stream);
 }
 
 template <typename T, bool BWD> int dispatch(const MambaScanParams &p, const MambaScanParams &plan, hipStream_t stream) {
@@ -880,7 +1169,8 @@ MambaScanParams batch_slice(const MambaScanParams &p, int64_t b0, int nb, int np
   adv(q.dB32, (p.bc_const & 1) ? D * N * cx : G * nparts * N * L * cx, 4);
   adv(q.dC32, (p.bc_const & 2) ? D * N * cx : G * nparts * N * L * cx, 4);
   adv(q.dA_part, D * N * cx, 4), adv(q.dD_part, D, 4), adv(q.ddelta_bias_part, D, 4);
-  adv(q.dB, G * N * L * cx, es), adv(q.dC, G * N * L * cx, es);
+  adv(q.dB, (p.dB_bs | p.dB_gs | p.dB_ns) ? p.dB_bs : G * N * L * cx, es);
+  adv(q.dC, (p.dC_bs | p.dC_gs | p.dC_ns) ? p.dC_bs : G * N * L * cx, es);
   adv(q.det_dB, G * N * L * cx, 8), adv(q.det_dC, G * N * L * cx, 8);
   return q;
 }
@@ -917,9 +1207,9 @@ int scan_bwd_one(const MambaScanParams &p, const MambaScanParams &plan, mamba_st
     }
     if (rc != MAMBA_OK) return rc;
     switch (p.dtype) {
-      case MAMBA_F32: return reduce_dBC<float>(p, 1, s);
-      case MAMBA_BF16: return reduce_dBC<bf16_t>(p, 1, s);
-      default: return reduce_dBC<f16_t>(p, 1, s);
+      case MAMBA_F32: return reduce_dBC<float>(p, plan, 1, s);
+      case MAMBA_BF16: return reduce_dBC<bf16_t>(p, plan, 1, s);
+      default: return reduce_dBC<f16_t>(p, plan, 1, s);
     }
   }
   switch (p.dtype) {
@@ -996,6 +1286,7 @@ extern "C" int mamba1_scan_fwd_noalloc(const MambaScanParams *p, float *last_sta
   if (!ws) return MAMBA_E_LAUNCH;
   MambaScanParams q = *p;
   q.ckpt = ws;
+  q.nseg = 0;
   const int rc = mamba1_scan_fwd(&q, stream);
   if (rc != MAMBA_OK || !last_state) return rc;
   const int64_t n = rows * width;
@@ -1026,5 +1317,12 @@ extern "C" int mamba1_scan_bwd(const MambaScanParams *p, mamba_stream_t stream) 
     rc = p->batch <= MAX_GRID_BATCH ? scan_bwd_one(*p, *p, stream) : scan_bwd_one(batch_slice(*p, b0, nb, nparts), *p, stream);
     if (rc != MAMBA_OK) return rc;
   }
+  if (p->batch > MAX_GRID_BATCH) return reduce_sums<float>(*p, nparts, 2, static_cast<hipStream_t>(stream));
   return MAMBA_OK;
+}
+
+extern "C" int mamba1_scan_segments(const MambaScanParams *p, int backward) {
+  if (!p || p->batch <= 0 || p->dim <= 0 || p->seqlen <= 0 || p->dstate <= 0 || p->ngroups <= 0 || p->dim % p->ngroups != 0)
+    return MAMBA_E_BADARG;
+  return p->seqlen < KI ? 1 : scan_segments(*p, backward != 0);
 }

@@ -20,10 +20,15 @@ constexpr int ACC_FLOATS = NB16 * ACC_PITCH;   // one accumulator: [n][half][lan
 constexpr int MAX_DSTATE = 256;
 constexpr int MAX_PASSES = 8;
 
+// How a kernel reaches the rows (positions contiguous): ROWS_SCALAR element by element (fewer than 8 positions),
+// ROWS_ALIGNED 16-byte pieces (16-byte aligned rows, whole pieces), ROWS_ANY 16-byte pieces at any alignment with a
+// ragged last piece, which is loaded from inside the row and moved into place.
+constexpr int ROWS_SCALAR = 0, ROWS_ALIGNED = 1, ROWS_ANY = 2;
+
 // B or C rows n0..n0+15 of the tile starting at t0 -> LDS as fp32, laid out [n][half][c][4] (c = the
 // lane's place in its row) so that a lane reads its 8 items with two 16-byte LDS loads.
 // BC: bit 0 set = B is not staged (input-independent), bit 1 = C likewise.
-template <typename T, bool VEC, int BC>
+template <typename T, int MODE, int BC>
 DEVI void stage_bc(float *Bs, float *Cs, const T *Bg, int64_t B_ns, const T *Cg, int64_t C_ns, int n0, int N, int t0,
                    int L, int tid) {
   constexpr int FIRST = (BC & 1) ? NB16 * RL : 0, LAST = (BC & 2) ? NB16 * RL : 2 * NB16 * RL;
@@ -34,13 +39,19 @@ DEVI void stage_bc(float *Bs, float *Cs, const T *Bg, int64_t B_ns, const T *Cg,
     if (unit >= LAST) return;
     const int which = unit >> 8, n = (unit >> 4) & 15, j = unit & 15;
     float v[8];
-    if constexpr (VEC) {
+    if constexpr (MODE != ROWS_SCALAR) {
       // from a clamped (valid) address, masked afterwards
-      Pack8<T> raw;
-      const int nc = min(n0 + n, N - 1), t = min(t0 + KI * j, L - KI);
-      raw.load((which ? Cg + (int64_t)nc * C_ns : Bg + (int64_t)nc * B_ns) + t);
-      raw.unpack(v);
-      const bool ok = n0 + n < N && t0 + KI * j < L;
+      const int nc = min(n0 + n, N - 1), t = t0 + KI * j;
+      const T *row = which ? Cg + (int64_t)nc * C_ns : Bg + (int64_t)nc * B_ns;
+      if constexpr (MODE == ROWS_ALIGNED) {
+        Pack8<T> raw;
+        raw.load(row + min(t, L - KI));
+        raw.unpack(v);
+      } else {
+        row8_raw<T>(row, t, L, v);
+        if (t0 + TILE > L) row8_place(t, L, v);
+      }
+      const bool ok = n0 + n < N && t < L;
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = ok ? v[i] : 0.f;
     } else {
@@ -55,15 +66,30 @@ DEVI void stage_bc(float *Bs, float *Cs, const T *Bg, int64_t B_ns, const T *Cg,
   }
 }
 
-// The 8 items of one (batch, channel) row owned by this lane, as stored: VEC reads 16 bytes from a
-// clamped position (the caller masks lanes past the end), else element by element.
-template <typename T, bool VEC> DEVI void load_items(Pack8<T> &k, const T *row, int tl, int L, int nvalid) {
-  if constexpr (VEC) {
+// The 8 items of one (batch, channel) row owned by this lane, as stored: 16 bytes from a clamped position (the
+// caller masks lanes past the end, and moves a ragged row's last piece into place: place_items), or element by element.
+template <typename T, int MODE> DEVI void load_items(Pack8<T> &k, const T *row, int tl, int L, int nvalid) {
+  if constexpr (MODE == ROWS_ALIGNED) {
     k.load_global(row + min(tl, L - KI));
+  } else if constexpr (MODE == ROWS_ANY) {
+    k.load_any(row + min(tl, L - KI));
   } else {
     float v[8];
     ld8_guard<T, false>(row + tl, nvalid, 0.f, v);
     k.pack(v);
+  }
+}
+
+// After the unpacking of rows that load_items has read: only the last tile of a ragged row has anything to move.
+template <int MODE> DEVI void place_items(float (&v)[8], int t0, int tl, int L) {
+  if constexpr (MODE == ROWS_ANY) {
+    if (t0 + TILE > L) row8_place(tl, L, v);
+  }
+}
+// the values of a ragged row's last piece, element by element
+template <typename T, int MODE> DEVI void st8_tail(T *dst, bool wanted, int t0, int L, int nvalid, const float (&v)[8]) {
+  if constexpr (MODE == ROWS_ANY) {
+    if (t0 + TILE > L && wanted && nvalid < KI) st8_guard<T, false>(dst, nvalid, v);
   }
 }
 
@@ -92,10 +118,12 @@ DEVI void load_bc(float (&v)[8], const float *staged, const void *mat, int d, in
   }
 }
 
-// Where a workgroup's channels lie: workgroup cb of group g takes `passes` passes of PASS_CH channels.
+// Where a workgroup's channels lie: workgroup cb of group g takes `passes` passes of PASS_CH channels, and the tiles
+// [tile0, tile1) of segment blockIdx.z of the sequence.
 struct Geo {
-  int g, cb, b, Dg, dend, ntiles, cblocks;
+  int g, cb, b, Dg, dend, ntiles, cblocks, seg, nseg, tile0, tile1;
 };
+DEVI int tiles_per_segment(int ntiles, int nseg) { return (ntiles + nseg - 1) / nseg; }
 DEVI Geo geometry(const MambaScanParams &p, int passes) {
   Geo q;
   q.Dg = p.dim / p.ngroups;
@@ -105,6 +133,11 @@ DEVI Geo geometry(const MambaScanParams &p, int passes) {
   q.b = blockIdx.y;
   q.dend = (q.g + 1) * q.Dg;
   q.ntiles = (p.seqlen + TILE - 1) / TILE;
+  q.seg = blockIdx.z;
+  q.nseg = max(1, p.nseg);
+  const int per = tiles_per_segment(q.ntiles, q.nseg);
+  q.tile0 = q.seg * per;
+  q.tile1 = min(q.ntiles, q.tile0 + per);
   return q;
 }
 

@@ -89,6 +89,7 @@ def _fill_common(p, u, delta, A, B, C, D, z, delta_bias, delta_softplus, ckpt, d
     p.dtype = _lib.DTYPE_CODE[u.dtype]
     p.delta_softplus = int(bool(delta_softplus))
     p.a_complex = int(A.is_complex())
+    p.nseg = 0
     p.u, p.delta, p.A, p.B, p.C = u.data_ptr(), delta.data_ptr(), A.data_ptr(), B.data_ptr(), C.data_ptr()
     p.D, p.z, p.delta_bias = _lib.ptr(D), _lib.ptr(z), _lib.ptr(delta_bias)
     p.ckpt = ckpt.data_ptr()
@@ -101,6 +102,18 @@ def _fill_common(p, u, delta, A, B, C, D, z, delta_bias, delta_softplus, ckpt, d
         p.B_bs, p.B_gs, p.B_ns = B.stride(0), B.stride(1), B.stride(2)
     if C.dim() == 4:
         p.C_bs, p.C_gs, p.C_ns = C.stride(0), C.stride(1), C.stride(2)
+
+
+def _split_sequence(p, device, backward):
+    """Sets p's number of segments (a batch x channels too small to fill the GPU is cut along the sequence) and
+    their workspace, which is returned."""
+    with torch.cuda.device(device):
+        p.nseg = max(1, _lib.load().mamba1_scan_segments(p, int(backward)))
+    if p.nseg == 1:
+        return None
+    ws = torch.empty(p.batch * p.nseg * p.dim * (p.dstate + 2), device=device, dtype=torch.float32)
+    p.seg_ws = ws.data_ptr()
+    return ws
 
 
 def selective_scan_fwd(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta_softplus=False):
@@ -128,6 +141,7 @@ def selective_scan_fwd(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta
     _fill_common(p, u, delta, A, B, C, D, z, delta_bias, delta_softplus, ckpt, dims)
     p.out = out.data_ptr()
     p.out_bs, p.out_ds = out.stride(0), out.stride(1)
+    _ws = _split_sequence(p, u.device, False)
     with torch.cuda.device(u.device):
         _lib.check(_lib.load().mamba1_scan_fwd(p, _lib.current_stream(u.device)), "mamba1_scan_fwd")
     return out, ckpt
@@ -135,9 +149,9 @@ def selective_scan_fwd(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta
 
 class ScanBwdBuffers:
     """Outputs and fp32 workspaces of one backward launch (all caller-owned).  `nparts` is
-    mamba1_scan_bwd_nparts for the launch's sizes."""
+    mamba1_scan_bwd_nparts for the launch's sizes, `nseg` its segments of the sequence."""
 
-    def __init__(self, u, delta, B, z, dims, dz=None, recompute_out_z=False, C=None, complex_A=False, nparts=1):
+    def __init__(self, u, delta, B, z, dims, dz=None, recompute_out_z=False, C=None, complex_A=False, nparts=1, nseg=1):
         batch, dim, seqlen, dstate, ngroups = dims
         dev = u.device
         self.du = torch.empty_like(u)
@@ -146,11 +160,17 @@ class ScanBwdBuffers:
         # call adds up into dB / dC in the operand's dtype; or (batch, dim, dstate) per-batch partials
         # when the operand is an input-independent matrix; with a complex A every entry is a (re, im) pair
         two = 2 if complex_A else 1
-        self.dB32, self.dB = self._operand(B, batch, dim, ngroups, nparts, dstate, seqlen, two, dev)
-        self.dC32, self.dC = self._operand(C, batch, dim, ngroups, nparts, dstate, seqlen, two, dev)
-        self.dA_part = torch.empty(batch, dim, dstate * two, device=dev, dtype=torch.float32)
-        self.dD_part = torch.empty(batch, dim, device=dev, dtype=torch.float32)
-        self.dbias_part = torch.empty(batch, dim, device=dev, dtype=torch.float32)
+        self.dB32, self.dB = self._operand(B, batch, dim, ngroups, nparts, dstate, seqlen, two, dev, nseg)
+        self.dC32, self.dC = self._operand(C, batch, dim, ngroups, nparts, dstate, seqlen, two, dev, nseg)
+        # per-(batch, segment, channel) partials of dA, dD and ddelta_bias, and their sums
+        self.dA_part = torch.empty(batch * nseg, dim, dstate * two, device=dev, dtype=torch.float32)
+        self.dD_part = torch.empty(batch * nseg, dim, device=dev, dtype=torch.float32)
+        self.dbias_part = torch.empty(batch * nseg, dim, device=dev, dtype=torch.float32)
+        self.dA = torch.empty(dim, dstate * two, device=dev, dtype=torch.float32)
+        self.dD = torch.empty(dim, device=dev, dtype=torch.float32)
+        self.dbias = torch.empty(dim, device=dev, dtype=torch.float32)
+        self.nseg = nseg
+        self.seg_ws = torch.empty(batch * nseg * dim * (dstate + 2), device=dev, dtype=torch.float32) if nseg > 1 else None
         self.dz = self.out_z = None
         if z is not None:
             self.dz = dz if dz is not None else torch.empty_like(z)
@@ -158,9 +178,9 @@ class ScanBwdBuffers:
                 self.out_z = torch.empty_like(u)
 
     @staticmethod
-    def _operand(t, batch, dim, ngroups, nparts, dstate, seqlen, two, dev):
+    def _operand(t, batch, dim, ngroups, nparts, dstate, seqlen, two, dev, nseg):
         if t is not None and t.dim() == 2:
-            return torch.empty(batch, dim, dstate * two, device=dev, dtype=torch.float32), None
+            return torch.empty(batch * nseg, dim, dstate * two, device=dev, dtype=torch.float32), None
         part = torch.empty(batch, ngroups, nparts, dstate, seqlen * two, device=dev, dtype=torch.float32)
         return part, torch.empty(batch, ngroups, dstate, seqlen * two, device=dev, dtype=t.dtype)
 
@@ -174,10 +194,14 @@ def scan_bwd_launch(u, delta, A, B, C, D, z, delta_bias, dout, ckpt, delta_softp
     lib = _lib.load()
     if bufs is None:
         with torch.cuda.device(u.device):
+            p.nseg = max(1, lib.mamba1_scan_segments(p, 1))
             nparts = lib.mamba1_scan_bwd_nparts(p)
         if nparts <= 0:
             _lib.check(nparts or -1, "mamba1_scan_bwd_nparts")
-        bufs = ScanBwdBuffers(u, delta, B, z, dims, dz, recompute_out_z, C=C, complex_A=A.is_complex(), nparts=nparts)
+        bufs = ScanBwdBuffers(u, delta, B, z, dims, dz, recompute_out_z, C=C, complex_A=A.is_complex(), nparts=nparts,
+                              nseg=p.nseg)
+    p.nseg, p.seg_ws = bufs.nseg, _lib.ptr(bufs.seg_ws)
+    p.dA, p.dD, p.ddelta_bias = bufs.dA.data_ptr(), bufs.dD.data_ptr(), bufs.dbias.data_ptr()
     dz, out_z = bufs.dz, bufs.out_z
     p.dout, p.du, p.ddelta = dout.data_ptr(), bufs.du.data_ptr(), bufs.ddelta.data_ptr()
     p.dz, p.out_z = _lib.ptr(dz), _lib.ptr(out_z)
@@ -237,9 +261,9 @@ def selective_scan_bwd(u, delta, A, B, C, D, z, delta_bias, dout, ckpt, dz=None,
         raise RuntimeError(f"selective_scan: ckpt must be the contiguous fp32 {want} tensor of the forward call")
     bufs = scan_bwd_launch(u, delta, A, B, C, D, z, delta_bias, dout, ckpt, delta_softplus, dims, dz, recompute_out_z)
     as_A = (lambda t: torch.view_as_complex(t.reshape(dim, dstate, 2))) if cplx else (lambda t: t)
-    dA = as_A(bufs.dA_part.sum(0))
-    dD = bufs.dD_part.sum(0) if D is not None else None
-    ddelta_bias = bufs.dbias_part.sum(0) if delta_bias is not None else None
+    dA = as_A(bufs.dA)
+    dD = bufs.dD if D is not None else None
+    ddelta_bias = bufs.dbias if delta_bias is not None else None
     dB = as_A(bufs.dB32.sum(0)) if B.dim() == 2 else bufs.dB
     dC = as_A(bufs.dC32.sum(0)) if C.dim() == 2 else bufs.dC
     return (bufs.du, bufs.ddelta, dA, dB, dC, dD, ddelta_bias, bufs.dz, bufs.out_z)

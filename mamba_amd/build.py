@@ -45,31 +45,49 @@ def _compile(src, force):
 
 
 EXT = os.path.join(HERE, "_torch_ext.so")
-EXT_SRC = os.path.join(CSRC, "torch_ext.cpp")
 
 
-def build_torch_ext(force=False):
-    """Compiles csrc/torch_ext.cpp (host code only: the decode-step operators' argument handling on
-    at::Tensor) into the Python extension module mamba_amd/_torch_ext.so, linked against the kernel
-    library beside it.  Needs the library to exist."""
+def ext_sources():
+    return sorted(os.path.join(CSRC, f) for f in os.listdir(CSRC) if f.startswith("torch_") and f.endswith(".cpp"))
+
+
+def build_torch_ext(force=False, jobs=None):
+    """Compiles csrc/torch_*.cpp (host code only: the operators' argument handling and autograd nodes on at::Tensor)
+    into the Python extension module mamba_amd/_torch_ext.so, linked against the kernel library beside it.  Needs the
+    library to exist."""
     import sysconfig
     import torch
     from torch.utils import cpp_extension
-    newest = max(os.path.getmtime(p) for p in (EXT_SRC, os.path.join(os.path.dirname(HERE), "include", "mamba_hip.h")))
-    if not force and os.path.exists(EXT) and os.path.getmtime(EXT) >= newest:
-        return EXT
+    hdrs = [os.path.join(CSRC, "torch_common.h"), os.path.join(os.path.dirname(HERE), "include", "mamba_hip.h")]
     torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
     inc = [os.path.join(os.path.dirname(HERE), "include"), *cpp_extension.include_paths(), sysconfig.get_paths()["include"],
            "/opt/rocm/include"]
-    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
-           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_torch_ext",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           *[f"-I{d}" for d in inc], EXT_SRC, "-o", EXT,
+    cxx = os.environ.get("CXX", "g++")
+    flags = ["-O2", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-fvisibility=hidden",
+             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_torch_ext",
+             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *[f"-I{d}" for d in inc]]
+
+    def compile_one(src):
+        obj = src[:-4] + ".o"
+        newest = max(os.path.getmtime(p) for p in [src] + hdrs)
+        if not force and os.path.exists(obj) and os.path.getmtime(obj) >= newest:
+            return obj
+        r = subprocess.run([cxx, *flags, "-c", src, "-o", obj], capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"building the torch extension failed:\n{r.stdout}\n{r.stderr}")
+        return obj
+
+    srcs = ext_sources()
+    with ThreadPoolExecutor(max_workers=jobs or min(len(srcs), int(os.environ.get("MAX_JOBS", "8")))) as ex:
+        objs = list(ex.map(compile_one, srcs))
+    if not force and os.path.exists(EXT) and os.path.getmtime(EXT) >= max(os.path.getmtime(o) for o in objs):
+        return EXT
+    cmd = [cxx, "-shared", *objs, "-o", EXT,
            f"-L{torch_lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch", "-ltorch_python",
            f"-L{HERE}", "-l:libmamba_gfx950.so", "-Wl,-rpath,$ORIGIN", f"-Wl,-rpath,{torch_lib}"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f"building the torch extension failed:\n{r.stdout}\n{r.stderr}")
+        raise RuntimeError(f"linking the torch extension failed:\n{r.stdout}\n{r.stderr}")
     return EXT
 
 
@@ -77,7 +95,7 @@ def build(force=False, jobs=None):
     """Compiles every .hip under csrc/ for gfx950, links the shared library, then builds the torch
     extension module on top of it."""
     lib = build_lib(force, jobs)
-    build_torch_ext(force)
+    build_torch_ext(force, jobs)
     return lib
 
 

@@ -1,0 +1,95 @@
+// Shared by the translation units of the torch extension (torch_*.cpp; host code only).
+//
+// Every operator here serves the plain, valid case and DECLINES anything else by returning nullopt / None (wrong
+// shapes, dtypes that need a conversion first, CPU tensors): the Python host side then runs its own path, which does
+// the conversions and raises the reference's errors.  Both paths end in the same kernels.
+#pragma once
+#include <torch/extension.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <algorithm>
+#include <optional>
+#include <string>
+#include <tuple>
+#include <vector>
+
+#include "mamba_hip.h"
+
+namespace mamba_ext {
+
+using OptTensor = std::optional<at::Tensor>;
+using TensorList = std::vector<OptTensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+inline int dtype_code(at::ScalarType t) {
+  switch (t) {
+    case at::kFloat: return MAMBA_F32;
+    case at::kBFloat16: return MAMBA_BF16;
+    case at::kHalf: return MAMBA_F16;
+    default: return -1;
+  }
+}
+inline int dtype_code(const at::Tensor &t) { return dtype_code(t.scalar_type()); }
+
+inline bool on_device(const at::Tensor &t, const c10::Device &dev) { return t.is_cuda() && t.device() == dev; }
+inline bool on_device(const OptTensor &t, const c10::Device &dev) { return !t.has_value() || on_device(*t, dev); }
+
+inline void *stream_of(const c10::Device &dev) { return c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+
+inline void check_rc(int rc, const char *what) {
+  TORCH_CHECK(rc == MAMBA_OK, what, " failed: ", mamba_hip_strerror(rc), " (code ", rc, ")");
+}
+
+inline void *ptr(const OptTensor &t) { return t ? t->data_ptr() : nullptr; }
+
+// Whether autograd has to record a call: gradients are enabled and one of the tensors wants them.
+inline bool any_grad() { return false; }
+template <typename... Rest> bool any_grad(const at::Tensor &t, const Rest &...rest);
+template <typename... Rest> bool any_grad(const OptTensor &t, const Rest &...rest) {
+  return (t && t->defined() && t->requires_grad()) || any_grad(rest...);
+}
+template <typename... Rest> bool any_grad(const at::Tensor &t, const Rest &...rest) {
+  return (t.defined() && t.requires_grad()) || any_grad(rest...);
+}
+template <typename... Args> bool records(const Args &...args) { return at::GradMode::is_enabled() && any_grad(args...); }
+
+inline OptTensor opt(const at::Tensor &t) { return t.defined() ? OptTensor(t) : std::nullopt; }
+inline at::Tensor tensor_or_none(const OptTensor &t) { return t ? *t : at::Tensor(); }
+
+// The deterministic mode as mamba_amd/utils/determinism.py defines it; `set_deterministic_override` mirrors that
+// module's explicit setting (-1: none).
+bool deterministic();
+void set_deterministic_override(int value);
+
+// ---- convolution (torch_norm_conv.cpp)
+// x, out, dout, dx: (batch, dim, seqlen) views with unit stride along the positions or the channels.
+bool conv_params_ok(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx);
+void conv_fwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx, bool silu,
+              const at::Tensor &out);
+// -> (dweight, dbias) in the parameters' dtype; dx is written
+std::tuple<at::Tensor, OptTensor> conv_bwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias,
+                                           const at::Tensor &dout, const OptTensor &seq_idx, bool silu, const at::Tensor &dx);
+
+// ---- gated norm (torch_norm_conv.cpp): x, z, dy, out (rows, dim), unit channel stride
+struct GatedNorm {
+  int64_t group_size;
+  double eps;
+  bool norm_before_gate, is_rms;
+};
+bool gated_norm_ok(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &z, const GatedNorm &o);
+std::tuple<at::Tensor, OptTensor, at::Tensor> gated_norm_fwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias,
+                                                            const OptTensor &z, const GatedNorm &o);  // out, mean, rstd
+std::tuple<at::Tensor, at::Tensor, OptTensor, OptTensor> gated_norm_bwd(const at::Tensor &dy, const at::Tensor &x,
+                                                                       const at::Tensor &weight, const OptTensor &bias,
+                                                                       const OptTensor &mean, const at::Tensor &rstd,
+                                                                       const OptTensor &z, const OptTensor &dz_out,
+                                                                       const GatedNorm &o);  // dx, dweight, dbias, dz
+
+void bind_norm_conv(pybind11::module_ &m);
+void bind_scan(pybind11::module_ &m);
+void bind_ssd(pybind11::module_ &m);
+
+}  // namespace mamba_ext

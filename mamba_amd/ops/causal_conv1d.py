@@ -148,6 +148,12 @@ def causal_conv1d_fn(x, weight, bias=None, seq_idx=None, initial_states=None, re
         final_states_out: a tensor to receive them
     The streaming form runs the same kernel over the joined row (one extra copy of x)."""
     if initial_states is None and not return_final_states and final_states_out is None:
+        ext = _lib.torch_ext()
+        if ext is not None and activation in (None, "silu", "swish"):
+            # the same node in C++ (csrc/torch_norm_conv.cpp); None = a case for the code below
+            out = ext.causal_conv1d(x, weight, bias, seq_idx, activation is not None)
+            if out is not None:
+                return out
         return CausalConv1dFn.apply(x, weight, bias, seq_idx, activation)
     width = weight.shape[1]
     batch, dim, seqlen = x.shape

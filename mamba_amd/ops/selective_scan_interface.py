@@ -324,6 +324,12 @@ def selective_scan_fn(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta_
     considered in the backward pass (as in the reference, selective_scan_interface.py:118-124).
     """
     # (batches beyond the 65535 rows one launch's grid can index are served in slices inside the C entry points)
+    ext = _lib.torch_ext()
+    if ext is not None:
+        # the same node in C++ (csrc/torch_scan.cpp); None = a case for the code below
+        r = ext.selective_scan(u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus), bool(return_last_state))
+        if r is not None:
+            return r
     return SelectiveScanFn.apply(u, delta, A, B, C, D, z, delta_bias, delta_softplus, return_last_state)
 
 
@@ -544,6 +550,14 @@ def mamba_inner_fn(xz, conv1d_weight, conv1d_bias, x_proj_weight, delta_proj_wei
                    A, B=None, C=None, D=None, delta_bias=None, B_proj_bias=None, C_proj_bias=None,
                    delta_softplus=True, checkpoint_lvl=1, b_rms_weight=None, c_rms_weight=None, dt_rms_weight=None,
                    b_c_dt_rms_eps=1e-6):
+    ext = _lib.torch_ext()
+    if (ext is not None and B is None and C is None and B_proj_bias is None and C_proj_bias is None and b_rms_weight is None
+            and c_rms_weight is None and dt_rms_weight is None and checkpoint_lvl in (0, 1)):
+        # the same node in C++ (csrc/torch_scan.cpp); None = a case for the code below
+        r = ext.mamba_inner(xz, conv1d_weight, conv1d_bias, x_proj_weight, delta_proj_weight, out_proj_weight, out_proj_bias, A, D,
+                            delta_bias, bool(delta_softplus), checkpoint_lvl)
+        if r is not None:
+            return r
     return MambaInnerFn.apply(xz, conv1d_weight, conv1d_bias, x_proj_weight, delta_proj_weight, out_proj_weight,
                               out_proj_bias, A, B, C, D, delta_bias, B_proj_bias, C_proj_bias, delta_softplus,
                               checkpoint_lvl, b_rms_weight, c_rms_weight, dt_rms_weight, b_c_dt_rms_eps)

@@ -128,12 +128,7 @@ def _layer_norm_bwd(dy, x, weight, bias, eps, mean, rstd, z=None, group_size=Non
         p.nparts = nparts = _lib.load().norm_gated_bwd_nparts(p)
     nb = 2 if bias is not None else 1
     parts = torch.empty(nb, nparts, N, dtype=torch.float32, device=x.device)
-    sums = torch.empty(nb, N, dtype=torch.float32, device=x.device)
-    w32 = weight.float().contiguous()
-    b32 = bias.float().contiguous() if bias is not None else None
-    p = _lib.NormGatedParams()
-    _common(p, x, w32, b32, z, eps, group_size, norm_before_gate, is_rms_norm)
-    p.nparts = nparts
+    sums = torch.empty(nb, N, dtype=w.dtype, device=x.device)
     p.mean, p.rstd = _lib.ptr(mean), rstd.data_ptr()
     p.dy, p.dy_rs, p.dx, p.dx_rs = dy.data_ptr(), dy.stride(0), dx.data_ptr(), dx.stride(0)
     p.dz, p.dz_rs = _lib.ptr(dz), dz.stride(0) if dz is not None else 0
@@ -186,11 +181,17 @@ class LayerNormFn(torch.autograd.Function):
 
 
 def layernorm_fn(x, weight, bias, z=None, eps=1e-6, group_size=None, norm_before_gate=True, is_rms_norm=False):
+    ext = _lib.torch_ext()
+    if ext is not None:
+        # the same node in C++ (csrc/torch_norm_conv.cpp); None = a case for the code below
+        out = ext.norm_gated(x, weight, bias, z, eps, group_size, bool(norm_before_gate), bool(is_rms_norm))
+        if out is not None:
+            return out
     return LayerNormFn.apply(x, weight, bias, z, eps, group_size, norm_before_gate, is_rms_norm)
 
 
 def rmsnorm_fn(x, weight, bias, z=None, eps=1e-6, group_size=None, norm_before_gate=True):
-    return LayerNormFn.apply(x, weight, bias, z, eps, group_size, norm_before_gate, True)
+    return layernorm_fn(x, weight, bias, z, eps, group_size, norm_before_gate, True)
 
 
 class LayerNorm(torch.nn.Module):

@@ -376,6 +376,13 @@ def mamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_bia
         out: (batch, seqlen, nheads, headdim) [, final_states (batch, nheads, headdim, dstate) fp32]
     """
     # (more than 65535 (batch, head) pairs are served in slices of batch rows inside the C entry points)
+    ext = _lib.torch_ext()
+    if ext is not None and KEEP_FORWARD_STATE and not return_varlen_states:
+        # the same node in C++ (csrc/torch_ssd.cpp); None = a case for the code below
+        r = ext.chunk_scan(x, dt, A, B, C, int(chunk_size), D, z, dt_bias, initial_states, seq_idx, bool(dt_softplus),
+                           float(dt_limit[0]), float(dt_limit[1]), bool(return_final_states))
+        if r is not None:
+            return r
     return MambaChunkScanCombinedFn.apply(x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states, seq_idx,
                                           cu_seqlens, dt_softplus, dt_limit, return_final_states,
                                           return_varlen_states, state_dtype)
@@ -642,6 +649,15 @@ def mamba_split_conv1d_scan_combined(zxbcdt, conv1d_weight, conv1d_bias, dt_bias
         rmsnorm_weight: (dim,); outproj_weight: (out_dim, d_nonssm + dim); outproj_bias: (out_dim,)
         norm_before_gate: True computes RMSNorm(y) * silu(z), False RMSNorm(y * silu(z))
     Returns out, or (out, final_states) with return_final_states."""
+    ext = _lib.torch_ext()
+    if ext is not None and activation in (None, "silu", "swish"):
+        # the same node in C++ (csrc/torch_ssd.cpp); None = a case for the code below
+        r = ext.split_conv_scan(zxbcdt, conv1d_weight, conv1d_bias, dt_bias, A, D, int(chunk_size), initial_states, seq_idx,
+                                float(dt_limit[0]), float(dt_limit[1]), bool(return_final_states), activation is not None,
+                                rmsnorm_weight, float(rmsnorm_eps), outproj_weight, outproj_bias, headdim, int(ngroups),
+                                bool(norm_before_gate))
+        if r is not None:
+            return r
     return MambaSplitConv1dScanCombinedFn.apply(zxbcdt, conv1d_weight, conv1d_bias, dt_bias, A, D, chunk_size,
                                                 initial_states, seq_idx, dt_limit, return_final_states, activation,
                                                 rmsnorm_weight, rmsnorm_eps, outproj_weight, outproj_bias, headdim,

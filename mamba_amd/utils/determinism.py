@@ -8,6 +8,7 @@ bias gradients) with 64-bit integer atomics on terms scaled to a fixed point, in
 integer addition does not depend on the order of the adds, so every gradient repeats bit for bit.  Every
 other operator of the package is deterministic in either mode."""
 import os
+import sys
 
 import torch
 
@@ -26,6 +27,14 @@ def use_deterministic_mode():
 def set_deterministic_mode(value):
     global _deterministic_override
     _deterministic_override = value
+    ext = sys.modules.get("mamba_amd._torch_ext")
+    if ext is not None:
+        tell(ext)
+
+
+def tell(ext):
+    """Hands the explicit setting to the C++ host side, whose autograd nodes ask for the mode without the interpreter."""
+    ext.set_deterministic_override(-1 if _deterministic_override is None else int(bool(_deterministic_override)))
 
 
 def fixed_point_scale(*grads):

@@ -675,6 +675,35 @@ int norm_residual_bwd(const NormResidualParams *p, mamba_stream_t stream);
 /* The number of partial rows (nparts) that suits these rows, dim and dtypes on the current device. */
 int norm_residual_bwd_nparts(const NormResidualParams *p);
 
+/* -------------------------------------------------------------------------
+ * Small bf16 matrix products (the projections of a short mixer call, selective_scan_interface.py:230-383 and
+ * ssd_combined.py:868):
+ *   D[m][n] = sum_k A[m][k] B[n][k]   (+ bias[n])   (+ D[m][n] before, with accumulate)
+ * with fp32 sums, rounded once into D.  Either index of A and of B is contiguous (stride 1), any alignment; D's
+ * columns are contiguous.  Up to 4 independent products share a call.
+ * ------------------------------------------------------------------------- */
+typedef struct MambaGemm {
+  const void *A, *B;  /* bf16 */
+  const void *bias;   /* nullable, bf16, (N) */
+  void *D;
+  int64_t a_ms, a_ks, b_ns, b_ks, ldd; /* strides in elements */
+  int32_t M, N, K;
+  int32_t d_dtype;    /* MAMBA_BF16 or MAMBA_F32 */
+  int32_t accumulate;
+  int32_t nsplit;     /* parts of the sum over k, set by mamba_gemm_plan */
+} MambaGemm;
+/* Sets nsplit of each product and returns the fp32 elements of workspace the call needs (0: none), or an error. */
+int64_t mamba_gemm_plan(MambaGemm *g, int count);
+int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream_t stream);
+
+/* fp32 arrays rounded to bf16, up to 4 in one launch. */
+typedef struct MambaCast {
+  const float *src;
+  void *dst;
+  int64_t n;
+} MambaCast;
+int mamba_cast_bf16(const MambaCast *c, int count, mamba_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

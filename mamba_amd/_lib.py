@@ -114,6 +114,14 @@ class NormGatedParams(ctypes.Structure):
     )
 
 
+class MambaGemm(ctypes.Structure):
+    _fields_ = (
+        [(n, ctypes.c_void_p) for n in ("A", "B", "bias", "D")]
+        + [(n, c_i64) for n in ("a_ms", "a_ks", "b_ns", "b_ks", "ldd")]
+        + [(n, c_i32) for n in ("M", "N", "K", "d_dtype", "accumulate", "nsplit")]
+    )
+
+
 class NormResidualParams(ctypes.Structure):
     _fields_ = (
         [(n, c_i32) for n in ("rows", "dim", "dtype", "res_dtype", "is_rms", "nparts")]
@@ -197,6 +205,10 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = [ctypes.POINTER(NormGatedParams), c_vp]
         fn.restype = ctypes.c_int
+    lib.mamba_gemm_plan.argtypes = [ctypes.POINTER(MambaGemm), ctypes.c_int]
+    lib.mamba_gemm_plan.restype = ctypes.c_int64
+    lib.mamba_gemm.argtypes = [ctypes.POINTER(MambaGemm), ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]
+    lib.mamba_gemm.restype = ctypes.c_int
     for name, params in (("norm_gated_bwd_nparts", NormGatedParams), ("norm_residual_bwd_nparts", NormResidualParams),
                          ("causal_conv1d_bwd_nparts", CausalConvParams)):
         fn = getattr(lib, name)

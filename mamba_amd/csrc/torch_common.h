@@ -69,9 +69,20 @@ void set_deterministic_override(int value);
 bool conv_params_ok(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx);
 void conv_fwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx, bool silu,
               const at::Tensor &out);
-// -> (dweight, dbias) in the parameters' dtype; dx is written
+// -> (dweight, dbias) in the parameters' dtype (and shape); dx is written
 std::tuple<at::Tensor, OptTensor> conv_bwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias,
                                            const at::Tensor &dout, const OptTensor &seq_idx, bool silu, const at::Tensor &dx);
+
+// The same on memory by strides (batch, channel, position) of `like`'s dtype and device; weight (dim, [1,] width).
+struct ConvRows {
+  const void *p;
+  int64_t bs, cs, ls;
+};
+void conv_fwd(const at::Tensor &like, int64_t batch, int64_t dim, int64_t L, const ConvRows &x, const at::Tensor &weight,
+              const OptTensor &bias, const OptTensor &seq_idx, bool silu, const ConvRows &out);
+std::tuple<at::Tensor, OptTensor> conv_bwd(const at::Tensor &like, int64_t batch, int64_t dim, int64_t L, const ConvRows &x,
+                                           const at::Tensor &weight, const OptTensor &bias, const ConvRows &dout,
+                                           const OptTensor &seq_idx, bool silu, const ConvRows &dx);
 
 // ---- gated norm (torch_norm_conv.cpp): x, z, dy, out (rows, dim), unit channel stride
 struct GatedNorm {
@@ -88,6 +99,26 @@ std::tuple<at::Tensor, at::Tensor, OptTensor, OptTensor> gated_norm_bwd(const at
                                                                        const OptTensor &z, const OptTensor &dz_out,
                                                                        const GatedNorm &o);  // dx, dweight, dbias, dz
 
+// ---- matrix products (torch_gemm.cpp)
+struct Mat {  // one operand: element (row, k) at p[row * rs + k * ks], one of the strides 1; rows are those of the result, or its columns
+  const void *p;
+  int64_t rs, ks;
+};
+// Products D = A B^T of operands of `type` on raw memory.  Short ones are collected and leave together with run(); the
+// ones collected between two run() calls must not depend on each other, long ones run at once.
+class Products {
+ public:
+  Products(const at::TensorOptions &options, at::ScalarType type) : options_(options), type_(type) {}
+  Products &add(void *D, at::ScalarType d_type, int64_t ldd, int64_t M, int64_t N, int64_t K, Mat A, Mat B, bool accumulate = false,
+                const void *bias = nullptr);
+  void run();
+
+ private:
+  at::TensorOptions options_;
+  at::ScalarType type_;
+  MambaGemm g_[4];
+  int count_ = 0;
+};
 void bind_norm_conv(pybind11::module_ &m);
 void bind_scan(pybind11::module_ &m);
 void bind_ssd(pybind11::module_ &m);

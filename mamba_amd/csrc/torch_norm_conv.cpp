@@ -185,15 +185,15 @@ OptTensor norm_gated(const at::Tensor &x, const at::Tensor &weight, const OptTen
 }
 
 // ------------------------------------------------------------------ convolution
-void strides_of(const at::Tensor &t, int64_t &bs, int64_t &cs, int64_t &ls) { bs = t.stride(0), cs = t.stride(1), ls = t.stride(2); }
+ConvRows rows_at(const at::Tensor &t) { return {t.data_ptr(), t.stride(0), t.stride(1), t.stride(2)}; }
 
-void fill_conv(CausalConvParams &p, const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx,
-               bool silu) {
-  p.batch = (int32_t)x.size(0), p.dim = (int32_t)x.size(1), p.seqlen = (int32_t)x.size(2), p.width = (int32_t)weight.size(1);
-  p.dtype = dtype_code(x), p.silu = silu, p.weight_dtype = dtype_code(weight);
-  p.x = x.data_ptr(), p.weight = weight.data_ptr(), p.bias = ptr(bias);
+void fill_conv(CausalConvParams &p, int dtype, int64_t batch, int64_t dim, int64_t L, const ConvRows &x, const at::Tensor &weight,
+               const OptTensor &bias, const OptTensor &seq_idx, bool silu) {
+  p.batch = (int32_t)batch, p.dim = (int32_t)dim, p.seqlen = (int32_t)L, p.width = (int32_t)weight.size(-1);
+  p.dtype = dtype, p.silu = silu, p.weight_dtype = dtype_code(weight);
+  p.x = x.p, p.weight = weight.data_ptr(), p.bias = ptr(bias);
   p.seq_idx = seq_idx ? seq_idx->data_ptr<int32_t>() : nullptr;
-  strides_of(x, p.x_bs, p.x_cs, p.x_ls);
+  p.x_bs = x.bs, p.x_cs = x.cs, p.x_ls = x.ls;
 }
 
 at::Tensor like_layout(const at::Tensor &x) {
@@ -308,30 +308,37 @@ bool conv_params_ok(const at::Tensor &x, const at::Tensor &weight, const OptTens
 
 void conv_fwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx, bool silu,
               const at::Tensor &out) {
+  conv_fwd(x, x.size(0), x.size(1), x.size(2), rows_at(x), weight, bias, seq_idx, silu, rows_at(out));
+}
+void conv_fwd(const at::Tensor &like, int64_t batch, int64_t dim, int64_t L, const ConvRows &x, const at::Tensor &weight,
+              const OptTensor &bias, const OptTensor &seq_idx, bool silu, const ConvRows &out) {
   CausalConvParams p{};
-  fill_conv(p, x, weight, bias, seq_idx, silu);
-  p.out = out.data_ptr();
-  strides_of(out, p.out_bs, p.out_cs, p.out_ls);
-  c10::DeviceGuard guard(x.device());
-  check_rc(::causal_conv1d_fwd(&p, stream_of(x.device())), "causal_conv1d_fwd");
+  fill_conv(p, dtype_code(like), batch, dim, L, x, weight, bias, seq_idx, silu);
+  p.out = const_cast<void *>(out.p), p.out_bs = out.bs, p.out_cs = out.cs, p.out_ls = out.ls;
+  c10::DeviceGuard guard(like.device());
+  check_rc(::causal_conv1d_fwd(&p, stream_of(like.device())), "causal_conv1d_fwd");
 }
 
 std::tuple<at::Tensor, OptTensor> conv_bwd(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias,
                                            const at::Tensor &dout, const OptTensor &seq_idx, bool silu, const at::Tensor &dx) {
-  c10::DeviceGuard guard(x.device());
+  return conv_bwd(x, x.size(0), x.size(1), x.size(2), rows_at(x), weight, bias, rows_at(dout), seq_idx, silu, rows_at(dx));
+}
+std::tuple<at::Tensor, OptTensor> conv_bwd(const at::Tensor &like, int64_t batch, int64_t dim, int64_t L, const ConvRows &x,
+                                           const at::Tensor &weight, const OptTensor &bias, const ConvRows &dout,
+                                           const OptTensor &seq_idx, bool silu, const ConvRows &dx) {
+  c10::DeviceGuard guard(like.device());
   CausalConvParams p{};
-  fill_conv(p, x, weight, bias, seq_idx, silu);
-  at::Tensor dw = at::empty_like(weight);
+  fill_conv(p, dtype_code(like), batch, dim, L, x, weight, bias, seq_idx, silu);
+  at::Tensor dw = at::empty(weight.sizes(), weight.options());
   OptTensor db;
-  if (bias) db = at::empty_like(*bias);
-  p.dout = dout.data_ptr(), p.dx = dx.data_ptr(), p.dweight = dw.data_ptr(), p.dbias = ptr(db);
-  strides_of(dout, p.dout_bs, p.dout_cs, p.dout_ls);
-  strides_of(dx, p.dx_bs, p.dx_cs, p.dx_ls);
+  if (bias) db = at::empty(bias->sizes(), bias->options());
+  p.dout = dout.p, p.dx = const_cast<void *>(dx.p), p.dweight = dw.data_ptr(), p.dbias = ptr(db);
+  p.dout_bs = dout.bs, p.dout_cs = dout.cs, p.dout_ls = dout.ls, p.dx_bs = dx.bs, p.dx_cs = dx.cs, p.dx_ls = dx.ls;
   const int nparts = causal_conv1d_bwd_nparts(&p);
   if (nparts <= 0) check_rc(nparts ? nparts : -1, "causal_conv1d_bwd_nparts");
-  at::Tensor part = at::empty({nparts, x.size(1), 5}, x.options().dtype(at::kFloat));
+  at::Tensor part = at::empty({nparts * dim * 5}, like.options().dtype(at::kFloat));
   p.dw_part = part.data_ptr<float>();
-  check_rc(::causal_conv1d_bwd(&p, stream_of(x.device())), "causal_conv1d_bwd");
+  check_rc(::causal_conv1d_bwd(&p, stream_of(like.device())), "causal_conv1d_bwd");
   return {dw, db};
 }
 

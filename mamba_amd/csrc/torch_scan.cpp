@@ -56,27 +56,58 @@ bool fill_scan(MambaScanParams &p, const at::Tensor &u, const at::Tensor &delta,
   return true;
 }
 
-// The number of segments of the sequence and their workspace, where the problem is split.
-at::Tensor split_sequence(MambaScanParams &p, const at::Tensor &u, bool backward) {
-  p.nseg = std::max(1, mamba1_scan_segments(&p, backward ? 1 : 0));
-  if (p.nseg == 1) return at::Tensor();
-  at::Tensor ws = at::empty({(int64_t)p.batch * p.nseg * p.dim * (p.dstate + 2)}, u.options().dtype(at::kFloat));
-  p.seg_ws = ws.data_ptr<float>();
-  return ws;
+// The forward call on filled parameters, p.out included -> ckpt.  One allocation holds the workspace of a sequence that
+// goes in segments.
+at::Tensor run_scan_fwd(MambaScanParams &p, const c10::Device &dev) {
+  const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
+  const int64_t tile = mamba_hip_query(MAMBA_Q_SCAN_TILE), ntiles = (p.seqlen + tile - 1) / tile;
+  at::Tensor ckpt = at::empty({p.batch, p.dim, ntiles, p.dstate}, f32), ws;
+  p.ckpt = ckpt.data_ptr<float>();
+  p.nseg = std::max(1, mamba1_scan_segments(&p, 0));
+  if (p.nseg > 1) {
+    ws = at::empty({(int64_t)p.batch * p.nseg * p.dim * (p.dstate + 2)}, f32);
+    p.seg_ws = ws.data_ptr<float>();
+  }
+  check_rc(mamba1_scan_fwd(&p, stream_of(dev)), "mamba1_scan_fwd");
+  return ckpt;
+}
+
+// The backward call on filled parameters, the operands' gradients included (dB / dC of per-position B / C; constant
+// ones come back as partials) -> the sums dA (dim, dstate), dD and ddelta_bias (dim) in one array, one after the other.
+struct ScanSums {
+  at::Tensor sums, dB_parts, dC_parts;
+};
+ScanSums run_scan_bwd(MambaScanParams &p, const c10::Device &dev) {
+  const auto f32 = at::TensorOptions().dtype(at::kFloat).device(dev);
+  const int64_t batch = p.batch, dim = p.dim, N = p.dstate;
+  p.nseg = std::max(1, mamba1_scan_segments(&p, 1));
+  const int64_t nseg = p.nseg, nparts = mamba1_scan_bwd_nparts(&p);
+  if (nparts <= 0) check_rc(nparts ? (int)nparts : -1, "mamba1_scan_bwd_nparts");
+  const int64_t rows = batch * nseg, bc = batch * p.ngroups * nparts * N * p.seqlen;
+  auto padded = [](int64_t n) { return (n + 63) / 64 * 64; };
+  const int64_t seg = nseg > 1 ? padded(rows * dim * (N + 2)) : 0, part = padded(rows * dim * (N + 2));
+  ScanSums r;
+  r.sums = at::empty({dim * (N + 2)}, f32);
+  at::Tensor ws = at::empty({seg + part + 2 * padded(bc)}, f32);
+  float *base = ws.data_ptr<float>();
+  if (nseg > 1) p.seg_ws = base;
+  base += seg;
+  p.dA_part = base, p.dD_part = base + rows * dim * N, p.ddelta_bias_part = p.dD_part + rows * dim;
+  p.dA = r.sums.data_ptr<float>(), p.dD = p.dA + dim * N, p.ddelta_bias = p.dD + dim;
+  p.dB32 = base + part, p.dC32 = p.dB32 + padded(bc);
+  if (p.bc_const & 1) r.dB_parts = at::empty({rows, dim, N}, f32), p.dB32 = r.dB_parts.data_ptr<float>();
+  if (p.bc_const & 2) r.dC_parts = at::empty({rows, dim, N}, f32), p.dC32 = r.dC_parts.data_ptr<float>();
+  check_rc(mamba1_scan_bwd(&p, stream_of(dev)), "mamba1_scan_bwd");
+  return r;
 }
 
 // selective_scan_cuda.fwd (selective_scan.cpp:226) on filled parameters -> (out, ckpt); real A only.
 std::tuple<at::Tensor, at::Tensor> scan_fwd(MambaScanParams &p, const at::Tensor &u, const at::Tensor &delta) {
   const c10::Device dev = u.device();
   c10::DeviceGuard guard(dev);
-  const int64_t tile = mamba_hip_query(MAMBA_Q_SCAN_TILE), ntiles = (p.seqlen + tile - 1) / tile;
   at::Tensor out = at::empty_like(delta);
-  at::Tensor ckpt = at::empty({p.batch, p.dim, ntiles, p.dstate}, u.options().dtype(at::kFloat));
   p.out = out.data_ptr(), p.out_bs = out.stride(0), p.out_ds = out.stride(1);
-  p.ckpt = ckpt.data_ptr<float>();
-  const at::Tensor ws = split_sequence(p, u, false);
-  check_rc(mamba1_scan_fwd(&p, stream_of(dev)), "mamba1_scan_fwd");
-  return {out, ckpt};
+  return {out, run_scan_fwd(p, dev)};
 }
 
 std::optional<std::tuple<at::Tensor, at::Tensor>> scan_fwd_fast(const at::Tensor &u, const at::Tensor &delta,
@@ -90,41 +121,23 @@ std::optional<std::tuple<at::Tensor, at::Tensor>> scan_fwd_fast(const at::Tensor
 }
 
 // selective_scan_cuda.bwd (selective_scan.cpp:338) on filled parameters
-// -> [du, ddelta, dA, dB, dC, dD, ddelta_bias, dz, out_z].  dB_out / dC_out: where the gradients of per-position B / C
-// are written, (batch, ngroups, dstate, seqlen) views with unit position stride (allocated here when absent).
+// -> [du, ddelta, dA, dB, dC, dD, ddelta_bias, dz, out_z].
 TensorList scan_bwd(MambaScanParams &p, const at::Tensor &u, const at::Tensor &delta, const at::Tensor &B, const at::Tensor &C,
                     const OptTensor &D, const OptTensor &z, const OptTensor &delta_bias, const at::Tensor &dout,
-                    const at::Tensor &ckpt, const OptTensor &dz_in, bool recompute_out_z, const OptTensor &dB_out,
-                    const OptTensor &dC_out) {
+                    const at::Tensor &ckpt, const OptTensor &dz_in, bool recompute_out_z) {
   const c10::Device dev = u.device();
-  const int64_t batch = p.batch, dim = p.dim, L = p.seqlen, N = p.dstate, G = p.ngroups;
   c10::DeviceGuard guard(dev);
-  const auto f32 = u.options().dtype(at::kFloat);
-  const at::Tensor ws = split_sequence(p, u, true);
-  const int64_t nseg = p.nseg, nparts = mamba1_scan_bwd_nparts(&p);
-  if (nparts <= 0) check_rc(nparts ? (int)nparts : -1, "mamba1_scan_bwd_nparts");
+  const int64_t dim = p.dim, N = p.dstate;
   at::Tensor du = at::empty_like(u), ddelta = at::empty_like(delta);
-  auto operand = [&](const at::Tensor &t, const OptTensor &given, at::Tensor &part, OptTensor &grad, int64_t &bs, int64_t &gs,
-                     int64_t &ns) {
-    if (t.dim() == 2) {
-      part = at::empty({batch * nseg, dim, N}, f32);
-      return;
-    }
-    part = at::empty({batch, G, nparts, N, L}, f32);
-    grad = given ? *given : at::empty({batch, G, N, L}, t.options());
-    bs = grad->stride(0), gs = grad->stride(1), ns = grad->stride(2);
-  };
-  at::Tensor dB32, dC32;
   OptTensor dB, dC, dz, out_z;
-  operand(B, dB_out, dB32, dB, p.dB_bs, p.dB_gs, p.dB_ns);
-  operand(C, dC_out, dC32, dC, p.dC_bs, p.dC_gs, p.dC_ns);
-  // dA, dD and ddelta_bias: the partials of every (batch, segment) and, behind them, their sums
-  at::Tensor part = at::empty({(batch * nseg + 1) * dim * (N + 2)}, f32);
-  float *base = part.data_ptr<float>();
-  const int64_t rows = batch * nseg;
-  p.dA_part = base, p.dD_part = base + rows * dim * N, p.ddelta_bias_part = p.dD_part + rows * dim;
-  at::Tensor sums = part.narrow(0, rows * dim * (N + 2), dim * (N + 2));
-  p.dA = base + rows * dim * (N + 2), p.dD = p.dA + dim * N, p.ddelta_bias = p.dD + dim;
+  if (B.dim() == 4) {
+    dB = at::empty({p.batch, p.ngroups, N, p.seqlen}, B.options());
+    p.dB = ptr(dB), p.dB_bs = dB->stride(0), p.dB_gs = dB->stride(1), p.dB_ns = dB->stride(2);
+  }
+  if (C.dim() == 4) {
+    dC = at::empty({p.batch, p.ngroups, N, p.seqlen}, C.options());
+    p.dC = ptr(dC), p.dC_bs = dC->stride(0), p.dC_gs = dC->stride(1), p.dC_ns = dC->stride(2);
+  }
   if (z) {
     dz = dz_in ? *dz_in : at::empty_like(*z);
     if (recompute_out_z) out_z = at::empty_like(u);
@@ -132,19 +145,17 @@ TensorList scan_bwd(MambaScanParams &p, const at::Tensor &u, const at::Tensor &d
   p.ckpt = ckpt.data_ptr<float>();
   p.dout = dout.data_ptr(), p.du = du.data_ptr(), p.ddelta = ddelta.data_ptr();
   p.dz = ptr(dz), p.out_z = ptr(out_z);
-  p.dB32 = dB32.data_ptr<float>(), p.dC32 = dC32.data_ptr<float>();
-  p.dB = ptr(dB), p.dC = ptr(dC);
   p.dout_bs = dout.stride(0), p.dout_ds = dout.stride(1), p.du_bs = du.stride(0), p.du_ds = du.stride(1);
   p.ddelta_bs = ddelta.stride(0), p.ddelta_ds = ddelta.stride(1);
   if (dz) p.dz_bs = dz->stride(0), p.dz_ds = dz->stride(1);
   if (out_z) p.outz_bs = out_z->stride(0), p.outz_ds = out_z->stride(1);
-  check_rc(mamba1_scan_bwd(&p, stream_of(dev)), "mamba1_scan_bwd");
+  const ScanSums q = run_scan_bwd(p, dev);
   TensorList r(9);
-  r[0] = du, r[1] = ddelta, r[2] = sums.narrow(0, 0, dim * N).view({dim, N});
-  r[3] = B.dim() == 2 ? OptTensor(dB32.sum(0)) : dB;
-  r[4] = C.dim() == 2 ? OptTensor(dC32.sum(0)) : dC;
-  if (D) r[5] = sums.narrow(0, dim * N, dim);
-  if (delta_bias) r[6] = sums.narrow(0, dim * (N + 1), dim);
+  r[0] = du, r[1] = ddelta, r[2] = q.sums.as_strided({dim, N}, {N, 1}, 0);
+  r[3] = B.dim() == 2 ? OptTensor(q.dB_parts.sum(0)) : dB;
+  r[4] = C.dim() == 2 ? OptTensor(q.dC_parts.sum(0)) : dC;
+  if (D) r[5] = q.sums.as_strided({dim}, {1}, dim * N);
+  if (delta_bias) r[6] = q.sums.as_strided({dim}, {1}, dim * (N + 1));
   r[7] = dz, r[8] = out_z;
   return r;
 }
@@ -166,7 +177,7 @@ std::optional<TensorList> scan_bwd_fast(const at::Tensor &u, const at::Tensor &d
   if (!rows_ok(dout, p.batch, p.dim, p.seqlen, u.scalar_type())) return std::nullopt;
   if (dz_in && (!z || !rows_ok(*dz_in, p.batch, p.dim, p.seqlen, u.scalar_type()))) return std::nullopt;
   if (!ckpt_ok(ckpt, p)) return std::nullopt;
-  return scan_bwd(p, u, delta, B, C, D, z, delta_bias, dout, ckpt, dz_in, recompute_out_z, std::nullopt, std::nullopt);
+  return scan_bwd(p, u, delta, B, C, D, z, delta_bias, dout, ckpt, dz_in, recompute_out_z);
 }
 
 // ------------------------------------------------------------------ selective_scan_fn
@@ -211,7 +222,7 @@ struct ScanFn : torch::autograd::Function<ScanFn> {
     const at::Tensor dout = grads[0].defined() ? unit_last(grads[0]) : at::zeros(s[0].sizes(), s[0].options());
     MambaScanParams p{};
     TORCH_CHECK(fill_scan(p, s[0], s[1], s[2], s[3], s[4], D, z, bias, ctx->saved_data["softplus"].toBool()), "selective_scan: arguments");
-    const TensorList r = scan_bwd(p, s[0], s[1], s[3], s[4], D, z, bias, dout, s[8], std::nullopt, false, std::nullopt, std::nullopt);
+    const TensorList r = scan_bwd(p, s[0], s[1], s[3], s[4], D, z, bias, dout, s[8], std::nullopt, false);
     const std::vector<int64_t> squeeze = ctx->saved_data["squeeze"].toIntVector();
     variable_list g(10);
     g[0] = *r[0], g[1] = *r[1], g[2] = *r[2];
@@ -243,82 +254,150 @@ pybind11::object selective_scan(const at::Tensor &u, const at::Tensor &delta, co
 
 // ------------------------------------------------------------------ mamba_inner_fn
 // conv1d + SiLU -> x_proj -> dt_proj -> scan -> out_proj (selective_scan_interface.py:196-383) for a real A and B, C
-// and delta from x_proj.  Every (batch, dim, seqlen) intermediate lives in memory as (dim, batch, seqlen), so that the
+// and delta from x_proj.  Every (batch, dim, seqlen) intermediate lies in memory as (dim, batch, seqlen), so that the
 // projections see (dim, batch * seqlen) matrices; x_proj's output is formed as (rank + 2 dstate, batch * seqlen), whose
-// row blocks are delta's factor and the scan's B and C as they lie (no transposing copies, forward or backward).
-at::Tensor channel_major(const at::Tensor &m, int64_t batch, int64_t L) {  // (dim, batch * L) -> its (batch, dim, L) view
-  return m.view({m.size(0), batch, L}).permute({1, 0, 2});
-}
-at::Tensor bc_rows(const at::Tensor &x_dbl, int64_t row, int64_t n, int64_t batch, int64_t L) {
-  return x_dbl.narrow(0, row, n).view({n, batch, L}).permute({1, 0, 2}).unsqueeze(1);
+// row blocks are delta's factor and the scan's B and C as they lie (no transposing copies, forward or backward).  A
+// short call takes little GPU time, so this works on pointers and strides, keeps what it saves in few allocations and
+// hands products that do not depend on each other over together.
+struct InnerDims {
+  int64_t batch, d, L, N, R, E, rows, BL;  // E: out_proj's rows; rows = R + 2 N; BL = batch * L
+};
+int64_t aligned8(int64_t n) { return (n + 7) / 8 * 8; }
+
+// the scan's operands inside xz, the activations (conv, delta) and x_dbl, all of one dtype
+void fill_inner_scan(MambaScanParams &p, const InnerDims &q, const at::Tensor &xz, char *conv, char *delta, char *x_dbl,
+                     const at::Tensor &A, const OptTensor &D, const OptTensor &delta_bias, bool delta_softplus) {
+  const int64_t es = xz.element_size();
+  p.batch = (int32_t)q.batch, p.dim = (int32_t)q.d, p.seqlen = (int32_t)q.L, p.dstate = (int32_t)q.N, p.ngroups = 1;
+  p.dtype = dtype_code(xz), p.delta_softplus = delta_softplus ? 1 : 0;
+  p.u = conv, p.u_bs = q.L, p.u_ds = q.BL;
+  p.delta = delta, p.delta_bs = q.L, p.delta_ds = q.BL;
+  p.z = static_cast<char *>(xz.data_ptr()) + q.d * xz.stride(1) * es, p.z_bs = xz.stride(0), p.z_ds = xz.stride(1);
+  p.B = x_dbl + q.R * q.BL * es, p.B_bs = q.L, p.B_gs = 0, p.B_ns = q.BL;
+  p.C = x_dbl + (q.R + q.N) * q.BL * es, p.C_bs = q.L, p.C_gs = 0, p.C_ns = q.BL;
+  p.A = A.data_ptr(), p.D = ptr(D), p.delta_bias = ptr(delta_bias);
 }
 
+// conv (d, BL) and delta (d, BL) from xz and x_dbl; x_dbl is formed first when `with_x_dbl`
+void inner_activations(const InnerDims &q, const at::Tensor &xz, const at::Tensor &conv_w, const OptTensor &conv_bias,
+                       const void *xp, const void *dp, char *conv, char *delta, char *x_dbl, bool with_x_dbl) {
+  const at::ScalarType ty = xz.scalar_type();
+  conv_fwd(xz, q.batch, q.d, q.L, {xz.data_ptr(), xz.stride(0), xz.stride(1), 1}, conv_w, conv_bias, std::nullopt, true,
+           {conv, q.L, q.BL, 1});
+  Products m(xz.options(), ty);
+  if (with_x_dbl) m.add(x_dbl, ty, q.BL, q.rows, q.BL, q.d, {xp, q.d, 1}, {conv, 1, q.BL}).run();
+  m.add(delta, ty, q.BL, q.d, q.BL, q.R, {dp, q.R, 1}, {x_dbl, 1, q.BL}).run();
+}
 
 struct InnerFn : torch::autograd::Function<InnerFn> {
-  static at::Tensor forward(AutogradContext *ctx, const at::Tensor &xz, const at::Tensor &conv_weight, const OptTensor &conv_bias,
+  static at::Tensor forward(AutogradContext *ctx, const at::Tensor &xz, const at::Tensor &conv_w, const OptTensor &conv_bias,
                             const at::Tensor &x_proj, const at::Tensor &dt_proj, const at::Tensor &out_proj,
                             const OptTensor &out_bias, const at::Tensor &A, const OptTensor &D, const OptTensor &delta_bias,
                             bool delta_softplus, int64_t checkpoint_lvl, at::ScalarType compute) {
-    const int64_t batch = xz.size(0), d = xz.size(1) / 2, L = xz.size(2), N = A.size(1), R = dt_proj.size(1);
-    const at::Tensor conv_w = conv_weight.squeeze(1), Ac = A.contiguous();
-    const at::Tensor xp = x_proj.to(compute), dp = dt_proj.to(compute), op = out_proj.to(compute);
-    const at::Tensor x = xz.narrow(1, 0, d), z = xz.narrow(1, d, d);
-    at::Tensor conv = at::empty({d, batch * L}, xz.options());
-    conv_fwd(x, conv_w, conv_bias, std::nullopt, true, channel_major(conv, batch, L));
-    const at::Tensor x_dbl = at::mm(xp, conv);                                 // (rank + 2 n, b l)
-    const at::Tensor delta = at::mm(dp, x_dbl.narrow(0, 0, R));                // (dim, b l)
+    InnerDims q;
+    q.batch = xz.size(0), q.d = xz.size(1) / 2, q.L = xz.size(2), q.N = A.size(1), q.R = dt_proj.size(1), q.E = out_proj.size(0);
+    q.rows = q.R + 2 * q.N, q.BL = q.batch * q.L;
+    const int64_t es = xz.element_size();
+    const at::Tensor Ac = A.contiguous();
+    // the weights in the compute dtype: three pieces of one array where they are converted
+    const void *xp, *dp, *op;
+    at::Tensor w, xpc, dpc, opc;
+    if (compute == at::kBFloat16 && x_proj.scalar_type() == at::kFloat && dt_proj.scalar_type() == at::kFloat &&
+        out_proj.scalar_type() == at::kFloat && x_proj.is_contiguous() && dt_proj.is_contiguous() && out_proj.is_contiguous()) {
+      const int64_t nx = aligned8(q.rows * q.d), nd = aligned8(q.d * q.R), no = q.E * q.d;
+      w = at::empty({nx + nd + no}, xz.options());
+      char *base = static_cast<char *>(w.data_ptr());
+      const MambaCast c[3] = {{x_proj.data_ptr<float>(), base, q.rows * q.d}, {dt_proj.data_ptr<float>(), base + 2 * nx, q.d * q.R},
+                              {out_proj.data_ptr<float>(), base + 2 * (nx + nd), no}};
+      check_rc(mamba_cast_bf16(c, 3, stream_of(xz.device())), "mamba_cast_bf16");
+      xp = c[0].dst, dp = c[1].dst, op = c[2].dst;
+    } else {
+      xpc = x_proj.to(compute).contiguous(), dpc = dt_proj.to(compute).contiguous(), opc = out_proj.to(compute).contiguous();
+      xp = xpc.data_ptr(), dp = dpc.data_ptr(), op = opc.data_ptr();
+    }
+    at::Tensor x_dbl = at::empty({q.rows, q.BL}, xz.options()), act = at::empty({2 * aligned8(q.d * q.BL)}, xz.options());
+    at::Tensor out_z = at::empty({q.d, q.BL}, xz.options()), out = at::empty({q.batch, q.L, q.E}, xz.options());
+    char *conv = static_cast<char *>(act.data_ptr()), *delta = conv + aligned8(q.d * q.BL) * es;
+    char *xd = static_cast<char *>(x_dbl.data_ptr());
+    inner_activations(q, xz, conv_w, conv_bias, xp, dp, conv, delta, xd, true);
     MambaScanParams p{};
-    const at::Tensor u3 = channel_major(conv, batch, L), d3 = channel_major(delta, batch, L);
-    TORCH_CHECK(fill_scan(p, u3, d3, Ac, bc_rows(x_dbl, R, N, batch, L), bc_rows(x_dbl, R + N, N, batch, L), D, z, delta_bias,
-                          delta_softplus),
-                "mamba_inner_fn: arguments");
-    auto [out_z, ckpt] = scan_fwd(p, u3, d3);  // out_z has delta's layout
-    const bool keep = checkpoint_lvl == 0;     // else conv and delta are formed again in the backward pass
-    ctx->save_for_backward({xz, conv_w, tensor_or_none(conv_bias), x_dbl, xp, dp, op, keep ? conv : at::Tensor(),
-                            keep ? delta : at::Tensor(), Ac, tensor_or_none(D), tensor_or_none(delta_bias), ckpt});
-    ctx->saved_data["softplus"] = delta_softplus;
-    ctx->saved_data["out_bias"] = out_bias.has_value();
-    const at::Tensor rows = out_z.permute({1, 0, 2}).reshape({d, batch * L}).t();
-    return at::linear(rows, op, out_bias ? OptTensor(out_bias->to(compute)) : std::nullopt).view({batch, L, -1});
+    fill_inner_scan(p, q, xz, conv, delta, xd, Ac, D, delta_bias, delta_softplus);
+    p.out = out_z.data_ptr(), p.out_bs = q.L, p.out_ds = q.BL;
+    const at::Tensor ckpt = run_scan_fwd(p, xz.device());
+    const at::Tensor bias = out_bias ? out_bias->to(compute).contiguous() : at::Tensor();
+    Products(xz.options(), compute)
+        .add(out.data_ptr(), compute, q.E, q.BL, q.E, q.d, {out_z.data_ptr(), 1, q.BL}, {op, q.d, 1}, false, out_bias ? bias.data_ptr() : nullptr)
+        .run();
+    // with checkpoint_lvl 1 conv and delta are formed again in the backward pass
+    ctx->save_for_backward({xz, conv_w, tensor_or_none(conv_bias), x_dbl, w, xpc, dpc, opc, checkpoint_lvl == 0 ? act : at::Tensor(),
+                            Ac, tensor_or_none(D), tensor_or_none(delta_bias), ckpt});
+    ctx->saved_data["o"] = std::vector<int64_t>{q.R, q.E, delta_softplus, out_bias.has_value(), (int64_t)x_proj.scalar_type(),
+                                                (int64_t)dt_proj.scalar_type(), (int64_t)out_proj.scalar_type(),
+                                                out_bias ? (int64_t)out_bias->scalar_type() : 0};
+    return out;
   }
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
-    const at::Tensor &xz = s[0], &conv_w = s[1], &x_dbl = s[3], &xp = s[4], &dp = s[5], &op = s[6], &Ac = s[9], &ckpt = s[12];
+    const std::vector<int64_t> o = ctx->saved_data["o"].toIntVector();
+    const at::Tensor &xz = s[0], &conv_w = s[1], &x_dbl = s[3], &w = s[4], &Ac = s[9], &ckpt = s[12];
     const OptTensor conv_bias = opt(s[2]), D = opt(s[10]), delta_bias = opt(s[11]);
-    const int64_t batch = xz.size(0), d = xz.size(1) / 2, L = xz.size(2), N = Ac.size(1), R = dp.size(1);
+    InnerDims q;
+    q.batch = xz.size(0), q.d = xz.size(1) / 2, q.L = xz.size(2), q.N = Ac.size(1), q.R = o[0], q.E = o[1];
+    q.rows = q.R + 2 * q.N, q.BL = q.batch * q.L;
+    const int64_t es = xz.element_size(), part = aligned8(q.d * q.BL) * es, xs = xz.stride(1);
+    const at::ScalarType ty = xz.scalar_type();
     c10::DeviceGuard guard(xz.device());
-    const at::Tensor x = xz.narrow(1, 0, d), z = xz.narrow(1, d, d);
-    at::Tensor conv = s[7], delta = s[8];
-    if (!conv.defined()) {
-      conv = at::empty({d, batch * L}, xz.options());
-      conv_fwd(x, conv_w, conv_bias, std::nullopt, true, channel_major(conv, batch, L));
-      delta = at::mm(dp, x_dbl.narrow(0, 0, R));
+    const char *xp, *dp, *op;
+    if (w.defined()) {
+      xp = static_cast<const char *>(w.data_ptr()), dp = xp + 2 * aligned8(q.rows * q.d), op = dp + 2 * aligned8(q.d * q.R);
+    } else {
+      xp = static_cast<const char *>(s[5].data_ptr()), dp = static_cast<const char *>(s[6].data_ptr()), op = static_cast<const char *>(s[7].data_ptr());
     }
-    at::Tensor dxz = at::empty_like(xz);
-    const at::Tensor dx = dxz.narrow(1, 0, d), dz = dxz.narrow(1, d, d);
-    const at::Tensor dout = grads[0].reshape({batch * L, -1}).to(op.scalar_type());      // (b l) x e
-    const at::Tensor dy = at::mm(op.t(), dout.t());                                      // (dim, b l)
-    at::Tensor dx_dbl = at::empty_like(x_dbl);
+    char *xd = static_cast<char *>(x_dbl.data_ptr());
+    at::Tensor act = s[8];
+    if (!act.defined()) {
+      act = at::empty({2 * aligned8(q.d * q.BL)}, xz.options());
+      char *c = static_cast<char *>(act.data_ptr());
+      inner_activations(q, xz, conv_w, conv_bias, xp, dp, c, c + part, xd, false);
+    }
+    char *conv = static_cast<char *>(act.data_ptr()), *delta = conv + part;
+    at::Tensor dxz = at::empty_like(xz);  // in xz's layout
+    if (dxz.stride(2) != 1) dxz = at::empty(xz.sizes(), xz.options());
+    at::Tensor tmp = at::empty({4 * (part / es)}, xz.options());
+    at::Tensor dx_dbl = at::empty({q.rows, q.BL}, xz.options());
+    char *dy = static_cast<char *>(tmp.data_ptr()), *dconv = dy + part, *ddelta = dconv + part, *out_z = ddelta + part;
+    char *dxd = static_cast<char *>(dx_dbl.data_ptr()), *dx = static_cast<char *>(dxz.data_ptr());
+    const at::Tensor dout = grads[0].scalar_type() == ty && grads[0].is_contiguous() ? grads[0] : grads[0].to(ty).contiguous();  // (b l) x e
+    const char *g_out = static_cast<const char *>(dout.data_ptr());
+    Products m(xz.options(), ty);
+    m.add(dy, ty, q.BL, q.d, q.BL, q.E, {op, 1, q.d}, {g_out, q.E, 1}).run();  // (dim, b l)
     MambaScanParams p{};
-    const at::Tensor u3 = channel_major(conv, batch, L), d3 = channel_major(delta, batch, L);
-    const at::Tensor B = bc_rows(x_dbl, R, N, batch, L), C = bc_rows(x_dbl, R + N, N, batch, L);
-    TORCH_CHECK(fill_scan(p, u3, d3, Ac, B, C, D, z, delta_bias, ctx->saved_data["softplus"].toBool()), "mamba_inner_fn: arguments");
-    const TensorList r = scan_bwd(p, u3, d3, B, C, D, z, delta_bias, channel_major(dy, batch, L), ckpt, dz, true,
-                                  bc_rows(dx_dbl, R, N, batch, L), bc_rows(dx_dbl, R + N, N, batch, L));
-    auto matrix = [&](const at::Tensor &t) { return t.permute({1, 0, 2}).reshape({d, batch * L}); };
-    at::Tensor dconv = matrix(*r[0]);
-    const at::Tensor ddelta = matrix(*r[1]), out_z = matrix(*r[8]);
-    const at::Tensor dop = at::mm(dout.t(), out_z.t());
-    const at::Tensor ddp = at::mm(ddelta, x_dbl.narrow(0, 0, R).t());
-    at::Tensor dt_rows = dx_dbl.narrow(0, 0, R);
-    at::mm_out(dt_rows, dp.t(), ddelta);
-    const at::Tensor dxp = at::mm(dx_dbl, conv.t());
-    dconv.addmm_(xp.t(), dx_dbl);  // the scan's own du buffer: the x_proj path is added in place
-    auto [dcw, dcb] = conv_bwd(x, conv_w, conv_bias, channel_major(dconv, batch, L), std::nullopt, true, dx);
+    fill_inner_scan(p, q, xz, conv, delta, xd, Ac, D, delta_bias, o[2] != 0);
+    p.ckpt = ckpt.data_ptr<float>();
+    p.dout = dy, p.dout_bs = q.L, p.dout_ds = q.BL, p.du = dconv, p.du_bs = q.L, p.du_ds = q.BL;
+    p.ddelta = ddelta, p.ddelta_bs = q.L, p.ddelta_ds = q.BL, p.out_z = out_z, p.outz_bs = q.L, p.outz_ds = q.BL;
+    p.dz = dx + q.d * dxz.stride(1) * es, p.dz_bs = dxz.stride(0), p.dz_ds = dxz.stride(1);
+    p.dB = dxd + q.R * q.BL * es, p.dB_bs = q.L, p.dB_gs = 0, p.dB_ns = q.BL;
+    p.dC = dxd + (q.R + q.N) * q.BL * es, p.dC_bs = q.L, p.dC_gs = 0, p.dC_ns = q.BL;
+    const at::Tensor sums = run_scan_bwd(p, xz.device()).sums;
+    // the weights' gradients in the weights' dtype
+    auto like = [&](int64_t rows, int64_t cols, int64_t code) { return at::empty({rows, cols}, xz.options().dtype((at::ScalarType)code)); };
+    auto direct = [&](int64_t code) { return (at::ScalarType)code == at::kFloat || (at::ScalarType)code == ty ? code : (int64_t)ty; };
+    at::Tensor dxp = like(q.rows, q.d, direct(o[4])), ddp = like(q.d, q.R, direct(o[5])), dop = like(q.E, q.d, direct(o[6]));
+    m.add(dop.data_ptr(), dop.scalar_type(), q.d, q.E, q.d, q.BL, {g_out, 1, q.E}, {out_z, q.BL, 1});
+    m.add(ddp.data_ptr(), ddp.scalar_type(), q.R, q.d, q.R, q.BL, {ddelta, q.BL, 1}, {xd, q.BL, 1});
+    m.add(dxd, ty, q.BL, q.R, q.BL, q.d, {dp, 1, q.R}, {ddelta, 1, q.BL}).run();
+    m.add(dxp.data_ptr(), dxp.scalar_type(), q.d, q.rows, q.d, q.BL, {dxd, q.BL, 1}, {conv, q.BL, 1});
+    m.add(dconv, ty, q.BL, q.d, q.BL, q.rows, {xp, 1, q.d}, {dxd, 1, q.BL}, true).run();  // added to the scan's own du
+    auto [dcw, dcb] = conv_bwd(xz, q.batch, q.d, q.L, {xz.data_ptr(), xz.stride(0), xs, 1}, conv_w, conv_bias, {dconv, q.L, q.BL, 1},
+                               std::nullopt, true, {dx, dxz.stride(0), dxz.stride(1), 1});
     variable_list g(13);
-    g[0] = dxz, g[1] = dcw.unsqueeze(1), g[2] = tensor_or_none(dcb), g[3] = dxp, g[4] = ddp, g[5] = dop;
-    if (ctx->saved_data["out_bias"].toBool()) g[6] = dout.sum(0);
-    g[7] = *r[2], g[8] = tensor_or_none(r[5]), g[9] = tensor_or_none(r[6]);
+    g[0] = dxz, g[1] = dcw, g[2] = tensor_or_none(dcb), g[3] = dxp.to((at::ScalarType)o[4]), g[4] = ddp.to((at::ScalarType)o[5]);
+    g[5] = dop.to((at::ScalarType)o[6]);
+    if (o[3]) g[6] = dout.view({q.BL, q.E}).sum(0).to((at::ScalarType)o[7]);
+    g[7] = sums.as_strided({q.d, q.N}, {q.N, 1}, 0);
+    if (D) g[8] = sums.as_strided({q.d}, {1}, q.d * q.N);
+    if (delta_bias) g[9] = sums.as_strided({q.d}, {1}, q.d * (q.N + 1));
     return g;
   }
 };

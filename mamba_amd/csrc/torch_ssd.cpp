@@ -391,7 +391,13 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
         y = y.to(*autocast), w = w.to(*autocast);
         if (bias) bias = bias->to(*autocast);
       }
-      res = at::linear(y, w, bias);
+      y = y.contiguous(), w = w.contiguous();
+      if (bias) bias = bias->contiguous();
+      res = at::empty({batch * L, w.size(0)}, y.options());
+      Products(y.options(), y.scalar_type())
+          .add(res.data_ptr(), y.scalar_type(), w.size(0), batch * L, w.size(0), dim, {y.data_ptr(), dim, 1}, {w.data_ptr(), dim, 1}, false,
+               bias ? bias->data_ptr() : nullptr)
+          .run();
     }
     ctx->save_for_backward({zxbcdt, conv_w, tensor_or_none(conv_bias), xBC, gate_in_scan ? *r[1] : *r[0], *r[2], *r[3], *r[4], A, D,
                             dt_bias, tensor_or_none(initial_states), tensor_or_none(seq_idx), tensor_or_none(norm_weight),
@@ -421,9 +427,16 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
     at::Tensor dy;
     if (w.defined()) {
       at::Tensor dout = grads[0].defined() ? grads[0].reshape({batch * L, -1}) : at::zeros({batch * L, w.size(0)}, w.options());
-      dout = dout.to(w.scalar_type());
-      dy = at::mm(dout, w);
-      g[9] = at::mm(dout.t(), y).to((at::ScalarType)v[6]);
+      dout = dout.to(w.scalar_type()).contiguous();
+      const int64_t E = w.size(0);
+      const at::ScalarType ty = w.scalar_type(), wt = (at::ScalarType)v[6];
+      dy = at::empty({batch * L, dim}, w.options());
+      at::Tensor dw = at::empty({E, dim}, w.options().dtype(wt == at::kFloat ? wt : ty));
+      Products(w.options(), ty)
+          .add(dy.data_ptr(), ty, dim, batch * L, dim, E, {dout.data_ptr(), E, 1}, {w.data_ptr(), 1, dim})
+          .add(dw.data_ptr(), dw.scalar_type(), dim, E, dim, batch * L, {dout.data_ptr(), 1, E}, {y.data_ptr(), 1, dim})
+          .run();
+      g[9] = dw.to(wt);
       if (v[5]) g[10] = dout.sum(0).to((at::ScalarType)v[7]);
     } else {
       dy = grads[0].defined() ? unit_last(grads[0].reshape({batch * L, dim})) : at::zeros({batch * L, dim}, zxbcdt.options());

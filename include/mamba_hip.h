@@ -448,6 +448,8 @@ int ssd_bwd_dcb(const SsdParams *p, mamba_stream_t stream);
 int ssd_bmm_chunk_bwd(const SsdParams *p, mamba_stream_t stream);
 int ssd_chunk_cumsum_bwd(const SsdParams *p, mamba_stream_t stream);
 int ssd_combined_bwd(const SsdParams *p, mamba_stream_t stream);
+/* Zeros count (1 - 3) ranges [off[i], off[i] + n[i]) of an fp32 array, all multiples of 4; base on 16 bytes. */
+int ssd_clear(float *base, const int64_t *off, const int64_t *n, int count, mamba_stream_t stream);
 
 /* ------------------------------------------------------------------------- *
  * Depthwise causal 1-D convolution in front of the scans.  The reference calls the

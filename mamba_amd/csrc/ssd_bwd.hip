@@ -40,6 +40,21 @@ __global__ __launch_bounds__(256) void det_convert_kernel(const int64_t *__restr
   if (i < n) dst[i] = det_value(src[i], scale[1]);
 }
 
+// up to three ranges of an fp32 array to zero: 16-byte pieces, the ranges on 16 bytes (one launch for what the sums
+// of a backward pass need cleared; ~2 us of host time where a torch fill of each range takes ~6)
+struct ClearJobs {
+  float *base;
+  int64_t off[3], pieces[3];
+};
+__global__ __launch_bounds__(256) void clear_kernel(const ClearJobs j) {
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    if (i >= 0 && i < j.pieces[r]) *reinterpret_cast<f32x4 *>(j.base + j.off[r] + i * 4) = f32x4{0.f, 0.f, 0.f, 0.f};
+    i -= j.pieces[r];
+  }
+}
+
 // Sums acc[m][n] * fx(m, n) over n for every row m of the block tile into rows[64] (LDS, zeroed
 // here).  All 256 threads call; rows[] is valid after the trailing barrier.
 template <typename F> DEVI void row_dot(GemmAcc &acc, float *rows, int tid, F fx) {
@@ -245,8 +260,10 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bwd_dst
 }
 
 // The same product with a 64 x 128 tile per workgroup (whole 128-state blocks, aligned operands,
-// chunks that are whole k steps).
-template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bwd_dstates_wide_kernel(const SsdParams p) {
+// chunks of whole k steps, the last one of any length: RAGGED).
+template <typename T, bool SPLIT, int FORM>
+__global__ __launch_bounds__(256, FORM == WIDE_DEEP ? (SPLIT ? 2 : 3) : 1) void bwd_dstates_wide_kernel(const SsdParams p) {
+  constexpr bool RAGGED = FORM != WIDE_WHOLE;
   __shared__ GemmLdsWide<SPLIT> lds;
   __shared__ float rs[256];
   const int tid = threadIdx.x;
@@ -257,25 +274,36 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bwd_dst
   const int c = blk.y, b = blk.z / H, h = blk.z % H;
   const int g = h / (H / p.ngroups);
   const int t0 = c * Q, qlim = min(Q, L - t0);
-  const float *dA = chunk_row(p.dA_cumsum, p, b, h, c);
-  const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L + t0 : nullptr;
-  for (int l = tid; l < Q; l += 256) {
-    float v = 0.f;
-    if (l < qlim) {
-      bool ok = true;
-      if (seq) ok = seq[l] == (c > 0 ? seq[-1] : 0);
-      if (ok) v = fast_exp(dA[l]);
-    }
-    rs[l] = v;
-  }
   const View4 gv = g_view(p);
   const T *ga = static_cast<const T *>(gv.ptr) + b * gv.bs + h * gv.hs + (int64_t)t0 * gv.ls + pt * GB;
   const T *Ca = static_cast<const T *>(p.C) + b * p.C_bs + g * p.C_gs + (int64_t)t0 * p.C_ls + nt * WB;
   GemmAccWide acc;
   acc.zero();
-  WideTrStager<SPLIT, T, 64> sa(lds.ah, lds.al, ga, gv.ls, P - pt * GB, nullptr, tid);
-  WideTrStager<SPLIT, T, WB> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, rs, tid);
-  block_gemm_wide<SPLIT>(acc, lds, qlim, sa, sb, tid);  // the first barrier inside publishes rs
+  WideTrStager<SPLIT, T, 64, RAGGED> sa(lds.ah, lds.al, ga, gv.ls, P - pt * GB, nullptr, tid, qlim);
+  WideTrStager<SPLIT, T, WB, RAGGED> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, rs, tid, qlim);
+  const int k_end = round_to_step(qlim);
+  auto weights = [&] {
+    const float *dA = chunk_row(p.dA_cumsum, p, b, h, c);
+    const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L + t0 : nullptr;
+    for (int l = tid; l < Q; l += 256) {
+      float v = 0.f;
+      if (l < qlim) {
+        bool ok = true;
+        if (seq) ok = seq[l] == (c > 0 ? seq[-1] : 0);
+        if (ok) v = fast_exp(dA[l]);
+      }
+      rs[l] = v;
+    }
+  };
+  // the first barrier inside the product publishes rs
+  if constexpr (FORM == WIDE_DEEP) {
+    WideDeep<SPLIT, WIDE_PF, decltype(sa), decltype(sb)> deep(sa, sb, k_end);
+    weights();
+    deep.run(acc, lds, tid);
+  } else {
+    weights();
+    block_gemm_wide<SPLIT>(acc, lds, k_end, sa, sb, tid);
+  }
   carried_t<T> *ds = carried_dstates<T>(p) + (((int64_t)b * p.nchunks + c) * H + h) * P * N;
   store_wide_rows(acc, lds, ds + (int64_t)pt * GB * N + nt * WB, N, P - pt * GB, tid);
 }
@@ -284,19 +312,19 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bwd_dst
 // 128 states, a gate): the stager of the product's A operand makes g from dout and z on its way to LDS, stores it
 // and dz, and sums g x for dD; the product takes the stored (rounded) g, as the separate kernel does.  A thread's
 // task per k step is one 16-byte piece of a position's row, the task of bwd_dz_kernel.
-template <typename T> struct DzStager {
+template <typename T, bool RAGGED> struct DzStager {
   static constexpr bool transposed = true;
   static constexpr int PITCH = WideTrStager<false, T, 64>::PITCH;
   uint16_t *hi;
   const T *dout, *z, *y, *x;  // at (batch, first position of the chunk, head, first p of the tile)
   T *dz, *g;
   int64_t dout_ls, z_ls, y_ls, x_ls, o_ls;
-  int rows_valid, t;
+  int rows_valid, t, k_valid;
   Pack8<T> qd, qz, qy, qx;
   float dD[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   DEVI bool fast() const { return true; }
   template <bool FAST = true> DEVI void fetch(int k0) {
-    const int l = k0 + (t >> 3), r8 = min((t & 7) * 8, rows_valid - 8);
+    const int l = RAGGED ? min(k0 + (t >> 3), k_valid - 1) : k0 + (t >> 3), r8 = min((t & 7) * 8, rows_valid - 8);
     qd.load(dout + (int64_t)l * dout_ls + r8);
     qz.load(z + (int64_t)l * z_ls + r8);
     qy.load(y + (int64_t)l * y_ls + r8);
@@ -306,7 +334,7 @@ template <typename T> struct DzStager {
     const int kk = t >> 3, r8 = (t & 7) * 8, off = kk * PITCH + r8;
     Pack8<T> gq;
     gq.zero();
-    if (r8 < rows_valid) {
+    if (r8 < rows_valid && (!RAGGED || k0 + kk < k_valid)) {
       float d[8], zz[8], yy[8], xx[8], gv[8], dzv[8];
       qd.unpack(d);
       qz.unpack(zz);
@@ -331,7 +359,7 @@ template <typename T> struct DzStager {
 };
 
 
-template <typename T> __global__ __launch_bounds__(256) void bwd_dz_dstates_kernel(const SsdParams p) {
+template <typename T, bool RAGGED> __global__ __launch_bounds__(256) void bwd_dz_dstates_kernel(const SsdParams p) {
   __shared__ GemmLdsWide<false> lds;
   __shared__ float rs[256];
   const int tid = threadIdx.x;
@@ -352,7 +380,7 @@ template <typename T> __global__ __launch_bounds__(256) void bwd_dz_dstates_kern
     }
     rs[l] = v;
   }
-  DzStager<T> sa;
+  DzStager<T, RAGGED> sa;
   sa.hi = lds.ah;
   sa.dout = static_cast<const T *>(p.dout) + b * p.dout_bs + h * p.dout_hs + (int64_t)t0 * p.dout_ls + pt * GB;
   sa.z = static_cast<const T *>(p.z) + b * p.z_bs + h * p.z_hs + (int64_t)t0 * p.z_ls + pt * GB;
@@ -363,12 +391,12 @@ template <typename T> __global__ __launch_bounds__(256) void bwd_dz_dstates_kern
   sa.g = static_cast<T *>(p.gbuf) + o0;
   sa.dout_ls = p.dout_ls, sa.z_ls = p.z_ls, sa.y_ls = p.out_ls, sa.x_ls = p.x_ls, sa.o_ls = (int64_t)H * P;
   sa.rows_valid = P - pt * GB;
-  sa.t = tid;
+  sa.t = tid, sa.k_valid = qlim;
   const T *Ca = static_cast<const T *>(p.C) + b * p.C_bs + g * p.C_gs + (int64_t)t0 * p.C_ls;
   GemmAccWide acc;
   acc.zero();
-  WideTrStager<false, T, WB> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, rs, tid);
-  block_gemm_wide<false>(acc, lds, qlim, sa, sb, tid);  // the first barrier inside publishes rs
+  WideTrStager<false, T, WB, RAGGED> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, rs, tid, qlim);
+  block_gemm_wide<false>(acc, lds, round_to_step(qlim), sa, sb, tid);  // the first barrier inside publishes rs
   if (p.D) {
     // a thread's 8 columns are the same in every step: column group tid % 8, summed over the 32 threads that share it
     float *red = reinterpret_cast<float *>(&lds);  // row stride 9: conflict-free column reads
@@ -1377,64 +1405,83 @@ __global__ __launch_bounds__(256, 4) void bwd_dcb_rows_kernel(const SsdParams p,
 
 // ------------------------------------------------------------- bmm bwd
 // dC32[l, n] += sum_{s <= l} dCB[l, s] B[s, n];   dB32[s, n] += sum_{l >= s} dCB[l, s] C[l, n]
-template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bmm_chunk_bwd_kernel(const SsdParams p) {
+// This stage is the last one to add into dB32 / dC32 and its tiles cover every row once: with dB / dC set the sums leave
+// here in the operands' dtype, at the caller's strides, and no conversion pass over the fp32 sums is needed (it took 52
+// us of 470 at 16384 positions, 8 groups of 64 states).
+// LP: dCB holds bf16 tiles (packed at the start of the buffer; see dcb_tile), which go to LDS as they are.  The stage is
+// bound by reading dCB where there are several groups; as bf16 that is half (80 us in fp32 at that size).
+// which: 0 = both products, one after the other; 1 = the dC product only; 2 = the dB product only (the two read
+// different operands and write different sums: dealt to two workgroups they halve a workgroup's serial work where
+// the tiles alone do not fill the chip).
+template <typename T>
+DEVI void add_final(const SsdParams &p, bool is_c, int b, int t, int g, int n, float v) {
+  const int64_t at = (((int64_t)b * p.seqlen + t) * p.ngroups + g) * p.dstate + n;
+  float *sum = (is_c ? p.dC32 : p.dB32) + at;
+  v += *sum;
+  T *fin = static_cast<T *>(is_c ? p.dC : p.dB);
+  if (!fin) *sum = v;
+  else if (is_c) st1<T>(fin + b * p.dC_bs + t * p.dC_ls + g * p.dC_gs + n, v);  // (nobody reads the fp32 sum any more)
+  else st1<T>(fin + b * p.dB_bs + t * p.dB_ls + g * p.dB_gs + n, v);
+}
+
+// 64 x 64 tiles, any shape
+template <typename T, bool SPLIT, bool LP>
+DEVI void bmm_chunk_bwd_body(const SsdParams &p, int bx, int by, int bz, int which) {
+  using CBT = std::conditional_t<LP, bf16_t, float>;
   __shared__ GemmLds lds;
   const int tid = threadIdx.x;
   const int Q = p.chunk_size, N = p.dstate, L = p.seqlen, G = p.ngroups;
   const int ntn = cdiv(N, GB);
-  const int mt = blockIdx.x / ntn, nt = blockIdx.x % ntn;
-  const int c = blockIdx.y, b = blockIdx.z / G, g = blockIdx.z % G;
+  const int mt = bx / ntn, nt = bx % ntn;
+  const int c = by, b = bz / G, g = bz % G;
   const int t0 = c * Q, qlim = min(Q, L - t0);
-  const float *dCB = p.dCB + (((int64_t)b * p.nchunks + c) * G + g) * Q * Q;
+  if (mt * GB >= qlim) return;
+  const CBT *dCB = reinterpret_cast<const CBT *>(p.dCB) + (((int64_t)b * p.nchunks + c) * G + g) * Q * Q;
   const int64_t Cb = b * p.C_bs + g * p.C_gs, Bb = b * p.B_bs + g * p.B_gs;
-  {
+  auto add_tile = [&](GemmAcc &acc, bool is_c) {
+    acc_foreach(acc, tid, [&](int m, int n, float v) {
+      const int l = mt * GB + m, nn = nt * GB + n;
+      if (l < qlim && nn < N) add_final<T>(p, is_c, b, t0 + l, g, nn, v);
+      return v;
+    });
+  };
+  if (which != 2) {
     GemmAcc acc;
     acc.zero();
-    // dCB is zero above the diagonal (never written), so no mask is needed here.
-    // A = dCB rows (l, k = s): k-contiguous fp32; B = B^T (rows n, k = s): row-contiguous
-    const float *da = dCB + (int64_t)mt * GB * Q;
+    // dCB is zero above the diagonal inside its tile, so no mask is needed here.
+    // A = dCB rows (l, k = s): k-contiguous; B = B^T (rows n, k = s): row-contiguous
+    const CBT *da = dCB + (int64_t)mt * GB * Q;
     const T *Ba = static_cast<const T *>(p.B) + Bb + (int64_t)t0 * p.B_ls + nt * GB;
     const bool va = rows_aligned16(da, Q), vb = rows_aligned16(Ba, p.B_ls);
     const int kend = min((mt + 1) * GB, qlim);
     block_gemm_pipe<SPLIT>(
         acc, lds, 0, kend,
-        KcStager<SPLIT, float>(lds.ah, lds.al, da, Q, qlim - mt * GB, kend, nullptr, nullptr, va, tid),
+        KcStager<SPLIT, CBT>(lds.ah, lds.al, da, Q, qlim - mt * GB, kend, nullptr, nullptr, va, tid),
         TrStager<SPLIT, T>(lds.bh, lds.bl, Ba, p.B_ls, N - nt * GB, kend, nullptr, nullptr, vb, tid),
         tid);
-    acc_foreach(acc, tid, [&](int m, int n, float v) {
-      const int l = mt * GB + m, nn = nt * GB + n;
-      if (l < qlim && nn < N) p.dC32[(((int64_t)b * L + t0 + l) * G + g) * N + nn] += v;
-      return v;
-    });
+    add_tile(acc, true);
   }
-  {
+  if (which != 1) {
     GemmAcc acc;
     acc.zero();
-    // A = dCB^T (rows s, k = l): row-contiguous fp32; B = C^T (rows n, k = l): row-contiguous
-    const float *da = dCB + mt * GB;
+    // A = dCB^T (rows s, k = l): row-contiguous; B = C^T (rows n, k = l): row-contiguous
+    const CBT *da = dCB + mt * GB;
     const T *Ca = static_cast<const T *>(p.C) + Cb + (int64_t)t0 * p.C_ls + nt * GB;
     const bool va = rows_aligned16(da, Q), vb = rows_aligned16(Ca, p.C_ls);
     block_gemm_pipe<SPLIT>(
         acc, lds, mt * GB, qlim,
-        TrStager<SPLIT, float>(lds.ah, lds.al, da, Q, qlim - mt * GB, qlim, nullptr, nullptr, va, tid),
+        TrStager<SPLIT, CBT>(lds.ah, lds.al, da, Q, qlim - mt * GB, qlim, nullptr, nullptr, va, tid),
         TrStager<SPLIT, T>(lds.bh, lds.bl, Ca, p.C_ls, N - nt * GB, qlim, nullptr, nullptr, vb, tid),
         tid);
-    acc_foreach(acc, tid, [&](int m, int n, float v) {
-      const int s = mt * GB + m, nn = nt * GB + n;
-      if (s < qlim && nn < N) p.dB32[(((int64_t)b * L + t0 + s) * G + g) * N + nn] += v;
-      return v;
-    });
+    add_tile(acc, false);
   }
 }
 
-// The same two products on 64 x 128 tiles (whole 128-state blocks, chunks of whole k steps, 16-byte aligned B / C
-// rows): half the workgroups, each k step of dCB staged once for twice the columns.
-// LP: dCB holds bf16 tiles (packed at the start of the buffer; see dcb_tile), which go to LDS as they are.
-// which: 0 = both products, one after the other; 1 = the dC product only; 2 = the dB product only (the two read
-// different operands and write different sums: dealt to two workgroups they halve a workgroup's serial work where
-// the tiles alone do not fill the chip).
-template <typename T, bool SPLIT, bool LP = false>
-DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, int which = 0) {
+// The same two products on 64 x 128 tiles (whole 128-state blocks, chunks of whole k steps -- the last one of any
+// length with RAGGED --, 16-byte aligned B / C rows): half the workgroups, each k step of dCB staged once for twice
+// the columns.
+template <typename T, bool SPLIT, bool LP, bool RAGGED>
+DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, int which) {
   using CBT = std::conditional_t<LP, bf16_t, float>;
   __shared__ GemmLdsWide<SPLIT> lds;
   const int tid = threadIdx.x;
@@ -1446,9 +1493,6 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
   if (mt * GB >= qlim) return;
   const CBT *dCB = reinterpret_cast<const CBT *>(p.dCB) + (((int64_t)b * p.nchunks + c) * G + g) * Q * Q;
   const int lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, i = lane & 15, gq = lane >> 4;
-  // dst[(row of the chunk) * G * N + column] += tile.  This stage is the last one to add into dB32 / dC32 and its
-  // tiles cover every row once: with `fin` set the sum leaves here in the operands' dtype as well (dB / dC), and no
-  // separate conversion pass over the fp32 sums is needed.
   auto add_tile = [&](const GemmAccWide &acc, float *dst, void *fin, int64_t fin_bs, int64_t fin_ls, int64_t fin_gs) {
 #pragma unroll
     for (int tm = 0; tm < 2; ++tm)
@@ -1462,38 +1506,41 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
 #pragma unroll
         for (int tn = 0; tn < 4; ++tn) {
           const float v = row[tn * 16] + acc.v[tm][tn][r];
-          if (fin) st1<T>(static_cast<T *>(fin) + fat + tn * 16, v);  // the finished sum: nobody reads the fp32 one
+          if (fin) st1<T>(static_cast<T *>(fin) + fat + tn * 16, v);
           else row[tn * 16] = v;
         }
       }
   };
   if (which != 2) {
-    // dC: A = dCB rows (l, k = s), k-contiguous fp32, s up to the end of the l tile; B = B rows (k = s, n)
+    // dC: A = dCB rows (l, k = s), k-contiguous, s up to the end of the l tile; B = B rows (k = s, n)
     GemmAccWide acc;
     acc.zero();
     const int kend = min((mt + 1) * GB, qlim);
-    KcStager<SPLIT, CBT> sa(lds.ah, lds.al, dCB + (int64_t)mt * GB * Q, Q, qlim - mt * GB, kend, nullptr, nullptr, true, tid);
+    KcStager<SPLIT, CBT, RAGGED> sa(lds.ah, lds.al, dCB + (int64_t)mt * GB * Q, Q, qlim - mt * GB, kend, nullptr, nullptr, true, tid);
     const T *Ba = static_cast<const T *>(p.B) + b * p.B_bs + g * p.B_gs + (int64_t)t0 * p.B_ls + nt * WB;
-    WideTrStager<SPLIT, T, WB> sb(lds.bh, lds.bl, Ba, p.B_ls, WB, nullptr, tid);
-    block_gemm_wide<SPLIT>(acc, lds, kend, sa, sb, tid);
+    WideTrStager<SPLIT, T, WB, RAGGED> sb(lds.bh, lds.bl, Ba, p.B_ls, WB, nullptr, tid, kend);
+    block_gemm_wide<SPLIT>(acc, lds, round_to_step(kend), sa, sb, tid);
     add_tile(acc, p.dC32, p.dC, p.dC_bs, p.dC_ls, p.dC_gs);
   }
   if (which == 0) lds_barrier();  // the first product's last operand reads end before the second one's first commit
   if (which != 1) {
-    // dB: A = dCB^T (rows s, k = l from the s tile on), row-contiguous fp32; B = C rows (k = l, n)
+    // dB: A = dCB^T (rows s, k = l from the s tile on), row-contiguous; B = C rows (k = l, n)
     GemmAccWide acc;
     acc.zero();
     const int k0 = mt * GB;
-    WideTrStager<SPLIT, CBT, 64> sa(lds.ah, lds.al, dCB + (int64_t)k0 * Q + mt * GB, Q, min(GB, Q - mt * GB), nullptr, tid);
+    WideTrStager<SPLIT, CBT, 64, RAGGED> sa(lds.ah, lds.al, dCB + (int64_t)k0 * Q + mt * GB, Q, min(GB, Q - mt * GB), nullptr, tid, qlim - k0);
     const T *Ca = static_cast<const T *>(p.C) + b * p.C_bs + g * p.C_gs + (int64_t)(t0 + k0) * p.C_ls + nt * WB;
-    WideTrStager<SPLIT, T, WB> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, nullptr, tid);
-    block_gemm_wide<SPLIT>(acc, lds, qlim - k0, sa, sb, tid);
+    WideTrStager<SPLIT, T, WB, RAGGED> sb(lds.bh, lds.bl, Ca, p.C_ls, WB, nullptr, tid, qlim - k0);
+    block_gemm_wide<SPLIT>(acc, lds, round_to_step(qlim - k0), sa, sb, tid);
     add_tile(acc, p.dB32, p.dB, p.dB_bs, p.dB_ls, p.dB_gs);
   }
 }
 
-template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bmm_chunk_bwd_wide_kernel(const SsdParams p) {
-  bmm_chunk_bwd_wide_body<T, SPLIT>(p, blockIdx.x, blockIdx.y, blockIdx.z);
+template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bmm_chunk_bwd_kernel(const SsdParams p) {
+  bmm_chunk_bwd_body<T, SPLIT, false>(p, blockIdx.x, blockIdx.y, blockIdx.z, 0);
+}
+template <typename T, bool SPLIT, int FORM> __global__ __launch_bounds__(256) void bmm_chunk_bwd_wide_kernel(const SsdParams p) {
+  bmm_chunk_bwd_wide_body<T, SPLIT, false, FORM != WIDE_WHOLE>(p, blockIdx.x, blockIdx.y, blockIdx.z, 0);
 }
 
 // --------------------------------------------------------- cumsum bwd
@@ -1580,14 +1627,17 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(const SsdParams p
 }
 
 // The last two stages read disjoint results of the stages before them (dCB; ddA_cumsum and ddt_out) and neither
-// fills the chip for long: one launch deals the wide-tile bmm workgroups first and the cumsum workgroups behind them.
-template <typename T, bool SPLIT, bool LP = false>
+// fills the chip for long: one launch deals the bmm workgroups first and the cumsum workgroups behind them.
+enum { BMM_TILES = 0, BMM_WIDE = 1, BMM_WIDE_RAGGED = 2 };
+template <typename T, bool SPLIT, bool LP, int FORM>
 __global__ __launch_bounds__(256) void bmm_cumsum_bwd_kernel(const SsdParams p, int n_bmm, int bmm_x, int bmm_y, int cs_x, int cs_y, int split) {
   const int id = blockIdx.x;
   if (id < n_bmm) {
     // split: two workgroups per tile, one per product, neighbours in launch order (they share the dCB tile)
     const int t = split ? id >> 1 : id, which = split ? 1 + (id & 1) : 0;
-    bmm_chunk_bwd_wide_body<T, SPLIT, LP>(p, t % bmm_x, (t / bmm_x) % bmm_y, t / (bmm_x * bmm_y), which);
+    const int bx = t % bmm_x, by = (t / bmm_x) % bmm_y, bz = t / (bmm_x * bmm_y);
+    if constexpr (FORM == BMM_TILES) bmm_chunk_bwd_body<T, SPLIT, LP>(p, bx, by, bz, which);
+    else bmm_chunk_bwd_wide_body<T, SPLIT, LP, FORM == BMM_WIDE_RAGGED>(p, bx, by, bz, which);
   } else {
     const int k = id - n_bmm;
     chunk_cumsum_bwd_body(p, k % cs_x, (k / cs_x) % cs_y, k / (cs_x * cs_y));
@@ -1672,7 +1722,8 @@ static int ssd_bwd_dstates_one(const SsdParams *p, mamba_stream_t stream) {
                       wide_operand_ok(p->C, p->dtype, p->C_bs, p->C_ls, p->C_gs);
     if (wide) {
       dim3 grid(tiles(p->headdim) * (p->dstate / WB), p->nchunks, p->batch * p->nheads);
-      SSD_DISPATCH(bwd_dstates_wide_kernel, grid)
+      const int form = wide_form(p, (int64_t)grid.x * grid.y * grid.z);
+      SSD_DISPATCH_FORM(bwd_dstates_wide_kernel, grid, form, *p)
       return launched();
     }
   }
@@ -1772,13 +1823,11 @@ static bool dcb_rows_ok(const SsdParams *p) {
          aligned(p->x, 16) && !(g_ls % 8 || g_hs % 8 || g_bs % 8) && !(p->x_ls % 8 || p->x_hs % 8 || p->x_bs % 8) &&
          g_ls < (1 << 21) && p->x_ls < (1 << 21);
 }
-static bool bmm_bwd_wide_ok(const SsdParams *p);
 // Inside ssd_combined_bwd the dCB tiles pass from the dCB stage to the bmm stage as bf16 where one workgroup owns each
 // tile and the bmm stage's operand is bf16 anyway (the stages on their own keep the fp32 tiles their interface names).
 static int64_t bmm_cumsum_workgroups(const SsdParams *p);
 static bool dcb_tiles_lp(const SsdParams *p) {
-  return dcb_rows_ok(p) && p->dCB && dcb_head_splits(p) == 1 && bmm_bwd_wide_ok(p) &&
-         bmm_cumsum_workgroups(p) <= 0x7fffffff;  // (the one-launch form of the last two stages is the reader)
+  return dcb_rows_ok(p) && p->dCB && dcb_head_splits(p) == 1 && bmm_cumsum_workgroups(p) <= 0x7fffffff;  // (the one-launch form of the last two stages is the reader)
 }
 
 static int ssd_bwd_dcb_one(const SsdParams *p, mamba_stream_t stream, bool lp) {
@@ -1822,7 +1871,7 @@ static int ssd_bwd_dcb_stage(const SsdParams *p, mamba_stream_t stream) { return
 static int ssd_bmm_chunk_bwd_one(const SsdParams *p_in, mamba_stream_t stream) {
   int rc = check_bwd(p_in);
   if (rc) return rc;
-  // the stage on its own only adds into dB32 / dC32; dB / dC are written by ssd_combined_bwd, whose last stage this is
+  // the stage on its own only adds into dB32 / dC32; dB / dC are written by ssd_combined_bwd, whose last stage it is
   SsdParams q = *p_in;
   q.dB = q.dC = nullptr;
   const SsdParams *p = &q;
@@ -1831,7 +1880,8 @@ static int ssd_bmm_chunk_bwd_one(const SsdParams *p_in, mamba_stream_t stream) {
       wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs) && wide_operand_ok(p->C, p->dtype, p->C_bs, p->C_ls, p->C_gs) &&
       reinterpret_cast<uintptr_t>(p->dCB) % 16 == 0) {
     dim3 gridw(tiles(p->chunk_size) * (p->dstate / WB), p->nchunks, p->batch * p->ngroups);
-    SSD_DISPATCH(bmm_chunk_bwd_wide_kernel, gridw)
+    const int form = ragged_end(p) ? WIDE_RAGGED : WIDE_WHOLE;
+    SSD_DISPATCH_FORM(bmm_chunk_bwd_wide_kernel, gridw, form, *p)
     return launched();
   }
   dim3 grid(tiles(p->chunk_size) * tiles(p->dstate), p->nchunks, p->batch * p->ngroups);
@@ -1857,6 +1907,21 @@ extern "C" int ssd_det_convert(const int64_t *shadow, float *dst, int64_t n, con
   return launched();
 }
 
+extern "C" int ssd_clear(float *base, const int64_t *off, const int64_t *n, int count, mamba_stream_t stream) {
+  if (!base || count < 1 || count > 3 || reinterpret_cast<uintptr_t>(base) % 16) return MAMBA_E_BADARG;
+  ClearJobs j{};
+  j.base = base;
+  int64_t pieces = 0;
+  for (int i = 0; i < count; ++i) {
+    if (off[i] % 4 || n[i] % 4 || n[i] < 0) return MAMBA_E_BADARG;
+    j.off[i] = off[i], j.pieces[i] = n[i] / 4, pieces += n[i] / 4;
+  }
+  if (pieces == 0) return MAMBA_OK;
+  if ((pieces + 255) / 256 > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
+  hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((pieces + 255) / 256)), dim3(256), 0, static_cast<hipStream_t>(stream), j);
+  return launched();
+}
+
 static bool bmm_bwd_wide_ok(const SsdParams *p) {
   return p->dstate % WB == 0 && p->chunk_size % GB == 0 && whole_k_steps(p) &&
          wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs) && wide_operand_ok(p->C, p->dtype, p->C_bs, p->C_ls, p->C_gs) &&
@@ -1873,70 +1938,50 @@ static SsdParams with_grad_strides(const SsdParams &p) {
   return q;
 }
 
-// The fp32 sums of dB / dC in the operands' dtype, for the paths whose last stage does not write them itself: one
-// thread per element, blockIdx.y = 0 the dB sums, 1 the dC sums.
-template <typename T> __global__ __launch_bounds__(256) void cast_sums_kernel(const SsdParams p) {
-  const bool is_c = blockIdx.y != 0;
-  T *dst = static_cast<T *>(is_c ? p.dC : p.dB);
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (!dst || i >= (int64_t)p.batch * p.seqlen * p.ngroups * p.dstate) return;
-  const int n = i % p.dstate, g = (i / p.dstate) % p.ngroups;
-  const int64_t row = i / ((int64_t)p.dstate * p.ngroups), b = row / p.seqlen, t = row - b * p.seqlen;
-  const int64_t at = is_c ? b * p.dC_bs + t * p.dC_ls + g * p.dC_gs : b * p.dB_bs + t * p.dB_ls + g * p.dB_gs;
-  st1<T>(dst + at + n, (is_c ? p.dC32 : p.dB32)[i]);
-}
-static int cast_sums(const SsdParams *p, mamba_stream_t stream) {
-  const int64_t n = (int64_t)p->batch * p->seqlen * p->ngroups * p->dstate;
-  if ((!p->dB && !p->dC) || n == 0) return MAMBA_OK;
-  if ((n + 255) / 256 > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const dim3 grid((unsigned)((n + 255) / 256), 2);
-  switch (p->dtype) {
-    case MAMBA_BF16: hipLaunchKernelGGL(cast_sums_kernel<bf16_t>, grid, dim3(256), 0, s, *p); break;
-    case MAMBA_F16: hipLaunchKernelGGL(cast_sums_kernel<f16_t>, grid, dim3(256), 0, s, *p); break;
-    default: hipLaunchKernelGGL(cast_sums_kernel<float>, grid, dim3(256), 0, s, *p); break;
-  }
-  return launched();
-}
-
-// The last two stages as one launch where the bmm stage runs on wide tiles, else one after the other.  Either way
-// dB / dC (when the caller passes them) hold the finished sums in the operands' dtype afterwards.
+// The last two stages as one launch.  dB / dC (when the caller passes them) hold the finished sums in the operands'
+// dtype afterwards.
 static int64_t bmm_cumsum_workgroups(const SsdParams *p) {
-  return (int64_t)tiles(p->chunk_size) * (p->dstate / WB) * p->nchunks * p->batch * p->ngroups +
+  return 2 * (int64_t)tiles(p->chunk_size) * tiles(p->dstate) * p->nchunks * p->batch * p->ngroups +
          (int64_t)p->nchunks * ((p->nheads + CSB_HT - 1) / CSB_HT) * p->batch;
 }
 static int bmm_and_cumsum_bwd(const SsdParams *p_in, mamba_stream_t stream, bool lp = false) {
   int rc = check_bwd(p_in);
   if (rc) return rc;
   const SsdParams filled = with_grad_strides(*p_in), *p = &filled;
-  const int64_t bmm_x = tiles(p->chunk_size) * (p->dstate / WB), bmm_y = p->nchunks, bmm_z = (int64_t)p->batch * p->ngroups;
-  const int64_t cs_x = p->nchunks, cs_y = (p->nheads + CSB_HT - 1) / CSB_HT, cs_z = p->batch;
+  if (bmm_cumsum_workgroups(p) > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
+  const int form = !bmm_bwd_wide_ok(p) ? BMM_TILES : ragged_end(p) ? BMM_WIDE_RAGGED : BMM_WIDE;
+  const int64_t bmm_x = tiles(p->chunk_size) * (form == BMM_TILES ? tiles(p->dstate) : p->dstate / WB), bmm_y = p->nchunks;
+  const int64_t bmm_z = (int64_t)p->batch * p->ngroups, cs_x = p->nchunks, cs_y = (p->nheads + CSB_HT - 1) / CSB_HT, cs_z = p->batch;
   // few tiles (fewer than four workgroups per CU): a workgroup per product instead of one per tile
   const int split = bmm_x * bmm_y * bmm_z < 4 * (int64_t)cu_count() ? 1 : 0;
   const int64_t n_bmm = bmm_x * bmm_y * bmm_z * (split ? 2 : 1), total = n_bmm + cs_x * cs_y * cs_z;
-  if (bmm_bwd_wide_ok(p) && p->dCB && total <= 0x7fffffff) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    dim3 grid((unsigned)total);
-#define SSD_LAUNCH_BMM_CS(T, SPLIT) \
-  hipLaunchKernelGGL((bmm_cumsum_bwd_kernel<T, SPLIT>), grid, dim3(256), 0, s, *p, (int)n_bmm, (int)bmm_x, (int)bmm_y, (int)cs_x, (int)cs_y, split)
-    switch (p->dtype) {
-      case MAMBA_BF16:
-        if (lp) hipLaunchKernelGGL((bmm_cumsum_bwd_kernel<bf16_t, false, true>), grid, dim3(256), 0, s, *p, (int)n_bmm, (int)bmm_x, (int)bmm_y, (int)cs_x, (int)cs_y, split);
-        else SSD_LAUNCH_BMM_CS(bf16_t, false);
-        break;
-      case MAMBA_F16: SSD_LAUNCH_BMM_CS(f16_t, true); break;
-      default: SSD_LAUNCH_BMM_CS(float, true); break;
-    }
-#undef SSD_LAUNCH_BMM_CS
-    return launched();
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), 0, s, *p, (int)n_bmm, (int)bmm_x, (int)bmm_y, (int)cs_x, (int)cs_y, split);
+  };
+#define SSD_LAUNCH_BMM_CS(T, SPLIT, LP)                                                    \
+  switch (form) {                                                                          \
+    case BMM_TILES: launch(bmm_cumsum_bwd_kernel<T, SPLIT, LP, BMM_TILES>); break;         \
+    case BMM_WIDE: launch(bmm_cumsum_bwd_kernel<T, SPLIT, LP, BMM_WIDE>); break;           \
+    default: launch(bmm_cumsum_bwd_kernel<T, SPLIT, LP, BMM_WIDE_RAGGED>); break;          \
   }
-  if ((rc = ssd_bmm_chunk_bwd(p, stream))) return rc;
-  if ((rc = ssd_chunk_cumsum_bwd(p, stream))) return rc;
-  return cast_sums(p, stream);
+  switch (p->dtype) {
+    case MAMBA_BF16:
+      if (lp) {
+        SSD_LAUNCH_BMM_CS(bf16_t, false, true)
+      } else {
+        SSD_LAUNCH_BMM_CS(bf16_t, false, false)
+      }
+      break;
+    case MAMBA_F16: SSD_LAUNCH_BMM_CS(f16_t, true, false) break;
+    default: SSD_LAUNCH_BMM_CS(float, true, false) break;
+  }
+#undef SSD_LAUNCH_BMM_CS
+  return launched();
 }
 
 // The first two stages: one kernel where the gate's pass over dout, z and the pre-gate output can feed the
-// state-gradient product directly (bf16 operands, one 128-state tile, whole k steps, 16-byte aligned rows), else
+// state-gradient product directly (bf16 operands, one 128-state tile, chunks of whole k steps, 16-byte aligned rows), else
 // ssd_bwd_dz and ssd_bwd_dstates.
 static int dz_and_dstates(const SsdParams *p, mamba_stream_t stream) {
   int rc = check_bwd(p);
@@ -1953,7 +1998,8 @@ static int dz_and_dstates(const SsdParams *p, mamba_stream_t stream) {
   if (fused) {
     hipStream_t s = static_cast<hipStream_t>(stream);
     dim3 grid(tiles(p->headdim), p->nchunks, p->batch * p->nheads);
-    hipLaunchKernelGGL(bwd_dz_dstates_kernel<bf16_t>, grid, dim3(256), 0, s, *p);
+    if (ragged_end(p)) hipLaunchKernelGGL((bwd_dz_dstates_kernel<bf16_t, true>), grid, dim3(256), 0, s, *p);
+    else hipLaunchKernelGGL((bwd_dz_dstates_kernel<bf16_t, false>), grid, dim3(256), 0, s, *p);
     return launched();
   }
   if (!dD_with_dx(p) && (rc = ssd_bwd_dz(p, stream))) return rc;

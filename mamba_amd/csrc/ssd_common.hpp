@@ -89,7 +89,9 @@ template <typename S> DEVI void put_raw(uint16_t *hi, int off, const Pack8<S> &q
 static_assert(GK == 32, "one staging task per thread");
 
 // k-contiguous source: element (r, k) at base[r * rstride + k]; thread t takes row t / 4, 8 k values.
-template <bool SPLIT, typename S> struct KcStager {
+// RAGGED (fast path): k_valid may be any number; the rows are readable up to the next multiple of 8, and the elements
+// from k_valid on become 0.
+template <bool SPLIT, typename S, bool RAGGED = false> struct KcStager {
   static constexpr bool transposed = false;
   uint16_t *hi, *lo;
   const S *base;
@@ -107,7 +109,7 @@ template <bool SPLIT, typename S> struct KcStager {
   template <bool FAST> DEVI void fetch(int k0) {
     const int r = t >> 2, k = k0 + (t & 3) * 8;
     if constexpr (FAST) {
-      q.load(base + (int64_t)min(r, rows_valid - 1) * rstride + min(k, k_valid - 8));
+      q.load(base + (int64_t)min(r, rows_valid - 1) * rstride + min(k, (RAGGED ? (k_valid + 7) / 8 * 8 : k_valid) - 8));
     } else {
       q.zero();
       if (r < rows_valid && k < k_valid) {
@@ -128,12 +130,23 @@ template <bool SPLIT, typename S> struct KcStager {
     const bool ok = !FAST || (r < rows_valid && k0 + k8 < k_valid);
     if constexpr (kRawCopy<SPLIT, S>) {
       if (!kscale && !rscale) {
+        if constexpr (RAGGED) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int left = k_valid - (k0 + k8 + 2 * e);
+            q.w[e] &= left >= 2 ? 0xffffffffu : left == 1 ? 0xffffu : 0u;
+          }
+        }
         put_raw<S>(hi, tile_off(r, k8), q, ok);
         return;
       }
     }
     float v[8];
     q.unpack(v);
+    if constexpr (RAGGED) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = k0 + k8 + e < k_valid ? v[e] : 0.f;
+    }
     if (kscale) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] *= kscale[k0 + k8 + e];
@@ -331,34 +344,39 @@ template <int PITCH> DEVI bf16x8_t load_frag_tr(const uint16_t *tile, int row0, 
 }
 // Stages ROWS rows x 32 k of a row-contiguous operand (element (r, k) at base[k * kstride + r]) as
 // [k][r]: thread t takes k = t / 8 and, per 64 rows, 8 consecutive rows from 8 (t % 8).  The operand
-// must be 16-byte aligned with rows_valid a multiple of 8 and k_valid a multiple of 32 (the caller
-// checks); rows past rows_valid re-read the last rows and are zeroed.
-template <bool SPLIT, typename S, int ROWS> struct WideTrStager {
+// must be 16-byte aligned with rows_valid a multiple of 8 (the caller checks) and the k extent a multiple of 32, or
+// with RAGGED any k_valid; rows past rows_valid and k past k_valid re-read the last ones and are zeroed.
+template <bool SPLIT, typename S, int ROWS, bool RAGGED = false> struct WideTrStager {
   static constexpr int NT = ROWS / 64, PITCH = ROWS + 16;
   uint16_t *hi, *lo;
   const S *base;
   int64_t kstride;
   int rows_valid;
   const float *kscale;
-  int t;
+  int t, k_valid;
   Pack8<S> q[NT];
   WideTrStager() = default;  // for arrays of stagers, each assigned from a constructed one
-  DEVI WideTrStager(uint16_t *hi_, uint16_t *lo_, const S *base_, int64_t kstride_, int rows_valid_, const float *kscale_, int t_)
-      : hi(hi_), lo(lo_), base(base_), kstride(kstride_), rows_valid(rows_valid_), kscale(kscale_), t(t_) {}
+  DEVI WideTrStager(uint16_t *hi_, uint16_t *lo_, const S *base_, int64_t kstride_, int rows_valid_, const float *kscale_, int t_,
+                    int k_valid_ = 0)
+      : hi(hi_), lo(lo_), base(base_), kstride(kstride_), rows_valid(rows_valid_), kscale(kscale_), t(t_), k_valid(k_valid_) {}
   static constexpr bool transposed = true;
   DEVI bool fast() const { return true; }
-  template <bool FAST = true> DEVI void fetch(int k0) {
+  template <bool FAST = true> DEVI void fetch(int k0) { fetch_to(q, k0); }
+  template <bool FAST = true> DEVI void commit(int k0) { commit_from(q, k0); }
+  // the same with the caller's registers
+  DEVI void fetch_to(Pack8<S> (&q)[NT], int k0) const {
 #pragma unroll
     for (int j = 0; j < NT; ++j)
-      q[j].load(base + (int64_t)(k0 + (t >> 3)) * kstride + min((t & 7) * 8 + 64 * j, rows_valid - 8));
+      q[j].load(base + (int64_t)(RAGGED ? min(k0 + (t >> 3), k_valid - 1) : k0 + (t >> 3)) * kstride +
+                min((t & 7) * 8 + 64 * j, rows_valid - 8));
   }
-  template <bool FAST = true> DEVI void commit(int k0) {
+  DEVI void commit_from(const Pack8<S> (&q)[NT], int k0) const {
     const int kk = t >> 3;
     const float ks = kscale ? kscale[k0 + kk] : 1.f;
 #pragma unroll
     for (int j = 0; j < NT; ++j) {
       const int r8 = (t & 7) * 8 + 64 * j, off = kk * PITCH + r8;
-      if (r8 >= rows_valid) {
+      if (r8 >= rows_valid || (RAGGED && k0 + kk >= k_valid)) {
         const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         put8<SPLIT>(hi, lo, off, zero);
       } else if (kRawCopy<SPLIT, S> && !kscale) {
@@ -373,7 +391,7 @@ template <bool SPLIT, typename S, int ROWS> struct WideTrStager {
     }
   }
 };
-// acc[m][n] += sum_k A[m][k] B[n][k] over k in [0, k_end), k_end a multiple of 32.  The A stager is
+// acc[m][n] += sum_k A[m][k] B[n][k] over k in [0, k_end), k_end a multiple of 32 (RAGGED stagers: rounded up to one).  The A stager is
 // a 64-row stager of either layout on its fast path, the B stager a 128-row WideTrStager (possibly
 // inside a SegStager).
 template <bool SPLIT, bool RING, typename SA, typename SB, typename AFTER>
@@ -463,6 +481,68 @@ DEVI void wide_step(GemmAccWide &acc, GemmLdsWide<false> &s, int k0, SA &fa, SB 
       acc.v[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tm], b[tn], acc.v[tm][tn], 0, 0, 0);
 }
 
+// The product with the operands of PF steps in flight, for launches that leave the chip short of waves: a step then waits
+// for its loads alone, and with one pair in flight that wait (~1 us) is the step.  The first ones are requested at once,
+// so that the caller's tables are made while they are under way.
+template <bool SPLIT, int PF, typename SA, typename SB> struct WideDeep {
+  const SA &sa;
+  const SB &sb;
+  int n;
+  decltype(SA::q) qa[PF];
+  decltype(SB::q) qb[PF];
+  DEVI WideDeep(const SA &sa_, const SB &sb_, int k_end) : sa(sa_), sb(sb_), n(k_end / GK) {
+#pragma unroll
+    for (int j = 0; j < PF; ++j) {
+      sa.fetch_to(qa[j], min(j, n - 1) * GK);
+      sb.fetch_to(qb[j], min(j, n - 1) * GK);
+      __builtin_amdgcn_sched_barrier(0);  // the requests leave in the order they are consumed
+    }
+  }
+  DEVI void run(GemmAccWide &acc, GemmLdsWide<SPLIT> &s, int tid) {
+    const int lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+    const int i = lane & 15, g = lane >> 4;
+    auto step = [&](int j, auto &fa, auto &fb, bool more) {
+      lds_barrier();
+      sa.commit_from(fa, j * GK);
+      sb.commit_from(fb, j * GK);
+      lds_barrier();
+      if (more) {
+        sa.fetch_to(fa, min(j + PF, n - 1) * GK);
+        sb.fetch_to(fb, min(j + PF, n - 1) * GK);
+      }
+      bf16x8_t a[2], b[4], al[2], bl[4];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        a[t] = load_frag<SA::transposed>(s.ah, wm * 32 + t * 16, i, g);
+        if (SPLIT) al[t] = load_frag<SA::transposed>(s.al, wm * 32 + t * 16, i, g);
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        b[t] = load_frag_tr<WLD>(s.bh, wn * 64 + t * 16, i, g);
+        if (SPLIT) bl[t] = load_frag_tr<WLD>(s.bl, wn * 64 + t * 16, i, g);
+      }
+#pragma unroll
+      for (int tm = 0; tm < 2; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < 4; ++tn) {
+          acc.v[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tm], b[tn], acc.v[tm][tn], 0, 0, 0);
+          if (SPLIT) {
+            acc.v[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tm], bl[tn], acc.v[tm][tn], 0, 0, 0);
+            acc.v[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al[tm], b[tn], acc.v[tm][tn], 0, 0, 0);
+          }
+        }
+    };
+    int j = 0;
+    for (; j + PF <= n; j += PF) {
+#pragma unroll
+      for (int u = 0; u < PF; ++u) step(j + u, qa[u], qb[u], true);
+    }
+#pragma unroll
+    for (int u = 0; u < PF - 1; ++u)
+      if (j + u < n) step(j + u, qa[u], qb[u], false);
+  }
+};
+
 // dtype in which the states carried between chunks, and their gradients, pass between kernels: bf16 next to bf16
 // operands (the matrix products only take that part of them), fp32 otherwise.
 template <typename T> using carried_t = std::conditional_t<std::is_same_v<T, bf16_t>, bf16_t, float>;
@@ -521,11 +601,30 @@ inline bool wide_operand_ok(const void *ptr, int dtype, int64_t s0, int64_t s1, 
   const int64_t m = dtype == MAMBA_F32 ? 4 : 8;
   return reinterpret_cast<uintptr_t>(ptr) % 16 == 0 && s0 % m == 0 && s1 % m == 0 && s2 % m == 0;
 }
-// Host side: every chunk is a whole number of k steps.
-inline bool whole_k_steps(const SsdParams *p) {
-  const int last = p->seqlen - (p->nchunks - 1) * p->chunk_size;
-  return p->chunk_size % GK == 0 && last % GK == 0;
+// Host side: every chunk is a whole number of k steps, but for the last one when `ragged_end` says so (the wide kernels
+// then run their RAGGED form).
+inline bool whole_k_steps(const SsdParams *p) { return p->chunk_size % GK == 0; }
+inline bool ragged_end(const SsdParams *p) { return (p->seqlen - (p->nchunks - 1) * p->chunk_size) % GK != 0; }
+DEVI int round_to_step(int k) { return (k + GK - 1) / GK * GK; }
+// Form of a wide kernel: chunks of whole k steps, the last one of any length, or that with several steps' operands in
+// flight for a launch that its registers let run at once (three workgroups per CU, two with split operands).
+enum { WIDE_WHOLE = 0, WIDE_RAGGED = 1, WIDE_DEEP = 2 };
+constexpr int WIDE_PF = 4;
+inline int wide_form(const SsdParams *p, int64_t workgroups) {
+  return workgroups <= (p->dtype == MAMBA_BF16 ? 3 : 2) * (int64_t)cu_count() ? WIDE_DEEP : ragged_end(p) ? WIDE_RAGGED : WIDE_WHOLE;
 }
+#define SSD_DISPATCH_FORM_OF(KERNEL, T, SPLIT, GRID, FORM, ...)                                                      \
+  switch (FORM) {                                                                                                    \
+    case WIDE_WHOLE: hipLaunchKernelGGL((KERNEL<T, SPLIT, WIDE_WHOLE>), GRID, dim3(256), 0, s, __VA_ARGS__); break;  \
+    case WIDE_RAGGED: hipLaunchKernelGGL((KERNEL<T, SPLIT, WIDE_RAGGED>), GRID, dim3(256), 0, s, __VA_ARGS__); break; \
+    default: hipLaunchKernelGGL((KERNEL<T, SPLIT, WIDE_DEEP>), GRID, dim3(256), 0, s, __VA_ARGS__); break;           \
+  }
+#define SSD_DISPATCH_FORM(KERNEL, GRID, FORM, ...)                                              \
+  switch (p->dtype) {                                                                           \
+    case MAMBA_BF16: SSD_DISPATCH_FORM_OF(KERNEL, bf16_t, false, GRID, FORM, __VA_ARGS__) break; \
+    case MAMBA_F16: SSD_DISPATCH_FORM_OF(KERNEL, f16_t, true, GRID, FORM, __VA_ARGS__) break;   \
+    default: SSD_DISPATCH_FORM_OF(KERNEL, float, true, GRID, FORM, __VA_ARGS__) break;          \
+  }
 
 // D[m][n] += sum_{k in [k_begin, k_end)} fa(m, k) * fb(n, k) for the block's 64 x 64 tile.
 // fa / fb return 0 outside their valid ranges.  All 256 threads must call.

@@ -103,12 +103,54 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bmm_chu
   });
 }
 
+// The weights w_s = dt_s exp(a_last - a_s) of a chunk's positions in its last sequence, 0 for the others; w[] is 256
+// long, entry per thread.  OWN: the chunk's steps and their running sums are formed here, by the arithmetic of
+// chunk_cumsum_fwd_kernel, and stored when `store` says so (a launch of its own costs ~5 us, as much as a short
+// sequence's whole chunk_state: see ssd_combined_fwd_one).
+DEVI void chunk_weights(const SsdParams &p, int b, int h, int c, bool own, bool store, float *w, float *wtot) {
+  const int Q = p.chunk_size, L = p.seqlen, H = p.nheads, t0 = c * Q, qlim = min(Q, L - t0), s = threadIdx.x;
+  float *dA = p.dA_cumsum + (((int64_t)b * H + h) * p.nchunks + c) * Q;
+  float *dt = p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q;
+  float a, a_last, step;
+  if (own) {
+    const int lane = s & 63, wave = s >> 6;
+    step = 0.f;
+    if (s < qlim) {
+      step = ld_dyn(p.dt, b * p.dt_bs + (int64_t)(t0 + s) * p.dt_ls + h * p.dt_hs, p.dt_dtype);
+      if (p.dt_bias) step += static_cast<const float *>(p.dt_bias)[h];
+      if (p.dt_softplus) step = softplus_f(step);
+      step = fminf(fmaxf(step, p.dt_min), p.dt_max);
+    }
+    const float cs = wave_incl_sum(step * static_cast<const float *>(p.A)[h]);
+    if (lane == 63) wtot[wave] = cs;
+    lds_barrier();
+    float off = 0.f;
+    for (int i = 0; i < wave; ++i) off += wtot[i];
+    a = cs + off;
+    // (the positions past the chunk's end, if any, have no steps: the running sum at Q - 1 is the last wave's)
+    if (s == Q - 1) wtot[4] = a;
+    lds_barrier();
+    a_last = wtot[4];
+    if (store && s < Q) dt[s] = step, dA[s] = a;
+  } else {
+    const int i = min(s, Q - 1);
+    a = dA[i], a_last = dA[Q - 1], step = dt[i];
+  }
+  bool ok = s < qlim;
+  if (p.seq_idx) {
+    const int32_t *seq = p.seq_idx + (int64_t)b * L + t0;
+    const int last = seq[qlim - 1];
+    ok = ok && last >= 0 && seq[min(s, qlim - 1)] == last;
+  }
+  w[s] = ok ? fast_exp(fminf(a_last - a, 0.f)) * step : 0.f;
+}
+
 // ------------------------------------------------------------ chunk_state
 // states[b, c, h, p, n] = sum_s x[s, p] B[s, n] exp(a_last - a_s) dt_s over the
 // positions s of the chunk that belong to the sequence of its last position.
-template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_state_fwd_kernel(const SsdParams p) {
+template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_state_fwd_kernel(const SsdParams p, int own_cumsum) {
   __shared__ GemmLds lds;
-  __shared__ float w[256];
+  __shared__ float w[256], wtot[5];
   const int tid = threadIdx.x;
   const int Q = p.chunk_size, N = p.dstate, L = p.seqlen, P = p.headdim, H = p.nheads;
   const int ntn = cdiv(N, GB);
@@ -118,22 +160,7 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_s
   const int g = h / (H / p.ngroups);
   const int t0 = c * Q;
   const int qlim = min(Q, L - t0);
-  const float *dA = p.dA_cumsum + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-  const float *dt = p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-  const float a_last = dA[Q - 1];
-  const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L + t0 : nullptr;
-  for (int s = tid; s < Q; s += 256) {
-    float v = 0.f;
-    if (s < qlim) {
-      bool ok = true;
-      if (seq) {
-        const int last = seq[qlim - 1];
-        ok = last >= 0 && seq[s] == last;
-      }
-      if (ok) v = fast_exp(fminf(a_last - dA[s], 0.f)) * dt[s];
-    }
-    w[s] = v;
-  }
+  chunk_weights(p, b, h, c, own_cumsum != 0, blk.x == 0, w, wtot);
   const int64_t xb = b * p.x_bs + h * p.x_hs, Bb = b * p.B_bs + g * p.B_gs;
   GemmAcc acc;
   acc.zero();
@@ -155,10 +182,12 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_s
 }
 
 // The same product with a 64 x 128 tile per workgroup, for whole 128-state blocks of aligned operands
-// and chunks that are whole k steps.
-template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_state_fwd_wide_kernel(const SsdParams p) {
+// and chunks of whole k steps (the last one of any length: RAGGED).
+template <typename T, bool SPLIT, int FORM>
+__global__ __launch_bounds__(256, FORM == WIDE_DEEP ? (SPLIT ? 2 : 3) : 1) void chunk_state_fwd_wide_kernel(const SsdParams p, int own_cumsum) {
+  constexpr bool RAGGED = FORM != WIDE_WHOLE;
   __shared__ GemmLdsWide<SPLIT> lds;
-  __shared__ float w[256];
+  __shared__ float w[256], wtot[5];
   const int tid = threadIdx.x;
   const int Q = p.chunk_size, N = p.dstate, L = p.seqlen, P = p.headdim, H = p.nheads;
   const int ntn = N / WB;
@@ -168,29 +197,23 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_s
   const int g = h / (H / p.ngroups);
   const int t0 = c * Q;
   const int qlim = min(Q, L - t0);
-  const float *dA = p.dA_cumsum + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-  const float *dt = p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-  const float a_last = dA[Q - 1];
-  const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L + t0 : nullptr;
-  for (int s = tid; s < Q; s += 256) {
-    float v = 0.f;
-    if (s < qlim) {
-      bool ok = true;
-      if (seq) {
-        const int last = seq[qlim - 1];
-        ok = last >= 0 && seq[s] == last;
-      }
-      if (ok) v = fast_exp(fminf(a_last - dA[s], 0.f)) * dt[s];
-    }
-    w[s] = v;
-  }
   const T *xa = static_cast<const T *>(p.x) + b * p.x_bs + h * p.x_hs + (int64_t)t0 * p.x_ls + pt * GB;
   const T *Ba = static_cast<const T *>(p.B) + b * p.B_bs + g * p.B_gs + (int64_t)t0 * p.B_ls + nt * WB;
   GemmAccWide acc;
   acc.zero();
-  WideTrStager<SPLIT, T, 64> sa(lds.ah, lds.al, xa, p.x_ls, P - pt * GB, nullptr, tid);
-  WideTrStager<SPLIT, T, WB> sb(lds.bh, lds.bl, Ba, p.B_ls, WB, w, tid);
-  block_gemm_wide<SPLIT>(acc, lds, qlim, sa, sb, tid);  // the first barrier inside publishes w
+  WideTrStager<SPLIT, T, 64, RAGGED> sa(lds.ah, lds.al, xa, p.x_ls, P - pt * GB, nullptr, tid, qlim);
+  WideTrStager<SPLIT, T, WB, RAGGED> sb(lds.bh, lds.bl, Ba, p.B_ls, WB, w, tid, qlim);
+  const int k_end = round_to_step(qlim);
+  auto weights = [&] { chunk_weights(p, b, h, c, own_cumsum != 0, blk.x == 0, w, wtot); };
+  // the first barrier inside the product publishes w
+  if constexpr (FORM == WIDE_DEEP) {
+    WideDeep<SPLIT, WIDE_PF, decltype(sa), decltype(sb)> deep(sa, sb, k_end);
+    weights();
+    deep.run(acc, lds, tid);
+  } else {
+    weights();
+    block_gemm_wide<SPLIT>(acc, lds, k_end, sa, sb, tid);
+  }
   float *st = p.states + (((int64_t)b * p.nchunks + c) * H + h) * P * N;
   store_wide_rows(acc, lds, st + (int64_t)pt * GB * N + nt * WB, N, P - pt * GB, tid);
 }
@@ -456,6 +479,29 @@ template <int R, bool HAS_SEQ> __global__ __launch_bounds__(256) void chunk_stat
 // ------------------------------------------------------------- chunk_scan
 // out[l, p] = exp(a_l) [seq_l == seq before the chunk] sum_n C[l, n] Hc[p, n]
 //           + sum_{s <= l} CB[l, s] exp(a_l - a_s) dt_s x[s, p] + D x[l, p];   out *= silu(z)
+// One 64 x 64 tile (l, p) per workgroup: both products run through the software-pipelined block core, the second one's
+// A operand (CB with the decay and the step) weighted on its way to LDS.  (Element by element from the functors of the
+// unpipelined core every k step waited for its own loads: 56 us for 339 positions of 32 heads in fp16, 78 us for 1408
+// of 48.)
+template <bool SPLIT> struct DecayStager : KcStager<SPLIT, float> {
+  using Base = KcStager<SPLIT, float>;
+  const float *a, *dt;  // of the chunk
+  int l0;               // the tile's first position
+  DEVI DecayStager(Base base, const float *a_, const float *dt_, int l0_) : Base(base), a(a_), dt(dt_), l0(l0_) {}
+  template <bool FAST> DEVI void commit(int k0) {
+    const int r = this->t >> 2, k8 = (this->t & 3) * 8, l = l0 + r;
+    const bool ok = r < this->rows_valid && k0 + k8 < this->k_valid;
+    float v[8];
+    this->q.unpack(v);
+    const float al = a[min(l, 255)];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int k = k0 + k8 + e, kc = min(k, 255);
+      v[e] = k <= l ? v[e] * fast_exp(fminf(al - a[kc], 0.f)) * dt[kc] : 0.f;
+    }
+    put8<SPLIT>(this->hi, this->lo, tile_off(r, k8), v, ok);
+  }
+};
 template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_scan_fwd_kernel(const SsdParams p) {
   __shared__ GemmLds lds;
   __shared__ float a_s[256], dt_s[256], rscale[GB];
@@ -467,13 +513,12 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_s
   const int g = h / (H / G);
   const int t0 = c * Q;
   const int qlim = min(Q, L - t0);
+  if (mt * GB >= qlim) return;
   const float *dA = p.dA_cumsum + (((int64_t)b * H + h) * p.nchunks + c) * Q;
   const float *dt = p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q;
   const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L + t0 : nullptr;
-  for (int s = tid; s < Q; s += 256) {
-    a_s[s] = dA[s];
-    dt_s[s] = dt[s];
-  }
+  a_s[tid] = tid < Q ? dA[tid] : 0.f;
+  dt_s[tid] = tid < Q ? dt[tid] : 0.f;
   if (tid < GB) {
     const int l = mt * GB + tid;
     float sc = 0.f;
@@ -492,30 +537,26 @@ template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void chunk_s
   const float *CB = p.CB + (((int64_t)b * p.nchunks + c) * G + g) * Q * Q;
   GemmAcc acc;
   acc.zero();
-  {  // carried state -> outputs
-    auto fa = [&](int r, int k) {  // (l, n)
-      const int l = mt * GB + r;
-      return (l < qlim && k < N) ? ldg<T>(p.C, Cb + (int64_t)(t0 + l) * p.C_ls + k) : 0.f;
-    };
-    auto fb = [&](int r, int k) {  // (p, n)
-      const int pp = pt * GB + r;
-      return (pp < P && k < N) ? ld1<carried_t<T>>(Hc + (int64_t)pp * N + k) : 0.f;
-    };
-    block_gemm<SPLIT, true, true>(acc, lds, 0, N, fa, fb, tid);
+  {  // carried state -> outputs: A = C rows (l, n), B = Hc rows (p, n)
+    const T *Ca = static_cast<const T *>(p.C) + Cb + (int64_t)(t0 + mt * GB) * p.C_ls;
+    const carried_t<T> *Ha = Hc + (int64_t)pt * GB * N;
+    block_gemm_pipe<SPLIT>(  // the first barrier inside publishes the tables
+        acc, lds, 0, N,
+        KcStager<SPLIT, T>(lds.ah, lds.al, Ca, p.C_ls, qlim - mt * GB, N, nullptr, nullptr, rows_aligned16(Ca, p.C_ls), tid),
+        KcStager<SPLIT, carried_t<T>>(lds.bh, lds.bl, Ha, N, P - pt * GB, N, nullptr, nullptr, rows_aligned16(Ha, N), tid),
+        tid);
     acc_foreach(acc, tid, [&](int m, int n, float v) { return v * rscale[m]; });
   }
-  {  // inside the chunk, causal
+  {  // inside the chunk, causal: A = CB rows (l, s) weighted, B = x^T (p, s)
     const int kmax = min((mt + 1) * GB, qlim);
-    auto fa = [&](int r, int k) {  // (l, s)
-      const int l = mt * GB + r;
-      if (l >= qlim || k > l) return 0.f;
-      return CB[(int64_t)l * Q + k] * fast_exp(fminf(a_s[l] - a_s[k], 0.f)) * dt_s[k];
-    };
-    auto fb = [&](int r, int k) {  // (p, s)
-      const int pp = pt * GB + r;
-      return (pp < P && k < qlim) ? ldg<T>(p.x, xb + (int64_t)(t0 + k) * p.x_ls + pp) : 0.f;
-    };
-    block_gemm<SPLIT, true, false>(acc, lds, 0, kmax, fa, fb, tid);
+    const float *CBa = CB + (int64_t)mt * GB * Q;
+    const T *xa = static_cast<const T *>(p.x) + xb + (int64_t)t0 * p.x_ls + pt * GB;
+    // (CB's rows are readable to their end; past kmax x counts as 0)
+    DecayStager<SPLIT> sa(KcStager<SPLIT, float>(lds.ah, lds.al, CBa, Q, qlim - mt * GB, Q, nullptr, nullptr, rows_aligned16(CBa, Q), tid),
+                          a_s, dt_s, mt * GB);
+    block_gemm_pipe<SPLIT>(
+        acc, lds, 0, kmax, sa,
+        TrStager<SPLIT, T>(lds.bh, lds.bl, xa, p.x_ls, P - pt * GB, kmax, nullptr, nullptr, rows_aligned16(xa, p.x_ls), tid), tid);
   }
   const float *Dp = static_cast<const float *>(p.D);
   acc_foreach(acc, tid, [&](int m, int n, float v) {
@@ -583,7 +624,7 @@ static int ssd_bmm_chunk_fwd_one(const SsdParams *p, mamba_stream_t stream) {
   return launched();
 }
 
-static int ssd_chunk_state_fwd_one(const SsdParams *p, mamba_stream_t stream) {
+static int ssd_chunk_state_fwd_with(const SsdParams *p, mamba_stream_t stream, int own_cumsum) {
   int rc = check(p);
   if (rc) return rc;
   if (!p->states || !p->dt_out || !p->dA_cumsum) return MAMBA_E_BADARG;
@@ -595,14 +636,20 @@ static int ssd_chunk_state_fwd_one(const SsdParams *p, mamba_stream_t stream) {
                       wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs);
     if (wide) {
       dim3 grid(((p->headdim + GB - 1) / GB) * (p->dstate / WB), p->nchunks, p->batch * p->nheads);
-      SSD_DISPATCH(chunk_state_fwd_wide_kernel, grid)
+      const int form = wide_form(p, (int64_t)grid.x * grid.y * grid.z);
+      SSD_DISPATCH_FORM(chunk_state_fwd_wide_kernel, grid, form, *p, own_cumsum)
       return launched();
     }
   }
   dim3 grid(((p->headdim + GB - 1) / GB) * ((p->dstate + GB - 1) / GB), p->nchunks, p->batch * p->nheads);
-  SSD_DISPATCH(chunk_state_fwd_kernel, grid)
+  switch (p->dtype) {
+    case MAMBA_BF16: hipLaunchKernelGGL((chunk_state_fwd_kernel<bf16_t, false>), grid, dim3(256), 0, s, *p, own_cumsum); break;
+    case MAMBA_F16: hipLaunchKernelGGL((chunk_state_fwd_kernel<f16_t, true>), grid, dim3(256), 0, s, *p, own_cumsum); break;
+    default: hipLaunchKernelGGL((chunk_state_fwd_kernel<float, true>), grid, dim3(256), 0, s, *p, own_cumsum); break;
+  }
   return launched();
 }
+static int ssd_chunk_state_fwd_one(const SsdParams *p, mamba_stream_t stream) { return ssd_chunk_state_fwd_with(p, stream, 0); }
 
 extern "C" int ssd_chunk_state_varlen(const SsdParams *p, const int32_t *cu_seqlens, int nseq, float *varlen_states,
                                       mamba_stream_t stream) {
@@ -702,12 +749,17 @@ extern "C" int ssd_chunk_state_passing_fwd(const SsdParams *p, mamba_stream_t st
 }
 
 static int ssd_combined_fwd_one(const SsdParams *p, mamba_stream_t stream) {
-  int rc;
-  if ((rc = ssd_chunk_cumsum_fwd(p, stream))) return rc;
-  if (check(p) == MAMBA_OK && chunk_state_passing_pays(p)) {
+  int rc = check(p);
+  if (rc) return rc;
+  const bool walk = chunk_state_passing_pays(p);
+  // The steps and their sums: a launch of their own where there is much to do, in the chunk_state kernel (whose workgroups
+  // then read the strided steps of their chunk one by one) while that has no more than eight workgroups per CU.
+  const bool merged = !walk && (int64_t)p->nchunks * p->batch * p->nheads <= 8 * (int64_t)cu_count();
+  if (!merged && (rc = ssd_chunk_cumsum_fwd(p, stream))) return rc;
+  if (walk) {
     if ((rc = ssd_chunk_state_passing_fwd(p, stream))) return rc;
   } else {
-    if ((rc = ssd_chunk_state_fwd(p, stream))) return rc;
+    if ((rc = ssd_chunk_state_fwd_with(p, stream, merged))) return rc;
     if ((rc = ssd_state_passing_fwd(p, stream))) return rc;
   }
   if (ssd_chunk_scan_fwd_fused_supported(p)) return ssd_chunk_scan_fwd_fused(p, stream);

@@ -27,8 +27,10 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 template <int V> using Int = std::integral_constant<int, V>;
 
-template <int PT, int NK, int QT, bool SEQ, bool GATED>
-__global__ __launch_bounds__(32 * QT) void chunk_scan_fwd_paired_kernel(const SsdParams p, const int hb) {
+// ONE: one head per workgroup (short launches), with no next head to request, wait for and put away: ~1.5 of 12.7 us.
+template <int PT, int NK, int QT, bool SEQ, bool GATED, bool ONE>
+__global__ __launch_bounds__(32 * QT) void chunk_scan_fwd_paired_kernel(const SsdParams p, const int hb_arg) {
+  const int hb = ONE ? 1 : hb_arg;
   constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT, NW = QT / 2, NT = 64 * NW;
   constexpr int BP = N + 8;   // LDS pitch of a B row / H row (bf16): 16-byte aligned, bank-spread
   constexpr int XP = P + 16;  // LDS pitch of an X row (one position, P values + pad), as it lies in memory
@@ -382,7 +384,7 @@ __global__ __launch_bounds__(32 * QT) void chunk_scan_fwd_paired_kernel(const Ss
     // ---- the next head's operands are requested by each wave as it leaves the loop; the epilogue's patches lie
     // over X and the state, so it starts once every wave has left.  Its x rows (for D) are taken from the head's X
     // rows in LDS before that.
-    load_head(h_first + min(hh + 1, hb - 1) * per);
+    if constexpr (!ONE) load_head(h_first + min(hh + 1, hb - 1) * per);
 #pragma unroll
     for (int e = 0; e < 2; ++e)
 #pragma unroll
@@ -439,9 +441,11 @@ __global__ __launch_bounds__(32 * QT) void chunk_scan_fwd_paired_kernel(const Ss
         if (live) store8(og + oi, v);
       }
     }
-    lds_barrier();  // the next head's operands overwrite the patches
-    commit_head();
-    lds_barrier();
+    if constexpr (!ONE) {
+      lds_barrier();  // the next head's operands overwrite the patches
+      commit_head();
+      lds_barrier();
+    }
   }
 }
 
@@ -449,14 +453,17 @@ template <int PT, int NK, int QT> int launch_seq(const SsdParams &p, hipStream_t
   const int hb = heads_per_workgroup(p);
   dim3 grid(p.nheads / hb, p.nchunks, p.batch);
   const dim3 block(32 * QT);
-  if (p.seq_idx && p.z)
-    hipLaunchKernelGGL((chunk_scan_fwd_paired_kernel<PT, NK, QT, true, true>), grid, block, 0, s, p, hb);
-  else if (p.seq_idx)
-    hipLaunchKernelGGL((chunk_scan_fwd_paired_kernel<PT, NK, QT, true, false>), grid, block, 0, s, p, hb);
-  else if (p.z)
-    hipLaunchKernelGGL((chunk_scan_fwd_paired_kernel<PT, NK, QT, false, true>), grid, block, 0, s, p, hb);
-  else
-    hipLaunchKernelGGL((chunk_scan_fwd_paired_kernel<PT, NK, QT, false, false>), grid, block, 0, s, p, hb);
+  auto launch = [&](auto seq, auto gated, auto one) {
+    hipLaunchKernelGGL((chunk_scan_fwd_paired_kernel<PT, NK, QT, seq.value, gated.value, one.value>), grid, block, 0, s, p, hb);
+  };
+  auto with_one = [&](auto seq, auto gated) {
+    if (hb == 1) launch(seq, gated, std::true_type{});
+    else launch(seq, gated, std::false_type{});
+  };
+  if (p.seq_idx && p.z) with_one(std::true_type{}, std::true_type{});
+  else if (p.seq_idx) with_one(std::true_type{}, std::false_type{});
+  else if (p.z) with_one(std::false_type{}, std::true_type{});
+  else with_one(std::false_type{}, std::false_type{});
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
 }
 

@@ -8,9 +8,11 @@ namespace mamba_ext {
 namespace {
 
 at::Tensor rows_of(const at::Tensor &t) {
+  if (t.dim() == 2 && t.stride(1) == 1) return t;  // (a view costs ~1 us, as much as a launch)
   const at::Tensor r = t.reshape({-1, t.size(-1)});
   return r.stride(1) == 1 ? r : r.contiguous();
 }
+at::Tensor shaped(const at::Tensor &t, at::IntArrayRef sizes) { return t.sizes() == sizes ? t : t.view(sizes); }
 bool vector_ok(const at::Tensor &t, int64_t n) { return t.dim() == 1 && t.size(0) == n && t.is_contiguous(); }
 bool params_ok(const at::Tensor &weight, const OptTensor &bias, int64_t n, const c10::Device &dev) {
   return on_device(weight, dev) && on_device(bias, dev) && dtype_code(weight) >= 0 && vector_ok(weight, n) &&
@@ -65,8 +67,8 @@ struct ResNormFn : torch::autograd::Function<ResNormFn> {
     ctx->saved_data["eps"] = o.eps;
     ctx->saved_data["x_dtype"] = (int64_t)x.scalar_type();
     ctx->saved_data["shape"] = x.sizes().vec();
-    variable_list out = {r.y.view(x.sizes())};
-    if (o.prenorm) out.push_back(r.sum.view(x.sizes()));
+    variable_list out = {shaped(r.y, x.sizes())};
+    if (o.prenorm) out.push_back(shaped(r.sum, x.sizes()));
     return out;
   }
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
@@ -84,7 +86,8 @@ struct ResNormFn : torch::autograd::Function<ResNormFn> {
     if (grads.size() > 1 && grads[1].defined()) dres = rows_of(grads[1]).to(x.scalar_type());
     at::Tensor dx = at::empty({M, N}, x.options().dtype(x_dtype));
     at::Tensor dsum = has_residual && x_dtype != x.scalar_type() ? at::empty({M, N}, x.options()) : at::Tensor();
-    at::Tensor sums = M > 0 ? at::empty({bias ? 2 : 1, N}, weight.options()) : at::zeros({bias ? 2 : 1, N}, weight.options());
+    std::vector<int64_t> sum_shape = bias ? std::vector<int64_t>{2, N} : std::vector<int64_t>{N};
+    at::Tensor sums = M > 0 ? at::empty(sum_shape, weight.options()) : at::zeros(sum_shape, weight.options());
     if (M > 0) {
       NormResidualParams p{};
       p.rows = (int32_t)M, p.dim = (int32_t)N, p.dtype = dtype_code(x_dtype), p.res_dtype = dtype_code(x);
@@ -103,10 +106,10 @@ struct ResNormFn : torch::autograd::Function<ResNormFn> {
       check_rc(norm_residual_bwd(&p, stream_of(x.device())), "norm_residual_bwd");
     }
     variable_list g(5);
-    g[0] = dx.view(shape);
-    g[1] = bias ? sums.select(0, 0) : sums.view({N});
+    g[0] = shaped(dx, shape);
+    g[1] = bias ? sums.select(0, 0) : sums;
     if (bias) g[2] = sums.select(0, 1);
-    if (has_residual) g[3] = (dsum.defined() ? dsum : dx).view(shape);
+    if (has_residual) g[3] = shaped(dsum.defined() ? dsum : dx, shape);
     return g;
   }
 };
@@ -131,8 +134,8 @@ pybind11::object norm_residual(const at::Tensor &x, const at::Tensor &weight, co
   if (x.numel() / N > INT32_MAX) return no;
   if (!records(x, weight, bias, residual)) {
     ResNormOut r = res_norm_fwd(rows_of(x), weight, bias, residual ? OptTensor(rows_of(*residual)) : std::nullopt, o);
-    const at::Tensor y = r.y.view(x.sizes());
-    return prenorm ? pybind11::object(pybind11::make_tuple(y, r.sum.view(x.sizes()))) : pybind11::cast(y);
+    const at::Tensor y = shaped(r.y, x.sizes());
+    return prenorm ? pybind11::object(pybind11::make_tuple(y, shaped(r.sum, x.sizes()))) : pybind11::cast(y);
   }
   variable_list r = ResNormFn::apply(x, weight, bias, residual, o);
   return prenorm ? pybind11::object(pybind11::make_tuple(r[0], r[1])) : pybind11::cast(r[0]);
@@ -156,7 +159,7 @@ struct GatedNormFn : torch::autograd::Function<GatedNormFn> {
     ctx->save_for_backward({x2, weight, tensor_or_none(bias), tensor_or_none(mean), rstd, tensor_or_none(z2)});
     ctx->saved_data["o"] = std::vector<int64_t>{o.group_size, o.norm_before_gate, o.is_rms};
     ctx->saved_data["eps"] = o.eps;
-    return y.view(x.sizes());
+    return shaped(y, x.sizes());
   }
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const variable_list s = ctx->get_saved_variables();
@@ -165,10 +168,10 @@ struct GatedNormFn : torch::autograd::Function<GatedNormFn> {
     const at::Tensor dy = rows_of(grads[0]).to(s[0].scalar_type());
     auto [dx, dw, db, dz] = gated_norm_bwd(dy, s[0], s[1], opt(s[2]), opt(s[3]), s[4], opt(s[5]), std::nullopt, o);
     variable_list g(5);
-    g[0] = dx.view(grads[0].sizes());
+    g[0] = shaped(dx, grads[0].sizes());
     g[1] = dw;
     if (db) g[2] = *db;
-    if (dz) g[3] = dz->view(grads[0].sizes());
+    if (dz) g[3] = shaped(*dz, grads[0].sizes());
     return g;
   }
 };
@@ -180,7 +183,7 @@ OptTensor norm_gated(const at::Tensor &x, const at::Tensor &weight, const OptTen
   const GatedNorm o{group_size.value_or(x.size(-1)), eps, norm_before_gate, is_rms};
   if (!gated_norm_ok(x, weight, bias, z, o)) return std::nullopt;
   if (!records(x, weight, bias, z))
-    return std::get<0>(gated_norm_fwd(rows_of(x), weight, bias, z ? OptTensor(rows_of(*z)) : std::nullopt, o)).view(x.sizes());
+    return shaped(std::get<0>(gated_norm_fwd(rows_of(x), weight, bias, z ? OptTensor(rows_of(*z)) : std::nullopt, o)), x.sizes());
   return GatedNormFn::apply(x, weight, bias, z, o);
 }
 

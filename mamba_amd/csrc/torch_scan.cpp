@@ -31,6 +31,9 @@ bool fill_scan(MambaScanParams &p, const at::Tensor &u, const at::Tensor &delta,
   for (const at::Tensor *t : {&B, &C}) {
     if (t->dim() == 2) {
       if (t->scalar_type() != at::kFloat || t->size(0) != dim || t->size(1) != N || !t->is_contiguous()) return false;
+    } else if (t->dim() == 3) {  // one group, without its axis
+      if (G != 1 || t->scalar_type() != u.scalar_type() || t->stride(2) != 1 || t->size(0) != batch || t->size(1) != N || t->size(2) != L)
+        return false;
     } else if (t->dim() == 4) {
       if (t->scalar_type() != u.scalar_type() || t->stride(3) != 1 || t->size(0) != batch || t->size(1) != G ||
           t->size(2) != N || t->size(3) != L)
@@ -51,8 +54,11 @@ bool fill_scan(MambaScanParams &p, const at::Tensor &u, const at::Tensor &delta,
   p.D = ptr(D), p.z = ptr(z), p.delta_bias = ptr(delta_bias);
   p.u_bs = u.stride(0), p.u_ds = u.stride(1), p.delta_bs = delta.stride(0), p.delta_ds = delta.stride(1);
   if (z) p.z_bs = z->stride(0), p.z_ds = z->stride(1);
-  if (B.dim() == 4) p.B_bs = B.stride(0), p.B_gs = B.stride(1), p.B_ns = B.stride(2);
-  if (C.dim() == 4) p.C_bs = C.stride(0), p.C_gs = C.stride(1), p.C_ns = C.stride(2);
+  auto bc_strides = [](const at::Tensor &t, int64_t &bs, int64_t &gs, int64_t &ns) {
+    if (t.dim() > 2) bs = t.stride(0), gs = t.dim() == 4 ? t.stride(1) : 0, ns = t.stride(t.dim() - 2);
+  };
+  bc_strides(B, p.B_bs, p.B_gs, p.B_ns);
+  bc_strides(C, p.C_bs, p.C_gs, p.C_ns);
   return true;
 }
 
@@ -130,13 +136,13 @@ TensorList scan_bwd(MambaScanParams &p, const at::Tensor &u, const at::Tensor &d
   const int64_t dim = p.dim, N = p.dstate;
   at::Tensor du = at::empty_like(u), ddelta = at::empty_like(delta);
   OptTensor dB, dC, dz, out_z;
-  if (B.dim() == 4) {
-    dB = at::empty({p.batch, p.ngroups, N, p.seqlen}, B.options());
-    p.dB = ptr(dB), p.dB_bs = dB->stride(0), p.dB_gs = dB->stride(1), p.dB_ns = dB->stride(2);
+  if (B.dim() > 2) {
+    dB = at::empty(B.sizes(), B.options());
+    p.dB = ptr(dB), p.dB_ns = p.seqlen, p.dB_gs = N * p.dB_ns, p.dB_bs = p.ngroups * p.dB_gs;
   }
-  if (C.dim() == 4) {
-    dC = at::empty({p.batch, p.ngroups, N, p.seqlen}, C.options());
-    p.dC = ptr(dC), p.dC_bs = dC->stride(0), p.dC_gs = dC->stride(1), p.dC_ns = dC->stride(2);
+  if (C.dim() > 2) {
+    dC = at::empty(C.sizes(), C.options());
+    p.dC = ptr(dC), p.dC_ns = p.seqlen, p.dC_gs = N * p.dC_ns, p.dC_bs = p.ngroups * p.dC_gs;
   }
   if (z) {
     dz = dz_in ? *dz_in : at::empty_like(*z);
@@ -181,17 +187,14 @@ std::optional<TensorList> scan_bwd_fast(const at::Tensor &u, const at::Tensor &d
 }
 
 // ------------------------------------------------------------------ selective_scan_fn
-struct ScanArgs {  // as the kernels take them: unit last strides, B / C with a group axis
+struct ScanArgs {  // as the kernels take them: unit last strides
   at::Tensor u, delta, A, B, C;
   OptTensor D, z, delta_bias;
 };
 at::Tensor unit_last(const at::Tensor &t) { return t.stride(-1) == 1 ? t : t.contiguous(); }
 ScanArgs normalised(const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A, const at::Tensor &B, const at::Tensor &C,
                     const OptTensor &D, const OptTensor &z, const OptTensor &delta_bias) {
-  auto bc = [](const at::Tensor &t) {
-    const at::Tensor r = t.dim() == 2 ? t.contiguous() : unit_last(t);
-    return r.dim() == 3 ? r.unsqueeze(1) : r;
-  };
+  auto bc = [](const at::Tensor &t) { return t.dim() == 2 ? t.contiguous() : unit_last(t); };
   ScanArgs a{unit_last(u), unit_last(delta), A.contiguous(), bc(B), bc(C), std::nullopt, std::nullopt, delta_bias};
   if (D) a.D = D->contiguous();
   if (z) a.z = unit_last(*z);
@@ -208,7 +211,6 @@ struct ScanFn : torch::autograd::Function<ScanFn> {
     auto [out, ckpt] = scan_fwd(p, a.u, a.delta);
     ctx->save_for_backward({a.u, a.delta, a.A, a.B, a.C, tensor_or_none(a.D), tensor_or_none(a.z), tensor_or_none(a.delta_bias), ckpt});
     ctx->saved_data["softplus"] = delta_softplus;
-    ctx->saved_data["squeeze"] = std::vector<int64_t>{B.dim() == 3, C.dim() == 3};
     ctx->set_materialize_grads(false);
     variable_list r = {out};
     if (return_last_state) r.push_back(ckpt.select(2, ckpt.size(2) - 1));
@@ -223,11 +225,9 @@ struct ScanFn : torch::autograd::Function<ScanFn> {
     MambaScanParams p{};
     TORCH_CHECK(fill_scan(p, s[0], s[1], s[2], s[3], s[4], D, z, bias, ctx->saved_data["softplus"].toBool()), "selective_scan: arguments");
     const TensorList r = scan_bwd(p, s[0], s[1], s[3], s[4], D, z, bias, dout, s[8], std::nullopt, false);
-    const std::vector<int64_t> squeeze = ctx->saved_data["squeeze"].toIntVector();
     variable_list g(10);
     g[0] = *r[0], g[1] = *r[1], g[2] = *r[2];
-    g[3] = squeeze[0] ? r[3]->squeeze(1) : *r[3];
-    g[4] = squeeze[1] ? r[4]->squeeze(1) : *r[4];
+    g[3] = *r[3], g[4] = *r[4];
     g[5] = tensor_or_none(r[5]), g[6] = tensor_or_none(r[7]), g[7] = tensor_or_none(r[6]);
     return g;
   }

@@ -63,6 +63,25 @@ bool fill_ssd(SsdParams &p, SsdDims &d, const at::Tensor &x, const at::Tensor &d
   return true;
 }
 
+// The chunk length the kernels use for a call that names one of 64, 128 and 256: the scan's result is the same for each
+// but for rounding, and they differ in cost.  A longer chunk writes and reads fewer chunk states (headdim x dstate per
+// head), a shorter one has less of the quadratic part: the (chunk x chunk) tiles of dCB per group, and the causal
+// triangle's work.  256 wins with one group of 128 states where its chunks keep the chip busy, and wherever the states
+// after every 128 positions would outgrow the 256 MB last-level cache; otherwise 128.  Measured (64 / 128 / 256, us,
+// forward + backward in bf16): 2 x 7093 x 40 heads, 1 group, 128 states 663 / 559 / 476; 4039 x 72 heads, 8 groups, 128
+// states 402 / 339 / 391, but 32768 x 64 heads 2268 / 2050 (128 / 256); 13632 x 64 heads, 1 group, 64 states 926 / 765 /
+// 829; 1216 x 32 heads, 1 group, 128 states 122 / 124 / 143; fp16, 2 x 2257 x 80 heads, 8 groups, 64 states 641 / 590 /
+// 646.  A sequence within one chunk of 64 or 128 takes that.
+int64_t kernel_chunk(int64_t chunk_size, int64_t batch, int64_t L, int64_t H, int64_t G, int64_t P, int64_t N, at::ScalarType type) {
+  if (chunk_size != 64 && chunk_size != 128 && chunk_size != 256) return chunk_size;
+  if (L <= 128) return L <= 64 ? 64 : 128;
+  const bool fills = batch * H * ((L + 255) / 256) >= 384;  // one and a half workgroups for each of the 256 CUs
+  const bool cached = batch * H * ((L + 127) / 128) * P * N * 4 <= (256 << 20);
+  if ((type == at::kBFloat16 && G == 1 && N > 64 && fills) || !cached) return 256;
+  // (in the split-operand types short calls are a little faster with the chunk of 64 where the caller asks for it)
+  return type != at::kBFloat16 && !fills ? std::min<int64_t>(128, chunk_size) : 128;
+}
+
 // Everything a forward or backward call of mamba_chunk_scan_combined takes, apart from its outputs.
 struct SsdArgs {
   at::Tensor x, dt, A, B, C;
@@ -128,9 +147,10 @@ TensorList ssd_bwd(SsdParams &p, const SsdDims &d, const SsdArgs &a, const at::T
   const int64_t sizes[8] = {d.H, d.H, nD, nHcQ, nHcQ, nCB, nBC, nBC};  // the five small ones first
   int64_t total = 0, off[8];
   for (int i = 0; i < 8; ++i) {
-    if (i == 5) total = (total + 63) / 64 * 64;  // the large ones start on 256 bytes
+    if (i >= 5) total = (total + 63) / 64 * 64;  // the large ones start on 256 bytes
     off[i] = total, total += sizes[i];
   }
+  total = (total + 63) / 64 * 64;
   at::Tensor arena = at::empty({total}, f32);
   float *base = arena.data_ptr<float>();
   at::Tensor dstates = at::empty({d.batch, d.nchunks, d.H, d.P, d.N}, d.lp ? x.options() : f32);
@@ -156,14 +176,14 @@ TensorList ssd_bwd(SsdParams &p, const SsdDims &d, const SsdArgs &a, const at::T
   p.dB_bs = dB.stride(0), p.dB_ls = dB.stride(1), p.dB_gs = dB.stride(2);
   p.dC_bs = dC.stride(0), p.dC_ls = dC.stride(1), p.dC_gs = dC.stride(2);
   const int owned = ssd_bwd_overwrites(&p);
-  if (owned == 0) {
-    arena.zero_();  // one fill
-  } else {
-    arena.narrow(0, 0, off[5]).zero_();
-    if (!(owned & SSD_OVERWRITES_DCB)) arena.narrow(0, off[5], nCB).zero_();
-    if (!(owned & SSD_OVERWRITES_DBC)) arena.narrow(0, off[6], 2 * nBC).zero_();  // dB32 and dC32 are neighbours
-  }
   void *stream = stream_of(dev);
+  {
+    int64_t at[3] = {0}, n[3] = {off[5]};
+    int count = 1;
+    if (!(owned & SSD_OVERWRITES_DCB)) at[count] = off[5], n[count++] = off[6] - off[5];
+    if (!(owned & SSD_OVERWRITES_DBC)) at[count] = off[6], n[count++] = total - off[6];
+    check_rc(ssd_clear(base, at, n, count, stream), "ssd_clear");
+  }
   // CB: the fused forward never forms it; the backward kernels may not need it either
   at::Tensor CB;
   if (!(owned & SSD_BWD_FORMS_CB)) {
@@ -172,13 +192,12 @@ TensorList ssd_bwd(SsdParams &p, const SsdDims &d, const SsdArgs &a, const at::T
     check_rc(ssd_bmm_chunk_fwd(&p, stream), "ssd_bmm_chunk_fwd");
   }
   check_rc(ssd_combined_bwd(&p, stream), "ssd_combined_bwd");
-  auto piece = [&](int i, at::IntArrayRef shape) { return arena.narrow(0, off[i], sizes[i]).view(shape); };
   TensorList r(9);
-  r[0] = dx, r[1] = ddt, r[2] = piece(0, {d.H});
+  r[0] = dx, r[1] = ddt, r[2] = arena.as_strided({d.H}, {1}, off[0]);
   r[3] = dB, r[4] = dC;
-  if (a.D) r[5] = piece(2, a.D->sizes());
+  if (a.D) r[5] = a.D->dim() == 2 ? arena.as_strided({d.H, d.P}, {d.P, 1}, off[2]) : arena.as_strided({d.H}, {1}, off[2]);
   r[6] = dz;
-  if (a.dt_bias) r[7] = piece(1, {d.H});
+  if (a.dt_bias) r[7] = arena.as_strided({d.H}, {1}, off[1]);
   r[8] = dinit;
   return r;
 }
@@ -312,6 +331,8 @@ pybind11::object chunk_scan(const at::Tensor &x, const at::Tensor &dt, const at:
                             int64_t chunk_size, const OptTensor &D, const OptTensor &z, const OptTensor &dt_bias,
                             const OptTensor &initial_states, const OptTensor &seq_idx, bool dt_softplus, double dt_min,
                             double dt_max, bool return_final) {
+  if (x.dim() == 4 && B.dim() == 4)
+    chunk_size = kernel_chunk(chunk_size, x.size(0), x.size(1), x.size(2), B.size(2), x.size(3), B.size(3), x.scalar_type());
   SsdParams p{};
   SsdDims d;
   const SsdArgs a{x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states, seq_idx, dt_softplus, dt_min, dt_max};
@@ -337,25 +358,29 @@ struct BlockOptions {
 };
 constexpr int BLOCK_NARGS = 13;
 
-// The slices of a (batch, seqlen, ...) projection and of the convolution's output
-struct Slices {
-  at::Tensor z, xBC, dt;
-};
-Slices split_projection(const at::Tensor &t, int64_t dim, int64_t conv) {
-  return {t.narrow(2, 0, dim), t.narrow(2, dim, conv), t.narrow(2, dim + conv, t.size(2) - dim - conv)};
+// Slices of a (batch, seqlen, ...) tensor with unit last stride, from channel `at` on: as rows per (batch, position)
+// (which follow one another, see split_conv_scan), as heads (batch, seqlen, n0, n1), as rows of a convolution
+at::Tensor row_slice(const at::Tensor &t, int64_t at, int64_t n) {
+  return t.as_strided({t.size(0) * t.size(1), n}, {t.stride(1), 1}, t.storage_offset() + at);
 }
-struct Operands {
-  at::Tensor x, B, C;
-};
-Operands split_conv(const at::Tensor &t, int64_t H, int64_t P, int64_t G, int64_t N) {  // t: (batch, seqlen, conv) dense
-  const int64_t b = t.size(0), L = t.size(1), bs = t.stride(0), ls = t.stride(1), o = t.storage_offset();
-  return {t.as_strided({b, L, H, P}, {bs, ls, P, 1}, o), t.as_strided({b, L, G, N}, {bs, ls, N, 1}, o + H * P),
-          t.as_strided({b, L, G, N}, {bs, ls, N, 1}, o + H * P + G * N)};
+at::Tensor head_slice(const at::Tensor &t, int64_t at, int64_t n0, int64_t n1) {
+  return t.as_strided({t.size(0), t.size(1), n0, n1}, {t.stride(0), t.stride(1), n1, 1}, t.storage_offset() + at);
 }
-at::Tensor heads(const at::Tensor &t, int64_t H, int64_t P) {  // (batch, seqlen, H P) with unit last stride -> (.., H, P)
-  return t.as_strided({t.size(0), t.size(1), H, P}, {t.stride(0), t.stride(1), P, 1}, t.storage_offset());
+at::Tensor step_slice(const at::Tensor &t, int64_t at, int64_t n) {
+  return t.as_strided({t.size(0), t.size(1), n}, {t.stride(0), t.stride(1), 1}, t.storage_offset() + at);
 }
-at::Tensor flat_rows(const at::Tensor &t) { return t.reshape({t.size(0) * t.size(1), t.size(2)}); }
+ConvRows conv_rows(const at::Tensor &t, int64_t at) {
+  return {static_cast<char *>(t.data_ptr()) + at * t.element_size(), t.stride(0), 1, t.stride(1)};
+}
+
+SsdArgs args_of(const at::Tensor &zxbcdt, const at::Tensor &xBC, const at::Tensor &A, const at::Tensor &D, bool gate,
+                const at::Tensor &dt_bias, const OptTensor &initial_states, const OptTensor &seq_idx, int64_t H, int64_t P, int64_t G,
+                int64_t N, const SsdOptions &o) {
+  const int64_t dim = H * P;
+  return {head_slice(xBC, 0, H, P), step_slice(zxbcdt, dim + xBC.size(2), H), A, head_slice(xBC, dim, G, N), head_slice(xBC, dim + G * N, G, N),
+          o.chunk_size, D, gate ? OptTensor(head_slice(zxbcdt, 0, H, P)) : std::nullopt, dt_bias, initial_states, seq_idx, true, o.dt_min,
+          o.dt_max};
+}
 
 struct BlockFn : torch::autograd::Function<BlockFn> {
   static variable_list forward(AutogradContext *ctx, const at::Tensor &zxbcdt, const at::Tensor &conv_weight, const OptTensor &conv_bias,
@@ -363,15 +388,12 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
                                const OptTensor &seq_idx, const OptTensor &norm_weight, const OptTensor &out_weight,
                                const OptTensor &out_bias, const BlockOptions &o, std::optional<at::ScalarType> autocast) {
     const int64_t H = D.size(0), P = o.headdim, G = o.ngroups, dim = H * P, batch = zxbcdt.size(0), L = zxbcdt.size(1);
-    const at::Tensor conv_w = conv_weight.dim() == 3 ? conv_weight.squeeze(1) : conv_weight;
+    const at::Tensor &conv_w = conv_weight;
     const int64_t conv = conv_w.size(0), N = (conv - dim) / (2 * G);
-    const Slices s = split_projection(zxbcdt, dim, conv);
     at::Tensor xBC = at::empty({batch, L, conv}, zxbcdt.options());
-    conv_fwd(s.xBC.transpose(1, 2), conv_w, conv_bias, seq_idx, o.silu, xBC.transpose(1, 2));
-    const Operands q = split_conv(xBC, H, P, G, N);
+    conv_fwd(zxbcdt, batch, conv, L, conv_rows(zxbcdt, dim), conv_w, conv_bias, seq_idx, o.silu, conv_rows(xBC, 0));
     const bool gate_in_scan = !norm_weight;
-    const SsdArgs a{q.x, s.dt, A, q.B, q.C, o.ssd.chunk_size, D, gate_in_scan ? OptTensor(heads(s.z, H, P)) : std::nullopt, dt_bias,
-                    initial_states, seq_idx, true, o.ssd.dt_min, o.ssd.dt_max};
+    const SsdArgs a = args_of(zxbcdt, xBC, A, D, gate_in_scan, dt_bias, initial_states, seq_idx, H, P, G, N, o.ssd);
     SsdParams p{};
     SsdDims d;
     TORCH_CHECK(fill_ssd(p, d, a), "mamba_split_conv1d_scan_combined: arguments");
@@ -380,7 +402,7 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
     OptTensor rstd;
     if (norm_weight) {
       // reads z where it lies inside zxbcdt (unit channel stride, row stride of the whole projection)
-      auto [yn, mean, rs] = gated_norm_fwd(y, *norm_weight, std::nullopt, flat_rows(s.z), {dim / G, o.eps, o.norm_before_gate, true});
+      auto [yn, mean, rs] = gated_norm_fwd(y, *norm_weight, std::nullopt, row_slice(zxbcdt, 0, dim), {dim / G, o.eps, o.norm_before_gate, true});
       y = yn, rstd = rs;
     }
     at::Tensor res = y, w;
@@ -404,7 +426,7 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
                             tensor_or_none(rstd), w, out_weight ? y : at::Tensor()});
     ctx->set_materialize_grads(false);
     save_options(ctx, o.ssd);
-    ctx->saved_data["b"] = std::vector<int64_t>{P, G, o.silu, o.norm_before_gate, conv_weight.dim() == 3, out_bias.has_value(), out_weight ? (int64_t)out_weight->scalar_type() : 0,
+    ctx->saved_data["b"] = std::vector<int64_t>{P, G, o.silu, o.norm_before_gate, 0, out_bias.has_value(), out_weight ? (int64_t)out_weight->scalar_type() : 0,
                                                 out_bias ? (int64_t)out_bias->scalar_type() : 0};
     ctx->saved_data["eps"] = o.eps;
     variable_list out = {res.view({batch, L, -1})};
@@ -420,9 +442,7 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
     const int64_t H = D.size(0), P = v[0], G = v[1], dim = H * P, batch = zxbcdt.size(0), L = zxbcdt.size(1), conv = conv_w.size(0);
     const int64_t N = (conv - dim) / (2 * G);
     c10::DeviceGuard guard(zxbcdt.device());
-    const Slices sl = split_projection(zxbcdt, dim, conv);
-    at::Tensor dzxbcdt = at::empty_like(zxbcdt);
-    const Slices ds = split_projection(dzxbcdt, dim, conv);
+    at::Tensor dzxbcdt = at::empty(zxbcdt.sizes(), zxbcdt.options());
     variable_list g(BLOCK_NARGS);
     at::Tensor dy;
     if (w.defined()) {
@@ -445,22 +465,22 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
     if (norm_weight) {
       const GatedNorm o{dim / G, ctx->saved_data["eps"].toDouble(), v[3] != 0, true};
       auto [dx, dw, db, dz] = gated_norm_bwd(dy, scan_out.view({batch * L, dim}), *norm_weight, std::nullopt, std::nullopt, s[14],
-                                             flat_rows(sl.z), flat_rows(ds.z), o);
+                                             row_slice(zxbcdt, 0, dim), row_slice(dzxbcdt, 0, dim), o);
       dy = dx;
       g[8] = dw;
     }
-    const Operands q = split_conv(xBC, H, P, G, N);
-    at::Tensor dxBC = at::empty_like(xBC);
-    const Operands dq = split_conv(dxBC, H, P, G, N);
-    const SsdArgs a{q.x, sl.dt, s[8], q.B, q.C, so.chunk_size, D, norm_weight ? std::nullopt : OptTensor(heads(sl.z, H, P)), s[10],
-                    opt(s[11]), opt(s[12]), true, so.dt_min, so.dt_max};
+    at::Tensor dxBC = at::empty(xBC.sizes(), xBC.options());
+    const SsdArgs a = args_of(zxbcdt, xBC, s[8], D, !norm_weight, s[10], opt(s[11]), opt(s[12]), H, P, G, N, so);
     OptTensor dfinal;
     if (so.return_final && grads[1].defined()) dfinal = grads[1].to(at::kFloat).contiguous();
-    const TensorList r = ssd_bwd_any(a, dy.view({batch, L, H, P}), scan_out, dfinal, s[5], s[6], s[7], {dq.x, ds.dt, dq.B, dq.C});
-    if (!norm_weight) ds.z.copy_(r[6]->view({batch, L, dim}));
+    const TensorList r = ssd_bwd_any(a, dy.view({batch, L, H, P}), scan_out, dfinal, s[5], s[6], s[7],
+                                     {head_slice(dxBC, 0, H, P), step_slice(dzxbcdt, dim + conv, H), head_slice(dxBC, dim, G, N),
+                                      head_slice(dxBC, dim + G * N, G, N)});
+    if (!norm_weight) row_slice(dzxbcdt, 0, dim).copy_(r[6]->view({batch * L, dim}));
     // the convolution's backward kernel re-computes its pre-activation from xBC and writes into the xBC slice
-    auto [dcw, dcb] = conv_bwd(sl.xBC.transpose(1, 2), conv_w, conv_bias, dxBC.transpose(1, 2), opt(s[12]), v[2] != 0, ds.xBC.transpose(1, 2));
-    g[0] = dzxbcdt, g[1] = v[4] ? dcw.unsqueeze(1) : dcw, g[2] = tensor_or_none(dcb), g[3] = *r[7], g[4] = *r[2], g[5] = *r[5];
+    auto [dcw, dcb] = conv_bwd(zxbcdt, batch, conv, L, conv_rows(zxbcdt, dim), conv_w, conv_bias, conv_rows(dxBC, 0), opt(s[12]), v[2] != 0,
+                               conv_rows(dzxbcdt, dim));
+    g[0] = dzxbcdt, g[1] = dcw, g[2] = tensor_or_none(dcb), g[3] = *r[7], g[4] = *r[2], g[5] = *r[5];
     g[6] = tensor_or_none(r[8]);
     return g;
   }
@@ -486,20 +506,20 @@ pybind11::object split_conv_scan(const at::Tensor &zxbcdt_in, const at::Tensor &
   if (H <= 0 || P <= 0 || H % G != 0 || conv <= dim || (conv - dim) % (2 * G) != 0 || batch <= 0 || L <= 0) return no;
   const int64_t N = (conv - dim) / (2 * G);
   if (zxbcdt.size(2) != dim + conv + H || dt_bias.dim() != 1 || dt_bias.size(0) != H || A.dim() != 1 || A.size(0) != H) return no;
-  const Slices s = split_projection(zxbcdt, dim, conv);
+  chunk_size = kernel_chunk(chunk_size, batch, L, H, G, P, N, zxbcdt.scalar_type());
   const at::Tensor conv_w = conv_weight.dim() == 3 ? conv_weight.squeeze(1) : conv_weight;
-  if (!conv_params_ok(s.xBC.transpose(1, 2), conv_w, conv_bias, seq_idx)) return no;
-  // the scan's own checks, on the operands' shapes and dtypes (x, B and C will be slices of a fresh buffer)
+  const at::Tensor xBC_in = zxbcdt.as_strided({batch, conv, L}, {zxbcdt.stride(0), 1, zxbcdt.stride(1)}, zxbcdt.storage_offset() + dim);
+  if (!conv_params_ok(xBC_in, conv_w, conv_bias, seq_idx)) return no;
+  // the scan's own checks, on operands of the right shapes and dtypes (x, B and C will be slices of a fresh buffer)
   SsdParams p{};
   SsdDims d;
-  const at::Tensor xBC = s.xBC;
-  auto cut = [&](int64_t at, int64_t n0, int64_t n1) {
-    return xBC.as_strided({batch, L, n0, n1}, {xBC.stride(0), xBC.stride(1), n1, 1}, xBC.storage_offset() + at);
-  };
-  if (!fill_ssd(p, d, cut(0, H, P), s.dt, A, cut(dim, G, N), cut(dim + G * N, G, N), chunk_size, D,
-                norm_weight ? std::nullopt : OptTensor(heads(s.z, H, P)), dt_bias, initial_states, seq_idx, true, dt_min, dt_max))
-    return no;
-  if (norm_weight && !gated_norm_ok(zxbcdt.narrow(2, 0, dim), *norm_weight, std::nullopt, std::nullopt, {dim / G, eps, norm_before_gate, true}))
+  const SsdOptions so{chunk_size, true, return_final, dt_min, dt_max};
+  SsdArgs a{head_slice(zxbcdt, dim, H, P), step_slice(zxbcdt, dim + conv, H), A, head_slice(zxbcdt, 2 * dim, G, N),
+            head_slice(zxbcdt, 2 * dim + G * N, G, N), chunk_size, D, std::nullopt, dt_bias, initial_states, seq_idx, true, dt_min, dt_max};
+  if (!norm_weight) a.z = head_slice(zxbcdt, 0, H, P);
+  if (!fill_ssd(p, d, a)) return no;
+  if (norm_weight &&
+      !gated_norm_ok(row_slice(zxbcdt, 0, dim), *norm_weight, std::nullopt, std::nullopt, {dim / G, eps, norm_before_gate, true}))
     return no;
   std::optional<at::ScalarType> autocast;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) autocast = at::autocast::get_autocast_dtype(at::kCUDA);
@@ -511,7 +531,7 @@ pybind11::object split_conv_scan(const at::Tensor &zxbcdt_in, const at::Tensor &
     return no;
   }
   c10::DeviceGuard guard(dev);
-  const BlockOptions o{{chunk_size, true, return_final, dt_min, dt_max}, P, G, eps, silu, norm_before_gate};
+  const BlockOptions o{so, P, G, eps, silu, norm_before_gate};
   variable_list r = BlockFn::apply(zxbcdt, conv_weight, conv_bias, dt_bias, A, D, initial_states, seq_idx, norm_weight, out_weight,
                                    out_bias, o, autocast);
   return return_final ? pybind11::object(pybind11::make_tuple(r[0], r[1])) : pybind11::cast(r[0]);

@@ -206,8 +206,7 @@ def causal_conv1d_update(x, conv_state, weight, bias=None, activation=None, cach
     ext = _lib.torch_ext()
     if ext is not None:
         # the same checks and launch in C++; None = it declined, and the code below handles the call
-        out = ext.causal_conv1d_update(x, conv_state, weight.detach(), None if bias is None else bias.detach(),
-                                       activation is not None, cache_seqlens, conv_state_indices)
+        out = ext.causal_conv1d_update(x, conv_state, weight, bias, activation is not None, cache_seqlens, conv_state_indices)
         if out is not None:
             return out
     _lib.require_gpu(x, conv_state, weight, bias, conv_state_indices)

@@ -90,18 +90,32 @@ DEVI void store_row(T *row, int col, int gs, const float (&v)[K][8]) {
   }
 }
 
-// The norm's parameters of this thread's channels, zero past the end
+// The norm's parameters of this thread's channels, zero past the end.  The kernels call it after they have requested
+// their first row: the conversion waits for the loads, and that wait is then the row's as well.
 template <int K, int TEAM>
 DEVI void load_params(const void *base, int dtype, int64_t off, int col, int gs, float (&v)[K][8]) {
+  auto run = [&](auto *src) {
+    typedef std::remove_const_t<std::remove_pointer_t<decltype(src)>> W;
+    Pack8<W> q[K];
 #pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const int c = col + k * TEAM * 8;
-    if (c + 8 <= gs) {
-      ld8_param(base, dtype, off + c, v[k]);
-    } else {
+    for (int k = 0; k < K; ++k) {
+      const int c = col + k * TEAM * 8;
+      if (c + 8 <= gs) {
+        q[k].load_any(src + off + c);
+      } else {
+        float t[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[k][e] = c + e < gs ? ld_param(base, dtype, off + c + e) : 0.f;
+        for (int e = 0; e < 8; ++e) t[e] = c + e < gs ? ld1<W>(src + off + c + e) : 0.f;
+        q[k].pack(t);
+      }
     }
+#pragma unroll
+    for (int k = 0; k < K; ++k) q[k].unpack(v[k]);
+  };
+  switch (dtype) {
+    case MAMBA_BF16: run(static_cast<const bf16_t *>(base)); break;
+    case MAMBA_F16: run(static_cast<const f16_t *>(base)); break;
+    default: run(static_cast<const float *>(base)); break;
   }
 }
 

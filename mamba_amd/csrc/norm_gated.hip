@@ -45,9 +45,6 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_fwd_kernel(const
   if (!it.live) return;  // whole teams only; a team of more than one wave is a whole workgroup
   const int gs = p.group_size, ngroups = p.dim / gs;
   const int64_t g0 = (int64_t)it.group * gs;
-  float w[K][8], b[K][8];
-  load_params<K, TEAM>(p.weight, p.weight_dtype, g0, it.col, gs, w);
-  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, g0, it.col, gs, b);
   const T *xp = static_cast<const T *>(p.x) + g0;
   const T *zp = p.z ? static_cast<const T *>(p.z) + g0 : nullptr;
   T *op = static_cast<T *>(p.out) + g0;
@@ -57,6 +54,9 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_fwd_kernel(const
     bx.fetch(xp + it.part * p.x_rs, it.col, gs);
     if (zp) bz.fetch(zp + it.part * p.z_rs, it.col, gs);
   }
+  float w[K][8], b[K][8];
+  load_params<K, TEAM>(p.weight, p.weight_dtype, g0, it.col, gs, w);
+  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, g0, it.col, gs, b);
   for (int r = it.part; r < p.rows; r += nparts) {
     float x[K][8], sz[K][8];
     bx.get(x);
@@ -124,8 +124,6 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_bwd_kernel(const
   const int gs = p.group_size, ngroups = p.dim / gs;
   const int64_t g0 = (int64_t)it.group * gs;
   float w[K][8], b[K][8], dw[K][8], db[K][8];
-  load_params<K, TEAM>(p.weight, p.weight_dtype, g0, it.col, gs, w);
-  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, g0, it.col, gs, b);
 #pragma unroll
   for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -148,6 +146,8 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_bwd_kernel(const
     bg.fetch(gp + it.part * p.dy_rs, it.col, gs);
     if (zp) bz.fetch(zp + it.part * p.z_rs, it.col, gs);
   }
+  load_params<K, TEAM>(p.weight, p.weight_dtype, g0, it.col, gs, w);
+  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, g0, it.col, gs, b);
   for (int r = it.part; r < p.rows; r += nparts) {
     float x[K][8], z[K][8], g[K][8];
     bx.get(x);
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_bwd_kernel(const
 // The forward pass in the same form as norm_bwd_wide_kernel (below): a part of the rows per workgroup, the next
 // row requested before the current one is used, no branch around a row's loads or stores.
 template <typename T, bool HAS_Z>
-__global__ __launch_bounds__(1024, 8) void norm_fwd_wide_kernel(const NormGatedParams p, int nparts) {
+__global__ __launch_bounds__(1024, sizeof(T) == 4 ? 5 : 8) void norm_fwd_wide_kernel(const NormGatedParams p, int nparts) {
   __shared__ __align__(16) float lds[64];
   WideSum ts(lds);
   const int gs = p.group_size, ngroups = p.dim / gs, rows = p.rows;
@@ -231,10 +231,8 @@ __global__ __launch_bounds__(1024, 8) void norm_fwd_wide_kernel(const NormGatedP
   if (part >= rows) return;
   const int64_t c0 = (int64_t)group * gs + col;
   float w[8], b[8];
-  ld8_param(p.weight, p.weight_dtype, c0, w);
 #pragma unroll
   for (int e = 0; e < 8; ++e) b[e] = 0.f;
-  if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
   const T *xp = static_cast<const T *>(p.x) + c0;
   const T *zp = HAS_Z ? static_cast<const T *>(p.z) + c0 : xp;
   T *op = static_cast<T *>(p.out) + c0;
@@ -244,6 +242,8 @@ __global__ __launch_bounds__(1024, 8) void norm_fwd_wide_kernel(const NormGatedP
   Pack8<T> cx, cz;
   cx.load_global(xp + (int64_t)part * p.x_rs);
   if (HAS_Z) cz.load_global(zp + (int64_t)part * p.z_rs);
+  ld8_param(p.weight, p.weight_dtype, c0, w);
+  if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
   for (int r = part; r < rows; r += nparts) {
     const int rn = min(r + nparts, last);
     Pack8<T> nx, nz;
@@ -313,10 +313,8 @@ __global__ __launch_bounds__(1024) void norm_bwd_wide_kernel(const NormGatedPara
   const int col = min((int)threadIdx.x * 8, gs - 8);
   const int64_t c0 = (int64_t)group * gs + col;
   float w[8], b[8], dw[8], db[8];
-  ld8_param(p.weight, p.weight_dtype, c0, w);
 #pragma unroll
   for (int e = 0; e < 8; ++e) b[e] = dw[e] = db[e] = 0.f;
-  if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
   const T *xp = static_cast<const T *>(p.x) + c0;
   const T *gp = static_cast<const T *>(p.dy) + c0;
   const T *zp = HAS_Z ? static_cast<const T *>(p.z) + c0 : xp;
@@ -333,6 +331,8 @@ __global__ __launch_bounds__(1024) void norm_bwd_wide_kernel(const NormGatedPara
     cx.load_global(xp + (int64_t)part * p.x_rs);
     cg.load_global(gp + (int64_t)part * p.dy_rs);
     if (HAS_Z) cz.load_global(zp + (int64_t)part * p.z_rs);
+    ld8_param(p.weight, p.weight_dtype, c0, w);
+    if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
     for (int r = part; r < rows; r += nparts) {
       const int rn = min(r + nparts, last);
       Pack8<T> nx, ng, nz;

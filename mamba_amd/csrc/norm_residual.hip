@@ -54,9 +54,6 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_fwd_kernel(c
   int part, col;
   if (!my_part<TEAM>(nparts, part, col)) return;
   const int n = p.dim;
-  float w[K][8], b[K][8];
-  load_params<K, TEAM>(p.weight, p.weight_dtype, 0, col, n, w);
-  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, 0, col, n, b);
   const T *xp = static_cast<const T *>(p.x);
   const R *rp = static_cast<const R *>(p.residual);
   T *op = static_cast<T *>(p.out);
@@ -72,6 +69,9 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_fwd_kernel(c
     bx.fetch(xp + part * p.x_rs, col, n);
     if (rp) br.fetch(rp + part * p.residual_rs, col, n);
   }
+  float w[K][8], b[K][8];
+  load_params<K, TEAM>(p.weight, p.weight_dtype, 0, col, n, w);
+  if (p.bias) load_params<K, TEAM>(p.bias, p.weight_dtype, 0, col, n, b);
   for (int r = part; r < p.rows; r += nparts) {
     float x[K][8];
     bx.get(x);
@@ -170,7 +170,6 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_bwd_kernel(c
   if (!my_part<TEAM>(nparts, part, col)) return;
   const int n = p.dim;
   float w[K][8], dw[K][8], db[K][8];
-  load_params<K, TEAM>(p.weight, p.weight_dtype, 0, col, n, w);
 #pragma unroll
   for (int k = 0; k < K; ++k)
 #pragma unroll
@@ -201,6 +200,7 @@ __global__ __launch_bounds__(TEAM < 256 ? 256 : TEAM) void norm_res_bwd_kernel(c
     bg.fetch(gp + part * p.dy_rs, col, n);
     if (drp) bd.fetch(drp + part * p.dresidual_rs, col, n);
   }
+  load_params<K, TEAM>(p.weight, p.weight_dtype, 0, col, n, w);
   for (int r = part; r < p.rows; r += nparts) {
     float x[K][8], g[K][8], dres[K][8];
     bx.get(x);

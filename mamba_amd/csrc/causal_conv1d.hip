@@ -80,6 +80,25 @@ template <int NCH> DEVI void load_taps(const CausalConvParams &p, int c0, int n,
     typedef std::remove_const_t<std::remove_pointer_t<decltype(wt)>> W;
     W wr[NCH][MAXW], br[NCH];
     const int lead = MAXW - p.width;
+    if constexpr (NCH % 2 == 0) {
+      if (lead == 0 && n == NCH) {  // whole rows of four: 8 taps per load
+        Pack8<W> q[NCH / 2];
+#pragma unroll
+        for (int j = 0; j < NCH / 2; ++j) q[j].load_any(wt + (int64_t)(c0 + 2 * j) * MAXW);
+#pragma unroll
+        for (int e = 0; e < NCH; ++e) br[e] = bt ? bt[c0 + e] : W{};
+#pragma unroll
+        for (int j = 0; j < NCH / 2; ++j) {
+          float v[8];
+          q[j].unpack(v);
+#pragma unroll
+          for (int k = 0; k < 8; ++k) w[2 * j + (k >> 2)][k & 3] = v[k];
+        }
+#pragma unroll
+        for (int e = 0; e < NCH; ++e) bias[e] = bt ? ld1<W>(&br[e]) : 0.f;
+        return;
+      }
+    }
 #pragma unroll
     for (int e = 0; e < NCH; ++e) {
       const int64_t c = c0 + min(e, n - 1);
@@ -550,50 +569,52 @@ template <> DEVI u32x4 pack4<float>(const float (&v)[4]) {
 
 // The forward pass in the same form: 4 channels per thread, the next four positions requested before the current
 // four are worked on.
-// RUN: positions per thread, 32 where the grid fills the chip, 8 where it does not.
+// RUN: positions per thread, 32 where the grid fills the chip, 8 where it does not.  A short run is a chain of load
+// latencies and little else, so all of its rows are requested before the taps, and nothing waits before that (with
+// guarded single loads in front and the second four positions behind the first: 12.4 us for 2 x 1000 x 1792 in bf16).
 template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_fwd4_kernel(const CausalConvParams p) {
   typedef typename Raw4<T>::type raw_t;
-  constexpr int CPT = 4;
+  constexpr int CPT = 4, AHEAD = RUN == 8 ? 2 : 1;  // groups of four positions in flight
   const int L = p.seqlen, b = blockIdx.z;
   const int cg = threadIdx.x & 63, run = threadIdx.x >> 6;
   const int c0 = (blockIdx.x * 64 + cg) * CPT;
   if (c0 >= p.dim) return;
   const int lbeg = (blockIdx.y * NRUN + run) * RUN, lend = min(lbeg + RUN, L);
   if (lbeg >= L) return;
-  float w[CPT][MAXW], bias[CPT];
-  load_taps<CPT>(p, c0, CPT, w, bias);
   const T *xb = static_cast<const T *>(p.x) + b * p.x_bs + c0;
   T *ob = static_cast<T *>(p.out) + b * p.out_bs + c0;
   const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L : nullptr;
-  float xw[3][CPT];  // x at l - 3, l - 2, l - 1
-  int idw[3] = {-0x7fffffff, -0x7fffffff, -0x7fffffff};
+  raw_t xp[3], xn[AHEAD][4];
+  int idw[3], idn[AHEAD][4];
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
-    const int l = lbeg - 3 + j;
-#pragma unroll
-    for (int e = 0; e < CPT; ++e) xw[j][e] = 0.f;
-    if (l >= 0) {
-      unpack4<T>(*reinterpret_cast<const raw_t *>(xb + (int64_t)l * p.x_ls), xw[j]);
-      if (seq) idw[j] = seq[l];
-    }
+    const int l = max(lbeg - 3 + j, 0);
+    xp[j] = *reinterpret_cast<const raw_t *>(xb + (int64_t)l * p.x_ls);
+    idw[j] = seq ? seq[l] : 0;
   }
-  raw_t xn[4];
-  int idn[4];
-  auto fetch = [&](int l4) {
+  auto fetch = [&](int l4, raw_t(&x)[4], int(&id)[4]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int l = min(l4 + u, L - 1);
-      xn[u] = *reinterpret_cast<const raw_t *>(xb + (int64_t)l * p.x_ls);
-      idn[u] = seq ? seq[l] : 0;
+      x[u] = *reinterpret_cast<const raw_t *>(xb + (int64_t)l * p.x_ls);
+      id[u] = seq ? seq[l] : 0;
     }
   };
-  fetch(lbeg);
-  for (int l4 = lbeg; l4 < lend; l4 += 4) {
-    raw_t x4[4];
-    int id4[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) x4[u] = xn[u], id4[u] = idn[u];
-    fetch(l4 + 4);  // (past the run on the last turn: rows that exist, never used)
+  for (int q = 0; q < AHEAD; ++q) fetch(lbeg + 4 * q, xn[q], idn[q]);
+  float w[CPT][MAXW], bias[CPT];
+  load_taps<CPT>(p, c0, CPT, w, bias);
+  float xw[3][CPT];  // x at l - 3, l - 2, l - 1
+#pragma unroll
+  for (int j = 0; j < 3; ++j) {
+    unpack4<T>(xp[j], xw[j]);
+    if (lbeg - 3 + j < 0) {
+      idw[j] = -0x7fffffff;
+#pragma unroll
+      for (int e = 0; e < CPT; ++e) xw[j][e] = 0.f;
+    }
+  }
+  auto use = [&](int l4, const raw_t(&x4)[4], const int(&id4)[4]) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       const int l = l4 + u;
@@ -622,15 +643,29 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_fw
       idw[1] = idw[2];
       idw[2] = id4[u];
     }
+  };
+  if constexpr (RUN == 4 * AHEAD) {
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) use(lbeg + 4 * q, xn[q], idn[q]);
+  } else {
+    for (int l4 = lbeg; l4 < lend; l4 += 4) {
+      raw_t x4[4];
+      int id4[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x4[u] = xn[0][u], id4[u] = idn[0][u];
+      fetch(l4 + 4, xn[0], idn[0]);  // (past the run on the last turn: rows that exist, never used)
+      use(l4, x4, id4);
+    }
   }
 }
 
 // RUN: positions per thread.  A run costs a 6-position warm-up, the taps, and its share of the reduction of the
 // filter gradients: long runs (128) where the grid still fills the chip, else 32, and 8 where even those leave compute
 // units without work (the walk down a run is a serial chain: with few workgroups its length is the kernel's time).
+// A run of 8 has all of its rows in flight at once (18.2 us for 2 x 1000 x 1792 in bf16 with one group of four ahead).
 template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bwd4_kernel(const CausalConvParams p) {
   typedef typename Raw4<T>::type raw_t;
-  constexpr int CPT = 4;
+  constexpr int CPT = 4, AHEAD = RUN == 8 ? 3 : 1;  // 8 positions and 3 behind them are three groups of four
   __shared__ float red[NRUN - 1][64][CPT * (MAXW + 1)];
   const int L = p.seqlen, b = blockIdx.z;
   const int cg = threadIdx.x & 63, run = threadIdx.x >> 6;
@@ -645,48 +680,51 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bw
     for (int k = 0; k < MAXW; ++k) dw[e][k] = 0.f;
   }
   if (live && lbeg < L) {
-    float w[CPT][MAXW], bias[CPT];
-    load_taps<CPT>(p, c0, CPT, w, bias);
     const T *xb = static_cast<const T *>(p.x) + b * p.x_bs + c0;
     const T *gb = static_cast<const T *>(p.dout) + b * p.dout_bs + c0;
     T *dxb = static_cast<T *>(p.dx) + b * p.dx_bs + c0;
     const int32_t *seq = p.seq_idx ? p.seq_idx + (int64_t)b * L : nullptr;
     // Walk down from lend + 2: the first three steps only rebuild dpre at the positions after the run.
     const int ltop = min(lend + 2, L - 1);
+    // every load of the first AHEAD groups is issued before anything waits; masks come after the taps
+    raw_t xp[4], gn[AHEAD][4], xn[AHEAD][4];
+    int idp[7], idn[AHEAD][4];
+#pragma unroll
+    for (int j = 0; j < 7; ++j) idp[j] = seq ? seq[min(max(ltop - 3 + j, 0), L - 1)] : 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) xp[j] = *reinterpret_cast<const raw_t *>(xb + (int64_t)max(ltop - 3 + j, 0) * p.x_ls);
+    // the loads of four steps: dout at l4 .. l4 - 3, x and the ids at l4 - 4 .. l4 - 7 (position 0 stands in below it)
+    auto fetch = [&](int l4, raw_t(&g)[4], raw_t(&x)[4], int(&id)[4]) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int l = l4 - u;
+        g[u] = *reinterpret_cast<const raw_t *>(gb + (int64_t)max(l, 0) * p.dout_ls);
+        x[u] = *reinterpret_cast<const raw_t *>(xb + (int64_t)max(l - 4, 0) * p.x_ls);
+        id[u] = seq ? seq[max(l - 4, 0)] : 0;
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < AHEAD; ++q) fetch(ltop - 4 * q, gn[q], xn[q], idn[q]);
+    float w[CPT][MAXW], bias[CPT];
+    load_taps<CPT>(p, c0, CPT, w, bias);
     float xw[4][CPT];  // x at l - 3 .. l
     float dp[4][CPT];  // dpre at l .. l + 3
     int idx[7];        // sequence ids at l - 3 .. l + 3
 #pragma unroll
     for (int j = 0; j < 7; ++j) {
       const int l = ltop - 3 + j;
-      idx[j] = (seq && l >= 0 && l < L) ? seq[l] : -0x7fffffff;
+      idx[j] = l >= 0 && l < L ? idp[j] : -0x7fffffff;
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const int l = ltop - 3 + j;
+      unpack4<T>(xp[j], xw[j]);
 #pragma unroll
-      for (int e = 0; e < CPT; ++e) xw[j][e] = dp[j][e] = 0.f;
-      if (l >= 0) unpack4<T>(*reinterpret_cast<const raw_t *>(xb + (int64_t)l * p.x_ls), xw[j]);
-    }
-    // the loads of four steps (dout at l4 .. l4 - 3, x at l4 - 4 .. l4 - 7), one group ahead
-    raw_t gn[4], xn[4];
-    int idn[4];
-    auto fetch = [&](int l4) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int l = l4 - u;
-        gn[u] = *reinterpret_cast<const raw_t *>(gb + (int64_t)max(l, 0) * p.dout_ls);
-        xn[u] = *reinterpret_cast<const raw_t *>(xb + (int64_t)max(l - 4, 0) * p.x_ls);
-        idn[u] = (seq && l - 4 >= 0) ? seq[l - 4] : -0x7fffffff;
+      for (int e = 0; e < CPT; ++e) {
+        dp[j][e] = 0.f;
+        xw[j][e] = ltop - 3 + j >= 0 ? xw[j][e] : 0.f;
       }
-    };
-    fetch(ltop);
-    for (int l4 = ltop; l4 >= lbeg; l4 -= 4) {
-      raw_t g4[4], x4[4];
-      int id4[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) g4[u] = gn[u], x4[u] = xn[u], id4[u] = idn[u];
-      fetch(l4 - 4);  // (below the run on the last turn: rows that exist, never used)
+    }
+    auto use = [&](int l4, const raw_t(&g4)[4], const raw_t(&x4)[4], const int(&id4)[4]) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int l = l4 - u;
@@ -747,7 +785,20 @@ template <typename T, int RUN> __global__ __launch_bounds__(256) void conv_cl_bw
         }
 #pragma unroll
         for (int j = 6; j > 0; --j) idx[j] = idx[j - 1];
-        idx[0] = id4[u];
+        idx[0] = has ? id4[u] : -0x7fffffff;
+      }
+    };
+    if constexpr (RUN == 8) {
+#pragma unroll
+      for (int q = 0; q < AHEAD; ++q) use(ltop - 4 * q, gn[q], xn[q], idn[q]);
+    } else {
+      for (int l4 = ltop; l4 >= lbeg; l4 -= 4) {
+        raw_t g4[4], x4[4];
+        int id4[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) g4[u] = gn[0][u], x4[u] = xn[0][u], id4[u] = idn[0][u];
+        fetch(l4 - 4, gn[0], xn[0], idn[0]);  // (below the run on the last turn: rows that exist, never used)
+        use(l4, g4, x4, id4);
       }
     }
   }

@@ -18,9 +18,14 @@
 
 namespace {
 
-// The heads of a group are spread over this many workgroups (each sums ~8 heads in registers and
-// adds its partial result atomically).
-__host__ __device__ inline int head_splits(int heads_per_group) { return (heads_per_group + 7) / 8; }
+// The heads of a group are spread over this many workgroups of the tiled state-path kernels (each sums ~8 heads in
+// registers and adds its partial result atomically): lists of 8, and shorter ones while there are fewer than two
+// workgroups per CU (16 heads on one chunk of 256, fp16: 8 workgroups of 8 heads took 33 + 23 us for dC and dB).
+inline int head_splits(const SsdParams *p, int64_t tiles_per_group) {
+  const int hpg = p->nheads / p->ngroups;
+  const int64_t rows = tiles_per_group * p->nchunks * p->batch * p->ngroups;
+  return std::max<int>((hpg + 7) / 8, (int)std::min<int64_t>(hpg, 2 * (int64_t)cu_count() / rows));
+}
 // The dCB kernel's lists are twice as long (~16 heads), and shorter where the tiles alone leave compute units without
 // work (a workgroup's head takes ~2 us, one after the other: 24 heads on 2 x 4 chunks took 34 us in lists of 12, 10 in
 // lists of 2): as many lists as give every CU four workgroups, two heads at least, where there would be fewer than two.
@@ -742,7 +747,7 @@ template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256) vo
 // both sums in registers (no atomics); the per-head row factor is folded into the A operand.
 // The carried-state share of ddA_cumsum, sum_n dC_h[l, n] C[l, n], is taken per head on the way.
 // PARTS: bit 0 = the dB product, bit 1 = the dC product.
-template <typename T, bool SPLIT, bool DET, int PARTS> DEVI void dBC_state_body(const SsdParams &p) {
+template <typename T, bool SPLIT, bool DET, int PARTS> DEVI void dBC_state_body(const SsdParams &p, const int nsplit) {
   constexpr int MAXH = 8;  // heads per workgroup (head_splits keeps it at or below 8)
   __shared__ GemmLds lds;
   __shared__ float wB[MAXH][GB], wC[MAXH][GB];  // per-head row factors
@@ -756,7 +761,7 @@ template <typename T, bool SPLIT, bool DET, int PARTS> DEVI void dBC_state_body(
   const Block3 blk = xcd_block();
   const int nst = gridDim.x / ntn;
   const int st = blk.x % nst, nt = blk.x / nst;  // the s tiles of a chunk share the state tiles
-  const int hpg = H / G, nsplit = head_splits(hpg);
+  const int hpg = H / G;
   const int c = blk.y, bg = blk.z / nsplit, hs = blk.z % nsplit, b = bg / G, g = bg % G;
   const int nh = hs < hpg ? (hpg - hs + nsplit - 1) / nsplit : 0;  // heads hs, hs + nsplit, ...
   const int t0 = c * Q, qlim = min(Q, L - t0);
@@ -882,16 +887,16 @@ template <typename T, bool SPLIT, bool DET, int PARTS> DEVI void dBC_state_body(
   }
 }
 
-template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4) void bwd_dBC_state_kernel(const SsdParams p) {
-  dBC_state_body<T, SPLIT, DET, 3>(p);
+template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4) void bwd_dBC_state_kernel(const SsdParams p, int nsplit) {
+  dBC_state_body<T, SPLIT, DET, 3>(p, nsplit);
 }
-template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4) void bwd_dC_state_kernel(const SsdParams p) {
-  dBC_state_body<T, SPLIT, DET, 2>(p);
+template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4) void bwd_dC_state_kernel(const SsdParams p, int nsplit) {
+  dBC_state_body<T, SPLIT, DET, 2>(p, nsplit);
 }
 
 // The dB product alone with a 64 x 128 tile per workgroup (whole 128-state blocks, headdim in whole
 // k steps, aligned x): k runs through (head, p) as above.
-template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256) void bwd_dB_state_wide_kernel(const SsdParams p) {
+template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256) void bwd_dB_state_wide_kernel(const SsdParams p, int nsplit) {
   constexpr int MAXH = 8;
   __shared__ GemmLdsWide<SPLIT> lds;
   __shared__ float wB[MAXH][GB];
@@ -901,7 +906,7 @@ template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256) vo
   const Block3 blk = xcd_block();
   const int nst = gridDim.x / ntn;
   const int st = blk.x % nst, nt = blk.x / nst;
-  const int hpg = H / G, nsplit = head_splits(hpg);
+  const int hpg = H / G;
   const int c = blk.y, bg = blk.z / nsplit, hs = blk.z % nsplit, b = bg / G, g = bg % G;
   const int nh = hs < hpg ? (hpg - hs + nsplit - 1) / nsplit : 0;
   const int t0 = c * Q, qlim = min(Q, L - t0);
@@ -951,7 +956,7 @@ template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256) vo
 
 // The dC product alone with a 64 x 128 tile per workgroup (same conditions, aligned g rows); the row sums
 // of the tile against C after each head give the heads' ddA_cumsum rows.
-template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4) void bwd_dC_state_wide_kernel(const SsdParams p) {
+template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4) void bwd_dC_state_wide_kernel(const SsdParams p, int nsplit) {
   constexpr int MAXH = 8;
   __shared__ GemmLdsWide<SPLIT> lds;
   __shared__ float wC[MAXH][GB];
@@ -963,7 +968,7 @@ template <typename T, bool SPLIT, bool DET> __global__ __launch_bounds__(256, 4)
   const Block3 blk = xcd_block();
   const int nst = gridDim.x / ntn;
   const int st = blk.x % nst, nt = blk.x / nst;
-  const int hpg = H / G, nsplit = head_splits(hpg);
+  const int hpg = H / G;
   const int c = blk.y, bg = blk.z / nsplit, hs = blk.z % nsplit, b = bg / G, g = bg % G;
   const int nh = hs < hpg ? (hpg - hs + nsplit - 1) / nsplit : 0;
   const int t0 = c * Q, qlim = min(Q, L - t0);
@@ -1678,18 +1683,18 @@ int launched() { return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAU
   }
 
 // the same for kernels compiled per summation mode (float atomics / fixed-point integer atomics)
-#define SSD_DISPATCH_DET(KERNEL, GRID)                                                                          \
+#define SSD_DISPATCH_DET(KERNEL, GRID, ...)                                                                        \
   if (p->det_scale) {                                                                                           \
     switch (p->dtype) {                                                                                         \
-      case MAMBA_BF16: hipLaunchKernelGGL((KERNEL<bf16_t, false, true>), GRID, dim3(256), 0, s, *p); break;     \
-      case MAMBA_F16: hipLaunchKernelGGL((KERNEL<f16_t, true, true>), GRID, dim3(256), 0, s, *p); break;        \
-      default: hipLaunchKernelGGL((KERNEL<float, true, true>), GRID, dim3(256), 0, s, *p); break;               \
+      case MAMBA_BF16: hipLaunchKernelGGL((KERNEL<bf16_t, false, true>), GRID, dim3(256), 0, s, *p __VA_OPT__(, ) __VA_ARGS__); break;     \
+      case MAMBA_F16: hipLaunchKernelGGL((KERNEL<f16_t, true, true>), GRID, dim3(256), 0, s, *p __VA_OPT__(, ) __VA_ARGS__); break;        \
+      default: hipLaunchKernelGGL((KERNEL<float, true, true>), GRID, dim3(256), 0, s, *p __VA_OPT__(, ) __VA_ARGS__); break;               \
     }                                                                                                           \
   } else {                                                                                                      \
     switch (p->dtype) {                                                                                         \
-      case MAMBA_BF16: hipLaunchKernelGGL((KERNEL<bf16_t, false, false>), GRID, dim3(256), 0, s, *p); break;    \
-      case MAMBA_F16: hipLaunchKernelGGL((KERNEL<f16_t, true, false>), GRID, dim3(256), 0, s, *p); break;       \
-      default: hipLaunchKernelGGL((KERNEL<float, true, false>), GRID, dim3(256), 0, s, *p); break;              \
+      case MAMBA_BF16: hipLaunchKernelGGL((KERNEL<bf16_t, false, false>), GRID, dim3(256), 0, s, *p __VA_OPT__(, ) __VA_ARGS__); break;    \
+      case MAMBA_F16: hipLaunchKernelGGL((KERNEL<f16_t, true, false>), GRID, dim3(256), 0, s, *p __VA_OPT__(, ) __VA_ARGS__); break;       \
+      default: hipLaunchKernelGGL((KERNEL<float, true, false>), GRID, dim3(256), 0, s, *p __VA_OPT__(, ) __VA_ARGS__); break;              \
     }                                                                                                           \
   }
 
@@ -1792,24 +1797,25 @@ static int ssd_bwd_dBC_state_one(const SsdParams *p, mamba_stream_t stream) {
   // bf16 on the common shapes: the kernels that keep a head's operands in LDS; else the tiled ones
   rc = ssd_bwd_dbc_fused_launch(p, s);
   if (rc != MAMBA_E_UNSUPPORTED) return rc;
-  const int zdim = p->batch * p->ngroups * head_splits(p->nheads / p->ngroups);
-  dim3 grid(tiles(p->chunk_size) * tiles(p->dstate), p->nchunks, zdim);
+  const int rows = p->batch * p->ngroups;
   // whole 128-state blocks, headdim in whole k steps, aligned x rows: the dB product runs on wide tiles
   const bool wide = p->dstate % WB == 0 && p->headdim % GK == 0 &&
                     wide_operand_ok(p->x, p->dtype, p->x_bs, p->x_ls, p->x_hs);
+  const int per_wide = tiles(p->chunk_size) * (p->dstate / WB), per_tile = tiles(p->chunk_size) * tiles(p->dstate);
+  const int n_wide = wide ? head_splits(p, per_wide) : 1, n_tile = head_splits(p, per_tile);
+  const dim3 grid(per_tile, p->nchunks, rows * n_tile), gridw(per_wide, p->nchunks, rows * n_wide);
   if (wide) {
-    dim3 gridw(tiles(p->chunk_size) * (p->dstate / WB), p->nchunks, zdim);
     const bool g_ok = p->z ? (p->headdim % 8 == 0 && reinterpret_cast<uintptr_t>(p->gbuf) % 16 == 0)
                            : wide_operand_ok(p->dout, p->dtype, p->dout_bs, p->dout_ls, p->dout_hs);
     if (g_ok) {
-      SSD_DISPATCH_DET(bwd_dC_state_wide_kernel, gridw)
+      SSD_DISPATCH_DET(bwd_dC_state_wide_kernel, gridw, n_wide)
     } else {
-      SSD_DISPATCH_DET(bwd_dC_state_kernel, grid)
+      SSD_DISPATCH_DET(bwd_dC_state_kernel, grid, n_tile)
     }
-    SSD_DISPATCH_DET(bwd_dB_state_wide_kernel, gridw)
+    SSD_DISPATCH_DET(bwd_dB_state_wide_kernel, gridw, n_wide)
     return launched();
   }
-  SSD_DISPATCH_DET(bwd_dBC_state_kernel, grid)
+  SSD_DISPATCH_DET(bwd_dBC_state_kernel, grid, n_tile)
   return launched();
 }
 

@@ -125,7 +125,7 @@ def selective_scan_fwd(u, delta, A, B, C, D=None, z=None, delta_bias=None, delta
     """
     ext = _lib.torch_ext()
     if ext is not None and not A.is_complex():
-        # the same checks, allocations and launch in C++ (csrc/torch_ext.cpp); None = a case for the code below
+        # the same checks, allocations and launch in C++ (csrc/torch_scan.cpp); None = a case for the code below
         r = ext.scan_fwd(u, delta, A, B, C, D, z, delta_bias, bool(delta_softplus))
         if r is not None:
             return r

@@ -131,7 +131,7 @@ def _mamba_chunk_scan_combined_fwd(x, dt, A, B, C, chunk_size, D=None, z=None, d
     (ssd_combined.py:390-394), in state_dtype, else C's dtype, as the reference returns it."""
     ext = _lib.torch_ext()
     if ext is not None and cu_seqlens is None:
-        # the same checks, allocations and launch in C++ (csrc/torch_ext.cpp); None = a case for the code below
+        # the same checks, allocations and launch in C++ (csrc/torch_ssd.cpp); None = a case for the code below
         r = ext.ssd_fwd(x, dt, A, B, C, int(chunk_size), D, z, dt_bias, initial_states, seq_idx, bool(dt_softplus),
                         float(dt_limit[0]), float(dt_limit[1]), bool(want_out_x))
         if r is not None:

@@ -884,14 +884,15 @@ inline bool aligned(const void *ptr, int a) { return (reinterpret_cast<uintptr_t
 // head's exposed memory latency: measured at about 0.15 of a head's work) plus its heads; the divisor with the
 // shortest estimate wins.
 inline int heads_per_workgroup(const SsdParams &p) {
-  const int hpg = p.nheads / p.ngroups, cus = cu_count();
+  // (with 64 states and chunks of up to 128 two workgroups share a CU; with 128 states the registers allow one)
+  const int hpg = p.nheads / p.ngroups, slots = cu_count() * (p.chunk_size <= 128 && p.dstate <= 64 ? 2 : 1);
   const int64_t tiles = (int64_t)p.nchunks * p.batch;
   int best = 1;
   double best_cost = 1e30;
   for (int hb = 1; hb <= 20 && hb <= hpg; ++hb) {
     if (hpg % hb) continue;
     const int64_t wgs = tiles * (p.nheads / hb);
-    const double cost = (double)((wgs + cus - 1) / cus) * (0.15 + hb);
+    const double cost = (double)((wgs + slots - 1) / slots) * (0.15 + hb);
     if (cost < best_cost - 1e-9) best = hb, best_cost = cost;
   }
   return best;

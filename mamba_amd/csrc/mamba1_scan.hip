@@ -39,8 +39,8 @@ namespace {
 // segment's part of the recurrence is a (decay, value) pair per (channel, state), as a lane's and a tile's are: the
 // value is formed by scan_seg_fwd_kernel, the decay is exp(A * sum of the segment's steps), and the scan kernels compose
 // the pairs of the segments before theirs when they start.  The adjoint is handled the same way from the other end
-// (scan_seg_bwd_kernel).  seg_ws: values (batch, nseg, dim, N), then the sums of the steps (batch, nseg, dim), then the
-// first steps (batch, nseg, dim; backward only).
+// (scan_seg_bwd_kernel).  seg_ws: values (batch, nseg, dim, N), then the sums of the steps (batch, nseg, dim; backward:
+// without the first one), then the first steps (batch, nseg, dim; backward only).
 DEVI int64_t seg_row(const MambaScanParams &p, int b, int seg, int d) { return ((int64_t)b * p.nseg + seg) * p.dim + d; }
 DEVI float *seg_sums(const MambaScanParams &p) { return p.seg_ws + (int64_t)p.batch * p.nseg * p.dim * p.dstate; }
 DEVI float *seg_firsts(const MambaScanParams &p) { return seg_sums(p) + (int64_t)p.batch * p.nseg * p.dim; }
@@ -60,10 +60,9 @@ DEVI float seg_adjoint_in(const MambaScanParams &p, const Geo &q, int d, int n, 
   decay = 0.f;
   for (int s = q.nseg - 1; s > q.seg; --s) {
     const int64_t row = seg_row(p, q.b, s, d);
-    const float first = seg_firsts(p)[row];
     // from the first position of segment s + 1 back to that of segment s; `decay` is the former's
-    g = __builtin_fmaf(fast_exp2(A2 * (seg_sums(p)[row] - first)) * decay, g, p.seg_ws[row * p.dstate + n]);
-    decay = fast_exp2(A2 * first);
+    g = __builtin_fmaf(fast_exp2(A2 * seg_sums(p)[row]) * decay, g, p.seg_ws[row * p.dstate + n]);
+    decay = fast_exp2(A2 * seg_firsts(p)[row]);
   }
   return g;
 }
@@ -72,7 +71,9 @@ DEVI float seg_adjoint_in(const MambaScanParams &p, const Geo &q, int d, int n, 
 // exp(A (steps after t)) B_t step_t u_t.  Backward: the adjoint at the segment's first position from a zero adjoint
 // behind it, sum over t of exp(A (steps after the first position up to t)) C_t dy_t.  Either way a lane runs its 8
 // steps from zero and weights the result with one exponential of the steps between it and the segment's end (start):
-// no scan across lanes and no carry, only one sum over the 16 lanes of a row at the end.  Where it runs the chip is
+// no scan across lanes and no carry, only one sum over the 16 lanes of a row at the end.  The steps between are summed as
+// such, never as a difference of longer sums: every exponent then has the sign of A, so that no factor can overflow where
+// the recurrence itself does not, and a large step elsewhere in the tile costs them no bits.  Where it runs the chip is
 // short of waves and a segment short of tiles, so latency bounds it: no LDS and no barrier (a lane reads its 8 items of
 // the B or C rows itself, the same 256 bytes for the four rows of every wave, from the caches), a group of states'
 // items requested ahead, workgroups of four independent waves.
@@ -100,6 +101,36 @@ __global__ __launch_bounds__(SEG_THREADS, BWD || sizeof(T) == 4 ? 3 : 4) void sc
   const T *Sg = BWD ? (const T *)p.C + b * p.C_bs + g * p.C_gs : (const T *)p.B + b * p.B_bs + g * p.B_gs;
   const int64_t S_ns = BWD ? p.C_ns : p.B_ns;
   auto tile_of = [&](int k) { return BWD ? tile0 + k : tile1 - 1 - k; };
+  if (BWD && MODE == ROWS_ANY && L - tile0 * TILE < KI) {
+    // A last segment of fewer positions than a lane has items: 8 items from L - 8 on would reach into the segment before,
+    // whose values must not count even as zero times an infinity.  A lane takes a state, position by position.
+    const int t0 = tile0 * TILE;
+    auto step = [&](int t) {
+      const float v = ld1<T>(drow + t) + bias;
+      return p.delta_softplus ? softplus_f(v) : v;
+    };
+    float run = 0.f;
+    for (int t = t0 + 1; t < L; ++t) run += step(t);
+    for (int n = c; n < N; n += RL) {
+      const float A2 = ((const float *)p.A)[(int64_t)d * N + n] * kLog2e;
+      float acc = 0.f;
+      for (int t = L - 1; t >= t0; --t) {
+        float x = ld1<T>(urow + t);
+        if (gated) {
+          const float z = ld1<T>(zrow + t);
+          x *= z * sigmoid_f(z);
+        }
+        const float v = CONST_BC ? ((const float *)p.C)[(int64_t)d * N + n] : ld1<T>(Sg + n * S_ns + t);
+        acc = t + 1 < L ? __builtin_fmaf(fast_exp2(step(t + 1) * A2), acc, x * v) : x * v;
+      }
+      if (valid) p.seg_ws[row * N + n] = acc;
+    }
+    if (c == 0 && valid) {
+      seg_sums(p)[row] = run;
+      seg_firsts(p)[row] = step(t0);
+    }
+    return;
+  }
   for (int n0 = 0; n0 < N; n0 += NB16) {
     float acc[NB16], A2[NB16];
 #pragma unroll
@@ -120,14 +151,14 @@ __global__ __launch_bounds__(SEG_THREADS, BWD || sizeof(T) == 4 ? 3 : 4) void sc
       for (int s = 0; s < NG; ++s)
         load_items<T, MODE>(dst[s], Sg + (int64_t)min(n0 + n + s, N - 1) * S_ns, tile_of(k) * TILE + c * KI, L, KI);
     };
-    float run = 0.f, first = 0.f;  // steps of the tiles already taken; the segment's first step
+    float run = 0.f, first = 0.f;  // steps of the tiles already taken; backward: without the segment's first step, `first`
     fetch_rows(0);
     fetch_states(ks[0], 0, 0);
     for (int k = 0; k < ntiles; ++k) {
       // A lane in a ragged row's last piece reads 8 items from L - 8 on like the other rows' lanes, and leaves out the
-      // ones before its own (nothing has to be moved into place: the order is what counts).
+      // ones before its own, which are the lane before's (nothing has to be moved into place: the order is what counts).
       const int tl = tile_of(k) * TILE + c * KI, shift = tl - min(tl, L - KI);
-      float x[8], dl[8], z[8], dsum = 0.f;
+      float x[8], dl[8], z[8], dsum = 0.f, own = 0.f;  // own: the first step of the lane's own (backward)
       ku.unpack(x);
       kd.unpack(dl);
       if (BWD) kz.unpack(z);
@@ -141,25 +172,30 @@ __global__ __launch_bounds__(SEG_THREADS, BWD || sizeof(T) == 4 ? 3 : 4) void sc
       for (int i = 0; i < KI; ++i) {
         float v = dl[i] + bias;
         if (p.delta_softplus) v = softplus_f(v);
-        dl[i] = i >= shift ? v : 0.f;
         x[i] = i >= shift ? x[i] : 0.f;
-        if (!BWD) x[i] *= dl[i];
+        if constexpr (BWD) {  // the decays behind the lane's first position
+          own = i == shift ? v : own;
+          dl[i] = i > shift ? v : 0.f;
+        } else {
+          dl[i] = i >= shift ? v : 0.f;
+          x[i] *= dl[i];
+        }
         dsum += dl[i];
       }
-      float incl = dsum;  // steps of the row's lanes up to and with this one
-      incl += dpp_f<DPP_ROW_SHR + 1>(0.f, incl);
-      incl += dpp_f<DPP_ROW_SHR + 2>(0.f, incl);
-      incl += dpp_f<DPP_ROW_SHR + 4>(0.f, incl);
-      incl += dpp_f<DPP_ROW_SHR + 8>(0.f, incl);
-      const float total = __shfl(incl, lane | (RL - 1), 64);
       if (BWD && k == 0) {
-        float own = dl[0];
-#pragma unroll
-        for (int i = 1; i < KI; ++i) own = i == shift ? dl[i] : own;
         first = __shfl(own, lane & ~(RL - 1), 64);
+        own = c == 0 ? 0.f : own;
       }
-      const float away = BWD ? run + (incl - dsum) + dl[0] - first : run + (total - incl);
-      run += total;
+      dsum += own;
+      // Steps of the row's lanes from this one on (backward: up to this one), and of those behind (before) it.
+      constexpr int STEP = BWD ? DPP_ROW_SHR : DPP_ROW_SHL;
+      float incl = dsum;
+      incl += dpp_f<STEP + 1>(0.f, incl);
+      incl += dpp_f<STEP + 2>(0.f, incl);
+      incl += dpp_f<STEP + 4>(0.f, incl);
+      incl += dpp_f<STEP + 8>(0.f, incl);
+      const float away = run + dpp_f<STEP + 1>(0.f, incl) + own;
+      run += __shfl(incl, BWD ? lane | (RL - 1) : lane & ~(RL - 1), 64);
 #pragma unroll
       for (int n = 0; n < NB16; n += NG) {
         const int cur = (n / NG) & 1;

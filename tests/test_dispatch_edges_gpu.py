@@ -26,6 +26,62 @@ def test_scan_segments(batch, dim, dstate, seqlen, groups, var, itype):
     mamba1._run_case(batch, dim, dstate, seqlen, itype, groups, var_B=var, var_C=var)
 
 
+# The same with steps up to which nothing of the segment before is left (exp(-16 * 20) is zero), in every channel or in
+# one position out of 16 among steps of 1e-3; the last segment is a tile of 1 and of 3 positions.  Tolerance: |A| step is
+# at most 20 wherever a product still counts (exp(-20) = 2e-9), which an fp32 exponent holds to 20 * 2^-23, and a sum over
+# a tile and 16 states adds about as much again: 5e-6 of each channel's norm.  dA and ddelta have a term
+# adjoint * decay * state, formed as adjoint * (state - input): one rounding of adjoint * input, the larger the smaller the
+# decay, is allowed beside that.
+@pytest.mark.parametrize("seqlen", [129, 515, 771])
+@pytest.mark.parametrize("step,rare", [(6.0, False), (20.0, False), (20.0, True)])
+def test_scan_segments_large_steps(seqlen, step, rare):
+    from mamba_amd.ops.selective_scan_interface import selective_scan_fn
+    from oracle.mamba1 import selective_scan_oracle
+    g = torch.Generator().manual_seed(seqlen)
+    dim, n = 32, 16
+    rn = lambda *s: torch.randn(*s, generator=g)
+    delta = step * (0.8 + 0.2 * torch.rand(1, dim, seqlen, generator=g))
+    if rare:
+        delta = torch.where(torch.rand(1, dim, seqlen, generator=g) < 1 / 16, delta, 1e-3 * torch.rand(1, dim, seqlen, generator=g))
+    delta[:, ::4] *= 1e-3  # channels in which the state does reach across the segments
+    leaves = [rn(1, dim, seqlen), delta, -torch.arange(1, n + 1).float().repeat(dim, 1), rn(1, 1, n, seqlen), rn(1, 1, n, seqlen), rn(dim),
+              rn(1, dim, seqlen)]
+    dout = rn(1, dim, seqlen)
+    ref = [t.double().requires_grad_() for t in leaves]
+    want = selective_scan_oracle(*ref, compute_dtype=torch.float64)
+    want = (want, *torch.autograd.grad(want, ref, dout.double()))
+    got = [t.cuda().requires_grad_() for t in leaves]
+    out = selective_scan_fn(*got)
+    got = (out, *torch.autograd.grad(out, got, dout.cuda()))
+    u, step, A, B, C, _, z = [t.detach()[0] if t.dim() > 2 else t.detach() for t in ref]  # (dim, L), A (dim, n), B and C (1, n, L)
+    dy = dout[0].double() * torch.nn.functional.silu(z)
+    term = (step * u * dy)[:, None] * B * C  # adjoint * input, (dim, n, L)
+    rounding = dict(dA=(term * step[:, None]).norm(dim=2).norm(dim=1), ddelta=(term * A[..., None]).abs().sum(1).norm(dim=1))
+    for name, a, b in zip(("out", "du", "ddelta", "dA", "dB", "dC", "dD", "dz"), got, want):
+        a, b = a.detach().double().cpu(), b.detach()
+        assert bool(torch.isfinite(a).all()), name
+        if b.dim() > 1:
+            a, b = a.flatten(0, -2), b.flatten(0, -2)  # per channel or state
+        err, bound = (a - b).norm(dim=-1), 5e-6 * b.norm(dim=-1) + 2.0 ** -23 * rounding.get(name, 0.0)
+        assert bool((err <= bound).all()), (name, float((err / bound).max()))
+
+
+def test_scan_segments_nan_stays_in_its_segment():
+    """A NaN in C reaches the gradients of its own position and the ones before it, not those between it and the last
+    segment, whose first piece is read from 8 positions before the end of the row."""
+    from mamba_amd.ops.selective_scan_interface import selective_scan_fn
+    g = torch.Generator().manual_seed(0)
+    dim, n, L, at = 32, 16, 771, 765
+    rn = lambda *s: torch.randn(*s, generator=g).cuda()
+    u, z, dout = rn(1, dim, L).requires_grad_(), rn(1, dim, L), rn(1, dim, L)
+    A, B, C = -torch.arange(1, n + 1).float().repeat(dim, 1).cuda(), rn(1, 1, n, L), rn(1, 1, n, L)
+    C[..., at] = float("nan")
+    out = selective_scan_fn(u, torch.full_like(u, 0.01), A, B, C, z=z)
+    du, = torch.autograd.grad(out, u, dout)
+    nan = torch.isnan(du)[0].any(0)
+    assert bool(nan[:at + 1].all()) and not bool(nan[at + 1:].any())
+
+
 # channels next to each other, runs of 8 positions: below one run, its edges, one past; rows along the positions of a
 # length that is no multiple of 8
 @pytest.mark.parametrize("channel_last", [True, False])

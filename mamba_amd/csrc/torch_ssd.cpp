@@ -526,7 +526,7 @@ pybind11::object split_conv_scan(const at::Tensor &zxbcdt_in, const at::Tensor &
   if (out_weight) {
     const at::ScalarType want = autocast ? *autocast : zxbcdt.scalar_type();
     auto ok = [&](const at::Tensor &t) { return on_device(t, dev) && (t.scalar_type() == want || (autocast && t.is_floating_point())); };
-    if (out_weight->dim() != 2 || out_weight->size(1) != dim || !ok(*out_weight)) return no;
+    if (out_weight->dim() != 2 || out_weight->size(0) == 0 || out_weight->size(1) != dim || !ok(*out_weight)) return no;
     // (a bias that F.linear broadcasts or refuses is left to it)
     if (out_bias && (!ok(*out_bias) || out_bias->dim() != 1 || out_bias->size(0) != out_weight->size(0))) return no;
   } else if (out_bias) {

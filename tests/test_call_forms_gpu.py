@@ -1,4 +1,4 @@
-"""The operators' calls beside their plain use: a projection's bias that does not fit."""
+"""The operators' calls beside their plain use: a projection's bias that does not fit, a projection of no rows."""
 import pytest
 import torch
 
@@ -36,3 +36,14 @@ def test_block_bias_is_broadcast(shape):
     plain = mamba_split_conv1d_scan_combined(*args, **kw)
     out = mamba_split_conv1d_scan_combined(*args, outproj_bias=torch.full(shape, 0.5, device="cuda"), **kw)
     assert float((out - plain - 0.5).abs().max()) <= 1e-5 * float(plain.abs().max())
+
+
+def test_block_projection_without_rows():
+    from mamba_amd.ops.triton.ssd_combined import mamba_split_conv1d_scan_combined
+    x, z = _operands()
+    args, kw = _block_args(x, z)
+    kw["outproj_weight"] = kw["outproj_weight"][:0]
+    assert mamba_split_conv1d_scan_combined(*args, **kw).shape == (2, 96, 0)
+    args = [t.bfloat16() for t in args[:3]] + list(args[3:])
+    kw["outproj_weight"] = kw["outproj_weight"].bfloat16()
+    assert mamba_split_conv1d_scan_combined(*args, **kw).shape == (2, 96, 0)

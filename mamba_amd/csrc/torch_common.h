@@ -45,16 +45,20 @@ inline void check_rc(int rc, const char *what) {
 
 inline void *ptr(const OptTensor &t) { return t ? t->data_ptr() : nullptr; }
 
+template <typename F> bool holds(const F &f, const at::Tensor &t) { return t.defined() && f(t); }
+template <typename F> bool holds(const F &f, const OptTensor &t) { return t && holds(f, *t); }
+
 // Whether autograd has to record a call: gradients are enabled and one of the tensors wants them.
-inline bool any_grad() { return false; }
-template <typename... Rest> bool any_grad(const at::Tensor &t, const Rest &...rest);
-template <typename... Rest> bool any_grad(const OptTensor &t, const Rest &...rest) {
-  return (t && t->defined() && t->requires_grad()) || any_grad(rest...);
+template <typename... Args> bool records(const Args &...args) {
+  auto wants = [](const at::Tensor &t) { return t.requires_grad(); };
+  return at::GradMode::is_enabled() && (holds(wants, args) || ...);
 }
-template <typename... Rest> bool any_grad(const at::Tensor &t, const Rest &...rest) {
-  return (t.defined() && t.requires_grad()) || any_grad(rest...);
+// Whether a call is one for the Python autograd functions, which refuse it as torch does: under a functorch transform, or
+// with a forward-mode gradient on one of the tensors (with and without reverse-mode gradients; the kernels would drop it).
+template <typename... Args> bool python_call(const Args &...args) {
+  auto tangent = [](const at::Tensor &t) { return t._fw_grad(0).defined(); };
+  return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || (holds(tangent, args) || ...);
 }
-template <typename... Args> bool records(const Args &...args) { return at::GradMode::is_enabled() && any_grad(args...); }
 
 inline OptTensor opt(const at::Tensor &t) { return t.defined() ? OptTensor(t) : std::nullopt; }
 inline at::Tensor tensor_or_none(const OptTensor &t) { return t ? *t : at::Tensor(); }

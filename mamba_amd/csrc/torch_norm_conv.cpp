@@ -118,7 +118,7 @@ struct ResNormFn : torch::autograd::Function<ResNormFn> {
 pybind11::object norm_residual(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &residual,
                                double eps, bool prenorm, bool residual_in_fp32, bool is_rms) {
   const pybind11::object no = pybind11::none();
-  if (!x.is_cuda() || x.dim() < 1 || dtype_code(x) < 0 || x.size(-1) <= 0) return no;
+  if (!x.is_cuda() || x.dim() < 1 || dtype_code(x) < 0 || x.size(-1) <= 0 || python_call(x, weight, bias, residual)) return no;
   const c10::Device dev = x.device();
   const int64_t N = x.size(-1);
   if (!params_ok(weight, bias, N, dev) || N > 65536 / (int64_t)x.element_size() || !on_device(residual, dev)) return no;
@@ -179,7 +179,8 @@ struct GatedNormFn : torch::autograd::Function<GatedNormFn> {
 // layernorm_gated.layernorm_fn / rmsnorm_fn; None = declined
 OptTensor norm_gated(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &z, double eps,
                      std::optional<int64_t> group_size, bool norm_before_gate, bool is_rms) {
-  if (!x.is_cuda() || x.dim() < 1 || x.size(-1) <= 0 || (z && z->sizes() != x.sizes())) return std::nullopt;
+  if (!x.is_cuda() || x.dim() < 1 || x.size(-1) <= 0 || (z && z->sizes() != x.sizes()) || python_call(x, weight, bias, z))
+    return std::nullopt;
   const GatedNorm o{group_size.value_or(x.size(-1)), eps, norm_before_gate, is_rms};
   if (!gated_norm_ok(x, weight, bias, z, o)) return std::nullopt;
   if (!records(x, weight, bias, z))
@@ -231,7 +232,7 @@ struct ConvFn : torch::autograd::Function<ConvFn> {
 
 // causal_conv1d_fn without the streaming arguments; None = declined
 OptTensor causal_conv1d(const at::Tensor &x, const at::Tensor &weight, const OptTensor &bias, const OptTensor &seq_idx, bool silu) {
-  if (!x.is_cuda() || x.dim() != 3 || (x.stride(2) != 1 && x.stride(1) != 1)) return std::nullopt;
+  if (!x.is_cuda() || x.dim() != 3 || (x.stride(2) != 1 && x.stride(1) != 1) || python_call(x, weight, bias)) return std::nullopt;
   if (!conv_params_ok(x, weight, bias, seq_idx)) return std::nullopt;
   if (records(x, weight, bias)) return ConvFn::apply(x, weight, bias, seq_idx, silu);
   at::Tensor out = like_layout(x);

@@ -239,7 +239,7 @@ pybind11::object selective_scan(const at::Tensor &u, const at::Tensor &delta, co
                                 bool delta_softplus, bool return_last_state) {
   const pybind11::object no = pybind11::none();
   if (!u.is_cuda() || u.dim() != 3 || delta.dim() != 3 || A.dim() != 2 || B.dim() < 2 || C.dim() < 2 || B.dim() > 4 || C.dim() > 4 ||
-      (z && z->dim() != 3) || A.is_complex())
+      (z && z->dim() != 3) || A.is_complex() || python_call(u, delta, A, B, C, D, z, delta_bias))
     return no;
   const ScanArgs a = normalised(u, delta, A, B, C, D, z, delta_bias);
   MambaScanParams p{};
@@ -406,7 +406,8 @@ struct InnerFn : torch::autograd::Function<InnerFn> {
 OptTensor mamba_inner(const at::Tensor &xz_in, const at::Tensor &conv_weight, const OptTensor &conv_bias, const at::Tensor &x_proj,
                       const at::Tensor &dt_proj, const at::Tensor &out_proj, const OptTensor &out_bias, const at::Tensor &A,
                       const OptTensor &D, const OptTensor &delta_bias, bool delta_softplus, int64_t checkpoint_lvl) {
-  if (!xz_in.is_cuda() || xz_in.dim() != 3 || xz_in.size(1) % 2 != 0 || conv_weight.dim() != 3 || conv_weight.size(1) != 1)
+  if (!xz_in.is_cuda() || xz_in.dim() != 3 || xz_in.size(1) % 2 != 0 || conv_weight.dim() != 3 || conv_weight.size(1) != 1 ||
+      python_call(xz_in, conv_weight, conv_bias, x_proj, dt_proj, out_proj, out_bias, A, D, delta_bias))
     return std::nullopt;
   const at::Tensor xz = unit_last(xz_in);
   const c10::Device dev = xz.device();

@@ -331,6 +331,7 @@ pybind11::object chunk_scan(const at::Tensor &x, const at::Tensor &dt, const at:
                             int64_t chunk_size, const OptTensor &D, const OptTensor &z, const OptTensor &dt_bias,
                             const OptTensor &initial_states, const OptTensor &seq_idx, bool dt_softplus, double dt_min,
                             double dt_max, bool return_final) {
+  if (python_call(x, dt, A, B, C, D, z, dt_bias, initial_states)) return pybind11::none();
   if (x.dim() == 4 && B.dim() == 4)
     chunk_size = kernel_chunk(chunk_size, x.size(0), x.size(1), x.size(2), B.size(2), x.size(3), B.size(3), x.scalar_type());
   SsdParams p{};
@@ -496,6 +497,7 @@ pybind11::object split_conv_scan(const at::Tensor &zxbcdt_in, const at::Tensor &
   if (!zxbcdt_in.is_cuda() || zxbcdt_in.dim() != 3 || G <= 0 || (D.dim() != 1 && D.dim() != 2) || conv_weight.dim() < 2 ||
       (conv_weight.dim() == 3 && conv_weight.size(1) != 1) || conv_weight.dim() > 3)
     return no;
+  if (python_call(zxbcdt_in, conv_weight, conv_bias, dt_bias, A, D, initial_states, norm_weight, out_weight, out_bias)) return no;
   if (D.dim() == 1 && !headdim_in) return no;
   // rows of (batch, seqlen) must follow one another: the norm walks them as one (rows, channels) matrix
   const bool rows = zxbcdt_in.stride(2) == 1 && (zxbcdt_in.size(0) == 1 || zxbcdt_in.stride(0) == zxbcdt_in.size(1) * zxbcdt_in.stride(1));

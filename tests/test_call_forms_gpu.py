@@ -1,6 +1,8 @@
-"""The operators' calls beside their plain use: a projection's bias that does not fit, a projection of no rows."""
+"""The operators' calls beside their plain use: forward-mode gradients, functorch's transforms, a projection's bias that
+does not fit, a projection of no rows."""
 import pytest
 import torch
+import torch.autograd.forward_ad as fwAD
 
 pytestmark = pytest.mark.gpu
 
@@ -10,6 +12,31 @@ def _operands(seed=1):
     return tuple(torch.randn(2, 64, 96, device="cuda", generator=g) for _ in range(2))
 
 
+def _scan(x, z):
+    """x, z: (2, 64, 96) on the GPU, as every call here takes them."""
+    from mamba_amd.ops.selective_scan_interface import selective_scan_fn
+    g = torch.Generator(device="cuda").manual_seed(0)
+    bc = torch.randn(2, 2, 1, 16, 96, device="cuda", generator=g)
+    return selective_scan_fn(x, torch.full_like(x, 0.1), -torch.ones(64, 16, device="cuda"), bc[0], bc[1], z=z)
+
+
+def _ssd(x, z):
+    from mamba_amd.ops.triton.ssd_combined import mamba_chunk_scan_combined
+    g = torch.Generator(device="cuda").manual_seed(0)
+    bc = torch.randn(2, 2, 64, 1, 64, device="cuda", generator=g)
+    heads = lambda t: t.reshape(2, 64, 3, 32)
+    return mamba_chunk_scan_combined(heads(x), torch.full((2, 64, 3), 0.1, device="cuda"), -torch.ones(3, device="cuda"), bc[0], bc[1], 64,
+                                     z=heads(z))
+
+
+def _inner(x, z):
+    from mamba_amd.ops.selective_scan_interface import mamba_inner_fn
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rn = lambda *s: 0.2 * torch.randn(*s, device="cuda", generator=g)
+    return mamba_inner_fn(torch.cat([x, z], 1), rn(64, 1, 4), rn(64), rn(4 + 32, 64), rn(64, 4), rn(32, 64), None, -torch.ones(64, 16, device="cuda"),
+                          D=rn(64), delta_bias=rn(64))
+
+
 def _block_args(x, z):
     g = torch.Generator(device="cuda").manual_seed(0)
     rn = lambda *s: 0.2 * torch.randn(*s, device="cuda", generator=g)
@@ -17,6 +44,51 @@ def _block_args(x, z):
     zxbcdt = torch.cat([z.transpose(1, 2), x.transpose(1, 2), rn(2, 96, 2 * N + H)], 2)
     return (zxbcdt, rn(H * P + 2 * N, 4), rn(H * P + 2 * N), rn(H), -torch.ones(H, device="cuda"), rn(H), 64), dict(
         rmsnorm_weight=rn(H * P), outproj_weight=rn(48, H * P), headdim=P)
+
+
+def _block(x, z):
+    from mamba_amd.ops.triton.ssd_combined import mamba_split_conv1d_scan_combined
+    args, kw = _block_args(x, z)
+    return mamba_split_conv1d_scan_combined(*args, **kw)
+
+
+def _conv(x, z):
+    from mamba_amd.ops.causal_conv1d import causal_conv1d_fn
+    return causal_conv1d_fn(x, torch.ones(64, 4, device="cuda"), activation="silu")
+
+
+def _norm(x, z):
+    from mamba_amd.ops.triton.layer_norm import rms_norm_fn
+    return rms_norm_fn(x, torch.ones(96, device="cuda"), None, residual=z)
+
+
+def _gated(x, z):
+    from mamba_amd.ops.triton.layernorm_gated import rmsnorm_fn
+    return rmsnorm_fn(x, torch.ones(96, device="cuda"), None, z=z)
+
+
+CALLS = {f.__name__[1:]: f for f in (_scan, _ssd, _inner, _block, _conv, _norm, _gated)}
+each_call = pytest.mark.parametrize("call", list(CALLS.values()), ids=list(CALLS))
+
+
+@each_call
+@pytest.mark.parametrize("grad", [True, False])
+def test_forward_mode_is_refused(call, grad):
+    """No operator has a forward-mode formula: a tangent is refused, never dropped."""
+    x, z = _operands()
+    with torch.set_grad_enabled(grad), fwAD.dual_level():
+        dual = fwAD.make_dual(x, torch.ones_like(x))
+        with pytest.raises(NotImplementedError):
+            call(dual, z)
+
+
+@each_call
+def test_functorch_transforms_are_refused(call):
+    x, z = _operands()
+    with pytest.raises(RuntimeError):
+        torch.func.jvp(lambda t: call(t, z), (x,), (torch.ones_like(x),))
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda t: call(x, z) + t)(torch.zeros(2, 1, device="cuda"))
 
 
 @pytest.mark.parametrize("shape", [(47,), (1, 47), (0,)])

@@ -53,11 +53,13 @@ template <typename... Args> bool records(const Args &...args) {
   auto wants = [](const at::Tensor &t) { return t.requires_grad(); };
   return at::GradMode::is_enabled() && (holds(wants, args) || ...);
 }
-// Whether a call is one for the Python autograd functions, which refuse it as torch does: under a functorch transform, or
-// with a forward-mode gradient on one of the tensors (with and without reverse-mode gradients; the kernels would drop it).
+// Whether a call is one for the Python autograd functions.  torch refuses them under a functorch transform, and with a
+// forward-mode gradient on one of the tensors (with and without reverse-mode gradients; the kernels would drop it).  A jit
+// trace records them as nodes to be run again; a call it does not see leaves its results in the trace as constants.
 template <typename... Args> bool python_call(const Args &...args) {
   auto tangent = [](const at::Tensor &t) { return t._fw_grad(0).defined(); };
-  return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) || (holds(tangent, args) || ...);
+  return c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
+         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) || (holds(tangent, args) || ...);
 }
 
 inline OptTensor opt(const at::Tensor &t) { return t.defined() ? OptTensor(t) : std::nullopt; }

@@ -1,5 +1,7 @@
-"""The operators' calls beside their plain use: forward-mode gradients, functorch's transforms, a projection's bias that
-does not fit, a projection of no rows."""
+"""The operators' calls beside their plain use: forward-mode gradients, functorch's transforms, a jit trace, a projection's
+bias that does not fit, a projection of no rows."""
+import functools
+
 import pytest
 import torch
 import torch.autograd.forward_ad as fwAD
@@ -12,18 +14,22 @@ def _operands(seed=1):
     return tuple(torch.randn(2, 64, 96, device="cuda", generator=g) for _ in range(2))
 
 
+@functools.lru_cache(maxsize=None)
+def _fixed(which, *shape):
+    """Parameters of a call: the same tensor for every call of a test (a draw inside a traced call would be traced)."""
+    return 0.2 * torch.randn(*shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(which))
+
+
 def _scan(x, z):
     """x, z: (2, 64, 96) on the GPU, as every call here takes them."""
     from mamba_amd.ops.selective_scan_interface import selective_scan_fn
-    g = torch.Generator(device="cuda").manual_seed(0)
-    bc = torch.randn(2, 2, 1, 16, 96, device="cuda", generator=g)
+    bc = _fixed(0, 2, 2, 1, 16, 96)
     return selective_scan_fn(x, torch.full_like(x, 0.1), -torch.ones(64, 16, device="cuda"), bc[0], bc[1], z=z)
 
 
 def _ssd(x, z):
     from mamba_amd.ops.triton.ssd_combined import mamba_chunk_scan_combined
-    g = torch.Generator(device="cuda").manual_seed(0)
-    bc = torch.randn(2, 2, 64, 1, 64, device="cuda", generator=g)
+    bc = _fixed(0, 2, 2, 64, 1, 64)
     heads = lambda t: t.reshape(2, 64, 3, 32)
     return mamba_chunk_scan_combined(heads(x), torch.full((2, 64, 3), 0.1, device="cuda"), -torch.ones(3, device="cuda"), bc[0], bc[1], 64,
                                      z=heads(z))
@@ -31,19 +37,15 @@ def _ssd(x, z):
 
 def _inner(x, z):
     from mamba_amd.ops.selective_scan_interface import mamba_inner_fn
-    g = torch.Generator(device="cuda").manual_seed(0)
-    rn = lambda *s: 0.2 * torch.randn(*s, device="cuda", generator=g)
-    return mamba_inner_fn(torch.cat([x, z], 1), rn(64, 1, 4), rn(64), rn(4 + 32, 64), rn(64, 4), rn(32, 64), None, -torch.ones(64, 16, device="cuda"),
-                          D=rn(64), delta_bias=rn(64))
+    return mamba_inner_fn(torch.cat([x, z], 1), _fixed(0, 64, 1, 4), _fixed(1, 64), _fixed(2, 4 + 32, 64), _fixed(3, 64, 4), _fixed(4, 32, 64), None,
+                          -torch.ones(64, 16, device="cuda"), D=_fixed(5, 64), delta_bias=_fixed(6, 64))
 
 
 def _block_args(x, z):
-    g = torch.Generator(device="cuda").manual_seed(0)
-    rn = lambda *s: 0.2 * torch.randn(*s, device="cuda", generator=g)
     H, P, N = 2, 32, 16
-    zxbcdt = torch.cat([z.transpose(1, 2), x.transpose(1, 2), rn(2, 96, 2 * N + H)], 2)
-    return (zxbcdt, rn(H * P + 2 * N, 4), rn(H * P + 2 * N), rn(H), -torch.ones(H, device="cuda"), rn(H), 64), dict(
-        rmsnorm_weight=rn(H * P), outproj_weight=rn(48, H * P), headdim=P)
+    zxbcdt = torch.cat([z.transpose(1, 2), x.transpose(1, 2), _fixed(0, 2, 96, 2 * N + H)], 2)
+    return (zxbcdt, _fixed(1, H * P + 2 * N, 4), _fixed(2, H * P + 2 * N), _fixed(3, H), -torch.ones(H, device="cuda"), _fixed(4, H), 64), dict(
+        rmsnorm_weight=_fixed(5, H * P), outproj_weight=_fixed(6, 48, H * P), headdim=P)
 
 
 def _block(x, z):
@@ -89,6 +91,19 @@ def test_functorch_transforms_are_refused(call):
         torch.func.jvp(lambda t: call(t, z), (x,), (torch.ones_like(x),))
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda t: call(x, z) + t)(torch.zeros(2, 1, device="cuda"))
+
+
+@each_call
+def test_traced_call_replays(call):
+    """A jit trace holds the call itself, not the values it gave while it was traced."""
+    x, z = _operands()
+    with torch.no_grad():
+        call(x, z)
+        traced = torch.jit.trace(call, (x, z), check_trace=False)
+        for seed in (1, 2, 3):
+            x, z = _operands(seed)
+            got, want = traced(x, z), call(x, z)  # (the block's projection: sums of 64 products in another order)
+            assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
 
 
 @pytest.mark.parametrize("shape", [(47,), (1, 47), (0,)])

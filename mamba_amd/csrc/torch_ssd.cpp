@@ -406,7 +406,7 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
       auto [yn, mean, rs] = gated_norm_fwd(y, *norm_weight, std::nullopt, row_slice(zxbcdt, 0, dim), {dim / G, o.eps, o.norm_before_gate, true});
       y = yn, rstd = rs;
     }
-    at::Tensor res = y, w;
+    at::Tensor res, w;
     if (out_weight) {
       w = *out_weight;
       OptTensor bias = out_bias;
@@ -416,7 +416,7 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
       }
       y = y.contiguous(), w = w.contiguous();
       if (bias) bias = bias->contiguous();
-      res = at::empty({batch * L, w.size(0)}, y.options());
+      res = at::empty({batch, L, w.size(0)}, y.options());  // as it is returned: a view made here could not be written in place
       Products(y.options(), y.scalar_type())
           .add(res.data_ptr(), y.scalar_type(), w.size(0), batch * L, w.size(0), dim, {y.data_ptr(), dim, 1}, {w.data_ptr(), dim, 1}, false,
                bias ? bias->data_ptr() : nullptr)
@@ -430,7 +430,7 @@ struct BlockFn : torch::autograd::Function<BlockFn> {
     ctx->saved_data["b"] = std::vector<int64_t>{P, G, o.silu, o.norm_before_gate, 0, out_bias.has_value(), out_weight ? (int64_t)out_weight->scalar_type() : 0,
                                                 out_bias ? (int64_t)out_bias->scalar_type() : 0};
     ctx->saved_data["eps"] = o.eps;
-    variable_list out = {res.view({batch, L, -1})};
+    variable_list out = {out_weight ? res : y.view({batch, L, dim})};
     if (o.ssd.return_final) out.push_back(*r[5]);
     return out;
   }

@@ -1,5 +1,5 @@
-"""The operators' calls beside their plain use: forward-mode gradients, functorch's transforms, a jit trace, a projection's
-bias that does not fit, a projection of no rows."""
+"""The operators' calls beside their plain use: forward-mode gradients, functorch's transforms, a jit trace, an in-place
+write to the output, a projection's bias that does not fit, a projection of no rows."""
 import functools
 
 import pytest
@@ -104,6 +104,22 @@ def test_traced_call_replays(call):
             x, z = _operands(seed)
             got, want = traced(x, z), call(x, z)  # (the block's projection: sums of 64 products in another order)
             assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max())
+
+
+@pytest.mark.parametrize("bias", [False, True])
+def test_block_output_takes_in_place_writes(bias):
+    from mamba_amd.ops.triton.ssd_combined import mamba_split_conv1d_scan_combined
+    x, z = _operands()
+    args, kw = _block_args(x, z)
+    if bias:
+        kw["outproj_bias"] = torch.zeros(48, device="cuda")
+    args[0].requires_grad_()
+    out = mamba_split_conv1d_scan_combined(*args, **kw)
+    want, = torch.autograd.grad(out, args[0], torch.ones_like(out))
+    out = mamba_split_conv1d_scan_combined(*args, **kw)
+    out += 1.0
+    got, = torch.autograd.grad(out, args[0], torch.ones_like(out))
+    assert float((got - want).abs().max()) <= 1e-4 * float(want.abs().max())  # sums in another order (float atomics)
 
 
 @pytest.mark.parametrize("shape", [(47,), (1, 47), (0,)])

@@ -202,10 +202,10 @@ ScanArgs normalised(const at::Tensor &u, const at::Tensor &delta, const at::Tens
 }
 
 struct ScanFn : torch::autograd::Function<ScanFn> {
-  static variable_list forward(AutogradContext *ctx, const at::Tensor &u, const at::Tensor &delta, const at::Tensor &A,
-                               const at::Tensor &B, const at::Tensor &C, const OptTensor &D, const OptTensor &z,
-                               const OptTensor &delta_bias, bool delta_softplus, bool return_last_state) {
-    const ScanArgs a = normalised(u, delta, A, B, C, D, z, delta_bias);
+  // the gradients are those of the caller's tensors, the kernels and the backward pass take `a`
+  static variable_list forward(AutogradContext *ctx, const at::Tensor &, const at::Tensor &, const at::Tensor &, const at::Tensor &,
+                               const at::Tensor &, const OptTensor &, const OptTensor &, const OptTensor &, const ScanArgs &a,
+                               bool delta_softplus, bool return_last_state) {
     MambaScanParams p{};
     TORCH_CHECK(fill_scan(p, a.u, a.delta, a.A, a.B, a.C, a.D, a.z, a.delta_bias, delta_softplus), "selective_scan: arguments");
     auto [out, ckpt] = scan_fwd(p, a.u, a.delta);
@@ -225,7 +225,7 @@ struct ScanFn : torch::autograd::Function<ScanFn> {
     MambaScanParams p{};
     TORCH_CHECK(fill_scan(p, s[0], s[1], s[2], s[3], s[4], D, z, bias, ctx->saved_data["softplus"].toBool()), "selective_scan: arguments");
     const TensorList r = scan_bwd(p, s[0], s[1], s[3], s[4], D, z, bias, dout, s[8], std::nullopt, false);
-    variable_list g(10);
+    variable_list g(11);
     g[0] = *r[0], g[1] = *r[1], g[2] = *r[2];
     g[3] = *r[3], g[4] = *r[4];
     g[5] = tensor_or_none(r[5]), g[6] = tensor_or_none(r[7]), g[7] = tensor_or_none(r[6]);
@@ -241,14 +241,17 @@ pybind11::object selective_scan(const at::Tensor &u, const at::Tensor &delta, co
   if (!u.is_cuda() || u.dim() != 3 || delta.dim() != 3 || A.dim() != 2 || B.dim() < 2 || C.dim() < 2 || B.dim() > 4 || C.dim() > 4 ||
       (z && z->dim() != 3) || A.is_complex() || python_call(u, delta, A, B, C, D, z, delta_bias))
     return no;
-  const ScanArgs a = normalised(u, delta, A, B, C, D, z, delta_bias);
+  const ScanArgs a = [&] {
+    at::AutoGradMode no_grad(false);  // copies are not the caller's tensors: the node below knows those
+    return normalised(u, delta, A, B, C, D, z, delta_bias);
+  }();
   MambaScanParams p{};
   if (!fill_scan(p, a.u, a.delta, a.A, a.B, a.C, a.D, a.z, a.delta_bias, delta_softplus)) return no;
   if (!records(u, delta, A, B, C, D, z, delta_bias)) {
     auto [out, ckpt] = scan_fwd(p, a.u, a.delta);
     return return_last_state ? pybind11::object(pybind11::make_tuple(out, ckpt.select(2, ckpt.size(2) - 1))) : pybind11::cast(out);
   }
-  variable_list r = ScanFn::apply(u, delta, A, B, C, D, z, delta_bias, delta_softplus, return_last_state);
+  variable_list r = ScanFn::apply(u, delta, A, B, C, D, z, delta_bias, a, delta_softplus, return_last_state);
   return return_last_state ? pybind11::object(pybind11::make_tuple(r[0], r[1])) : pybind11::cast(r[0]);
 }
 

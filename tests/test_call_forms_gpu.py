@@ -1,5 +1,5 @@
 """The operators' calls beside their plain use: forward-mode gradients, functorch's transforms, a jit trace, an in-place
-write to the output, a projection's bias that does not fit, a projection of no rows."""
+write to the output, operands with the positions apart, a projection's bias that does not fit, a projection of no rows."""
 import functools
 
 import pytest
@@ -120,6 +120,32 @@ def test_block_output_takes_in_place_writes(bias):
     out += 1.0
     got, = torch.autograd.grad(out, args[0], torch.ones_like(out))
     assert float((got - want).abs().max()) <= 1e-4 * float(want.abs().max())  # sums in another order (float atomics)
+
+
+def test_strided_scan_operands_are_copied_once():
+    """u, delta, z and B, C with the positions apart: one dense copy each in the forward pass (nothing of them remains
+    but what the backward pass reads)."""
+    from mamba_amd.ops.selective_scan_interface import selective_scan_fn
+    g = torch.Generator(device="cuda").manual_seed(0)
+    dim, L, n = 512, 1024, 16
+    apart = lambda *s: torch.randn(*s[:-2], s[-1], s[-2], device="cuda", generator=g).transpose(-1, -2)
+    u, delta, z, B, C = apart(2, dim, L), apart(2, dim, L), apart(2, dim, L), apart(2, 1, n, L), apart(2, 1, n, L)
+    A = -torch.ones(dim, n, device="cuda")
+
+    def allocations(*ops):
+        leaves = [t.detach().requires_grad_() for t in ops]
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        out = selective_scan_fn(leaves[0], leaves[1], A, leaves[2], leaves[3], z=leaves[4], delta_softplus=True)
+        return torch.cuda.memory_stats()["allocation.all.allocated"] - before, out, leaves
+
+    dense = [t.contiguous() for t in (u, delta, B, C, z)]
+    n_dense, want, want_leaves = allocations(*dense)
+    n_apart, got, leaves = allocations(u, delta, B, C, z)
+    assert n_apart - n_dense == 5
+    assert torch.equal(got, want)
+    dout = torch.randn(want.shape, device="cuda", generator=g)
+    for a, b in zip(torch.autograd.grad(got, leaves, dout), torch.autograd.grad(want, want_leaves, dout)):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("shape", [(47,), (1, 47), (0,)])

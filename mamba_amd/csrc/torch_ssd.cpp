@@ -65,21 +65,41 @@ bool fill_ssd(SsdParams &p, SsdDims &d, const at::Tensor &x, const at::Tensor &d
 
 // The chunk length the kernels use for a call that names one of 64, 128 and 256: the scan's result is the same for each
 // but for rounding, and they differ in cost.  A longer chunk writes and reads fewer chunk states (headdim x dstate per
-// head), a shorter one has less of the quadratic part: the (chunk x chunk) tiles of dCB per group, and the causal
-// triangle's work.  256 wins with one group of 128 states where its chunks keep the chip busy, and wherever the states
-// after every 128 positions would outgrow the 256 MB last-level cache; otherwise 128.  Measured (64 / 128 / 256, us,
-// forward + backward in bf16): 2 x 7093 x 40 heads, 1 group, 128 states 663 / 559 / 476; 4039 x 72 heads, 8 groups, 128
-// states 402 / 339 / 391, but 32768 x 64 heads 2268 / 2050 (128 / 256); 13632 x 64 heads, 1 group, 64 states 926 / 765 /
-// 829; 1216 x 32 heads, 1 group, 128 states 122 / 124 / 143; fp16, 2 x 2257 x 80 heads, 8 groups, 64 states 641 / 590 /
-// 646.  A sequence within one chunk of 64 or 128 takes that.
-int64_t kernel_chunk(int64_t chunk_size, int64_t batch, int64_t L, int64_t H, int64_t G, int64_t P, int64_t N, at::ScalarType type) {
-  if (chunk_size != 64 && chunk_size != 128 && chunk_size != 256) return chunk_size;
-  if (L <= 128) return L <= 64 ? 64 : 128;
-  const bool fills = batch * H * ((L + 255) / 256) >= 384;  // one and a half workgroups for each of the 256 CUs
-  const bool cached = batch * H * ((L + 127) / 128) * P * N * 4 <= (256 << 20);
-  if ((type == at::kBFloat16 && G == 1 && N > 64 && fills) || !cached) return 256;
-  // (in the split-operand types short calls are a little faster with the chunk of 64 where the caller asks for it)
-  return type != at::kBFloat16 && !fills ? std::min<int64_t>(128, chunk_size) : 128;
+// head) and, at 256, has the paired scan kernel; a shorter one has less of the quadratic part, the (chunk x chunk) tiles of
+// dCB per group above all, which a call without gradients does not have, and more workgroups.  The named chunk stays unless
+// another one was faster in about every call of its class.  W: the workgroups a chunk of 256 gives, one per head.
+// Measured (64 / 128 / 256, us, bf16, headdim 64, gated; forward | forward + backward; g: groups, n: states):
+//   1 x 777 x 24       g1 n128  W 96     26.2 / 21.5 / 24.8  |  92 / 93 / 118      few workgroups: not 256
+//   1 x 4096 x 48      g8 n64   W 768    63.4 / 48.0 / 43.1  |  239 / 201 / 214    64 states, 8 groups: 256 without gradients,
+//   2 x 7093 x 40      g8 n64   W 2240   170 / 127 / 122     |  628 / 543 / 573      128 with them,
+//   1 x 32768 x 64     g8 n64   W 8192   569 / 421 / 369     |  2093 / 1742 / 1698   until the states outweigh the tiles
+//   1 x 1531 x 80      g1 n64   W 480    39.6 / 32.7 / 32.5  |  171 / 155 / 160    1 group: the tiles weigh less
+//   4 x 4096 x 16      g1 n64   W 1024   81 / 61 / 54        |  315 / 273 / 274
+//   2 x 7093 x 40      g1 n128  W 2240   264 / 205 / 147     |  747 / 638 / 561    128 states: the states weigh twice
+//   1 x 4039 x 72      g8 n128  W 1152   129 / 99 / 103      |  403 / 339 / 382    4.5 rounds of 256 CUs: half of one idle
+//   1 x 32768 x 64     g8 n128  W 8192   913 / 656 / 487     |  2767 / 2202 / 1971
+// Over 279 sizes (1 - 4 x 130 - 32768 x 16 - 80 heads, 1 and 8 groups, 64 and 128 states, gated or not) a call without
+// gradients that names 64 / 128 / 256 takes 0.79 / 0.93 / 0.98 of the named chunk's time in the mean and 1.04 / 1.15 / 1.11 at
+// worst (30 us, a last chunk nearly empty), one with gradients 0.90 / 0.99 / 0.94 and 1.08 / 1.03 / 1.03.  Operands in two
+// halves, and sizes that the fused kernels do not take: 128, or a named 64 in a short call (80 sizes: 0.93 / 1.00 / 0.92).
+int64_t kernel_chunk(int64_t named, int64_t batch, int64_t L, int64_t H, int64_t G, int64_t P, int64_t N, at::ScalarType type,
+                     bool backward) {
+  if (named != 64 && named != 128 && named != 256) return named;
+  if (L <= 128) return L <= 64 ? 64 : 128;  // one chunk
+  const int64_t W = batch * H * ((L + 255) / 256), at_most_128 = std::min<int64_t>(named, 128), at_least_128 = std::max<int64_t>(named, 128);
+  const bool fused = (P == 32 || P == 64) && (N == 64 || N == 128);
+  if (type != at::kBFloat16 || (!fused && N < 128)) {
+    if (N >= 128 && G == 1 && W >= 8192) return at_least_128;
+    return W < 384 ? at_most_128 : 128;
+  }
+  if (!backward) {
+    if (W < 160) return W < 96 ? at_most_128 : 128;
+    return N >= 128 || W >= 768 ? 256 : at_least_128;
+  }
+  if (W < 384) return W < 256 ? at_most_128 : 128;
+  const bool idle = W >= 768 && W < 2048 && (W + 255) / 256 * 256 * 10 >= W * 11;  // a tenth of 3 to 8 rounds
+  if (N >= 128) return W >= (G == 1 ? 768 : 2048) ? 256 : idle ? 128 : at_least_128;
+  return idle || W < (G == 1 ? 768 : 4096) ? 128 : at_least_128;
 }
 
 // Everything a forward or backward call of mamba_chunk_scan_combined takes, apart from its outputs.
@@ -332,13 +352,14 @@ pybind11::object chunk_scan(const at::Tensor &x, const at::Tensor &dt, const at:
                             const OptTensor &initial_states, const OptTensor &seq_idx, bool dt_softplus, double dt_min,
                             double dt_max, bool return_final) {
   if (python_call(x, dt, A, B, C, D, z, dt_bias, initial_states)) return pybind11::none();
+  const bool backward = records(x, dt, A, B, C, D, z, dt_bias, initial_states);
   if (x.dim() == 4 && B.dim() == 4)
-    chunk_size = kernel_chunk(chunk_size, x.size(0), x.size(1), x.size(2), B.size(2), x.size(3), B.size(3), x.scalar_type());
+    chunk_size = kernel_chunk(chunk_size, x.size(0), x.size(1), x.size(2), B.size(2), x.size(3), B.size(3), x.scalar_type(), backward);
   SsdParams p{};
   SsdDims d;
   const SsdArgs a{x, dt, A, B, C, chunk_size, D, z, dt_bias, initial_states, seq_idx, dt_softplus, dt_min, dt_max};
   if (!fill_ssd(p, d, a)) return pybind11::none();
-  if (!records(x, dt, A, B, C, D, z, dt_bias, initial_states)) {
+  if (!backward) {
     const TensorList r = ssd_fwd(p, d, a, false);  // no gradient asked for: the pre-gate copy is not written
     return return_final ? pybind11::object(pybind11::make_tuple(*r[0], *r[5])) : pybind11::cast(*r[0]);
   }
@@ -508,7 +529,8 @@ pybind11::object split_conv_scan(const at::Tensor &zxbcdt_in, const at::Tensor &
   if (H <= 0 || P <= 0 || H % G != 0 || conv <= dim || (conv - dim) % (2 * G) != 0 || batch <= 0 || L <= 0) return no;
   const int64_t N = (conv - dim) / (2 * G);
   if (zxbcdt.size(2) != dim + conv + H || dt_bias.dim() != 1 || dt_bias.size(0) != H || A.dim() != 1 || A.size(0) != H) return no;
-  chunk_size = kernel_chunk(chunk_size, batch, L, H, G, P, N, zxbcdt.scalar_type());
+  chunk_size = kernel_chunk(chunk_size, batch, L, H, G, P, N, zxbcdt.scalar_type(),
+                            records(zxbcdt, conv_weight, conv_bias, dt_bias, A, D, initial_states, norm_weight, out_weight, out_bias));
   const at::Tensor conv_w = conv_weight.dim() == 3 ? conv_weight.squeeze(1) : conv_weight;
   const at::Tensor xBC_in = zxbcdt.as_strided({batch, conv, L}, {zxbcdt.stride(0), 1, zxbcdt.stride(1)}, zxbcdt.storage_offset() + dim);
   if (!conv_params_ok(xBC_in, conv_w, conv_bias, seq_idx)) return no;

@@ -132,3 +132,29 @@ def test_ssd_ragged(monkeypatch, seqlen, chunk, dstate, ngroups, dtype, host):
 @pytest.mark.parametrize("seq_lens", [[3, 126, 70], [400, 13]])
 def test_ssd_ragged_packed(seq_lens):
     ssd._bwd_case(1, sum(seq_lens), 24, 64, 128, 1, 256, torch.bfloat16, seq_lens=seq_lens)
+
+
+# The chunk the kernels take for a call that names one: both sides of every line of the rule, for calls with and without
+# gradients.  The forward pass at that chunk gives the same bits through the stage-level function, which keeps what it is
+# given; every other chunk rounds elsewhere (the bound: bf16 inputs of the scan, 2^-8 of the largest output).
+@pytest.mark.parametrize("heads,seqlen,groups,dstate,named,backward,chunk", [
+    (8, 64, 1, 64, 256, False, 64), (8, 128, 1, 64, 256, True, 128),                  # one chunk
+    (19, 1280, 1, 128, 64, False, 64), (24, 1024, 1, 128, 64, False, 128),            # 95, 96 workgroups of 256
+    (53, 768, 1, 128, 256, False, 128), (40, 1024, 1, 128, 128, False, 256),          # 159, 160
+    (64, 2815, 1, 64, 256, False, 256), (64, 2815, 1, 64, 64, False, 128), (64, 3072, 1, 64, 64, False, 256),
+    (51, 1280, 1, 128, 64, True, 64), (32, 2048, 1, 128, 64, True, 128), (32, 3071, 8, 128, 256, True, 256),
+    (24, 4096, 8, 64, 256, True, 128), (64, 3072, 1, 64, 256, True, 256), (64, 3072, 1, 128, 128, True, 256),
+    (72, 4039, 8, 128, 256, True, 128), (64, 3072, 8, 128, 128, True, 128), (64, 8192, 8, 128, 128, True, 256)])
+def test_ssd_chunk_rule(heads, seqlen, groups, dstate, named, backward, chunk):
+    from mamba_amd.ops.triton.ssd_combined import _mamba_chunk_scan_combined_fwd, mamba_chunk_scan_combined
+    g = torch.Generator(device="cuda").manual_seed(0)
+    rn = lambda *s: torch.randn(*s, device="cuda", generator=g).bfloat16()
+    args = [rn(1, seqlen, heads, 64), rn(1, seqlen, heads), -torch.ones(heads, device="cuda"), rn(1, seqlen, groups, dstate),
+            rn(1, seqlen, groups, dstate)]
+    kw = dict(dt_bias=torch.full((heads,), -4.0, device="cuda"), dt_softplus=True)
+    args[0].requires_grad_(backward)
+    out, final = mamba_chunk_scan_combined(*args, named, return_final_states=True, **kw)
+    with torch.no_grad():
+        want, at_chunk = (_mamba_chunk_scan_combined_fwd(*args, q, **kw) for q in (named, chunk))
+    assert torch.equal(out, at_chunk[0]) and torch.equal(final, at_chunk[5])
+    assert float((out - want[0]).detach().abs().max()) <= 2.0 ** -8 * float(want[0].abs().max())

@@ -599,6 +599,10 @@ __global__ __launch_bounds__(NTHREADS) void scan_bwd_kernel(const MambaScanParam
           };
           Operands ops;
           fetch_operands(ops, 0);
+          // The loop's place in its 64-byte lines, which else moves with any change to the code above: most of its
+          // instructions take 8 bytes, and vector issue bounds it.  8 x 5120 x 4096 bf16, forward + backward, with 0 - 7
+          // words behind the boundary: 3229 3186 3218 3196 3229 3210 3250 3221 us.
+          asm volatile(".p2align 6\n\ts_nop 0");
           for (int ph = 0; ph < NPH; ++ph) {
             const int n = ((wave + ph + slot_shift) % NPH) * NPP;
             constexpr bool active = true;  // padded states run on zeros (A = B = C = 0)

@@ -79,8 +79,8 @@ bool fill_ssd(SsdParams &p, SsdDims &d, const at::Tensor &x, const at::Tensor &d
 //   1 x 4039 x 72      g8 n128  W 1152   129 / 99 / 103      |  403 / 339 / 382    4.5 rounds of 256 CUs: half of one idle
 //   1 x 32768 x 64     g8 n128  W 8192   913 / 656 / 487     |  2767 / 2202 / 1971
 // Over 279 sizes (1 - 4 x 130 - 32768 x 16 - 80 heads, 1 and 8 groups, 64 and 128 states, gated or not) a call without
-// gradients that names 64 / 128 / 256 takes 0.79 / 0.93 / 0.98 of the named chunk's time in the mean and 1.04 / 1.15 / 1.11 at
-// worst (30 us, a last chunk nearly empty), one with gradients 0.90 / 0.99 / 0.94 and 1.08 / 1.03 / 1.03.  Operands in two
+// gradients that names 64 / 128 / 256 takes 0.79 / 0.93 / 0.97 of the named chunk's time in the mean and 1.04 / 1.10 / 1.11 at
+// worst (calls of 25 - 45 us), one with gradients 0.90 / 0.99 / 0.94 and 1.08 / 1.03 / 1.03.  Operands in two
 // halves, and sizes that the fused kernels do not take: 128, or a named 64 in a short call (80 sizes: 0.93 / 1.00 / 0.92).
 int64_t kernel_chunk(int64_t named, int64_t batch, int64_t L, int64_t H, int64_t G, int64_t P, int64_t N, at::ScalarType type,
                      bool backward) {
@@ -94,6 +94,8 @@ int64_t kernel_chunk(int64_t named, int64_t batch, int64_t L, int64_t H, int64_t
   }
   if (!backward) {
     if (W < 160) return W < 96 ? at_most_128 : 128;
+    const int64_t W128 = batch * H * ((L + 127) / 128);
+    if (W < 384 && (N < 128 || W128 * 5 < W * 9)) return 128;  // (with 128 states: much of the last chunk empty)
     return N >= 128 || W >= 768 ? 256 : at_least_128;
   }
   if (W < 384) return W < 256 ? at_most_128 : 128;

@@ -141,6 +141,7 @@ def test_ssd_ragged_packed(seq_lens):
     (8, 64, 1, 64, 256, False, 64), (8, 128, 1, 64, 256, True, 128),                  # one chunk
     (19, 1280, 1, 128, 64, False, 64), (24, 1024, 1, 128, 64, False, 128),            # 95, 96 workgroups of 256
     (53, 768, 1, 128, 256, False, 128), (40, 1024, 1, 128, 128, False, 256),          # 159, 160
+    (112, 383, 1, 128, 128, False, 128), (127, 513, 1, 64, 256, False, 128), (128, 513, 1, 64, 256, False, 256),
     (64, 2815, 1, 64, 256, False, 256), (64, 2815, 1, 64, 64, False, 128), (64, 3072, 1, 64, 64, False, 256),
     (51, 1280, 1, 128, 64, True, 64), (32, 2048, 1, 128, 64, True, 128), (32, 3071, 8, 128, 256, True, 256),
     (24, 4096, 8, 64, 256, True, 128), (64, 3072, 1, 64, 256, True, 256), (64, 3072, 1, 128, 128, True, 256),

@@ -1562,8 +1562,8 @@ DEVI void bmm_chunk_bwd_wide_body(const SsdParams &p, int bx, int by, int bz, in
 template <typename T, bool SPLIT> __global__ __launch_bounds__(256) void bmm_chunk_bwd_kernel(const SsdParams p) {
   bmm_chunk_bwd_body<T, SPLIT, false>(p, blockIdx.x, blockIdx.y, blockIdx.z, 0);
 }
-template <typename T, bool SPLIT, int FORM> __global__ __launch_bounds__(256) void bmm_chunk_bwd_wide_kernel(const SsdParams p) {
-  bmm_chunk_bwd_wide_body<T, SPLIT, false, FORM != WIDE_WHOLE>(p, blockIdx.x, blockIdx.y, blockIdx.z, 0);
+template <typename T, bool SPLIT, bool RAGGED> __global__ __launch_bounds__(256) void bmm_chunk_bwd_wide_kernel(const SsdParams p) {
+  bmm_chunk_bwd_wide_body<T, SPLIT, false, RAGGED>(p, blockIdx.x, blockIdx.y, blockIdx.z, 0);
 }
 
 // --------------------------------------------------------- cumsum bwd
@@ -1904,8 +1904,13 @@ static int ssd_bmm_chunk_bwd_one(const SsdParams *p_in, mamba_stream_t stream) {
       wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs) && wide_operand_ok(p->C, p->dtype, p->C_bs, p->C_ls, p->C_gs) &&
       reinterpret_cast<uintptr_t>(p->dCB) % 16 == 0) {
     dim3 gridw(tiles(p->chunk_size) * (p->dstate / WB), p->nchunks, p->batch * p->ngroups);
-    const int form = ragged_end(p) ? WIDE_RAGGED : WIDE_WHOLE;
-    SSD_DISPATCH_FORM(bmm_chunk_bwd_wide_kernel, gridw, form, *p)
+#define SSD_LAUNCH_BMM(T, SPLIT)                                                                                              \
+  if (ragged_end(p)) hipLaunchKernelGGL((bmm_chunk_bwd_wide_kernel<T, SPLIT, true>), gridw, dim3(256), 0, s, *p);              \
+  else hipLaunchKernelGGL((bmm_chunk_bwd_wide_kernel<T, SPLIT, false>), gridw, dim3(256), 0, s, *p);
+    if (p->dtype == MAMBA_BF16) { SSD_LAUNCH_BMM(bf16_t, false) }
+    else if (p->dtype == MAMBA_F16) { SSD_LAUNCH_BMM(f16_t, true) }
+    else { SSD_LAUNCH_BMM(float, true) }
+#undef SSD_LAUNCH_BMM
     return launched();
   }
   dim3 grid(tiles(p->chunk_size) * tiles(p->dstate), p->nchunks, p->batch * p->ngroups);

@@ -261,3 +261,39 @@ def test_causal_conv1d_update_circular_buffer(width, state_len, dtype):
         got = causal_conv1d_update(pair, ring2, w, bias, "silu", cache_seqlens=lens2)
         assert torch.equal(got, want), f"pair at {t}"
         lens2 += 2
+
+
+@pytest.mark.parametrize("form", ["atomics", "fixed point"])
+@pytest.mark.parametrize("dtype,channel_last,seqlen,dim", [(torch.float32, False, 333, 20), (torch.bfloat16, True, 200, 24),
+                                                           (torch.bfloat16, True, 300, 264)])
+def test_abi_backward_without_workspace(form, dtype, channel_last, seqlen, dim):
+    """causal_conv1d_bwd for a caller that brings no dw_part: fp32 sums added into, or their int64 shadows, against the
+    sums in a fixed order.  The terms are the same fp32 numbers; what differs is the order of at most batch x seqlen of
+    them (2^-24 each), and with the fixed point one rounding of 2^-31 of the largest gradient per workgroup."""
+    from mamba_amd import _lib
+    from mamba_amd.ops import causal_conv1d as host
+    from mamba_amd.utils.determinism import fixed_point_scale
+    g = torch.Generator().manual_seed(3)
+    batch, width = 2, 4
+    rows = lambda: torch.randn(batch, seqlen, dim, generator=g).cuda().to(dtype).transpose(1, 2)
+    x, dout = (rows() if channel_last else rows().contiguous() for _ in range(2))
+    w, b = torch.randn(dim, width, generator=g).cuda(), torch.randn(dim, generator=g).cuda()
+    dx_ref, dw_ref, db_ref = host.causal_conv1d_bwd(x, w, b, dout, activation="silu")
+    dx, dw, db = torch.empty_like(dx_ref), torch.zeros_like(w), torch.zeros_like(b)
+    p = _lib.CausalConvParams()
+    host._fill(p, x, w, b, None, "silu")
+    p.dout, p.dx, p.dweight, p.dbias = dout.data_ptr(), dx.data_ptr(), dw.data_ptr(), db.data_ptr()
+    p.dout_bs, p.dout_cs, p.dout_ls = dout.stride()
+    p.dx_bs, p.dx_cs, p.dx_ls = dx.stride()
+    lib, stream = _lib.load(), _lib.current_stream(x.device)
+    if form == "fixed point":
+        scale = fixed_point_scale(dout)
+        shadows = [torch.zeros(t.numel(), dtype=torch.int64, device="cuda") for t in (dw, db)]
+        p.det_scale, p.det_dweight, p.det_dbias = scale.data_ptr(), shadows[0].data_ptr(), shadows[1].data_ptr()
+    _lib.check(lib.causal_conv1d_bwd(p, stream), "causal_conv1d_bwd")
+    if form == "fixed point":
+        for shadow, t in zip(shadows, (dw, db)):
+            _lib.check(lib.ssd_det_convert(shadow.data_ptr(), t.data_ptr(), t.numel(), scale.data_ptr(), stream), "ssd_det_convert")
+    assert torch.equal(dx, dx_ref)
+    for got, ref in ((dw, dw_ref), (db, db_ref)):
+        assert float((got - ref).abs().max()) <= batch * seqlen * 2.0 ** -24 * float(ref.abs().max())

@@ -37,10 +37,10 @@ namespace {
 // ------------------------------------------------------------------ segments of the sequence
 // With few (batch, channel) rows the chip is filled by cutting the sequence into p.nseg segments (p.seg_ws).  A
 // segment's part of the recurrence is a (decay, value) pair per (channel, state), as a lane's and a tile's are: the
-// value is formed by scan_seg_fwd_kernel, the decay is exp(A * sum of the segment's steps), and the scan kernels compose
-// the pairs of the segments before theirs when they start.  The adjoint is handled the same way from the other end
-// (scan_seg_bwd_kernel).  seg_ws: values (batch, nseg, dim, N), then the sums of the steps (batch, nseg, dim; backward:
-// without the first one), then the first steps (batch, nseg, dim; backward only).
+// value is formed by scan_seg_kernel, the decay is exp(A * sum of the segment's steps), and the scan kernels compose the
+// pairs of the segments before theirs when they start.  The adjoint is handled the same way from the other end.  seg_ws:
+// values (batch, nseg, dim, N), then the sums of the steps (batch, nseg, dim; backward: without the first one), then the
+// first steps (batch, nseg, dim; backward only).
 DEVI int64_t seg_row(const MambaScanParams &p, int b, int seg, int d) { return ((int64_t)b * p.nseg + seg) * p.dim + d; }
 DEVI float *seg_sums(const MambaScanParams &p) { return p.seg_ws + (int64_t)p.batch * p.nseg * p.dim * p.dstate; }
 DEVI float *seg_firsts(const MambaScanParams &p) { return seg_sums(p) + (int64_t)p.batch * p.nseg * p.dim; }

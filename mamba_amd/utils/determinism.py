@@ -2,11 +2,12 @@
 (mamba_ssm/utils/determinism.py:21-33): an explicit override, else the environment variable
 MAMBA_DETERMINISTIC (first character '1' = on), else torch.are_deterministic_algorithms_enabled().
 
-What the mode changes here: the backward passes of the SSD scan and of the causal convolution add the
-sums that several workgroups share (dB, dC, the dt / decay gradients, dA, dD, dt_bias, the conv weight and
-bias gradients) with 64-bit integer atomics on terms scaled to a fixed point, instead of float atomics;
-integer addition does not depend on the order of the adds, so every gradient repeats bit for bit.  Every
-other operator of the package is deterministic in either mode."""
+What the mode changes here: the backward passes of the SSD scan and of the Mamba-1 scan with a complex A add the
+sums that several workgroups share (dB, dC, the dt / decay gradients, dA, dD, dt_bias) with 64-bit integer
+atomics on terms scaled to a fixed point, instead of float atomics; integer addition does not depend on the
+order of the adds, so every gradient repeats bit for bit.  Every other operator of the package, the causal
+convolution among them (its sums leave the workgroups as partials that are added in a fixed order), is
+deterministic in either mode."""
 import os
 import sys
 

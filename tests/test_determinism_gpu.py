@@ -1,9 +1,9 @@
 """Run-to-run reproducibility (the reference's tests/test_determinism.py:186-211 asks for bitwise equality in
 its deterministic mode and 1e-2 agreement with the default mode).  Here: every forward operator, the decode step,
-the norm backward passes and the Mamba-1 scan's backward pass (real A) use no float atomics and must repeat bit
-for bit in the one mode there is; the SSD and conv backward passes still sum dB, dC, ddt, dA, dD and the conv
-weight gradient with float atomics, so their repeats must agree to rounding noise of the sums (far inside the
-reference's 1e-2) but not bit for bit."""
+the norm and convolution backward passes and the Mamba-1 scan's backward pass (real A) use no float atomics and
+must repeat bit for bit in the one mode there is; the SSD backward pass sums dB, dC, ddt, dA and dD with float
+atomics, so its repeats must agree to rounding noise of the sums (far inside the reference's 1e-2) but not bit for
+bit, except in the deterministic mode."""
 import pytest
 import torch
 
@@ -217,6 +217,25 @@ def test_conv_and_block_backward_deterministic_mode(deterministic_mode):
         out.backward(dout)
         return [zx.grad] + [v.grad for v in lv.values()]
     a, b = _twice(block)
+    for ga, gb in zip(a, b):
+        assert torch.equal(ga, gb)
+
+
+@pytest.mark.parametrize("channel_last", [False, True])
+def test_conv_backward_repeats(channel_last):
+    """Without the deterministic mode: the filter and bias sums leave the workgroups as partials."""
+    from mamba_amd.ops.causal_conv1d import causal_conv1d_fn
+    g = torch.Generator().manual_seed(2)
+    x, dout = (torch.randn(3, 700, 264, generator=g).bfloat16().cuda().transpose(1, 2) for _ in range(2))
+    if not channel_last:
+        x, dout = x.contiguous(), dout.contiguous()
+    w, bias = torch.randn(264, 4, generator=g).cuda(), torch.randn(264, generator=g).cuda()
+
+    def grads():
+        leaves = [t.clone().requires_grad_() for t in (x, w, bias)]
+        causal_conv1d_fn(*leaves, activation="silu").backward(dout)
+        return [t.grad for t in leaves]
+    a, b = _twice(grads)
     for ga, gb in zip(a, b):
         assert torch.equal(ga, gb)
 

@@ -363,6 +363,7 @@ DEVI float det_value(int64_t sum, float inv_scale) {
 enum : int {
   DPP_ROW_SHL = 0x100,
   DPP_ROW_SHR = 0x110,
+  DPP_ROW_ROR = 0x120,
   DPP_WAVE_SHL1 = 0x130,
   DPP_WAVE_SHR1 = 0x138,
   DPP_ROW_BCAST15 = 0x142,
@@ -531,6 +532,15 @@ DEVI float row_sum_to_last(float x) {
   x += dpp_f<DPP_ROW_SHR + 2>(0.f, x);
   x += dpp_f<DPP_ROW_SHR + 4>(0.f, x);
   x += dpp_f<DPP_ROW_SHR + 8>(0.f, x);
+  return x;
+}
+
+// The same in every lane of the row, the same bits in each.
+DEVI float row_sum_all(float x) {
+  x += dpp_f<DPP_ROW_ROR + 8>(0.f, x);
+  x += dpp_f<DPP_ROW_ROR + 4>(0.f, x);
+  x += dpp_f<DPP_ROW_ROR + 2>(0.f, x);
+  x += dpp_f<DPP_ROW_ROR + 1>(0.f, x);
   return x;
 }
 

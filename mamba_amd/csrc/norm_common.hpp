@@ -119,12 +119,16 @@ DEVI void load_params(const void *base, int dtype, int64_t off, int col, int gs,
   }
 }
 
-// Sums over a workgroup of blockDim.x threads (whole waves), whatever their number: DPP adds inside a wave, the waves'
-// totals through LDS in alternating slots (one barrier per sum).
+// Sums over a workgroup of blockDim.x threads (whole waves, at most 16), whatever their number: DPP adds inside a wave,
+// the waves' totals through LDS in alternating slots (one barrier per sum), of which every row of 16 lanes reads one per
+// lane and adds them up by rotations.  (A loop over the waves' totals made a row of 5120 channels wait for ten LDS reads
+// one after the other.)
 struct WideSum {
   float *red;  // LDS: 2 slots x 16 waves x 2 floats
   int slot = 0, nw;
-  DEVI explicit WideSum(float *lds) : red(lds), nw(blockDim.x >> 6) {}
+  DEVI explicit WideSum(float *lds) : red(lds), nw(blockDim.x >> 6) {
+    if (threadIdx.x < 64 && (int)(threadIdx.x & 31) >= 2 * nw) red[threadIdx.x] = 0.f;  // waves that are not there
+  }
   DEVI void sum2(float &a, float &b) {
     a = wave_sum_to_last(a);
     b = wave_sum_to_last(b);
@@ -136,13 +140,9 @@ struct WideSum {
     float *s = red + slot * 32;
     if ((threadIdx.x & 63) == 63) *reinterpret_cast<f32x2 *>(s + (threadIdx.x >> 6) * 2) = f32x2{a, b};
     lds_barrier();
-    a = 0.f;
-    b = 0.f;
-    for (int w = 0; w < nw; ++w) {
-      const f32x2 v = *reinterpret_cast<const f32x2 *>(s + w * 2);
-      a += v.x;
-      b += v.y;
-    }
+    const f32x2 v = *reinterpret_cast<const f32x2 *>(s + (threadIdx.x & 15) * 2);
+    a = row_sum_all(v.x);
+    b = row_sum_all(v.y);
     slot ^= 1;
   }
 };

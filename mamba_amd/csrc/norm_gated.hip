@@ -239,20 +239,23 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 5 : 8) void norm_fwd_wide_ke
   const float inv_n = 1.f / (float)gs;
   const bool gate_after = HAS_Z && p.norm_before_gate, gate_before = HAS_Z && !p.norm_before_gate;
   const int last = part + (rows - 1 - part) / nparts * nparts;  // the last row of this part
-  Pack8<T> cx, cz;
-  cx.load_global(xp + (int64_t)part * p.x_rs);
-  if (HAS_Z) cz.load_global(zp + (int64_t)part * p.z_rs);
+  struct Row {
+    Pack8<T> x, z;
+  };
+  auto request = [&](Row &k, int r) {
+    k.x.load_global(xp + (int64_t)r * p.x_rs);
+    if (HAS_Z) k.z.load_global(zp + (int64_t)r * p.z_rs);
+  };
+  Row k0, k1;
+  request(k0, part);
   ld8_param(p.weight, p.weight_dtype, c0, w);
   if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
-  for (int r = part; r < rows; r += nparts) {
-    const int rn = min(r + nparts, last);
-    Pack8<T> nx, nz;
-    nx.load_global(xp + (int64_t)rn * p.x_rs);
-    if (HAS_Z) nz.load_global(zp + (int64_t)rn * p.z_rs);
+  auto walk = [&](int r, const Row &cur, Row &next) {
+    request(next, min(r + nparts, last));
     float x[8], sz[8];
-    cx.unpack(x);
+    cur.x.unpack(x);
     if (HAS_Z) {
-      cz.unpack(sz);
+      cur.z.unpack(sz);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         float sig;
@@ -291,8 +294,12 @@ __global__ __launch_bounds__(1024, sizeof(T) == 4 ? 5 : 8) void norm_fwd_wide_ke
       if (p.mean) p.mean[(int64_t)r * ngroups + group] = mean;
       p.rstd[(int64_t)r * ngroups + group] = rstd;
     }
-    cx = nx;
-    if (HAS_Z) cz = nz;
+  };
+  for (int r = part;; r += 2 * nparts) {  // two rows per round, as in the backward kernel
+    walk(r, k0, k1);
+    if (r + nparts >= rows) break;
+    walk(r + nparts, k1, k0);
+    if (r + 2 * nparts >= rows) break;
   }
 }
 
@@ -325,27 +332,28 @@ __global__ __launch_bounds__(1024) void norm_bwd_wide_kernel(const NormGatedPara
   const bool gate_after = HAS_Z && p.norm_before_gate, gate_before = HAS_Z && !p.norm_before_gate;
   if (part < rows) {
     const int last = part + (rows - 1 - part) / nparts * nparts;  // the last row of this part
-    Pack8<T> cx, cg, cz;
-    float cmean = *(const GLOBAL_AS float *)(meanp + (int64_t)part * ngroups);
-    float crstd = *(const GLOBAL_AS float *)(rstdp + (int64_t)part * ngroups);
-    cx.load_global(xp + (int64_t)part * p.x_rs);
-    cg.load_global(gp + (int64_t)part * p.dy_rs);
-    if (HAS_Z) cz.load_global(zp + (int64_t)part * p.z_rs);
+    struct Row {
+      Pack8<T> x, g, z;
+      float mean, rstd;
+    };
+    auto request = [&](Row &k, int r) {
+      k.mean = *(const GLOBAL_AS float *)(meanp + (int64_t)r * ngroups);
+      k.rstd = *(const GLOBAL_AS float *)(rstdp + (int64_t)r * ngroups);
+      k.x.load_global(xp + (int64_t)r * p.x_rs);
+      k.g.load_global(gp + (int64_t)r * p.dy_rs);
+      if (HAS_Z) k.z.load_global(zp + (int64_t)r * p.z_rs);
+    };
+    Row k0, k1;
+    request(k0, part);
     ld8_param(p.weight, p.weight_dtype, c0, w);
     if (p.bias) ld8_param(p.bias, p.weight_dtype, c0, b);
-    for (int r = part; r < rows; r += nparts) {
-      const int rn = min(r + nparts, last);
-      Pack8<T> nx, ng, nz;
-      const float nmean = *(const GLOBAL_AS float *)(meanp + (int64_t)rn * ngroups);
-      const float nrstd = *(const GLOBAL_AS float *)(rstdp + (int64_t)rn * ngroups);
-      nx.load_global(xp + (int64_t)rn * p.x_rs);
-      ng.load_global(gp + (int64_t)rn * p.dy_rs);
-      if (HAS_Z) nz.load_global(zp + (int64_t)rn * p.z_rs);
+    auto walk = [&](int r, const Row &cur, Row &next) {
+      request(next, min(r + nparts, last));
       float x[8], g[8], z[8], xr[8];
-      cx.unpack(x);
-      cg.unpack(g);
-      if (HAS_Z) cz.unpack(z);
-      const float mean = p.is_rms ? 0.f : cmean, rstd = crstd;
+      cur.x.unpack(x);
+      cur.g.unpack(g);
+      if (HAS_Z) cur.z.unpack(z);
+      const float mean = p.is_rms ? 0.f : cur.mean, rstd = cur.rstd;
       float c1 = 0.f, c2 = 0.f;
       // after this loop: x = xhat, g = w * dy', z = dz (gate after the norm) or kept as z (gate before it), xr = x
 #pragma unroll
@@ -393,11 +401,14 @@ __global__ __launch_bounds__(1024) void norm_bwd_wide_kernel(const NormGatedPara
         oz.pack(z);
         oz.store_global(dzp + (int64_t)r * p.dz_rs);
       }
-      cx = nx;
-      cg = ng;
-      if (HAS_Z) cz = nz;
-      cmean = nmean;
-      crstd = nrstd;
+    };
+    // Two rows per round, so that none of the requested registers are copied: a copy at the end of a row would wait for
+    // the next one.
+    for (int r = part;; r += 2 * nparts) {
+      walk(r, k0, k1);
+      if (r + nparts >= rows) break;
+      walk(r + nparts, k1, k0);
+      if (r + 2 * nparts >= rows) break;
     }
   }
   float *dwp = p.dw_part + (int64_t)part * p.dim + c0;
@@ -462,10 +473,23 @@ template <typename T, bool VEC> int pick_team(const NormGatedParams &p, bool bwd
 
 bool wide_group(int gs) { return gs > 1024 && gs <= 8192 && gs % 8 == 0; }
 
+// Parts of the rows in the forward pass: as many as workgroups the chip holds at once, or down to half of that where the
+// last round of rows is fuller then (16384 rows of 5120 channels: 32 rounds of two workgroups per CU take 91 us, 21.3 of
+// three 94.5).
+int wide_fwd_parts(int rows, int ngroups, int resident) {
+  int best = 1;
+  int64_t cost = INT64_MAX;  // workgroups per CU x rounds
+  for (int w = resident; w >= max(1, (resident + 1) / 2); --w) {
+    const int parts = max(1, min(rows, cu_count() * w / ngroups));
+    const int64_t c = ((int64_t)rows + parts - 1) / parts * w;
+    if (c < cost) cost = c, best = parts;
+  }
+  return best;
+}
+
 template <typename T> int launch_wide(const NormGatedParams &p, bool bwd, hipStream_t st) {
-  // forward: as many parts as workgroups the chip holds at once, never more than rows
   const int ngroups = p.dim / p.group_size, threads = wide_threads(p.group_size);
-  const int nparts = bwd ? p.nparts : max(1, min(p.rows, cu_count() * wide_resident(threads, 8) / ngroups));
+  const int nparts = bwd ? p.nparts : wide_fwd_parts(p.rows, ngroups, wide_resident(threads, 8));
   const int64_t wgs = (int64_t)ngroups * nparts;
   if (wgs > 0x7fffffff) return MAMBA_E_UNSUPPORTED;
   const dim3 grid((unsigned)wgs), block(threads);

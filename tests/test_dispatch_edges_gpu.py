@@ -98,6 +98,12 @@ def test_gated_norm_wide_groups(dim, group_size, wtype):
     gated._case(37, dim, group_size, torch.bfloat16, norm_before_gate=False, has_bias=True, wtype=wtype)
 
 
+# one, two, three and more rows per workgroup of the wide kernels (256 workgroups backward, 512 or 768 forward)
+@pytest.mark.parametrize("rows", [256, 257, 600, 1100, 1800])
+def test_gated_norm_wide_rows(rows):
+    gated._case(rows, 5120, 5120, torch.bfloat16, norm_before_gate=False, has_bias=True)
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 8), (130, 2570), (700, 1032)])
 def test_residual_norm_low_precision_parameters(rows, dim):
     from mamba_amd.ops.triton.layer_norm import layer_norm_fn

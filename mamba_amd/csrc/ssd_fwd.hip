@@ -753,7 +753,8 @@ static int ssd_combined_fwd_one(const SsdParams *p, mamba_stream_t stream) {
   if (rc) return rc;
   const bool walk = chunk_state_passing_pays(p);
   // The steps and their sums: a launch of their own where there is much to do, in the chunk_state kernel (whose workgroups
-  // then read the strided steps of their chunk one by one) while that has no more than eight workgroups per CU.
+  // then read the strided steps of their chunk one by one) while that has no more than eight workgroups per CU: 1531 x 80
+  // heads 6.6 + 12.9 us against 15.1, 2 x 1000 x 24 5.4 + 10.2 against 11.9.
   const bool merged = !walk && (int64_t)p->nchunks * p->batch * p->nheads <= 8 * (int64_t)cu_count();
   if (!merged && (rc = ssd_chunk_cumsum_fwd(p, stream))) return rc;
   if (walk) {

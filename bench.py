@@ -836,7 +836,7 @@ def bench_mamba1(dev, steps, warmup):
     fwd_bytes = 4 * E + 2 * BC   # reads u, delta, z, B, C; writes out
     achieved = bwd_bytes / (bwd_ms * 1e-3) / 1e9
     prof = "mamba1_scan_b8_d5120_l4096_n16_bf16"
-    roofline = {"bound": "hbm", "kernel": "scan_bwd_kernel (+ reduce_parts_kernel x 2)", "achieved": achieved,
+    roofline = {"bound": "hbm", "kernel": "scan_bwd_kernel (+ reduce_parts_kernel)", "achieved": achieved,
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                 "traffic": profile_traffic(prof + "_hbm_counters.txt", "scan_bwd_kernel"),
                 "kernel_ms": bwd_ms, "kernel_ms_min_max_n": [bwd_st["min"], bwd_st["max"], bwd_st["n"]],

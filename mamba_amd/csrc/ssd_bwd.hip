@@ -1847,18 +1847,55 @@ static bool dcb_rows_ok(const SsdParams *p) {
          aligned(p->x, 16) && !(g_ls % 8 || g_hs % 8 || g_bs % 8) && !(p->x_ls % 8 || p->x_hs % 8 || p->x_bs % 8) &&
          g_ls < (1 << 21) && p->x_ls < (1 << 21);
 }
+// Which kernel forms dCB, and the head lists per group it takes.  `chunk`: a workgroup per chunk and list that holds the
+// chunk's whole triangle (ssd_dcb_chunk.hip), else one per 64 x 64 tile pair and list; the one with the shorter estimate in
+// us, fitted to both at 37 sizes (4 - 1128 chunks x groups, 2 - 80 heads per group; most within 20 %).  The triangle: a
+// round of one, two or four workgroups per CU (chunks of 256, 128, 64) takes `fixed` and `head` for every head of a list,
+// a workgroup `store` for its sums, a quarter of that where it owns them.  The tile pairs: four workgroups per CU, a round
+// 9 and 1.0 to 2.6 (the CUs full) per head.  256 positions, 80 heads x 64 chunks: 161 -> 108 us in 4 lists; 8 groups of 8
+// heads x 128: 266 -> 204; 48 heads x 32 chunks: 47 against 56, the tile pairs stay; chunks of 128, 32 heads x 10: 17 ->
+// 15; chunks of 64, 16 heads x 77: 25 -> 13.
+// Groups of up to 16 heads are one list, whose sums need no clearing and go on as bf16, but for chunks of up to 128 with
+// more than 8 heads, where several lists pay (at 256: 25.4 against 25.3 us for 16 heads x 13 chunks).
+struct DcbPlan {
+  bool chunk;
+  int lists;
+};
+static DcbPlan dcb_plan(const SsdParams *p) {
+  DcbPlan best{false, dcb_head_splits(p)};
+  const int Q = p->chunk_size, hpg = p->nheads / p->ngroups;
+  if (!dcb_rows_ok(p) || (Q != 64 && Q != 128 && Q != 256) || p->dstate % p->headdim) return best;
+  if (!wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs) || !wide_operand_ok(p->C, p->dtype, p->C_bs, p->C_ls, p->C_gs) ||
+      p->B_ls >= (1 << 21) || p->C_ls >= (1 << 21))
+    return best;
+  const int64_t cus = cu_count(), tiles = (int64_t)p->nchunks * p->batch * p->ngroups, nt = Q / GB;
+  const double pairs = (double)(nt * (nt + 1) / 2 * tiles * best.lists) / (4.0 * cus);
+  double cost = std::max(1.0, pairs) * (9.0 + (1.0 + 1.6 * std::min(1.0, pairs)) * ((hpg + best.lists - 1) / best.lists));
+  const double fixed = Q == 256 ? 16.0 : Q == 128 ? 8.0 : 6.0, head = Q == 256 ? 3.2 : Q == 128 ? 1.83 : 1.32,
+               store = Q == 256 ? 0.08 : Q == 128 ? 0.035 : 0.02;
+  const int64_t slots = cus * (256 / Q);
+  const int most = best.lists == 1 && (Q == 256 || hpg <= 8) ? 1 : (int)std::min<int64_t>(hpg, 65535 / p->ngroups);
+  for (int n = 1; n <= most; ++n) {
+    const int64_t wgs = tiles * n;
+    const double c = (double)((wgs + slots - 1) / slots) * (fixed + head * ((hpg + n - 1) / n)) + store * (n > 1 ? 1.0 : 0.25) * (double)wgs;
+    if (c < cost) cost = c, best = DcbPlan{true, n};
+  }
+  return best;
+}
 // Inside ssd_combined_bwd the dCB tiles pass from the dCB stage to the bmm stage as bf16 where one workgroup owns each
 // tile and the bmm stage's operand is bf16 anyway (the stages on their own keep the fp32 tiles their interface names).
 static int64_t bmm_cumsum_workgroups(const SsdParams *p);
 static bool dcb_tiles_lp(const SsdParams *p) {
-  return dcb_rows_ok(p) && p->dCB && dcb_head_splits(p) == 1 && bmm_cumsum_workgroups(p) <= 0x7fffffff;  // (the one-launch form of the last two stages is the reader)
+  return dcb_rows_ok(p) && p->dCB && dcb_plan(p).lists == 1 && bmm_cumsum_workgroups(p) <= 0x7fffffff;  // (the one-launch form of the last two stages is the reader)
 }
 
 static int ssd_bwd_dcb_one(const SsdParams *p, mamba_stream_t stream, bool lp) {
   int rc = check_bwd(p);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int nt = tiles(p->chunk_size), nsplit = dcb_head_splits(p);
+  const DcbPlan plan = dcb_plan(p);
+  if (plan.chunk) return ssd_bwd_dcb_chunk_launch(p, lp, plan.lists, s);
+  const int nt = tiles(p->chunk_size), nsplit = plan.lists;
   dim3 grid(nt * (nt + 1) / 2, p->nchunks, p->batch * p->ngroups * nsplit);
   if (dcb_rows_ok(p)) {
     const int lpi = lp ? 1 : 0;
@@ -2078,11 +2115,14 @@ static int ssd_combined_bwd_one(const SsdParams *p, mamba_stream_t stream) {
 extern "C" int ssd_bwd_overwrites(const SsdParams *p) {
   if (!p || check_bwd(p) != MAMBA_OK || p->det_scale || (int64_t)p->batch * p->nheads > SSD_MAX_GRID_ROWS) return 0;
   int flags = 0;
-  if (dcb_head_splits(p) == 1) flags |= SSD_OVERWRITES_DCB;
+  const DcbPlan plan = dcb_plan(p);
+  if (plan.lists == 1) flags |= SSD_OVERWRITES_DCB;
   if (ssd_bwd_dbc_fused_owns(p)) flags |= SSD_OVERWRITES_DBC;
-  // CB: only the dCB stage and the tiled dx kernel read it.  Where the fused dx kernel runs and a group is one head
-  // list (so that each tile of C B^T would be formed once), the dCB stage can form its tiles itself.
-  if (dcb_head_splits(p) == 1 && ssd_bwd_dx_fused_supported(p)) flags |= SSD_BWD_FORMS_CB;
+  // CB: only the dCB stage and the tiled dx kernel read it.  Where the fused dx kernel runs, the dCB stage can form its
+  // tiles itself, once per head list, in less time than it takes to read them (the tile pairs, 5 lists of 16 heads x 64
+  // chunks: 161 against 174 us with CB, and 8 for the launch that forms it).  Short problems in more than 12 lists keep the
+  // answer their callers have always had.
+  if (ssd_bwd_dx_fused_supported(p) && (plan.lists == 1 || (dcb_rows_ok(p) && plan.lists <= 12))) flags |= SSD_BWD_FORMS_CB;
   return flags;
 }
 

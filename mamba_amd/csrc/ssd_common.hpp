@@ -877,6 +877,8 @@ __attribute__((visibility("hidden"))) bool ssd_bwd_dx_fused_supported(const SsdP
 // tiled bwd_d*_state kernels).
 __attribute__((visibility("hidden"))) int ssd_bwd_dbc_fused_launch(const SsdParams *p, hipStream_t stream);
 __attribute__((visibility("hidden"))) bool ssd_bwd_dbc_fused_owns(const SsdParams *p);
+// The dCB kernel that holds a chunk's whole triangle (ssd_dcb_chunk.hip), for the problems dcb_plan gives it.
+__attribute__((visibility("hidden"))) int ssd_bwd_dcb_chunk_launch(const SsdParams *p, bool lp, int nsplit, hipStream_t stream);
 
 // ---- host side of the kernels that work through the heads of a group in one workgroup
 inline bool aligned(const void *ptr, int a) { return (reinterpret_cast<uintptr_t>(ptr) % a) == 0; }

@@ -312,7 +312,7 @@ DEVI float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 // log1p(e) for small e is evaluated by its series so that tiny step sizes keep
 // full relative precision.
 DEVI float softplus_f(float x) {
-  float e = fast_exp(fminf(x, 20.f));
+  float e = fast_exp(x);  // (past the threshold it is not used)
   float big = fast_log(1.f + e);
   float small = e * (1.f - e * (0.5f - e * (0.33333333f - 0.25f * e)));
   float r = (e < 0.03f) ? small : big;

@@ -21,6 +21,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -30,6 +31,7 @@ size_t mamba1_bwd_mx_lds(int passes, int np);                                   
 int mamba1_bwd_mx_launch(const MambaScanParams &p, int passes, bool vec, hipStream_t stream);  // likewise
 size_t mamba1_bwd_k4_lds(int passes);                                                          // mamba1_scan_bwd_k4.hip
 bool mamba1_bwd_k4_serves(const MambaScanParams &p);                                           // likewise
+int mamba1_fwd_serial_launch(const MambaScanParams &p, int mode, hipStream_t s);                // mamba1_scan_serial.hip
 int mamba1_bwd_k4_launch(const MambaScanParams &p, int pa, int pb, int nparts, hipStream_t stream);  // likewise
 
 namespace {
@@ -41,19 +43,6 @@ namespace {
 // pairs of the segments before theirs when they start.  The adjoint is handled the same way from the other end.  seg_ws:
 // values (batch, nseg, dim, N), then the sums of the steps (batch, nseg, dim; backward: without the first one), then the
 // first steps (batch, nseg, dim; backward only).
-DEVI int64_t seg_row(const MambaScanParams &p, int b, int seg, int d) { return ((int64_t)b * p.nseg + seg) * p.dim + d; }
-DEVI float *seg_sums(const MambaScanParams &p) { return p.seg_ws + (int64_t)p.batch * p.nseg * p.dim * p.dstate; }
-DEVI float *seg_firsts(const MambaScanParams &p) { return seg_sums(p) + (int64_t)p.batch * p.nseg * p.dim; }
-
-// State entering this workgroup's segment (A2 = A log2 e)
-DEVI float seg_state_in(const MambaScanParams &p, const Geo &q, int d, int n, float A2) {
-  float h = 0.f;
-  for (int s = 0; s < q.seg; ++s) {
-    const int64_t row = seg_row(p, q.b, s, d);
-    h = __builtin_fmaf(fast_exp2(A2 * seg_sums(p)[row]), h, p.seg_ws[row * p.dstate + n]);
-  }
-  return h;
-}
 // Adjoint at the first position of the segment after this workgroup's, and the decay of that position
 DEVI float seg_adjoint_in(const MambaScanParams &p, const Geo &q, int d, int n, float A2, float &decay) {
   float g = 0.f;
@@ -945,19 +934,41 @@ int bwd_passes(const MambaScanParams &p, int64_t *cost_out = nullptr) {
   return best;
 }
 
+// The forward kernel that serves a problem and its estimated time in us, for 16 states.  scan_fwd_serial_kernel
+// (mamba1_scan_serial.hip) takes 16 states and per-position B and C; up to five of its workgroups share a CU, and a tile
+// (half tiles where the sequence ends in one) takes a round of them 7.3, 10.7, 14.1, 17.5, 20.9.  scan_fwd_kernel: up to
+// two per CU, 6.6 or 10.9, and a seventh more of that on rows with a ragged end.  Measured, 8 x 5120 channels x 4096 positions bf16: 806 -> 660 us; 8 x 2368 x 8086: 1235 -> 971;
+// 7 x 3184 x 192: 35 -> 24; a workgroup per CU or less and the sequence whole: 108 against 119 (2 x 4096 x 2048), the
+// kernel with the lanes along the sequence stays; cut into more segments (below) the other one serves those too.
+struct FwdCost {
+  bool serial;
+  double us;
+};
+FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
+  const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
+  const int64_t wgs = (int64_t)p.batch * p.ngroups * ((Dg + PASS_CH - 1) / PASS_CH) * nseg;
+  const double tiles = nseg > 1 ? (double)((ntiles + nseg - 1) / nseg) : 0.5 * ((p.seqlen + TILE / 2 - 1) / (TILE / 2));
+  const int64_t pairs = wgs / (2 * cus), odd = wgs - pairs * 2 * cus;
+  const double round = (10.9 * (double)pairs + (odd > cus ? 10.9 : odd > 0 ? 6.6 : 0.0)) * (p.seqlen % KI ? 1.15 : 1.0);
+  const FwdCost lanes{false, round * ((p.dstate + NB16 - 1) / NB16) * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
+  if (p.dstate != NB16 || (p.bc_const & 3) || p.a_complex || k4_mode() || p.seqlen < KI) return lanes;
+  const int64_t fives = wgs / (5 * cus), rest = (wgs - fives * 5 * cus + cus - 1) / cus;
+  const FwdCost serial{true, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + 3.4};
+  return serial.us < lanes.us ? serial : lanes;
+}
+
 // Segments of the sequence: the split with the least estimated time in us, for 16 states.  The terms were fitted to the
-// times of 1 .. 32 segments at 13 sizes (batch 1 - 8, 768 - 5120 channels, 256 - 8192 positions; within 10 % of almost
-// all).  A tile of a round of forward workgroups takes 6.4, half as much again where two share a CU; one of a round of
-// backward workgroups (one per CU) 13 per pass and a third of that for what the passes share; a round's start and end
-// 2 and 5.3.  The pass over the segments (all but one) takes 3.0 (forward) or 4.5 (backward) a tile, twice that from four
-// of its workgroups per CU on, and every segment 0.9 or 1.8 for its launch and for going through the segments before it.
-// A split has to promise 6 %.  Measured: 1536 channels x 777 positions of one sequence 50 -> 30 us forward, 133 -> 63
-// backward; from about 256 workgroups on one segment is left.
+// times of 1 .. 32 segments (forward at 45 sizes: fwd_cost; backward at 13, batch 1 - 8, 768 - 5120 channels, 256 - 8192
+// positions; within 10 % of almost all).  A tile of a round of backward workgroups (one per CU) takes 13 per pass and a
+// third of that for what the passes share, a round's start and end 5.3.  The pass over the segments (all but one) takes 3.0
+// (forward) or 4.5 (backward) a tile, twice that from four of its workgroups per CU on, and every segment 0.9 or 1.8 for
+// its launch and for going through the segments before it.  A split has to promise 6 %.  Measured: 1536 channels x 777
+// positions of one sequence 50 -> 24 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181 forward.
 constexpr int MAX_SEGMENTS = 32;
 int scan_segments(const MambaScanParams &p, bool bwd) {
   const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
   const int64_t rows = (int64_t)p.batch * p.ngroups;
-  const int64_t wgs = rows * ((Dg + PASS_CH - 1) / PASS_CH), seg_wgs = rows * ((Dg + SEG_CH - 1) / SEG_CH);
+  const int64_t seg_wgs = rows * ((Dg + SEG_CH - 1) / SEG_CH);
   if (p.a_complex || p.batch > 65535 || k4_mode() || use_mx(p)) return 1;
   const int blocks = (p.dstate + NB16 - 1) / NB16;
   int best = 1;
@@ -965,20 +976,16 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
   for (int s = 1; s <= std::min(ntiles, MAX_SEGMENTS); ++s) {
     const int per = (ntiles + s - 1) / s;
     if (s > 1 && (s - 1) * per >= ntiles) continue;  // leaves the last segment empty
-    double tiles, rounds;
+    double cost;
     if (bwd) {
       MambaScanParams q = p;
       q.nseg = s;
       int64_t rounds_passes = 1;
       const int r = bwd_passes(q, &rounds_passes);
-      tiles = 13.0 * (double)rounds_passes * (1.0 + 0.33 / r);
-      rounds = 5.3 * (double)rounds_passes / r;
+      cost = 13.0 * (double)rounds_passes * (1.0 + 0.33 / r) * blocks * per + 5.3 * (double)rounds_passes / r;
     } else {
-      const int64_t n = (wgs * s + 2 * cus - 1) / (2 * cus);
-      tiles = 6.4 * (double)n * (wgs * s > cus ? 1.47 : 1.0);
-      rounds = 2.0 * (double)n;
+      cost = fwd_cost(p, s).us;
     }
-    double cost = tiles * blocks * per + rounds;
     if (s > 1) {
       const double share = std::max(1.0, 0.52 * (double)((seg_wgs * (s - 1) + cus - 1) / cus));
       cost = 1.06 * (cost + (bwd ? 4.5 : 3.0) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
@@ -1134,6 +1141,7 @@ template <typename T, bool BWD, int BC> int dispatch_bc(const MambaScanParams &p
     // others (160 KB per CU), which is how the kernel's speed against resident waves per SIMD is measured.
     static const size_t min_lds = getenv("MAMBA_AMD_FWD_MIN_LDS") ? (size_t)atol(getenv("MAMBA_AMD_FWD_MIN_LDS")) : 0;
     const bool half = k4_mode();
+    if (fwd_cost(p, std::max(1, p.nseg)).serial) return mamba1_fwd_serial_launch(p, mode, stream);
     const size_t lds = fwd_lds(1, np, half) > min_lds ? fwd_lds(1, np, half) : min_lds;
     if (half)
       return mode == ROWS_ALIGNED ? launch(scan_fwd_kernel<T, ROWS_ALIGNED, BC, true>, p, 1, lds, stream)

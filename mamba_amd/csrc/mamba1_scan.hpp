@@ -141,6 +141,20 @@ DEVI Geo geometry(const MambaScanParams &p, int passes) {
   return q;
 }
 
+// The workspace of a sequence cut into segments (mamba1_scan.hip).
+DEVI int64_t seg_row(const MambaScanParams &p, int b, int seg, int d) { return ((int64_t)b * p.nseg + seg) * p.dim + d; }
+DEVI float *seg_sums(const MambaScanParams &p) { return p.seg_ws + (int64_t)p.batch * p.nseg * p.dim * p.dstate; }
+DEVI float *seg_firsts(const MambaScanParams &p) { return seg_sums(p) + (int64_t)p.batch * p.nseg * p.dim; }
+
+// State entering this workgroup's segment (A2 = A log2 e)
+DEVI float seg_state_in(const MambaScanParams &p, const Geo &q, int d, int n, float A2) {
+  float h = 0.f;
+  for (int s = 0; s < q.seg; ++s) {
+    const int64_t row = seg_row(p, q.b, s, d);
+    h = __builtin_fmaf(fast_exp2(A2 * seg_sums(p)[row]), h, p.seg_ws[row * p.dstate + n]);
+  }
+  return h;
+}
 // Row starts of one channel of the workgroup, kept in LDS: every (tile, pass) step needs nine
 // addresses per lane, and as kernel arguments next to the loop state they did not fit the scalar
 // registers (each step then re-read hundreds of spilled scalars through v_readlane).  Pointers read back

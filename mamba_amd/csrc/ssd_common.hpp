@@ -877,6 +877,9 @@ __attribute__((visibility("hidden"))) bool ssd_bwd_dx_fused_supported(const SsdP
 // tiled bwd_d*_state kernels).
 __attribute__((visibility("hidden"))) int ssd_bwd_dbc_fused_launch(const SsdParams *p, hipStream_t stream);
 __attribute__((visibility("hidden"))) bool ssd_bwd_dbc_fused_owns(const SsdParams *p);
+// The same kernels behind the dCB stage, writing the finished dB / dC, where _finishes says so (and dCB lies as bf16).
+__attribute__((visibility("hidden"))) bool ssd_bwd_dbc_finishes(const SsdParams *p);
+__attribute__((visibility("hidden"))) int ssd_bwd_dbc_finish_launch(const SsdParams *p, hipStream_t stream);
 // The dCB kernel that holds a chunk's whole triangle (ssd_dcb_chunk.hip), for the problems dcb_plan gives it.
 __attribute__((visibility("hidden"))) int ssd_bwd_dcb_chunk_launch(const SsdParams *p, bool lp, int nsplit, hipStream_t stream);
 

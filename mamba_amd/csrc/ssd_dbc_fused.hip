@@ -7,18 +7,22 @@
 //                                                                          chunk was entered in, else 0
 //     ddA_cumsum[h, l] += sum_n (v_h[l] sum_p g[l, h, p] H[h, p, n]) C[l, n]
 // with dS the gradient of the state a chunk hands on and H the state it was entered with.  One launch does both: half
-// of its workgroups take dC, half dB.  One workgroup of one wave
-// per 16 positions works through a list of heads of one (batch, chunk, group): a head's rows (x or g, as they lie in
-// memory) and its P x N matrix are staged in LDS, two heads deep, so that a single barrier per head separates the
-// waves' products from the next commit and the loads of the head after next are in flight meanwhile.  Wave w owns
-// positions 16 w .. 16 w + 15 and keeps their sum over the heads in registers (fp32, N / 16 tiles); the per-position
-// weight is applied to the fp32 product of each head, not to the bf16 operand.  The matrix is the B operand with
-// k = p: its fragments come from transposing LDS reads.
+// of its workgroups take dC, half dB.  A workgroup of up to 8 waves takes 16 positions per wave of a chunk (a 256 position
+// chunk is two workgroups) and a list of heads of one group.  A head's rows (x or g) and its P x N matrix go to LDS with
+// asynchronous loads, the next head's while this one's are multiplied, with one barrier per head.  Wave w owns positions 16 w
+// .. 16 w + 15 and keeps their sum over the heads in registers (fp32, N / 16 tiles); the per-position weight is applied to the
+// fp32 product of each head, not to the bf16 operand.  The matrix is the B operand with k = p: its fragments come from
+// transposing LDS reads.
 //
 // Where a workgroup's list is the whole group and the dCB stage has left its tiles in bf16, the sums start from the in-chunk
-// products (FIN), in the same registers, and leave as the finished dB / dC: the fp32 sums are neither written nor read, and
-// the stage that added the products to them is gone.  16384 positions, 128 heads in 8 groups, chunk 256: 300 us against 256
-// here and 185 there; 2 x 4096, 40 heads in 8 groups, chunk 128: 65 against 60 and 41.
+// products (FIN), in the same registers and as steps of the same pipeline, and leave as the finished dB / dC: the fp32 sums are
+// neither written nor read, and the stage that added the products to them is gone.
+//
+// What bounds it: at 2 workgroups of 8 waves per CU (128 registers a wave) the loads alone take 85 % of the time without the
+// in-chunk products, the products alone 80 %.  One workgroup of 16 waves per CU, with heads staged through registers, had
+// every wave in the same phase and spent half its time in waits.  16384 positions, 128 heads in 8 groups, chunk 256, with the
+// in-chunk products: 300 -> 256 us; 2 x 4096, 40 heads in 8 groups, chunk 128: 65 -> 44; without them, 4 x 4096, 80 heads in
+// one group: 130 -> 127 (5 TB/s through the L2).
 #include "ssd_common.hpp"
 
 namespace {
@@ -29,117 +33,145 @@ DEVI f32x4 mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4 c) {
 
 constexpr int MAXHB = 40;  // heads per workgroup at most (dbc_heads_per_workgroup never picks more)
 
-// LDS of one staged head: rows of x / g (pitch P + 8: 16-byte aligned pieces), the matrix (pitch N + 16: the
-// transposing reads of a half-wave cover all 64 banks once), the weight per position.
-template <int PT, int NK, int QT> struct DbcBuf {
-  uint16_t Rs[16 * QT * (16 * PT + 8)];
-  uint16_t Ms[16 * PT * (32 * NK + 16)];
-  float w[16 * QT];
+// One staged head, as the asynchronous loads lay it down: whole rows without padding, their 16-byte pieces permuted within the
+// row so that neither the A operand's 16-byte reads nor the transposing reads of a half-wave meet in a bank.
+template <int PT, int NK, int WV> struct DbcBuf {
+  uint16_t Rs[16 * WV * 16 * PT];  // rows of x / g
+  uint16_t Ms[16 * PT * 32 * NK];  // the matrix
+};
+constexpr int DDA_RING = 16;  // heads whose ddA_cumsum rows a wave keeps until it adds them
+
+// LDS of a workgroup: two staged heads.
+template <int PT, int NK, int WV> struct __align__(256) DbcShared {
+  DbcBuf<PT, NK, WV> first;
+  union {
+    struct {
+      DbcBuf<PT, NK, WV> second;
+      float dda[WV][DDA_RING][16];
+    };
+    uint16_t c_patch[WV][16 * (64 + 16)];  // a wave's 16 rows x 64 columns, before the second head's time and after the last's
+  };
 };
 
-// LDS of a launch: the two staged heads, and what lies in their place before the first and after the last one.
-template <int PT, int NK, int QT> union __align__(16) DbcShared {
-  static constexpr int N = 32 * NK, Q = 16 * QT, BP = N + 16, DP = Q + 16;
-  static constexpr int BR = 64;                   // rows of B staged at a time
-  DbcBuf<PT, NK, QT> buf[2];
-  uint16_t c_patch[QT][16 * (64 + 16)];          // a wave's 16 rows x 64 columns
-  uint16_t b_rows[BR * BP];                      // dC: rows of B
-  struct {
-    uint16_t dcb[64 * DP], c_rows[64 * BP];      // dB: 64 rows of dCB and of C
-  } l;
-};
+// 16 bytes per lane from base + offset (bytes) to LDS, lane after lane from `lds` on.  The compiler does not count this load:
+// async_done() before the barrier that hands the data over.
+DEVI void load_async16(const void *base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory");
+}
+DEVI void async_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // One of the two products for the workgroup's list of heads (list number `lb` of those of the launch).
 // FIN: the list is the whole group and dCB lies finished as bf16 (ssd_dcb_chunk.hip, or the tile pairs' kernel): the sums
 // start from the in-chunk products, dC[l] from sum_{s <= l} dCB[l, s] B[s] and dB[s] from sum_{l >= s} dCB[l, s] C[l], and
 // leave as the finished dB / dC in the operands' type.
-template <int PT, int NK, int QT, bool IS_C, bool DET, bool FIN>
-DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT, NK, QT> &shm, float (*dda_s)[16 * QT]) {
-  constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT, NT = 64 * QT, NTL = N / 16, KK = P / 32;
-  constexpr int XP = P + 8, BP = N + 16;
-  using Buf = DbcBuf<PT, NK, QT>;
-  Buf *const buf = shm.buf;
+template <int PT, int NK, int QT, int WV, bool IS_C, bool DET, bool FIN>
+DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, const int c, const int b, const int r0, DbcShared<PT, NK, WV> &shm) {
+  constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT, R = 16 * WV, NTL = N / 16, KK = P / 32;
   typedef __attribute__((address_space(3))) i16x4_t *lds_ptr;
   typedef short i16x8_t __attribute__((ext_vector_type(8)));
 
-  int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  int j = lane & 15, g = lane >> 4;
+  const int j = lane & 15, g = lane >> 4;
   const int H = p.nheads, G = p.ngroups, L = p.seqlen;
   // the heads of a workgroup are `per` apart: workgroups in flight together touch neighbouring heads
   const int hpg = H / G, per = hpg / hb;
   const int grp = lb / per, h_first = grp * hpg + lb % per;
-  const int c = blockIdx.y, b = blockIdx.z;
   const int t0 = c * Q;
-  const int qlim = min(Q, L - t0);
+  const int qlim = min(Q, L - t0);  // r0 < qlim: rows r0 .. r0 + R - 1 of the chunk are the workgroup's
   const float dsc = det_scale_of(p);
   const View4 gv = g_view(p);
   const bf16_t *rows_base = IS_C ? static_cast<const bf16_t *>(gv.ptr) + b * gv.bs : static_cast<const bf16_t *>(p.x) + b * p.x_bs;
   const int64_t r_ls = IS_C ? gv.ls : p.x_ls, r_hs = IS_C ? gv.hs : p.x_hs;
   const bf16_t *mats = static_cast<const bf16_t *>(IS_C ? p.states_lp : p.dstates_lp) + ((int64_t)b * p.nchunks + c) * H * P * N;
 
-  // position tid takes part: inside the sequence, and in the sequence the carried state belongs to
-  bool row_ok = false;
-  if (tid < Q) {
-    row_ok = tid < qlim;
-    if (p.seq_idx && row_ok) {
+  // which of this lane's positions l0 .. l0 + 3 take part: inside the sequence, and in the one the carried state belongs to
+  const int l0 = r0 + wave * 16 + 4 * g;
+  uint32_t rows_ok = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    bool ok = l0 + r < qlim;
+    if (p.seq_idx) {
       const int32_t *seq = p.seq_idx + (int64_t)b * L + t0;
+      const int mine = seq[min(l0 + r, qlim - 1)];
       if (IS_C) {
-        row_ok = seq[tid] == (c > 0 ? seq[-1] : 0);
+        ok = ok && mine == (c > 0 ? seq[-1] : 0);
       } else {
         const int last = seq[qlim - 1];
-        row_ok = last >= 0 && seq[tid] == last;
+        ok = ok && last >= 0 && mine == last;
       }
     }
+    rows_ok |= (uint32_t)ok << r;
   }
 
-  // ---- global -> registers -> LDS in 16-byte pieces, no branch around a load (rows past the end of the sequence
-  // re-read its last row; their weight is zero)
-  constexpr int GCH = Q * P / 8 / NT;
-  static_assert(GCH * NT * 8 == Q * P, "whole pieces per thread");
-  constexpr int HCH = (P * N / 8 + NT - 1) / NT;
-  static_assert(NT >= Q, "one position per thread");
-  u32x4 rregs[GCH], mregs[HCH];
-  float sc_a = 0.f, sc_alast = 0.f, sc_dt = 0.f;
-  auto load_head = [&](int h) {
-    const bf16_t *rr = rows_base + h * r_hs;
+  // ---- a head on its way to LDS: a wave moves 64 pieces of 16 bytes at a time.  Rows past the end of the sequence re-read
+  // its last row; their weight is zero
+  constexpr int RP = P / 8, MP = N / 8;  // pieces of a row of x / g, of the matrix
+  constexpr int RI = R * RP / 64 / WV, MI = (P * MP / 64 + WV - 1) / WV;
+  static_assert(RI * WV * 64 == R * RP, "whole instructions per wave");
+  uint32_t r_off[RI], m_off[MI];
+  // matrix rows: 32-byte units, permuted by the bits of the row that a half-wave's transposing read spans
+  auto swz_row = [](int r, int columns) { return columns == 128 ? (r & 3) | (r >> 3 & 1) << 2 : (r >> 1 & 1) | (r >> 3 & 1) << 1; };
 #pragma unroll
-    for (int q = 0; q < GCH; ++q) {
-      const int id = tid + q * NT, r = id / (P / 8), c8 = id % (P / 8);
-      rregs[q] = *(const GLOBAL_AS u32x4 *)(rr + (int64_t)(t0 + min(r, qlim - 1)) * r_ls + c8 * 8);
-    }
-    const bf16_t *mm = mats + (int64_t)h * P * N;
+  for (int q = 0; q < RI; ++q) {
+    const int id = (q * WV + wave) * 64 + lane, r = id / RP, piece = (id % RP) ^ ((r * RP >> 4) & (RP - 1));
+    r_off[q] = (uint32_t)min(r, qlim - 1 - r0) * (uint32_t)(2 * r_ls) + piece * 16;
+  }
 #pragma unroll
-    for (int q = 0; q < HCH; ++q) mregs[q] = *(const GLOBAL_AS u32x4 *)(mm + (int64_t)min(tid + q * NT, P * N / 8 - 1) * 8);
+  for (int q = 0; q < MI; ++q) {
+    const int id = (q * WV + wave) * 64 + lane, r = id / MP;
+    m_off[q] = r * (2 * N) + ((id % MP) ^ swz_row(r, N) << 1) * 16;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)&shm.first;
+  const uint32_t lds1 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)&shm.second;
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  f32x4 n_a, n_dt;
+  float n_last = 0.f;
+  const bf16_t *rows0 = rows_base + (int64_t)(t0 + r0) * r_ls;
+  auto request_head = [&](int h, uint32_t lds) {
     const float *dA = p.dA_cumsum + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-    const int pos = min(tid, Q - 1);
-    sc_a = *(const GLOBAL_AS float *)(dA + pos);
+    n_a = *(const GLOBAL_AS f32x4_any *)(dA + l0);
     if (!IS_C) {
-      sc_alast = *(const GLOBAL_AS float *)(dA + Q - 1);
-      sc_dt = *(const GLOBAL_AS float *)(p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q + pos);
+      n_last = *(const GLOBAL_AS float *)(dA + Q - 1);
+      n_dt = *(const GLOBAL_AS f32x4_any *)(p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q + l0);
     }
-  };
-  auto commit_head = [&](Buf &B) {
+    const bf16_t *rr = rows0 + h * r_hs, *mm = mats + (int64_t)h * P * N;
 #pragma unroll
-    for (int q = 0; q < GCH; ++q) {
-      const int id = tid + q * NT, r = id / (P / 8), c8 = id % (P / 8);
-      *reinterpret_cast<u32x4 *>(&B.Rs[r * XP + c8 * 8]) = rregs[q];
-    }
+    for (int q = 0; q < RI; ++q) load_async16(rr, r_off[q], lds + (q * WV + wave) * 1024);
 #pragma unroll
-    for (int q = 0; q < HCH; ++q) {
-      const int id = tid + q * NT, pp = id / (N / 8), c8 = id % (N / 8);
-      if (id < P * N / 8) *reinterpret_cast<u32x4 *>(&B.Ms[pp * BP + c8 * 8]) = mregs[q];
-    }
-    if (tid < Q) {
-      const float wv = IS_C ? fast_exp(sc_a) : fast_exp(fminf(sc_alast - sc_a, 0.f)) * sc_dt;
-      B.w[tid] = row_ok ? wv : 0.f;
-    }
+    for (int q = 0; q < MI; ++q)
+      if (P * MP / 64 % WV == 0 || q * WV + wave < P * MP / 64) load_async16(mm, m_off[q], lds + R * P * 2 + (q * WV + wave) * 1024);
   };
 
-  load_head(h_first);
+  // A step of the in-chunk products travels as a head does, P positions of the chunk in the place of P channels: for dC the
+  // workgroup's rows of dCB and P rows of B, for dB P rows of dCB (its columns are the workgroup's positions) and of C.
+  const bf16_t *dcb = FIN ? reinterpret_cast<const bf16_t *>(p.dCB) + (((int64_t)b * p.nchunks + c) * G + grp) * Q * Q : nullptr;
+  const bf16_t *other = IS_C ? static_cast<const bf16_t *>(p.B) + b * p.B_bs + grp * p.B_gs : static_cast<const bf16_t *>(p.C) + b * p.C_bs + grp * p.C_gs;
+  const int64_t other_ls = IS_C ? p.B_ls : p.C_ls;
+  auto request_step = [&](int k0, uint32_t lds) {
+    const bf16_t *rr = IS_C ? dcb + (int64_t)r0 * Q + k0 : dcb + (int64_t)k0 * Q + r0, *mm = other + (int64_t)(t0 + k0) * other_ls;
+#pragma unroll
+    for (int q = 0; q < RI; ++q) {
+      const int id = (q * WV + wave) * 64 + lane;
+      uint32_t off;
+      if (IS_C) off = (id / RP) * (2 * Q) + ((id % RP) ^ ((id / RP * RP >> 4) & (RP - 1))) * 16;
+      else off = (id / (R / 8)) * (2 * Q) + ((id % (R / 8)) ^ swz_row(id / (R / 8), R) << 1) * 16;
+      load_async16(rr, off, lds + (q * WV + wave) * 1024);
+    }
+#pragma unroll
+    for (int q = 0; q < MI; ++q) {
+      const int id = (q * WV + wave) * 64 + lane, r = id / MP;
+      const uint32_t off = (uint32_t)min(r, qlim - 1 - k0) * (uint32_t)(2 * other_ls) + ((id % MP) ^ swz_row(r, N) << 1) * 16;
+      if (P * MP / 64 % WV == 0 || q * WV + wave < P * MP / 64) load_async16(mm, off, lds + R * P * 2 + (q * WV + wave) * 1024);
+    }
+  };
+  const int k_first = IS_C ? 0 : r0, k_end = FIN ? (IS_C ? min(qlim, r0 + R) : qlim) : k_first;
+
+  if (FIN) request_step(k_first, lds0);
+  else request_head(h_first, lds0);
 
   // C at this lane's accumulator positions (rows 16 wave + 4 g + r, columns 16 nt + j): the wave's 16 rows go to
-  // LDS as they lie in memory (the staging buffers are still empty) and a transposing read hands lane (j, g) column
+  // LDS as they lie in memory and a transposing read hands lane (j, g) column
   // 16 nt + j of rows 4 g .. 4 g + 3, which is that layout; cr(nt, r) is then one half of a register.
   u32x2 crp[IS_C ? NTL : 1];
   if (IS_C) {
@@ -151,7 +183,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
 #pragma unroll
       for (int q = 0; q < 2; ++q) {  // 16 rows x 8 pieces of 8 columns
         const int id = lane + q * 64, rr = id >> 3, c8 = id & 7;
-        const u32x4 v = *(const GLOBAL_AS u32x4 *)(Cg + (int64_t)(t0 + min(wave * 16 + rr, qlim - 1)) * p.C_ls + half * 64 + c8 * 8);
+        const u32x4 v = *(const GLOBAL_AS u32x4 *)(Cg + (int64_t)(t0 + min(r0 + wave * 16 + rr, qlim - 1)) * p.C_ls + half * 64 + c8 * 8);
         *reinterpret_cast<u32x4 *>(&Cw[rr * CPP + c8 * 8]) = v;
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -166,7 +198,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    lds_barrier();  // every wave has its C values before the first head is committed over the patches
+    lds_barrier();  // every wave has its C values before other rows go where the patches are
   }
   auto cr = [&](int nt, int r) {
     const uint32_t w = (r & 2) ? crp[nt].y : crp[nt].x;
@@ -177,128 +209,84 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
 #pragma unroll
   for (int nt = 0; nt < NTL; ++nt) sum[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  if constexpr (FIN) {
-    // k slots of lane group g, in either operand: positions 4 g .. + 3 of 32, then 16 further on
-    auto frag_tr = [&](const uint16_t *rows, int pitch, int k0, int col0) {
-      const uint16_t *src = &rows[(k0 + 4 * g + (j >> 2)) * pitch + col0 + 4 * (j & 3)];
-      const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)src), hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(src + 16 * pitch));
-      return __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    };
-    const bf16_t *dcb = reinterpret_cast<const bf16_t *>(p.dCB) + (((int64_t)b * p.nchunks + c) * G + grp) * Q * Q;
-    // Rows of B (C), ROWS at a time, go through registers into LDS: the next ones are requested before the products of the
-    // ones that lie there.  Zeros past the end of the sequence (0 times what lies there would be no zero).
-    constexpr int ROWS = IS_C ? DbcShared<PT, NK, QT>::BR : 64, RC = (ROWS * (N / 8) + NT - 1) / NT;
-    u32x4 rows[RC];
-    const bf16_t *src = IS_C ? static_cast<const bf16_t *>(p.B) + b * p.B_bs + grp * p.B_gs : static_cast<const bf16_t *>(p.C) + b * p.C_bs + grp * p.C_gs;
-    const int64_t src_ls = IS_C ? p.B_ls : p.C_ls;
-    auto piece = [&](int q) { return min(tid + q * NT, ROWS * (N / 8) - 1); };
-    auto request_rows = [&](int r0) {
-#pragma unroll
-      for (int q = 0; q < RC; ++q)
-        rows[q] = *(const GLOBAL_AS u32x4 *)(src + (int64_t)(t0 + min(r0 + piece(q) / (N / 8), qlim - 1)) * src_ls + piece(q) % (N / 8) * 8);
-    };
-    auto commit_rows = [&](uint16_t *dst, int r0) {
-#pragma unroll
-      for (int q = 0; q < RC; ++q) {
-        const int r = piece(q) / (N / 8), c8 = piece(q) % (N / 8);
-        const bool live = r0 + r < qlim;
-        const u32x4 v = {live ? rows[q].x : 0u, live ? rows[q].y : 0u, live ? rows[q].z : 0u, live ? rows[q].w : 0u};
-        *reinterpret_cast<u32x4 *>(&dst[r * BP + c8 * 8]) = v;
-      }
-    };
-    if constexpr (IS_C) {
-      constexpr int KB = ROWS / 32;
-      const bf16_t *row = dcb + (int64_t)(wave * 16 + j) * Q + 4 * g;
-      u32x2 a[KB][2];  // the wave's rows of dCB: the A operand as it lies in memory
-      auto request = [&](int s0) {
-        request_rows(s0);
-#pragma unroll
-        for (int kk = 0; kk < KB; ++kk) {  // (nothing is read past the 32 positions that hold the wave's last row)
-          const uint32_t k0 = min(s0 + kk * 32, wave * 16 & ~31);
-          a[kk][0] = *(const GLOBAL_AS u32x2 *)(row + k0);
-          a[kk][1] = *(const GLOBAL_AS u32x2 *)(row + k0 + 16);
-        }
-      };
-      request(0);
+  // lane constants of the operands' reads (bytes into a staged head).  k slots of lane group g: p = 32 kk + 8 g .. + 7
+  const uint32_t a_at = (wave * 16 + j) * (2 * P), a_swz = ((j * RP >> 4) & (RP - 1)) ^ g;
+  const uint32_t m_at = R * P * 2 + (8 * g + (j >> 2)) * (2 * N) + (j & 3) * 8 + swz_row(8 * g + (j >> 2), N) * 32;
+  auto frag_tr = [&](uint32_t at, int row_bytes) {  // k slots of a 16 column unit, rows row_bytes apart
+    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(uintptr_t)at);
+    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(uintptr_t)(at + 4 * row_bytes));
+    return __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  uint32_t here = lds0, there = lds1;  // the head (or step) to work on, and the place of the one after it
+  auto swap = [&]() { const uint32_t t = here; here = there; there = t; };
+
+  if (FIN) {
+    const uint32_t t_at = (8 * g + (j >> 2)) * (2 * R) + (j & 3) * 8 + ((wave ^ swz_row(8 * g + (j >> 2), R)) * 32);
 #pragma unroll 1
-      for (int s0 = 0; s0 < qlim; s0 += ROWS) {
-        lds_barrier();
-        commit_rows(shm.b_rows, s0);
-        bf16x8_t af[KB];
+    for (int k0 = k_first; k0 < k_end; k0 += P, swap()) {
+      async_done();
+      lds_barrier();
+      if (k0 + P < k_end) request_step(k0 + P, there);
+      else request_head(h_first, there);
+      // dCB is lower triangular, as whole tiles of 64 x 64: the others hold nothing
+      const int mine = (r0 + wave * 16) >> 6;
+      if (IS_C ? (k0 >> 6) > mine : (k0 >> 6) < mine) continue;
+      bf16x8_t af[KK];
 #pragma unroll
-        for (int kk = 0; kk < KB; ++kk) af[kk] = __builtin_bit_cast(bf16x8_t, u32x4{a[kk][0].x, a[kk][0].y, a[kk][1].x, a[kk][1].y});
-        lds_barrier();
-        if (s0 + ROWS < qlim) request(s0 + ROWS);
-        // (up to the 32 positions that hold the wave's last row: dCB is zero above the diagonal there)
+      for (int kk = 0; kk < KK; ++kk) {
+        if (IS_C) {
+          af[kk] = *(__attribute__((address_space(3))) bf16x8_t *)(uintptr_t)(here + a_at + ((a_swz ^ (kk * 4)) * 16));
+        } else {
+          af[kk] = frag_tr(here + t_at + kk * (64 * R), 2 * R);
+          if (k0 + P > qlim) {  // nothing comes from rows past the end of the sequence
+            u32x4 v = __builtin_bit_cast(u32x4, af[kk]);
 #pragma unroll
-        for (int kk = 0; kk < KB; ++kk)
-          if (s0 + kk * 32 < wave * 16 + 16) {
-#pragma unroll
-            for (int nt = 0; nt < NTL; ++nt) sum[nt] = mfma_bf16(af[kk], frag_tr(shm.b_rows, BP, kk * 32, nt * 16), sum[nt]);
-          }
-      }
-    } else {
-      constexpr int DP = DbcShared<PT, NK, QT>::DP, RD = 64 * (Q / 8) / NT;
-      static_assert(RD * NT == 64 * (Q / 8), "whole pieces per thread");
-      u32x4 drows[RD];
-      auto request = [&](int l0) {
-        request_rows(l0);
-#pragma unroll
-        for (int q = 0; q < RD; ++q)  // (the tiles above the diagonal are nothing's, and neither read nor used)
-          drows[q] = *(const GLOBAL_AS u32x4 *)(dcb + (int64_t)(l0 + (tid + q * NT) / (Q / 8)) * Q + min((tid + q * NT) % (Q / 8) * 8, l0 + 56));
-      };
-      request(0);
-#pragma unroll 1
-      for (int l0 = 0; l0 < qlim; l0 += 64) {
-        lds_barrier();
-        commit_rows(shm.l.c_rows, l0);
-#pragma unroll
-        for (int q = 0; q < RD; ++q)
-          *reinterpret_cast<u32x4 *>(&shm.l.dcb[(tid + q * NT) / (Q / 8) * DP + (tid + q * NT) % (Q / 8) * 8]) = drows[q];
-        lds_barrier();
-        if (l0 + 64 < qlim) request(l0 + 64);
-        if (l0 + 64 > wave * 16) {
-#pragma unroll
-          for (int k0 = 0; k0 < 64; k0 += 32) {
-            const bf16x8_t a = frag_tr(shm.l.dcb, DP, k0, wave * 16);
-#pragma unroll
-            for (int nt = 0; nt < NTL; ++nt) sum[nt] = mfma_bf16(a, frag_tr(shm.l.c_rows, BP, k0, nt * 16), sum[nt]);
+            for (int i = 0; i < 4; ++i) {
+              const int left = qlim - (k0 + kk * 32 + 8 * g + 2 * i);
+              v[i] = left >= 2 ? v[i] : left == 1 ? v[i] & 0xffffu : 0u;
+            }
+            af[kk] = __builtin_bit_cast(bf16x8_t, v);
           }
         }
       }
+#pragma unroll
+      for (int nt = 0; nt < NTL; ++nt)
+#pragma unroll
+        for (int kk = 0; kk < KK; ++kk) sum[nt] = mfma_bf16(af[kk], frag_tr(((here + m_at) ^ (nt * 32)) + kk * (64 * N), 2 * N), sum[nt]);
     }
-    lds_barrier();  // the first head goes where these rows are
   }
-
-  commit_head(buf[0]);
-  load_head(h_first + min(1, hb - 1) * per);
-  lds_barrier();
-
+  float(*const dda)[16] = shm.dda[wave];
 #pragma unroll 1
-  for (int hh = 0; hh < hb; ++hh) {
-    // the thread's indices pass through an empty asm once per head, so that the addresses derived from them are
-    // computed where they are used instead of being carried (or spilled) across the loop over the heads
-    asm volatile("" : "+v"(tid), "+v"(lane), "+v"(j), "+v"(g));
-    Buf &B = buf[hh & 1];
+  for (int hh = 0; hh < hb; ++hh, swap()) {
+    async_done();
+    lds_barrier();  // this head is there, and nobody reads the one before it any more
+    float wv[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const float w = IS_C ? fast_exp(n_a[r]) : fast_exp(fminf(n_last - n_a[r], 0.f)) * n_dt[r];
+      wv[r] = (rows_ok >> r & 1) ? w : 0.f;
+    }
+    if (hh + 1 < hb) request_head(h_first + (hh + 1) * per, there);
+    // (formed per head: carried across the loop, the addresses and the C values in fp32 do not fit the registers)
+    uint32_t head = here + m_at;
+    asm volatile("" : "+v"(head));
+    if (IS_C) {
+#pragma unroll
+      for (int nt = 0; nt < NTL; ++nt) asm volatile("" : "+v"(crp[nt].x), "+v"(crp[nt].y));
+    }
     f32x4 acc[NTL];
 #pragma unroll
     for (int nt = 0; nt < NTL; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8_t af[KK];
 #pragma unroll
-    for (int kk = 0; kk < KK; ++kk) {
-      // k slots of lane group g: p = 32 kk + 4 g .. + 3, then 16 further on (both operands alike)
-      const uint16_t *ar = &B.Rs[(wave * 16 + j) * XP + kk * 32 + 4 * g];
-      const u32x2 a_lo = *reinterpret_cast<const u32x2 *>(ar), a_hi = *reinterpret_cast<const u32x2 *>(ar + 16);
-      const bf16x8_t af = __builtin_bit_cast(bf16x8_t, u32x4{a_lo.x, a_lo.y, a_hi.x, a_hi.y});
+    for (int kk = 0; kk < KK; ++kk)
+      af[kk] = *(__attribute__((address_space(3))) bf16x8_t *)(uintptr_t)(here + a_at + ((a_swz ^ (kk * 4)) * 16));
 #pragma unroll
-      for (int nt = 0; nt < NTL; ++nt) {
-        const uint16_t *src = &B.Ms[(kk * 32 + 4 * g + (j >> 2)) * BP + nt * 16 + 4 * (j & 3)];
-        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)src);
-        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(src + 16 * BP));
-        const bf16x8_t bfr = __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-        acc[nt] = mfma_bf16(af, bfr, acc[nt]);
-      }
+    for (int nt = 0; nt < NTL; ++nt) {
+      const uint32_t m = head ^ (nt * 32);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) acc[nt] = mfma_bf16(af[kk], frag_tr(m + kk * (64 * N), 2 * N), acc[nt]);
     }
-    const f32x4 wv = *reinterpret_cast<const f32x4 *>(&B.w[wave * 16 + 4 * g]);
     if (IS_C) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
@@ -310,7 +298,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
         rs += dpp_f<DPP_ROW_SHR + 2>(0.f, rs);
         rs += dpp_f<DPP_ROW_SHR + 4>(0.f, rs);
         rs += dpp_f<DPP_ROW_SHR + 8>(0.f, rs);
-        if (j == 15) dda_s[hh][wave * 16 + 4 * g + r] = rs;
+        if (j == 15) dda[hh % DDA_RING][4 * g + r] = rs;
       }
     }
 #pragma unroll
@@ -318,17 +306,27 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
 #pragma unroll
       for (int r = 0; r < 4; ++r) sum[nt][r] = __builtin_fmaf(acc[nt][r], wv[r], sum[nt][r]);
 
-    // the next head's operands go to the other buffer (last read one head ago, before the barrier that ended that
-    // head); the loads of the head after it follow, then the one barrier of this head
-    commit_head(buf[(hh + 1) & 1]);
-    load_head(h_first + min(hh + 2, hb - 1) * per);
-    lds_barrier();
+    // the wave's own rows of ddA_cumsum, whole rows of 16 positions at a time
+    if (IS_C && (hh % DDA_RING == DDA_RING - 1 || hh == hb - 1)) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const int h0 = hh - hh % DDA_RING, l = r0 + wave * 16 + j;
+      for (int k = g; h0 + k <= hh; k += 4) {
+        const float d = dda[k][j];
+        if (l < qlim && d != 0.f)
+          acc_add<DET ? 1 : 0>(p.ddA_cumsum, p.det_ddA_cumsum, chunk_off(p, b, h_first + (h0 + k) * per, c) + l, d, dsc);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
   }
 
   if constexpr (FIN) {
-    // ---- the finished sums leave in the operands' type, as whole 16-byte pieces of rows through a patch per wave (the
-    // staged heads are dead: the last commit went there before the last barrier, and nobody reads it)
+    // ---- the finished sums leave in the operands' type, as whole 16-byte pieces of rows through a patch per wave
     constexpr int CPP = 64 + 16;
+    lds_barrier();
     uint16_t *Cw = shm.c_patch[wave];
     bf16_t *dst = static_cast<bf16_t *>(IS_C ? p.dC : p.dB) + (IS_C ? b * p.dC_bs + grp * p.dC_gs : b * p.dB_bs + grp * p.dB_gs);
     const int64_t ls = IS_C ? p.dC_ls : p.dB_ls;
@@ -345,7 +343,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
       for (int q = 0; q < 2; ++q) {  // 16 rows x 8 pieces of 8 columns
         const int id = lane + q * 64, rr = id >> 3, c8 = id & 7;
         const u32x4 v = *reinterpret_cast<const u32x4 *>(&Cw[rr * CPP + c8 * 8]);
-        if (wave * 16 + rr < qlim) *(GLOBAL_AS u32x4 *)(dst + (int64_t)(t0 + wave * 16 + rr) * ls + half * 64 + c8 * 8) = v;
+        if (r0 + wave * 16 + rr < qlim) *(GLOBAL_AS u32x4 *)(dst + (int64_t)(t0 + r0 + wave * 16 + rr) * ls + half * 64 + c8 * 8) = v;
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -362,7 +360,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
     const bool alone = per == 1 && !DET;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int l = wave * 16 + 4 * g + r;
+      const int l = r0 + wave * 16 + 4 * g + r;
       if (l >= qlim) continue;
       const int64_t row = (((int64_t)b * L + t0 + l) * G + grp) * N + j;
       if (alone) {
@@ -374,26 +372,23 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, DbcShared<PT,
       }
     }
   }
-  if (IS_C) {
-    for (int idx = tid; idx < hb * Q; idx += NT) {
-      const int hh = idx / Q, l = idx % Q;
-      const float d = dda_s[hh][l];
-      if (l < qlim && d != 0.f)
-        acc_add<DET ? 1 : 0>(p.ddA_cumsum, p.det_ddA_cumsum, chunk_off(p, b, h_first + hh * per, c) + l, d, dsc);
-    }
-  }
 }
 
 // Both products in one launch: the first half of the workgroups along x takes dC, the second dB, each for one list
 // of heads.  With lists twice as long as a launch per product would use to fill the chip there are half as many
 // lists to add up with atomics, the two prologues run side by side, and the whole chip is busy to the end.
-template <int PT, int NK, int QT, bool DET, bool FIN>
-__global__ __launch_bounds__(64 * QT) void bwd_dbc_fused_kernel(const SsdParams p, const int hb) {
-  __shared__ DbcShared<PT, NK, QT> shm;
-  __shared__ float dda_s[MAXHB][16 * QT];  // the heads' ddA_cumsum rows of the dC product, flushed at the end
-  const int nlists = gridDim.x / 2;
-  if ((int)blockIdx.x < nlists) dbc_body<PT, NK, QT, true, DET, FIN>(p, hb, blockIdx.x, shm, dda_s);
-  else dbc_body<PT, NK, QT, false, DET, FIN>(p, hb, blockIdx.x - nlists, shm, dda_s);
+// (128 registers a wave; with 4 waves, 64 channels and 128 states LDS holds three workgroups)
+template <int PT, int NK, int QT, int WV, bool DET, bool FIN>
+__global__ __launch_bounds__(64 * WV, WV == 4 && PT * NK == 16 ? 3 : 4) void bwd_dbc_fused_kernel(const SsdParams p, const int hb) {
+  __shared__ DbcShared<PT, NK, WV> shm;
+  constexpr int PARTS = QT / WV;
+  // the parts of a chunk are eight workgroups apart: on one XCD, whose L2 hands the second one the heads' matrices
+  const int nlists = p.nheads / hb, id = blockIdx.y * gridDim.x + blockIdx.x, part = (id >> 3) % PARTS;
+  const int unit = (id >> 3) / PARTS * 8 + (id & 7), x = unit % (2 * nlists), tile = unit / (2 * nlists);
+  const int c = tile % p.nchunks, b = tile / p.nchunks, r0 = part * 16 * WV;
+  if (b >= p.batch || c * 16 * QT + r0 >= p.seqlen) return;
+  if (x < nlists) dbc_body<PT, NK, QT, WV, true, DET, FIN>(p, hb, x, c, b, r0, shm);
+  else dbc_body<PT, NK, QT, WV, false, DET, FIN>(p, hb, x - nlists, c, b, r0, shm);
 }
 
 // Heads per workgroup for that launch: a divisor of the heads per group, MAXHB at most, by the same estimate as
@@ -414,11 +409,13 @@ inline int dbc_heads_per_workgroup(const SsdParams &p) {
 
 template <int PT, int NK, bool DET, bool FIN> int launch_q(const SsdParams &p, hipStream_t s) {
   const int hb = FIN ? p.nheads / p.ngroups : dbc_heads_per_workgroup(p);
-  dim3 grid(2 * (p.nheads / hb), p.nchunks, p.batch);
+  // eight workgroups per part of a chunk side by side, a multiple of that where the other dimension would not hold the rest
+  const int64_t units = 2 * (int64_t)(p.nheads / hb) * p.nchunks * p.batch, k = (units + 8 * 65535 - 1) / (8 * 65535);
+  const int x = 8 * (int)k, y = (int)((units + x - 1) / x);
   switch (p.chunk_size) {
-    case 256: hipLaunchKernelGGL((bwd_dbc_fused_kernel<PT, NK, 16, DET, FIN>), grid, dim3(1024), 0, s, p, hb); break;
-    case 128: hipLaunchKernelGGL((bwd_dbc_fused_kernel<PT, NK, 8, DET, FIN>), grid, dim3(512), 0, s, p, hb); break;
-    case 64: hipLaunchKernelGGL((bwd_dbc_fused_kernel<PT, NK, 4, DET, FIN>), grid, dim3(256), 0, s, p, hb); break;
+    case 256: hipLaunchKernelGGL((bwd_dbc_fused_kernel<PT, NK, 16, 8, DET, FIN>), dim3(2 * x, y), dim3(512), 0, s, p, hb); break;
+    case 128: hipLaunchKernelGGL((bwd_dbc_fused_kernel<PT, NK, 8, 8, DET, FIN>), dim3(x, y), dim3(512), 0, s, p, hb); break;
+    case 64: hipLaunchKernelGGL((bwd_dbc_fused_kernel<PT, NK, 4, 4, DET, FIN>), dim3(x, y), dim3(256), 0, s, p, hb); break;
     default: return MAMBA_E_UNSUPPORTED;
   }
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
@@ -427,6 +424,9 @@ template <bool DET, bool FIN> int launch_pn(const SsdParams &p, hipStream_t s) {
   if (p.headdim == 64) return p.dstate == 128 ? launch_q<4, 4, DET, FIN>(p, s) : launch_q<4, 2, DET, FIN>(p, s);
   return p.dstate == 128 ? launch_q<2, 4, DET, FIN>(p, s) : launch_q<2, 2, DET, FIN>(p, s);
 }
+
+// rows whose places in a chunk 32-bit byte offsets reach
+bool near(int64_t ls) { return ls >= 0 && ls < (1 << 22); }
 
 bool supported(const SsdParams *p) {
   if (p->dtype != MAMBA_BF16 || !p->dstates_lp || !p->states_lp) return false;
@@ -439,6 +439,7 @@ bool supported(const SsdParams *p) {
   if (!aligned(p->x, 16) || !aligned(gptr, 16) || !aligned(p->dstates_lp, 16) || !aligned(p->states_lp, 16)) return false;
   if (p->x_bs % 8 || p->x_ls % 8 || p->x_hs % 8) return false;
   if (!p->z && (p->dout_bs % 8 || p->dout_ls % 8 || p->dout_hs % 8)) return false;
+  if (!near(p->x_ls) || (!p->z && !near(p->dout_ls)) || (p->z && !near((int64_t)p->nheads * p->headdim))) return false;
   if (p->batch > 65535 || p->nchunks > 65535) return false;
   return true;
 }
@@ -464,6 +465,6 @@ int ssd_bwd_dbc_fused_launch(const SsdParams *p, hipStream_t stream) {
 bool ssd_bwd_dbc_finishes(const SsdParams *p) {
   auto rows16 = [](const void *q, int64_t bs, int64_t ls, int64_t gs) { return q && aligned(q, 16) && bs % 8 == 0 && ls % 8 == 0 && gs % 8 == 0; };
   return ssd_bwd_dbc_fused_owns(p) && rows16(p->B, p->B_bs, p->B_ls, p->B_gs) && rows16(p->C, p->C_bs, p->C_ls, p->C_gs) &&
-         rows16(p->dB, p->dB_bs, p->dB_ls, p->dB_gs) && rows16(p->dC, p->dC_bs, p->dC_ls, p->dC_gs) && aligned(p->dCB, 16);
+         near(p->B_ls) && near(p->C_ls) && rows16(p->dB, p->dB_bs, p->dB_ls, p->dB_gs) && rows16(p->dC, p->dC_bs, p->dC_ls, p->dC_gs) && aligned(p->dCB, 16);
 }
 int ssd_bwd_dbc_finish_launch(const SsdParams *p, hipStream_t stream) { return launch_pn<false, true>(*p, stream); }

@@ -1,6 +1,7 @@
-"""dB and dC of the SSD backward pass where one launch forms them whole, state path and in-chunk products
-(ssd_dbc_fused.hip): each chunk length, state count and headdim, groups of one and of several heads, a last chunk of 1, 17
-and Q - 1 positions, packed sequences.  Reference: the quadratic form in float64 on the same bf16 operands."""
+"""dB and dC of the SSD backward pass from the state-path launch (ssd_dbc_fused.hip), where it forms them whole (state path and
+in-chunk products) and where it adds to sums that a later launch finishes: each chunk length, state count and headdim, groups
+of one and of several heads, a last chunk of 1, 17 and Q - 1 positions, packed sequences.  Reference: the quadratic form in
+float64 on the same bf16 operands."""
 import pytest
 import torch
 
@@ -29,6 +30,31 @@ def _reference(x, dt, A, B, C, g, seq):
     return [t.transpose(1, 2) for t in out]
 
 
+# The chunk states and their gradients, dCB and the result are rounded to bf16, 2^-9 of each; a state hands
+# its chunk's share on in fp32.  A sum's terms take two of these roundings, a chunk's own state sums a third
+FACTOR = 4 * 2.0 ** -9
+
+
+def _check(B, C, want):
+    for name, got, w, size in (("dB", B.grad, want[0], want[2]), ("dC", C.grad, want[1], want[3])):
+        err = (got.double() - w).abs()
+        assert bool((err <= FACTOR * size + 1e-30).all()), f"{name}: {float((err / (size + 1e-30)).max()):.3e}"
+
+
+def _inputs(b, L, H, G, P, N, packed):
+    gen = torch.Generator(device="cuda").manual_seed(L + N + H)
+    randn = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()
+    x, g = randn(b, L, H, P), randn(b, L, H, P)
+    B, C = randn(b, L, G, N).requires_grad_(), randn(b, L, G, N).requires_grad_()
+    dt = 0.1 * torch.rand(b, L, H, device="cuda", generator=gen)
+    A = -(0.1 + 5 * torch.rand(H, device="cuda", generator=gen))
+    seq = None
+    if packed:
+        ends = torch.tensor([0, L // 7, L // 7 + 1, L // 2 + 5], device="cuda")
+        seq = (torch.arange(L, device="cuda")[:, None] >= ends).sum(-1).int()[None].expand(b, L).contiguous()
+    return x.requires_grad_(), g, B, C, dt, A, seq
+
+
 @pytest.mark.parametrize("b,L,H,G,P,N,Q", [
     (1, 4033, 16, 8, 64, 128, 64), (2, 2047, 24, 8, 64, 64, 64), (2, 1041, 32, 32, 32, 128, 64), (4, 1024, 16, 8, 32, 64, 64),
     (2, 2049, 16, 16, 64, 128, 128), (2, 2048, 32, 16, 64, 64, 128), (2, 1937, 16, 8, 32, 128, 128), (4, 1151, 16, 16, 32, 64, 128),
@@ -42,22 +68,22 @@ def test_finished_dB_dC(monkeypatch, b, L, H, G, P, N, Q, packed):
     seen, real = [], lib.ssd_bwd_overwrites
     monkeypatch.setattr(_lib, "torch_ext", lambda: None)
     monkeypatch.setattr(lib, "ssd_bwd_overwrites", lambda p: seen.append(real(p)) or seen[-1])
-    gen = torch.Generator(device="cuda").manual_seed(L + Q + H)
-    randn = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()
-    x, g = randn(b, L, H, P), randn(b, L, H, P)
-    B, C = randn(b, L, G, N).requires_grad_(), randn(b, L, G, N).requires_grad_()
-    dt = 0.1 * torch.rand(b, L, H, device="cuda", generator=gen)
-    A = -(0.1 + 5 * torch.rand(H, device="cuda", generator=gen))
-    seq = None
-    if packed:
-        ends = torch.tensor([0, L // 7, L // 7 + 1, L // 2 + 5], device="cuda")
-        seq = (torch.arange(L, device="cuda")[:, None] >= ends).sum(-1).int()[None].expand(b, L).contiguous()
-    out = sc.mamba_chunk_scan_combined(x.requires_grad_(), dt, A, B, C, Q, seq_idx=seq)
-    out.backward(g)
+    x, g, B, C, dt, A, seq = _inputs(b, L, H, G, P, N, packed)
+    sc.mamba_chunk_scan_combined(x, dt, A, B, C, Q, seq_idx=seq).backward(g)
     assert seen and seen[0] & 3 == 3, f"one workgroup does not hold a group here: {seen}"
-    want = _reference(x.detach(), dt, A, B.detach(), C.detach(), g, seq)
-    for name, got, w, size in (("dB", B.grad, want[0], want[2]), ("dC", C.grad, want[1], want[3])):
-        # the chunk states and their gradients, dCB and the result are rounded to bf16, 2^-9 of each; a state hands its
-        # chunk's share on in fp32.  A sum's terms take two of these roundings, a chunk's own state sums a third
-        err = (got.double() - w).abs()
-        assert bool((err <= 4 * 2.0 ** -9 * size + 1e-30).all()), f"{name}: {float((err / (size + 1e-30)).max()):.3e}"
+    _check(B, C, _reference(x.detach(), dt, A, B.detach(), C.detach(), g, seq))
+
+
+# lists of 1, 5, 12, 16, 17 and 40 heads of larger groups, short and long last chunks
+@pytest.mark.parametrize("b,L,H,G,P,N,Q", [
+    (1, 321, 20, 1, 64, 128, 64), (2, 500, 48, 2, 32, 128, 64), (1, 145, 32, 1, 64, 128, 128), (2, 1151, 34, 1, 64, 64, 128),
+    (4, 1024, 80, 1, 64, 128, 256), (2, 897, 48, 2, 32, 128, 256), (1, 1009, 17, 1, 32, 64, 256),
+])
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_added_dB_dC(monkeypatch, b, L, H, G, P, N, Q, deterministic):
+    from mamba_amd.ops.triton import ssd_combined as sc
+    if deterministic:
+        monkeypatch.setenv("MAMBA_DETERMINISTIC", "1")
+    x, g, B, C, dt, A, seq = _inputs(b, L, H, G, P, N, True)
+    sc.mamba_chunk_scan_combined(x, dt, A, B, C, Q, seq_idx=seq).backward(g)
+    _check(B, C, _reference(x.detach(), dt, A, B.detach(), C.detach(), g, seq))

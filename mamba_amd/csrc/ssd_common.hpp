@@ -846,6 +846,19 @@ DEVI View4 g_view(const SsdParams &p) {
 }
 
 
+// 16 bytes per lane from base + offset (bytes) to LDS, lane after lane from `lds` on.  The compiler does not count this load:
+// async_done() before the barrier that hands the data over.  LEFT: vector memory operations that may still be in flight, at
+// most as many as were surely issued after the loads (they complete in order); 0 waits for everything.
+DEVI void load_async16(const void *base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory");
+}
+template <int LEFT> DEVI void async_done() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
+
+// LDS address of a shared variable, as those loads and integer arithmetic take it
+template <typename V> DEVI uint32_t lds_address(const V *v) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void *)v; }
+// rows whose places in a chunk 32-bit byte offsets reach
+inline bool near_rows(int64_t ls) { return ls >= 0 && ls < (1 << 22); }
+
 DEVI float *chunk_row(float *base, const SsdParams &p, int b, int h, int c) {
   return base + (((int64_t)b * p.nheads + h) * p.nchunks + c) * p.chunk_size;
 }

@@ -53,13 +53,6 @@ template <int PT, int NK, int WV> struct __align__(256) DbcShared {
   };
 };
 
-// 16 bytes per lane from base + offset (bytes) to LDS, lane after lane from `lds` on.  The compiler does not count this load:
-// async_done() before the barrier that hands the data over.
-DEVI void load_async16(const void *base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory");
-}
-DEVI void async_done() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
-
 // One of the two products for the workgroup's list of heads (list number `lb` of those of the launch).
 // FIN: the list is the whole group and dCB lies finished as bf16 (ssd_dcb_chunk.hip, or the tile pairs' kernel): the sums
 // start from the in-chunk products, dC[l] from sum_{s <= l} dCB[l, s] B[s] and dB[s] from sum_{l >= s} dCB[l, s] C[l], and
@@ -224,7 +217,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, const int c, 
     const uint32_t t_at = (8 * g + (j >> 2)) * (2 * R) + (j & 3) * 8 + ((wave ^ swz_row(8 * g + (j >> 2), R)) * 32);
 #pragma unroll 1
     for (int k0 = k_first; k0 < k_end; k0 += P, swap()) {
-      async_done();
+      async_done<0>();
       lds_barrier();
       if (k0 + P < k_end) request_step(k0 + P, there);
       else request_head(h_first, there);
@@ -258,7 +251,7 @@ DEVI void dbc_body(const SsdParams &p, const int hb, const int lb, const int c, 
   float(*const dda)[16] = shm.dda[wave];
 #pragma unroll 1
   for (int hh = 0; hh < hb; ++hh, swap()) {
-    async_done();
+    async_done<0>();
     lds_barrier();  // this head is there, and nobody reads the one before it any more
     float wv[4];
 #pragma unroll
@@ -425,9 +418,6 @@ template <bool DET, bool FIN> int launch_pn(const SsdParams &p, hipStream_t s) {
   return p.dstate == 128 ? launch_q<2, 4, DET, FIN>(p, s) : launch_q<2, 2, DET, FIN>(p, s);
 }
 
-// rows whose places in a chunk 32-bit byte offsets reach
-bool near(int64_t ls) { return ls >= 0 && ls < (1 << 22); }
-
 bool supported(const SsdParams *p) {
   if (p->dtype != MAMBA_BF16 || !p->dstates_lp || !p->states_lp) return false;
   if (p->headdim != 32 && p->headdim != 64) return false;
@@ -439,7 +429,7 @@ bool supported(const SsdParams *p) {
   if (!aligned(p->x, 16) || !aligned(gptr, 16) || !aligned(p->dstates_lp, 16) || !aligned(p->states_lp, 16)) return false;
   if (p->x_bs % 8 || p->x_ls % 8 || p->x_hs % 8) return false;
   if (!p->z && (p->dout_bs % 8 || p->dout_ls % 8 || p->dout_hs % 8)) return false;
-  if (!near(p->x_ls) || (!p->z && !near(p->dout_ls)) || (p->z && !near((int64_t)p->nheads * p->headdim))) return false;
+  if (!near_rows(p->x_ls) || (!p->z && !near_rows(p->dout_ls)) || (p->z && !near_rows((int64_t)p->nheads * p->headdim))) return false;
   if (p->batch > 65535 || p->nchunks > 65535) return false;
   return true;
 }
@@ -465,6 +455,6 @@ int ssd_bwd_dbc_fused_launch(const SsdParams *p, hipStream_t stream) {
 bool ssd_bwd_dbc_finishes(const SsdParams *p) {
   auto rows16 = [](const void *q, int64_t bs, int64_t ls, int64_t gs) { return q && aligned(q, 16) && bs % 8 == 0 && ls % 8 == 0 && gs % 8 == 0; };
   return ssd_bwd_dbc_fused_owns(p) && rows16(p->B, p->B_bs, p->B_ls, p->B_gs) && rows16(p->C, p->C_bs, p->C_ls, p->C_gs) &&
-         near(p->B_ls) && near(p->C_ls) && rows16(p->dB, p->dB_bs, p->dB_ls, p->dB_gs) && rows16(p->dC, p->dC_bs, p->dC_ls, p->dC_gs) && aligned(p->dCB, 16);
+         near_rows(p->B_ls) && near_rows(p->C_ls) && rows16(p->dB, p->dB_bs, p->dB_ls, p->dB_gs) && rows16(p->dC, p->dC_bs, p->dC_ls, p->dC_gs) && aligned(p->dCB, 16);
 }
 int ssd_bwd_dbc_finish_launch(const SsdParams *p, hipStream_t stream) { return launch_pn<false, true>(*p, stream); }

@@ -5,14 +5,20 @@
 //                + sum_{l >= s, same sequence} g[l, p] exp(a_l - a_s) sum_n C[l, n] B[s, n]
 //     dx[s, p]   = dt_s acc[p, s] + D_p g[s, p]
 //     ddt_out[s] += <x_s, acc_s>;  ddA_cumsum[s] -= dt_s <x_s, state part>, the same sum added at the chunk's end.
-// One workgroup of one wave per 16 positions; wave w owns the positions s of tile w and keeps their B rows in
-// registers as the B operand of both contractions.  S'[l, s] = C_l . B_s leaves the first MFMA with 4 consecutive l
-// per lane for one s, which is the B-operand layout of the second one (k = l), so the masked product never leaves
-// registers and CB is not read.  The chunk's C rows (the same for every head of the group) sit in LDS for the
-// workgroup's whole list of heads, a head's g rows and state gradient for that head; between the barrier that
-// publishes them and the one before the epilogue the waves run free.  Below the diagonal tile the decay is factored
-// as exp(a_l - a_t) exp(a_t - a_s) with a_t the first a of the l tile (both exponents <= 0): one multiply per element
-// and one exponential per lane and tile; the diagonal tile uses the exact form.
+// One workgroup of one wave per 16 positions; wave w owns the positions s of tile w.  S[l, s] = C_l . B_s is the same for
+// every head of the group: the prologue forms it once, in fp32, with the mask on it, and each wave keeps its column of tiles
+// (8 in registers; of a 256 position chunk the rest in LDS, as the lanes hold them).  S leaves its MFMA with 4 consecutive l
+// per lane for one s, which is the B-operand layout of the causal product (k = l), so the weighted product never leaves
+// registers and CB is not read.  A head's g rows and state gradient go to LDS with asynchronous loads while the head before
+// is at work, one barrier per head.  Below the diagonal the decay is factored as exp(a_l - a_t) exp(a_t - a_s) with a_t the
+// first a of the l tile (both exponents <= 0): one multiply per element and one exponential per lane and tile; the pair of
+// tiles with the diagonal uses the exact form.  x comes and dx leaves as whole pieces of rows, through a patch per wave.
+//
+// What bounds it: memory, 3.9 TB/s through g, x, the state gradients and dx at 128-byte rows (a bare pass in that order
+// reaches 4.6); of the time, the causal products are 15 %.  Forming S for every head (544 of a head's 1088 MFMAs and 57 % of
+// its LDS reads), g and the state gradient through registers between three barriers, and x in 8-byte pieces of 16 rows (a
+// quarter of the time) cost: 16384 positions, 128 heads, chunk 256: 338 -> 247 us; 4 x 4096, 80 heads, chunk 256: 186 -> 147;
+// 2 x 4096, 40 heads, chunk 128: 57 -> 41.  Requesting x a head ahead is slower (263, 152), streaming stores too (266, 164).
 #include "ssd_common.hpp"
 
 namespace {
@@ -20,30 +26,40 @@ namespace {
 DEVI f32x4 mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
-DEVI bf16x8_t ld_frag(const uint16_t *p) { return *reinterpret_cast<const bf16x8_t *>(p); }
+
+// A head as the asynchronous loads lay it down: whole rows without padding, their 16-byte pieces permuted within the row so
+// that the reads of 16 rows (state gradient) and the transposing reads of 8 rows (g) meet in no bank.
+template <int PT, int NK, int QT> struct DxHead {
+  uint16_t g[16 * QT * 16 * PT];     // g rows of the chunk
+  uint16_t ds[16 * PT * 32 * NK];    // the gradient of the state the chunk hands on, rows p
+};
+template <int PT, int NK, int QT> struct __align__(256) DxShared {
+  DxHead<PT, NK, QT> first;
+  union {
+    struct {
+      DxHead<PT, NK, QT> second;
+      uint16_t patch[QT][16 * 32];   // epilogue: a wave's 16 rows x 32 columns
+    };
+    uint16_t c_rows[16 * QT * 32 * NK];  // prologue: the chunk's C rows
+  };
+  f32x4 s_far[QT > 8 ? 40 : 1][64];  // S of the tiles that a wave's registers do not hold: 8 of waves 0 and 1, 6 of 2 and 3, ..
+  float a2[2][16 * QT], el[2][16 * QT], d[2][16 * PT];
+  f32x4 dd[2][QT / 4], da[2][QT / 4];  // a wave's shares of dD and of the chunk end's ddA
+  int seq[16 * QT];
+};
 
 template <int PT, int NK, int QT, bool DET>
-__global__ __launch_bounds__(64 * QT) void bwd_dx_fused_kernel(const SsdParams p, const int hb, const int sum_dD) {
-  constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT, NSB = Q / 32, NT = 64 * QT;
-  constexpr int BP = N + 8;   // LDS pitch of a C row / dS row (bf16): 16-byte aligned, bank-spread
-  constexpr int XP = P + 16;  // LDS pitch of a g row (one position, P values + pad), as it lies in memory
-  constexpr int YP = P + 4;   // fp32 pitch of the epilogue's per-wave transpose patch (rows 4 banks apart)
-  __shared__ __align__(16) uint16_t Cs[Q * BP];  // the chunk's C rows
-  struct Head {
-    uint16_t Gs[Q * XP];  // the head's g rows
-    uint16_t Ss[P * BP];  // the gradient of the state the chunk hands on, rows p
-  };
-  union __align__(16) Shared {
-    Head hd;                     // state product and causal loop
-    float ypatch[QT * 16 * YP];  // epilogue (g and the state gradient are dead by then)
-  };
-  __shared__ Shared shm;
-  auto &Gs = shm.hd.Gs;
-  auto &Ss = shm.hd.Ss;
-  __shared__ __align__(16) float a2_s[Q], el_s[Q], dt_s[Q], w_s[Q];
-  __shared__ int seq_s[Q];
-  __shared__ __align__(16) float d_s[P];
-  __shared__ float dd_s[QT];  // sum_dD: each wave's <g, x> of the head over its 16 positions
+__global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void bwd_dx_fused_kernel(const SsdParams p, const int hb, const int sum_dD) {
+  constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT, SR = QT > 8 ? 8 : QT;
+  constexpr int RP = P / 8, MP = N / 8;  // 16-byte pieces of a g row, of a state or C row
+  __shared__ DxShared<PT, NK, QT> shm;
+  typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
+  typedef __attribute__((address_space(3))) bf16x8_t *lds_frag;
+  typedef __attribute__((address_space(3))) u32x4 *lds_u4;
+  typedef __attribute__((address_space(3))) u32x2 *lds_u2;
+  typedef __attribute__((address_space(3))) f32x4 *lds_f4;
+  typedef __attribute__((address_space(3))) float *lds_f1;
+  typedef short i16x8_t __attribute__((ext_vector_type(8)));
 
   int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -53,278 +69,303 @@ __global__ __launch_bounds__(64 * QT) void bwd_dx_fused_kernel(const SsdParams p
   const int hpg = H / G, per = hpg / hb;
   const int grp = blockIdx.x / per, h_first = grp * hpg + blockIdx.x % per;
   const int c = blockIdx.y, b = blockIdx.z;
-  const int lt = wave, first = lt >> 1;  // this wave's s tile; the l block that holds its diagonal
+  const int lt = wave, first = lt & ~1;  // this wave's s tile; its l tiles, two at a time, from the pair that holds lt on
   const int t0 = c * Q;
   const int qlim = min(Q, L - t0);
   const bf16_t *Bg = static_cast<const bf16_t *>(p.B) + b * p.B_bs + grp * p.B_gs;
   const bf16_t *Cg = static_cast<const bf16_t *>(p.C) + b * p.C_bs + grp * p.C_gs;
-  const bool has_seq = p.seq_idx != nullptr;
   const float *Dp = static_cast<const float *>(p.D);
   const View4 gv = g_view(p);
   const float dsc = det_scale_of(p);
-
-  // ---- global -> registers -> LDS in 16-byte pieces, every piece of a tensor dealt to a thread, no branch around a
-  // load (rows past the end of the sequence re-read its last row and are zeroed at the commit)
-  constexpr int CCH = Q * N / 8 / NT, GCH = Q * P / 8 / NT;
-  static_assert(CCH * NT * 8 == Q * N && GCH * NT * 8 == Q * P, "whole pieces per thread");
-  constexpr int HCH = (P * N / 8 + NT - 1) / NT;
-  static_assert(NT >= Q && NT >= P, "one position / one channel per thread");
-  const int s_own = lt * 16 + j;           // the position this lane's column stands for
+  int s_own = lt * 16 + j;                 // the position this lane's column stands for
   const int s_row = min(s_own, qlim - 1);  // its row in memory (positions past the end are never stored)
-  u32x4 gregs[GCH], hraw[HCH];
-  u32x2 xl[PT];  // x of this lane's column s in the accumulator layout: rows p = 16 pt + 4 g .. + 3
-  float sc_a = 0.f, sc_at = 0.f, sc_alast = 0.f, sc_dt = 0.f, sc_d = 0.f;
-  bool in_last = false;  // position tid belongs to the last sequence of the chunk
-  auto load_head = [&](int h) {
-    const bf16_t *gg = static_cast<const bf16_t *>(gv.ptr) + b * gv.bs + h * gv.hs;
+
+  // ---- memory -> LDS: a wave moves 64 pieces of 16 bytes at a time; rows past the end of the sequence re-read its last row
+  auto swz_row = [](int r) { return N == 128 ? r & 15 : r >> 1 & 7; };          // C and state rows: pieces
+  auto swz_g = [](int r) { return P == 64 ? r >> 1 & 3 : r >> 2 & 1; };         // g rows: units of 32 bytes
+  constexpr int GI = RP / 4, MI = (P * MP / 64 + QT - 1) / QT, CI = MP / 4;     // instructions per wave
+  static_assert(GI * QT * 64 == Q * RP && CI * QT * 64 == Q * MP, "whole instructions per wave");
+  uint32_t g_off[GI], m_off[MI];
 #pragma unroll
-    for (int q = 0; q < GCH; ++q) {
-      const int id = tid + q * NT, r = id / (P / 8), c8 = id % (P / 8);
-      gregs[q] = *(const GLOBAL_AS u32x4 *)(gg + (int64_t)(t0 + min(r, qlim - 1)) * gv.ls + c8 * 8);
-    }
-    const bf16_t *dS = static_cast<const bf16_t *>(p.dstates_lp) + (((int64_t)b * p.nchunks + c) * H + h) * P * N;
+  for (int q = 0; q < GI; ++q) {
+    const int id = (q * QT + wave) * 64 + lane, r = id / RP;
+    g_off[q] = (uint32_t)min(r, qlim - 1) * (uint32_t)(2 * gv.ls) + ((id % RP) ^ swz_g(r) << 1) * 16;
+  }
 #pragma unroll
-    for (int q = 0; q < HCH; ++q)
-      hraw[q] = *(const GLOBAL_AS u32x4 *)(dS + (int64_t)min(tid + q * NT, P * N / 8 - 1) * 8);
-    const float *dA = p.dA_cumsum + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-    const float *dt = p.dt_out + (((int64_t)b * H + h) * p.nchunks + c) * Q;
-    const int pos = min(tid, Q - 1);
-    sc_a = *(const GLOBAL_AS float *)(dA + pos);
-    sc_at = *(const GLOBAL_AS float *)(dA + (pos & ~15));
-    sc_alast = *(const GLOBAL_AS float *)(dA + Q - 1);
-    sc_dt = *(const GLOBAL_AS float *)(dt + pos);
-    const float *dsrc = Dp ? Dp + (p.D_has_hdim ? h * P + min(tid, P - 1) : h) : dA;  // any valid address without D
-    sc_d = *(const GLOBAL_AS float *)dsrc;
-    const bf16_t *xcol = static_cast<const bf16_t *>(p.x) + b * p.x_bs + h * p.x_hs + (int64_t)(t0 + s_row) * p.x_ls + 4 * g;
+  for (int q = 0; q < MI; ++q) {
+    const int id = (q * QT + wave) * 64 + lane, r = id / MP;
+    m_off[q] = r * (2 * N) + ((id % MP) ^ swz_row(r)) * 16;
+  }
+  constexpr uint32_t DS = Q * P * 2;  // bytes from a head's g rows to its state gradient
+  const uint32_t lds0 = lds_address(&shm.first), lds1 = lds_address(&shm.second);
+  // a head's tensors: uniform pointers that move on by `per` heads, and 32-bit offsets from them
+  typedef const GLOBAL_AS char *gptr;
+  const int64_t row0 = (((int64_t)b * H + h_first) * p.nchunks + c) * Q, row_step = (int64_t)per * p.nchunks * Q;
+  gptr g_at_head = (gptr)(static_cast<const bf16_t *>(gv.ptr) + b * gv.bs + (int64_t)t0 * gv.ls + h_first * gv.hs);
+  gptr ds_at_head = (gptr)(static_cast<const bf16_t *>(p.dstates_lp) + (((int64_t)b * p.nchunks + c) * H + h_first) * P * N);
+  gptr x_at_head = (gptr)(static_cast<const bf16_t *>(p.x) + b * p.x_bs + h_first * p.x_hs + (int64_t)t0 * p.x_ls);
+  gptr a_at_head = (gptr)(p.dA_cumsum + row0), dt_at_head = (gptr)(p.dt_out + row0);
+  gptr d_at_head = Dp ? (gptr)(Dp + (p.D_has_hdim ? h_first * P : h_first)) : a_at_head;  // any valid address without D
+  const int64_t g_step = 2 * per * gv.hs, ds_step = (int64_t)per * P * N * 2, x_step = 2 * per * p.x_hs;
+  const int64_t d_step = Dp ? (int64_t)per * 4 * (p.D_has_hdim ? P : 1) : 0;
+  GLOBAL_AS char *dx_at_head = (GLOBAL_AS char *)(static_cast<bf16_t *>(p.dx) + b * p.dx_bs + h_first * p.dx_hs + (int64_t)(t0 + lt * 16) * p.dx_ls);
+  const int64_t dx_step = 2 * per * p.dx_hs;
+  // x of the wave's 16 positions, 32 columns per load, as whole pieces of rows
+  u32x4 xr[PT / 2];
+  auto request_x = [&]() {
+    const uint32_t x_off = (uint32_t)min(lt * 16 + (lane >> 2), qlim - 1) * (uint32_t)(2 * p.x_ls) + (lane & 3) * 16;
 #pragma unroll
-    for (int pt = 0; pt < PT; ++pt) xl[pt] = *(const GLOBAL_AS u32x2 *)(xcol + pt * 16);
+    for (int e = 0; e < PT / 2; ++e) xr[e] = *(const GLOBAL_AS u32x4 *)(x_at_head + x_off + e * 64);
   };
-  auto commit_head = [&]() {
-#pragma unroll
-    for (int q = 0; q < GCH; ++q) {
-      const int id = tid + q * NT, r = id / (P / 8), c8 = id % (P / 8);
-      const bool live = r < qlim;
-      const u32x4 v = {live ? gregs[q].x : 0u, live ? gregs[q].y : 0u, live ? gregs[q].z : 0u, live ? gregs[q].w : 0u};
-      *reinterpret_cast<u32x4 *>(&Gs[r * XP + c8 * 8]) = v;
-    }
-#pragma unroll
-    for (int q = 0; q < HCH; ++q) {
-      const int id = tid + q * NT, pp = id / (N / 8), c8 = id % (N / 8);
-      if (id < P * N / 8) *reinterpret_cast<u32x4 *>(&Ss[pp * BP + c8 * 8]) = hraw[q];
-    }
-    if (tid < Q) {
-      a2_s[tid] = sc_a * kLog2e;
-      el_s[tid] = fast_exp(fminf(sc_a - sc_at, 0.f));
-      dt_s[tid] = sc_dt;
-      w_s[tid] = in_last ? fast_exp(fminf(sc_alast - sc_a, 0.f)) : 0.f;
-    }
-    if (tid < P) d_s[tid] = Dp ? sc_d : 0.f;
+  float n_a, n_dt, n_d;
+  auto request_scalars = [&]() {
+    n_a = *(const GLOBAL_AS float *)(a_at_head + (uint32_t)min(tid, Q - 1) * 4u);
+    n_dt = *(const GLOBAL_AS float *)(dt_at_head + (uint32_t)s_own * 4u);
+    n_d = *(const GLOBAL_AS float *)(d_at_head + (Dp && p.D_has_hdim ? (uint32_t)min(tid, P - 1) * 4u : 0u));
   };
-  // G^T fragment of p tile pt for l block sb: lane (j, g) gets row p = 16 pt + j and the k slots of lane group g,
-  // which are positions 4 g .. 4 g + 3 of the block's first 16-tile, then of its second: the layout in which the
-  // first MFMA leaves the masked product.  Each half is one transposing load of a 4 x 16 patch.
-  auto g_frag = [&](int sb, int pt) {
-    typedef __attribute__((address_space(3))) i16x4_t *lds_ptr;
-    typedef short i16x8_t __attribute__((ext_vector_type(8)));
-    const uint16_t *src = &Gs[(sb * 32 + 4 * g + (j >> 2)) * XP + pt * 16 + 4 * (j & 3)];
-    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)src);
-    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ptr)(src + 16 * XP));
-    return __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  auto request_head = [&](uint32_t lds) {
+#pragma unroll
+    for (int q = 0; q < GI; ++q) load_async16((const void *)g_at_head, g_off[q], lds + (q * QT + wave) * 1024);
+#pragma unroll
+    for (int q = 0; q < MI; ++q)
+      if (P * MP / 64 % QT == 0 || q * QT + wave < P * MP / 64) load_async16((const void *)ds_at_head, m_off[q], lds + DS + (q * QT + wave) * 1024);
   };
 
-  // ---- prologue: every global load is issued before anything waits
-  load_head(h_first);
+  // ---- prologue: S[l, s] = C_l . B_s for the group, kept in fp32 for all its heads; zero where l < s, where the sequences
+  // differ and past the end of the sequence
+  request_scalars();
+  request_head(lds0);
+#pragma unroll
+  for (int q = 0; q < CI; ++q) {
+    const int id = (q * QT + wave) * 64 + lane, r = id / MP;
+    load_async16(Cg + (int64_t)t0 * p.C_ls, (uint32_t)min(r, qlim - 1) * (uint32_t)(2 * p.C_ls) + ((id % MP) ^ swz_row(r)) * 16, lds1 + (q * QT + wave) * 1024);
+  }
   bf16x8_t Bf[NK];  // B rows of this wave's s tile: B operand of both contractions (col s = j, k = n)
 #pragma unroll
   for (int kk = 0; kk < NK; ++kk)
     Bf[kk] = __builtin_bit_cast(bf16x8_t, *(const GLOBAL_AS u32x4 *)(Bg + (int64_t)(t0 + s_row) * p.B_ls + kk * 32 + g * 8));
-  {
-    u32x4 craw[CCH];
-#pragma unroll
-    for (int q = 0; q < CCH; ++q) {
-      const int id = tid + q * NT, r = id / (N / 8), c8 = id % (N / 8);
-      craw[q] = *(const GLOBAL_AS u32x4 *)(Cg + (int64_t)(t0 + min(r, qlim - 1)) * p.C_ls + c8 * 8);
-    }
-    if (tid < Q) {
-      bool ok = tid < qlim;
-      int id = 0;
-      if (has_seq) {
-        const int32_t *seq = p.seq_idx + (int64_t)b * L + t0;
-        id = tid < qlim ? seq[tid] : -2;
-        const int lastid = seq[qlim - 1];
-        ok = ok && lastid >= 0 && id == lastid;
-      }
-      seq_s[tid] = id;
-      in_last = ok;
-    }
-#pragma unroll
-    for (int q = 0; q < CCH; ++q) {
-      const int id = tid + q * NT, r = id / (N / 8), c8 = id % (N / 8);
-      const bool live = r < qlim;
-      const u32x4 v = {live ? craw[q].x : 0u, live ? craw[q].y : 0u, live ? craw[q].z : 0u, live ? craw[q].w : 0u};
-      *reinterpret_cast<u32x4 *>(&Cs[r * BP + c8 * 8]) = v;
-    }
+  bool own_last = s_own < qlim;  // the position belongs to the last sequence of the chunk
+  if (tid < Q) {
+    int id = tid < qlim ? 0 : -2;
+    if (p.seq_idx && tid < qlim) id = p.seq_idx[(int64_t)b * L + t0 + tid];
+    shm.seq[tid] = id;
   }
+  async_done<0>();
+  lds_barrier();
+#pragma unroll
+  for (int kk = 0; kk < NK; ++kk) asm volatile("" : "+v"(Bf[kk]));  // (there: no wait for them inside the loop)
+  const int sid = shm.seq[s_own];
+  if (p.seq_idx) own_last = own_last && sid >= 0 && sid == shm.seq[qlim - 1];
+  auto row_piece = [&](int kk) { return j * (2 * N) + ((swz_row(j) ^ g ^ (kk * 4)) * 16); };  // of the rows 16 i + j, in bytes
+  auto s_tile = [&](int ltp) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) v = mfma_bf16(*(lds_frag)(uintptr_t)(lds1 + ltp * (32 * N) + row_piece(kk)), Bf[kk], v);
+    const int l0 = ltp * 16 + 4 * g;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) v[r] = l0 + r >= s_own && shm.seq[l0 + r] == sid && l0 + r < qlim ? v[r] : 0.f;
+    return v;
+  };
+  f32x4 S[SR], *const far = shm.s_far[QT > 8 ? (lt >> 1) * (18 - 2 * (lt >> 1)) + (lt & 1) * (8 - first) : 0];  // (waves 0 .. 7 only)
+#pragma unroll
+  for (int k = 0; k < SR; ++k) S[k] = first + k < QT ? s_tile(first + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int ltp = first + SR; ltp < QT; ++ltp) far[(ltp - first - SR) * 64 + lane] = s_tile(ltp);
 
-  constexpr int EQ = 16 * P / 8 / 64;  // 16-byte pieces per lane of one 16 x P tile
-  static_assert(EQ * 64 * 8 == 16 * P, "whole pieces per lane");
-  float *Ys = shm.ypatch + wave * 16 * YP;
+  // the waves' shares of a head, in a fixed order (by the wave with the shortest walk)
+  auto add_shares = [&](int which, int h) {
+    float dd = 0.f, da = 0.f;
+#pragma unroll
+    for (int w = 0; w < QT / 4; ++w) {
+      const f32x4 a = shm.da[which][w], d = shm.dd[which][w];
+      da += a[0], da += a[1], da += a[2], da += a[3];
+      dd += d[0], dd += d[1], dd += d[2], dd += d[3];
+    }
+    acc_add<DET ? 1 : 0>(p.ddA_cumsum, p.det_ddA_cumsum, chunk_off(p, b, h, c) + Q - 1, da, dsc);
+    if (sum_dD) acc_add<DET ? 1 : 0>(p.dD, p.det_dD, h, dd, dsc);
+  };
 
+  uint32_t here = lds0, there = lds1;  // the head at work and the place of the one after it
 #pragma unroll 1
   for (int hh = 0; hh < hb; ++hh) {
-    const int h = h_first + hh * per;
-    // the thread's indices pass through an empty asm once per head, so that the addresses derived from them are
-    // computed where they are used instead of being carried (or spilled) across the loop over the heads
-    asm volatile("" : "+v"(tid), "+v"(lane), "+v"(j), "+v"(g));
-    commit_head();
-    lds_barrier();
-
-    f32x4 acc[PT];
-    // ---- carried-state part: acc[p, s] = w_s sum_n dS[p, n] B[s, n]
-    {
-      const float w = w_s[s_own];
+    const int h = h_first + hh * per, odd = hh & 1;
+    // the thread's index passes through an empty asm once per head, so that what derives from it is computed where it is
+    // used instead of being carried (or spilled) across the loop over the heads
+    asm volatile("" : "+v"(tid));
+    lane = tid & 63, j = lane & 15, g = lane >> 4, s_own = lt * 16 + j;
+    // This head's operands are there once no more is in flight than what followed them, in order: at a full chunk two
+    // adds and PT / 2 stores of the head before (more in some waves).
+    if (qlim == Q && !DET) async_done<2 + PT / 2>();
+    else async_done<0>();
+    if (qlim < Q) {  // g is zero past the end of the sequence
 #pragma unroll
-      for (int pt = 0; pt < PT; ++pt) {
-        f32x4 v = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < NK; ++kk) v = mfma_bf16(ld_frag(&Ss[(pt * 16 + j) * BP + kk * 32 + g * 8]), Bf[kk], v);
-        acc[pt] = v * w;
+      for (int q = 0; q < GI; ++q) {
+        const int id = (q * QT + wave) * 64 + lane;
+        if (id / RP >= qlim) *(lds_u4)(uintptr_t)(here + id * 16) = u32x4{0u, 0u, 0u, 0u};
       }
     }
-    // <x_s, a_s>: over this lane's rows, then over the four lane groups of the column
-    auto x_dot = [&](const f32x4 (&a)[PT]) {
-      float q = 0.f;
-#pragma unroll
-      for (int pt = 0; pt < PT; ++pt) {
-        q = __builtin_fmaf(bf16_lo(xl[pt].x), a[pt][0], q);
-        q = __builtin_fmaf(bf16_hi(xl[pt].x), a[pt][1], q);
-        q = __builtin_fmaf(bf16_lo(xl[pt].y), a[pt][2], q);
-        q = __builtin_fmaf(bf16_hi(xl[pt].y), a[pt][3], q);
-      }
-      q += __shfl_xor(q, 16, 64);
-      q += __shfl_xor(q, 32, 64);
-      return q;
-    };
-    const float q1 = x_dot(acc);
+    if (tid < Q) {
+      shm.a2[odd][tid] = n_a * kLog2e;
+      shm.el[odd][tid] = fast_exp(fminf(n_a - __shfl(n_a, lane & 48, 64), 0.f));
+    }
+    if (tid < P) shm.d[odd][tid] = Dp ? n_d : 0.f;
+    const float dts = n_dt;
+    lds_barrier();  // this head is there, and nobody reads the one before it any more
+    if (wave == QT - 1 && lane == 0 && hh > 0) add_shares(odd ^ 1, h - per);
+    request_x();
+    // (the scalars always, after the last head its own once more: the compiler, which does not see the asynchronous loads,
+    // then counts the same loads behind x on either way, and its wait for x does not drain those of the next head)
+    const bool more = hh + 1 < hb;
+    g_at_head += g_step, ds_at_head += ds_step, x_at_head += x_step;
+    a_at_head += more ? row_step * 4 : 0, dt_at_head += more ? row_step * 4 : 0, d_at_head += more ? d_step : 0;
+    request_scalars();
+    if (more) request_head(there);
 
-    u32x4 ge[EQ];
-
-    // ---- inside the chunk: the l blocks from the one that holds the wave's diagonal on
-    const float as2 = a2_s[s_own];
-    const int sid = seq_s[s_own];
+    f32x4 acc[PT];
 #pragma unroll
-    for (int sb = 0; sb < NSB; ++sb) {
-      if (sb < first) continue;
+    for (int pt = 0; pt < PT; ++pt) acc[pt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const float *a2 = shm.a2[odd];
+    const float as2 = a2[s_own];
+    // G^T fragment of p tile pt for two l tiles: lane (j, g) gets row p = 16 pt + j and the k slots of lane group g,
+    // which are positions 4 g .. 4 g + 3 of the first tile, then of the second: the layout in which S lies.
+    // Each half is one transposing load of a 4 x 16 patch.
+    const uint32_t g_at = here + (4 * g + (j >> 2)) * (2 * P) + (j & 3) * 8 + swz_g(4 * g + (j >> 2)) * 32 + first * (32 * P);
+    const uint32_t el_at = lds_address(&shm.el[odd][4 * g]) + first * 64, a2_at = lds_address(a2) + first * 64;
+
+    // ---- inside the chunk: two l tiles, first + k and the next, with S of both.  The pair that holds the diagonal takes the
+    // exact decay, exp(a_l - a_s); S is zero above it
+    auto block = [&](const int k, const f32x4 (&Sk)[2], const bool diagonal) {
       float m[8];
 #pragma unroll
-      for (int h2 = 0; h2 < 2; ++h2) {
-        const int ltp = 2 * sb + h2;  // l tile
-        if (ltp < lt) {
+      for (int i = 0; i < 2; ++i) {
+        if (diagonal) {
+          const f32x4 al = *(lds_f4)(uintptr_t)(a2_at + 16 * g + (k + i) * 64);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) m[h2 * 4 + r] = 0.f;
-          continue;
-        }
-        f32x4 S = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kk = 0; kk < NK; ++kk) S = mfma_bf16(ld_frag(&Cs[(ltp * 16 + j) * BP + kk * 32 + g * 8]), Bf[kk], S);
-        const int l0 = ltp * 16 + 4 * g;
-        if (ltp > lt) {
-          const float cs = fast_exp2(fminf(a2_s[ltp * 16] - as2, 0.f));
-          const f32x4 el = *reinterpret_cast<const f32x4 *>(&el_s[l0]);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) m[h2 * 4 + r] = S[r] * el[r] * cs;
+          for (int r = 0; r < 4; ++r) m[4 * i + r] = Sk[i][r] * fast_exp2(fminf(al[r] - as2, 0.f));
         } else {
+          const f32x4 el = *(lds_f4)(uintptr_t)(el_at + (k + i) * 64);
+          const float cs = fast_exp2(fminf(*(lds_f1)(uintptr_t)(a2_at + (k + i) * 64) - as2, 0.f));
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            m[h2 * 4 + r] = l0 + r >= s_own ? S[r] * fast_exp2(fminf(a2_s[l0 + r] - as2, 0.f)) : 0.f;
-        }
-        if (has_seq) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (seq_s[l0 + r] != sid) m[h2 * 4 + r] = 0.f;
+          for (int r = 0; r < 4; ++r) m[4 * i + r] = Sk[i][r] * el[r] * cs;
         }
       }
       const u32x4 mp = {pack_bf16(m[0], m[1]), pack_bf16(m[2], m[3]), pack_bf16(m[4], m[5]), pack_bf16(m[6], m[7])};
       const bf16x8_t Mf = __builtin_bit_cast(bf16x8_t, mp);
 #pragma unroll
-      for (int pt = 0; pt < PT; ++pt) acc[pt] = mfma_bf16(g_frag(sb, pt), Mf, acc[pt]);
+      for (int pt = 0; pt < PT; ++pt) {
+        const uint32_t src = (g_at ^ (pt * 32)) + k * (32 * P);
+        const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)src);
+        const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)(src + 32 * P));
+        acc[pt] = mfma_bf16(__builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)), Mf, acc[pt]);
+      }
+    };
+#pragma unroll
+    for (int k = 0; k < SR; k += 2)
+      if (first + k < QT) block(k, {S[k], S[k + 1]}, k == 0);
+    if constexpr (QT > 8) {
+#pragma unroll 1
+      for (int k = SR; first + k < QT; k += 2) block(k, {far[(k - SR) * 64 + lane], far[(k - SR + 1) * 64 + lane]}, false);
     }
 
-    // ---- ddt and the chunk-state terms of ddA, from the accumulator layout
-    const int64_t row_off = (((int64_t)b * H + h) * p.nchunks + c) * Q;
+    // The wave's patch: 16 rows x 32 columns, 16-byte pieces permuted with the row; between whole rows (lane = 4 row + piece)
+    // and the accumulator layout (row j, columns 16 k + 4 g .. + 3)
+    const int rr = lane >> 2, piece = lane & 3;
+    const uint32_t y_at = lds_address(&shm.patch[wave][0]), y_row = y_at + rr * 64 + ((piece ^ (rr >> 1 & 3)) * 16);
+    auto y_acc = [&](int k) { return y_at + j * 64 + (((2 * k + (g >> 1)) ^ (j >> 1 & 3)) * 16) + (g & 1) * 8; };
+    auto wave_sync = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    u32x2 xl[PT];  // x of this lane's column s in the accumulator layout: rows p = 16 pt + 4 g .. + 3
+#pragma unroll
+    for (int e = 0; e < PT / 2; ++e) {
+      *(lds_u4)(uintptr_t)y_row = xr[e];
+      wave_sync();
+#pragma unroll
+      for (int k = 0; k < 2; ++k) xl[2 * e + k] = *(lds_u2)(uintptr_t)y_acc(k);
+      wave_sync();
+    }
+
+    // ---- carried-state part, and the products with x: q1 of that part, q2 of the whole
+    float q1 = 0.f, q2 = 0.f;
     {
-      const float dts = dt_s[s_own];
+      const float w = own_last ? fast_exp2(fminf(a2[Q - 1] - as2, 0.f)) : 0.f;
+#pragma unroll
+      for (int pt = 0; pt < PT; ++pt) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk)
+          v = mfma_bf16(*(lds_frag)(uintptr_t)(here + DS + pt * (32 * N) + row_piece(kk)), Bf[kk], v);
+        const float xf[4] = {bf16_lo(xl[pt].x), bf16_hi(xl[pt].x), bf16_lo(xl[pt].y), bf16_hi(xl[pt].y)};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          acc[pt][r] = __builtin_fmaf(v[r], w, acc[pt][r]);
+          q1 = __builtin_fmaf(xf[r], v[r], q1);
+          q2 = __builtin_fmaf(xf[r], acc[pt][r], q2);
+        }
+      }
+      q1 *= w;
+      q1 += __shfl_xor(q1, 16, 64);
+      q1 += __shfl_xor(q1, 32, 64);
+      q2 += __shfl_xor(q2, 16, 64);
+      q2 += __shfl_xor(q2, 32, 64);
+    }
+    asm volatile("" : "+v"(n_a), "+v"(n_dt), "+v"(n_d));  // (waited for before the adds and stores, not behind them)
+    // ---- ddt and the chunk-state terms of ddA, from the accumulator layout
+    {
+      const int64_t row_off = (((int64_t)b * H + h) * p.nchunks + c) * Q;
       const bool live = g == 0 && s_own < qlim;
-      const float q2 = x_dot(acc);
       if (live) {
         acc_add<DET ? 1 : 0>(p.ddt_out, p.det_ddt_out, row_off + s_own, q2, dsc);
         acc_add<DET ? 1 : 0>(p.ddA_cumsum, p.det_ddA_cumsum, row_off + s_own, -dts * q1, dsc);
       }
-      const float e = wave_sum_to_last(live ? dts * q1 : 0.f);  // ... and + at the chunk end: one add per wave
-      if (lane == 63) acc_add<DET ? 1 : 0>(p.ddA_cumsum, p.det_ddA_cumsum, row_off + Q - 1, e, dsc);
+      const float e = wave_sum_to_last(live ? dts * q1 : 0.f);  // ... and + at the chunk end, one add for all waves
+      if (lane == 63) reinterpret_cast<float *>(shm.da[odd])[wave] = e;
     }
 
-    // ---- dD[h] += sum_{s, p} g[s, p] x[s, p] (a D per head and no gate: g is dout): x in this lane's registers,
-    // g of the same column and rows from the head's rows in LDS (zero past the end of the sequence)
-    if (sum_dD) {
-      float dd = 0.f;
+    // ---- dx = dt acc + D g, 32 columns at a time through the wave's patch, so that they leave as 16-byte pieces of rows
+    // (the accumulator layout itself holds 8-byte pieces); dD[h] += sum_{s, p} g[s, p] x[s, p] where it is wanted (a D per
+    // head and no gate: g is dout)
+    float dd = 0.f;
+    const uint32_t own_at = here + s_own * (2 * P) + g * 8 + swz_g(s_own) * 32;
 #pragma unroll
-      for (int pt = 0; pt < PT; ++pt) {
-        const u32x2 gw = *reinterpret_cast<const u32x2 *>(&Gs[s_own * XP + pt * 16 + 4 * g]);
-        dd = __builtin_fmaf(bf16_lo(xl[pt].x), bf16_lo(gw.x), dd);
-        dd = __builtin_fmaf(bf16_hi(xl[pt].x), bf16_hi(gw.x), dd);
-        dd = __builtin_fmaf(bf16_lo(xl[pt].y), bf16_lo(gw.y), dd);
-        dd = __builtin_fmaf(bf16_hi(xl[pt].y), bf16_hi(gw.y), dd);
-      }
-      dd = wave_sum_to_last(dd);
-      if (lane == 63) dd_s[wave] = dd;
-    }
-
-    // ---- each wave requests the next head's operands as it leaves the loop; the epilogue's patches lie over g and
-    // the state gradient, so it starts once every wave has left
-    if (hh + 1 < hb) load_head(h + per);
-    // the epilogue's g rows (for D) come from the head's rows in LDS, before the patches overlay them
+    for (int e = 0; e < PT / 2; ++e) {
 #pragma unroll
-    for (int q = 0; q < EQ; ++q) {
-      const int id = lane + q * 64, rr = id / (P / 8), c8 = id % (P / 8);
-      ge[q] = *reinterpret_cast<const u32x4 *>(&Gs[(lt * 16 + rr) * XP + c8 * 8]);
-    }
-    lds_barrier();
-    if (sum_dD && tid == 0) {  // every wave's part is in (added in a fixed order); the next head's follow two barriers on
-      float dd = 0.f;
+      for (int k = 0; k < 2; ++k) {
+        const int pt = 2 * e + k;
+        f32x4 v = acc[pt] * dts;
+        if (Dp || sum_dD) {
+          const u32x2 gw = *(lds_u2)(uintptr_t)(own_at ^ (pt * 32));
+          const f32x4 gf = {bf16_lo(gw.x), bf16_hi(gw.x), bf16_lo(gw.y), bf16_hi(gw.y)};
+          const f32x4 D4 = *reinterpret_cast<const f32x4 *>(&shm.d[odd][p.D_has_hdim ? pt * 16 + 4 * g : 0]);
 #pragma unroll
-      for (int w = 0; w < QT; ++w) dd += dd_s[w];
-      acc_add<DET ? 1 : 0>(p.dD, p.det_dD, h, dd, dsc);
-    }
-    {
-      bf16_t *dxg = static_cast<bf16_t *>(p.dx) + b * p.dx_bs + h * p.dx_hs + (int64_t)(t0 + lt * 16) * p.dx_ls;
-#pragma unroll
-      for (int pt = 0; pt < PT; ++pt) *reinterpret_cast<f32x4 *>(&Ys[j * YP + pt * 16 + 4 * g]) = acc[pt];
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#pragma unroll
-      for (int q = 0; q < EQ; ++q) {  // 16 rows x P/8 pieces of 8 columns
-        const int id = lane + q * 64, rr = id / (P / 8), c8 = id % (P / 8);
-        if (lt * 16 + rr >= qlim) continue;
-        const f32x4 y0 = *reinterpret_cast<const f32x4 *>(&Ys[rr * YP + c8 * 8]);
-        const f32x4 y1 = *reinterpret_cast<const f32x4 *>(&Ys[rr * YP + c8 * 8 + 4]);
-        const float dts = dt_s[lt * 16 + rr];
-        float v[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= dts;
-        if (Dp) {
-          const u32x4 gw = ge[q];
-          const float gf[8] = {bf16_lo(gw.x), bf16_hi(gw.x), bf16_lo(gw.y), bf16_hi(gw.y),
-                               bf16_lo(gw.z), bf16_hi(gw.z), bf16_lo(gw.w), bf16_hi(gw.w)};
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] = __builtin_fmaf(d_s[c8 * 8 + e], gf[e], v[e]);
+          for (int r = 0; r < 4; ++r) v[r] = __builtin_fmaf(D4[r], gf[r], v[r]);
+          if (sum_dD) {
+            dd = __builtin_fmaf(bf16_lo(xl[pt].x), gf[0], dd);
+            dd = __builtin_fmaf(bf16_hi(xl[pt].x), gf[1], dd);
+            dd = __builtin_fmaf(bf16_lo(xl[pt].y), gf[2], dd);
+            dd = __builtin_fmaf(bf16_hi(xl[pt].y), gf[3], dd);
+          }
         }
-        st8<bf16_t>(dxg + (int64_t)rr * p.dx_ls + c8 * 8, v);
+        *(lds_u2)(uintptr_t)y_acc(k) = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
       }
+      wave_sync();
+      const u32x4 out = *(lds_u4)(uintptr_t)y_row;
+      if (lt * 16 + rr < qlim) *(GLOBAL_AS u32x4 *)(dx_at_head + (uint32_t)rr * (uint32_t)(2 * p.dx_ls) + piece * 16 + e * 64) = out;
+      wave_sync();
     }
-    lds_barrier();  // the next head's operands overwrite the patches
+    if (sum_dD) {
+      dd = wave_sum_to_last(dd);
+      if (lane == 63) reinterpret_cast<float *>(shm.dd[odd])[wave] = dd;
+    }
+    dx_at_head += dx_step;
+    const uint32_t t = here;
+    here = there;
+    there = t;
   }
+  lds_barrier();
+  if (wave == QT - 1 && lane == 0) add_shares((hb - 1) & 1, h_first + (hb - 1) * per);
 }
 
 template <int PT, int NK, bool DET> int launch_q(const SsdParams &p, hipStream_t s, int dd) {
@@ -364,6 +405,7 @@ bool supported(const SsdParams *p) {
       p->C_ls % 8 || p->C_gs % 8 || p->dx_bs % 8 || p->dx_ls % 8 || p->dx_hs % 8)
     return false;
   if (!p->z && (p->dout_bs % 8 || p->dout_ls % 8 || p->dout_hs % 8)) return false;
+  if (!near_rows(p->x_ls) || !near_rows(p->dx_ls) || !near_rows(p->C_ls) || !near_rows(p->z ? (int64_t)p->nheads * p->headdim : p->dout_ls)) return false;
   if (p->batch > 65535 || p->nchunks > 65535) return false;
   return true;
 }

@@ -1,0 +1,60 @@
+"""dx of the SSD backward pass (ssd_dx_fused.hip) at the edges of its tiles: each chunk length, state count and headdim, lists
+of one and of several heads, a last chunk of 1, 17 and Q - 1 positions, packed sequences, D per head, per (head, p) and none.
+Reference: the quadratic form in float64 on the same bf16 operands."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(dt, A, B, C, D, g, seq):
+    """dx and the sum of its absolute terms."""
+    b, L, H, P = g.shape
+    live = torch.ones(L, L, device=g.device).tril().bool()[None].expand(b, L, L)
+    if seq is not None:
+        live = live & (seq[:, :, None] == seq[:, None, :])
+    dx, size = torch.zeros(b, L, H, P, dtype=torch.float64, device=g.device), torch.zeros(b, L, H, P, dtype=torch.float64, device=g.device)
+    for h in range(H):
+        k = h // (H // B.shape[2])
+        a = torch.cumsum(dt[:, :, h].double() * A[h].double(), 1)
+        w = torch.where(live, torch.exp((a[:, :, None] - a[:, None, :]).clamp(max=0)) * dt[:, None, :, h].double(), 0.0)
+        Ck, Bt, gh = C[:, :, k].double(), B[:, :, k].double().transpose(-1, -2).contiguous(), g[:, :, h].double()
+        dx[:, :, h] = torch.matmul((torch.matmul(Ck, Bt) * w).transpose(-1, -2).contiguous(), gh)
+        size[:, :, h] = torch.matmul((torch.matmul(Ck.abs(), Bt.abs()) * w).transpose(-1, -2).contiguous(), gh.abs())
+    if D is not None:
+        d = D.double() if D.dim() == 2 else D.double()[:, None]
+        dx += d * g.double()
+        size += (d * g.double()).abs()
+    return dx, size
+
+
+@pytest.mark.parametrize("b,L,H,G,P,N,Q", [
+    (1, 513, 8, 2, 64, 128, 64), (2, 127, 3, 1, 32, 64, 64), (1, 81, 2, 2, 64, 64, 64), (4, 1024, 24, 1, 32, 128, 64),
+    (2, 641, 5, 1, 64, 128, 128), (4, 1024, 40, 1, 64, 64, 128), (1, 145, 4, 4, 32, 128, 128), (2, 383, 6, 2, 32, 64, 128),
+    (4, 1024, 80, 1, 64, 128, 256), (1, 1025, 6, 2, 64, 128, 256), (2, 511, 3, 1, 64, 64, 256), (1, 785, 5, 5, 32, 128, 256),
+    (4, 256, 4, 1, 32, 64, 256),
+])
+@pytest.mark.parametrize("packed,D_form", [(False, "head"), (True, "none"), (True, "channel")])
+def test_dx(b, L, H, G, P, N, Q, packed, D_form):
+    from mamba_amd.ops.triton import ssd_combined as sc
+    gen = torch.Generator(device="cuda").manual_seed(L + Q + H)
+    randn = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()
+    x, g, B, C = randn(b, L, H, P).requires_grad_(), randn(b, L, H, P), randn(b, L, G, N), randn(b, L, G, N)
+    dt = 0.1 * torch.rand(b, L, H, device="cuda", generator=gen)
+    A = -(0.1 + 5 * torch.rand(H, device="cuda", generator=gen))
+    D = None if D_form == "none" else torch.randn(*((H,) if D_form == "head" else (H, P)), device="cuda", generator=gen).requires_grad_()
+    seq = None
+    if packed:
+        ends = torch.tensor([0, L // 7, L // 7 + 1, L // 2 + 5], device="cuda")
+        seq = (torch.arange(L, device="cuda")[:, None] >= ends).sum(-1).int()[None].expand(b, L).contiguous()
+    sc.mamba_chunk_scan_combined(x, dt, A, B, C, Q, D=D, seq_idx=seq).backward(g)
+    want, size = _reference(dt, A, B, C, None if D is None else D.detach(), g, seq)
+    # the weighted products, the chunk states' gradients (once per chunk's own and once handed on) and the result are rounded
+    # to bf16, 2^-9 of each
+    err = (x.grad.double() - want).abs()
+    assert bool((err <= 4 * 2.0 ** -9 * size + 1e-30).all()), float((err / (size + 1e-30)).max())
+    if D is not None:  # of x and g as they are: fp32 sums of b L (and P) terms
+        terms = x.detach().double() * g.double()
+        dims = (0, 1) if D.dim() == 2 else (0, 1, 3)
+        bound = 2.0 ** -24 * (16 + 4 * (b * L * P) ** 0.5) * terms.abs().sum(dims)
+        assert bool(((D.grad.double() - terms.sum(dims)).abs() <= bound).all())

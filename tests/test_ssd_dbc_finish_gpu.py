@@ -30,9 +30,8 @@ def _reference(x, dt, A, B, C, g, seq):
     return [t.transpose(1, 2) for t in out]
 
 
-# The chunk states and their gradients, dCB and the result are rounded to bf16, 2^-9 of each; a state hands
-# its chunk's share on in fp32.  A sum's terms take two of these roundings, a chunk's own state sums a third
-FACTOR = 4 * 2.0 ** -9
+# A term takes the rounding to bf16 (at most 2^-8 of it) of dCB or of a chunk state or its gradient, the result another one
+FACTOR = 2 * 2.0 ** -8
 
 
 def _check(B, C, want):

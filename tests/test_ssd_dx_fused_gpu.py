@@ -49,10 +49,9 @@ def test_dx(b, L, H, G, P, N, Q, packed, D_form):
         seq = (torch.arange(L, device="cuda")[:, None] >= ends).sum(-1).int()[None].expand(b, L).contiguous()
     sc.mamba_chunk_scan_combined(x, dt, A, B, C, Q, D=D, seq_idx=seq).backward(g)
     want, size = _reference(dt, A, B, C, None if D is None else D.detach(), g, seq)
-    # the weighted products, the chunk states' gradients (once per chunk's own and once handed on) and the result are rounded
-    # to bf16, 2^-9 of each
+    # the weighted products or the chunk states' gradients, and the result, are rounded to bf16: at most 2^-8 of each, twice
     err = (x.grad.double() - want).abs()
-    assert bool((err <= 4 * 2.0 ** -9 * size + 1e-30).all()), float((err / (size + 1e-30)).max())
+    assert bool((err <= 2 * 2.0 ** -8 * size + 1e-30).all()), float((err / (size + 1e-30)).max())
     if D is not None:  # of x and g as they are: fp32 sums of b L (and P) terms
         terms = x.detach().double() * g.double()
         dims = (0, 1) if D.dim() == 2 else (0, 1, 3)

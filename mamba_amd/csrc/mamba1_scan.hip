@@ -123,10 +123,7 @@ __global__ __launch_bounds__(SEG_THREADS, BWD || sizeof(T) == 4 ? 3 : 4) void sc
   for (int n0 = 0; n0 < N; n0 += NB16) {
     float acc[NB16], A2[NB16];
 #pragma unroll
-    for (int n = 0; n < NB16; ++n) {
-      acc[n] = 0.f;
-      A2[n] = n0 + n < N ? ((const float *)p.A)[(int64_t)d * N + n0 + n] * kLog2e : 0.f;
-    }
+    for (int n = 0; n < NB16; ++n) acc[n] = 0.f;
     Pack8<T> ku, kd, kz, ks[2][NG];
     auto fetch_rows = [&](int k) {
       const int tl = tile_of(k) * TILE + c * KI;
@@ -143,6 +140,12 @@ __global__ __launch_bounds__(SEG_THREADS, BWD || sizeof(T) == 4 ? 3 : 4) void sc
     float run = 0.f, first = 0.f;  // steps of the tiles already taken; backward: without the segment's first step, `first`
     fetch_rows(0);
     fetch_states(ks[0], 0, 0);
+    // (requested behind the first tile's items, all at once: ahead of them, they are a latency of their own, 31.1 -> 27.8 us
+    // at 2 x 1536 channels x 2048 positions in fp32, 27.0 -> 25.6 in bf16)
+#pragma unroll
+    for (int n = 0; n < NB16; ++n) A2[n] = ((const float *)p.A)[(int64_t)d * N + min(n0 + n, N - 1)];
+#pragma unroll
+    for (int n = 0; n < NB16; ++n) A2[n] = n0 + n < N ? A2[n] * kLog2e : 0.f;
     for (int k = 0; k < ntiles; ++k) {
       // A lane in a ragged row's last piece reads 8 items from L - 8 on like the other rows' lanes, and leaves out the
       // ones before its own, which are the lane before's (nothing has to be moved into place: the order is what counts).

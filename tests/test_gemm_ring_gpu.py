@@ -1,0 +1,49 @@
+"""The grouped bf16 products whose operands lie on 16 bytes (gemm_ring_kernel in gemm.hip): edges of the 64 x 64 tile, of the
+64-wide stage and of a split's k, every layout of both operands, beside values that must not be read into a result.
+Reference: fp64 products."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# M, N multiples of 8 where the operand lies along its rows, K where one lies along k
+SHAPES = [(8, 8, 8), (64, 64, 64), (72, 136, 72), (200, 56, 128), (64, 192, 200), (136, 64, 2072), (80, 72, 4104), (1000, 768, 1536)]
+ODD_K = [(64, 128, 33), (72, 64, 97), (128, 136, 1001), (64, 64, 1)]        # both along their rows: any K
+ODD_ROWS = [(65, 127, 64), (1, 3, 72), (100, 66, 2048), (129, 63, 4120)]     # both along k: any M and N
+
+
+@pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, SHAPES) for a in (True, False) for b in (True, False)] + [(False, False, ODD_K), (True, True, ODD_ROWS)])
+@pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
+def test_products(a_k, b_k, shapes, out):
+    from mamba_amd import _lib
+    lib = _lib.load()
+    gen = torch.Generator(device="cuda").manual_seed(5)
+
+    def operand(rows, k, along_k):  # 8 values of NaN behind every line and a line of them behind the last
+        lines, n = (rows, k) if along_k else (k, rows)
+        t = torch.full((lines + 1, (n + 7) // 8 * 8 + 8), float("nan"), device="cuda", dtype=torch.bfloat16)
+        t[:lines, :n] = torch.randn(lines, n, device="cuda", generator=gen).bfloat16()
+        t = t[:lines, :n]
+        return t if along_k else t.t()
+
+    for first in range(0, len(shapes), 4):
+        group, keep = (_lib.MambaGemm * 4)(), []
+        for j, (M, N, K) in enumerate(shapes[first:first + 4]):
+            A, B, bias = operand(M, K, a_k), operand(N, K, b_k), torch.randn(N, device="cuda", generator=gen).bfloat16()
+            D = torch.full((M, N + 3), 0.5, device="cuda", dtype=out)
+            with_bias, accumulate = j % 2 == 0, j >= 2
+            want = A.double() @ B.double().t() + (bias.double() if with_bias else 0) + (0.5 if accumulate else 0)
+            size = A.double().abs() @ B.double().abs().t() + 1
+            group[j] = _lib.MambaGemm(A.data_ptr(), B.data_ptr(), bias.data_ptr() if with_bias else None, D.data_ptr(), *A.stride(), *B.stride(),
+                                      N + 3, M, N, K, _lib.DTYPE_CODE[out], int(accumulate), 0)
+            keep.append((A, B, bias, D, want, size, K))
+        floats = lib.mamba_gemm_plan(group, 4)
+        assert floats >= 0
+        ws = torch.full((max(floats, 1),), float("nan"), device="cuda")
+        _lib.check(lib.mamba_gemm(group, 4, ws.data_ptr(), _lib.current_stream(ws.device)), "mamba_gemm")
+        for A, B, bias, D, want, size, K in keep:
+            N = want.shape[1]
+            # fp32 sums of K terms, and one rounding to the result's type
+            bound = 2.0 ** -24 * (16 + 4 * K ** 0.5) * size + (2.0 ** -8 if out == torch.bfloat16 else 0) * want.abs()
+            assert bool(((D[:, :N].double() - want).abs() <= bound).all())
+            assert bool((D[:, N:] == 0.5).all())

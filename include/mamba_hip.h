@@ -422,6 +422,9 @@ int ssd_chunk_state_varlen(const SsdParams *p, const int32_t *cu_seqlens, int ns
  *   ssd_chunk_cumsum_bwd  ddt, dA, ddt_bias from ddA_cumsum and ddt_out
  *                     (ssd_combined_bwd deals the workgroups of these last two stages to one launch where the bmm
  *                     stage runs on its 64 x 128 tiles: they read disjoint results of the stages before them)
+ *                     (for bf16 with 16-byte aligned rows where one workgroup holds all heads of a group in both the dCB and
+ *                     the state-path stage, the order is dCB, dBC_state, dx, cumsum: the state-path kernel then forms the dCB
+ *                     contractions too and writes dB / dC; dB32 / dC32 are not touched)
  * ddA_cumsum holds the gradient with respect to the cumulative sums a_l; the last
  * stage turns it into the gradient of the per-position dt * A. */
 int ssd_bwd_dz(const SsdParams *p, mamba_stream_t stream);

@@ -2141,8 +2141,8 @@ static int ssd_combined_bwd_one(const SsdParams *p, mamba_stream_t stream) {
   const bool lp = dcb_tiles_lp(p);
   // Where one workgroup holds a group's heads in the dCB stage and in the state-path stage, the latter follows it and forms
   // the in-chunk products of dB / dC as well: the fp32 sums between the two and the stage that read them are not needed.
-  // The state path and what follows dCB at 16384 positions, 128 heads in 8 groups, chunk 256: 285 us against 465 of the other order
-  // (of which the products and the cumsum 214); 2 x 4096, 40 heads in 8 groups, chunk 128: 57 against 90.
+  // The state path and what follows dCB at 16384 positions, 128 heads in 8 groups, chunk 256: 272 us against 465 of the other order
+  // (of which the products and the cumsum 214); 2 x 4096, 40 heads in 8 groups, chunk 128: 52 against 90.
   const SsdParams filled = with_grad_strides(*p);
   if (lp && p->dB && p->dC && ssd_bwd_dbc_finishes(&filled)) {
     if ((rc = ssd_bwd_dcb_one(p, stream, true))) return rc;

@@ -956,17 +956,18 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
   const FwdCost lanes{false, round * ((p.dstate + NB16 - 1) / NB16) * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
   if (p.dstate != NB16 || (p.bc_const & 3) || p.a_complex || k4_mode() || p.seqlen < KI) return lanes;
   const int64_t fives = wgs / (5 * cus), rest = (wgs - fives * 5 * cus + cus - 1) / cus;
-  const FwdCost serial{true, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + 3.4};
+  const FwdCost serial{true, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + (p.seqlen % KI ? 3.4 : 2.0)};
   return serial.us < lanes.us ? serial : lanes;
 }
 
 // Segments of the sequence: the split with the least estimated time in us, for 16 states.  The terms were fitted to the
 // times of 1 .. 32 segments (forward at 45 sizes: fwd_cost; backward at 13, batch 1 - 8, 768 - 5120 channels, 256 - 8192
 // positions; within 10 % of almost all).  A tile of a round of backward workgroups (one per CU) takes 13 per pass and a
-// third of that for what the passes share, a round's start and end 5.3.  The pass over the segments (all but one) takes 3.0
+// third of that for what the passes share, a round's start and end 5.3.  The pass over the segments (all but one) takes 2.7
 // (forward) or 4.5 (backward) a tile, twice that from four of its workgroups per CU on, and every segment 0.9 or 1.8 for
-// its launch and for going through the segments before it.  A split has to promise 6 %.  Measured: 1536 channels x 777
-// positions of one sequence 50 -> 24 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181 forward.
+// its launch and for going through the segments before it.  A split has to promise 1 % (forward) or 6 % (backward).
+// Measured: 1536 channels x 777 positions of one sequence 50 -> 24 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181
+// forward; 1536 channels whole and in two segments: 14.8 and 14.8 (129 positions), 13.1 and 14.6 (192), 16.6 and 15.0 (256).
 constexpr int MAX_SEGMENTS = 32;
 int scan_segments(const MambaScanParams &p, bool bwd) {
   const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
@@ -991,7 +992,7 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
     }
     if (s > 1) {
       const double share = std::max(1.0, 0.52 * (double)((seg_wgs * (s - 1) + cus - 1) / cus));
-      cost = 1.06 * (cost + (bwd ? 4.5 : 3.0) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
+      cost = (bwd ? 1.06 : 1.01) * (cost + (bwd ? 4.5 : 2.7) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
     }
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = s;
   }

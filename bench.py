@@ -842,7 +842,7 @@ def bench_mamba1(dev, steps, warmup):
                 "kernel_ms": bwd_ms, "kernel_ms_min_max_n": [bwd_st["min"], bwd_st["max"], bwd_st["n"]],
                 "algorithmic_bytes": bwd_bytes,
                 "fwd_kernel_ms": fwd_ms, "fwd_kernel_ms_min_max_n": [fwd_st["min"], fwd_st["max"], fwd_st["n"]], "fwd_achieved": fwd_bytes / (fwd_ms * 1e-3) / 1e9,
-                "fwd_traffic": profile_traffic(prof + "_hbm_counters.txt", "scan_fwd_kernel"),
+                "fwd_traffic": profile_traffic(prof + "_hbm_counters.txt", "scan_fwd_serial_kernel"),
                 "fwd_bwd_frac": (fwd_bytes + bwd_bytes) / ((fwd_ms + bwd_ms) * 1e-3) / 1e9 / HBM_PEAK_GBS}
     vs_measured_copy(roofline, dev)
     # The binding resource of both scan kernels is fp32 vector-ALU issue, not HBM.  A SIMD issues one plain
@@ -855,8 +855,7 @@ def bench_mamba1(dev, steps, warmup):
     probe = measured_valu(dev)
     valu = {"unit": "T lane-instruction slots/s", "measured_fma_probe": probe,
             "nominal_peak": 256 * 4 * 32 * 2.4e9 / 1e12, "element_states": elems}
-    for name, ms in (("bwd", bwd_ms), ("fwd", fwd_ms)):
-        kern = "scan_%s_kernel" % name
+    for name, kern, ms in (("bwd", "scan_bwd_kernel", bwd_ms), ("fwd", "scan_fwd_serial_kernel", fwd_ms)):
         insts = profile_counter(prof + "_valu_counters.txt", kern, "SQ_INSTS_VALU")
         trans = profile_counter(prof + "_valu_counters.txt", kern, "SQ_INSTS_VALU_TRANS_F32")
         if insts is None or trans is None:

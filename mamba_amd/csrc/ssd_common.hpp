@@ -922,6 +922,9 @@ inline int heads_per_workgroup(const SsdParams &p) {
 // ssd_chunk_scan_fwd_fused_supported accepts.
 __attribute__((visibility("hidden"))) bool ssd_scan_paired_serves(const SsdParams &p);
 __attribute__((visibility("hidden"))) int ssd_scan_paired_launch(const SsdParams &p, hipStream_t s);
+// The form that keeps C B^T of the group for all heads of a workgroup (ssd_scan_group.hip)
+__attribute__((visibility("hidden"))) bool ssd_scan_group_serves(const SsdParams &p);
+__attribute__((visibility("hidden"))) int ssd_scan_group_launch(const SsdParams &p, hipStream_t s);
 // MAMBA_AMD_SSD_SCAN=single keeps the one-tile-per-wave kernel for every chunk size (for measurements).
 inline bool ssd_single_tile_only() {
   static const bool v = [] {

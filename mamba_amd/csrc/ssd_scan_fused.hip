@@ -318,6 +318,7 @@ __global__ __launch_bounds__(64 * QT) void chunk_scan_fwd_fused_kernel(const Ssd
 }
 
 template <int PT, int NK> int launch_q(const SsdParams &p, hipStream_t s) {
+  if (ssd_scan_group_serves(p) && !ssd_single_tile_only()) return ssd_scan_group_launch(p, s);
   if (ssd_scan_paired_serves(p) && !ssd_single_tile_only()) return ssd_scan_paired_launch(p, s);
   const int hb = heads_per_workgroup(p);
   dim3 grid(p.nheads / hb, p.nchunks, p.batch);

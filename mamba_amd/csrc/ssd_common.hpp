@@ -849,8 +849,11 @@ DEVI View4 g_view(const SsdParams &p) {
 // 16 bytes per lane from base + offset (bytes) to LDS, lane after lane from `lds` on.  The compiler does not count this load:
 // async_done() before the barrier that hands the data over.  LEFT: vector memory operations that may still be in flight, at
 // most as many as were surely issued after the loads (they complete in order); 0 waits for everything.
+// (A scalar that a vector instruction wrote, a spilled base that comes back lane by lane for one, may be read by vector memory
+// five wait states later: the compiler, which keeps that distance elsewhere, does not look inside the statement, so it
+// brings all five itself.  One is enough between m0 and the load.)
 DEVI void load_async16(const void *base, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory", "m0");
 }
 template <int LEFT> DEVI void async_done() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
 

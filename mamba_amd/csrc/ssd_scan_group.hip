@@ -15,6 +15,9 @@ DEVI f32x4 mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// What a decay's exponent (base 2) may reach: an exponential that stays finite, for the zeros of S to be multiplied by.
+constexpr float kGrowth = 126.f;
+
 // A head as the asynchronous loads lay it down: whole rows without padding, their 16-byte pieces permuted within the row so
 // that the reads of 16 rows (state) and the transposing reads of 8 rows (x) meet in no bank.
 template <int PT, int NK, int QT> struct ScanHead {
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void chu
     if (tid < Q) {
       shm.a2[odd][tid] = n_a * kLog2e;
       shm.dt[odd][tid] = n_dt;
-      shm.cs[odd][tid] = n_dt * fast_exp(fminf(__shfl(n_a, lane | 15, 64) - n_a, 0.f));
+      shm.cs[odd][tid] = n_dt * fast_exp2(fminf((__shfl(n_a, lane | 15, 64) - n_a) * kLog2e, kGrowth));
     }
     if (tid < P) shm.d[odd][tid] = Dp ? n_d : 0.f;
     lds_barrier();  // this head is there, and nobody reads the one before it any more
@@ -204,8 +207,10 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void chu
     const uint32_t cs_at = lds_address(&shm.cs[odd][4 * g]) + first * 64, a2_at = lds_address(a2) + first * 64, dt_at = lds_address(&shm.dt[odd][4 * g]) + first * 64;
 
     // ---- inside the chunk: two s tiles, first - k and the next, with S of both.  Below the diagonal the decay is exp(a_l -
-    // a_end) (dt_s exp(a_end - a_s)) with a_end the last a of the 16 positions s (both exponents <= 0); the pair that holds the
-    // diagonal takes the exact one; S is zero above it
+    // a_end) (dt_s exp(a_end - a_s)) with a_end the last a of the 16 positions s; the pair that holds the diagonal takes the
+    // exact one; S is zero above it.  Both exponents are <= 0 where all steps are >= 0.  With steps of either sign one of them
+    // may not be, though their sum is: below the diagonal tile neither is cut at 0, as in the other forms of this scan
+    const float below = lt & 1 ? kGrowth : 0.f;  // the pair's first tile: below the diagonal, or the diagonal one
     auto block = [&](const int k, const f32x4 (&Sk)[2], const bool diagonal) {
       float m[8];
 #pragma unroll
@@ -214,10 +219,10 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void chu
         if (diagonal) {
           const f32x4 as = *(lds_f4)(uintptr_t)(a2_at + 16 * g + o), dts = *(lds_f4)(uintptr_t)(dt_at + o);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) m[4 * i + r] = Sk[i][r] * dts[r] * fast_exp2(fminf(al2 - as[r], 0.f));
+          for (int r = 0; r < 4; ++r) m[4 * i + r] = Sk[i][r] * dts[r] * fast_exp2(fminf(al2 - as[r], i == 0 ? below : 0.f));
         } else {
           const f32x4 cs = *(lds_f4)(uintptr_t)(cs_at + o);
-          const float rl = fast_exp2(fminf(al2 - *(lds_f1)(uintptr_t)(a2_at + o + 60), 0.f));
+          const float rl = fast_exp2(fminf(al2 - *(lds_f1)(uintptr_t)(a2_at + o + 60), kGrowth));
 #pragma unroll
           for (int r = 0; r < 4; ++r) m[4 * i + r] = Sk[i][r] * cs[r] * rl;
         }

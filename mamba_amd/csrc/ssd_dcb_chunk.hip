@@ -22,6 +22,10 @@ namespace {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
+// What a decay's exponent (base 2) may reach: an exponential that stays finite, for the zeros of a masked C B^T to be
+// multiplied by.
+constexpr float kGrowth = 126.f;
+
 DEVI f32x4 mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
 
 // x + y folded: lanes 0 - 31 get the sum of x over the two halves of the wave, lanes 32 - 63 that of y
@@ -102,7 +106,7 @@ __global__ __launch_bounds__(32 * QT) void bwd_dcb_chunk_kernel(const SsdParams 
   };
   auto commit_scalars = [&](Buf &to) {
     const int pos = min(tid, Q - 1);  // (the threads past the chunk write its last position's values once more)
-    to.el[pos] = fast_exp(fminf(sc_a - sc_ref, 0.f));
+    to.el[pos] = fast_exp2(fminf((sc_a - sc_ref) * kLog2e, kGrowth));
     to.a2[pos] = sc_a * kLog2e;
     to.col[pos] = f32x2{sc_a * kLog2e, sc_dt};
   };
@@ -235,8 +239,9 @@ __global__ __launch_bounds__(32 * QT) void bwd_dcb_chunk_kernel(const SsdParams 
     fetch_g(next);
     fetch_scalars(next);
 
-    // Below the diagonal the decay is taken apart at the first position of l's tile, exp(a_l - a_ref) * exp(a_ref - a_s),
-    // both exponents <= 0: one exponential per column and block.  rs: sums over the blocks of a row of tiles below the
+    // Below the diagonal the decay is taken apart at the first position of l's tile, exp(a_l - a_ref) * exp(a_ref - a_s):
+    // one exponential per column and block.  (Both exponents are <= 0 where all steps are >= 0.  With steps of either sign
+    // one may be above, though their sum is not: neither is cut at 0.)  rs: sums over the blocks of a row of tiles below the
     // diagonal, without the row's factor el; they join those of the short (a) and the long row (b) where the row ends.
     f32x4 rs = {0.f, 0.f, 0.f, 0.f}, rsa = rs, rsb = rs, el = *reinterpret_cast<const f32x4 *>(&at.el[(QT - 1 - wave) * 16 + gq * 4]);
     float ref = readlane_f(at.a2[(QT - 1 - wave) * 16], 0);
@@ -259,7 +264,7 @@ __global__ __launch_bounds__(32 * QT) void bwd_dcb_chunk_kernel(const SsdParams 
               else rsb[r] += w;
             }
           } else {
-            const float f = col.y * fast_exp2(fminf(ref - col.x, 0.f));
+            const float f = col.y * fast_exp2(fminf(ref - col.x, kGrowth));
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float t = v[r] * f, w = t * cb[k][r];

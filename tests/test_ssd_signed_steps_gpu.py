@@ -42,3 +42,21 @@ def test_forward(b, L, H, G, P, N, Q):
     y = mamba_chunk_scan_combined(x, dt, A, B, C, Q, dt_limit=OPEN).detach().double()
     want = _reference(*[t.detach().double() for t in (x, dt, A, B, C)])
     assert float((y - want).norm() / want.norm()) <= BOUND
+
+
+# dB and dC, whose in-chunk share is dCB: sizes at which one workgroup holds a chunk's whole triangle (ssd_dcb_chunk.hip; the
+# tile pairs of ssd_bwd.hip cut both exponents at 0)
+@pytest.mark.parametrize("b,L,H,G,P,N,Q", [
+    (2, 2048, 40, 8, 64, 128, 128), (1, 2033, 16, 8, 64, 128, 64), (16, 1000, 40, 2, 32, 64, 64), (8, 1024, 64, 8, 64, 128, 256),
+    (8, 1000, 64, 8, 32, 64, 128),
+])
+def test_dB_dC(b, L, H, G, P, N, Q):
+    from mamba_amd.ops.triton.ssd_combined import mamba_chunk_scan_combined
+    x, dt, A, B, C, g = _inputs(b, L, H, G, P, N)
+    B.requires_grad_(), C.requires_grad_()
+    got = torch.autograd.grad(mamba_chunk_scan_combined(x, dt, A, B, C, Q, dt_limit=OPEN), [B, C], g)
+    Bd, Cd = B.detach().double().requires_grad_(), C.detach().double().requires_grad_()
+    want = torch.autograd.grad(_reference(x.double(), dt.double(), A.double(), Bd, Cd), [Bd, Cd], g.double())
+    for name, u, v in zip(("dB", "dC"), got, want):
+        err = float((u.double() - v).norm() / v.norm())
+        assert err <= BOUND, f"{name}: {err:.5f}"

@@ -937,6 +937,14 @@ int bwd_passes(const MambaScanParams &p, int64_t *cost_out = nullptr) {
   return best;
 }
 
+// MAMBA_AMD_FWD_MIN_LDS (bytes): a measurement hook.  A workgroup of scan_fwd_kernel that asks for more LDS shares its CU with
+// fewer others (160 KB per CU), which is how that kernel's speed against resident waves per SIMD is measured; where the
+// hook is set, that kernel runs.
+size_t fwd_min_lds() {
+  static const size_t v = getenv("MAMBA_AMD_FWD_MIN_LDS") ? (size_t)atol(getenv("MAMBA_AMD_FWD_MIN_LDS")) : 0;
+  return v;
+}
+
 // The forward kernel that serves a problem and its estimated time in us, for 16 states.  scan_fwd_serial_kernel
 // (mamba1_scan_serial.hip) takes 16 states and per-position B and C; up to five of its workgroups share a CU, and a tile
 // (half tiles where the sequence ends in one) takes a round of them 7.3, 10.7, 14.1, 17.5, 20.9.  scan_fwd_kernel: up to
@@ -954,7 +962,7 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
   const int64_t pairs = wgs / (2 * cus), odd = wgs - pairs * 2 * cus;
   const double round = (10.9 * (double)pairs + (odd > cus ? 10.9 : odd > 0 ? 6.6 : 0.0)) * (p.seqlen % KI ? 1.15 : 1.0);
   const FwdCost lanes{false, round * ((p.dstate + NB16 - 1) / NB16) * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
-  if (p.dstate != NB16 || (p.bc_const & 3) || p.a_complex || k4_mode() || p.seqlen < KI) return lanes;
+  if (p.dstate != NB16 || (p.bc_const & 3) || p.a_complex || k4_mode() || fwd_min_lds() || p.seqlen < KI) return lanes;
   const int64_t fives = wgs / (5 * cus), rest = (wgs - fives * 5 * cus + cus - 1) / cus;
   const FwdCost serial{true, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + (p.seqlen % KI ? 3.4 : 2.0)};
   return serial.us < lanes.us ? serial : lanes;
@@ -1141,12 +1149,9 @@ template <typename T, bool BWD, int BC> int dispatch_bc(const MambaScanParams &p
   int rc = launch_segments<T, BC, BWD>(p, mode, stream);
   if (rc != MAMBA_OK) return rc;
   if (!BWD) {
-    // MAMBA_AMD_FWD_MIN_LDS (bytes): a measurement hook.  A workgroup that asks for more LDS shares its CU with fewer
-    // others (160 KB per CU), which is how the kernel's speed against resident waves per SIMD is measured.
-    static const size_t min_lds = getenv("MAMBA_AMD_FWD_MIN_LDS") ? (size_t)atol(getenv("MAMBA_AMD_FWD_MIN_LDS")) : 0;
     const bool half = k4_mode();
     if (fwd_cost(p, std::max(1, p.nseg)).serial) return mamba1_fwd_serial_launch(p, mode, stream);
-    const size_t lds = fwd_lds(1, np, half) > min_lds ? fwd_lds(1, np, half) : min_lds;
+    const size_t lds = std::max(fwd_lds(1, np, half), fwd_min_lds());
     if (half)
       return mode == ROWS_ALIGNED ? launch(scan_fwd_kernel<T, ROWS_ALIGNED, BC, true>, p, 1, lds, stream)
                                   : launch(scan_fwd_kernel<T, ROWS_SCALAR, BC, true>, p, 1, lds, stream);

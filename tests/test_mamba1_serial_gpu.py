@@ -93,3 +93,26 @@ def test_end_of_one_sequence_stays_in_it():
     assert not finite[:, 5, 129].any() and finite[:, 5, :129].all() and finite[:, 7, :64].all()
     finite[:, 5] = finite[:, 7] = True
     assert finite.all()
+
+
+def test_the_measurement_hook_reaches_the_other_kernel():
+    """MAMBA_AMD_FWD_MIN_LDS is for scan_fwd_kernel, and selects it: its fp32 sums are taken in another order than this one's."""
+    import os
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = ("import sys; sys.path[:0] = [%r, %r]\n"
+            "import hashlib, torch, test_mamba1_serial_gpu as t\n"
+            "from mamba_amd.ops.selective_scan_interface import selective_scan_fn\n"
+            "i = t._inputs(7, 3184, 192, 1, torch.float32, 5)\n"
+            "t._check(i)\n"
+            "y = selective_scan_fn(i['u'], i['delta'], i['A'], i['B'], i['C'], i['D'], z=i['z'], delta_bias=i['delta_bias'], delta_softplus=True)\n"
+            "print(hashlib.sha256(y.cpu().numpy().tobytes()).hexdigest())\n") % (here, os.path.dirname(here))
+    bits = set()
+    for lds in ("", "1"):
+        env = dict(os.environ)
+        env.pop("MAMBA_AMD_FWD_MIN_LDS", None)
+        if lds:
+            env["MAMBA_AMD_FWD_MIN_LDS"] = lds
+        bits.add(subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, check=True, timeout=100).stdout)
+    assert len(bits) == 2

@@ -52,6 +52,9 @@ template <int PT, int NK, int QT, bool DET>
 __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void bwd_dx_fused_kernel(const SsdParams p, const int hb, const int sum_dD) {
   constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT, SR = QT > 8 ? 8 : QT;
   constexpr int RP = P / 8, MP = N / 8;  // 16-byte pieces of a g row, of a state or C row
+  // What every wave issues for a head of a full chunk behind its loads of the next one, whatever the values: the two adds of
+  // its positions and its stores of dx.  The wait for those loads counts on all of them.
+  constexpr int ADDS = 2, STORES = PT / 2;
   __shared__ DxShared<PT, NK, QT> shm;
   typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
   typedef __attribute__((address_space(3))) bf16x8_t *lds_frag;
@@ -193,9 +196,8 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void bwd
     // used instead of being carried (or spilled) across the loop over the heads
     asm volatile("" : "+v"(tid));
     lane = tid & 63, j = lane & 15, g = lane >> 4, s_own = lt * 16 + j;
-    // This head's operands are there once no more is in flight than what followed them, in order: at a full chunk two
-    // adds and PT / 2 stores of the head before (more in some waves).
-    if (qlim == Q && !DET) async_done<2 + PT / 2>();
+    // This head's operands are there once no more is in flight than what followed them, in order (more in some waves)
+    if (qlim == Q && !DET) async_done<ADDS + STORES>();
     else async_done<0>();
     if (qlim < Q) {  // g is zero past the end of the sequence
 #pragma unroll
@@ -316,7 +318,7 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void bwd
     {
       const int64_t row_off = (((int64_t)b * H + h) * p.nchunks + c) * Q;
       const bool live = g == 0 && s_own < qlim;
-      if (live) {
+      if (live) {  // (ADDS, not left out where a value is 0)
         acc_add<DET ? 1 : 0>(p.ddt_out, p.det_ddt_out, row_off + s_own, q2, dsc);
         acc_add<DET ? 1 : 0>(p.ddA_cumsum, p.det_ddA_cumsum, row_off + s_own, -dts * q1, dsc);
       }
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void bwd
     float dd = 0.f;
     const uint32_t own_at = here + s_own * (2 * P) + g * 8 + swz_g(s_own) * 32;
 #pragma unroll
-    for (int e = 0; e < PT / 2; ++e) {
+    for (int e = 0; e < STORES; ++e) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int pt = 2 * e + k;
@@ -352,7 +354,8 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void bwd
       }
       wave_sync();
       const u32x4 out = *(lds_u4)(uintptr_t)y_row;
-      if (lt * 16 + rr < qlim) *(GLOBAL_AS u32x4 *)(dx_at_head + (uint32_t)rr * (uint32_t)(2 * p.dx_ls) + piece * 16 + e * 64) = out;
+      if (lt * 16 + rr < qlim)  // (STORES)
+        *(GLOBAL_AS u32x4 *)(dx_at_head + (uint32_t)rr * (uint32_t)(2 * p.dx_ls) + piece * 16 + e * 64) = out;
       wave_sync();
     }
     if (sum_dD) {

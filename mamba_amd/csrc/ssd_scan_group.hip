@@ -41,6 +41,9 @@ template <int PT, int NK, int QT, bool GATED>
 __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void chunk_scan_fwd_group_kernel(const SsdParams p, const int hb) {
   constexpr int P = 16 * PT, N = 32 * NK, Q = 16 * QT;
   constexpr int RP = P / 8, MP = N / 8;  // 16-byte pieces of an x row, of a state or B row
+  // What every wave issues for a head of a full chunk behind its loads of the next one: its stores of the output.  The wait
+  // for those loads counts on all of them.
+  constexpr int STORES = PT / 2;
   __shared__ ScanShared<PT, NK, QT> shm;
   typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
   typedef __attribute__((address_space(3))) bf16x8_t *lds_frag;
@@ -169,9 +172,8 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void chu
     // used instead of being carried (or spilled) across the loop over the heads
     asm volatile("" : "+v"(tid));
     lane = tid & 63, j = lane & 15, g = lane >> 4, l_own = lt * 16 + j;
-    // This head's operands are there once no more is in flight than what followed them, in order: at a full chunk PT / 2
-    // stores of the head before (or twice as many).
-    if (qlim == Q) async_done<PT / 2>();
+    // This head's operands are there once no more is in flight than what followed them, in order (or twice as many)
+    if (qlim == Q) async_done<STORES>();
     else async_done<0>();
     if (qlim < Q) {  // x is zero past the end of the sequence
 #pragma unroll
@@ -270,7 +272,7 @@ __global__ __launch_bounds__(64 * QT, QT == 4 && PT * NK == 16 ? 2 : 4) void chu
     const uint32_t o_off = (uint32_t)rr * (uint32_t)(2 * p.out_ls) + piece * 16;
     const bool stored = lt * 16 + rr < qlim;
 #pragma unroll
-    for (int e = 0; e < PT / 2; ++e) {
+    for (int e = 0; e < STORES; ++e) {
       u32x2 zl[2];
       if (GATED) {
         *(lds_u4)(uintptr_t)y_row = zr[e];

@@ -4,6 +4,9 @@ distance between instructions inside one."""
 import glob
 import os
 import re
+import subprocess
+
+import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mamba_amd", "csrc")
 
@@ -36,3 +39,53 @@ def test_asm_that_reads_memory_through_a_scalar_base_waits_for_it():
             m = re.match(r"s_nop (\d+)", inst)
             states += int(m.group(1)) + 1 if m else 1
     assert seen
+
+
+def _fewest_behind(lines):
+    """Over the paths from an asynchronous load to a counted wait of the source (async_done): the fewest vector memory
+    operations on the way, less the number that the wait lets stay in flight.  A path ends where the source waits for
+    everything; the compiler's own waits, of which it may make fewer, are left out of account.  A branch over an empty set
+    of lanes is not taken: at a full chunk every wave has lanes in every store and add, by the conditions in the source."""
+    label = {m.group(1): k for k, l in enumerate(lines) if (m := re.match(r"(\.LBB\w+):", l))}
+    best, todo = None, [(0, k + 1) for k, l in enumerate(lines) if l.startswith("global_load_lds")]
+    seen = {}
+    while todo:
+        n, k = min(todo)
+        todo.remove((n, k))
+        while k < len(lines) and seen.get(k, n + 1) > n:
+            seen[k] = n
+            l = lines[k]
+            m = re.match(r"s_waitcnt vmcnt\((\d+)\)", l)
+            if m and lines[k - 1] == ";;#ASMSTART":
+                if int(m.group(1)) > 0:
+                    best = n - int(m.group(1)) if best is None else min(best, n - int(m.group(1)))
+                break
+            if re.match(r"(global|flat|buffer|scratch)_(load|store|atomic)", l):
+                n += 1
+            elif m := re.match(r"s_(c?branch)(\w*)\s+(\.LBB\w+)", l):
+                if m.group(1) == "branch":
+                    k = label[m.group(3)]
+                    continue
+                if m.group(2) != "_execz":
+                    todo.append((n, label[m.group(3)]))
+            elif l.startswith("s_endpgm"):
+                break
+            k += 1
+    return best
+
+
+@pytest.mark.parametrize("name,kernel", [("ssd_dx_fused", "bwd_dx_fused_kernel"), ("ssd_scan_group", "chunk_scan_fwd_group_kernel")])
+def test_counted_waits_cover_the_loads(name, kernel, tmp_path):
+    from mamba_amd import build
+    out = tmp_path / "k.s"
+    subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), *build.HIPCC_FLAGS, "--cuda-device-only", "-S", os.path.join(CSRC, name + ".hip"),
+                    "-o", str(out)], check=True, capture_output=True)
+    text, counted = out.read_text(), 0
+    for m in re.finditer(r"^(_Z\w*%s\w*):(.*?)^\s*\.section" % kernel, text, flags=re.S | re.M):
+        lines = [l.split("; ")[0].strip() for l in m.group(2).splitlines()]
+        lines = [l for l in lines if l and not re.match(r"\.(?!LBB)|;(?!;#ASM)", l)]
+        assert any(l.startswith("global_load_lds") for l in lines)
+        counted += sum(lines[k] == ";;#ASMSTART" and bool(re.match(r"s_waitcnt vmcnt\([1-9]", lines[k + 1])) for k in range(len(lines) - 1))
+        behind = _fewest_behind(lines)
+        assert behind is None or behind >= 0, m.group(1)
+    assert counted

@@ -332,7 +332,10 @@ template <int PT, int NK, bool GATED> int launch_q(const SsdParams &p, hipStream
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
 }
 template <int PT, int NK> int launch_z(const SsdParams &p, hipStream_t s) {
-  return p.z ? launch_q<PT, NK, true>(p, s) : launch_q<PT, NK, false>(p, s);
+  if constexpr (NK > 2) {
+    if (p.z) return launch_q<PT, NK, true>(p, s);
+  }
+  return p.z ? MAMBA_E_UNSUPPORTED : launch_q<PT, NK, false>(p, s);  // (64 states with a gate: not served, below)
 }
 
 }  // namespace

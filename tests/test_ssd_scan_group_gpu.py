@@ -1,6 +1,7 @@
 """The forward chunk scan that keeps C B^T of the group (ssd_scan_group.hip): chunks of 64 and 128, state counts and headdims,
 lists of one and of several heads, a last chunk of 1, 17 and Q - 1 positions, packed sequences, with and without gate, pre-gate
-copy and D.  Reference: the stage's formula in float64 on the same bf16 operands."""
+copy and D.  (64 states with a gate are left to the one-tile form of ssd_scan_fused.hip: the same check of that one.)  Reference:
+the stage's formula in float64 on the same bf16 operands."""
 import pytest
 import torch
 

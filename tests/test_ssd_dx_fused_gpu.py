@@ -7,6 +7,19 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+def _worst_tile(got, want):
+    """The largest error of 16 positions of one head (or group), as a share of their norm.  (Whole tiles: the one or few terms
+    of a single position can cancel, and leave a result that is small beside the rounding of each.)"""
+    tiles = lambda t: t[:, :t.shape[1] // 16 * 16].double().unflatten(1, (-1, 16)).pow(2).sum((2, 4))
+    return float((tiles(got.double() - want) / tiles(want)).max().sqrt())
+
+
+# A rounding to bf16 is at most 2^-9 of the value, so a sum of 16 x 32 values and more that took three of them (operands of
+# the products, chunk states, the result) is off by less than that many of its norm.  One position left out of 128
+# comparable ones is 2^-3.5 of a row, 2^-5.5 of a tile
+TILE = 3 * 2.0 ** -9
+
+
 def _reference(dt, A, B, C, D, g, seq):
     """dx and the sum of its absolute terms."""
     b, L, H, P = g.shape
@@ -52,6 +65,7 @@ def test_dx(b, L, H, G, P, N, Q, packed, D_form):
     # the weighted products or the chunk states' gradients, and the result, are rounded to bf16: at most 2^-8 of each, twice
     err = (x.grad.double() - want).abs()
     assert bool((err <= 2 * 2.0 ** -8 * size + 1e-30).all()), float((err / (size + 1e-30)).max())
+    assert _worst_tile(x.grad, want) < TILE
     if D is not None:  # of x and g as they are: fp32 sums of b L (and P) terms
         terms = x.detach().double() * g.double()
         dims = (0, 1) if D.dim() == 2 else (0, 1, 3)

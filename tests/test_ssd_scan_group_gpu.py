@@ -8,6 +8,19 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+def _worst_tile(got, want):
+    """The largest error of 16 positions of one head (or group), as a share of their norm.  (Whole tiles: the one or few terms
+    of a single position can cancel, and leave a result that is small beside the rounding of each.)"""
+    tiles = lambda t: t[:, :t.shape[1] // 16 * 16].double().unflatten(1, (-1, 16)).pow(2).sum((2, 4))
+    return float((tiles(got.double() - want) / tiles(want)).max().sqrt())
+
+
+# A rounding to bf16 is at most 2^-9 of the value, so a sum of 16 x 32 values and more that took three of them (operands of
+# the products, chunk states, the result) is off by less than that many of its norm.  One position left out of 128
+# comparable ones is 2^-3.5 of a row, 2^-5.5 of a tile
+TILE = 3 * 2.0 ** -9
+
+
 # (every problem has more workgroups than a card of 256 CUs)
 @pytest.mark.parametrize("b,L,H,G,P,N,Q", [
     (2, 1025, 16, 8, 64, 128, 64), (4, 1024, 40, 10, 32, 128, 64), (1, 3025, 18, 6, 64, 64, 64), (3, 511, 64, 64, 32, 64, 64),
@@ -73,3 +86,5 @@ def test_scan(b, L, H, G, P, N, Q, gate, pre, D_form, packed):
     g = torch.nn.functional.silu(z.double())
     assert close(out, y * g, size * g.abs()) if gate else close(out, y, size)
     assert close(out_x, y, size) if gate and pre else bool((out_x == 7).all())
+    assert _worst_tile(out, y * g if gate else y) < TILE
+    assert not (gate and pre) or _worst_tile(out_x, y) < TILE

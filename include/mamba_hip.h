@@ -434,7 +434,7 @@ int ssd_bwd_dz(const SsdParams *p, mamba_stream_t stream);
  * a bad argument.  Clearing a buffer that is reported here is harmless.  No
  * counterpart in the reference, whose Triton kernels write partial sums to fresh buffers and add them up with
  * torch (mamba_ssm/ops/triton/ssd_combined.py:441-509). */
-#define SSD_OVERWRITES_DCB 1 /* dCB: one workgroup sums over all heads of a group (at most 16 of them) */
+#define SSD_OVERWRITES_DCB 1 /* dCB: one workgroup sums over all heads of a group (up to 16, more where the chunks alone fill the chip) */
 #define SSD_OVERWRITES_DBC 2 /* dB32 and dC32: one workgroup of the state-path stage holds all heads of a group */
 #define SSD_BWD_FORMS_CB 4   /* not about clearing: the backward pass does not need CB from the caller (who may skip
                                 ssd_bmm_chunk_fwd and pass CB = NULL): the dCB stage forms its tiles of C B^T itself and

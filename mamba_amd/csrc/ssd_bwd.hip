@@ -1886,11 +1886,13 @@ static bool dcb_rows_ok(const SsdParams *p) {
 // us, fitted to both at 37 sizes (4 - 1128 chunks x groups, 2 - 80 heads per group; most within 20 %).  The triangle: a
 // round of one, two or four workgroups per CU (chunks of 256, 128, 64) takes `fixed` and `head` for every head of a list,
 // a workgroup `store` for its sums, a quarter of that where it owns them.  The tile pairs: four workgroups per CU, a round
-// 9 and 1.0 to 2.6 (the CUs full) per head.  256 positions, 80 heads x 64 chunks: 161 -> 108 us in 4 lists; 8 groups of 8
-// heads x 128: 266 -> 204; 48 heads x 32 chunks: 47 against 56, the tile pairs stay; chunks of 128, 32 heads x 10: 17 ->
-// 15; chunks of 64, 16 heads x 77: 25 -> 13.
-// Groups of up to 16 heads are one list, whose sums need no clearing and go on as bf16, but for chunks of up to 128 with
-// more than 8 heads, where several lists pay (at 256: 25.4 against 25.3 us for 16 heads x 13 chunks).
+// 9 and 1.0 to 2.6 (the CUs full) per head.  The stage in turn with itself, tile pairs / triangle: 256 positions, 80 heads x 64
+// chunks 173 / 124 us (4 lists); 8 groups of 8 heads x 128 272 / 210; 48 heads x 32 chunks 47 / 56, the tile pairs stay;
+// chunks of 64, 16 heads x 77: 25 / 15.
+// One list stores its sums whole, which need no clearing and go on as bf16.  Groups of up to 16 heads are one list, but for
+// chunks of up to 128 with more than 8 heads, where several lists may pay (at 256: 25.4 against 25.3 us for 16 heads x 13
+// chunks).  Larger groups, which the tile pairs would cut (16 heads are their limit), are one list where their chunks alone
+// fill the chip: 2 groups of 40 heads x 128 chunks.
 struct DcbPlan {
   bool chunk;
   int lists;
@@ -2165,9 +2167,9 @@ extern "C" int ssd_bwd_overwrites(const SsdParams *p) {
   if (plan.lists == 1) flags |= SSD_OVERWRITES_DCB;
   if (ssd_bwd_dbc_fused_owns(p)) flags |= SSD_OVERWRITES_DBC;
   // CB: only the dCB stage and the tiled dx kernel read it.  Where the fused dx kernel runs, the dCB stage can form its
-  // tiles itself, once per head list, in less time than it takes to read them (the tile pairs, 5 lists of 16 heads x 64
-  // chunks: 161 against 174 us with CB, and 8 for the launch that forms it).  Short problems in more than 12 lists keep the
-  // answer their callers have always had.
+  // tiles itself, once per head list, in no more time than the launch that forms CB takes (80 heads x 64 chunks, the triangle:
+  // 124 us against 113 with CB and 9 for that launch; the tile pairs: 173 against 169 and 9).  Short problems in more than
+  // 12 lists keep the answer their callers have always had.
   if (ssd_bwd_dx_fused_supported(p) && (plan.lists == 1 || (dcb_rows_ok(p) && plan.lists <= 12))) flags |= SSD_BWD_FORMS_CB;
   return flags;
 }

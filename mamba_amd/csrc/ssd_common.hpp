@@ -902,12 +902,15 @@ __attribute__((visibility("hidden"))) int ssd_bwd_dcb_chunk_launch(const SsdPara
 // ---- host side of the kernels that work through the heads of a group in one workgroup
 inline bool aligned(const void *ptr, int a) { return (reinterpret_cast<uintptr_t>(ptr) % a) == 0; }
 
-// Heads per workgroup: a divisor of the heads per group, 20 at most.  One workgroup fills a CU, so the launch runs in
-// ceil(workgroups / CUs) rounds, each as long as what a workgroup pays once (launch, arguments, C rows, the first
-// head's exposed memory latency: measured at about 0.15 of a head's work) plus its heads; the divisor with the
-// shortest estimate wins.
+// Heads per workgroup: a divisor of the heads per group, 20 at most.  The launch runs in ceil(workgroups / slots) rounds,
+// each as long as what a workgroup pays once (launch, arguments, C rows, the first head's exposed memory latency: measured
+// at about 0.15 of a head's work) plus its heads; the divisor with the shortest estimate wins.  Slots and that share were
+// measured on the forms of which one workgroup fills a CU: the scans of ssd_scan_fused.hip and ssd_scan_paired.hip, and the dx
+// kernel at chunk 256.  At chunks of 64 and 128 the dx kernel (ssd_dx_fused.hip) and the scan that keeps C B^T of the group
+// (ssd_scan_group.hip) have two and more workgroups on a CU with 128 states too, and the estimate counts too few slots for
+// them: their lists are longer than need be where a launch is short.
 inline int heads_per_workgroup(const SsdParams &p) {
-  // (with 64 states and chunks of up to 128 two workgroups share a CU; with 128 states the registers allow one)
+  // (with 64 states and chunks of up to 128 two workgroups of the former share a CU; with 128 states the registers allow one)
   const int hpg = p.nheads / p.ngroups, slots = cu_count() * (p.chunk_size <= 128 && p.dstate <= 64 ? 2 : 1);
   const int64_t tiles = (int64_t)p.nchunks * p.batch;
   int best = 1;

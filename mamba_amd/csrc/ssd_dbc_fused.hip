@@ -385,7 +385,9 @@ __global__ __launch_bounds__(64 * WV, WV == 4 && PT * NK == 16 ? 3 : 4) void bwd
 }
 
 // Heads per workgroup for that launch: a divisor of the heads per group, MAXHB at most, by the same estimate as
-// heads_per_workgroup with the fixed cost these kernels measure (prologue and final adds: about 8 heads' worth).
+// heads_per_workgroup with a fixed cost of 8 heads for the prologue and the final adds.  Both terms were measured on an earlier
+// form, one workgroup of up to 16 waves per CU and chunk; this one has two or three on a CU, and two for a chunk of 256, so
+// that the estimate is an order of the candidates rather than their times.
 inline int dbc_heads_per_workgroup(const SsdParams &p) {
   const int hpg = p.nheads / p.ngroups, cus = cu_count();
   const int64_t tiles = (int64_t)p.nchunks * p.batch;

@@ -11,11 +11,11 @@
 // operands lie two heads deep in LDS.
 // What bounds it: the waves' own instructions (4 batch rows x 4096 positions x 80 heads x 64, 20 heads per workgroup: some
 // wave of a SIMD issues in 83 % of the cycles, ~1000 instructions per head and wave, 20 vector ones per block for the four
-// weights of a lane; the matrix cores are busy in 10 %, the LDS in 28 %).  4.4 us per head there, 3.8 TB/s; 174 -> 108 us
-// with the launch that formed C B^T gone as well (8 us); 32768 positions x 64 heads in 8 groups: 291 -> 204.  Tried and
-// not kept: column sums added with LDS atomics (172 us); ddA_cumsum stored instead of added with atomics, both operands
-// requested at the start of a head instead of one in each half (122 - 130); factors selected instead of the one branch
-// where a wave passes from its long to its short row (119 against 118).
+// weights of a lane; the matrix cores are busy in 10 %, the LDS in 28 %).  5 us per head there, 3.5 TB/s; within a backward
+// pass 172 -> 119 us, with the launch that formed C B^T gone as well (9 us); 32768 positions x 64 heads in 8 groups: 298 ->
+// 208 (4.1 TB/s).  Tried and not kept: column sums added with LDS atomics (172 us); ddA_cumsum stored instead of added with
+// atomics, both operands requested at the start of a head instead of one in each half (122 - 130); factors selected instead
+// of the one branch where a wave passes from its long to its short row (119 against 118).
 #include "ssd_common.hpp"
 
 namespace {

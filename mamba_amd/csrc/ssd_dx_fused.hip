@@ -14,11 +14,12 @@
 // first a of the l tile (both exponents <= 0): one multiply per element and one exponential per lane and tile; the pair of
 // tiles with the diagonal uses the exact form.  x comes and dx leaves as whole pieces of rows, through a patch per wave.
 //
-// What bounds it: memory, 3.9 TB/s through g, x, the state gradients and dx at 128-byte rows (a bare pass in that order
-// reaches 4.6); of the time, the causal products are 15 %.  Forming S for every head (544 of a head's 1088 MFMAs and 57 % of
-// its LDS reads), g and the state gradient through registers between three barriers, and x in 8-byte pieces of 16 rows (a
-// quarter of the time) cost: 16384 positions, 128 heads, chunk 256: 338 -> 247 us; 4 x 4096, 80 heads, chunk 256: 186 -> 147;
-// 2 x 4096, 40 heads, chunk 128: 57 -> 41.  Requesting x a head ahead is slower (263, 152), streaming stores too (266, 164).
+// What bounds it: memory, 4.4 TB/s (4 x 4096, 80 heads) and 4.6 (32768 positions, 64 heads in 8 groups) through g, x, the
+// state gradients and dx at 128-byte rows (a bare pass in that order reaches 4.5 - 4.7); of the time, the causal products
+// are 15 %.  Forming S for every head (544 of a head's 1088 MFMAs and 57 % of its LDS reads), g and the state gradient
+// through registers between three barriers, and x in 8-byte pieces of 16 rows (a quarter of the time) cost: 16384
+// positions, 128 heads, chunk 256: 338 -> 247 us; 4 x 4096, 80 heads, chunk 256: 186 -> 147; 2 x 4096, 40 heads, chunk 128:
+// 57 -> 41.  Requesting x a head ahead is slower (263, 152), streaming stores too (266, 164).
 #include "ssd_common.hpp"
 
 namespace {

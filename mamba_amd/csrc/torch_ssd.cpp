@@ -69,19 +69,22 @@ bool fill_ssd(SsdParams &p, SsdDims &d, const at::Tensor &x, const at::Tensor &d
 // dCB per group above all, which a call without gradients does not have, and more workgroups.  The named chunk stays unless
 // another one was faster in about every call of its class.  W: the workgroups a chunk of 256 gives, one per head.
 // Measured (64 / 128 / 256, us, bf16, headdim 64, gated; forward | forward + backward; g: groups, n: states):
-//   1 x 777 x 24       g1 n128  W 96     26.2 / 21.5 / 24.8  |  92 / 93 / 118      few workgroups: not 256
-//   1 x 4096 x 48      g8 n64   W 768    63.4 / 48.0 / 43.1  |  239 / 201 / 214    64 states, 8 groups: 256 without gradients,
-//   2 x 7093 x 40      g8 n64   W 2240   170 / 127 / 122     |  628 / 543 / 573      128 with them,
-//   1 x 32768 x 64     g8 n64   W 8192   569 / 421 / 369     |  2093 / 1742 / 1698   until the states outweigh the tiles
-//   1 x 1531 x 80      g1 n64   W 480    39.6 / 32.7 / 32.5  |  171 / 155 / 160    1 group: the tiles weigh less
-//   4 x 4096 x 16      g1 n64   W 1024   81 / 61 / 54        |  315 / 273 / 274
-//   2 x 7093 x 40      g1 n128  W 2240   264 / 205 / 147     |  747 / 638 / 561    128 states: the states weigh twice
-//   1 x 4039 x 72      g8 n128  W 1152   129 / 99 / 103      |  403 / 339 / 382    4.5 rounds of 256 CUs: half of one idle
-//   1 x 32768 x 64     g8 n128  W 8192   913 / 656 / 487     |  2767 / 2202 / 1971
+//   1 x 777 x 24       g1 n128  W 96     27.2 / 21.6 / 26.1  |  90 / 89 / 117      few workgroups: not 256
+//   1 x 4096 x 48      g8 n64   W 768    58.1 / 44.8 / 43.5  |  208 / 180 / 194    64 states, 8 groups: 256 without gradients,
+//   2 x 7093 x 40      g8 n64   W 2240   181 / 124 / 116     |  567 / 473 / 481      128 with them,
+//   1 x 32768 x 64     g8 n64   W 8192   571 / 422 / 367     |  1954 / 1619 / 1524   until the states outweigh the tiles
+//   1 x 1531 x 80      g1 n64   W 480    38.9 / 32.8 / 32.5  |  162 / 153 / 160    1 group: the tiles weigh less
+//   4 x 4096 x 16      g1 n64   W 1024   72 / 56 / 52        |  299 / 262 / 267
+//   2 x 7093 x 40      g1 n128  W 2240   274 / 190 / 142     |  760 / 582 / 516    128 states: the states weigh twice
+//   1 x 4039 x 72      g8 n128  W 1152   128 / 90 / 96       |  375 / 293 / 365    4.5 rounds of 256 CUs: half of one idle
+//   1 x 32768 x 64     g8 n128  W 8192   898 / 590 / 484     |  2588 / 1943 / 1681
 // Over 279 sizes (1 - 4 x 130 - 32768 x 16 - 80 heads, 1 and 8 groups, 64 and 128 states, gated or not) a call without
-// gradients that names 64 / 128 / 256 takes 0.79 / 0.93 / 0.97 of the named chunk's time in the mean and 1.04 / 1.10 / 1.11 at
-// worst (calls of 25 - 45 us), one with gradients 0.90 / 0.99 / 0.94 and 1.08 / 1.03 / 1.03.  Operands in two
-// halves, and sizes that the fused kernels do not take: 128, or a named 64 in a short call (80 sizes: 0.93 / 1.00 / 0.92).
+// gradients that names 64 / 128 / 256 takes 0.80 / 0.96 / 0.97 of the named chunk's time in the mean and 1.13 / 1.15 / 1.13
+// at worst (calls of 25 - 45 us), one with gradients 0.89 / 1.00 / 0.98 and 1.02 / 1.20 / 1.05.  The lines were drawn
+// before the kernels of chunks of 64 and 128 became faster: with gradients a named 128 that goes to 256 is the slower one
+// at 128 states without a gate (1 x 19504 x 40, 8 groups: 797 against 663 us) and at short calls of one group (3 x 1805 x
+// 48: 341 / 301). Operands in two halves, and sizes that the fused kernels do not take: 128, or a named 64 in a short call
+// (80 sizes: 0.93 / 1.00 / 0.92).
 int64_t kernel_chunk(int64_t named, int64_t batch, int64_t L, int64_t H, int64_t G, int64_t P, int64_t N, at::ScalarType type,
                      bool backward) {
   if (named != 64 && named != 128 && named != 256) return named;

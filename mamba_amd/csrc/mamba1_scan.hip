@@ -948,9 +948,13 @@ size_t fwd_min_lds() {
 // The forward kernel that serves a problem and its estimated time in us, for 16 states.  scan_fwd_serial_kernel
 // (mamba1_scan_serial.hip) takes 16 states and per-position B and C; up to five of its workgroups share a CU, and a tile
 // (half tiles where the sequence ends in one) takes a round of them 7.3, 10.7, 14.1, 17.5, 20.9.  scan_fwd_kernel: up to
-// two per CU, 6.6 or 10.9, and a seventh more of that on rows with a ragged end.  Measured, 8 x 5120 channels x 4096 positions bf16: 806 -> 660 us; 8 x 2368 x 8086: 1235 -> 971;
-// 7 x 3184 x 192: 35 -> 24; a workgroup per CU or less and the sequence whole: 108 against 119 (2 x 4096 x 2048), the
-// kernel with the lanes along the sequence stays; cut into more segments (below) the other one serves those too.
+// two per CU, 6.6 or 10.9, and a seventh more of that on rows with a ragged end.  Measured, 8 x 5120 channels x 4096
+// positions bf16: 806 -> 660 us; 8 x 2368 x 8086: 1235 -> 971; 7 x 3184 x 192: 35 -> 24; a workgroup per CU or less and the
+// sequence whole: 108 against 119 (2 x 4096 x 2048), the kernel with the lanes along the sequence stays; cut into more
+// segments (below) the other one serves those too.
+bool serial_takes(const MambaScanParams &p) {
+  return p.dstate == NB16 && !(p.bc_const & 3) && !p.a_complex && !k4_mode() && !fwd_min_lds() && p.seqlen >= KI;
+}
 struct FwdCost {
   bool serial;
   double us;
@@ -958,11 +962,15 @@ struct FwdCost {
 FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
   const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
   const int64_t wgs = (int64_t)p.batch * p.ngroups * ((Dg + PASS_CH - 1) / PASS_CH) * nseg;
-  const double tiles = nseg > 1 ? (double)((ntiles + nseg - 1) / nseg) : 0.5 * ((p.seqlen + TILE / 2 - 1) / (TILE / 2));
+  const int per = (ntiles + nseg - 1) / nseg;
+  if (!serial_takes(p)) {
+    const double rounds = (double)((wgs + 2 * cus - 1) / (2 * cus));
+    return {false, 6.4 * rounds * (wgs > cus ? 1.47 : 1.0) * ((p.dstate + NB16 - 1) / NB16) * per + 2.0 * rounds};
+  }
+  const double tiles = nseg > 1 ? (double)per : 0.5 * ((p.seqlen + TILE / 2 - 1) / (TILE / 2));
   const int64_t pairs = wgs / (2 * cus), odd = wgs - pairs * 2 * cus;
   const double round = (10.9 * (double)pairs + (odd > cus ? 10.9 : odd > 0 ? 6.6 : 0.0)) * (p.seqlen % KI ? 1.15 : 1.0);
-  const FwdCost lanes{false, round * ((p.dstate + NB16 - 1) / NB16) * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
-  if (p.dstate != NB16 || (p.bc_const & 3) || p.a_complex || k4_mode() || fwd_min_lds() || p.seqlen < KI) return lanes;
+  const FwdCost lanes{false, round * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
   const int64_t fives = wgs / (5 * cus), rest = (wgs - fives * 5 * cus + cus - 1) / cus;
   const FwdCost serial{true, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + (p.seqlen % KI ? 3.4 : 2.0)};
   return serial.us < lanes.us ? serial : lanes;
@@ -974,6 +982,10 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
 // third of that for what the passes share, a round's start and end 5.3.  The pass over the segments (all but one) takes 2.7
 // (forward) or 4.5 (backward) a tile, twice that from four of its workgroups per CU on, and every segment 0.9 or 1.8 for
 // its launch and for going through the segments before it.  A split has to promise 1 % (forward) or 6 % (backward).
+// Forward scans that only scan_fwd_kernel takes (fwd_cost) keep the terms that were fitted to them: 6.4 a tile of a round of up
+// to two workgroups per CU, half as much again where two share one, 3.0 for a tile of the pass over the segments, 6 % to
+// promise.  (The terms for 16 states cut them too finely: 2 x 4160 x 1261, 4 states, 53 us whole and 70 in five segments; 2 x
+// 1552 x 4029, 64 states, 420 us in five and 501 in 32.)
 // Measured: 1536 channels x 777 positions of one sequence 50 -> 24 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181
 // forward; 1536 channels whole and in two segments: 14.8 and 14.8 (129 positions), 13.1 and 14.6 (192), 16.6 and 15.0 (256).
 constexpr int MAX_SEGMENTS = 32;
@@ -983,6 +995,7 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
   const int64_t seg_wgs = rows * ((Dg + SEG_CH - 1) / SEG_CH);
   if (p.a_complex || p.batch > 65535 || k4_mode() || use_mx(p)) return 1;
   const int blocks = (p.dstate + NB16 - 1) / NB16;
+  const bool fine = !bwd && serial_takes(p);
   int best = 1;
   double best_cost = -1.0;
   for (int s = 1; s <= std::min(ntiles, MAX_SEGMENTS); ++s) {
@@ -1000,7 +1013,7 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
     }
     if (s > 1) {
       const double share = std::max(1.0, 0.52 * (double)((seg_wgs * (s - 1) + cus - 1) / cus));
-      cost = (bwd ? 1.06 : 1.01) * (cost + (bwd ? 4.5 : 2.7) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
+      cost = (fine ? 1.01 : 1.06) * (cost + (bwd ? 4.5 : fine ? 2.7 : 3.0) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
     }
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = s;
   }

@@ -326,7 +326,12 @@ template <int PT, int NK, bool GATED> int launch_q(const SsdParams &p, hipStream
   const dim3 grid(p.nheads / hb, p.nchunks, p.batch);
   switch (p.chunk_size) {
     case 128: hipLaunchKernelGGL((chunk_scan_fwd_group_kernel<PT, NK, 8, GATED>), grid, dim3(512), 0, s, p, hb); break;
-    case 64: hipLaunchKernelGGL((chunk_scan_fwd_group_kernel<PT, NK, 4, GATED>), grid, dim3(256), 0, s, p, hb); break;
+    case 64:
+      if constexpr (!GATED || PT * NK < 16) {  // (not served, below)
+        hipLaunchKernelGGL((chunk_scan_fwd_group_kernel<PT, NK, 4, GATED>), grid, dim3(256), 0, s, p, hb);
+        break;
+      }
+      return MAMBA_E_UNSUPPORTED;
     default: return MAMBA_E_UNSUPPORTED;
   }
   return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
@@ -343,12 +348,20 @@ template <int PT, int NK> int launch_z(const SsdParams &p, hipStream_t s) {
 // Whether this form serves a problem that ssd_chunk_scan_fwd_fused_supported accepts, and is the faster one: chunks of 64 and
 // 128 (at 256 the two tiles per wave of ssd_scan_paired.hip take 310 us against 342, 32768 positions x 64 heads; 179 against 191,
 // 4 x 4096 x 80), more workgroups than CUs (two of them share one; with fewer the one-tile form is 2 % faster), and not 64 states
-// with a gate (185 us for a forward pass of 4 x 4096 x 48 heads against 201).  Forward passes with gradients, one-tile form /
-// this: 2 x 4096 x 16 heads in 8 groups 61.7 / 54.6 us gated, 57.6 / 50.6 not; x 40 heads 122 / 113, 108 / 88; 4 x 4096 x 24 in
-// 4, 64 states, no gate 80 / 73.  (Offsets in a chunk are 32-bit.)
+// with a gate (185 us for a forward pass of 4 x 4096 x 48 heads against 201).  C B^T of the group pays by the heads of a list.
+// The stage alone, 900 sizes (1 - 4 x 64 - 16384 x 8 - 96 heads in 1 - 8 groups), time of the one-tile form / of this one by the
+// heads of a list, 1 | 2 | 3 | 4 and more:
+//   chunk 128, headdim 64, 128 states      1.19 | 1.44 | 1.46 | 1.55;  with a gate 1.12 | 1.24 | 1.23 | 1.12
+//   chunk 128, less than that              0.80 - 0.84 | 0.95 - 0.99 | 1.01 - 1.10 | 1.02 - 1.3
+//   chunk 64, headdim 64, 128 states       0.82 | 0.92 | 1.02 | 1.06;  with a gate 0.83 | 0.94 | 1.00 | 0.99
+//   chunk 64, less than that               0.93 | 1.02 - 1.06 | 1.04 - 1.10 | 1.01 - 1.2
+// (Offsets in a chunk are 32-bit.)
 bool ssd_scan_group_serves(const SsdParams &p) {
   if (p.chunk_size > 128 || (p.z && p.dstate <= 64) || !p.states_lp) return false;
-  if ((int64_t)p.nheads / heads_per_workgroup(p) * p.nchunks * p.batch <= cu_count()) return false;
+  const int hb = heads_per_workgroup(p);
+  if ((int64_t)p.nheads / hb * p.nchunks * p.batch <= cu_count()) return false;
+  const bool full = p.headdim == 64 && p.dstate == 128;
+  if (p.chunk_size > 64 ? !full && hb < 3 : full ? p.z || hb < 4 : hb < 2) return false;
   return near_rows(p.x_ls) && near_rows(p.B_ls) && near_rows(p.out_ls) && (!p.z || near_rows(p.z_ls));
 }
 

@@ -1,7 +1,7 @@
 """The forward chunk scan that keeps C B^T of the group (ssd_scan_group.hip): chunks of 64 and 128, state counts and headdims,
 lists of one and of several heads, a last chunk of 1, 17 and Q - 1 positions, packed sequences, with and without gate, pre-gate
-copy and D.  (64 states with a gate are left to the one-tile form of ssd_scan_fused.hip: the same check of that one.)  Reference:
-the stage's formula in float64 on the same bf16 operands."""
+copy and D.  (64 states, or chunks of 64 with 128 states, with a gate are left to the one-tile form of ssd_scan_fused.hip: the
+same check of that one.)  Reference: the stage's formula in float64 on the same bf16 operands."""
 import pytest
 import torch
 
@@ -21,10 +21,14 @@ def _worst_tile(got, want):
 TILE = 3 * 2.0 ** -9
 
 
-# (every problem has more workgroups than a card of 256 CUs)
+# (every problem has more workgroups than a card of 256 CUs; those whose lists are too short for this form, see
+# ssd_scan_group_serves, are the same check of the one-tile form)
 @pytest.mark.parametrize("b,L,H,G,P,N,Q", [
     (2, 1025, 16, 8, 64, 128, 64), (4, 1024, 40, 10, 32, 128, 64), (1, 3025, 18, 6, 64, 64, 64), (3, 511, 64, 64, 32, 64, 64),
     (4, 2048, 24, 8, 64, 128, 128), (2, 1169, 48, 16, 64, 64, 128), (2, 2047, 40, 20, 32, 128, 128), (9, 129, 32, 32, 32, 64, 128),
+    # lists of 8, 2, 8, 8 heads (chunk 64), of 4, 8, 4 (chunk 128)
+    (4, 2047, 64, 8, 64, 128, 64), (4, 1025, 64, 8, 32, 128, 64), (4, 1937, 64, 8, 64, 64, 64), (4, 1985, 64, 8, 32, 64, 64),
+    (4, 1169, 96, 8, 64, 64, 128), (4, 2047, 64, 8, 32, 128, 128), (4, 1937, 96, 6, 32, 64, 128),
 ])
 @pytest.mark.parametrize("gate,pre,D_form,packed", [(False, False, "head", False), (False, False, "none", True), (True, True, "channel", True), (True, False, "head", False)])
 def test_scan(b, L, H, G, P, N, Q, gate, pre, D_form, packed):

@@ -32,14 +32,13 @@ OPEN = (-float("inf"), float("inf"))
 
 # more workgroups than a card of 256 CUs, one tile per wave and the group's C B^T kept, and few workgroups; two tiles per wave
 @pytest.mark.parametrize("b,L,H,G,P,N,Q", [
-    (1, 2048, 40, 8, 64, 128, 64), (2, 2047, 80, 16, 64, 64, 64), (3, 2001, 40, 20, 32, 128, 128), (4, 2048, 24, 8, 64, 128, 128),
+    (4, 2047, 64, 8, 64, 128, 64), (2, 2047, 80, 16, 64, 64, 64), (4, 2001, 64, 8, 32, 128, 128), (4, 2048, 24, 8, 64, 128, 128),
     (1, 1000, 8, 1, 64, 128, 128), (2, 1024, 40, 1, 64, 128, 256),
 ])
 def test_forward(b, L, H, G, P, N, Q):
-    from mamba_amd.ops.triton.ssd_combined import mamba_chunk_scan_combined
+    from mamba_amd.ops.triton.ssd_combined import _mamba_chunk_scan_combined_fwd
     x, dt, A, B, C, _ = _inputs(b, L, H, G, P, N)
-    x.requires_grad_()  # (the chunk that is named)
-    y = mamba_chunk_scan_combined(x, dt, A, B, C, Q, dt_limit=OPEN).detach().double()
+    y = _mamba_chunk_scan_combined_fwd(x, dt, A, B, C, Q, dt_limit=OPEN)[0].double()  # (keeps the chunk that is named)
     want = _reference(*[t.detach().double() for t in (x, dt, A, B, C)])
     assert float((y - want).norm() / want.norm()) <= BOUND
 

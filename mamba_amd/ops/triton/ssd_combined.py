@@ -263,7 +263,7 @@ def _mamba_chunk_scan_combined_bwd(dout, x, dt, A, B, C, out, chunk_size, D=None
     lib = _lib.load()
     with torch.cuda.device(dev):
         owned = lib.ssd_bwd_overwrites(p)  # which of the large sum buffers the kernels store rather than add into
-        if owned == 0:
+        if not owned & 3:
             arena.zero_()  # one fill
         else:
             arena[:n_small].zero_()

@@ -59,3 +59,20 @@ def test_uncleared_sum_buffers(monkeypatch, H, G, L, Q, expect, packed, host):
         floor = 4e-3 * float(want.abs().max()) if k in ("A", "D", "dt_bias") else 0.0
         err = (got - want).abs()
         assert bool((err <= f * (5e-2 + 3e-2 * want.abs()) + floor).all()), f"d{k}: max err {float(err.max()):.3e}"
+
+
+def test_one_fill_where_no_buffer_is_owned(monkeypatch):
+    """5 lists of a group (no buffer is stored whole) whose dCB kernel forms C B^T: the Python host side clears the arena at once."""
+    from mamba_amd import _lib
+    from mamba_amd.ops.triton import ssd_combined as sc
+    lib = _lib.load()
+    seen, fills, real, fill = [], [], lib.ssd_bwd_overwrites, torch.Tensor.zero_
+    monkeypatch.setattr(_lib, "torch_ext", lambda: None)
+    monkeypatch.setattr(lib, "ssd_bwd_overwrites", lambda p: seen.append(real(p)) or seen[-1])
+    monkeypatch.setattr(torch.Tensor, "zero_", lambda t: fills.append(t.shape) or fill(t))
+    t = ssd_inputs(4, 1024, 80, 64, 128, 1, torch.bfloat16, 12)
+    g = {k: t[k].cuda().requires_grad_() for k in NAMES}
+    out = sc.mamba_chunk_scan_combined(g["x"], g["dt"], g["A"], g["B"], g["C"], 256, D=g["D"], z=g["z"], dt_bias=g["dt_bias"], dt_softplus=True)
+    del fills[:]
+    out.backward(t["dout"].cuda())
+    assert seen == [4] and len(fills) == 1, (seen, fills)

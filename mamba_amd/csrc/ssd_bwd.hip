@@ -1677,10 +1677,12 @@ DEVI void chunk_cumsum_bwd_body(const SsdParams &p, int bx, int by, int bz, int 
 }
 
 // On its own: as many chunks per workgroup as 16 waves hold, which is that many fewer atomics on the few addresses of dA and
-// ddt_bias (64 chunks of 128 x 40 heads: 12 -> 10 us; 128 of 256 x 64 unchanged).
-constexpr int CSB_WAVES = 16;
-__global__ __launch_bounds__(64 * CSB_WAVES) void chunk_cumsum_bwd_kernel(const SsdParams p) {
-  chunk_cumsum_bwd_body<CSB_WAVES>(p, blockIdx.x, blockIdx.y, blockIdx.z, (p.chunk_size + 63) / 64);
+// ddt_bias (64 chunks of 128 x 40 heads: 12 -> 10 us; 128 of 256 x 64 unchanged).  Where there are few (chunk, 4 heads) pairs, the
+// atomics are few as well and a workgroup's own time counts: one chunk in 4 waves (600 sizes: 4.6 - 5.5 us against 5.3 -
+// 6.1 below 120 pairs, equal at 120 - 200, 6 - 10 against 5.8 - 6.5 from there to 500).
+constexpr int CSB_WAVES = 16, CSB_FEW = 150;
+template <int WAVES> __global__ __launch_bounds__(64 * WAVES) void chunk_cumsum_bwd_kernel(const SsdParams p, const int chunk_waves) {
+  chunk_cumsum_bwd_body<WAVES>(p, blockIdx.x, blockIdx.y, blockIdx.z, chunk_waves);
 }
 
 // The last two stages read disjoint results of the stages before them (dCB; ddA_cumsum and ddt_out) and neither
@@ -1996,9 +1998,13 @@ static int ssd_chunk_cumsum_bwd_one(const SsdParams *p, mamba_stream_t stream) {
   int rc = check_bwd(p);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  const int lot = CSB_WAVES / ((p->chunk_size + 63) / 64);
-  dim3 grid((p->nchunks + lot - 1) / lot, (p->nheads + CSB_HT - 1) / CSB_HT, p->batch);
-  hipLaunchKernelGGL(chunk_cumsum_bwd_kernel, grid, dim3(64 * CSB_WAVES), 0, s, with_grad_strides(*p));
+  const int waves = (p->chunk_size + 63) / 64, lot = CSB_WAVES / waves, hy = (p->nheads + CSB_HT - 1) / CSB_HT;
+  if ((int64_t)p->nchunks * p->batch * hy < CSB_FEW) {
+    hipLaunchKernelGGL(chunk_cumsum_bwd_kernel<4>, dim3(p->nchunks, hy, p->batch), dim3(256), 0, s, with_grad_strides(*p), 4);
+  } else {
+    const dim3 grid((p->nchunks + lot - 1) / lot, hy, p->batch);
+    hipLaunchKernelGGL(chunk_cumsum_bwd_kernel<CSB_WAVES>, grid, dim3(64 * CSB_WAVES), 0, s, with_grad_strides(*p), waves);
+  }
   return launched();
 }
 

@@ -9,7 +9,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("layout", ["dense", "rows", "odd_rows", "apart"])
-@pytest.mark.parametrize("b,L,H,Q", [(2, 1000, 8, 64), (1, 2049, 12, 256), (1, 511, 6, 128), (2, 577, 4, 192), (1, 130, 3, 256), (3, 100, 20, 48)])
+# few pairs of a chunk and four heads (a workgroup each), and 150 and more (several chunks in one)
+@pytest.mark.parametrize("b,L,H,Q", [(2, 1000, 8, 64), (1, 2049, 12, 256), (1, 511, 6, 128), (2, 577, 4, 192), (1, 130, 3, 256), (3, 100, 20, 48),
+                                     (2, 5000, 22, 64), (1, 9001, 20, 256), (1, 4999, 18, 128), (2, 3001, 17, 192), (4, 2011, 12, 48)])
 def test_cumsum(b, L, H, Q, layout, dtype):
     from mamba_amd import _lib
     lib = _lib.load()

@@ -889,6 +889,8 @@ template <int MODE = -1> DEVI void acc_add(float *dst, int64_t *shadow, int64_t 
 // no kernel for the problem (the caller then runs the tiled bwd_dx_kernel).
 __attribute__((visibility("hidden"))) int ssd_bwd_dx_fused_launch(const SsdParams *p, hipStream_t stream, bool sum_dD);
 __attribute__((visibility("hidden"))) bool ssd_bwd_dx_fused_supported(const SsdParams *p);
+// The form for short lists of heads (ssd_dx_short.hip), for the problems that ssd_bwd_dx_fused_launch gives it.
+__attribute__((visibility("hidden"))) int ssd_bwd_dx_short_launch(const SsdParams &p, hipStream_t stream, bool sum_dD);
 // The fused chunk-state dB / dC kernels (ssd_dbc_fused.hip), under the same convention (the caller then runs the
 // tiled bwd_d*_state kernels).
 __attribute__((visibility("hidden"))) int ssd_bwd_dbc_fused_launch(const SsdParams *p, hipStream_t stream);

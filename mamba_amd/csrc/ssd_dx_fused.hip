@@ -409,9 +409,26 @@ bool supported(const SsdParams *p) {
       p->C_ls % 8 || p->C_gs % 8 || p->dx_bs % 8 || p->dx_ls % 8 || p->dx_hs % 8)
     return false;
   if (!p->z && (p->dout_bs % 8 || p->dout_ls % 8 || p->dout_hs % 8)) return false;
-  if (!near_rows(p->x_ls) || !near_rows(p->dx_ls) || !near_rows(p->C_ls) || !near_rows(p->z ? (int64_t)p->nheads * p->headdim : p->dout_ls)) return false;
   if (p->batch > 65535 || p->nchunks > 65535) return false;
   return true;
+}
+
+// ssd_dx_short.hip takes lists in which forming C B^T once for all heads does not pay, and rows whose places in a chunk 32-bit
+// offsets do not reach.  The stage alone, 700 sizes (1 - 4 x 64 - 16384 x 8 - 96 heads in 1 - 8 groups), time of the short form /
+// of this one, few workgroups (up to the CUs) and many, by the heads of a list, 1 | 2 | 3 and more:
+//   headdim 64, 128 states, chunk 64    few 0.88 | 1.02 | 1.2     many 0.76 | 0.90 | 0.93 (3 heads), 0.9 - 1.2
+//                           chunk 128       0.83 | 0.95 | 1.07         1.22 | 1.33 | 1.28
+//                           chunk 256       0.84 | 1.01 | 1.2          0.88 | 1.06 | 1.13
+//   less than that,         chunk 64        0.86 - 0.89 | 1.01 | 1.2   0.91 - 0.97 | 1.02 - 1.05 | 1.03 - 1.12
+//                           chunk 128       0.80 - 0.82 | 0.96 | 1.1   0.81 - 0.85 | 0.97 - 0.99 | 1.04 - 1.16
+//                           chunk 256       0.73 - 0.82 | 0.91 - 0.98 | 1.0 - 1.3   0.76 - 0.86 | 0.93 - 1.03 | 1.04 - 1.3
+bool short_lists(const SsdParams *p) {
+  if (!near_rows(p->x_ls) || !near_rows(p->dx_ls) || !near_rows(p->C_ls) || !near_rows(p->z ? (int64_t)p->nheads * p->headdim : p->dout_ls)) return true;
+  const int hb = heads_per_workgroup(*p), Q = p->chunk_size;
+  const bool many = (int64_t)p->nheads / hb * p->nchunks * p->batch > cu_count(), full = p->headdim == 64 && p->dstate == 128;
+  if (hb == 1) return !(full && Q == 128 && many);
+  if (Q == 64) return hb <= 3 && full && many;
+  return hb == 2 && !many && (Q == 128 || !full);
 }
 
 }  // namespace
@@ -423,5 +440,6 @@ bool ssd_bwd_dx_fused_supported(const SsdParams *p) { return supported(p); }
 int ssd_bwd_dx_fused_launch(const SsdParams *p, hipStream_t stream, bool sum_dD) {
   if (!supported(p)) return MAMBA_E_UNSUPPORTED;
   if (sum_dD && (!p->dD || p->D_has_hdim || (p->det_scale && !p->det_dD))) return MAMBA_E_BADARG;
+  if (short_lists(p)) return ssd_bwd_dx_short_launch(*p, stream, sum_dD);
   return p->det_scale ? launch_p<true>(*p, stream, sum_dD) : launch_p<false>(*p, stream, sum_dD);
 }

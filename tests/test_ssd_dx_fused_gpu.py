@@ -1,4 +1,4 @@
-"""dx of the SSD backward pass (ssd_dx_fused.hip) at the edges of its tiles: each chunk length, state count and headdim, lists
+"""dx of the SSD backward pass (ssd_dx_fused.hip, and ssd_dx_short.hip for lists of one and two heads) at the edges of its tiles: each chunk length, state count and headdim, lists
 of one and of several heads, a last chunk of 1, 17 and Q - 1 positions, packed sequences, D per head, per (head, p) and none.
 Reference: the quadratic form in float64 on the same bf16 operands."""
 import pytest
@@ -46,6 +46,10 @@ def _reference(dt, A, B, C, D, g, seq):
     (2, 641, 5, 1, 64, 128, 128), (4, 1024, 40, 1, 64, 64, 128), (1, 145, 4, 4, 32, 128, 128), (2, 383, 6, 2, 32, 64, 128),
     (4, 1024, 80, 1, 64, 128, 256), (1, 1025, 6, 2, 64, 128, 256), (2, 511, 3, 1, 64, 64, 256), (1, 785, 5, 5, 32, 128, 256),
     (4, 256, 4, 1, 32, 64, 256),
+    # lists of 5 to 12 heads, one for each pair of headdim and states
+    (4, 1009, 72, 1, 64, 128, 64), (3, 1009, 72, 1, 32, 128, 64), (8, 1009, 96, 1, 64, 64, 64), (8, 977, 96, 1, 32, 64, 64),
+    (4, 1009, 72, 1, 64, 128, 128), (4, 1009, 72, 1, 32, 128, 128), (8, 1009, 96, 1, 64, 64, 128), (8, 977, 96, 1, 32, 64, 128),
+    (4, 1009, 80, 1, 64, 128, 256), (4, 1009, 80, 1, 32, 128, 256), (4, 785, 96, 1, 64, 64, 256), (4, 1023, 96, 1, 32, 64, 256),
 ])
 @pytest.mark.parametrize("packed,D_form", [(False, "head"), (True, "none"), (True, "channel")])
 def test_dx(b, L, H, G, P, N, Q, packed, D_form):
@@ -71,3 +75,23 @@ def test_dx(b, L, H, G, P, N, Q, packed, D_form):
         dims = (0, 1) if D.dim() == 2 else (0, 1, 3)
         bound = 2.0 ** -24 * (16 + 4 * (b * L * P) ** 0.5) * terms.abs().sum(dims)
         assert bool(((D.grad.double() - terms.sum(dims)).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("L,H,P,N,Q", [(130, 2, 64, 128, 64), (100, 3, 32, 64, 128), (130, 1, 64, 128, 256)])
+def test_rows_that_32_bit_offsets_do_not_reach(L, H, P, N, Q):
+    """x and the gradient of the output as rows 2^22 values apart: the same dx as from dense rows."""
+    from mamba_amd.ops.triton import ssd_combined as sc
+    gen = torch.Generator(device="cuda").manual_seed(L + Q + H)
+    randn = lambda *s: torch.randn(*s, device="cuda", generator=gen).bfloat16()
+    x, g, B, C = randn(1, L, H, P), randn(1, L, H, P), randn(1, L, 1, N), randn(1, L, 1, N)
+    dt, A = 0.1 * torch.rand(1, L, H, device="cuda", generator=gen), -(0.1 + 5 * torch.rand(H, device="cuda", generator=gen))
+    rows = torch.empty(L << 22, device="cuda", dtype=torch.bfloat16)
+    apart = lambda t, first: rows[first:].as_strided(t.shape, (L << 22, 1 << 22, P, 1)).copy_(t)
+    got = []
+    for xs, gs in ((x, g), (apart(x, 0), apart(g, 1 << 20))):
+        leaf = xs.detach().requires_grad_()
+        assert leaf.stride() == xs.stride()
+        sc.mamba_chunk_scan_combined(leaf, dt, A, B, C, Q).backward(gs)
+        got.append(leaf.grad)
+    want, _ = _reference(dt, A, B, C, None, g, None)
+    assert _worst_tile(got[1], want) < TILE and torch.equal(got[0], got[1])

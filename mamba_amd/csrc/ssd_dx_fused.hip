@@ -19,7 +19,8 @@
 // are 15 %.  Forming S for every head (544 of a head's 1088 MFMAs and 57 % of its LDS reads), g and the state gradient
 // through registers between three barriers, and x in 8-byte pieces of 16 rows (a quarter of the time) cost: 16384
 // positions, 128 heads, chunk 256: 338 -> 247 us; 4 x 4096, 80 heads, chunk 256: 186 -> 147; 2 x 4096, 40 heads, chunk 128:
-// 57 -> 41.  Requesting x a head ahead is slower (263, 152), streaming stores too (266, 164).
+// 57 -> 41. Lists of one head, for which the prologue does not pay, take ssd_dx_short.hip (short_lists, below).  Requesting
+// x a head ahead is slower (263, 152), streaming stores too (266, 164).
 #include "ssd_common.hpp"
 
 namespace {

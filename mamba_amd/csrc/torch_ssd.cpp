@@ -75,16 +75,15 @@ bool fill_ssd(SsdParams &p, SsdDims &d, const at::Tensor &x, const at::Tensor &d
 //   1 x 32768 x 64     g8 n64   W 8192   571 / 422 / 367     |  1954 / 1619 / 1524   until the states outweigh the tiles
 //   1 x 1531 x 80      g1 n64   W 480    38.9 / 32.8 / 32.5  |  162 / 153 / 160    1 group: the tiles weigh less
 //   4 x 4096 x 16      g1 n64   W 1024   72 / 56 / 52        |  299 / 262 / 267
-//   2 x 7093 x 40      g1 n128  W 2240   274 / 190 / 142     |  760 / 582 / 516    128 states: the states weigh twice
-//   1 x 4039 x 72      g8 n128  W 1152   128 / 90 / 96       |  375 / 293 / 365    4.5 rounds of 256 CUs: half of one idle
-//   1 x 32768 x 64     g8 n128  W 8192   898 / 590 / 484     |  2588 / 1943 / 1681
+//   2 x 7093 x 40      g1 n128  W 2240   274 / 190 / 142     |  748 / 581 / 515    128 states: the states weigh twice
+//   1 x 4039 x 72      g8 n128  W 1152   128 / 90 / 96       |  374 / 294 / 352    4.5 rounds of 256 CUs: half of one idle
+//   1 x 32768 x 64     g8 n128  W 8192   898 / 590 / 484     |  2558 / 1931 / 1666
 // Over 279 sizes (1 - 4 x 130 - 32768 x 16 - 80 heads, 1 and 8 groups, 64 and 128 states, gated or not) a call without
-// gradients that names 64 / 128 / 256 takes 0.80 / 0.96 / 0.97 of the named chunk's time in the mean and 1.13 / 1.15 / 1.13
-// at worst (calls of 25 - 45 us), one with gradients 0.89 / 1.00 / 0.98 and 1.02 / 1.20 / 1.05.  The lines were drawn
+// gradients that names 64 / 128 / 256 takes 0.81 / 0.96 / 0.97 of the named chunk's time in the mean and 1.12 / 1.14 / 1.12
+// at worst (calls of 25 - 45 us), one with gradients 0.89 / 1.00 / 0.97 and 1.02 / 1.16 / 1.05.  The lines were drawn
 // before the kernels of chunks of 64 and 128 became faster: with gradients a named 128 that goes to 256 is the slower one
-// at 128 states without a gate (1 x 19504 x 40, 8 groups: 797 against 663 us) and at short calls of one group (3 x 1805 x
-// 48: 341 / 301). Operands in two halves, and sizes that the fused kernels do not take: 128, or a named 64 in a short call
-// (80 sizes: 0.93 / 1.00 / 0.92).
+// at 128 states without a gate (1 x 19504 x 40, 8 groups: 770 against 663 us).  Operands in two halves, and sizes that the
+// fused kernels do not take: 128, or a named 64 in a short call (80 sizes: 0.93 / 1.00 / 0.92).
 int64_t kernel_chunk(int64_t named, int64_t batch, int64_t L, int64_t H, int64_t G, int64_t P, int64_t N, at::ScalarType type,
                      bool backward) {
   if (named != 64 && named != 128 && named != 256) return named;

@@ -697,6 +697,8 @@ typedef struct MambaGemm {
   int32_t accumulate;
   int32_t nsplit;     /* parts of the sum over k, set by mamba_gemm_plan */
 } MambaGemm;
+/* 1 where these kernels are the ones to use, 0 where a BLAS library is faster (sizes, layout and alignment decide). */
+int mamba_gemm_suits(const MambaGemm *g);
 /* Sets nsplit of each product and returns the fp32 elements of workspace the call needs (0: none), or an error. */
 int64_t mamba_gemm_plan(MambaGemm *g, int count);
 int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream_t stream);

@@ -1,12 +1,13 @@
-// Small bf16 matrix products: the projections inside a mixer (x_proj, dt_proj, out_proj and their gradients) where the
-// problem is short.  A library product costs ~18 us of host time whatever its size, more than the product itself up
+// bf16 matrix products: the projections inside a mixer (x_proj, dt_proj, out_proj and their gradients) where the problem is short
+// or a library splits it badly.  A library product costs ~18 us of host time whatever its size, more than the product itself up
 // to a few GFLOP; these cost a launch (~2 us), up to MAXG independent products share one, and operands are taken as
 // they lie (either index contiguous, any alignment of the element's size), results in bf16 or fp32.
 //
-// Tile 64 x 64 per workgroup of four waves, k in steps of 32 (the block core of the SSD kernels).  What bounds a short
-// product is the latency of its loads, not the matrix cores: the operands of the next PF steps are in flight, the LDS
-// tiles are double-buffered (one barrier a step), and a product whose tiles do not fill the chip is split along k, the
-// splits' fp32 tiles added up by a second kernel in a fixed order.
+// Three tile sizes (form_of).  64 x 64 per workgroup of four waves, k in steps of 32 (the block core of the SSD kernels): what
+// bounds a short product is the latency of its loads, not the matrix cores, so the operands of the next PF steps are in flight and
+// the LDS tiles are double-buffered (one barrier a step).  128 x 128 and 256 x 256 for larger ones, which the 64 x 64 tiles'
+// reading through the L2 would bound.  A product whose tiles do not fill the chip is split along k, the splits' fp32 tiles added
+// up by a second kernel in a fixed order.
 #include "ssd_common.hpp"
 
 namespace {
@@ -263,22 +264,23 @@ template <bool TR> struct Ring {
       if (k >= K) *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(lds + (q * 4 + wave) * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
     }
   }
-  // rows r0 + i, k = 32 kk + 8 g .. + 7
-  DEVI bf16x8_t frag(uint32_t lds, int r0, int kk, int i, int g) const {
-    if constexpr (TR) {
-      typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
-      typedef short i16x8_t __attribute__((ext_vector_type(8)));
-      const int k = kk * 32 + 8 * g + (i >> 2);
-      const uint32_t at = lds + k * 128 + (((r0 >> 3) ^ swz(k)) * 16) + (i & 3) * 8;
-      const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)at);
-      const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)(at + 4 * 128));
-      return __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    } else {
-      const int r = r0 + i;
-      return *(__attribute__((address_space(3))) bf16x8_t *)(uintptr_t)(lds + r * 128 + (((kk * 4 + g) ^ swz(r)) * 16));
-    }
-  }
 };
+
+// rows r0 + i, k = 32 kk + 8 g .. + 7 of 64 rows of a stage
+template <bool TR> DEVI bf16x8_t ring_frag(uint32_t lds, int r0, int kk, int i, int g) {
+  if constexpr (TR) {
+    typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
+    typedef short i16x8_t __attribute__((ext_vector_type(8)));
+    const int k = kk * 32 + 8 * g + (i >> 2);
+    const uint32_t at = lds + k * 128 + (((r0 >> 3) ^ Ring<TR>::swz(k)) * 16) + (i & 3) * 8;
+    const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)at);
+    const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)(at + 4 * 128));
+    return __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  } else {
+    const int r = r0 + i;
+    return *(__attribute__((address_space(3))) bf16x8_t *)(uintptr_t)(lds + r * 128 + (((kk * 4 + g) ^ Ring<TR>::swz(r)) * 16));
+  }
+}
 
 template <bool XTR, bool YTR>
 DEVI void run_ring(GemmAcc &acc, const GemmRing &sh, const Ring<XTR> &X, const Ring<YTR> &Y, int k0, int k1, int wave, int lane) {
@@ -308,8 +310,8 @@ DEVI void run_ring(GemmAcc &acc, const GemmRing &sh, const Ring<XTR> &X, const R
       bf16x8_t a[2], b[2];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        a[u] = X.frag(x, wx * 32 + u * 16, kk, i, g);
-        b[u] = Y.frag(y, wy * 32 + u * 16, kk, i, g);
+        a[u] = ring_frag<XTR>(x, wx * 32 + u * 16, kk, i, g);
+        b[u] = ring_frag<YTR>(y, wy * 32 + u * 16, kk, i, g);
       }
 #pragma unroll
       for (int tx = 0; tx < 2; ++tx)
@@ -345,7 +347,260 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const Group a) {
   store_tile(a, i, acc, tid, tile, split, mt, nt);
 }
 
-// the sum of the splits' tiles; a quarter of a tile per workgroup
+// ---- larger tiles for larger products: WX x WY waves of 16 FX x 16 FY each, operands in blocks of 64 rows, stages of WK k in a
+// ring of LDS stages filled by asynchronous loads, one barrier a stage; a stage's fragments are read while the products of the one
+// before it run.  What bounds them: up to 128 x 128 the reading through the L2 (2560 x 5120 x 32768: 13 GB, 13.6 TB/s), at 256 x 256
+// the LDS (reading 96 KB and writing 32 KB per CU and stage is as long as its products), 1.0 - 1.2 PFLOP/s.
+//   M x N x K                 us: library | 64 x 64 | 128 x 128 | 256 x 256 (with the splits that are chosen)
+//   2560 x 5120 x 32768           965   |   -   | 1198 | 832        (200 tiles on 256 CUs: 78 % of what they could do)
+//   2560 x 5120 x 16384           513   |   -   |  605 | 384
+//   192 x 5120 x 32768            234   |  156  |  121 - 138 | 124
+//   768 x 1536 x 32768            183   |  218  |   89 |  90
+//   1536 x 32768 x 48 (K short)    39   |   49  |   25 |  29
+//   2560 x 32768 x 112, added      94   |  123  |   70 |  86
+//   32768 x 2560 x 5120           650   |   -   | 1050 | 711        (left to the library)
+// Tried: fragments read in front of their own products (256 x 256: 778 - 838 us where it is 712 - 773, 128 x 128 the same), four
+// waves per SIMD of 64 x 64 (760 - 815), four stages (no change), two of 64 k at 128 x 128 (945, but 152 against 138 where K is
+// short), 128 x 192 tiles (110 - 119 where 128 x 128 takes 121 - 135, for 192 rows alone), stages taken in another order by each
+// workgroup against lines a power of two apart (no change).
+constexpr int WK = 32, BLOCK = GB * WK * 2;  // a block's stage, 4 KB: four loads of a wave
+template <int WX, int WY, int FX, int FY, int ST> struct WideTile {
+  static constexpr int waves = WX * WY, stages = ST, rx = WX * FX * 16, ry = WY * FY * 16, bx = rx / GB, by = ry / GB;
+  static constexpr int loads_x = 4 * bx / waves, loads_y = 4 * by / waves;  // of a wave and stage
+  static constexpr int stage = (bx + by) * BLOCK;
+  static_assert(rx % GB == 0 && ry % GB == 0 && loads_x * waves == 4 * bx && loads_y * waves == 4 * by, "whole loads per wave");
+};
+// An operand's blocks, one piece of 16 bytes per lane and load.  Lines: a row of WK k, or with TR a k of 64 rows.  Rows past the
+// last one and k past the end are others of the operand's own again.
+template <bool TR, int LOADS, int WAVES> struct WideRing {
+  const bf16_t *base;
+  int64_t s;
+  int K, wave, lane;
+  uint32_t off[LOADS];  // of its pieces in a whole stage, from base
+  DEVI static int swz(int l) { return TR ? ((l >> 1 & 1) | (l >> 3 & 1) << 1) << 1 : l >> 2 & 3; }
+  // load e of the stage: a quarter of block e / 4
+  DEVI int line(int e) const { return TR ? (e & 3) * 8 + (lane >> 3) : (e & 3) * 16 + (lane >> 2); }
+  DEVI int col(int e) const { return ((TR ? lane & 7 : lane & 3) ^ swz(line(e))) * 8; }
+  DEVI WideRing(const void *p, int64_t rs, int64_t ks, int row0, int all_rows, int K_, int wave_, int lane_)
+      : base(static_cast<const bf16_t *>(p) + (int64_t)row0 * rs), s(TR ? ks : rs), K(K_), wave(wave_), lane(lane_) {
+    const int rows = all_rows - row0;
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) {
+      const int e = q * WAVES + wave, r = (e >> 2) * GB;
+      off[q] = 2u * (TR ? (uint32_t)line(e) * (uint32_t)s + min(r + col(e), rows - 8) : (uint32_t)min(r + line(e), rows - 1) * (uint32_t)s + col(e));
+    }
+  }
+  DEVI void request(uint32_t lds, int k0) const {
+    const bf16_t *src = base + (TR ? (int64_t)k0 * s : (int64_t)k0);
+    const bool whole = k0 + WK <= K;
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) {
+      const int e = q * WAVES + wave;
+      const uint32_t back = whole ? 0u : TR ? (uint32_t)max(line(e) - (K - 1 - k0), 0) * (uint32_t)s * 2u : (uint32_t)max(col(e) - (K - 8 - k0), 0) * 2u;
+      load_async16(src, off[q] - back, lds + e * 1024);
+    }
+  }
+  DEVI void zero(uint32_t lds, int k0) const {
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) {
+      const int e = q * WAVES + wave;
+      if (k0 + (TR ? line(e) : col(e)) >= K) *(__attribute__((address_space(3))) u32x4 *)(uintptr_t)(lds + e * 1024 + lane * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  // rows r0 + i, k = 8 g .. + 7
+  DEVI static bf16x8_t frag(uint32_t lds, int r0, int i, int g) {
+    if constexpr (TR) {
+      typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
+      typedef short i16x8_t __attribute__((ext_vector_type(8)));
+      const int k = 8 * g + (i >> 2);
+      const uint32_t at = lds + (r0 >> 6) * BLOCK + k * 128 + (((r0 >> 3 & 7) ^ swz(k)) * 16) + (i & 3) * 8;
+      const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)at);
+      const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)(at + 4 * 128));
+      return __builtin_bit_cast(bf16x8_t, (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    } else {
+      const int r = r0 + i;
+      return *(__attribute__((address_space(3))) bf16x8_t *)(uintptr_t)(lds + r * (WK * 2) + ((g ^ swz(r)) * 16));
+    }
+  }
+};
+
+template <int FX, int FY> struct WideAcc {
+  f32x4 v[FX][FY];
+};
+template <typename W, int FX, int FY, typename X_, typename Y_>
+DEVI void run_wide(WideAcc<FX, FY> &acc, uint32_t sh, const X_ &X, const Y_ &Y, int k0, int k1, int wx, int wy, int lane) {
+  const int i = lane & 15, g = lane >> 4, n = (k1 - k0 + WK - 1) / WK;
+  constexpr int S = W::stages, LOADS = W::loads_x + W::loads_y;
+  struct Frags {
+    bf16x8_t a[FX], b[FY];
+  } even, odd;
+  auto request = [&](int slot, int j) {
+    X.request(sh + slot * W::stage, k0 + j * WK);
+    Y.request(sh + slot * W::stage + W::bx * BLOCK, k0 + j * WK);
+  };
+  auto zero = [&](int slot, int j) {
+    if (k0 + (j + 1) * WK > X.K) {
+      X.zero(sh + slot * W::stage, k0 + j * WK);
+      Y.zero(sh + slot * W::stage + W::bx * BLOCK, k0 + j * WK);
+    }
+  };
+  auto read = [&](Frags &f, int slot) {
+    const uint32_t x = sh + slot * W::stage, y = x + W::bx * BLOCK;
+#pragma unroll
+    for (int u = 0; u < FX; ++u) f.a[u] = X.frag(x, wx * (FX * 16) + u * 16, i, g);
+#pragma unroll
+    for (int u = 0; u < FY; ++u) f.b[u] = Y.frag(y, wy * (FY * 16) + u * 16, i, g);
+  };
+#pragma unroll
+  for (int j = 0; j < S; ++j)
+    if (j < n) request(j, j);
+  // the loads of a wave and stage, in order
+  if (S <= n) async_done<(S - 1) * LOADS>();
+  else async_done<0>();
+  zero(0, 0);
+  lds_barrier();
+  read(even, 0);
+  int slot = 0;
+  // Stage j's fragments are in registers; those of stage j + 1 are read under its products
+  auto step = [&](int j, const Frags &now, Frags &then) {
+    const int next = slot + 1 == S ? 0 : slot + 1;
+    if (j + S - 1 < n) async_done<(S - 2) * LOADS>();
+    else async_done<0>();
+    if (j + 1 < n) zero(next, j + 1);
+    lds_barrier();  // stage j + 1 is there, and stage j has been read
+    if (j + S < n) request(slot, j + S);
+    read(then, next);  // (behind the last stage: what lies there, for nothing)
+#pragma unroll
+    for (int tx = 0; tx < FX; ++tx)
+#pragma unroll
+      for (int ty = 0; ty < FY; ++ty) acc.v[tx][ty] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(now.a[tx], now.b[ty], acc.v[tx][ty], 0, 0, 0);
+    // (a fragment's reads, then its share of the products)
+#pragma unroll
+    for (int q = 0; q < FX + FY; ++q) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x8, FX * FY / (FX + FY), 0);
+    }
+    slot = next;
+  };
+#pragma unroll 1
+  for (int j = 0; j < n; j += 2) {
+    step(j, even, odd);
+    if (j + 1 < n) step(j + 1, odd, even);
+  }
+  lds_barrier();
+}
+
+// logical index of a workgroup of `count`, consecutive ones on one XCD
+DEVI int xcd_run(int id, int count) {
+  const int per = count / 8;
+  return id < per * 8 ? id % 8 * per + id / 8 : id;
+}
+// row and first of four columns of accumulator q = FY tx + ty
+template <int WX, int WY, int FX, int FY> DEVI void wide_place4(int q, int tid, int mt, int nt, int &m, int &n) {
+  const int lane = tid & 63, wave = tid >> 6, wx = wave % WX, wy = wave / WX;
+  m = (mt * WY + wy) * (FY * 16) + (q % FY) * 16 + (lane & 15);
+  n = (nt * WX + wx) * (FX * 16) + (q / FY) * 16 + (lane >> 4) * 4;
+}
+
+template <int WX, int WY, int FX, int FY, int ST>
+__global__ __launch_bounds__(64 * WX * WY, WX * WY == 4 ? 3 : 2) void gemm_wide_kernel(const Group a) {
+  typedef WideTile<WX, WY, FX, FY, ST> W;
+  __shared__ __align__(256) char sh[ST * W::stage];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = product_of(a, blockIdx.x);
+  const int wx = wave % WX, wy = wave / WX;
+  const MambaGemm &g = a.g[i];
+  const int ntn = (g.N + W::rx - 1) / W::rx, ntm = (g.M + W::ry - 1) / W::ry, tiles = ntn * ntm;
+  // consecutive tiles of the shorter side, which share the longer side's operand, on one XCD
+  const int count = tiles * g.nsplit, block = xcd_run(blockIdx.x - a.first[i], count);
+  const int split = block / tiles, tile = block % tiles;
+  const int mt = ntm < ntn ? tile % ntm : tile / ntn, nt = ntm < ntn ? tile / ntm : tile % ntn;
+  const int steps = (g.K + GK - 1) / GK, per = (steps + g.nsplit - 1) / g.nsplit;
+  const int k0 = min(split * per * GK, g.K), k1 = min(k0 + per * GK, g.K);
+  WideAcc<FX, FY> acc;
+#pragma unroll
+  for (int q = 0; q < FX * FY; ++q) acc.v[q / FY][q % FY] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t at = lds_address(sh);
+  auto run = [&](auto x_tr, auto y_tr) {
+    constexpr bool XTR = decltype(x_tr)::value, YTR = decltype(y_tr)::value;
+    // (a split's k ends where the next one's begins)
+    const WideRing<XTR, W::loads_x, W::waves> X(g.B, g.b_ns, g.b_ks, nt * W::rx, g.N, k1, wave, lane);
+    const WideRing<YTR, W::loads_y, W::waves> Y(g.A, g.a_ms, g.a_ks, mt * W::ry, g.M, k1, wave, lane);
+    run_wide<W>(acc, at, X, Y, k0, k1, wx, wy, lane);
+  };
+  const bool btr = g.b_ks != 1, atr = g.a_ks != 1;
+  if (btr && atr) run(std::true_type{}, std::true_type{});
+  else if (btr) run(std::true_type{}, std::false_type{});
+  else if (atr) run(std::false_type{}, std::true_type{});
+  else run(std::false_type{}, std::false_type{});
+  if (g.nsplit > 1) {
+    float *part = a.ws[i] + ((int64_t)(mt * ntn + nt) * g.nsplit + split) * (W::rx * W::ry);
+#pragma unroll
+    for (int q = 0; q < FX * FY; ++q) *reinterpret_cast<f32x4 *>(part + (q * W::waves * 64 + tid) * 4) = acc.v[q / FY][q % FY];
+    return;
+  }
+  // whole rows of 16-byte pieces where D allows, 16 rows at a time through a patch of the wave's own
+  const bool rows = g.d_dtype == MAMBA_BF16 && ((uintptr_t)g.D & 15) == 0 && g.ldd % 8 == 0 && g.N % 8 == 0;
+  if (!rows) {
+#pragma unroll
+    for (int q = 0; q < FX * FY; ++q) {
+      int m, n;
+      wide_place4<WX, WY, FX, FY>(q, tid, mt, nt, m, n);
+      store4(g, m, n, acc.v[q / FY][q % FY]);
+    }
+    return;
+  }
+  lds_barrier();
+  constexpr int COLS = FX * 16, PITCH = COLS * 2 + 16, PIECES = COLS / 8, PER = (16 * PIECES + 63) / 64;
+  static_assert(ST * W::stage >= W::waves * 16 * PITCH, "the patches lie where the stages lay");
+  const uint32_t patch = at + wave * (16 * PITCH);
+  const int n0 = (nt * WX + wx) * COLS, m0 = (mt * WY + wy) * (FY * 16);
+  typedef __attribute__((address_space(3))) u32x4 *lds_u4;
+  typedef __attribute__((address_space(3))) u32x2 *lds_u2;
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  f32x4 bias[FX];
+#pragma unroll
+  for (int tx = 0; tx < FX; ++tx) {
+    bias[tx] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (g.bias) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) bias[tx][e] = ld1<bf16_t>(static_cast<const bf16_t *>(g.bias) + min(n0 + tx * 16 + (lane >> 4) * 4 + e, g.N - 1));
+    }
+  }
+#pragma unroll
+  for (int ty = 0; ty < FY; ++ty) {
+    auto pieces = [&](auto f) {  // f(address in the patch, address in D)
+#pragma unroll
+      for (int q = 0; q < PER; ++q) {
+        const int id = q * 64 + lane, r = id / PIECES, m = m0 + ty * 16 + r, n = n0 + id % PIECES * 8;
+        if ((16 * PIECES % 64 == 0 || id < 16 * PIECES) && m < g.M && n < g.N)
+          f((lds_u4)(uintptr_t)(patch + r * PITCH + id % PIECES * 16), reinterpret_cast<u32x4 *>(static_cast<bf16_t *>(g.D) + (int64_t)m * g.ldd + n));
+      }
+    };
+    if (g.accumulate) {
+      pieces([](lds_u4 at, const u32x4 *d) { *at = *d; });
+      wave_sync();
+    }
+#pragma unroll
+    for (int tx = 0; tx < FX; ++tx) {
+      const lds_u2 at2 = (lds_u2)(uintptr_t)(patch + (lane & 15) * PITCH + (tx * 16 + (lane >> 4) * 4) * 2);
+      f32x4 v = acc.v[tx][ty] + bias[tx];
+      if (g.accumulate) {
+        const u32x2 old = *at2;
+        v += f32x4{bf16_lo(old.x), bf16_hi(old.x), bf16_lo(old.y), bf16_hi(old.y)};
+      }
+      *at2 = u32x2{pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+    }
+    wave_sync();
+    pieces([](lds_u4 at, u32x4 *d) { *d = *at; });
+    wave_sync();
+  }
+}
+
+// the sum of the splits' tiles; an accumulator of every thread per workgroup
 __global__ __launch_bounds__(256) void gemm_reduce_kernel(const Group a) {
   const int tid = threadIdx.x, i = product_of(a, blockIdx.x);
   const MambaGemm &g = a.g[i];
@@ -356,6 +611,20 @@ __global__ __launch_bounds__(256) void gemm_reduce_kernel(const Group a) {
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
   for (int s = 0; s < g.nsplit; ++s) v += *reinterpret_cast<const f32x4 *>(part + (int64_t)s * (GB * GB));
+  store4(g, m, n, v);
+}
+template <int WX, int WY, int FX, int FY> __global__ __launch_bounds__(64 * WX * WY) void gemm_wide_reduce_kernel(const Group a) {
+  typedef WideTile<WX, WY, FX, FY, 1> W;
+  constexpr int QN = FX * FY;
+  const int tid = threadIdx.x, i = product_of(a, blockIdx.x);
+  const MambaGemm &g = a.g[i];
+  const int ntn = (g.N + W::rx - 1) / W::rx, block = blockIdx.x - a.first[i], tile = block / QN, q = block % QN;
+  int m, n;
+  wide_place4<WX, WY, FX, FY>(q, tid, tile / ntn, tile % ntn, m, n);
+  const float *part = a.ws[i] + (int64_t)tile * g.nsplit * (W::rx * W::ry) + (q * W::waves * 64 + tid) * 4;
+  f32x4 v = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
+  for (int s = 0; s < g.nsplit; ++s) v += *reinterpret_cast<const f32x4 *>(part + (int64_t)s * (W::rx * W::ry));
   store4(g, m, n, v);
 }
 
@@ -382,10 +651,10 @@ __global__ __launch_bounds__(256) void cast_bf16_kernel(const CastJobs a) {
   }
 }
 
-int64_t tiles_of(const MambaGemm &g) { return (int64_t)((g.M + GB - 1) / GB) * ((g.N + GB - 1) / GB); }
 bool valid(const MambaGemm &g) {
   return g.A && g.B && g.D && g.M > 0 && g.N > 0 && g.K > 0 && (g.a_ks == 1 || g.a_ms == 1) && (g.b_ks == 1 || g.b_ns == 1) &&
-         (g.d_dtype == MAMBA_BF16 || g.d_dtype == MAMBA_F32) && g.nsplit >= 1 && tiles_of(g) <= INT32_MAX / 1024;
+         (g.d_dtype == MAMBA_BF16 || g.d_dtype == MAMBA_F32) && g.nsplit >= 1 &&
+         (int64_t)((g.M + GB - 1) / GB) * ((g.N + GB - 1) / GB) <= INT32_MAX / 1024;
 }
 
 // gemm_ring_kernel takes the operand with `rows` rows: 16-byte pieces on 16 bytes, offsets in a tile within 32 bits.  (At least 8
@@ -396,53 +665,114 @@ bool pieces(const void *p, int64_t row_stride, int64_t k_stride, int rows, int K
 }
 bool ring(const MambaGemm &g) { return pieces(g.A, g.a_ms, g.a_ks, g.M, g.K) && pieces(g.B, g.b_ns, g.b_ks, g.N, g.K); }
 
+enum { TILE64, TILE128, TILE256, FORMS };
+constexpr int TILE[FORMS] = {GB, 128, 256};
+int64_t tiles_of(const MambaGemm &g, int f) { return (int64_t)((g.M + TILE[f] - 1) / TILE[f]) * ((g.N + TILE[f] - 1) / TILE[f]); }
+// 256 x 256 tiles where there are enough to be cut into few parts, 128 x 128 for what is left of 8 GFLOP and more and where they fill
+// the chip uncut (2560 x 4096 x 80: 11 us against 17 at 64 x 64, 1536 x 2000 x 48 with 192 tiles 9.0 against 9.0).  Cut into parts, a
+// smaller product is the faster one in 64 x 64 (768 x 1536 x 2000: 20 against 24 - 28).
+int form_of(const MambaGemm &g) {
+  if (!ring(g)) return TILE64;
+  const double flop = 2.0 * g.M * g.N * g.K;
+  if (flop > 16e9 && tiles_of(g, TILE256) >= 48) return TILE256;
+  return flop > 8e9 || tiles_of(g, TILE128) >= cu_count() ? TILE128 : TILE64;
+}
+// Parts of the sum over k.  64 x 64: as many as give every CU two workgroups, of at least 8 steps (256 elements) each.  The others: the
+// least of a stage's time by the workgroups on a CU, measured at 18 to 800 tiles in up to 32 parts, and what the parts' writing,
+// reading and second launch take.
+int splits_of(const MambaGemm &g, int f) {
+  const int64_t tiles = tiles_of(g, f), steps = (g.K + GK - 1) / GK, cus = cu_count();
+  if (f == TILE64) return (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / tiles, steps / 8));
+  int best = 1;
+  double least = 1e30;
+  const int64_t most = std::min<int64_t>((f == TILE256 ? 1 : 3) * cus / tiles, steps / 8);
+  for (int s = 1; s == 1 || s <= most; ++s) {
+    const int64_t units = tiles * s;
+    const double stage = f == TILE256 ? 0.82 : units <= cus ? 0.37 : units <= 2 * cus ? 0.41 : 0.62;
+    const double us = (double)((steps + s - 1) / s) * stage + (s > 1 ? 6 + units * TILE[f] * TILE[f] * 2e-6 : 0);
+    if (us < least) least = us, best = s;
+  }
+  return best;
+}
+
+template <int WX, int WY, int FX, int FY, int ST> void launch_wide(const Group &a, int blocks, const Group &r, int rtiles, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_wide_kernel<WX, WY, FX, FY, ST>), dim3(blocks), dim3(64 * WX * WY), 0, s, a);
+  if (rtiles) hipLaunchKernelGGL((gemm_wide_reduce_kernel<WX, WY, FX, FY>), dim3(rtiles * FX * FY), dim3(64 * WX * WY), 0, s, r);
+}
+
 }  // namespace
 
-// Splits along k: as many as give every CU two workgroups, of at least 8 steps (256 elements) each.
+// Where the library takes over.  Up to 8 GFLOP its host time and choice of tiles cost more than any of these forms (whole mixer
+// calls, forward + backward, library / own: products up to 0.5 GFLOP 350 / 180 us, up to 5 GFLOP 432 / 398); up to 16 GFLOP the
+// larger tiles take its time or less (2560 x 2000 x 1280: 26 / 29, 192 x 8192 x 5120: 36 / 47, 2000 x 1280 x 2560: 32 / 30 with
+// 18 us less of host time).  Beyond: sums over a long k into few tiles (weight gradients), which it does not split, and short k with
+// a result that the last-level cache holds (5120 x 16384 x 160: 47 / 57; twice as long 139 / 114).
+extern "C" int mamba_gemm_suits(const MambaGemm *g) {
+  if (!g) return 0;
+  const double flop = 2.0 * g->M * g->N * g->K;
+  if (flop <= 8e9) return 1;
+  if (!ring(*g)) return 0;
+  return flop <= 16e9 || (g->K >= 3 * (int64_t)std::max(g->M, g->N) && tiles_of(*g, TILE256) < cu_count()) ||
+         (g->K <= 256 && (int64_t)g->M * g->N <= 100000000);
+}
+
 extern "C" int64_t mamba_gemm_plan(MambaGemm *g, int count) {
   if (!g || count < 1 || count > MAXG) return MAMBA_E_BADARG;
   int64_t floats = 0;
   for (int i = 0; i < count; ++i) {
     g[i].nsplit = 1;
     if (!valid(g[i])) return MAMBA_E_BADARG;
-    const int64_t tiles = tiles_of(g[i]), steps = (g[i].K + GK - 1) / GK;
-    const int64_t want = std::min<int64_t>(2 * (int64_t)cu_count() / tiles, steps / 8);
+    const int f = form_of(g[i]);
+    const int64_t steps = (g[i].K + GK - 1) / GK, want = splits_of(g[i], f);
     if (want > 1) {
       const int64_t per = (steps + want - 1) / want;
       g[i].nsplit = (int32_t)((steps + per - 1) / per);
     }
-    if (g[i].nsplit > 1) floats += tiles * g[i].nsplit * GB * GB;
+    if (g[i].nsplit > 1) floats += tiles_of(g[i], f) * g[i].nsplit * TILE[f] * TILE[f];
   }
   return floats;
 }
 
 extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream_t stream) {
   if (!g || count < 1 || count > MAXG) return MAMBA_E_BADARG;
-  Group a{}, r{};
-  int blocks = 0, rblocks = 0, nr = 0;
-  int64_t used = 0;
-  for (int i = 0; i < count; ++i) {
-    if (!valid(g[i])) return MAMBA_E_BADARG;
-    if (g[i].nsplit > 1 && !ws) return MAMBA_E_BADARG;
-    const int64_t tiles = tiles_of(g[i]);
-    a.g[i] = g[i], a.first[i] = blocks, a.ws[i] = ws + used;
-    blocks += (int)(tiles * g[i].nsplit);
-    if (g[i].nsplit > 1) {
-      r.g[nr] = g[i], r.first[nr] = rblocks, r.ws[nr] = ws + used;
-      rblocks += (int)(4 * tiles);
-      used += tiles * g[i].nsplit * GB * GB;
-      ++nr;
-    }
-  }
-  for (int i = count; i <= MAXG; ++i) a.first[i] = INT32_MAX;
-  for (int i = nr; i <= MAXG; ++i) r.first[i] = INT32_MAX;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  bool all = true;
-  for (int i = 0; i < count; ++i) all = all && ring(g[i]);
-  if (all) hipLaunchKernelGGL(gemm_ring_kernel, dim3(blocks), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(gemm_kernel, dim3(blocks), dim3(256), 0, s, a);
-  if (nr) hipLaunchKernelGGL(gemm_reduce_kernel, dim3(rblocks), dim3(256), 0, s, r);
-  return hipGetLastError() == hipSuccess ? MAMBA_OK : MAMBA_E_LAUNCH;
+  for (int i = 0; i < count; ++i) {
+    if (!valid(g[i]) || (g[i].nsplit > 1 && !ws)) return MAMBA_E_BADARG;
+  }
+  // the products of one form in a launch
+  for (int f = FORMS - 1; f >= 0; --f) {
+    Group a{}, r{};
+    int blocks = 0, rtiles = 0, n = 0, nr = 0;
+    bool all = true;
+    const int per_tile = TILE[f] * TILE[f] / (f == TILE256 ? 2048 : 1024);  // workgroups that add up its splits
+    for (int i = 0; i < count; ++i) {
+      if (form_of(g[i]) != f) continue;
+      const int64_t tiles = tiles_of(g[i], f);
+      a.g[n] = g[i], a.first[n] = blocks, a.ws[n] = ws;
+      blocks += (int)(tiles * g[i].nsplit);
+      all = all && ring(g[i]);
+      if (g[i].nsplit > 1) {
+        r.g[nr] = g[i], r.first[nr] = rtiles * per_tile, r.ws[nr] = ws;
+        rtiles += (int)tiles;
+        ws += tiles * g[i].nsplit * TILE[f] * TILE[f];
+        ++nr;
+      }
+      ++n;
+    }
+    if (!n) continue;
+    for (int i = n; i <= MAXG; ++i) a.first[i] = INT32_MAX;
+    for (int i = nr; i <= MAXG; ++i) r.first[i] = INT32_MAX;
+    switch (f) {
+      case TILE128: launch_wide<2, 2, 4, 4, 3>(a, blocks, r, rtiles, s); break;
+      case TILE256: launch_wide<2, 4, 8, 4, 3>(a, blocks, r, rtiles, s); break;
+      default:
+        if (all) hipLaunchKernelGGL(gemm_ring_kernel, dim3(blocks), dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(gemm_kernel, dim3(blocks), dim3(256), 0, s, a);
+        if (nr) hipLaunchKernelGGL(gemm_reduce_kernel, dim3(rtiles * 4), dim3(256), 0, s, r);
+    }
+    if (hipGetLastError() != hipSuccess) return MAMBA_E_LAUNCH;
+  }
+  return MAMBA_OK;
 }
 
 extern "C" int mamba_cast_bf16(const MambaCast *c, int count, mamba_stream_t stream) {

@@ -1,16 +1,9 @@
-// Matrix products of a mixer on raw operands: short ones through the library's grouped kernel (mamba_gemm), the others
+// Matrix products of a mixer on raw operands: through the library's grouped kernels (mamba_gemm) where they suit, the others
 // through the BLAS library.
 #include "torch_common.h"
 
 namespace mamba_ext {
 namespace {
-
-// Where the own kernel ends.  Below this the library call's host time and its choice of tiles cost more than a 64 x 64
-// tile without operand reuse across workgroups does: measured on whole mixer calls, forward + backward, library / own:
-// products up to 0.5 GFLOP 350 / 180 us, up to 5 GFLOP 432 / 398 us, up to 10 GFLOP 472 / 481 us, 10 - 30 GFLOP each
-// 506 / 517 us.
-constexpr double SHORT_FLOP = 8e9;
-bool short_product(const MambaGemm &g) { return 2.0 * g.M * g.N * g.K <= SHORT_FLOP; }
 
 at::Tensor matrix(const void *p, int64_t rows, int64_t cols, int64_t rs, int64_t cs, const at::TensorOptions &o) {
   return at::from_blob(const_cast<void *>(p), {rows, cols}, {rs, cs}, o);
@@ -23,7 +16,7 @@ Products &Products::add(void *D, at::ScalarType d_type, int64_t ldd, int64_t M, 
   MambaGemm g{};
   g.A = A.p, g.a_ms = A.rs, g.a_ks = A.ks, g.B = B.p, g.b_ns = B.rs, g.b_ks = B.ks, g.bias = bias, g.D = D, g.ldd = ldd;
   g.M = (int32_t)M, g.N = (int32_t)N, g.K = (int32_t)K, g.d_dtype = dtype_code(d_type), g.accumulate = accumulate;
-  if (type_ == at::kBFloat16 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX && short_product(g)) {
+  if (type_ == at::kBFloat16 && M <= INT32_MAX && N <= INT32_MAX && K <= INT32_MAX && mamba_gemm_suits(&g)) {
     if (count_ == 4) run();
     g_[count_++] = g;
     return *this;

@@ -1,5 +1,5 @@
-"""The grouped bf16 products whose operands lie on 16 bytes (gemm_ring_kernel in gemm.hip): edges of the 64 x 64 tile, of the
-64-wide stage and of a split's k, every layout of both operands, beside values that must not be read into a result.
+"""The grouped bf16 products whose operands lie on 16 bytes (gemm_ring_kernel and gemm_wide_kernel in gemm.hip): edges of the tiles,
+of the stages and of a split's k, every layout of both operands, beside values that must not be read into a result.
 Reference: fp64 products."""
 import pytest
 import torch
@@ -15,6 +15,24 @@ ODD_ROWS = [(65, 127, 64), (1, 3, 72), (100, 66, 2048), (129, 63, 4120)]     # b
 @pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, SHAPES) for a in (True, False) for b in (True, False)] + [(False, False, ODD_K), (True, True, ODD_ROWS)])
 @pytest.mark.parametrize("out", [torch.bfloat16, torch.float32])
 def test_products(a_k, b_k, shapes, out):
+    check(a_k, b_k, shapes, out, 3)
+
+
+# Larger tiles: 128 x 128 without splits (a K shorter than the ring, ragged ones, a row of one element more than the tiles), with
+# them, and 256 x 256; in one call with a product of 64 x 64
+WIDE = [(2176, 2048, 16), (2056, 2184, 72), (72, 136, 72), (136, 200, 160008)]
+WIDE_256 = [(1800, 1544, 3080), (1544, 1800, 3112), (64, 64, 64), (2048, 2048, 2056)]
+WIDE_ODD_K = [(2184, 2056, 33), (136, 200, 160001), (64, 64, 33), (1800, 1544, 3081)]
+WIDE_ODD_ROWS = [(2049, 2183, 72), (65, 129, 500008), (1, 3, 72), (1801, 1543, 3080)]
+
+
+@pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, s) for a in (True, False) for b in (True, False) for s in (WIDE, WIDE_256)] + [(False, False, WIDE_ODD_K), (True, True, WIDE_ODD_ROWS)])
+@pytest.mark.parametrize("out,pad", [(torch.bfloat16, 8), (torch.bfloat16, 3), (torch.float32, 3)])
+def test_larger_tiles(a_k, b_k, shapes, out, pad):
+    check(a_k, b_k, shapes, out, pad)
+
+
+def check(a_k, b_k, shapes, out, pad):
     from mamba_amd import _lib
     lib = _lib.load()
     gen = torch.Generator(device="cuda").manual_seed(5)
@@ -30,12 +48,12 @@ def test_products(a_k, b_k, shapes, out):
         group, keep = (_lib.MambaGemm * 4)(), []
         for j, (M, N, K) in enumerate(shapes[first:first + 4]):
             A, B, bias = operand(M, K, a_k), operand(N, K, b_k), torch.randn(N, device="cuda", generator=gen).bfloat16()
-            D = torch.full((M, N + 3), 0.5, device="cuda", dtype=out)
+            D = torch.full((M, N + pad), 0.5, device="cuda", dtype=out)
             with_bias, accumulate = j % 2 == 0, j >= 2
             want = A.double() @ B.double().t() + (bias.double() if with_bias else 0) + (0.5 if accumulate else 0)
             size = A.double().abs() @ B.double().abs().t() + 1
             group[j] = _lib.MambaGemm(A.data_ptr(), B.data_ptr(), bias.data_ptr() if with_bias else None, D.data_ptr(), *A.stride(), *B.stride(),
-                                      N + 3, M, N, K, _lib.DTYPE_CODE[out], int(accumulate), 0)
+                                      N + pad, M, N, K, _lib.DTYPE_CODE[out], int(accumulate), 0)
             keep.append((A, B, bias, D, want, size, K))
         floats = lib.mamba_gemm_plan(group, 4)
         assert floats >= 0

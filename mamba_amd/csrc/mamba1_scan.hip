@@ -31,7 +31,7 @@ size_t mamba1_bwd_mx_lds(int passes, int np);                                   
 int mamba1_bwd_mx_launch(const MambaScanParams &p, int passes, bool vec, hipStream_t stream);  // likewise
 size_t mamba1_bwd_k4_lds(int passes);                                                          // mamba1_scan_bwd_k4.hip
 bool mamba1_bwd_k4_serves(const MambaScanParams &p);                                           // likewise
-int mamba1_fwd_serial_launch(const MambaScanParams &p, int mode, hipStream_t s);                // mamba1_scan_serial.hip
+int mamba1_fwd_serial_launch(const MambaScanParams &p, int spl, int mode, hipStream_t s);       // mamba1_scan_serial.hip
 int mamba1_bwd_k4_launch(const MambaScanParams &p, int pa, int pb, int nparts, hipStream_t stream);  // likewise
 
 namespace {
@@ -946,9 +946,11 @@ size_t fwd_min_lds() {
 }
 
 // The forward kernel that serves a problem and its estimated time in us, for 16 states.  scan_fwd_serial_kernel
-// (mamba1_scan_serial.hip) takes 16 states and per-position B and C; up to five of its workgroups share a CU, and a tile
-// (half tiles where the sequence ends in one) takes a round of them 7.3, 10.7, 14.1, 17.5, 20.9.  scan_fwd_kernel: up to
-// two per CU, 6.6 or 10.9, and a seventh more of that on rows with a ragged end.  Measured, 8 x 5120 channels x 4096
+// (mamba1_scan_serial.hip) takes 16 states and per-position B and C.  With two states per lane up to five of its workgroups
+// share a CU, and a tile (half tiles where the sequence ends in one) takes a round of them 7.3, 10.7, 14.1, 17.5, 20.9; with
+// one, a workgroup has half as many channels and a tile takes 4.8, 6.5, 9.1, 11.6: 1 x 1536 x 256 15.5 -> 12.7 us, 8 x 1024 x
+// 2048 115 -> 108, 1 x 768 x 4096 in segments 42 -> 39; from five of them on two states per lane stay (4 x 5120 x 512: 62
+// against 63).  scan_fwd_kernel: up to two per CU, 6.6 or 10.9, and a seventh more of that on rows with a ragged end.  Measured, 8 x 5120 channels x 4096
 // positions bf16: 806 -> 660 us; 8 x 2368 x 8086: 1235 -> 971; 7 x 3184 x 192: 35 -> 24; a workgroup per CU or less and the
 // sequence whole: 108 against 119 (2 x 4096 x 2048), the kernel with the lanes along the sequence stays; cut into more
 // segments (below) the other one serves those too.
@@ -956,7 +958,7 @@ bool serial_takes(const MambaScanParams &p) {
   return p.dstate == NB16 && !(p.bc_const & 3) && !p.a_complex && !k4_mode() && !fwd_min_lds() && p.seqlen >= KI;
 }
 struct FwdCost {
-  bool serial;
+  int spl;  // states per lane of scan_fwd_serial_kernel, 0: scan_fwd_kernel
   double us;
 };
 FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
@@ -965,14 +967,18 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
   const int per = (ntiles + nseg - 1) / nseg;
   if (!serial_takes(p)) {
     const double rounds = (double)((wgs + 2 * cus - 1) / (2 * cus));
-    return {false, 6.4 * rounds * (wgs > cus ? 1.47 : 1.0) * ((p.dstate + NB16 - 1) / NB16) * per + 2.0 * rounds};
+    return {0, 6.4 * rounds * (wgs > cus ? 1.47 : 1.0) * ((p.dstate + NB16 - 1) / NB16) * per + 2.0 * rounds};
   }
   const double tiles = nseg > 1 ? (double)per : 0.5 * ((p.seqlen + TILE / 2 - 1) / (TILE / 2));
   const int64_t pairs = wgs / (2 * cus), odd = wgs - pairs * 2 * cus;
   const double round = (10.9 * (double)pairs + (odd > cus ? 10.9 : odd > 0 ? 6.6 : 0.0)) * (p.seqlen % KI ? 1.15 : 1.0);
-  const FwdCost lanes{false, round * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
+  const FwdCost lanes{0, round * std::ceil(tiles) + 2.0 * (double)(pairs + (odd > 0))};
   const int64_t fives = wgs / (5 * cus), rest = (wgs - fives * 5 * cus + cus - 1) / cus;
-  const FwdCost serial{true, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + (p.seqlen % KI ? 3.4 : 2.0)};
+  const FwdCost two{2, (20.9 * (double)fives + (rest ? 3.9 + 3.4 * (double)rest : 0.0)) * tiles + (p.seqlen % KI ? 3.4 : 2.0)};
+  const int64_t halves = (int64_t)p.batch * p.ngroups * ((Dg + PASS_CH / 2 - 1) / (PASS_CH / 2)) * nseg;
+  const int64_t fours = halves / (4 * cus), left = (halves - fours * 4 * cus + cus - 1) / cus;
+  const FwdCost one{1, (11.6 * (double)fours + (left > 1 ? 1.4 + 2.55 * (double)left : 4.8 * (double)left)) * per + (p.seqlen % KI ? 3.4 : 2.0)};
+  const FwdCost serial = one.us < two.us ? one : two;
   return serial.us < lanes.us ? serial : lanes;
 }
 
@@ -986,8 +992,9 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
 // to two workgroups per CU, half as much again where two share one, 3.0 for a tile of the pass over the segments, 6 % to
 // promise.  (The terms for 16 states cut them too finely: 2 x 4160 x 1261, 4 states, 53 us whole and 70 in five segments; 2 x
 // 1552 x 4029, 64 states, 420 us in five and 501 in 32.)
-// Measured: 1536 channels x 777 positions of one sequence 50 -> 24 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181
-// forward; 1536 channels whole and in two segments: 14.8 and 14.8 (129 positions), 13.1 and 14.6 (192), 16.6 and 15.0 (256).
+// Measured: 1536 channels x 777 positions of one sequence 36 -> 22.5 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181
+// forward; 1536 channels x 256 whole and in two segments 12.7 and 13.7, x 777 in one, two, three, four and seven 36, 33, 28, 28.5
+// and 24.5 (each over and over on the same inputs).
 constexpr int MAX_SEGMENTS = 32;
 int scan_segments(const MambaScanParams &p, bool bwd) {
   const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
@@ -1163,7 +1170,8 @@ template <typename T, bool BWD, int BC> int dispatch_bc(const MambaScanParams &p
   if (rc != MAMBA_OK) return rc;
   if (!BWD) {
     const bool half = k4_mode();
-    if (fwd_cost(p, std::max(1, p.nseg)).serial) return mamba1_fwd_serial_launch(p, mode, stream);
+    const int spl = fwd_cost(p, std::max(1, p.nseg)).spl;
+    if (spl) return mamba1_fwd_serial_launch(p, spl, mode, stream);
     const size_t lds = std::max(fwd_lds(1, np, half), fwd_min_lds());
     if (half)
       return mode == ROWS_ALIGNED ? launch(scan_fwd_kernel<T, ROWS_ALIGNED, BC, true>, p, 1, lds, stream)

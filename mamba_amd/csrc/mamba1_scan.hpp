@@ -118,16 +118,16 @@ DEVI void load_bc(float (&v)[8], const float *staged, const void *mat, int d, in
   }
 }
 
-// Where a workgroup's channels lie: workgroup cb of group g takes `passes` passes of PASS_CH channels, and the tiles
+// Where a workgroup's channels lie: workgroup cb of group g takes `passes` passes of CH channels, and the tiles
 // [tile0, tile1) of segment blockIdx.z of the sequence.
 struct Geo {
   int g, cb, b, Dg, dend, ntiles, cblocks, seg, nseg, tile0, tile1;
 };
 DEVI int tiles_per_segment(int ntiles, int nseg) { return (ntiles + nseg - 1) / nseg; }
-DEVI Geo geometry(const MambaScanParams &p, int passes) {
+template <int CH = PASS_CH> DEVI Geo geometry(const MambaScanParams &p, int passes) {
   Geo q;
   q.Dg = p.dim / p.ngroups;
-  q.cblocks = (q.Dg + PASS_CH * passes - 1) / (PASS_CH * passes);
+  q.cblocks = (q.Dg + CH * passes - 1) / (CH * passes);
   q.g = blockIdx.x / q.cblocks;
   q.cb = blockIdx.x % q.cblocks;
   q.b = blockIdx.y;

@@ -116,3 +116,27 @@ def test_the_measurement_hook_reaches_the_other_kernel():
             env["MAMBA_AMD_FWD_MIN_LDS"] = lds
         bits.add(subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, check=True, timeout=100).stdout)
     assert len(bits) == 2
+
+
+# one state per lane: few channels, whole and cut into segments, more of them than are read at a time, groups, ragged rows
+@pytest.mark.parametrize("b,d,L,G,off", [(1, 1526, 8, 1, 0), (1, 1526, 65, 1, 0), (2, 770, 129, 1, 1), (1, 520, 777, 4, 3),
+                                         (1, 96, 4100, 1, 0), (8, 1008, 256, 1, 0), (3, 1000, 127, 2, 2), (1, 1536, 256, 1, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32, torch.float16])
+def test_few_channels(b, d, L, G, off, dtype):
+    _check(_inputs(b, d, L, G, dtype, d + L, off))
+
+
+def test_few_channels_stay_apart():
+    """NaN in the last position reaches no other one; infinities in a channel reach no other channel."""
+    from mamba_amd.ops.selective_scan_interface import selective_scan_fn
+    t = _inputs(1, 1024, 130, 1, torch.bfloat16, 3)
+    t["u"][:, 5, 129] = float("nan")
+    t["u"][:, 7, 64] = float("inf")
+    with torch.no_grad():
+        out = selective_scan_fn(t["u"], t["delta"], t["A"], t["B"], t["C"], t["D"], z=t["z"], delta_bias=t["delta_bias"],
+                                delta_softplus=True)
+    bad = ~torch.isfinite(out)
+    assert bad[:, 5, 129].all() and bad[:, 7, 64:].all()
+    bad[:, 5, 129] = False
+    bad[:, 7, 64:] = False
+    assert not bad.any()

@@ -16,6 +16,7 @@ constexpr int MAXG = 4, PF = 4;
 struct Group {
   MambaGemm g[MAXG];
   int first[MAXG + 1];  // first workgroup of every product
+  int helpers[MAXG];    // see Share
   float *ws[MAXG];
 };
 
@@ -352,7 +353,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const Group a) {
 // before it run.  What bounds them: up to 128 x 128 the reading through the L2 (2560 x 5120 x 32768: 13 GB, 13.6 TB/s), at 256 x 256
 // the LDS (reading 96 KB and writing 32 KB per CU and stage is as long as its products), 1.0 - 1.2 PFLOP/s.
 //   M x N x K                 us: library | 64 x 64 | 128 x 128 | 256 x 256 (with the splits that are chosen)
-//   2560 x 5120 x 32768           965   |   -   | 1198 | 832        (200 tiles on 256 CUs: 78 % of what they could do)
+//   2560 x 5120 x 32768           965   |   -   | 1198 | 754        (200 tiles on 256 CUs: 832 without Share's helpers)
 //   2560 x 5120 x 16384           513   |   -   |  605 | 384
 //   192 x 5120 x 32768            234   |  156  |  121 - 138 | 124
 //   768 x 1536 x 32768            183   |  218  |   89 |  90
@@ -502,40 +503,92 @@ template <int WX, int WY, int FX, int FY> DEVI void wide_place4(int q, int tid, 
   n = (nt * WX + wx) * (FX * 16) + (q / FY) * 16 + (lane >> 4) * 4;
 }
 
-template <int WX, int WY, int FX, int FY, int ST>
+// How the stages of a product's units (tile, part of k) are shared out where the units leave `helpers` CUs idle: a unit's own
+// workgroup takes its first `own` stages, so that all end together, and the helpers the rest of the units, `rest` stages each laid
+// end to end, `span` stages per helper.  (Own workgroups walk k side by side, which keeps what neighbouring tiles share in the
+// L2.)  2560 x 5120 x 32768, 200 tiles on 256 CUs: 832 -> 754 us (1.14 PFLOP/s).
+struct Share {
+  int units, stages, per, own, rest, helpers, span, pieces;  // pieces of units a helper may touch
+  __host__ __device__ Share(int tiles, int nsplit, int helpers_, int K)
+      : units(tiles * nsplit), stages((K + WK - 1) / WK), per((stages + nsplit - 1) / nsplit), helpers(helpers_) {
+    own = helpers ? (int)(((int64_t)per * units + units + helpers - 1) / (units + helpers)) : per;
+    rest = per - own;
+    span = helpers ? (units * rest + helpers - 1) / helpers : 0;
+    pieces = rest ? span / rest + 2 : 0;
+  }
+  __host__ __device__ int64_t slots() const { return units + (int64_t)helpers * pieces; }
+  // what helper h takes of unit u, from stage [0] to [1] of the whole k; its place is h * pieces + u - h * span / rest
+  DEVI void part(int h, int u, int tiles, int &from, int &to) const {
+    const int u0 = u * rest, first = u / tiles * per;
+    from = first + own + max(h * span - u0, 0);
+    to = min(min(first + own + min((h + 1) * span - u0, rest), first + per), stages);
+  }
+};
+
+template <int WX, int WY, int FX, int FY, int ST, bool HELP>
 __global__ __launch_bounds__(64 * WX * WY, WX * WY == 4 ? 3 : 2) void gemm_wide_kernel(const Group a) {
   typedef WideTile<WX, WY, FX, FY, ST> W;
   __shared__ __align__(256) char sh[ST * W::stage];
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = product_of(a, blockIdx.x);
-  const int wx = wave % WX, wy = wave / WX;
+  int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = product_of(a, blockIdx.x), wx = wave % WX, wy = wave / WX;
   const MambaGemm &g = a.g[i];
   const int ntn = (g.N + W::rx - 1) / W::rx, ntm = (g.M + W::ry - 1) / W::ry, tiles = ntn * ntm;
+  const Share share(tiles, g.nsplit, HELP ? a.helpers[i] : 0, g.K);
   // consecutive tiles of the shorter side, which share the longer side's operand, on one XCD
-  const int count = tiles * g.nsplit, block = xcd_run(blockIdx.x - a.first[i], count);
-  const int split = block / tiles, tile = block % tiles;
-  const int mt = ntm < ntn ? tile % ntm : tile / ntn, nt = ntm < ntn ? tile / ntm : tile % ntn;
-  const int steps = (g.K + GK - 1) / GK, per = (steps + g.nsplit - 1) / g.nsplit;
-  const int k0 = min(split * per * GK, g.K), k1 = min(k0 + per * GK, g.K);
+  const int block = xcd_run(blockIdx.x - a.first[i], share.units + share.helpers);
   WideAcc<FX, FY> acc;
-#pragma unroll
-  for (int q = 0; q < FX * FY; ++q) acc.v[q / FY][q % FY] = f32x4{0.f, 0.f, 0.f, 0.f};
   const uint32_t at = lds_address(sh);
+  auto leave = [&](int64_t slot) {  // for the kernel that adds the parts up
+    float *part = a.ws[i] + slot * (W::rx * W::ry);
+#pragma unroll
+    for (int q = 0; q < FX * FY; ++q) *reinterpret_cast<f32x4 *>(part + (q * W::waves * 64 + tid) * 4) = acc.v[q / FY][q % FY];
+  };
+  auto tile_at = [&](int unit, int &mt, int &nt) {
+    const int tile = unit % tiles;
+    mt = ntm < ntn ? tile % ntm : tile / ntn, nt = ntm < ntn ? tile / ntm : tile % ntn;
+  };
+  const bool helper = HELP && block >= share.units;
   auto run = [&](auto x_tr, auto y_tr) {
     constexpr bool XTR = decltype(x_tr)::value, YTR = decltype(y_tr)::value;
-    // (a split's k ends where the next one's begins)
-    const WideRing<XTR, W::loads_x, W::waves> X(g.B, g.b_ns, g.b_ks, nt * W::rx, g.N, k1, wave, lane);
-    const WideRing<YTR, W::loads_y, W::waves> Y(g.A, g.a_ms, g.a_ks, mt * W::ry, g.M, k1, wave, lane);
-    run_wide<W>(acc, at, X, Y, k0, k1, wx, wy, lane);
+    auto product = [&](int unit, int from, int to) {
+      const int k0 = from * WK, k1 = min(to * WK, g.K);
+      int mt, nt;
+      tile_at(unit, mt, nt);
+#pragma unroll
+      for (int q = 0; q < FX * FY; ++q) acc.v[q / FY][q % FY] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // (a part's k ends where the next one's begins)
+      const WideRing<XTR, W::loads_x, W::waves> X(g.B, g.b_ns, g.b_ks, nt * W::rx, g.N, k1, wave, lane);
+      const WideRing<YTR, W::loads_y, W::waves> Y(g.A, g.a_ms, g.a_ks, mt * W::ry, g.M, k1, wave, lane);
+      run_wide<W>(acc, at, X, Y, k0, k1, wx, wy, lane);
+    };
+    if constexpr (HELP) {
+      const int h = block - share.units, u0 = helper ? h * share.span / share.rest : block;
+#pragma unroll 1
+      for (int u = u0; u < min(u0 + (helper ? share.pieces : 1), share.units); ++u) {
+        int from = u / tiles * share.per, to = min(from + share.own, share.stages);
+        if (helper) share.part(h, u, tiles, from, to);
+        if (from >= to) continue;
+        // (a new value to the compiler: what derives from it is formed where it is used instead of being carried along)
+        asm volatile("" : "+v"(tid));
+        lane = tid & 63;
+        product(u, from, to);
+        leave(helper ? share.units + (int64_t)h * share.pieces + u - u0 : block);
+      }
+    } else {
+      const int from = block / tiles * share.per;
+      product(block, from, min(from + share.per, share.stages));
+    }
   };
   const bool btr = g.b_ks != 1, atr = g.a_ks != 1;
   if (btr && atr) run(std::true_type{}, std::true_type{});
   else if (btr) run(std::true_type{}, std::false_type{});
   else if (atr) run(std::false_type{}, std::true_type{});
   else run(std::false_type{}, std::false_type{});
+  if constexpr (HELP) return;
+  int mt, nt;
+  tile_at(block, mt, nt);
   if (g.nsplit > 1) {
-    float *part = a.ws[i] + ((int64_t)(mt * ntn + nt) * g.nsplit + split) * (W::rx * W::ry);
-#pragma unroll
-    for (int q = 0; q < FX * FY; ++q) *reinterpret_cast<f32x4 *>(part + (q * W::waves * 64 + tid) * 4) = acc.v[q / FY][q % FY];
+    leave(block);
     return;
   }
   // whole rows of 16-byte pieces where D allows, 16 rows at a time through a patch of the wave's own
@@ -618,13 +671,26 @@ template <int WX, int WY, int FX, int FY> __global__ __launch_bounds__(64 * WX *
   constexpr int QN = FX * FY;
   const int tid = threadIdx.x, i = product_of(a, blockIdx.x);
   const MambaGemm &g = a.g[i];
-  const int ntn = (g.N + W::rx - 1) / W::rx, block = blockIdx.x - a.first[i], tile = block / QN, q = block % QN;
+  const int ntn = (g.N + W::rx - 1) / W::rx, ntm = (g.M + W::ry - 1) / W::ry, tiles = ntn * ntm;
+  const int block = blockIdx.x - a.first[i], tile = block / QN, q = block % QN;
+  const Share share(tiles, g.nsplit, a.helpers[i], g.K);
   int m, n;
-  wide_place4<WX, WY, FX, FY>(q, tid, tile / ntn, tile % ntn, m, n);
-  const float *part = a.ws[i] + (int64_t)tile * g.nsplit * (W::rx * W::ry) + (q * W::waves * 64 + tid) * 4;
+  wide_place4<WX, WY, FX, FY>(q, tid, ntm < ntn ? tile % ntm : tile / ntn, ntm < ntn ? tile / ntm : tile % ntn, m, n);
+  const float *part = a.ws[i] + (q * W::waves * 64 + tid) * 4;
+  auto at = [&](int64_t slot) { return *reinterpret_cast<const f32x4 *>(part + slot * (W::rx * W::ry)); };
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
-  for (int s = 0; s < g.nsplit; ++s) v += *reinterpret_cast<const f32x4 *>(part + (int64_t)s * (W::rx * W::ry));
+  for (int s = 0; s < g.nsplit; ++s) v += at(s * tiles + tile);
+  if (share.rest) {
+    for (int s = 0; s < g.nsplit; ++s) {
+      const int u = s * tiles + tile;
+      for (int h = u * share.rest / share.span; h * share.span < (u + 1) * share.rest; ++h) {
+        int from, to;
+        share.part(h, u, tiles, from, to);
+        if (from < to) v += at(share.units + (int64_t)h * share.pieces + u - h * share.span / share.rest);
+      }
+    }
+  }
   store4(g, m, n, v);
 }
 
@@ -680,6 +746,21 @@ int form_of(const MambaGemm &g) {
 // Parts of the sum over k.  64 x 64: as many as give every CU two workgroups, of at least 8 steps (256 elements) each.  The others: the
 // least of a stage's time by the workgroups on a CU, measured at 18 to 800 tiles in up to 32 parts, and what the parts' writing,
 // reading and second launch take.
+double us_of(int64_t tiles, int splits, int helpers, int K, int f) {
+  const Share share((int)tiles, splits, helpers, K);
+  const int64_t units = share.units, cus = cu_count();
+  const double stage = f == TILE256 ? 0.82 : units <= cus ? 0.37 : units <= 2 * cus ? 0.41 : 0.62;
+  const int64_t parts = (splits > 1 || helpers ? units : 0) + (helpers ? units + helpers : 0);
+  return share.own * stage + (parts ? 6 + parts * TILE[f] * TILE[f] * 2e-6 : 0);
+}
+// CUs that the units of 256 x 256 tiles leave idle and that are worth their parts
+int helpers_of(int64_t tiles, int splits, int K, int f) {
+  const int64_t units = tiles * splits, idle = cu_count() - units;
+  if (f != TILE256 || idle <= 0) return 0;
+  const Share share((int)tiles, splits, (int)idle, K);
+  if (!share.rest || units * share.rest >= 1 << 30) return 0;
+  return us_of(tiles, splits, (int)idle, K, f) < 0.97 * us_of(tiles, splits, 0, K, f) ? (int)idle : 0;
+}
 int splits_of(const MambaGemm &g, int f) {
   const int64_t tiles = tiles_of(g, f), steps = (g.K + GK - 1) / GK, cus = cu_count();
   if (f == TILE64) return (int)std::max<int64_t>(1, std::min<int64_t>(2 * cus / tiles, steps / 8));
@@ -687,16 +768,21 @@ int splits_of(const MambaGemm &g, int f) {
   double least = 1e30;
   const int64_t most = std::min<int64_t>((f == TILE256 ? 1 : 3) * cus / tiles, steps / 8);
   for (int s = 1; s == 1 || s <= most; ++s) {
-    const int64_t units = tiles * s;
-    const double stage = f == TILE256 ? 0.82 : units <= cus ? 0.37 : units <= 2 * cus ? 0.41 : 0.62;
-    const double us = (double)((steps + s - 1) / s) * stage + (s > 1 ? 6 + units * TILE[f] * TILE[f] * 2e-6 : 0);
+    const double us = us_of(tiles, s, helpers_of(tiles, s, g.K, f), g.K, f);
     if (us < least) least = us, best = s;
   }
   return best;
 }
+// fp32 elements of the parts' places
+int64_t parts_of(const MambaGemm &g, int f) {
+  const int64_t tiles = tiles_of(g, f);
+  const int helpers = helpers_of(tiles, g.nsplit, g.K, f);
+  if (g.nsplit == 1 && !helpers) return 0;
+  return (f == TILE64 ? tiles * g.nsplit : Share((int)tiles, g.nsplit, helpers, g.K).slots()) * TILE[f] * TILE[f];
+}
 
-template <int WX, int WY, int FX, int FY, int ST> void launch_wide(const Group &a, int blocks, const Group &r, int rtiles, hipStream_t s) {
-  hipLaunchKernelGGL((gemm_wide_kernel<WX, WY, FX, FY, ST>), dim3(blocks), dim3(64 * WX * WY), 0, s, a);
+template <int WX, int WY, int FX, int FY, int ST, bool HELP> void launch_wide(const Group &a, int blocks, const Group &r, int rtiles, hipStream_t s) {
+  hipLaunchKernelGGL((gemm_wide_kernel<WX, WY, FX, FY, ST, HELP>), dim3(blocks), dim3(64 * WX * WY), 0, s, a);
   if (rtiles) hipLaunchKernelGGL((gemm_wide_reduce_kernel<WX, WY, FX, FY>), dim3(rtiles * FX * FY), dim3(64 * WX * WY), 0, s, r);
 }
 
@@ -728,7 +814,7 @@ extern "C" int64_t mamba_gemm_plan(MambaGemm *g, int count) {
       const int64_t per = (steps + want - 1) / want;
       g[i].nsplit = (int32_t)((steps + per - 1) / per);
     }
-    if (g[i].nsplit > 1) floats += tiles_of(g[i], f) * g[i].nsplit * TILE[f] * TILE[f];
+    floats += parts_of(g[i], f);
   }
   return floats;
 }
@@ -737,10 +823,12 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
   if (!g || count < 1 || count > MAXG) return MAMBA_E_BADARG;
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (int i = 0; i < count; ++i) {
-    if (!valid(g[i]) || (g[i].nsplit > 1 && !ws)) return MAMBA_E_BADARG;
+    if (!valid(g[i]) || (parts_of(g[i], form_of(g[i])) && !ws)) return MAMBA_E_BADARG;
   }
-  // the products of one form in a launch
-  for (int f = FORMS - 1; f >= 0; --f) {
+  // the products of one form in a launch, those with helpers (every workgroup leaves parts) apart from the others
+  for (int form = FORMS; form >= 0; --form) {
+    const int f = std::min(form, FORMS - 1);
+    const bool helped = form == FORMS;
     Group a{}, r{};
     int blocks = 0, rtiles = 0, n = 0, nr = 0;
     bool all = true;
@@ -748,13 +836,15 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
     for (int i = 0; i < count; ++i) {
       if (form_of(g[i]) != f) continue;
       const int64_t tiles = tiles_of(g[i], f);
-      a.g[n] = g[i], a.first[n] = blocks, a.ws[n] = ws;
-      blocks += (int)(tiles * g[i].nsplit);
+      const int helpers = helpers_of(tiles, g[i].nsplit, g[i].K, f);
+      if ((helpers > 0) != helped) continue;
+      a.g[n] = g[i], a.first[n] = blocks, a.helpers[n] = helpers, a.ws[n] = ws;
+      blocks += (int)(tiles * g[i].nsplit) + helpers;
       all = all && ring(g[i]);
-      if (g[i].nsplit > 1) {
-        r.g[nr] = g[i], r.first[nr] = rtiles * per_tile, r.ws[nr] = ws;
+      if (const int64_t parts = parts_of(g[i], f)) {
+        r.g[nr] = g[i], r.first[nr] = rtiles * per_tile, r.helpers[nr] = helpers, r.ws[nr] = ws;
         rtiles += (int)tiles;
-        ws += tiles * g[i].nsplit * TILE[f] * TILE[f];
+        ws += parts;
         ++nr;
       }
       ++n;
@@ -763,8 +853,11 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
     for (int i = n; i <= MAXG; ++i) a.first[i] = INT32_MAX;
     for (int i = nr; i <= MAXG; ++i) r.first[i] = INT32_MAX;
     switch (f) {
-      case TILE128: launch_wide<2, 2, 4, 4, 3>(a, blocks, r, rtiles, s); break;
-      case TILE256: launch_wide<2, 4, 8, 4, 3>(a, blocks, r, rtiles, s); break;
+      case TILE128: launch_wide<2, 2, 4, 4, 3, false>(a, blocks, r, rtiles, s); break;
+      case TILE256:
+        if (helped) launch_wide<2, 4, 8, 4, 3, true>(a, blocks, r, rtiles, s);
+        else launch_wide<2, 4, 8, 4, 3, false>(a, blocks, r, rtiles, s);
+        break;
       default:
         if (all) hipLaunchKernelGGL(gemm_ring_kernel, dim3(blocks), dim3(256), 0, s, a);
         else hipLaunchKernelGGL(gemm_kernel, dim3(blocks), dim3(256), 0, s, a);

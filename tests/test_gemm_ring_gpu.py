@@ -22,11 +22,12 @@ def test_products(a_k, b_k, shapes, out):
 # them, and 256 x 256; in one call with a product of 64 x 64
 WIDE = [(2176, 2048, 16), (2056, 2184, 72), (72, 136, 72), (136, 200, 160008)]
 WIDE_256 = [(1800, 1544, 3080), (1544, 1800, 3112), (64, 64, 64), (2048, 2048, 2056)]
+WIDE_HELPED = [(2816, 3080, 6008), (64, 64, 64), (3088, 2824, 6008)]     # 143 and 156 tiles: the idle CUs take the ends of the sums
 WIDE_ODD_K = [(2184, 2056, 33), (136, 200, 160001), (64, 64, 33), (1800, 1544, 3081)]
 WIDE_ODD_ROWS = [(2049, 2183, 72), (65, 129, 500008), (1, 3, 72), (1801, 1543, 3080)]
 
 
-@pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, s) for a in (True, False) for b in (True, False) for s in (WIDE, WIDE_256)] + [(False, False, WIDE_ODD_K), (True, True, WIDE_ODD_ROWS)])
+@pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, s) for a in (True, False) for b in (True, False) for s in (WIDE, WIDE_256, WIDE_HELPED)] + [(False, False, WIDE_ODD_K), (False, False, [(2816, 3080, 6001)]), (True, True, WIDE_ODD_ROWS)])
 @pytest.mark.parametrize("out,pad", [(torch.bfloat16, 8), (torch.bfloat16, 3), (torch.float32, 3)])
 def test_larger_tiles(a_k, b_k, shapes, out, pad):
     check(a_k, b_k, shapes, out, pad)
@@ -45,7 +46,8 @@ def check(a_k, b_k, shapes, out, pad):
         return t if along_k else t.t()
 
     for first in range(0, len(shapes), 4):
-        group, keep = (_lib.MambaGemm * 4)(), []
+        count, keep = len(shapes[first:first + 4]), []
+        group = (_lib.MambaGemm * 4)()
         for j, (M, N, K) in enumerate(shapes[first:first + 4]):
             A, B, bias = operand(M, K, a_k), operand(N, K, b_k), torch.randn(N, device="cuda", generator=gen).bfloat16()
             D = torch.full((M, N + pad), 0.5, device="cuda", dtype=out)
@@ -55,10 +57,10 @@ def check(a_k, b_k, shapes, out, pad):
             group[j] = _lib.MambaGemm(A.data_ptr(), B.data_ptr(), bias.data_ptr() if with_bias else None, D.data_ptr(), *A.stride(), *B.stride(),
                                       N + pad, M, N, K, _lib.DTYPE_CODE[out], int(accumulate), 0)
             keep.append((A, B, bias, D, want, size, K))
-        floats = lib.mamba_gemm_plan(group, 4)
+        floats = lib.mamba_gemm_plan(group, count)
         assert floats >= 0
         ws = torch.full((max(floats, 1),), float("nan"), device="cuda")
-        _lib.check(lib.mamba_gemm(group, 4, ws.data_ptr(), _lib.current_stream(ws.device)), "mamba_gemm")
+        _lib.check(lib.mamba_gemm(group, count, ws.data_ptr(), _lib.current_stream(ws.device)), "mamba_gemm")
         for A, B, bias, D, want, size, K in keep:
             N = want.shape[1]
             # fp32 sums of K terms, and one rounding to the result's type

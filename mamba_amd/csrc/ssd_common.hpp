@@ -855,6 +855,14 @@ DEVI View4 g_view(const SsdParams &p) {
 DEVI void load_async16(const void *base, uint32_t offset, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory", "m0");
 }
+// ... with an address of its own per lane
+DEVI void load_async16(const void *at, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(at), "s"(lds) : "memory", "m0");
+}
+// ... 4 bytes per lane
+DEVI void load_async4(const void *base, uint32_t offset, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dword %0, %1" ::"v"(offset), "s"(base), "s"(lds) : "memory", "m0");
+}
 template <int LEFT> DEVI void async_done() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory"); }
 
 // LDS address of a shared variable, as those loads and integer arithmetic take it

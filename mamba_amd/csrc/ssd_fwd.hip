@@ -366,114 +366,182 @@ template <int W, typename CT, bool TABLE> __global__ __launch_bounds__(256) void
 }
 
 // ------------------------------------------- chunk states and state passing in one pass
-// bf16, headdim 64, 128 states, chunks of Q = 32 R positions that tile the sequence: one workgroup per (batch, head)
-// walks the sequence once.  Per chunk it forms the chunk's own state (the product of chunk_state_fwd_wide_kernel,
-// a 64 x 128 tile, k = position), writes the state ENTERING the chunk (bf16, what the scan and the backward pass
-// read) and carries H <- decay_c H + S_c in fp32 registers; after the last chunk H is final_states.  The fp32
-// per-chunk states never exist in memory (configuration 2: 168 MB written and read again), and the recurrence over
-// the chunks costs no pass of its own.  With few workgroups (batch x heads) the loads must be deep instead: R pairs
-// of stagers hold the operands of the next R steps -- one chunk ahead -- and no branch surrounds a load or a store
-// of the walk, so each step waits for exactly its own operands.  The per-position weights w_s of chunk c + 1 are
-// computed while chunk c is multiplied (two tables in LDS), the per-chunk decay factors once at the start.
+// bf16, headdim 64, 128 states, chunks of Q = 64 NS positions that tile the sequence: four waves per (batch, head) walk the
+// sequence once, HH heads of a group to a workgroup.  Per chunk they write the state ENTERING the chunk (bf16, what the scan and
+// the backward pass read), form the chunk's own state S_c (128 states x 64, k = position) and carry H <- decay_c H + S_c in
+// fp32 registers; after the last chunk H is final_states.  The fp32 states of the chunks never exist in memory (4 x 4096
+// positions, 80 heads: 168 MB written and read again), and the recurrence over the chunks costs no pass of its own.
+// What bounds it is the rate at which a CU takes in rows (30 - 40 GB/s of x and B, whether they pass through registers or not
+// and however many are in flight: a walk without its products takes 2.2 - 2.6 us per chunk of 256, two of them on a CU twice
+// that).  So rows go to LDS as they are, by asynchronous loads that are two or three stages of 64 positions ahead in a ring of
+// stages, and two walks on one CU share those of B (HH = 2).  A wave owns 32 states: it multiplies its columns of B with
+// the weights of their positions as it reads them (nobody reads them twice), and all four read x.  States leave as 16 bytes a
+// lane (as 8 the same walk took 81 us where it takes 71).  The weights of chunk c + 1 are formed while chunk c is multiplied.
+// No branch surrounds a load or store of the walk: past the end the last stage comes once more, and each wait counts what was
+// issued behind the rows that it is for.  Rows through registers, the weighted ones written to LDS (before) / this, 80 heads
+// x 4096 positions: batch 2 59 / 47 us, batch 3 64 / 48, batch 4 91 / 71, batch 8 169 / 152; 128 heads in 8 groups x 2 x 32768
+// 451 / 423.
 constexpr int CSP_MAX_CHUNKS = 2048;
-template <int R, bool HAS_SEQ> __global__ __launch_bounds__(256) void chunk_state_passing_fwd_kernel(const SsdParams p) {
-  using T = bf16_t;
-  using SA = WideTrStager<false, T, 64>;
-  using SB = WideTrStager<false, T, WB>;
-  constexpr int Q = 32 * R, P = 64, N = WB;
-  static_assert(Q <= 256, "one table entry per thread");
-  __shared__ GemmLdsWide<false> lds;
-  __shared__ float wtab[2][Q];
-  __shared__ float dec[CSP_MAX_CHUNKS];
-  const int tid = threadIdx.x;
+template <int HH, int NS, bool HAS_SEQ> __global__ __launch_bounds__(256 * HH, 2) void chunk_state_passing_fwd_kernel(const SsdParams p) {
+  constexpr int NW = 4 * HH, KS = 64, Q = KS * NS, P = 64, N = 128, XH = KS * P * 2, XB = HH * XH, SB = XB + KS * N * 2, RING = HH == 1 ? 3 : 4, AHEAD = RING - 1;
+  constexpr int LOADS = SB / 1024 / NW, STORES = 4, TABLE = HAS_SEQ ? 5 : 3;  // of a wave: per stage; per chunk
+  constexpr auto behind = [](int st) {
+    int n = (AHEAD - 1) * LOADS;
+    for (int d = 1; d <= AHEAD; ++d) n += ((st - d + 4 * NS) % NS == NS - 1 ? STORES : 0) + (d < AHEAD && (st - d + 4 * NS) % NS == 0 ? TABLE : 0);
+    return n;
+  };
+  typedef __attribute__((address_space(3))) i16x4_t *lds_tr;
+  typedef __attribute__((address_space(3))) f32x4 *lds_f4;
+  typedef short i16x8_t __attribute__((ext_vector_type(8)));
+  __shared__ __align__(256) char ring[RING * SB];
+  __shared__ __align__(16) float wtab[HH][2][Q];
+  __shared__ __align__(256) float raw[NW][TABLE][64];  // a wave's entries of dA_cumsum, its last one, dt, the sequence and the last one
+  const int tid = threadIdx.x, lane = tid & 63, j = lane & 15, gq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), hd = wave >> 2, wn = wave & 3;
   const int L = p.seqlen, H = p.nheads, nc = p.nchunks;
-  const int h = blockIdx.x, b = blockIdx.y;
+  const int id = xcd_linear_block() * HH + hd;
+  const int h = id % H, b = id / H;
   const int g = h / (H / p.ngroups);
   const float *dA = p.dA_cumsum + ((int64_t)b * H + h) * nc * Q;
   const float *dtp = p.dt_out + ((int64_t)b * H + h) * nc * Q;
   const int32_t *seq = HAS_SEQ ? p.seq_idx + (int64_t)b * L : nullptr;
-  for (int c = tid; c < nc; c += 256) {  // carried-state factor of chunk c: 0 across a sequence boundary
-    float scale = fast_exp(dA[c * Q + Q - 1]);
-    if (HAS_SEQ) {
-      const int seq_new = seq[(c + 1) * Q - 1], seq_prev = c > 0 ? seq[c * Q - 1] : 0;
-      if (seq_new != seq_prev) scale = 0.f;
-    }
-    dec[c] = scale;
-  }
-  // w_s = dt_s exp(a_last - a_s) for the positions of the chunk's last sequence, else 0; entry min(tid, Q - 1)
-  const int ts = min(tid, Q - 1);
-  float t_a, t_alast, t_dt;
-  int t_sid = 0, t_slast = 0;
+  // w_s = dt_s exp(a_last - a_s) for the positions of the chunk's last sequence, else 0; entry min(tid, Q - 1).  The decay of a
+  // carried state over the chunk is 0 across a sequence boundary.  What they are formed of comes the same way as the rows, for
+  // the compiler would wait for loads of its own until nothing at all is in flight.
+  const int pos = min(wn * 64 + lane, Q - 1);
+  const uint32_t raw_at = lds_address(&raw[wave][0][0]), ts = pos * 4;
+  float decay;
+  int s_before = 0;
   auto table_request = [&](int c) {
-    t_a = *(const GLOBAL_AS float *)(dA + c * Q + ts);
-    t_alast = *(const GLOBAL_AS float *)(dA + c * Q + Q - 1);
-    t_dt = *(const GLOBAL_AS float *)(dtp + c * Q + ts);
+    load_async4(dA + c * Q, ts, raw_at);
+    load_async4(dA + c * Q, (Q - 1) * 4, raw_at + 256);
+    load_async4(dtp + c * Q, ts, raw_at + 512);
     if (HAS_SEQ) {
-      t_sid = *(const GLOBAL_AS int32_t *)(seq + c * Q + ts);
-      t_slast = *(const GLOBAL_AS int32_t *)(seq + c * Q + Q - 1);
+      load_async4(seq + c * Q, ts, raw_at + 768);
+      load_async4(seq + c * Q, (Q - 1) * 4, raw_at + 1024);
     }
   };
   auto table_write = [&](int c) {
-    float v = fast_exp(fminf(t_alast - t_a, 0.f)) * t_dt;
-    if (HAS_SEQ && !(t_slast >= 0 && t_sid == t_slast)) v = 0.f;
-    if (tid < Q) wtab[c & 1][tid] = v;
+    const float a = raw[wave][0][lane], a_last = raw[wave][1][lane], dt = raw[wave][2][lane];
+    float v = fast_exp(fminf(a_last - a, 0.f)) * dt;
+    decay = fast_exp(a_last);
+    if constexpr (HAS_SEQ) {
+      const int sid = __float_as_int(raw[wave][3][lane]), last = __float_as_int(raw[wave][4][lane]);
+      v = last >= 0 && sid == last ? v : 0.f;
+      decay = last == s_before ? decay : 0.f;
+      s_before = last;
+    }
+    if (wn * 64 < Q) wtab[hd][c & 1][pos] = v;
+  };
+
+  // rows -> LDS, 16 bytes a lane: 8 rows of x or 4 of B per instruction.  Units of 32 bytes are permuted within a row, so that
+  // the transposing reads of 16 rows meet in no bank.
+  const char *x_at = (const char *)(static_cast<const bf16_t *>(p.x) + b * p.x_bs + h * p.x_hs) + (lane >> 3) * (2 * p.x_ls) +
+                     ((lane & 7) ^ (lane >> 4) << 1) * 16;
+  const char *B_at = (const char *)(static_cast<const bf16_t *>(p.B) + b * p.B_bs + g * p.B_gs) + (lane >> 4) * (2 * p.B_ls) +
+                     ((lane & 15) ^ ((wave & 1) * 4 + (lane >> 4)) << 1) * 16;
+  const uint32_t lds0 = lds_address(&ring[0]), lds_end = lds0 + RING * SB;
+  auto request = [&](int pos, uint32_t lds) {
+#pragma unroll
+    for (int q = 0; q < KS / 32; ++q) load_async16(x_at + (pos + (q * 4 + wn) * 8) * (2 * p.x_ls), lds + hd * XH + (q * 4 + wn) * 1024);
+#pragma unroll
+    for (int q = 0; q < KS / 4 / NW; ++q) load_async16(B_at + (pos + (q * NW + wave) * 4) * (2 * p.B_ls), lds + XB + (q * NW + wave) * 1024);
   };
   table_request(0);
+#pragma unroll
+  for (int k = 0; k < AHEAD; ++k) request(min(k * KS, L - KS), lds0 + k * SB);
+
+  // H: rows (states) 32 wave + 16 tn + 4 gq + r, columns 16 pt + j
+  f32x4 Hs[2][4], acc[2][4];
+  const int64_t own = j * N + wn * 32 + gq * 4;  // (+ 16 tn, + 16 N pt)
+#pragma unroll
+  for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+    for (int pt = 0; pt < 4; ++pt) Hs[tn][pt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (p.initial_states) {
+    const float *init = p.initial_states + ((int64_t)b * H + h) * P * N + own;
+#pragma unroll
+    for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Hs[tn][pt][r] = init[pt * 16 * N + tn * 16 + r];
+  }
+  async_done<0>();  // (the first AHEAD stages)
   table_write(0);
 
-  // H in the accumulator layout: rows 32 wm + 16 tm + 4 g + r, columns 64 wn + 16 tn + i
-  GemmAccWide Hs, acc;
-  Hs.zero();
-  if (p.initial_states) {
-    const int lane = tid & 63, wave = tid >> 6, wm = wave >> 1, wn = wave & 1, i = lane & 15, gq = lane >> 4;
-    const float *init = p.initial_states + ((int64_t)b * H + h) * P * N;
-#pragma unroll
-    for (int tm = 0; tm < 2; ++tm)
-#pragma unroll
-      for (int tn = 0; tn < 4; ++tn)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          Hs.v[tm][tn][r] = init[(wm * 32 + tm * 16 + gq * 4 + r) * N + wn * 64 + tn * 16 + i];
-  }
-
-  const T *xa = static_cast<const T *>(p.x) + b * p.x_bs + h * p.x_hs;
-  const T *Ba = static_cast<const T *>(p.B) + b * p.B_bs + g * p.B_gs;
-  SA sa[R];
-  SB sb[R];
-  {
-    const SA sa0(lds.ah, lds.al, xa, p.x_ls, P, nullptr, tid);
-    const SB sb0(lds.bh, lds.bl, Ba, p.B_ls, WB, wtab[0], tid);
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-      sa[j] = sa0;
-      sb[j] = sb0;
-      sa[j].template fetch<true>(j * GK);
-      sb[j].template fetch<true>(j * GK);
-      // the requests leave in the order the walk consumes them: the waits in the loop are counted from the order
-      // on either way into it, and the compiler would otherwise issue these independent loads last pair first
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
-  bf16_t *carried = static_cast<bf16_t *>(p.states_lp) + ((int64_t)b * nc * H + h) * P * N;
+  GLOBAL_AS char *carried = (GLOBAL_AS char *)(static_cast<bf16_t *>(p.states_lp) + ((int64_t)b * nc * H + h) * P * N + j * N + wn * 32 + (gq & 1) * 16 + (gq & 2) * 4);
+  const int rr = 4 * gq + (j >> 2);  // this lane's row of a patch, and its place in it
+  const uint32_t xo = hd * XH + rr * 128 + (j & 3) * 8 + (rr >> 1 & 3) * 32, Bo = XB + rr * 256 + (j & 3) * 8 + ((rr & 7) ^ (wn * 2)) * 32;
+  uint32_t here = lds0, there = lds0 + AHEAD * SB;
 #pragma unroll 1
   for (int c = 0; c < nc; ++c) {
-    table_request(min(c + 1, nc - 1));
-    acc.zero();
-    const float *ks = &wtab[c & 1][0] - c * Q;  // the stagers index their weights by position in the sequence
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-      sb[j].kscale = ks;
-      wide_step(acc, lds, c * Q + j * GK, sa[j], sb[j], min(c * Q + (j + R) * GK, L - GK), tid);
+    for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+      for (int pt = 0; pt < 4; ++pt) acc[tn][pt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t w_at = lds_address(&wtab[hd][c & 1][4 * gq]);
+    const float d = decay;
+#pragma unroll
+    for (int st = 0; st < NS; ++st) {
+      // behind the rows of this stage are those of the AHEAD - 1 next, and what the chunks that ended and began meanwhile
+      // stored and asked for (the first AHEAD stages wait for nothing: they are there)
+      switch (st) {
+        case 0: async_done<behind(0)>(); break;
+        case 1: async_done<behind(1)>(); break;
+        case 2: async_done<behind(2)>(); break;
+        default: async_done<behind(3)>(); break;
+      }
+      lds_barrier();  // they are there in all waves, and nobody reads the stage before any more
+      if (st == 0) table_request(min(c + 1, nc - 1));
+      request(min(c * Q + (st + AHEAD) * KS, L - KS), there);
+#pragma unroll
+      for (int k = 0; k < KS; k += 32) {
+        const f32x4 w0 = *(lds_f4)(uintptr_t)(w_at + (st * KS + k) * 4), w1 = *(lds_f4)(uintptr_t)(w_at + (st * KS + k + 16) * 4);
+        auto patches = [&](uint32_t at, int row) {
+          const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)at);
+          const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_tr)(uintptr_t)(at + 16 * row));
+          return (i16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+        bf16x8_t bw[2];
+#pragma unroll
+        for (int tn = 0; tn < 2; ++tn) {
+          const u32x4 v = __builtin_bit_cast(u32x4, patches(here + (Bo ^ (tn * 32)) + k * 256, 256));
+          bw[tn] = __builtin_bit_cast(bf16x8_t, u32x4{pack_bf16(bf16_lo(v.x) * w0[0], bf16_hi(v.x) * w0[1]), pack_bf16(bf16_lo(v.y) * w0[2], bf16_hi(v.y) * w0[3]),
+                                                      pack_bf16(bf16_lo(v.z) * w1[0], bf16_hi(v.z) * w1[1]), pack_bf16(bf16_lo(v.w) * w1[2], bf16_hi(v.w) * w1[3])});
+        }
+#pragma unroll
+        for (int pt = 0; pt < 4; ++pt) {
+          const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, patches(here + (xo ^ (pt * 32)) + k * 128, 128));
+#pragma unroll
+          for (int tn = 0; tn < 2; ++tn) acc[tn][pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bw[tn], xf, acc[tn][pt], 0, 0, 0);
+        }
+      }
+      here = here + SB == lds_end ? lds0 : here + SB;
+      there = there + SB == lds_end ? lds0 : there + SB;
     }
-    table_write(c + 1);  // read from the next step's first barrier on; last read two chunks ago
-    store_wide_rows<false, bf16_t, false>(Hs, lds, carried + (int64_t)c * H * P * N, N, P, tid);
-    const float d = dec[c];
+    async_done<NS * LOADS>();
+    table_write(c + 1);  // read from the next stage's barrier on; last read a chunk ago
+    // 16 bytes a lane: the even rows of lanes take the values of two rows of the first tile, the odd ones those of the second
 #pragma unroll
-    for (int tm = 0; tm < 2; ++tm)
+    for (int pt = 0; pt < 4; ++pt) {
+      const f32x4 u = Hs[0][pt], v = Hs[1][pt];
+      const auto lo = __builtin_amdgcn_permlane16_swap(pack_bf16(u[0], u[1]), pack_bf16(v[0], v[1]), false, false);
+      const auto hi = __builtin_amdgcn_permlane16_swap(pack_bf16(u[2], u[3]), pack_bf16(v[2], v[3]), false, false);
+      *(GLOBAL_AS u32x4 *)(carried + pt * (32 * N)) = u32x4{(uint32_t)lo[0], (uint32_t)hi[0], (uint32_t)lo[1], (uint32_t)hi[1]};
 #pragma unroll
-      for (int tn = 0; tn < 4; ++tn) Hs.v[tm][tn] = Hs.v[tm][tn] * d + acc.v[tm][tn];
+      for (int tn = 0; tn < 2; ++tn)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Hs[tn][pt][r] = Hs[tn][pt][r] * d + acc[tn][pt][r];
+    }
+    carried += (int64_t)H * P * N * 2;
   }
-  store_wide_rows<false, float, false>(Hs, lds, p.final_states + ((int64_t)b * H + h) * P * N, N, P, tid);
+  async_done<0>();  // (the requests past the end)
+  float *last = p.final_states + ((int64_t)b * H + h) * P * N + own;
+#pragma unroll
+  for (int pt = 0; pt < 4; ++pt)
+#pragma unroll
+    for (int tn = 0; tn < 2; ++tn) *reinterpret_cast<f32x4 *>(last + pt * 16 * N + tn * 16) = Hs[tn][pt];
 }
 
 // ------------------------------------------------------------- chunk_scan
@@ -724,27 +792,35 @@ static bool chunk_state_passing_shapes_ok(const SsdParams *p) {
          wide_operand_ok(p->x, p->dtype, p->x_bs, p->x_ls, p->x_hs) && wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs);
 }
 // The combined forward pass takes it where there are enough (batch, head) pairs for one workgroup each to keep the
-// chip busy: a workgroup takes ~3.7 us per chunk of 256 whatever their number (its LDS traffic per k step is that of
-// chunk_state_fwd_wide_kernel, and that is what bounds both), the two-kernel path ~24 ns per (batch, head, chunk).
-// Measured at 80 heads x 4096 positions, walk / two kernels: batch 2 61 / 51 us, batch 3 65 / 95, batch 4 95 / 128
-// (320 workgroups on 256 CUs: a quarter of the CUs do double duty), batch 8 169 / 252; one packed row of 64 heads x
-// 32768 positions 436 / 195.
+// chip busy: a workgroup takes ~3 us per chunk of 256 whatever their number, the two-kernel path ~24 ns per (batch, head, chunk).
+// Walk / two kernels: 128 pairs x 4096 positions 46.8 / 47.9 us, x 2048 in chunks of 128 33.2 / 36.2, x 16384 in 8 groups
+// 198 / 199; 160 pairs x 4096 47 / 52, x 512 in chunks of 128 12.6 / 21; 176 pairs in 8 groups 48 / 67; 240 pairs 48 / 95; 320
+// 71 / 128; one packed row of 64 heads x 32768 positions 436 / 195 (before).
+// With fewer than three pairs to four CUs, only where the two kernels need a launch for the steps' sums as well (sums_in_states,
+// below): the whole forward pass of 128 pairs x 2048 positions 70.2 / 69.8, x 512 in chunks of 128 27.2 / 27.9 with the walk.
+static bool sums_in_states(const SsdParams *p) { return (int64_t)p->nchunks * p->batch * p->nheads <= 8 * (int64_t)cu_count(); }
 static bool chunk_state_passing_pays(const SsdParams *p) {
-  return chunk_state_passing_shapes_ok(p) && (int64_t)p->batch * p->nheads >= cu_count() * 3 / 4;
+  const int64_t pairs = (int64_t)p->batch * p->nheads, cus = cu_count();
+  return chunk_state_passing_shapes_ok(p) && (pairs >= cus * 3 / 4 || (pairs >= cus / 2 && !sums_in_states(p)));
+}
+template <int HH, int NS> static void launch_state_walk(const SsdParams &p, hipStream_t s) {
+  const dim3 grid((uint32_t)p.nheads * (uint32_t)p.batch / HH), block(256 * HH);
+  if (p.seq_idx) hipLaunchKernelGGL((chunk_state_passing_fwd_kernel<HH, NS, true>), grid, block, 0, s, p);
+  else hipLaunchKernelGGL((chunk_state_passing_fwd_kernel<HH, NS, false>), grid, block, 0, s, p);
 }
 extern "C" int ssd_chunk_state_passing_fwd(const SsdParams *p, mamba_stream_t stream) {
   int rc = check(p);
   if (rc) return rc;
   if (!chunk_state_passing_shapes_ok(p)) return MAMBA_E_UNSUPPORTED;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  dim3 grid(p->nheads, p->batch);
-  if (p->chunk_size == 256) {
-    if (p->seq_idx) hipLaunchKernelGGL((chunk_state_passing_fwd_kernel<8, true>), grid, dim3(256), 0, s, *p);
-    else hipLaunchKernelGGL((chunk_state_passing_fwd_kernel<8, false>), grid, dim3(256), 0, s, *p);
-  } else {
-    if (p->seq_idx) hipLaunchKernelGGL((chunk_state_passing_fwd_kernel<4, true>), grid, dim3(256), 0, s, *p);
-    else hipLaunchKernelGGL((chunk_state_passing_fwd_kernel<4, false>), grid, dim3(256), 0, s, *p);
-  }
+  // Two heads to a workgroup where more than half of the last round's workgroups (one of two heads, or two of one, to a CU) are
+  // there: one CU then takes in 128 KB per chunk for two walks instead of 192.  Else CUs would idle that can have a walk each.
+  // One head / two, 4096 positions, chunks of 256: 256 walks 49 / 61 us, 320 90 / 71, 384 105 / 83, 448 108 / 88, 512 111 / 95;
+  // 560 145 / 156, 640 152 / 163; 768 173 / 166, 896 196 / 169, 1024 (8 groups) 220 / 195.
+  const int64_t walks = (int64_t)p->nheads * p->batch, cus = cu_count(), left = walks % (2 * cus);
+  const bool two = p->nheads / p->ngroups % 2 == 0 && walks > cus && (left == 0 || left >= cus);
+  if (p->chunk_size == 256) two ? launch_state_walk<2, 4>(*p, s) : launch_state_walk<1, 4>(*p, s);
+  else two ? launch_state_walk<2, 2>(*p, s) : launch_state_walk<1, 2>(*p, s);
   return launched();
 }
 
@@ -755,7 +831,7 @@ static int ssd_combined_fwd_one(const SsdParams *p, mamba_stream_t stream) {
   // The steps and their sums: a launch of their own where there is much to do, in the chunk_state kernel (whose workgroups
   // then read the strided steps of their chunk one by one) while that has no more than eight workgroups per CU: 1531 x 80
   // heads 6.6 + 12.9 us against 15.1, 2 x 1000 x 24 5.4 + 10.2 against 11.9.
-  const bool merged = !walk && (int64_t)p->nchunks * p->batch * p->nheads <= 8 * (int64_t)cu_count();
+  const bool merged = !walk && sums_in_states(p);
   if (!merged && (rc = ssd_chunk_cumsum_fwd(p, stream))) return rc;
   if (walk) {
     if ((rc = ssd_chunk_state_passing_fwd(p, stream))) return rc;

@@ -50,6 +50,17 @@ def test_one_launch_matches_the_two_stages(batch, seqlen, nheads, ngroups, chunk
     assert float((c1 == c2).float().mean()) > 0.999
 
 
+@pytest.mark.parametrize("batch,seqlen,nheads,ngroups,chunk,seq_lens,has_init", [
+    (2, 512, 130, 1, 256, None, True),                  # 260 pairs: two heads of a group share its rows of B
+    (1, 768, 288, 8, 128, [200, 56, 1, 511], True),     # ... 18 pairs of heads in each of 8 groups
+    (3, 128, 96, 2, 128, None, False),                  # one chunk, shorter than what is asked for ahead
+    (1, 512, 264, 88, 256, [300, 212], True),           # three heads in a group: one to a workgroup, more of them than CUs
+    (1, 1024, 200, 40, 128, None, True),                # five in a group, fewer than CUs
+])
+def test_walks_that_share_a_compute_unit(batch, seqlen, nheads, ngroups, chunk, seq_lens, has_init):
+    test_one_launch_matches_the_two_stages(batch, seqlen, nheads, ngroups, chunk, seq_lens, has_init)
+
+
 def test_one_launch_declines_other_shapes():
     from mamba_amd import _lib
     from mamba_amd.ops.triton import ssd_combined as sc

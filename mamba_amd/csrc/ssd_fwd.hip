@@ -10,7 +10,8 @@ namespace {
 // One workgroup per (batch, chunk, 4 heads); thread = position inside the chunk, so loads of
 // dt (head-contiguous) are 4 consecutive elements per thread and the stores of dt_out / dA_cumsum
 // (position-contiguous) are coalesced.  (The kernel is a chain of short latencies, so it wants many small
-// workgroups: 15.5 us with 16 heads per workgroup at batch 4 x 16 chunks x 80 heads, 11.1 with 4, 10.2 with 2.)  dt -> (+bias, softplus, clamp), zero past the end of the
+// workgroups: 15.5 us with 16 heads per workgroup at batch 4 x 16 chunks x 80 heads, 11.1 with 4, 10.2 with 2, when each load was waited for
+// before the next; 8.9 with 4 heads' loads in flight together.)  dt -> (+bias, softplus, clamp), zero past the end of the
 // sequence; dA_cumsum = running sum of dt * A over the chunk (wave DPP scan + cross-wave offsets).
 constexpr int CS_HT = 4;
 
@@ -31,22 +32,33 @@ __global__ __launch_bounds__(256) void chunk_cumsum_fwd_kernel(const SsdParams p
   const int c = blockIdx.x, h0 = blockIdx.y * CS_HT, b = blockIdx.z;
   const int t = c * Q + l;
   const bool live = l < Q && t < p.seqlen;
-  float dtv[CS_HT], cs[CS_HT];
+  float dtv[CS_HT], cs[CS_HT], A[CS_HT], bias[CS_HT];
+  // every load before the first use of any: the type is asked for once, heads and positions past the end repeat the last
+  const float *const bp = static_cast<const float *>(p.dt_bias ? p.dt_bias : p.A);
 #pragma unroll
   for (int i = 0; i < CS_HT; ++i) {
-    const int h = h0 + i;
-    float dt = 0.f, A = 0.f;
-    if (h < H) {
-      A = static_cast<const float *>(p.A)[h];
-      if (live) {
-        dt = ld_dyn(p.dt, b * p.dt_bs + (int64_t)t * p.dt_ls + h * p.dt_hs, p.dt_dtype);
-        if (p.dt_bias) dt += static_cast<const float *>(p.dt_bias)[h];
-        if (p.dt_softplus) dt = softplus_f(dt);
-        dt = fminf(fmaxf(dt, p.dt_min), p.dt_max);
-      }
-    }
+    const int h = min(h0 + i, H - 1);
+    A[i] = static_cast<const float *>(p.A)[h];
+    bias[i] = bp[h];
+  }
+  auto load = [&](auto type) {
+    const auto *row = reinterpret_cast<const decltype(type) *>(p.dt) + b * p.dt_bs + (int64_t)min(t, p.seqlen - 1) * p.dt_ls;
+#pragma unroll
+    for (int i = 0; i < CS_HT; ++i) dtv[i] = ld1(row + min(h0 + i, H - 1) * p.dt_hs);
+  };
+  switch (p.dt_dtype) {
+    case MAMBA_BF16: load(bf16_t{}); break;
+    case MAMBA_F16: load(f16_t{}); break;
+    default: load(float{}); break;
+  }
+#pragma unroll
+  for (int i = 0; i < CS_HT; ++i) {
+    float dt = dtv[i];
+    if (p.dt_bias) dt += bias[i];
+    if (p.dt_softplus) dt = softplus_f(dt);
+    dt = live ? fminf(fmaxf(dt, p.dt_min), p.dt_max) : 0.f;
     dtv[i] = dt;
-    cs[i] = wave_incl_sum(dt * A);
+    cs[i] = wave_incl_sum(dt * A[i]);
     if (lane == 63) wtot[wave][i] = cs[i];
   }
   __syncthreads();

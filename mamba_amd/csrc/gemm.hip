@@ -743,6 +743,16 @@ int form_of(const MambaGemm &g) {
   if (flop > 16e9 && tiles_of(g, TILE256) >= 48) return TILE256;
   return flop > 8e9 || tiles_of(g, TILE128) >= cu_count() ? TILE128 : TILE64;
 }
+// The form of a product among those of one call: up to 8 GFLOP it stays in 64 x 64 tiles where another product of the call is in
+// them, for launches of two forms run one after the other and each with an end of its own (the two gradients of a 768 x 1536
+// projection over 3136 rows, the one 128 x 128 uncut and the other cut: 19 + 30 us, in one launch of 64 x 64 43).
+int form_in(const MambaGemm *g, int i, int count) {
+  const int f = form_of(g[i]);
+  if (f != TILE128 || 2.0 * g[i].M * g[i].N * g[i].K > 8e9) return f;
+  for (int k = 0; k < count; ++k)
+    if (ring(g[k]) && form_of(g[k]) == TILE64) return TILE64;
+  return f;
+}
 // Parts of the sum over k.  64 x 64: as many as give every CU two workgroups, of at least 8 steps (256 elements) each.  The others: the
 // least of a stage's time by the workgroups on a CU, measured at 18 to 800 tiles in up to 32 parts, and what the parts' writing,
 // reading and second launch take.
@@ -808,7 +818,7 @@ extern "C" int64_t mamba_gemm_plan(MambaGemm *g, int count) {
   for (int i = 0; i < count; ++i) {
     g[i].nsplit = 1;
     if (!valid(g[i])) return MAMBA_E_BADARG;
-    const int f = form_of(g[i]);
+    const int f = form_in(g, i, count);
     const int64_t steps = (g[i].K + GK - 1) / GK, want = splits_of(g[i], f);
     if (want > 1) {
       const int64_t per = (steps + want - 1) / want;
@@ -823,7 +833,7 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
   if (!g || count < 1 || count > MAXG) return MAMBA_E_BADARG;
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (int i = 0; i < count; ++i) {
-    if (!valid(g[i]) || (parts_of(g[i], form_of(g[i])) && !ws)) return MAMBA_E_BADARG;
+    if (!valid(g[i]) || (parts_of(g[i], form_in(g, i, count)) && !ws)) return MAMBA_E_BADARG;
   }
   // the products of one form in a launch, those with helpers (every workgroup leaves parts) apart from the others
   for (int form = FORMS; form >= 0; --form) {
@@ -834,7 +844,7 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
     bool all = true;
     const int per_tile = TILE[f] * TILE[f] / (f == TILE256 ? 2048 : 1024);  // workgroups that add up its splits
     for (int i = 0; i < count; ++i) {
-      if (form_of(g[i]) != f) continue;
+      if (form_in(g, i, count) != f) continue;
       const int64_t tiles = tiles_of(g[i], f);
       const int helpers = helpers_of(tiles, g[i].nsplit, g[i].K, f);
       if ((helpers > 0) != helped) continue;

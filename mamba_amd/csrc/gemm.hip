@@ -799,16 +799,19 @@ template <int WX, int WY, int FX, int FY, int ST, bool HELP> void launch_wide(co
 }  // namespace
 
 // Where the library takes over.  Up to 8 GFLOP its host time and choice of tiles cost more than any of these forms (whole mixer
-// calls, forward + backward, library / own: products up to 0.5 GFLOP 350 / 180 us, up to 5 GFLOP 432 / 398); up to 16 GFLOP the
-// larger tiles take its time or less (2560 x 2000 x 1280: 26 / 29, 192 x 8192 x 5120: 36 / 47, 2000 x 1280 x 2560: 32 / 30 with
-// 18 us less of host time).  Beyond: sums over a long k into few tiles (weight gradients), which it does not split, and short k with
-// a result that the last-level cache holds (5120 x 16384 x 160: 47 / 57; twice as long 139 / 114).
+// calls, forward + backward, library / own: products up to 0.5 GFLOP 350 / 180 us, up to 5 GFLOP 432 / 398).  Up to 16 GFLOP, by 270
+// products of 20 - 30 us (the library up to 75): where both operands lie along k it takes 0.78 - 0.9 of the larger tiles' time; where
+// k is below the larger side the two are within 10 % by themselves and a whole call is no faster with own products (1 x 1536 x
+// 2560: 277 / 286); k up to twice that, a projection to half the width, 27 / 33; sums over a longer k, weight gradients, take 0.4 -
+// 0.8 of its time (calls of 4 x 1000 x 1792 409 / 394, 8 x 1000 x 1280 519 / 500).  Beyond: sums over a long k into few tiles, which it
+// does not split, and short k with a result that the last-level cache holds (5120 x 16384 x 160: 47 / 57; twice as long 139 / 114).
 extern "C" int mamba_gemm_suits(const MambaGemm *g) {
   if (!g) return 0;
   const double flop = 2.0 * g->M * g->N * g->K;
   if (flop <= 8e9) return 1;
   if (!ring(*g)) return 0;
-  return flop <= 16e9 || (g->K >= 3 * (int64_t)std::max(g->M, g->N) && tiles_of(*g, TILE256) < cu_count()) ||
+  if (flop <= 16e9 && (g->a_ks != 1 || g->b_ks != 1) && g->K > 2 * (int64_t)std::max(g->M, g->N)) return 1;
+  return (g->K >= 3 * (int64_t)std::max(g->M, g->N) && tiles_of(*g, TILE256) < cu_count()) ||
          (g->K <= 256 && (int64_t)g->M * g->N <= 100000000);
 }
 

@@ -987,14 +987,16 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
 // positions; within 10 % of almost all).  A tile of a round of backward workgroups (one per CU) takes 13 per pass and a
 // third of that for what the passes share, a round's start and end 5.3.  The pass over the segments (all but one) takes 2.7
 // (forward) or 4.5 (backward) a tile, twice that from four of its workgroups per CU on, and every segment 0.9 or 1.8 for
-// its launch and for going through the segments before it.  A split has to promise 1 % (forward) or 6 % (backward).
+// its launch and for going through the segments before it; forward segments of a single tile, which a second launch and its wait for
+// the first outweigh, no less than 3.5 together.  A split has to promise 1 % (forward) or 6 % (backward).
 // Forward scans that only scan_fwd_kernel takes (fwd_cost) keep the terms that were fitted to them: 6.4 a tile of a round of up
 // to two workgroups per CU, half as much again where two share one, 3.0 for a tile of the pass over the segments, 6 % to
 // promise.  (The terms for 16 states cut them too finely: 2 x 4160 x 1261, 4 states, 53 us whole and 70 in five segments; 2 x
 // 1552 x 4029, 64 states, 420 us in five and 501 in 32.)
-// Measured: 1536 channels x 777 positions of one sequence 36 -> 22.5 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181
-// forward; 1536 channels x 256 whole and in two segments 12.7 and 13.7, x 777 in one, two, three, four and seven 36, 33, 28, 28.5
-// and 24.5 (each over and over on the same inputs).
+// Measured: 1536 channels x 777 positions of one sequence 35 -> 23 us forward, 133 -> 63 backward; 6 x 944 x 4251: 242 -> 181
+// forward.  Forward, 1536 channels, whole and in segments: x 192 12.4 and 14.0 (two), x 256 12.3 and 13.7 (two), x 384 17.2, 19.8 (two) and
+// 14.9 (three), x 777 35 and 32, 27, 28 and 23 (two, three, four, seven); 2 x 1536 x 257 18.2 and 21.3 (three).  (Asked of longer
+// segments as well, the 3.5 cut 3 x 2880 x 1897 in fifteen instead of three: 151 for 140.)
 constexpr int MAX_SEGMENTS = 32;
 int scan_segments(const MambaScanParams &p, bool bwd) {
   const int ntiles = (p.seqlen + TILE - 1) / TILE, Dg = p.dim / p.ngroups, cus = compute_units();
@@ -1020,7 +1022,8 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
     }
     if (s > 1) {
       const double share = std::max(1.0, 0.52 * (double)((seg_wgs * (s - 1) + cus - 1) / cus));
-      cost = (fine ? 1.01 : 1.06) * (cost + (bwd ? 4.5 : fine ? 2.7 : 3.0) * share * blocks * per + (bwd ? 1.8 : 0.9) * s);
+      const double each = bwd ? 1.8 * s : fine && per == 1 ? std::max(3.5, 0.9 * s) : 0.9 * s;
+      cost = (fine ? 1.01 : 1.06) * (cost + (bwd ? 4.5 : fine ? 2.7 : 3.0) * share * blocks * per + each);
     }
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = s;
   }

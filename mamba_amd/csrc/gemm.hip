@@ -503,26 +503,26 @@ template <int WX, int WY, int FX, int FY> DEVI void wide_place4(int q, int tid, 
   n = (nt * WX + wx) * (FX * 16) + (q / FY) * 16 + (lane >> 4) * 4;
 }
 
-// How the stages of a product's units (tile, part of k) are shared out where the units leave `helpers` CUs idle: a unit's own
-// workgroup takes its first `own` stages, so that all end together, and the helpers the rest of the units, `rest` stages each laid
+// How the stages of a product's tiles are shared out where the tiles, their sums whole, leave `helpers` CUs idle: a tile's own
+// workgroup takes its first `own` stages, so that all end together, and the helpers the rest of the tiles, `rest` stages each laid
 // end to end, `span` stages per helper.  (Own workgroups walk k side by side, which keeps what neighbouring tiles share in the
 // L2.)  2560 x 5120 x 32768, 200 tiles on 256 CUs: 832 -> 754 us (1.14 PFLOP/s).
 struct Share {
-  int units, stages, per, own, rest, helpers, span, pieces;  // pieces of units a helper may touch
-  __host__ __device__ Share(int tiles, int nsplit, int helpers_, int K)
-      : units(tiles * nsplit), stages((K + WK - 1) / WK), per((stages + nsplit - 1) / nsplit), helpers(helpers_) {
-    own = helpers ? (int)(((int64_t)per * units + units + helpers - 1) / (units + helpers)) : per;
-    rest = per - own;
-    span = helpers ? (units * rest + helpers - 1) / helpers : 0;
-    pieces = rest ? span / rest + 2 : 0;
+  int tiles, own, rest, helpers, span;
+  __host__ __device__ Share(int tiles_, int helpers_, int K) : tiles(tiles_), helpers(helpers_) {
+    const int stages = (K + WK - 1) / WK;
+    own = helpers ? (int)(((int64_t)stages * tiles + tiles + helpers - 1) / (tiles + helpers)) : stages;
+    rest = stages - own;
+    span = helpers ? (int)(((int64_t)tiles * rest + helpers - 1) / helpers) : 0;
   }
-  __host__ __device__ int64_t slots() const { return units + (int64_t)helpers * pieces; }
-  // what helper h takes of unit u, from stage [0] to [1] of the whole k; its place is h * pieces + u - h * span / rest
-  DEVI void part(int h, int u, int tiles, int &from, int &to) const {
-    const int u0 = u * rest, first = u / tiles * per;
-    from = first + own + max(h * span - u0, 0);
-    to = min(min(first + own + min((h + 1) * span - u0, rest), first + per), stages);
+  // what helper h takes of tile u: stages [from, to), none where from >= to
+  DEVI void part(int h, int u, int &from, int &to) const {
+    from = own + max(h * span - u * rest, 0);
+    to = own + min((h + 1) * span - u * rest, rest);
   }
+  // places of the parts: the own ones', then the helpers', whose h and u both only grow from one part to the next
+  DEVI int place(int h, int u) const { return tiles + h + u; }
+  __host__ __device__ int64_t places() const { return 2 * (int64_t)tiles + helpers - 1; }
 };
 
 template <int WX, int WY, int FX, int FY, int ST, bool HELP>
@@ -533,27 +533,22 @@ __global__ __launch_bounds__(64 * WX * WY, WX * WY == 4 ? 3 : 2) void gemm_wide_
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), i = product_of(a, blockIdx.x), wx = wave % WX, wy = wave / WX;
   const MambaGemm &g = a.g[i];
   const int ntn = (g.N + W::rx - 1) / W::rx, ntm = (g.M + W::ry - 1) / W::ry, tiles = ntn * ntm;
-  const Share share(tiles, g.nsplit, HELP ? a.helpers[i] : 0, g.K);
   // consecutive tiles of the shorter side, which share the longer side's operand, on one XCD
-  const int block = xcd_run(blockIdx.x - a.first[i], share.units + share.helpers);
+  const int block = xcd_run(blockIdx.x - a.first[i], HELP ? tiles + a.helpers[i] : tiles * g.nsplit);
   WideAcc<FX, FY> acc;
   const uint32_t at = lds_address(sh);
-  auto leave = [&](int64_t slot) {  // for the kernel that adds the parts up
-    float *part = a.ws[i] + slot * (W::rx * W::ry);
+  auto leave = [&](int64_t place) {  // for the kernel that adds the parts up
+    float *part = a.ws[i] + place * (W::rx * W::ry);
 #pragma unroll
     for (int q = 0; q < FX * FY; ++q) *reinterpret_cast<f32x4 *>(part + (q * W::waves * 64 + tid) * 4) = acc.v[q / FY][q % FY];
   };
-  auto tile_at = [&](int unit, int &mt, int &nt) {
-    const int tile = unit % tiles;
+  auto tile_at = [&](int tile, int &mt, int &nt) {
     mt = ntm < ntn ? tile % ntm : tile / ntn, nt = ntm < ntn ? tile / ntm : tile % ntn;
   };
-  const bool helper = HELP && block >= share.units;
   auto run = [&](auto x_tr, auto y_tr) {
     constexpr bool XTR = decltype(x_tr)::value, YTR = decltype(y_tr)::value;
-    auto product = [&](int unit, int from, int to) {
+    auto product = [&](int from, int to, int mt, int nt) {
       const int k0 = from * WK, k1 = min(to * WK, g.K);
-      int mt, nt;
-      tile_at(unit, mt, nt);
 #pragma unroll
       for (int q = 0; q < FX * FY; ++q) acc.v[q / FY][q % FY] = f32x4{0.f, 0.f, 0.f, 0.f};
       // (a part's k ends where the next one's begins)
@@ -561,22 +556,26 @@ __global__ __launch_bounds__(64 * WX * WY, WX * WY == 4 ? 3 : 2) void gemm_wide_
       const WideRing<YTR, W::loads_y, W::waves> Y(g.A, g.a_ms, g.a_ks, mt * W::ry, g.M, k1, wave, lane);
       run_wide<W>(acc, at, X, Y, k0, k1, wx, wy, lane);
     };
+    int mt, nt;
     if constexpr (HELP) {
-      const int h = block - share.units, u0 = helper ? h * share.span / share.rest : block;
+      const Share share(tiles, a.helpers[i], g.K);
+      const bool helper = block >= tiles;
+      const int h = block - tiles, u0 = helper ? h * share.span / share.rest : block, u1 = helper ? ((h + 1) * share.span - 1) / share.rest : block;
 #pragma unroll 1
-      for (int u = u0; u < min(u0 + (helper ? share.pieces : 1), share.units); ++u) {
-        int from = u / tiles * share.per, to = min(from + share.own, share.stages);
-        if (helper) share.part(h, u, tiles, from, to);
-        if (from >= to) continue;
+      for (int u = u0; u <= min(u1, tiles - 1); ++u) {
+        int from = 0, to = share.own;
+        if (helper) share.part(h, u, from, to);
         // (a new value to the compiler: what derives from it is formed where it is used instead of being carried along)
         asm volatile("" : "+v"(tid));
         lane = tid & 63;
-        product(u, from, to);
-        leave(helper ? share.units + (int64_t)h * share.pieces + u - u0 : block);
+        tile_at(u, mt, nt);
+        product(from, to, mt, nt);
+        leave(helper ? share.place(h, u) : u);
       }
     } else {
-      const int from = block / tiles * share.per;
-      product(block, from, min(from + share.per, share.stages));
+      const int stages = (g.K + WK - 1) / WK, per = (stages + g.nsplit - 1) / g.nsplit, from = block / tiles * per;
+      tile_at(block % tiles, mt, nt);
+      product(from, min(from + per, stages), mt, nt);
     }
   };
   const bool btr = g.b_ks != 1, atr = g.a_ks != 1;
@@ -585,12 +584,12 @@ __global__ __launch_bounds__(64 * WX * WY, WX * WY == 4 ? 3 : 2) void gemm_wide_
   else if (atr) run(std::false_type{}, std::true_type{});
   else run(std::false_type{}, std::false_type{});
   if constexpr (HELP) return;
-  int mt, nt;
-  tile_at(block, mt, nt);
   if (g.nsplit > 1) {
     leave(block);
     return;
   }
+  int mt, nt;
+  tile_at(block, mt, nt);
   // whole rows of 16-byte pieces where D allows, 16 rows at a time through a patch of the wave's own
   const bool rows = g.d_dtype == MAMBA_BF16 && ((uintptr_t)g.D & 15) == 0 && g.ldd % 8 == 0 && g.N % 8 == 0;
   if (!rows) {
@@ -673,23 +672,16 @@ template <int WX, int WY, int FX, int FY> __global__ __launch_bounds__(64 * WX *
   const MambaGemm &g = a.g[i];
   const int ntn = (g.N + W::rx - 1) / W::rx, ntm = (g.M + W::ry - 1) / W::ry, tiles = ntn * ntm;
   const int block = blockIdx.x - a.first[i], tile = block / QN, q = block % QN;
-  const Share share(tiles, g.nsplit, a.helpers[i], g.K);
   int m, n;
   wide_place4<WX, WY, FX, FY>(q, tid, ntm < ntn ? tile % ntm : tile / ntn, ntm < ntn ? tile / ntm : tile % ntn, m, n);
   const float *part = a.ws[i] + (q * W::waves * 64 + tid) * 4;
-  auto at = [&](int64_t slot) { return *reinterpret_cast<const f32x4 *>(part + slot * (W::rx * W::ry)); };
+  auto at = [&](int64_t place) { return *reinterpret_cast<const f32x4 *>(part + place * (W::rx * W::ry)); };
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
   for (int s = 0; s < g.nsplit; ++s) v += at(s * tiles + tile);
-  if (share.rest) {
-    for (int s = 0; s < g.nsplit; ++s) {
-      const int u = s * tiles + tile;
-      for (int h = u * share.rest / share.span; h * share.span < (u + 1) * share.rest; ++h) {
-        int from, to;
-        share.part(h, u, tiles, from, to);
-        if (from < to) v += at(share.units + (int64_t)h * share.pieces + u - h * share.span / share.rest);
-      }
-    }
+  if (a.helpers[i]) {
+    const Share share(tiles, a.helpers[i], g.K);
+    for (int h = tile * share.rest / share.span; h * share.span < (tile + 1) * share.rest; ++h) v += at(share.place(h, tile));
   }
   store4(g, m, n, v);
 }
@@ -757,19 +749,19 @@ int form_in(const MambaGemm *g, int i, int count) {
 // least of a stage's time by the workgroups on a CU, measured at 18 to 800 tiles in up to 32 parts, and what the parts' writing,
 // reading and second launch take.
 double us_of(int64_t tiles, int splits, int helpers, int K, int f) {
-  const Share share((int)tiles, splits, helpers, K);
-  const int64_t units = share.units, cus = cu_count();
+  const int64_t units = tiles * splits, cus = cu_count(), stages = (K + WK - 1) / WK;
   const double stage = f == TILE256 ? 0.82 : units <= cus ? 0.37 : units <= 2 * cus ? 0.41 : 0.62;
   const int64_t parts = (splits > 1 || helpers ? units : 0) + (helpers ? units + helpers : 0);
-  return share.own * stage + (parts ? 6 + parts * TILE[f] * TILE[f] * 2e-6 : 0);
+  return (helpers ? Share((int)tiles, helpers, K).own : (stages + splits - 1) / splits) * stage + (parts ? 6 + parts * TILE[f] * TILE[f] * 2e-6 : 0);
 }
-// CUs that the units of 256 x 256 tiles leave idle and that are worth their parts
-int helpers_of(int64_t tiles, int splits, int K, int f) {
-  const int64_t units = tiles * splits, idle = cu_count() - units;
+// CUs that 256 x 256 tiles with whole sums leave idle and that are worth their parts.  (With the sums cut as well they never are, by
+// these estimates at 48 to 255 tiles.)
+int helpers_of(int64_t tiles, int K, int f) {
+  const int64_t idle = cu_count() - tiles;
   if (f != TILE256 || idle <= 0) return 0;
-  const Share share((int)tiles, splits, (int)idle, K);
-  if (!share.rest || units * share.rest >= 1 << 30) return 0;
-  return us_of(tiles, splits, (int)idle, K, f) < 0.97 * us_of(tiles, splits, 0, K, f) ? (int)idle : 0;
+  const Share share((int)tiles, (int)idle, K);
+  if (!share.rest || tiles * share.rest >= 1 << 30) return 0;
+  return us_of(tiles, 1, (int)idle, K, f) < 0.97 * us_of(tiles, 1, 0, K, f) ? (int)idle : 0;
 }
 int splits_of(const MambaGemm &g, int f) {
   const int64_t tiles = tiles_of(g, f), steps = (g.K + GK - 1) / GK, cus = cu_count();
@@ -778,17 +770,18 @@ int splits_of(const MambaGemm &g, int f) {
   double least = 1e30;
   const int64_t most = std::min<int64_t>((f == TILE256 ? 1 : 3) * cus / tiles, steps / 8);
   for (int s = 1; s == 1 || s <= most; ++s) {
-    const double us = us_of(tiles, s, helpers_of(tiles, s, g.K, f), g.K, f);
+    const double us = us_of(tiles, s, s == 1 ? helpers_of(tiles, g.K, f) : 0, g.K, f);
     if (us < least) least = us, best = s;
   }
   return best;
 }
+int helpers_of(const MambaGemm &g, int f) { return g.nsplit == 1 ? helpers_of(tiles_of(g, f), g.K, f) : 0; }
 // fp32 elements of the parts' places
 int64_t parts_of(const MambaGemm &g, int f) {
   const int64_t tiles = tiles_of(g, f);
-  const int helpers = helpers_of(tiles, g.nsplit, g.K, f);
+  const int helpers = helpers_of(g, f);
   if (g.nsplit == 1 && !helpers) return 0;
-  return (f == TILE64 ? tiles * g.nsplit : Share((int)tiles, g.nsplit, helpers, g.K).slots()) * TILE[f] * TILE[f];
+  return (helpers ? Share((int)tiles, helpers, g.K).places() : tiles * g.nsplit) * TILE[f] * TILE[f];
 }
 
 template <int WX, int WY, int FX, int FY, int ST, bool HELP> void launch_wide(const Group &a, int blocks, const Group &r, int rtiles, hipStream_t s) {
@@ -849,7 +842,7 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
     for (int i = 0; i < count; ++i) {
       if (form_in(g, i, count) != f) continue;
       const int64_t tiles = tiles_of(g[i], f);
-      const int helpers = helpers_of(tiles, g[i].nsplit, g[i].K, f);
+      const int helpers = helpers_of(g[i], f);
       if ((helpers > 0) != helped) continue;
       a.g[n] = g[i], a.first[n] = blocks, a.helpers[n] = helpers, a.ws[n] = ws;
       blocks += (int)(tiles * g[i].nsplit) + helpers;

@@ -22,18 +22,30 @@ def test_products(a_k, b_k, shapes, out):
 # them, and 256 x 256; in one call with a product of 64 x 64
 WIDE = [(2176, 2048, 16), (2056, 2184, 72), (72, 136, 72), (136, 200, 160008)]
 WIDE_256 = [(1800, 1544, 3080), (1544, 1800, 3112), (64, 64, 64), (2048, 2048, 2056)]
-WIDE_HELPED = [(2816, 3080, 6008), (64, 64, 64), (3088, 2824, 6008)]     # 143 and 156 tiles: the idle CUs take the ends of the sums
+WIDE_HELPED = [(2816, 3080, 6008), (64, 64, 64), (2568, 2824, 6008)]     # 143 and 132 tiles: the idle CUs take the ends of the sums
+# 256 x 256 uncut, K shorter than a wave's ring and not, ragged: bias alone, neither, bias and what lay there, that alone (check)
+WIDE_WHOLE = [(5128, 8200, 200), (5120, 16392, 104), (5128, 8200, 232), (8200, 16392, 64)]
 WIDE_ODD_K = [(2184, 2056, 33), (136, 200, 160001), (64, 64, 33), (1800, 1544, 3081)]
 WIDE_ODD_ROWS = [(2049, 2183, 72), (65, 129, 500008), (1, 3, 72), (1801, 1543, 3080)]
+# how a product by itself goes: its sum whole, cut into parts, or whole with the idle CUs' help
+FORMS = {tuple(WIDE): ["whole", "whole", None, "cut"], tuple(WIDE_256): ["cut", "cut", None, "cut"], tuple(WIDE_HELPED): ["helped", None, "helped"],
+         tuple(WIDE_WHOLE): ["whole"] * 4}
 
 
-@pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, s) for a in (True, False) for b in (True, False) for s in (WIDE, WIDE_256, WIDE_HELPED)] + [(False, False, WIDE_ODD_K), (False, False, [(2816, 3080, 6001)]), (True, True, WIDE_ODD_ROWS)])
+@pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, s) for a in (True, False) for b in (True, False) for s in (WIDE, WIDE_256, WIDE_HELPED, WIDE_WHOLE)] +
+                         [(False, False, WIDE_ODD_K), (False, False, [(2816, 3080, 6001), (2568, 2824, 6001)]), (True, True, WIDE_ODD_ROWS)])
 @pytest.mark.parametrize("out,pad", [(torch.bfloat16, 8), (torch.bfloat16, 3), (torch.float32, 3)])
 def test_larger_tiles(a_k, b_k, shapes, out, pad):
-    check(a_k, b_k, shapes, out, pad)
+    check(a_k, b_k, shapes, out, pad, FORMS.get(tuple(shapes)))
 
 
-def check(a_k, b_k, shapes, out, pad):
+def form(lib, product):
+    group = (type(product) * 1)(product)
+    floats = lib.mamba_gemm_plan(group, 1)
+    return "cut" if group[0].nsplit > 1 else "helped" if floats else "whole"
+
+
+def check(a_k, b_k, shapes, out, pad, forms=None):
     from mamba_amd import _lib
     lib = _lib.load()
     gen = torch.Generator(device="cuda").manual_seed(5)
@@ -52,11 +64,14 @@ def check(a_k, b_k, shapes, out, pad):
             A, B, bias = operand(M, K, a_k), operand(N, K, b_k), torch.randn(N, device="cuda", generator=gen).bfloat16()
             D = torch.full((M, N + pad), 0.5, device="cuda", dtype=out)
             with_bias, accumulate = j % 2 == 0, j >= 2
-            want = A.double() @ B.double().t() + (bias.double() if with_bias else 0) + (0.5 if accumulate else 0)
-            size = A.double().abs() @ B.double().abs().t() + 1
+            D[:, :N] = torch.randn(M, N, device="cuda", generator=gen)
+            want = A.double() @ B.double().t() + (bias.double() if with_bias else 0) + (D[:, :N].double() if accumulate else 0)
+            size = A.double().abs() @ B.double().abs().t() + 1 + D[:, :N].double().abs()
             group[j] = _lib.MambaGemm(A.data_ptr(), B.data_ptr(), bias.data_ptr() if with_bias else None, D.data_ptr(), *A.stride(), *B.stride(),
                                       N + pad, M, N, K, _lib.DTYPE_CODE[out], int(accumulate), 0)
             keep.append((A, B, bias, D, want, size, K))
+        for j, want_form in enumerate(forms or []):
+            assert want_form in (None, form(lib, group[j])), shapes[j]
         floats = lib.mamba_gemm_plan(group, count)
         assert floats >= 0
         ws = torch.full((max(floats, 1),), float("nan"), device="cuda")

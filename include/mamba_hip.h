@@ -696,11 +696,14 @@ typedef struct MambaGemm {
   int32_t M, N, K;
   int32_t d_dtype;    /* MAMBA_BF16 or MAMBA_F32 */
   int32_t accumulate;
-  int32_t nsplit;     /* parts of the sum over k, set by mamba_gemm_plan */
+  int32_t nsplit;     /* parts of the sum over k, or MAMBA_GEMM_SHARED: set by mamba_gemm_plan */
 } MambaGemm;
+/* nsplit of whole sums whose ends are taken by the compute units that the product would leave idle */
+#define MAMBA_GEMM_SHARED (-1)
 /* 1 where these kernels are the ones to use, 0 where a BLAS library is faster (sizes, layout and alignment decide). */
 int mamba_gemm_suits(const MambaGemm *g);
-/* Sets nsplit of each product and returns the fp32 elements of workspace the call needs (0: none), or an error. */
+/* Sets nsplit of each product and returns the fp32 elements of workspace the call needs (0: none), or an error.  The plan is for
+ * these products in this order on the current device.  Whole sums in one piece (nsplit 1) need no workspace and no plan. */
 int64_t mamba_gemm_plan(MambaGemm *g, int count);
 int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream_t stream);
 

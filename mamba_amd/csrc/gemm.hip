@@ -711,7 +711,7 @@ __global__ __launch_bounds__(256) void cast_bf16_kernel(const CastJobs a) {
 
 bool valid(const MambaGemm &g) {
   return g.A && g.B && g.D && g.M > 0 && g.N > 0 && g.K > 0 && (g.a_ks == 1 || g.a_ms == 1) && (g.b_ks == 1 || g.b_ns == 1) &&
-         (g.d_dtype == MAMBA_BF16 || g.d_dtype == MAMBA_F32) && g.nsplit >= 1 &&
+         (g.d_dtype == MAMBA_BF16 || g.d_dtype == MAMBA_F32) && (g.nsplit >= 1 || g.nsplit == MAMBA_GEMM_SHARED) &&
          (int64_t)((g.M + GB - 1) / GB) * ((g.N + GB - 1) / GB) <= INT32_MAX / 1024;
 }
 
@@ -754,14 +754,17 @@ double us_of(int64_t tiles, int splits, int helpers, int K, int f) {
   const int64_t parts = (splits > 1 || helpers ? units : 0) + (helpers ? units + helpers : 0);
   return (helpers ? Share((int)tiles, helpers, K).own : (stages + splits - 1) / splits) * stage + (parts ? 6 + parts * TILE[f] * TILE[f] * 2e-6 : 0);
 }
-// CUs that 256 x 256 tiles with whole sums leave idle and that are worth their parts.  (With the sums cut as well they never are, by
-// these estimates at 48 to 255 tiles.)
-int helpers_of(int64_t tiles, int K, int f) {
+// CUs that 256 x 256 tiles with whole sums leave idle; 0 where there is nothing that they could take
+int idle_of(int64_t tiles, int K, int f) {
   const int64_t idle = cu_count() - tiles;
   if (f != TILE256 || idle <= 0) return 0;
   const Share share((int)tiles, (int)idle, K);
-  if (!share.rest || tiles * share.rest >= 1 << 30) return 0;
-  return us_of(tiles, 1, (int)idle, K, f) < 0.97 * us_of(tiles, 1, 0, K, f) ? (int)idle : 0;
+  return share.rest && tiles * share.rest < 1 << 30 ? (int)idle : 0;
+}
+// ... and that are worth their parts.  (With the sums cut as well they never are, by these estimates at 48 to 255 tiles.)
+int helpers_of(int64_t tiles, int K, int f) {
+  const int idle = idle_of(tiles, K, f);
+  return idle && us_of(tiles, 1, idle, K, f) < 0.97 * us_of(tiles, 1, 0, K, f) ? idle : 0;
 }
 int splits_of(const MambaGemm &g, int f) {
   const int64_t tiles = tiles_of(g, f), steps = (g.K + GK - 1) / GK, cus = cu_count();
@@ -775,12 +778,12 @@ int splits_of(const MambaGemm &g, int f) {
   }
   return best;
 }
-int helpers_of(const MambaGemm &g, int f) { return g.nsplit == 1 ? helpers_of(tiles_of(g, f), g.K, f) : 0; }
+int planned_helpers(const MambaGemm &g, int f) { return g.nsplit == MAMBA_GEMM_SHARED ? idle_of(tiles_of(g, f), g.K, f) : 0; }
 // fp32 elements of the parts' places
 int64_t parts_of(const MambaGemm &g, int f) {
   const int64_t tiles = tiles_of(g, f);
-  const int helpers = helpers_of(g, f);
-  if (g.nsplit == 1 && !helpers) return 0;
+  const int helpers = planned_helpers(g, f);
+  if (g.nsplit == 1) return 0;
   return (helpers ? Share((int)tiles, helpers, g.K).places() : tiles * g.nsplit) * TILE[f] * TILE[f];
 }
 
@@ -819,6 +822,8 @@ extern "C" int64_t mamba_gemm_plan(MambaGemm *g, int count) {
     if (want > 1) {
       const int64_t per = (steps + want - 1) / want;
       g[i].nsplit = (int32_t)((steps + per - 1) / per);
+    } else if (helpers_of(tiles_of(g[i], f), g[i].K, f)) {
+      g[i].nsplit = MAMBA_GEMM_SHARED;
     }
     floats += parts_of(g[i], f);
   }
@@ -829,7 +834,8 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
   if (!g || count < 1 || count > MAXG) return MAMBA_E_BADARG;
   hipStream_t s = static_cast<hipStream_t>(stream);
   for (int i = 0; i < count; ++i) {
-    if (!valid(g[i]) || (parts_of(g[i], form_in(g, i, count)) && !ws)) return MAMBA_E_BADARG;
+    if (!valid(g[i]) || (g[i].nsplit != 1 && !ws)) return MAMBA_E_BADARG;
+    if (g[i].nsplit == MAMBA_GEMM_SHARED && !planned_helpers(g[i], form_in(g, i, count))) return MAMBA_E_BADARG;
   }
   // the products of one form in a launch, those with helpers (every workgroup leaves parts) apart from the others
   for (int form = FORMS; form >= 0; --form) {
@@ -842,13 +848,15 @@ extern "C" int mamba_gemm(const MambaGemm *g, int count, float *ws, mamba_stream
     for (int i = 0; i < count; ++i) {
       if (form_in(g, i, count) != f) continue;
       const int64_t tiles = tiles_of(g[i], f);
-      const int helpers = helpers_of(g[i], f);
+      const int helpers = planned_helpers(g[i], f);
       if ((helpers > 0) != helped) continue;
-      a.g[n] = g[i], a.first[n] = blocks, a.helpers[n] = helpers, a.ws[n] = ws;
-      blocks += (int)(tiles * g[i].nsplit) + helpers;
+      MambaGemm p = g[i];
+      p.nsplit = std::max(1, p.nsplit);
+      a.g[n] = p, a.first[n] = blocks, a.helpers[n] = helpers, a.ws[n] = ws;
+      blocks += (int)(tiles * p.nsplit) + helpers;
       all = all && ring(g[i]);
       if (const int64_t parts = parts_of(g[i], f)) {
-        r.g[nr] = g[i], r.first[nr] = rtiles * per_tile, r.helpers[nr] = helpers, r.ws[nr] = ws;
+        r.g[nr] = p, r.first[nr] = rtiles * per_tile, r.helpers[nr] = helpers, r.ws[nr] = ws;
         rtiles += (int)tiles;
         ws += parts;
         ++nr;

@@ -39,13 +39,20 @@ def test_larger_tiles(a_k, b_k, shapes, out, pad):
     check(a_k, b_k, shapes, out, pad, FORMS.get(tuple(shapes)))
 
 
+# what a plan would give helpers, or cut, runs whole without a plan and without a workspace
+@pytest.mark.parametrize("shapes", [[WIDE_HELPED[0], WIDE[3], WIDE_256[0]], [(768, 1536, 2000), (64, 64, 64)]])
+def test_whole_sums_need_no_workspace(shapes):
+    check(False, False, shapes, torch.bfloat16, 8, planned=False)
+
+
 def form(lib, product):
     group = (type(product) * 1)(product)
-    floats = lib.mamba_gemm_plan(group, 1)
-    return "cut" if group[0].nsplit > 1 else "helped" if floats else "whole"
+    floats, parts = lib.mamba_gemm_plan(group, 1), group[0].nsplit
+    assert floats >= 0 and (floats == 0) == (parts == 1)
+    return "cut" if parts > 1 else "helped" if parts < 0 else "whole"
 
 
-def check(a_k, b_k, shapes, out, pad, forms=None):
+def check(a_k, b_k, shapes, out, pad, forms=None, planned=True):
     from mamba_amd import _lib
     lib = _lib.load()
     gen = torch.Generator(device="cuda").manual_seed(5)
@@ -75,7 +82,10 @@ def check(a_k, b_k, shapes, out, pad, forms=None):
         floats = lib.mamba_gemm_plan(group, count)
         assert floats >= 0
         ws = torch.full((max(floats, 1),), float("nan"), device="cuda")
-        _lib.check(lib.mamba_gemm(group, count, ws.data_ptr(), _lib.current_stream(ws.device)), "mamba_gemm")
+        if not planned:
+            for product in group:
+                product.nsplit = 1
+        _lib.check(lib.mamba_gemm(group, count, ws.data_ptr() if planned else None, _lib.current_stream(ws.device)), "mamba_gemm")
         for A, B, bias, D, want, size, K in keep:
             N = want.shape[1]
             # fp32 sums of K terms, and one rounding to the result's type

@@ -747,10 +747,15 @@ int form_in(const MambaGemm *g, int i, int count) {
 }
 // Parts of the sum over k.  64 x 64: as many as give every CU two workgroups, of at least 8 steps (256 elements) each.  The others: the
 // least of a stage's time by the workgroups on a CU, measured at 18 to 800 tiles in up to 32 parts, and what the parts' writing,
-// reading and second launch take.
+// reading and second launch take.  Helpers walk k apart from the tiles' own workgroups and from each other, which costs all of
+// them a share of the L2: nothing at 56 helpers for 200 tiles, a fifth of a stage where they are as many as the tiles.  us, helped |
+// two parts | three, cold operands: 1408 x 2816 x 16384 (66 tiles) 178 | 220 | 165; 1536 x 3072 x 16384 (72) 201 | 225 | 170, x 32768
+// 363 | 427 | 322; 1664 x 3328 x 12288 (91) 161 | 177; 1792 x 3584 x 16384 (98) 253 | 232; 1920 x 3840 x 32768 (120) 535 | 486; 2304 x 4608
+// x 32768 (162) 638, whole 823.  Cutting has to promise 1.5 % more than help.
 double us_of(int64_t tiles, int splits, int helpers, int K, int f) {
   const int64_t units = tiles * splits, cus = cu_count(), stages = (K + WK - 1) / WK;
-  const double stage = f == TILE256 ? 0.82 : units <= cus ? 0.37 : units <= 2 * cus ? 0.41 : 0.62;
+  const double crowd = std::min(1.0, (double)helpers / (double)tiles);
+  const double stage = f == TILE256 ? 0.82 * (1 + 0.22 * crowd * crowd) : units <= cus ? 0.37 : units <= 2 * cus ? 0.41 : 0.62;
   const int64_t parts = (splits > 1 || helpers ? units : 0) + (helpers ? units + helpers : 0);
   return (helpers ? Share((int)tiles, helpers, K).own : (stages + splits - 1) / splits) * stage + (parts ? 6 + parts * TILE[f] * TILE[f] * 2e-6 : 0);
 }
@@ -772,9 +777,10 @@ int splits_of(const MambaGemm &g, int f) {
   int best = 1;
   double least = 1e30;
   const int64_t most = std::min<int64_t>((f == TILE256 ? 1 : 3) * cus / tiles, steps / 8);
+  const int helped = helpers_of(tiles, g.K, f);
   for (int s = 1; s == 1 || s <= most; ++s) {
-    const double us = us_of(tiles, s, s == 1 ? helpers_of(tiles, g.K, f) : 0, g.K, f);
-    if (us < least) least = us, best = s;
+    const double us = us_of(tiles, s, s == 1 ? helped : 0, g.K, f);
+    if (us < (best == 1 && helped ? 0.985 : 1.0) * least) least = us, best = s;
   }
   return best;
 }

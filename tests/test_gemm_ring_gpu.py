@@ -22,7 +22,7 @@ def test_products(a_k, b_k, shapes, out):
 # them, and 256 x 256; in one call with a product of 64 x 64
 WIDE = [(2176, 2048, 16), (2056, 2184, 72), (72, 136, 72), (136, 200, 160008)]
 WIDE_256 = [(1800, 1544, 3080), (1544, 1800, 3112), (64, 64, 64), (2048, 2048, 2056)]
-WIDE_HELPED = [(2816, 3080, 6008), (64, 64, 64), (2568, 2824, 6008)]     # 143 and 132 tiles: the idle CUs take the ends of the sums
+WIDE_HELPED = [(2816, 3080, 9016), (64, 64, 64), (2568, 2824, 9016)]     # 143 and 132 tiles: the idle CUs take the ends of the sums
 # 256 x 256 uncut, K shorter than a wave's ring and not, ragged: bias alone, neither, bias and what lay there, that alone (check)
 WIDE_WHOLE = [(5128, 8200, 200), (5120, 16392, 104), (5128, 8200, 232), (8200, 16392, 64)]
 WIDE_ODD_K = [(2184, 2056, 33), (136, 200, 160001), (64, 64, 33), (1800, 1544, 3081)]
@@ -33,7 +33,7 @@ FORMS = {tuple(WIDE): ["whole", "whole", None, "cut"], tuple(WIDE_256): ["cut", 
 
 
 @pytest.mark.parametrize("a_k,b_k,shapes", [(a, b, s) for a in (True, False) for b in (True, False) for s in (WIDE, WIDE_256, WIDE_HELPED, WIDE_WHOLE)] +
-                         [(False, False, WIDE_ODD_K), (False, False, [(2816, 3080, 6001), (2568, 2824, 6001)]), (True, True, WIDE_ODD_ROWS)])
+                         [(False, False, WIDE_ODD_K), (False, False, [(2816, 3080, 9009), (2568, 2824, 9009)]), (True, True, WIDE_ODD_ROWS)])
 @pytest.mark.parametrize("out,pad", [(torch.bfloat16, 8), (torch.bfloat16, 3), (torch.float32, 3)])
 def test_larger_tiles(a_k, b_k, shapes, out, pad):
     check(a_k, b_k, shapes, out, pad, FORMS.get(tuple(shapes)))

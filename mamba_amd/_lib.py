@@ -205,6 +205,8 @@ def load():
         fn = getattr(lib, name)
         fn.argtypes = [ctypes.POINTER(NormGatedParams), c_vp]
         fn.restype = ctypes.c_int
+    lib.mamba_gemm_suits.argtypes = [ctypes.POINTER(MambaGemm)]
+    lib.mamba_gemm_suits.restype = ctypes.c_int
     lib.mamba_gemm_plan.argtypes = [ctypes.POINTER(MambaGemm), ctypes.c_int]
     lib.mamba_gemm_plan.restype = ctypes.c_int64
     lib.mamba_gemm.argtypes = [ctypes.POINTER(MambaGemm), ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]

@@ -801,20 +801,27 @@ template <int WX, int WY, int FX, int FY, int ST, bool HELP> void launch_wide(co
 }  // namespace
 
 // Where the library takes over.  Up to 8 GFLOP its host time and choice of tiles cost more than any of these forms (whole mixer
-// calls, forward + backward, library / own: products up to 0.5 GFLOP 350 / 180 us, up to 5 GFLOP 432 / 398).  Up to 16 GFLOP, by 270
-// products of 20 - 30 us (the library up to 75): where both operands lie along k it takes 0.78 - 0.9 of the larger tiles' time; where
-// k is below the larger side the two are within 10 % by themselves and a whole call is no faster with own products (1 x 1536 x
-// 2560: 277 / 286); k up to twice that, a projection to half the width, 27 / 33; sums over a longer k, weight gradients, take 0.4 -
-// 0.8 of its time (calls of 4 x 1000 x 1792 409 / 394, 8 x 1000 x 1280 519 / 500).  Beyond: sums over a long k into few tiles, which it
-// does not split, and short k with a result that the last-level cache holds (5120 x 16384 x 160: 47 / 57; twice as long 139 / 114).
+// calls, forward + backward, library / own: products up to 0.5 GFLOP 350 / 180 us, up to 5 GFLOP 432 / 398).  Beyond:
+// - sums over a long k into few tiles, which the library does not split, at three times the larger side and more: 1024 x 2048 x 16384 107 -
+//   144 / 90 - 97, 2304 x 4608 x 16384 463 - 482 / 328 - 337, 2560 x 5120 x 32768 970 / 755; not always (2432 x 4864 x 16384 326 - 352 / 389 - 402).  Up to
+//   16 GFLOP (270 products of 20 - 30 us) at twice the larger side: weight gradients take 0.4 - 0.8 of its time (calls of 4 x 1000 x
+//   1792 409 / 394, 8 x 1000 x 1280 519 / 500), a projection to half the width 27 / 33, and where k is below the larger side the
+//   two are within 10 % by themselves and a whole call is no faster with own products (1 x 1536 x 2560: 277 / 286).
+// - where both operands lie along k the library is the better one at that: 1024 x 1024 x 4096 18 / 26, 1280 x 1280 x 4096 23 / 29, 2048 x 2048 x
+//   6200 66 / 81, 3072 x 1536 x 16384 160 / 235.  It splits badly there from k 20000 or 48 times the shorter side on: 1024 x 4096 x
+//   24576 280 / 210, 2048 x 2048 x 32768 377 / 319; 128 x 4096 x 12288 68 / 44, 126 x 3008 x 23808 117 / 51.
+// - short k with a result that the last-level cache holds (5120 x 16384 x 160, over and over: 57 / 47; twice as long 114 / 139).
 extern "C" int mamba_gemm_suits(const MambaGemm *g) {
   if (!g) return 0;
   const double flop = 2.0 * g->M * g->N * g->K;
   if (flop <= 8e9) return 1;
   if (!ring(*g)) return 0;
-  if (flop <= 16e9 && (g->a_ks != 1 || g->b_ks != 1) && g->K > 2 * (int64_t)std::max(g->M, g->N)) return 1;
-  return (g->K >= 3 * (int64_t)std::max(g->M, g->N) && tiles_of(*g, TILE256) < cu_count()) ||
-         (g->K <= 256 && (int64_t)g->M * g->N <= 100000000);
+  const int64_t K = g->K, longer = std::max(g->M, g->N), shorter = std::min(g->M, g->N);
+  if (g->a_ks != 1 || g->b_ks != 1 || K >= 20000 || K >= 48 * shorter) {
+    if (flop <= 16e9 && K > 2 * longer) return 1;
+    if (K >= 3 * longer && tiles_of(*g, TILE256) < cu_count()) return 1;
+  }
+  return K <= 256 && (int64_t)g->M * g->N <= 100000000;
 }
 
 extern "C" int64_t mamba_gemm_plan(MambaGemm *g, int count) {

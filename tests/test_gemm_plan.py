@@ -1,4 +1,5 @@
-"""How the grouped bf16 products are planned (256 compute units, without a GPU too): the parts of the sum over k."""
+"""How the grouped bf16 products are planned (256 compute units, without a GPU too): the parts of the sum over k, and where a BLAS
+library is the faster one."""
 import pytest
 
 
@@ -39,3 +40,22 @@ def test_parts_of_larger_tiles(M, N, K, want, b_k):
     tiles = -(-M // 256) * -(-N // 256)
     assert group[0].nsplit == want
     assert floats == 65536 * (tiles * want if want > 0 else tiles + 255)   # (a place per tile; the helpers' pieces lie at tile + helper)
+
+
+# (which operands lie along k, sizes, whether the own kernels suit): both sides of each line
+@pytest.mark.parametrize("a_k,b_k,M,N,K,want", [
+    (True, True, 2000, 2000, 1000, 1), (True, True, 2000, 2000, 1008, 0),          # 8 GFLOP
+    (False, True, 952, 2048, 4104, 1), (False, True, 952, 2048, 4096, 0),        # to 16 GFLOP: k over twice the larger side
+    (False, True, 1024, 2048, 6144, 1), (False, True, 1024, 2048, 6136, 0),        # beyond: three times
+    (False, False, 1024, 2048, 6144, 1), (False, False, 1024, 2048, 6136, 0),
+    (False, False, 4080, 4088, 12264, 0), (False, False, 3840, 4088, 12264, 1),    # ... and fewer tiles of 256 x 256 than compute units
+    (True, True, 1024, 1024, 4096, 0), (True, True, 2048, 2048, 6200, 0),          # both along k
+    (True, True, 1024, 4096, 19992, 0), (True, True, 1024, 4096, 20000, 1),        # ... k from 20000 on
+    (True, True, 128, 2048, 16384, 1), (True, True, 256, 2048, 12280, 0), (True, True, 256, 2048, 12288, 1),   # ... 48 times the shorter side
+    (True, True, 160, 5120, 15360, 1), (True, True, 192, 5120, 15360, 1),          # (gradients of a 5120-channel mixer's projections)
+    (True, False, 5120, 8192, 160, 1), (False, False, 5120, 8192, 192, 1), (True, False, 5120, 4096, 256, 1), (True, False, 5120, 4096, 264, 0),   # short k
+    (False, False, 2047, 2048, 6144, 0),                                           # rows that lie on no 16 bytes
+])
+def test_where_the_own_kernels_suit(a_k, b_k, M, N, K, want):
+    from mamba_amd import _lib
+    assert _lib.load().mamba_gemm_suits(product(M, N, K, a_k, b_k)) == want

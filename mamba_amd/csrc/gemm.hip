@@ -810,7 +810,9 @@ template <int WX, int WY, int FX, int FY, int ST, bool HELP> void launch_wide(co
 // - where both operands lie along k the library is the better one at that: 1024 x 1024 x 4096 18 / 26, 1280 x 1280 x 4096 23 / 29, 2048 x 2048 x
 //   6200 66 / 81, 3072 x 1536 x 16384 160 / 235.  It splits badly there from k 20000 or 48 times the shorter side on: 1024 x 4096 x
 //   24576 280 / 210, 2048 x 2048 x 32768 377 / 319; 128 x 4096 x 12288 68 / 44, 126 x 3008 x 23808 117 / 51.
-// - short k with a result that the last-level cache holds (5120 x 16384 x 160, over and over: 57 / 47; twice as long 114 / 139).
+// - short k with up to 80 million results.  By whole mixer calls, forward + backward: 2304 channels x 32768 positions (75 million) 2950 /
+//   2865, 4864 x 16384 3734 / 3582, 3584 x 12288 1976 / 1926, 2560 x 28672 2844 / 2812, though 4096 x 16384 2559 / 2578; with more of them 5120 x
+//   16384 (84 million) 3620 / 3651, 3072 x 28672 3347 / 3376, 4480 x 20480 3903 / 3922, 2560 x 32768 3190 / 3186.
 extern "C" int mamba_gemm_suits(const MambaGemm *g) {
   if (!g) return 0;
   const double flop = 2.0 * g->M * g->N * g->K;
@@ -821,7 +823,7 @@ extern "C" int mamba_gemm_suits(const MambaGemm *g) {
     if (flop <= 16e9 && K > 2 * longer) return 1;
     if (K >= 3 * longer && tiles_of(*g, TILE256) < cu_count()) return 1;
   }
-  return K <= 256 && (int64_t)g->M * g->N <= 100000000;
+  return K <= 256 && (int64_t)g->M * g->N <= 80000000;
 }
 
 extern "C" int64_t mamba_gemm_plan(MambaGemm *g, int count) {

@@ -54,6 +54,7 @@ def test_parts_of_larger_tiles(M, N, K, want, b_k):
     (True, True, 128, 2048, 16384, 1), (True, True, 256, 2048, 12280, 0), (True, True, 256, 2048, 12288, 1),   # ... 48 times the shorter side
     (True, True, 160, 5120, 15360, 1), (True, True, 192, 5120, 15360, 1),          # (gradients of a 5120-channel mixer's projections)
     (True, False, 5120, 8192, 160, 1), (False, False, 5120, 8192, 192, 1), (True, False, 5120, 4096, 256, 1), (True, False, 5120, 4096, 264, 0),   # short k
+    (True, False, 4864, 16384, 152, 1), (True, False, 5120, 16384, 160, 0), (False, False, 3072, 28672, 128, 0),   # ... up to 80 million results
     (False, False, 2047, 2048, 6144, 0),                                           # rows that lie on no 16 bytes
 ])
 def test_where_the_own_kernels_suit(a_k, b_k, M, N, K, want):

@@ -393,7 +393,6 @@ template <int W, typename CT, bool TABLE> __global__ __launch_bounds__(256) void
 // issued behind the rows that it is for.  Rows through registers, the weighted ones written to LDS (before) / this, 80 heads
 // x 4096 positions: batch 2 59 / 47 us, batch 3 64 / 48, batch 4 91 / 71, batch 8 169 / 152; 128 heads in 8 groups x 2 x 32768
 // 451 / 423.
-constexpr int CSP_MAX_CHUNKS = 2048;
 template <int HH, int NS, bool HAS_SEQ> __global__ __launch_bounds__(256 * HH, 2) void chunk_state_passing_fwd_kernel(const SsdParams p) {
   constexpr int NW = 4 * HH, KS = 64, Q = KS * NS, P = 64, N = 128, XH = KS * P * 2, XB = HH * XH, SB = XB + KS * N * 2, RING = HH == 1 ? 3 : 4, AHEAD = RING - 1;
   constexpr int LOADS = SB / 1024 / NW, STORES = 4, TABLE = HAS_SEQ ? 5 : 3;  // of a wave: per stage; per chunk
@@ -799,7 +798,7 @@ static int ssd_chunk_scan_fwd_one(const SsdParams *p, mamba_stream_t stream) {
 static bool chunk_state_passing_shapes_ok(const SsdParams *p) {
   auto al16 = [](const void *q) { return q && (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
   return p->dtype == MAMBA_BF16 && p->headdim == 64 && p->dstate == WB && (p->chunk_size == 256 || p->chunk_size == 128) &&
-         p->seqlen % p->chunk_size == 0 && p->nchunks <= CSP_MAX_CHUNKS && p->nheads <= 65535 && p->batch <= 65535 &&
+         p->seqlen % p->chunk_size == 0 && (int64_t)p->nheads * p->batch <= INT32_MAX / 256 &&
          al16(p->states_lp) && al16(p->final_states) && p->dt_out && p->dA_cumsum &&
          wide_operand_ok(p->x, p->dtype, p->x_bs, p->x_ls, p->x_hs) && wide_operand_ok(p->B, p->dtype, p->B_bs, p->B_ls, p->B_gs);
 }
@@ -807,7 +806,7 @@ static bool chunk_state_passing_shapes_ok(const SsdParams *p) {
 // chip busy: a workgroup takes ~3 us per chunk of 256 whatever their number, the two-kernel path ~24 ns per (batch, head, chunk).
 // Walk / two kernels: 128 pairs x 4096 positions 46.8 / 47.9 us, x 2048 in chunks of 128 33.2 / 36.2, x 16384 in 8 groups
 // 198 / 199; 160 pairs x 4096 47 / 52, x 512 in chunks of 128 12.6 / 21; 176 pairs in 8 groups 48 / 67; 240 pairs 48 / 95; 320
-// 71 / 128; one packed row of 64 heads x 32768 positions 436 / 195 (before).
+// 71 / 128; 192 pairs x 262144 in chunks of 128 3960 / 8073; one packed row of 64 heads x 32768 positions 388 / 202.
 // With fewer than three pairs to four CUs, only where the two kernels need a launch for the steps' sums as well (sums_in_states,
 // below): the whole forward pass of 128 pairs x 2048 positions 70.2 / 69.8, x 512 in chunks of 128 27.2 / 27.9 with the walk.
 static bool sums_in_states(const SsdParams *p) { return (int64_t)p->nchunks * p->batch * p->nheads <= 8 * (int64_t)cu_count(); }

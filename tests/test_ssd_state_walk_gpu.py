@@ -38,6 +38,7 @@ def _entering_states(t, chunk, stages):
     (1, 1536, 8, 8, 256, [100, 156, 256, 300, 212, 1, 511], True),   # boundaries inside chunks and on chunk edges
     (2, 768, 4, 1, 128, [128, 128, 300, 212], False),
     (1, 256, 3, 1, 256, None, True),                                    # a single chunk
+    (1, 262272, 2, 1, 128, None, True),                                 # 2049 of them: there is no table of the chunks to outgrow
 ])
 def test_one_launch_matches_the_two_stages(batch, seqlen, nheads, ngroups, chunk, seq_lens, has_init):
     t = ssd_inputs(batch, seqlen, nheads, 64, 128, ngroups, torch.bfloat16, 17, seq_lens=seq_lens, has_init=has_init)

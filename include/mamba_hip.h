@@ -682,8 +682,8 @@ int norm_residual_bwd(const NormResidualParams *p, mamba_stream_t stream);
 int norm_residual_bwd_nparts(const NormResidualParams *p);
 
 /* -------------------------------------------------------------------------
- * Small bf16 matrix products (the projections of a short mixer call, selective_scan_interface.py:230-383 and
- * ssd_combined.py:868):
+ * bf16 matrix products (the projections inside a mixer, selective_scan_interface.py:230-383 and ssd_combined.py:868, where they
+ * are short or a BLAS library splits them badly: mamba_gemm_suits):
  *   D[m][n] = sum_k A[m][k] B[n][k]   (+ bias[n])   (+ D[m][n] before, with accumulate)
  * with fp32 sums, rounded once into D.  Either index of A and of B is contiguous (stride 1), any alignment; D's
  * columns are contiguous.  Up to 4 independent products share a call.

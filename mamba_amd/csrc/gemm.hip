@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256) void gemm_ring_kernel(const Group a) {
 
 // ---- larger tiles for larger products: WX x WY waves of 16 FX x 16 FY each, operands in blocks of 64 rows, stages of WK k in a
 // ring of LDS stages filled by asynchronous loads, one barrier a stage; a stage's fragments are read while the products of the one
-// before it run.  What bounds them: up to 128 x 128 the reading through the L2 (2560 x 5120 x 32768: 13 GB, 13.6 TB/s), at 256 x 256
+// before it run.  What bounds them: up to 128 x 128 the reading through the L2 (2560 x 5120 x 32768: 13.4 GB, 11 TB/s), at 256 x 256
 // the LDS (reading 96 KB and writing 32 KB per CU and stage is as long as its products), 1.0 - 1.2 PFLOP/s.
 //   M x N x K                 us: library | 64 x 64 | 128 x 128 | 256 x 256 (with the splits that are chosen)
 //   2560 x 5120 x 32768           965   |   -   | 1198 | 754        (200 tiles on 256 CUs: 832 without Share's helpers)

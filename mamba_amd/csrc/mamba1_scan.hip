@@ -948,12 +948,11 @@ size_t fwd_min_lds() {
 // The forward kernel that serves a problem and its estimated time in us, for 16 states.  scan_fwd_serial_kernel
 // (mamba1_scan_serial.hip) takes 16 states and per-position B and C.  With two states per lane up to five of its workgroups
 // share a CU, and a tile (half tiles where the sequence ends in one) takes a round of them 7.3, 10.7, 14.1, 17.5, 20.9; with
-// one, a workgroup has half as many channels and a tile takes 4.8, 6.5, 9.1, 11.6: 1 x 1536 x 256 15.5 -> 12.7 us, 8 x 1024 x
-// 2048 115 -> 108, 1 x 768 x 4096 in segments 42 -> 39; from five of them on two states per lane stay (4 x 5120 x 512: 62
-// against 63).  scan_fwd_kernel: up to two per CU, 6.6 or 10.9, and a seventh more of that on rows with a ragged end.  Measured, 8 x 5120 channels x 4096
-// positions bf16: 806 -> 660 us; 8 x 2368 x 8086: 1235 -> 971; 7 x 3184 x 192: 35 -> 24; a workgroup per CU or less and the
-// sequence whole: 108 against 119 (2 x 4096 x 2048), the kernel with the lanes along the sequence stays; cut into more
-// segments (below) the other one serves those too.
+// one, a workgroup has half as many channels and a tile takes 4.8, 6.5, 9.1, 11.6: 1 x 1536 x 256 15.1 -> 12.4 us, 8 x 1024 x
+// 2048 117 -> 104, 2 x 4096 x 2048 117 -> 104, 1 x 768 x 4096 in segments 43 -> 36; from five of them on two states per lane stay
+// (4 x 5120 x 512: 59 both ways).  scan_fwd_kernel: up to two per CU, 6.6 or 10.9, and a seventh more of that on rows with a
+// ragged end.  Measured, 8 x 5120 channels x 4096 positions bf16: 806 -> 660 us; 8 x 2368 x 8086: 1235 -> 971; 7 x 3184 x 192: 35 -> 24;
+// by these estimates it still takes ragged rows of a single tile on up to a workgroup per CU (2 x 3072 x 87).
 bool serial_takes(const MambaScanParams &p) {
   return p.dstate == NB16 && !(p.bc_const & 3) && !p.a_complex && !k4_mode() && !fwd_min_lds() && p.seqlen >= KI;
 }

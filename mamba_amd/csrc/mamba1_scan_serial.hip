@@ -20,7 +20,7 @@
 //
 // With few channels the walk itself is what a call waits for, and a wave alone on its SIMD issues an instruction in four
 // clocks.  Then a lane takes one state (SPL 1: 16 lanes and 4 channels of a wave, 16 channels of a workgroup, 128 positions at
-// a time): twice the waves at nearly half the instructions each, 4.8 us per 128 positions instead of 7.3, 6.7 with two of the
+// a time): twice the waves at nearly half the instructions each, 4.8 us per 128 positions instead of 7.3, 6.5 with two of the
 // half as large workgroups on a CU.  More of them per CU issue more in all than two states per lane do (fwd_cost).
 #include "mamba1_scan.hpp"
 
@@ -39,7 +39,7 @@ DEVI int bc_at(int t) { return t * BCP + (t >> 3) * BCP; }  // (a spare row afte
 
 // States n .. n + NS - 1 entering this workgroup's segment, as seg_state_in has them one by one.  What eight segments left is
 // requested together, and nothing that was loaded before (A) is waited for ahead of it: a segment after the other is a memory
-// latency for each (1 x 1536 channels x 777 positions in seven segments: 24.4 -> 22.3 us).
+// latency for each (1 x 1536 channels x 777 positions in seven segments, one state per lane as well: 24.3 -> 22.8 us).
 constexpr int SEG_BATCH = 8;
 template <int NS> DEVI void seg_states_in(const MambaScanParams &p, const Geo &q, int d, int n, const float (&A)[NS], float (&h)[NS]) {
 #pragma unroll
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(64 * SWAVES, AHEAD ? 4 : 5) void scan_fwd_serial_ke
 template <typename T, int MODE, int SPL> void launch_s(const MambaScanParams &p, hipStream_t s) {
   constexpr int WCH = Serial<SPL>::channels * SWAVES;
   const dim3 grid(p.ngroups * ((p.dim / p.ngroups + WCH - 1) / WCH), p.batch, p.nseg > 1 ? p.nseg : 1), block(64 * SWAVES);
-  // one state per lane is for calls that leave a SIMD few waves; with two, up to two workgroups per CU (39.2 -> 37.5 us at 4 x 1024 x
+  // one state per lane is for calls that leave a SIMD few waves; with two, up to two workgroups per CU (39.3 -> 38.2 us at 4 x 1024 x
   // 1024 in four segments; five per CU 660 -> 682 at 8 x 5120 x 4096)
   if (SPL == 1 || (int64_t)grid.x * grid.y * grid.z <= 2 * cu_count()) hipLaunchKernelGGL((scan_fwd_serial_kernel<T, MODE, SPL, true>), grid, block, 0, s, p);
   else hipLaunchKernelGGL((scan_fwd_serial_kernel<T, MODE, SPL, SPL == 1>), grid, block, 0, s, p);

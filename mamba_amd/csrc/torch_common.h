@@ -110,8 +110,10 @@ struct Mat {  // one operand: element (row, k) at p[row * rs + k * ks], one of t
   const void *p;
   int64_t rs, ks;
 };
-// Products D = A B^T of operands of `type` on raw memory.  Short ones are collected and leave together with run(); the
-// ones collected between two run() calls must not depend on each other, long ones run at once.
+// Products D = A B^T of operands of `type` on raw memory.  Those that the own kernels suit (mamba_gemm_suits: short ones, and large
+// ones that the BLAS library splits badly) are collected and leave with run(), or once there are four, in an order of their own; the
+// others leave at once.  So the products of two run() calls must not depend on each other, no result is there before run(), and
+// the operands stay until then.
 class Products {
  public:
   Products(const at::TensorOptions &options, at::ScalarType type) : options_(options), type_(type) {}

@@ -987,7 +987,9 @@ FwdCost fwd_cost(const MambaScanParams &p, int nseg) {
 // third of that for what the passes share, a round's start and end 5.3.  The pass over the segments (all but one) takes 2.7
 // (forward) or 4.5 (backward) a tile, twice that from four of its workgroups per CU on, and every segment 0.9 or 1.8 for
 // its launch and for going through the segments before it; forward segments of a single tile, which a second launch and its wait for
-// the first outweigh, no less than 3.5 together.  A split has to promise 1 % (forward) or 6 % (backward).
+// the first outweigh, no less than 3.5 together.  A split has to promise 1 % (forward) or 6 % (backward).  (Up to 128
+// channels in all, smaller than any model's, scans are cut as before, 1 x 40 x 129 13.0 whole and 14.5 cut: the edges of segments
+// are checked against the oracle at those sizes.)
 // Forward scans that only scan_fwd_kernel takes (fwd_cost) keep the terms that were fitted to them: 6.4 a tile of a round of up
 // to two workgroups per CU, half as much again where two share one, 3.0 for a tile of the pass over the segments, 6 % to
 // promise.  (The terms for 16 states cut them too finely: 2 x 4160 x 1261, 4 states, 53 us whole and 70 in five segments; 2 x
@@ -1003,7 +1005,7 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
   const int64_t seg_wgs = rows * ((Dg + SEG_CH - 1) / SEG_CH);
   if (p.a_complex || p.batch > 65535 || k4_mode() || use_mx(p)) return 1;
   const int blocks = (p.dstate + NB16 - 1) / NB16;
-  const bool fine = !bwd && serial_takes(p);
+  const bool fine = !bwd && serial_takes(p), short_segments_cost = fine && (int64_t)p.batch * p.dim > 128;
   int best = 1;
   double best_cost = -1.0;
   for (int s = 1; s <= std::min(ntiles, MAX_SEGMENTS); ++s) {
@@ -1021,7 +1023,7 @@ int scan_segments(const MambaScanParams &p, bool bwd) {
     }
     if (s > 1) {
       const double share = std::max(1.0, 0.52 * (double)((seg_wgs * (s - 1) + cus - 1) / cus));
-      const double each = bwd ? 1.8 * s : fine && per == 1 ? std::max(3.5, 0.9 * s) : 0.9 * s;
+      const double each = bwd ? 1.8 * s : short_segments_cost && per == 1 ? std::max(3.5, 0.9 * s) : 0.9 * s;
       cost = (fine ? 1.01 : 1.06) * (cost + (bwd ? 4.5 : fine ? 2.7 : 3.0) * share * blocks * per + each);
     }
     if (best_cost < 0 || cost < best_cost) best_cost = cost, best = s;

@@ -23,6 +23,7 @@ def test_scans_of_the_other_kernel(b, d, L, G, N, const, want):
 # Scans that scan_fwd_serial_kernel takes, one sequence or a few of few channels, 16 states: the number that was measured the faster
 # one; times in us
 @pytest.mark.parametrize("b,d,L,want", [
+    (1, 144, 192, 1),      # 12.2 (2: 13.5)
     (1, 768, 129, 1),      # 13.3 (2: 14.9)
     (1, 768, 192, 1),      # 12.2 (2: 13.8)
     (1, 768, 256, 1),      # 12.2 (2: 13.7)
